@@ -79,6 +79,20 @@ VMI_LAYER_API int vmi_gpt2_embed_f16(const int64_t* input_ids, const int64_t* po
 VMI_LAYER_API int vmi_gpt2_argmax_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int64_t* out,
                                       int32_t device, void* stream);
 
+/* Causal self-attention of whole prompts straight from the projection's rows, and their keys and values into the paged cache:
+ * out[t, h] = softmax(scale q k^T) v over the positions 0 .. of t's prompt up to t's own (vllmini/model/gpt2.py:46-58, 71-78), and the
+ * bytes that cache_ops.reshape_and_cache writes for these rows (ext/cache_kernels.cu:152-207).
+ *   qkv          half [T, 3 E] rows of stride ld, q | k | v, E = num_heads * head_size; a prompt's rows are consecutive
+ *   tiles        int32 [num_tiles, 4], 16-byte aligned: prompt, its first row, first position of the tile, the prompt's length — one
+ *                for every tile_rows (64; heads of 128: 64 or 128) positions of every prompt, in any order
+ *   block_table  int32 [prompts, table_ld]: block of positions 16 j .. 16 j + 15; caches in the reference layout (head_size 64 or
+ *                128, block_size 16, float16), strides in elements, the same for both */
+VMI_LAYER_API int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, void* out, int64_t ldo, const int32_t* tiles,
+                                                int32_t num_tiles, int32_t tile_rows, int32_t num_heads, int32_t head_size,
+                                                float scale, void* key_cache, void* value_cache, const int32_t* block_table,
+                                                int32_t table_ld, int32_t block_size, int64_t kv_block_stride,
+                                                int64_t kv_head_stride, int32_t device, void* stream);
+
 /* Scheduler.sample_next_token (vllmini/scheduler.py:144-153: logits / temperature, top-k, softmax, one multinomial draw) for a
  * batch of rows in one launch: out[r] = the index drawn from softmax(top_k largest of logits[r, :] / temperature), the draw made by
  * inverse CDF over those top_k in descending order (ties: smaller index first) at uniform[r] in [0, 1) — the caller's random

@@ -448,3 +448,55 @@ def test_top_k_sampling_kernel_draws_from_the_reference_distribution():
     out = sample_top_k(row.expand(64, V).contiguous(), generator=torch.Generator(device=dev).manual_seed(1))
     assert out.dtype == torch.int64 and set(out.tolist()) <= set(torch.topk(row.float(), 50).indices[0].tolist())
 
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,lens,tile_rows", [(3, 64, [1, 15, 16, 17], 64), (2, 64, [63, 64, 65, 130], 64), (5, 64, [400], 64), (2, 128, [31, 257], 64),
+                                                (1, 128, [127, 128, 129, 1], 64), (1, 128, [127, 128, 129, 1], 128), (3, 128, [300, 17], 128)])
+def test_prompt_attention_matches_plain_attention_and_leaves_reshape_and_caches_bytes(H, D, lens, tile_rows):
+    """One launch over whole prompts against plain attention in float64, and its cache writes against cache_ops.reshape_and_cache: the
+    same bytes at the prompts' slots, nothing anywhere else.  A probability is rounded to half (2^-11 of it) and so is the result:
+    |error| <= 2^-11 sum p |v| + 2^-11 |out|, and as much again for float32 sums and exponentials."""
+    from vllmini_amd import cache_ops, gpt2_layer as gl
+
+    dev, E, T = torch.device("cuda:0"), H * D, sum(lens)
+    g = torch.Generator(device=dev).manual_seed(T * H + D)
+    wide = torch.randn((T, 3 * E + 8), generator=g, device=dev, dtype=torch.float32).half()
+    qkv = wide[:, : 3 * E]                                # (rows of a stride of their own)
+    per = [-(-n // 16) for n in lens]
+    blocks = torch.randperm(sum(per) + 3, generator=g, device=dev).to(torch.int32)
+    table = torch.full((len(lens), max(per) + 1), -1, dtype=torch.int32, device=dev)
+    slots, at = [], 0
+    for i, n in enumerate(lens):
+        table[i, : per[i]] = blocks[at: at + per[i]]
+        at += per[i]
+        pos = torch.arange(n, device=dev)
+        slots.append(table[i, pos // 16].long() * 16 + pos % 16)
+    kc = torch.randn((sum(per) + 3, H, D // 8, 16, 8), generator=g, device=dev).half()
+    vc = torch.randn((sum(per) + 3, H, D, 16), generator=g, device=dev).half()
+    kw, vw = kc.clone(), vc.clone()
+    q, k, v = (qkv[:, i * E:(i + 1) * E].view(T, H, D) for i in range(3))
+    cache_ops.reshape_and_cache(k, v, kw, vw, torch.cat(slots), "auto", 1.0)
+    tiles = torch.tensor([[i, sum(lens[:i]), a, n] for i, n in enumerate(lens) for a in range(0, n, tile_rows)], dtype=torch.int32, device=dev)
+    out = gl.prompt_attention(qkv, tiles, tile_rows, kc, vc, table, H, D ** -0.5)
+    assert torch.equal(kc, kw) and torch.equal(vc, vw)
+    at = 0
+    for n in lens:
+        a, b, c = (t[at: at + n].double().cpu().transpose(0, 1) for t in (q, k, v))
+        s = (a @ b.transpose(1, 2).contiguous()) * D ** -0.5 + torch.full((n, n), float("-inf"), dtype=torch.float64).triu(1)
+        w = torch.softmax(s, dim=-1)
+        want, size = (w @ c).transpose(0, 1), (w @ c.abs()).transpose(0, 1)
+        got = out[at: at + n].view(n, H, D).double().cpu()
+        assert bool(((got - want).abs() <= 2 * 2.0 ** -11 * (size + want.abs())).all())
+        at += n
+
+
+def test_prompt_tiles_cover_every_position_once():
+    from vllmini_amd import gpt2_layer as gl
+
+    for lens, heads, dim in (([5], 12, 64), ([1, 64, 65, 128, 900], 12, 128), (list(range(1, 120)), 16, 64), (list(range(1, 140)), 16, 128)):
+        tiles, rows = gl.prompt_tiles(lens, heads, dim)
+        assert rows == (128 if dim == 128 and sum(-(-n // 128) for n in lens) * heads >= 512 else 64)
+        seen = sorted((int(i), int(r) + q) for i, r, a, n in tiles for q in range(a, min(n, a + rows)))
+        assert seen == [(i, sum(lens[:i]) + q) for i, n in enumerate(lens) for q in range(n)]
+        assert all(int(n) == lens[i] for i, _, _, n in tiles)

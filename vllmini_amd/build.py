@@ -82,6 +82,7 @@ EXTRAS_LIB_PATH = os.path.join(OUT_DIR, "libvmi_paged_attention_extras.so")
 # the decode harness's own library (include/vmi_gpt2_layer.h): the GPT-2 block's linear layers — one unit, no shared objects,
 # not part of the operators' boundary; loaded by vllmini_amd/gpt2_layer.py only
 SRC_LAYER = os.path.join(CSRC, "gpt2_layer.hip")
+HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(INCLUDE, "vmi_gpt2_layer.h")]
 LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 
 # the layers of decoders that mix recurrences, linear and softmax attention (include/vmi_hybrid.h), loaded by hybrid_ops.py only
@@ -205,7 +206,7 @@ def layer_is_stale() -> bool:
     if not os.path.exists(LAYER_LIB_PATH):
         return True
     t = os.path.getmtime(LAYER_LIB_PATH)
-    return any(os.path.getmtime(d) > t for d in (SRC_LAYER, os.path.join(INCLUDE, "vmi_gpt2_layer.h")))
+    return any(os.path.getmtime(d) > t for d in (SRC_LAYER, *HDRS_LAYER))
 
 
 def build_layer(force: bool = False, verbose: bool = False) -> str:

@@ -640,6 +640,12 @@ __global__ __launch_bounds__(SK_T) void sample_top_k_kernel(const h16* __restric
   if (lane == pick) out[blockIdx.x] = 65535 - (int)(skey & 0xffffu);
 }
 
+}  // namespace vmi_layer
+
+#include "gpt2_prompt.hpp"
+
+namespace vmi_layer {
+
 // ---- host side ------------------------------------------------------------------------------------------------------------
 
 static thread_local std::string g_err;
@@ -706,6 +712,21 @@ static int launch(const LinearParams& p, const Shape& s, hipStream_t stream) {
     set_err("launch: ", hipGetErrorString(e));
     return VMI_LAYER_E_HIP;
   }
+  return VMI_LAYER_OK;
+}
+
+template <int D, int MI>
+static int launch_prompt(const PromptParams& p, int n_tiles, hipStream_t stream) {
+  auto* fn = prompt_attention_kernel<D, MI>;
+  constexpr size_t lds = (size_t)4 * PKT * (D + 8) * 2;
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      set_err("hipFuncSetAttribute: ", hipGetErrorString(e));
+      return VMI_LAYER_E_HIP;
+    }
+  }
+  hipLaunchKernelGGL(fn, dim3(n_tiles, p.heads), dim3(256), lds, stream, p);
   return VMI_LAYER_OK;
 }
 
@@ -837,6 +858,39 @@ int vmi_gpt2_embed_f16(const int64_t* input_ids, const int64_t* position_ids, co
   hipLaunchKernelGGL(embed_kernel, dim3(num_tokens), dim3(256), 0, static_cast<hipStream_t>(stream), input_ids, position_ids,
                      static_cast<const h16*>(wte), static_cast<const h16*>(wpe), static_cast<h16*>(out), hidden);
   return after_launch("vmi_gpt2_embed_f16", prev, device);
+}
+
+int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, void* out, int64_t ldo, const int32_t* tiles, int32_t num_tiles,
+                                  int32_t tile_rows, int32_t num_heads, int32_t head_size, float scale, void* key_cache,
+                                  void* value_cache, const int32_t* block_table, int32_t table_ld, int32_t block_size,
+                                  int64_t kv_block_stride, int64_t kv_head_stride, int32_t device, void* stream) {
+  using namespace vmi_layer;
+  static const char* who = "vmi_gpt2_prompt_attention_f16";
+  if (!qkv || !out || !tiles || !key_cache || !value_cache || !block_table || num_tiles <= 0 || num_heads <= 0 || num_heads > 65535 ||
+      table_ld <= 0 || kv_block_stride <= 0 || kv_head_stride <= 0 || !(scale > 0.f) || (tile_rows != 64 && tile_rows != 128)) {
+    set_err(who, ": null pointer, a size out of range, or tiles that are not of 64 or 128 rows");
+    return VMI_LAYER_E_ARG;
+  }
+  if ((head_size != 64 && head_size != 128) || (head_size == 64 && tile_rows != 64) || block_size != PROMPT_BS || (ld & 7) || ld < 3 * (int64_t)num_heads * head_size || (ldo & 3) ||
+      (kv_block_stride & 7) || (kv_head_stride & 7) || ((uintptr_t)qkv & 15) || ((uintptr_t)tiles & 15) || ((uintptr_t)out & 7) ||
+      ((uintptr_t)key_cache & 15) || ((uintptr_t)value_cache & 15)) {
+    set_err(who, ": built for heads of 64 (tiles of 64) or 128 over blocks of 16, rows and blocks aligned to 16 bytes");
+    return VMI_LAYER_E_SHAPE;
+  }
+  int prev = -1;
+  if (int rc = with_device(who, device, &prev)) return rc;
+  const PromptParams p{static_cast<const h16*>(qkv), ld, static_cast<h16*>(out), ldo, tiles, block_table, table_ld, num_heads,
+                       static_cast<h16*>(key_cache), static_cast<h16*>(value_cache), kv_block_stride, kv_head_stride,
+                       scale * 1.4426950408889634f};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  int rc;
+  if (head_size == 64) rc = launch_prompt<64, 1>(p, num_tiles, st);
+  else rc = tile_rows == 64 ? launch_prompt<128, 1>(p, num_tiles, st) : launch_prompt<128, 2>(p, num_tiles, st);
+  if (rc != VMI_LAYER_OK) {
+    if (prev != device) (void)hipSetDevice(prev);
+    return rc;
+  }
+  return after_launch(who, prev, device);
 }
 
 int vmi_gpt2_argmax_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int64_t* out, int32_t device,

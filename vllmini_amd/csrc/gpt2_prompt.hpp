@@ -1,0 +1,206 @@
+// Causal attention over whole prompts, and their keys and values into the paged cache, in one launch per layer (included by
+// gpt2_layer.hip; include/vmi_gpt2_layer.h: vmi_gpt2_prompt_attention_f16).
+//
+// A prompt's q, k and v lie in the projection's rows, so nothing is read back from the cache: a workgroup takes 64 * MI query
+// positions of one head and walks the keys up to its last position in tiles of 64, each through LDS once (requested one tile ahead,
+// two buffers, one barrier a tile).  A wave owns 16 * MI queries for all of it:
+//   * scores are formed transposed, S^T = K Q^T (D[row = key 4 kc + r][col = query r16]), so a lane keeps the scores of ONE query: its
+//     statistics need no LDS, its maximum two cross-lane swaps, and its probabilities, as they lie, are the B operand of
+//     O^T = V^T P^T: the sum over keys may take them in any order, so k-index 8 kc + e of a step of 32 stands for key 4 kc + e
+//     (e < 4) and 16 + 4 kc + e - 4, and the V^T operand is read column-wise from LDS in that same order (ds_read_b64_tr_b16);
+//   * the key tiles that lie on the workgroup's own positions are its prompt's pages: they leave from LDS as whole 16-byte pieces of
+//     the cache's layout, K[blk, h, d / 8, off, d % 8] and V[blk, h, d, off] — the bytes that reshape_and_cache would write.
+// Scores, softmax and accumulators are fp32; a probability is rounded once to half and what is summed is what multiplies V.
+//
+// What bounds it: the chain of a tile (LDS, scores, softmax, values: about 1.5 us) times the longest prompt's tiles, and from some
+// thousand workgroups on the vector unit's share of the softmax; the matrix cores are mostly idle, as few of a prompt's products are
+// here.  As a sequence of its own per position, for paged_attention_v1, every position read its keys again, and the cache was written by
+// a launch in front in 2-byte pieces.  24 prompts of up to 512 tokens (6 146 in all), 12 heads of 64, a layer: 205.6 + 30.2 -> 23.4 us; one
+// prompt of 37: 5.1 + 3.2 -> 3.9 us.
+#pragma once
+
+namespace vmi_layer {
+
+struct PromptParams {
+  const h16* qkv;         // [T][ld]: q | k | v, heads * D columns each
+  int64_t ld;
+  h16* out;               // [T][ldo]
+  int64_t ldo;
+  const int32_t* tiles;   // [n][4]: prompt, its first packed row, the tile's first position, the prompt's length
+  const int32_t* table;   // [prompts][table_ld]: this layer's blocks
+  int table_ld, heads;
+  h16* kcache;
+  h16* vcache;
+  int64_t bstride, hstride;
+  float scale2;           // scale * log2(e): scores in units of log 2
+};
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// four consecutive rows of one column of an LDS tile: lane r16 of each 16 holds column col0 + r16
+__device__ __forceinline__ h16x4 column4(const h16* tile, int ld, int row0, int col0, int r16) {
+  const h16* a = tile + (row0 + (r16 >> 2)) * ld + col0 + 4 * (r16 & 3);
+  return __builtin_bit_cast(h16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)a));
+}
+__device__ __forceinline__ h16x8 join(const h16x4& lo, const h16x4& hi) { return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7); }
+
+// over the four lanes that share r16: the rows of 16 lanes are swapped pairwise, no LDS round trip
+template <typename F>
+__device__ __forceinline__ float over_kc(float v, F op) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, v);
+  const auto s = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  const uint32_t b = __builtin_bit_cast(uint32_t, op(__builtin_bit_cast(float, (uint32_t)s[0]), __builtin_bit_cast(float, (uint32_t)s[1])));
+  const auto t = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return op(__builtin_bit_cast(float, (uint32_t)t[0]), __builtin_bit_cast(float, (uint32_t)t[1]));
+}
+
+constexpr int PKT = 64;      // keys of a tile: four pages of 16
+constexpr int PROMPT_BS = 16;
+
+template <int D, int MI>
+__global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptParams p) {
+  constexpr int LD = D + 8, NK = D / 32, NT = D / 16, UPR = D / 8, U = PKT * UPR / 256;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  h16* lds = reinterpret_cast<h16*>(smem);   // [2 buffers][K, V][64][LD]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int4 tile = *reinterpret_cast<const int4*>(p.tiles + 4 * blockIdx.x);
+  const int h = blockIdx.y, q0 = tile.z, len = tile.w, E = p.heads * D;
+  const h16* row0 = p.qkv + (int64_t)tile.y * p.ld + h * D;
+  const int32_t* table = p.table + (int64_t)tile.x * p.table_ld;
+  const int end = min(len, q0 + 64 * MI), nkt = (end + PKT - 1) / PKT;
+
+  h16x8 kr[U], vr[U];
+  auto load = [&](int kt) {   // (keys past the end repeat the last one: no lane-wise condition around a load)
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int u = tid + 256 * i;
+      const h16* src = row0 + (int64_t)min(kt * PKT + u / UPR, len - 1) * p.ld + E + (u % UPR) * 8;
+      kr[i] = *reinterpret_cast<const h16x8*>(src);
+      vr[i] = *reinterpret_cast<const h16x8*>(src + E);
+    }
+  };
+  load(0);
+  const int w0 = q0 + wave * 16 * MI;   // this wave's first position
+  h16x8 qf[MI][NK];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+      qf[mi][k] = *reinterpret_cast<const h16x8*>(row0 + (int64_t)min(w0 + mi * 16 + r16, len - 1) * p.ld + 32 * k + 8 * kc);
+  f32x4 o[MI][NT];
+  float mrun[MI], lrun[MI];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    mrun[mi] = -1e30f;
+    lrun[mi] = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) o[mi][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  for (int kt = 0; kt < nkt; ++kt) {
+    h16* ks = lds + (kt & 1) * 2 * PKT * LD;
+    h16* vs = ks + PKT * LD;
+    const int key0 = kt * PKT;
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int u = tid + 256 * i;
+      *reinterpret_cast<h16x8*>(ks + (u / UPR) * LD + (u % UPR) * 8) = kr[i];
+      *reinterpret_cast<h16x8*>(vs + (u / UPR) * LD + (u % UPR) * 8) = vr[i];
+    }
+    if (kt + 1 < nkt) load(kt + 1);
+    __syncthreads();   // (the writes of tile kt + 1 go where tile kt - 1 was read, which every wave has left behind)
+    if (key0 >= q0) {   // this workgroup's own positions: four pages into the cache
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int u = tid + 256 * i, pg = u / (16 * UPR), off = u & 15, d8 = (u >> 4) % UPR, pos = key0 + pg * PROMPT_BS;
+        if (pos + off < len)
+          *reinterpret_cast<h16x8*>(p.kcache + table[pos / PROMPT_BS] * p.bstride + h * p.hstride + (d8 * PROMPT_BS + off) * 8) =
+              *reinterpret_cast<const h16x8*>(ks + (pg * PROMPT_BS + off) * LD + d8 * 8);
+      }
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const int g = (tid >> 4) + 16 * i, half = g & 1, nt = (g >> 1) % NT, pg = g / (2 * NT), pos = key0 + pg * PROMPT_BS + half * 8;
+        const int at = pg * PROMPT_BS + half * 8;
+        const h16x8 v = join(column4(vs, LD, at, nt * 16, r16), column4(vs, LD, at + 4, nt * 16, r16));
+        if (pos < len) {
+          h16* dst = p.vcache + table[pos / PROMPT_BS] * p.bstride + h * p.hstride + (nt * 16 + r16) * PROMPT_BS + half * 8;
+          if (pos + 8 <= len) {
+            *reinterpret_cast<h16x8*>(dst) = v;
+          } else {   // the prompt ends inside: slots behind it are not this prompt's to write
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (pos + e < len) dst[e] = v[e];
+          }
+        }
+      }
+    }
+    if (w0 >= len || key0 > w0 + 16 * MI - 1) continue;   // (wave-uniform: none of its queries exists, or sees the tile)
+    f32x4 sc[MI][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi) sc[mi][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const h16x8 kf = *reinterpret_cast<const h16x8*>(ks + (j * 16 + r16) * LD + 32 * k + 8 * kc);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) sc[mi][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[mi][k], sc[mi][j], 0, 0, 0);
+      }
+    }
+    const bool whole = key0 + PKT - 1 <= w0;   // every query sees every key
+    h16x8 pf[MI][2];
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi) {
+      const int q = w0 + mi * 16 + r16;
+      float mx = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[mi][j][r] *= p.scale2;
+          if (!whole && key0 + j * 16 + 4 * kc + r > q) sc[mi][j][r] = -INFINITY;
+          mx = fmaxf(mx, sc[mi][j][r]);
+        }
+      mx = fmaxf(mrun[mi], over_kc(mx, [](float a, float b) { return fmaxf(a, b); }));
+      const float alpha = __builtin_amdgcn_exp2f(mrun[mi] - mx);
+      mrun[mi] = mx;
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const h16 pr = (h16)__builtin_amdgcn_exp2f(sc[mi][j][r] - mx);
+          sum += (float)pr;
+          pf[mi][j >> 1][(j & 1) * 4 + r] = pr;
+        }
+      lrun[mi] = lrun[mi] * alpha + sum;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) o[mi][nt] *= alpha;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const h16x8 vf = join(column4(vs, LD, 32 * k + 4 * kc, nt * 16, r16), column4(vs, LD, 32 * k + 16 + 4 * kc, nt * 16, r16));
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) o[mi][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[mi][k], o[mi][nt], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    const float inv = 1.f / over_kc(lrun[mi], [](float a, float b) { return a + b; });
+    const int q = w0 + mi * 16 + r16;
+    if (q >= len) continue;
+    h16* out = p.out + (int64_t)(tile.y + q) * p.ldo + h * D + 4 * kc;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      h16x4 y;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) y[r] = (h16)(o[mi][nt][r] * inv);
+      *reinterpret_cast<h16x4*>(out + nt * 16) = y;
+    }
+  }
+}
+
+}  // namespace vmi_layer

@@ -157,6 +157,13 @@ class GPT2PagedDecoder:
         # cache — instead of the reference's eager masked attention (gpt2.py:46-58): one launch per layer for all prompts of
         # the call, and prefill logits with the decode path's own arithmetic.  None = on a HIP device; False = eager.
         self.paged_prefill = (pool.device.type == "cuda") if paged_prefill is None else bool(paged_prefill)
+        # ... by one launch over whole prompts that also writes the cache, where it is built (gpt2_layer.prompt_attention): float16 pages
+        # of 16 tokens, heads of 64 or 128; the operators otherwise, and where the caller wants no native layers
+        self.prompt_kernel = self.paged_prefill and native_layers is not False and pool.device.type == "cuda" and wdt == torch.float16 \
+            and pool.kv_cache_dtype == "auto" and pool.block_size == gpt2_layer.PROMPT_BLOCK_SIZE \
+            and dims.head_size in gpt2_layer.PROMPT_HEAD_SIZES
+        if self.prompt_kernel:
+            gpt2_layer.load()
         self.pad_batch_to = int(pad_batch_to)      # decode steps are laid out for the next multiple of this many rows (0: as they come)
 
     # ---- pieces shared by prefill and decode --------------------------------------------------------
@@ -206,9 +213,10 @@ class GPT2PagedDecoder:
     def prefill_batch(self, seq_ids: Sequence[int], prompts: Sequence[Sequence[int]]) -> torch.Tensor:
         """Admission of several prompts in ONE pass (round 6): the prompts' tokens run through the block's layers as one
         packed [sum T, E] matrix, every layer writes ALL their K / V rows with one reshape_and_cache (concatenated slots —
-        the op is batched over tokens, cache_kernels.cu:219-260), and the causal attention is ONE paged_attention_v1 launch
-        over sum T "sequences" — position t of a prompt attends to the first t + 1 tokens of that prompt's pages, a ragged
-        batch the balanced kernels are built for (paged_prefill) — or, eager as the reference's prefill (gpt2.py:46-58,
+        the op is batched over tokens, cache_kernels.cu:219-260), and the causal attention is one launch for all prompts:
+        gpt2_layer.prompt_attention straight from the projection's rows, the cache write included (prompt_kernel), or
+        paged_attention_v1 over sum T "sequences" — position t of a prompt attends to the first t + 1 tokens of that prompt's
+        pages, a ragged batch the balanced kernels are built for (paged_prefill) — or, eager as the reference's prefill (gpt2.py:46-58,
         71-78), on the prompts padded to the longest, [n, H, T, T] scores at a time.
         Returns the last-token logits [n, V]; per sequence the arithmetic of prefill() up to GEMM tiling (eager) / of the
         decode steps that would have produced the same context (paged)."""
@@ -230,16 +238,22 @@ class GPT2PagedDecoder:
             for sid in done:       # all or nothing: the caller retries with a smaller group
                 pool.free(sid)
             raise
-        slots_dev = torch.from_numpy(np.ascontiguousarray(np.concatenate(slots, axis=1))).to(dev)     # [layers, sum T]
+        paged = self.paged_prefill
+        whole = paged and self.prompt_kernel
+        if not whole:
+            slots_dev = torch.from_numpy(np.ascontiguousarray(np.concatenate(slots, axis=1))).to(dev)     # [layers, sum T]
         ids = torch.as_tensor([t for p in prompts for t in p], dtype=torch.long, device=dev)
         starts = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
         pos = torch.from_numpy(np.concatenate([np.arange(T, dtype=np.int64) for T in lens])).to(dev)
         x = self.sd["transformer.wte.weight"][ids] + self.sd["transformer.wpe.weight"][pos]
-        paged = self.paged_prefill
         if paged:
             mbe = -(-max(lens) // pool.block_size)
-            seq_of_tok = torch.from_numpy(np.repeat(np.arange(n, dtype=np.int64), lens)).to(dev)
             tables_seq = torch.from_numpy(np.ascontiguousarray(np.stack(tabs, axis=1)[:, :, :mbe])).to(dev)   # [layers, n, mbe]
+        if whole:
+            tiles, tile_rows = gpt2_layer.prompt_tiles(lens, H, D)
+            tiles = torch.from_numpy(tiles).to(dev)
+        elif paged:
+            seq_of_tok = torch.from_numpy(np.repeat(np.arange(n, dtype=np.int64), lens)).to(dev)
             tables_tok = tables_seq[:, seq_of_tok, :].contiguous()                                              # [layers, sum T, mbe]
             lens_tok = (pos + 1).to(torch.int32)
             pvar = self._prefill_variant()
@@ -266,10 +280,14 @@ class GPT2PagedDecoder:
                           torch.from_numpy(idx[valid]).to(dev), mask))
         for i in range(d.n_layer):
             p = f"transformer.h.{i}."
-            q, k, v = self._qkv(self._ln(x, p + "ln_1"), p)                                       # [sum T, H, D] views
-            cache_ops.reshape_and_cache(k, v, pool.key_cache, pool.value_cache, slots_dev[i], pool.kv_cache_dtype, pool.kv_scale)
             a = torch.empty((x.shape[0], E), dtype=x.dtype, device=dev)
-            if paged:
+            if whole:
+                qkv = F.linear(self._ln(x, p + "ln_1"), self.sd[p + "attn.c_attn.weight"], self.sd[p + "attn.c_attn.bias"])
+                gpt2_layer.prompt_attention(qkv, tiles, tile_rows, pool.key_cache, pool.value_cache, tables_seq[i], H, self.scale, out=a)
+            else:
+                q, k, v = self._qkv(self._ln(x, p + "ln_1"), p)                                   # [sum T, H, D] views
+                cache_ops.reshape_and_cache(k, v, pool.key_cache, pool.value_cache, slots_dev[i], pool.kv_cache_dtype, pool.kv_scale)
+            if paged and not whole:
                 ops.paged_attention_v1(a.view(-1, H, D), q, pool.key_cache, pool.value_cache, H, self.scale, tables_tok[i], lens_tok,
                                        pool.block_size, mbe * pool.block_size, None, pool.kv_cache_dtype, pool.kv_scale, 0, 0, 1, 1, 0,
                                        _variant=pvar)

@@ -13,6 +13,7 @@ import os
 import threading
 from typing import Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import build as _build
@@ -27,6 +28,8 @@ SIGNATURES = {
     "vmi_gpt2_linear_qkv_cache_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i64, _i32, _i32, _i32,
                                                      _vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
+    "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
+                                                     _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_argmax_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_gpt2_sample_top_k_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, ctypes.c_float, _vp, _vp, _i32, _vp]),
     "vmi_gpt2_linear_kernel_name": (ctypes.c_char_p, [_i32, _i32, _i32, _i32, _i32]),
@@ -206,6 +209,56 @@ def embed(input_ids: torch.Tensor, position_ids: torch.Tensor, wte: torch.Tensor
         out = torch.empty((T, E), dtype=torch.float16, device=wte.device)
     _check(lib.vmi_gpt2_embed_f16(input_ids.data_ptr(), position_ids.data_ptr(), wte.data_ptr(), wpe.data_ptr(), out.data_ptr(),
                                   T, E, wte.device.index or 0, torch.cuda.current_stream(wte.device).cuda_stream))
+    return out
+
+
+PROMPT_HEAD_SIZES, PROMPT_BLOCK_SIZE = (64, 128), 16      # what prompt_attention is built for
+
+
+def prompt_tiles(lens, num_heads: int, head_size: int) -> Tuple[np.ndarray, int]:
+    """How prompt_attention's launch is cut: int32 [n, 4] (prompt, its first packed row, first position, length), the longest walks over
+    keys first, and the positions of a tile.  64 of them, a row tile a wave.  Heads of 128 take 128 (a key tile read from LDS serves two
+    row tiles of a wave) where that leaves two workgroups for every compute unit: 16 heads, 40 prompts of 500 tokens 165.8 -> 145.4 us,
+    4 of 900 57.7 -> 49.5, but 16 of 128 13.9 -> 14.7 (256 workgroups).  Heads of 64 lose by it at every size: 12 heads, 40 of 500
+    52.3 -> 54.3, 24 of up to 512 23.4 -> 26.7, one of 900 15.9 -> 24.0."""
+    lens = np.asarray(lens, dtype=np.int64)
+    rows = 128 if head_size == 128 and int((-(-lens // 128)).sum()) * num_heads >= 512 else 64
+    per = -(-lens // rows)
+    prompt = np.repeat(np.arange(len(lens)), per)
+    at = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * rows
+    tiles = np.stack([prompt, (np.cumsum(lens) - lens)[prompt], at, lens[prompt]], axis=1).astype(np.int32)
+    return np.ascontiguousarray(tiles[np.argsort(-np.minimum(at + rows, lens[prompt]), kind="stable")]), rows
+
+
+def prompt_attention(qkv: torch.Tensor, tiles: torch.Tensor, tile_rows: int, key_cache: torch.Tensor, value_cache: torch.Tensor,
+                     block_table: torch.Tensor, num_heads: int, scale: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Causal attention of whole prompts from the rows of their projection, qkv [T, 3E] half, and cache_ops.reshape_and_cache of those
+    rows, in one launch.  tiles: prompt_tiles() on the device; block_table int32 [prompts, n]: the blocks of every prompt."""
+    lib = load()
+    if qkv.device.type != "cuda":
+        raise RuntimeError("gpt2_layer.prompt_attention: there is no CPU path")
+    T, E = qkv.shape[0], qkv.shape[1] // 3
+    D = E // num_heads
+    if qkv.dtype != torch.float16 or qkv.stride(1) != 1 or qkv.shape[1] != 3 * num_heads * D or D not in PROMPT_HEAD_SIZES:
+        raise RuntimeError(f"gpt2_layer.prompt_attention: qkv half [T, 3E] of heads of {PROMPT_HEAD_SIZES}")
+    if key_cache.dtype != torch.float16 or value_cache.dtype != torch.float16 or key_cache.dim() != 5 or value_cache.dim() != 4 \
+            or tuple(key_cache.shape[1:]) != (num_heads, D // 8, PROMPT_BLOCK_SIZE, 8) \
+            or tuple(value_cache.shape[1:]) != (num_heads, D, PROMPT_BLOCK_SIZE) or not key_cache[0].is_contiguous() \
+            or not value_cache[0].is_contiguous() or key_cache.stride(0) != value_cache.stride(0):
+        raise RuntimeError("gpt2_layer.prompt_attention: float16 caches in the reference layout [NB, H, D/8, 16, 8] / [NB, H, D, 16]")
+    if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4 or not tiles.is_contiguous() or tile_rows not in ((64, 128) if D == 128 else (64,)) \
+            or block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1 \
+            or any(t.device != qkv.device for t in (tiles, block_table, key_cache, value_cache)):
+        raise RuntimeError("gpt2_layer.prompt_attention: tiles int32 [n, 4], block_table int32 [prompts, blocks], all on qkv's device")
+    if out is None:
+        out = torch.empty((T, E), dtype=torch.float16, device=qkv.device)
+    if out.shape != (T, E) or out.stride(1) != 1 or out.dtype != torch.float16 or out.device != qkv.device:
+        raise RuntimeError("gpt2_layer.prompt_attention: out [T, E] half with unit stride in E")
+    _check(lib.vmi_gpt2_prompt_attention_f16(qkv.data_ptr(), qkv.stride(0), out.data_ptr(), out.stride(0), tiles.data_ptr(), tiles.shape[0],
+                                             tile_rows, num_heads, D, float(scale), key_cache.data_ptr(), value_cache.data_ptr(),
+                                             block_table.data_ptr(), block_table.stride(0), PROMPT_BLOCK_SIZE, key_cache.stride(0),
+                                             key_cache.stride(1), qkv.device.index or 0,
+                                             torch.cuda.current_stream(qkv.device).cuda_stream))
     return out
 
 
