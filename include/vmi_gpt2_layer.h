@@ -93,6 +93,12 @@ VMI_LAYER_API int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, voi
                                                 int32_t table_ld, int32_t block_size, int64_t kv_block_stride,
                                                 int64_t kv_head_stride, int32_t device, void* stream);
 
+/* x [., E] += add [M, E] (NULL: nothing), and out [M, E] = layer norm of x's rows — of rows[m] where given (then without `add`) — in
+ * one launch: the residual add and the norm behind it (GPT2Block.forward), each rounded to half as the torch modules round.  All rows
+ * contiguous, 16-byte aligned, E % 8 == 0, E <= 4096. */
+VMI_LAYER_API int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const void* gamma, const void* beta, float eps,
+                                        void* out, int32_t M, int32_t E, int32_t device, void* stream);
+
 /* Scheduler.sample_next_token (vllmini/scheduler.py:144-153: logits / temperature, top-k, softmax, one multinomial draw) for a
  * batch of rows in one launch: out[r] = the index drawn from softmax(top_k largest of logits[r, :] / temperature), the draw made by
  * inverse CDF over those top_k in descending order (ties: smaller index first) at uniform[r] in [0, 1) — the caller's random

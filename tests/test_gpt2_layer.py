@@ -500,3 +500,29 @@ def test_prompt_tiles_cover_every_position_once():
         seen = sorted((int(i), int(r) + q) for i, r, a, n in tiles for q in range(a, min(n, a + rows)))
         assert seen == [(i, sum(lens[:i]) + q) for i, n in enumerate(lens) for q in range(n)]
         assert all(int(n) == lens[i] for i, _, _, n in tiles)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E", [8, 64, 520, 768, 1032, 2048, 4096])
+@pytest.mark.parametrize("M", [1, 4, 7])
+def test_add_norm_is_the_add_and_the_layer_norm(M, E):
+    """Against torch's add (the same rounding: equal) and layer_norm in float32 on the rounded stream: one rounding of the result (2^-11
+    of it), and as much again for the float32 steps before it."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(E + M)
+    x, y = ((torch.randn((M, E), generator=g, device=dev) * 3 + 1).half() for _ in range(2))
+    ln = (torch.randn(E, generator=g, device=dev).half(), torch.randn(E, generator=g, device=dev).half(), 1e-5)
+
+    def close(got, rows):
+        want = F.layer_norm(rows.double(), (E,), ln[0].double(), ln[1].double(), ln[2])
+        size = want.abs() + ln[0].double().abs() * 4 + ln[1].double().abs()      # (terms that may cancel)
+        assert bool(((got.double() - want).abs() <= 2.0 ** -10 * size).all())
+
+    z = x.clone()
+    close(gl.add_norm(z, ln, y), x + y)
+    assert torch.equal(z, x + y)
+    rows = torch.tensor([M - 1, 0], dtype=torch.int32, device=dev)
+    close(gl.add_norm(z, ln, rows=rows), z[rows.long()])
+    assert torch.equal(z, x + y)

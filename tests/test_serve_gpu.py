@@ -244,3 +244,26 @@ def test_newest_entry_reads_the_rows_and_leaves_the_cache_alone():
             ops.set_workspace_enabled(prev)
         torch.cuda.synchronize()
         assert torch.equal(out_n.view(torch.int16), out_p.view(torch.int16)), B
+
+
+def test_prompts_through_the_vendors_products_or_the_decode_kernels_give_the_same_logits():
+    """prefill_batch over whole prompts, on either side of NATIVE_PROMPT_MAX_TOKENS, against one prompt at a time; ids that no table
+    holds are refused before anything is allocated, negative ones count from the end."""
+    rng = np.random.default_rng(9)
+    prompts = [rng.integers(0, 500, n).tolist() for n in (70, 1, 128, 16)]
+    _, one = _model(num_blocks=400, paged_prefill=False)
+    ref = torch.stack([one.prefill(i, p) for i, p in enumerate(prompts)])
+    for most in (0, 10 ** 6):
+        _, many = _model(num_blocks=400)
+        assert many.prompt_kernel
+        many.NATIVE_PROMPT_MAX_TOKENS = most
+        got = many.prefill_batch(list(range(len(prompts))), prompts)
+        err = (got.float() - ref.float()).abs().max()
+        assert float(err) <= 2e-2 + 2e-2 * float(ref.float().abs().max()), (most, float(err))
+        with pytest.raises(IndexError):
+            many.prefill_batch([50], [[1, 2, many.dims.vocab_size]])
+        with pytest.raises(IndexError):
+            many.prefill_batch([50], [[1] * (many.dims.n_positions + 1)])
+        assert 50 not in many.pool.allocated_blocks
+        same = many.prefill_batch([51, 52], [[7, -1], [7, many.dims.vocab_size - 1]])
+        assert torch.equal(same[0], same[1])

@@ -893,6 +893,31 @@ int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, void* out, int64_
   return after_launch(who, prev, device);
 }
 
+int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const void* gamma, const void* beta, float eps, void* out,
+                          int32_t M, int32_t E, int32_t device, void* stream) {
+  using namespace vmi_layer;
+  static const char* who = "vmi_gpt2_add_norm_f16";
+  if (!x || !gamma || !beta || !out || M <= 0 || E <= 0 || (add && rows)) {
+    set_err(who, ": null pointer, non-positive size, or an addend together with chosen rows");
+    return VMI_LAYER_E_ARG;
+  }
+  if ((E & 7) || E > 4096 || ((uintptr_t)x & 15) || ((uintptr_t)add & 15) || ((uintptr_t)gamma & 15) || ((uintptr_t)beta & 15) ||
+      ((uintptr_t)out & 15)) {
+    set_err(who, ": needs E % 8 == 0, E <= 4096 and rows aligned to 16 bytes");
+    return VMI_LAYER_E_SHAPE;
+  }
+  int prev = -1;
+  if (int rc = with_device(who, device, &prev)) return rc;
+  auto go = [&](auto fn) {
+    hipLaunchKernelGGL(fn, dim3((M + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<h16*>(x), static_cast<const h16*>(add),
+                       rows, static_cast<const h16*>(gamma), static_cast<const h16*>(beta), static_cast<h16*>(out), M, E, eps);
+  };
+  if (E <= 1024) go(add_norm_kernel<2>);
+  else if (E <= 2048) go(add_norm_kernel<4>);
+  else go(add_norm_kernel<8>);
+  return after_launch(who, prev, device);
+}
+
 int vmi_gpt2_argmax_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int64_t* out, int32_t device,
                         void* stream) {
   using namespace vmi_layer;

@@ -203,4 +203,61 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
   }
 }
 
+// x += add (if given), and the layer norm of x (of `rows` of it) in half: one wave a row, the row in registers between the sum, the two
+// passes of its statistics (fp32) and the result.  Bound by memory: two rows read, two written.  As torch's add and layer_norm, two
+// launches that between them read the stream three times, 6 439 rows of 768: 6.0 + 13.5 -> 9.1 us.
+template <int UPL>   // 16-byte units of a row per lane
+__global__ __launch_bounds__(256) void add_norm_kernel(h16* __restrict__ x, const h16* __restrict__ add, const int32_t* __restrict__ rows,
+                                                       const h16* __restrict__ gamma, const h16* __restrict__ beta, h16* __restrict__ out,
+                                                       int M, int E, float eps) {
+  const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, units = E >> 3;
+  if (m >= M) return;
+  h16* row = x + (int64_t)(rows ? rows[m] : m) * E;
+  h16x8 v[UPL], y[UPL];
+  float f[UPL][8];
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) {   // (lanes past the row read its last unit again)
+    const int u = min(lane + 64 * i, units - 1) * 8;
+    v[i] = *reinterpret_cast<const h16x8*>(row + u);
+    if (add) y[i] = *reinterpret_cast<const h16x8*>(add + (int64_t)m * E + u);
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) {
+    const bool on = lane + 64 * i < units;
+    if (add) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = (h16)((float)v[i][e] + (float)y[i][e]);
+      if (on) *reinterpret_cast<h16x8*>(row + (lane + 64 * i) * 8) = v[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[i][e] = (float)v[i][e];
+      s += on ? f[i][e] : 0.f;
+    }
+  }
+  const float mean = group_sum<64>(s) / (float)E;
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) {
+    const bool on = lane + 64 * i < units;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[i][e] -= mean;
+      q = on ? fmaf(f[i][e], f[i][e], q) : q;
+    }
+  }
+  const float rstd = rsqrtf(group_sum<64>(q) / (float)E + eps);
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) {
+    if (lane + 64 * i >= units) continue;
+    const int u = (lane + 64 * i) * 8;
+    const h16x8 g = *reinterpret_cast<const h16x8*>(gamma + u), b = *reinterpret_cast<const h16x8*>(beta + u);
+    h16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (h16)fmaf(f[i][e] * rstd, (float)g[e], (float)b[e]);
+    *reinterpret_cast<h16x8*>(out + (int64_t)m * E + u) = o;
+  }
+}
+
 }  // namespace vmi_layer

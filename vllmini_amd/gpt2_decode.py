@@ -25,6 +25,7 @@ gpt2.py:240-241) so a reference checkpoint loads unchanged.
 from __future__ import annotations
 
 import dataclasses
+import itertools
 import math
 from typing import Dict, List, Optional, Sequence
 
@@ -84,6 +85,10 @@ class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
+    # prompts of more tokens in all take the vendor's products: by the GPU's time alone they are ahead from 400 tokens on (a layer's linears
+    # at 384 / 512 / 1024 / 1536 tokens 47 / 49 / 59 / 70 us, the decode step's kernels 46 / 51 / 77 / 109), but their eight launches a layer take the
+    # host 150 us where the five take 75, and that is what a call of so few tokens waits for: 1.96 against 1.12 ms at 1024, 2.02 against 1.54 at 1536
+    NATIVE_PROMPT_MAX_TOKENS = 1536
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
@@ -161,7 +166,8 @@ class GPT2PagedDecoder:
         # of 16 tokens, heads of 64 or 128; the operators otherwise, and where the caller wants no native layers
         self.prompt_kernel = self.paged_prefill and native_layers is not False and pool.device.type == "cuda" and wdt == torch.float16 \
             and pool.kv_cache_dtype == "auto" and pool.block_size == gpt2_layer.PROMPT_BLOCK_SIZE \
-            and dims.head_size in gpt2_layer.PROMPT_HEAD_SIZES
+            and dims.head_size in gpt2_layer.PROMPT_HEAD_SIZES and E <= gpt2_layer.ADD_NORM_MAX_WIDTH \
+            and all(state_dict[f"transformer.{k}.weight"].is_contiguous() for k in ("wte", "wpe"))
         if self.prompt_kernel:
             gpt2_layer.load()
         self.pad_batch_to = int(pad_batch_to)      # decode steps are laid out for the next multiple of this many rows (0: as they come)
@@ -226,6 +232,9 @@ class GPT2PagedDecoder:
             return torch.empty((0, self.dims.vocab_size), dtype=torch.float16, device=self.device)
         d, pool, dev = self.dims, self.pool, self.device
         H, D, E = d.n_head, d.head_size, d.n_embd
+        whole = self.paged_prefill and self.prompt_kernel
+        if whole:
+            ids_host = self._checked_ids(prompts, lens)
         done = []
         try:
             slots, tabs = [], []
@@ -238,10 +247,10 @@ class GPT2PagedDecoder:
             for sid in done:       # all or nothing: the caller retries with a smaller group
                 pool.free(sid)
             raise
+        if whole:
+            return self._whole_prompts(ids_host, lens, tabs)
         paged = self.paged_prefill
-        whole = paged and self.prompt_kernel
-        if not whole:
-            slots_dev = torch.from_numpy(np.ascontiguousarray(np.concatenate(slots, axis=1))).to(dev)     # [layers, sum T]
+        slots_dev = torch.from_numpy(np.ascontiguousarray(np.concatenate(slots, axis=1))).to(dev)     # [layers, sum T]
         ids = torch.as_tensor([t for p in prompts for t in p], dtype=torch.long, device=dev)
         starts = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
         pos = torch.from_numpy(np.concatenate([np.arange(T, dtype=np.int64) for T in lens])).to(dev)
@@ -249,10 +258,6 @@ class GPT2PagedDecoder:
         if paged:
             mbe = -(-max(lens) // pool.block_size)
             tables_seq = torch.from_numpy(np.ascontiguousarray(np.stack(tabs, axis=1)[:, :, :mbe])).to(dev)   # [layers, n, mbe]
-        if whole:
-            tiles, tile_rows = gpt2_layer.prompt_tiles(lens, H, D)
-            tiles = torch.from_numpy(tiles).to(dev)
-        elif paged:
             seq_of_tok = torch.from_numpy(np.repeat(np.arange(n, dtype=np.int64), lens)).to(dev)
             tables_tok = tables_seq[:, seq_of_tok, :].contiguous()                                              # [layers, sum T, mbe]
             lens_tok = (pos + 1).to(torch.int32)
@@ -280,14 +285,10 @@ class GPT2PagedDecoder:
                           torch.from_numpy(idx[valid]).to(dev), mask))
         for i in range(d.n_layer):
             p = f"transformer.h.{i}."
+            q, k, v = self._qkv(self._ln(x, p + "ln_1"), p)                                       # [sum T, H, D] views
+            cache_ops.reshape_and_cache(k, v, pool.key_cache, pool.value_cache, slots_dev[i], pool.kv_cache_dtype, pool.kv_scale)
             a = torch.empty((x.shape[0], E), dtype=x.dtype, device=dev)
-            if whole:
-                qkv = F.linear(self._ln(x, p + "ln_1"), self.sd[p + "attn.c_attn.weight"], self.sd[p + "attn.c_attn.bias"])
-                gpt2_layer.prompt_attention(qkv, tiles, tile_rows, pool.key_cache, pool.value_cache, tables_seq[i], H, self.scale, out=a)
-            else:
-                q, k, v = self._qkv(self._ln(x, p + "ln_1"), p)                                   # [sum T, H, D] views
-                cache_ops.reshape_and_cache(k, v, pool.key_cache, pool.value_cache, slots_dev[i], pool.kv_cache_dtype, pool.kv_scale)
-            if paged and not whole:
+            if paged:
                 ops.paged_attention_v1(a.view(-1, H, D), q, pool.key_cache, pool.value_cache, H, self.scale, tables_tok[i], lens_tok,
                                        pool.block_size, mbe * pool.block_size, None, pool.kv_cache_dtype, pool.kv_scale, 0, 0, 1, 1, 0,
                                        _variant=pvar)
@@ -300,6 +301,65 @@ class GPT2PagedDecoder:
             x = x + self._mlp(self._ln(x, p + "ln_2"), p)
         last = torch.from_numpy(starts[1:] - 1).to(dev)
         return F.linear(self._ln(x[last], "transformer.ln_f"), self.sd["lm_head.weight"])
+
+    def _checked_ids(self, prompts, lens) -> np.ndarray:
+        """The prompts' tokens in one row, as an index would take them: a negative one counts from the end, others past the tables are
+        refused (no kernel checks them)."""
+        V, P = self.sd["transformer.wte.weight"].shape[0], self.sd["transformer.wpe.weight"].shape[0]
+        ids = np.fromiter(itertools.chain.from_iterable(prompts), dtype=np.int64, count=sum(lens))
+        ids[ids < 0] += V
+        if len(ids) and (int(ids.min()) < 0 or int(ids.max()) >= V):
+            raise IndexError(f"a token id is out of range (vocabulary of {V})")
+        if max(lens) > P:
+            raise IndexError(f"a prompt of {max(lens)} tokens: the model has {P} positions")
+        return ids
+
+    def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
+        """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
+        takes four launches (the decode step's linear kernels) up to NATIVE_PROMPT_MAX_TOKENS tokens, seven beyond: the vendor's
+        products, and one kernel for the residual add with the norm behind it."""
+        d, pool, dev, sd, pw, n = self.dims, self.pool, self.device, self.sd, self._packed, len(lens)
+        H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
+        if T == 0:
+            raise RuntimeError("prefill_batch: a prompt needs at least one token")
+        tiles, tile_rows = gpt2_layer.prompt_tiles(lens, H, d.head_size)
+        parts = {"tiles": tiles, "tables": np.stack(tabs, axis=1)[:, :, :mbe], "ids": ids,
+                 "pos": np.concatenate([np.arange(k, dtype=np.int64) for k in lens]),
+                 "last": ((np.cumsum(lens) - 1) % T).astype(np.int32)}
+        at, total = {}, 0
+        for name, a in parts.items():
+            at[name] = total
+            total += (a.nbytes + 15) // 16 * 16
+        # (pinned, so the copy is asynchronous: from pageable memory it would wait for everything queued on the stream)
+        host = torch.empty(total, dtype=torch.uint8, pin_memory=True)
+        view = host.numpy()
+        for name, a in parts.items():
+            np.copyto(view[at[name]: at[name] + a.nbytes].view(a.dtype).reshape(a.shape), a)
+        up = host.to(dev, non_blocking=True)
+        kinds = {np.dtype(np.int32): torch.int32, np.dtype(np.int64): torch.int64}
+        up = {name: up[at[name]: at[name] + a.nbytes].view(kinds[a.dtype]).view(a.shape) for name, a in parts.items()}
+
+        x = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"])
+        native, add = self.native_layers and T <= self.NATIVE_PROMPT_MAX_TOKENS, None
+        for i in range(d.n_layer):
+            p = f"transformer.h.{i}."
+            ln_1, ln_2 = ((sd[f"{p}{k}.weight"], sd[f"{p}{k}.bias"], d.layer_norm_epsilon) for k in ("ln_1", "ln_2"))
+            if native:
+                qkv = gpt2_layer.linear(x, pw[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"], ln=ln_1)
+            else:
+                qkv = F.linear(gpt2_layer.add_norm(x, ln_1, add), sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
+            a = gpt2_layer.prompt_attention(qkv, up["tiles"], tile_rows, pool.key_cache, pool.value_cache, up["tables"][i], H, self.scale)
+            if native:
+                gpt2_layer.linear(a, pw[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"], residual=x, out=x)
+                h = gpt2_layer.linear(x, pw[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True, ln=ln_2)
+                gpt2_layer.linear(h, pw[p + "mlp.c_proj.weight"], sd[p + "mlp.c_proj.bias"], residual=x, out=x)
+            else:
+                h = gpt2_layer.add_norm(x, ln_2, F.linear(a, sd[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"]))
+                add = self._mlp(h, p)
+        if add is not None:
+            x += add
+        h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
+        return F.linear(h, sd["lm_head.weight"])
 
     def _prefill_variant(self) -> int:
         """The work decomposition of the prefill launch.  Its "sequences" are the positions of a few prompts: thousands of short

@@ -30,6 +30,7 @@ SIGNATURES = {
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
                                                      _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
+    "vmi_gpt2_add_norm_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_argmax_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_gpt2_sample_top_k_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, ctypes.c_float, _vp, _vp, _i32, _vp]),
     "vmi_gpt2_linear_kernel_name": (ctypes.c_char_p, [_i32, _i32, _i32, _i32, _i32]),
@@ -209,6 +210,33 @@ def embed(input_ids: torch.Tensor, position_ids: torch.Tensor, wte: torch.Tensor
         out = torch.empty((T, E), dtype=torch.float16, device=wte.device)
     _check(lib.vmi_gpt2_embed_f16(input_ids.data_ptr(), position_ids.data_ptr(), wte.data_ptr(), wpe.data_ptr(), out.data_ptr(),
                                   T, E, wte.device.index or 0, torch.cuda.current_stream(wte.device).cuda_stream))
+    return out
+
+
+ADD_NORM_MAX_WIDTH = 4096
+
+
+def add_norm(x: torch.Tensor, ln: Tuple[torch.Tensor, torch.Tensor, float], add: Optional[torch.Tensor] = None,
+             rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x += add in place (if given), then layer_norm(x) — of x[rows] where given — as a new tensor; half [., E], contiguous, one launch."""
+    lib = load()
+    if x.device.type != "cuda":
+        raise RuntimeError("gpt2_layer.add_norm: there is no CPU path")
+    E = x.shape[-1]
+    if x.dim() != 2 or x.dtype != torch.float16 or not x.is_contiguous() or (add is not None and (rows is not None or add.shape != x.shape
+                                                                             or add.dtype != torch.float16 or not add.is_contiguous()
+                                                                             or add.device != x.device)):
+        raise RuntimeError("gpt2_layer.add_norm: half [T, E], contiguous; add of the same shape, not together with rows")
+    if rows is not None and (rows.dtype != torch.int32 or rows.dim() != 1 or not rows.is_contiguous() or rows.device != x.device):
+        raise RuntimeError("gpt2_layer.add_norm: rows int32 [M]")
+    for t in ln[:2]:
+        if t.dtype != torch.float16 or t.shape != (E,) or not t.is_contiguous() or t.device != x.device:
+            raise RuntimeError("gpt2_layer.add_norm: gamma and beta half [E] on x's device")
+    M = x.shape[0] if rows is None else rows.shape[0]
+    out = torch.empty((M, E), dtype=torch.float16, device=x.device)
+    _check(lib.vmi_gpt2_add_norm_f16(x.data_ptr(), add.data_ptr() if add is not None else None, rows.data_ptr() if rows is not None else None,
+                                     ln[0].data_ptr(), ln[1].data_ptr(), float(ln[2]), out.data_ptr(), M, E, x.device.index or 0,
+                                     torch.cuda.current_stream(x.device).cuda_stream))
     return out
 
 
