@@ -61,6 +61,9 @@ typedef struct {
   int32_t x_kind, epilogue, dtype, device;
 } vmi_hy_linear_args;
 VMI_HY_API int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream);
+/* Whether a product of these sizes behind a norm keeps its rows in LDS: then it is ahead of a norm, a library product and what
+ * follows it, at any number of rows it is built for. */
+VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype);
 
 /* x[t, 0:width) = table[ids[t]] * scale (bfloat16 table of row length ld), zeros up to ld; float32 out */
 VMI_HY_API int vmi_hy_embed(const int64_t* ids, const void* table, float* x, int32_t T, int32_t width, int32_t ld, int32_t vocab,

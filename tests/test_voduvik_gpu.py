@@ -12,6 +12,7 @@ import sys
 import numpy as np
 import pytest
 import torch
+import torch.nn.functional as F
 
 from oracle import voduvik as plain
 from tests import voduvik_cases as cases
@@ -91,6 +92,37 @@ def test_linear_kinds(dtype, M, N, K):
     if K % 64 == 0:
         a, b = rnd(M, K // 2).to(dev()), rnd(M, K // 2).to(dev())
         close(ops.linear(a, t, x2=b, float_out=(N, 1.0)), torch.cat([a, b], 1).double() @ W.T, dtype)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16 * 3, 256), (2, 16 * 600, 288), (3, 16 * 514, 1024), (5, 32, 4096), (8, 16 * 1030, 320), (16, 16 * 258, 2080), (17, 16 * 512, 256),
+                                   (12, 512, 4096), (32, 16 * 515, 1024), (31, 16 * 600, 2048)])
+def test_rows_behind_a_norm_stay_in_lds(M, N, K):
+    """resident_kernel at the edges of what it deals out: rows over waves, k-steps over waves, slabs over workgroups (fewer, one more than a round,
+    several), one and two places for partial tiles; every epilogue against float64, the norm over fewer columns than there are."""
+    from vllmini_amd import hybrid_ops as ops
+
+    N = ops.pad32(N)
+    g = torch.Generator(device=dev()).manual_seed(M * K + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    t = ops.MatrixTiles((rnd(N, K) / K ** 0.5).to(torch.bfloat16), torch.bfloat16, dense=True)
+    assert ops.linear_resident(M, t) and not ops.linear_resident(33, t)
+    n, x, bias = K - 13, rnd(M + 2, K + 8)[:, :K] * 3 + 40, rnd(N)
+    nw = torch.zeros(K, device=dev())
+    nw[:n] = 1 + 0.5 * rnd(n)
+    x[:, n:] = 0
+    for rms in (False, True):
+        d = x[:, :n].double()
+        h = torch.zeros(M + 2, K, dtype=torch.float64, device=dev())
+        h[:, :n] = d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-5) * nw[:n] if rms else plain.layer_norm(d, nw[:n].double(), 1e-5)
+        y, norm = h @ t.dense.double().T, (nw, n, 1e-5, rms)
+        close(ops.linear(x[:M], t, norm=norm, bias=bias), y[:M] + bias, torch.bfloat16)
+        rows = torch.arange(M + 1, 1, -1, dtype=torch.int32, device=dev())
+        close(ops.linear(x, t, norm=norm, rows=rows, float_out=(N - 5, 0.3)), y[rows.long(), : N - 5] * 0.3, torch.bfloat16)
+        gate, up = y[:M, 0::2].clamp(max=0.8), y[:M, 1::2].clamp(-0.8, 0.8)
+        close(ops.linear(x[:M], t, norm=norm, glu=ops.GatedUnit.clamped(0.8)), gate * torch.sigmoid(1.702 * gate) * (up + 1), torch.bfloat16, tol16=3e-2)
+        split, rest = 16 * (N // 32), torch.empty((M, (N - 16 * (N // 32)) // 2), dtype=torch.bfloat16, device=dev())
+        close(ops.linear(x[:M], t, norm=norm, glu=ops.SILU_UNIT, glu_from=split, glu_out=rest), y[:M, :split], torch.bfloat16)
+        close(rest, F.silu(y[:M, split::2]) * y[:M, split + 1::2], torch.bfloat16, tol16=3e-2)
 
 
 @pytest.mark.parametrize("dtype", BOTH)

@@ -68,6 +68,55 @@ struct XUnit<T, VMI_HY_X_CONCAT> {
   __device__ __forceinline__ V8<T> finish(const float*, int, float, float) const { return from_f32<T>(v); }
 };
 
+// Four consecutive columns n .. n + 3 of row m, accumulated, on their way out.  n0: the first column of their tile (scalar)
+template <typename T, int EPI>
+__device__ __forceinline__ void epilogue(const vmi_hy_linear_args& p, const f32x4& acc, int m, int n, int n0, int grp) {
+  const int64_t yoff = (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride;
+  if constexpr (EPI == VMI_HY_E_STORE) {
+    f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (p.bias) b = *reinterpret_cast<const f32x4*>(p.bias + n);
+    V4<T> o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (T)(acc[r] + b[r]);
+    *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
+  } else if constexpr (EPI == VMI_HY_E_RESIDUAL) {
+    f32x4* y = reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + yoff + n);
+    *y = *y + acc;
+  } else if constexpr (EPI == VMI_HY_E_FLOAT) {
+    float* y = static_cast<float*>(p.y) + yoff + n;
+    if (n + 4 <= p.n_out && (p.ldy & 3) == 0) {
+      *reinterpret_cast<f32x4*>(y) = acc * p.scale;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (n + r < p.n_out) y[r] = acc[r] * p.scale;
+    }
+  } else if constexpr (EPI == VMI_HY_E_GLU) {
+    typename Elem<T>::v2 o;
+    o[0] = (T)glu(acc[0], acc[1], p.scale, p.glu_alpha, p.glu_up);
+    o[1] = (T)glu(acc[2], acc[3], p.scale, p.glu_alpha, p.glu_up);
+    *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y) + yoff + (n >> 1)) = o;
+  } else if constexpr (EPI == VMI_HY_E_STORE_GLU) {
+    if (n0 < p.n_split) {
+      V4<T> o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = (T)acc[r];
+      *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
+    } else {
+      typename Elem<T>::v2 o;
+      o[0] = (T)glu(acc[0], acc[1], p.scale, p.glu_alpha, p.glu_up);
+      o[1] = (T)glu(acc[2], acc[3], p.scale, p.glu_alpha, p.glu_up);
+      *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y2) + (int64_t)m * p.ldy2 + ((n - p.n_split) >> 1)) = o;
+    }
+  } else {   // VMI_HY_E_GATED
+    const float g = sigmoid((float)static_cast<const T*>(p.gate)[(int64_t)m * p.ldg + grp]);
+    V4<T> o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (T)(acc[r] * g);
+    *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
+  }
+}
+
 template <typename T, int BM, int NW, int KS, int XK, int EPI>
 __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear_args p) {
   using CK = Chunk<T, BM, KS>;
@@ -222,56 +271,206 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear
   }
   if (!nvalid) return;
 
-  const int n = n0 + 4 * kc;
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) {
     const int m = m0 + mi * 16 + r16;
-    if (m >= p.M) continue;
-    const int64_t yoff = (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride;
-    if constexpr (EPI == VMI_HY_E_STORE) {
-      f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (p.bias) b = *reinterpret_cast<const f32x4*>(p.bias + n);
-      V4<T> o;
+    if (m < p.M) epilogue<T, EPI>(p, acc[mi], m, n0 + 4 * kc, n0, grp);
+  }
+}
+
+// Steps of few rows whose x fits a compute unit's LDS (bfloat16, one group).  Such a product is the reading of its weights, so nothing but
+// that reading may take time:
+//   * a workgroup puts all rows of x into LDS once, normed / concatenated / rounded on the way: every wave has a share of a row and all of
+//     its loads in flight; after that the walk over K has no barrier and no load but the weights';
+//   * then it walks over slabs of 16 columns, blockIdx, blockIdx + grid, ..: its W waves take a W-th of K each and the ring of weight
+//     tiles runs on across slabs; a slab's partial tiles meet in LDS (two places, one barrier a slab) and one wave, another each time,
+//     adds them in a fixed order and stores;
+//   * rows past M repeat the last one: their results go nowhere.
+// In linear_kernel x comes in chunks of K behind a barrier each, and ONE wave makes a row's statistics in front of everything, behind the first
+// weights.  One row, K 4096: N 24576 57.4 -> 37.1 us (5.4 TB/s), N 8192 25.6 -> 17.1; K 1024: N 6144 10.1 -> 7.7, N 50272 30.6 -> 22.0; 16 rows, K 4096,
+// N 24576 67.6 -> 46.6; 32 rows, K 2048: N 22528 40.4 -> 29.9, N 50272 85.8 -> 51.9.  (Non-temporal loads of the weights: 36.5, but 77 against 74 us
+// for 412 MB and slower wherever they stay in the Infinity Cache.  16 waves a workgroup where there is one slab a compute unit: 9.9 -> 11.3.)
+template <int MT, int W, int PL, int CU, int XK, int EPI>
+__global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_linear_args p, const int slabs) {
+  constexpr int CS = 4, NB = CU > 1 ? 4 : 6;   // k-steps of a chunk, chunks of weights in registers (NB - 1 of them ahead)
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int LD = p.K + 8, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
+  f32x4* red = reinterpret_cast<f32x4*>(smem);                         // [PL][W - 1][MT][64]
+  float* part = reinterpret_cast<float*>(red + PL * (W - 1) * MT * 64);       // [W][2] parts of a row's sums
+  b16* xs = reinterpret_cast<b16*>(part + 2 * W);                      // [M][LD]
+  const int nks = p.K >> 5, kpw = (nks + W - 1) / W, nch = (kpw + CS - 1) / CS;
+  const int mine = (slabs - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, total = mine * nch;   // slabs, chunks of this workgroup
+
+  b16x8 wb[NB][CS];
+  const b16* wp = static_cast<const b16*>(p.w) + lane * 8;
+  int ls = blockIdx.x, lc = 0;   // the chunk to load next: slab and chunk of it
+  auto load_w = [&](b16x8(&dst)[CS]) {
+    const b16* at = wp + (int64_t)ls * nks * 512;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (T)(acc[mi][r] + b[r]);
-      *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
-    } else if constexpr (EPI == VMI_HY_E_RESIDUAL) {
-      f32x4* y = reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + yoff + n);
-      *y = *y + acc[mi];
-    } else if constexpr (EPI == VMI_HY_E_FLOAT) {
-      float* y = static_cast<float*>(p.y) + yoff + n;
-      if (n + 4 <= p.n_out && (p.ldy & 3) == 0) {
-        *reinterpret_cast<f32x4*>(y) = acc[mi] * p.scale;
-      } else {
+    for (int j = 0; j < CS; ++j) dst[j] = load8(at + (int64_t)min(wave * kpw + min(lc * CS + j, kpw - 1), nks - 1) * 512);
+    if (lc + 1 < nch) {
+      ++lc;
+    } else if (ls + (int)gridDim.x < slabs) {   // (past the last chunk: that one again, a cache hit)
+      lc = 0;
+      ls += gridDim.x;
+    }
+  };
+
+  // x into LDS: wpr waves a row, rpp rows at a time
+  const int M = p.M, upr = p.K >> 3;
+  const int wpr = M == 1 ? W : M == 2 ? W / 2 : M <= 4 ? W / 4 : M <= 8 ? W / 8 : 1, rpp = W / wpr, sub = wave % wpr, step8 = 64 * wpr;
+  const int u0 = sub * 64 + lane, upl = (upr + step8 - 1) / step8;   // this lane's units of a row of its wave: u0, u0 + step8, ..
+  auto row_at = [&](int round) { return min(round * rpp + wave / wpr, M - 1); };
+  const int rounds = (M + rpp - 1) / rpp;
+  auto open_ring = [&]() {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (n + r < p.n_out) y[r] = acc[mi][r] * p.scale;
+    for (int b = 0; b < NB - 1; ++b) load_w(wb[b]);
+  };
+  if constexpr (XK == VMI_HY_X_NORM) {
+    constexpr int HOLD = CU > 1 ? 2 : 4;   // units of 8 columns a lane keeps; longer shares are read again
+    f32x8 w[HOLD];
+    f32x8 v[HOLD];
+    float sh;
+    const float* row;
+    auto fetch = [&](int round) {
+      const int m = row_at(round);
+      row = static_cast<const float*>(p.x) + (p.rows ? p.rows[m] : m) * p.ldx;
+      sh = p.rms ? 0.f : row[0];
+#pragma unroll
+      for (int i = 0; i < HOLD; ++i) v[i] = load8(row + min(u0 + i * step8, upr - 1) * 8);
+    };
+    fetch(0);
+#pragma unroll
+    for (int i = 0; i < HOLD; ++i) w[i] = load8(p.norm_w + min(u0 + i * step8, upr - 1) * 8);
+    open_ring();   // (behind the first loads of x, so that waiting for those leaves the weights in flight)
+    for (int round = 0; round < rounds; ++round) {
+      float s = 0.f, q = 0.f;
+      auto sums = [&](const f32x8& x, int u) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = u * 8 + e < p.norm_n ? x[e] - sh : 0.f;
+          s += d;
+          q = fmaf(d, d, q);
+        }
+      };
+#pragma unroll
+      for (int i = 0; i < HOLD; ++i)
+        if (u0 + i * step8 < upr) sums(v[i], u0 + i * step8);
+      for (int u = u0 + HOLD * step8; u < upr; u += step8) sums(load8(row + u * 8), u);
+      s = wave_sum(s);
+      q = wave_sum(q);
+      if (wpr > 1) {
+        if (lane == 0) part[2 * wave] = s, part[2 * wave + 1] = q;
+        __syncthreads();
+        s = q = 0.f;
+        for (int i = 0; i < wpr; ++i) s += part[2 * (wave - sub + i)], q += part[2 * (wave - sub + i) + 1];
+        if (round + 1 < rounds) __syncthreads();
       }
-    } else if constexpr (EPI == VMI_HY_E_GLU) {
-      typename Elem<T>::v2 o;
-      o[0] = (T)glu(acc[mi][0], acc[mi][1], p.scale, p.glu_alpha, p.glu_up);
-      o[1] = (T)glu(acc[mi][2], acc[mi][3], p.scale, p.glu_alpha, p.glu_up);
-      *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y) + yoff + (n >> 1)) = o;
-    } else if constexpr (EPI == VMI_HY_E_STORE_GLU) {
-      if (n0 < p.n_split) {
-        V4<T> o;
+      const float ms = p.rms ? 0.f : s / (float)p.norm_n, mean = sh + ms;
+      const float rstd = 1.f / sqrtf(fmaxf(q / (float)p.norm_n - ms * ms, 0.f) + p.eps);
+      b16* to = xs + row_at(round) * LD;
+      auto put = [&](const f32x8& x, const f32x8& g, int u) {
+        f32x8 r;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = (T)acc[mi][r];
-        *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
-      } else {
-        typename Elem<T>::v2 o;
-        o[0] = (T)glu(acc[mi][0], acc[mi][1], p.scale, p.glu_alpha, p.glu_up);
-        o[1] = (T)glu(acc[mi][2], acc[mi][3], p.scale, p.glu_alpha, p.glu_up);
-        *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y2) + (int64_t)m * p.ldy2 + ((n - p.n_split) >> 1)) = o;
+        for (int e = 0; e < 8; ++e) r[e] = (x[e] - mean) * rstd * g[e];   // (the weight is zero past norm_n)
+        *reinterpret_cast<b16x8*>(to + u * 8) = from_f32<b16>(r);
+      };
+#pragma unroll
+      for (int i = 0; i < HOLD; ++i)
+        if (u0 + i * step8 < upr) put(v[i], w[i], u0 + i * step8);
+      for (int u = u0 + HOLD * step8; u < upr; u += step8) put(load8(row + u * 8), load8(p.norm_w + u * 8), u);
+      if (round + 1 < rounds) fetch(round + 1);
+    }
+  } else {
+    constexpr int HOLD = 4;
+    XUnit<b16, XK> v[HOLD];
+    int r0 = 0, i0 = 0;   // round and unit of the batch's first
+    for (int at = 0; at < rounds * upl; at += HOLD) {
+      int r = r0, i = i0;
+#pragma unroll
+      for (int h = 0; h < HOLD; ++h) {
+        v[h].load(p, row_at(r), 0, min(u0 + i * step8, upr - 1) * 8);
+        if (++i == upl) i = 0, ++r;
       }
-    } else {   // VMI_HY_E_GATED
-      const float g = sigmoid((float)static_cast<const T*>(p.gate)[(int64_t)m * p.ldg + grp]);
-      V4<T> o;
+      if (at == 0) open_ring();
+      r = r0, i = i0;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (T)(acc[mi][r] * g);
-      *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
+      for (int h = 0; h < HOLD; ++h) {   // (a clamped unit is written again with the same values)
+        *reinterpret_cast<b16x8*>(xs + row_at(r) * LD + min(u0 + i * step8, upr - 1) * 8) = v[h].finish(nullptr, 0, 0.f, 0.f);
+        if (++i == upl) i = 0, ++r;
+      }
+      r0 = r, i0 = i;
     }
   }
+  __syncthreads();
+
+  const b16* xa[MT];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) xa[mi] = xs + min(mi * 16 + r16, M - 1) * LD + 8 * kc;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int slab = blockIdx.x, c = 0, i = 0;   // of the chunk to multiply next; slabs done
+  auto step = [&](b16x8(&cur)[CS], b16x8(&nxt)[CS]) {
+    load_w(nxt);
+#pragma unroll
+    for (int j = 0; j < CS; ++j) {
+      const int kk = c * CS + j, k = wave * kpw + kk;
+      if (kk < kpw && k < nks) {   // (scalar)
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], load8(xa[mi] + k * 32));
+      }
+    }
+    if (++c < nch) return;
+    f32x4* to = red + (PL > 1 ? (i & 1) * (W - 1) * MT * 64 : 0);
+    const int behind = (wave - i) & (W - 1);   // 0: the wave that adds up; the others' places in their order behind it
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+      if (behind) to[((behind - 1) * MT + mi) * 64 + lane] = acc[mi];
+    __syncthreads();   // (two places: who still adds up slab i has not passed the barrier of slab i + 1; one: a second barrier)
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) {
+      if (behind == 0) {
+#pragma unroll
+        for (int w = 0; w < W - 1; ++w) acc[mi] += to[(w * MT + mi) * 64 + lane];
+        if (mi * 16 + r16 < M) epilogue<b16, EPI>(p, acc[mi], mi * 16 + r16, slab * 16 + 4 * kc, slab * 16, 0);
+      }
+      acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    if constexpr (PL == 1) __syncthreads();
+    c = 0;
+    ++i;
+    slab += gridDim.x;
+  };
+  for (int t = 0; t < total; t += NB) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      if (t + b < total) step(wb[b], wb[(b + NB - 1) % NB]);
+  }
+}
+
+inline size_t resident_lds(int M, int K, int W, int PL) { return (size_t)PL * (W - 1) * ((M + 15) / 16) * 1024 + 8 * W + (size_t)M * (K + 8) * 2; }
+
+// Whether, and how, a product behind a norm runs in resident_kernel.  2: two places for partial tiles and two workgroups a compute unit; 3: one place,
+// so that two workgroups still fit; 1: one workgroup, with a longer ring of weights; 0: not at all.  From 17 rows on a workgroup's reading of
+// x (32 rows of 1024: 128 KiB) needs enough slabs behind it: 32 rows, N 6144, K 1024 take 13.2 us here and 11.6 in linear_kernel, N 50272 28.4 and
+// 43.8.  Rows that need no norm (K 1024 .. 12288, N 1024 .. 4096) stay in linear_kernel, whose waves see x as early: 3.5 us there, 4.5 here
+// for one row of 1024, 22.0 and 21.5 for one of 12288.
+static int resident_kind(int M, int N, int K) {
+  if (M > 32 || K < 256 || (M > 16 && N < 16 * 512)) return 0;
+  if (resident_lds(M, K, 8, 2) <= LDS_PER_CU / 2) return 2;
+  if (M > 16 && resident_lds(M, K, 8, 1) <= LDS_PER_CU / 2) return 3;
+  return resident_lds(M, K, 8, 1) <= LDS_PER_CU ? 1 : 0;
+}
+
+template <int MT, int W, int PL, int CU, int XK, int EPI>   // CU workgroups a compute unit
+static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
+  auto* fn = resident_kernel<MT, W, PL, CU, XK, EPI>;
+  const size_t lds = resident_lds(p.M, p.K, W, PL);
+  if (int rc = allow_lds(fn, lds, "vmi_hy_linear")) return rc;
+  const int slabs = p.N / 16;
+  hipLaunchKernelGGL(fn, dim3(slabs < 256 * CU ? slabs : 256 * CU), dim3(64 * W), lds, st, p, slabs);
+  return launched("vmi_hy_linear");
 }
 
 template <typename T, int BM, int NW, int KS, int XK, int EPI>
@@ -290,6 +489,14 @@ template <typename T, int XK, int EPI>
 static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   // few rows: 16-row tiles; a layer with few columns splits K over the waves of a workgroup so that all compute units read
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
+  if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
+    switch (p.groups == 1 ? resident_kind(p.M, p.N, p.K) : 0) {
+      case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, XK, EPI>(p, st) : launch_resident<2, 8, 2, 2, XK, EPI>(p, st);
+      case 3: return launch_resident<2, 8, 1, 2, XK, EPI>(p, st);
+      case 1: return p.M <= 16 ? launch_resident<1, 8, 1, 1, XK, EPI>(p, st) : launch_resident<2, 8, 1, 1, XK, EPI>(p, st);
+      default: break;
+    }
+  }
   if (p.M <= 32) {
     const int64_t wgs = slabs * ((p.M + 15) / 16);
     if (wgs >= 2048) return launch_linear<T, 16, 4, 1, XK, EPI>(p, st);
@@ -495,6 +702,10 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ 
 using namespace vmi_hybrid;
 
 extern "C" {
+
+int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && resident_kind(M, N, K) != 0;
+}
 
 int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   static const char* who = "vmi_hy_linear";

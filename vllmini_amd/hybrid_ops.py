@@ -66,6 +66,7 @@ GqaArgs = _struct("GqaArgs", [(_vp, "q cache out bias sink gate tiles partial"),
 
 SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
+    "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "vmi_hy_add_norm": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp]),
     "vmi_hy_merge": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _f32, _i32, _i32, _vp]),
@@ -239,6 +240,11 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
                    x_kind=kind, epilogue=epi, dtype=DTYPES[T], device=device)
     _check(lib.vmi_hy_linear(ctypes.byref(a), stream))
     return out
+
+
+def linear_resident(M: int, w: MatrixTiles) -> bool:
+    """Whether linear(x, w, norm=...) of M rows keeps x in LDS."""
+    return w.groups == 1 and bool(load().vmi_hy_linear_resident(M, w.N, w.K, DTYPES[w.tiles.dtype]))
 
 
 def embed(ids: torch.Tensor, table: torch.Tensor, width: int, scale: float) -> torch.Tensor:
