@@ -2288,3 +2288,55 @@ def test_pa_v2_grouped_query_kernels(D):
                     continue
                 ran += 1
         assert ran >= 1, (D, H, hkv)
+
+
+def test_native_call_path_takes_the_plain_cases_and_leaves_the_others(monkeypatch):
+    """_vmi_host's functions launch the plain cases (same bits as the interpreter's own checks and call) and answer None, having written
+    nothing, for everything else: the operators then go their own way."""
+    from vllmini_amd import _lib, ops
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(4)
+    S, H, D, NB = 3, 4, 64, 12
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).half()      # noqa: E731
+    qkv, kc, vc = rnd(S, 3 * H * D), rnd(NB, H, D // 8, 16, 8), rnd(NB, H, D, 16)
+    q, k, v = (qkv[:, i * H * D:(i + 1) * H * D].view(S, H, D) for i in range(3))
+    tables = torch.randperm(NB, generator=g, device=dev)[:9].view(3, 3).to(torch.int32)
+    lens = torch.tensor([1, 17, 40], dtype=torch.int32, device=dev)
+    slots = torch.tensor([5, -1, 100], device=dev)
+    ops.paged_attention_v1(torch.empty_like(q), q, kc, vc, H, 0.1, tables, lens, 16, 48, None, "auto", 1.0)      # (loads library and workspace)
+    at, host = _lib.entries(), _lib.host()
+    for scale8 in (None, 0.5):
+        a, b = (kc, vc) if scale8 is None else (t.view(torch.uint8)[..., :16].contiguous() & 0x3f for t in
+                                                (kc.view(NB, H, D // 16, 16, 16), vc))
+        kind, ks = ("auto", 1.0) if scale8 is None else ("fp8", scale8)
+        args = lambda o, q=q, a=a, t=tables, n=lens, m=48, p=kind: (o, q, a, b, H, 0.1, t, n, 16, m, p, ks, 0, ops._WS)      # noqa: E731
+        got = torch.full((S, H, D), 9.0, dtype=torch.float16, device=dev)
+        assert host.attend(at, *args(got)) == 0
+        want = torch.empty_like(got)
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "entries", lambda: None)
+            ops.paged_attention_v1(want, q, a, b, H, 0.1, tables, lens, 16, 48, None, kind, ks)
+        assert torch.equal(got, want)
+        untouched = torch.full((S, H, D), 9.0, dtype=torch.float16, device=dev)
+        for other in (args(untouched, q=q.float()), args(untouched, q=q[:, :, ::2]), args(untouched.cpu()), args(untouched, t=tables.long()),
+                      args(untouched, t=tables[:, :2]), args(untouched, n=lens[:2]), args(untouched, a=a[:, 1:]), args(untouched, m=48.0),
+                      args(untouched, p="fp8_e5m2"), args(untouched[1:]), args(torch.nn.Module()), args(None)):
+            assert host.attend(at, *other) is None
+        assert bool((untouched == 9.0).all())
+        a1, b1, a2, b2 = a.clone(), b.clone(), a.clone(), b.clone()
+        assert host.cache(at, k, v, a1, b1, slots, kind, ks) == 0
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "entries", lambda: None)
+            ops.reshape_and_cache(k, v, a2, b2, slots, kind, ks)
+        assert torch.equal(a1, a2) and torch.equal(b1, b2) and not torch.equal(a1, a)
+        for other in ((k.float(), v, a, b, slots), (k, v[1:], a, b, slots), (k, v, a, b, slots.int()), (k, v, a, b, slots[1:]),
+                      (k, v, a[:, :, :, :, ::2], b, slots), (k, v, a.cpu(), b, slots), (k.transpose(1, 2), v.transpose(1, 2), a, b, slots)):
+            assert host.cache(at, *other, kind, ks) is None
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):      # a stream without a workspace yet: left to the operator, which makes one
+        out = torch.empty_like(q)
+        assert host.attend(at, out, q, kc, vc, H, 0.1, tables, lens, 16, 48, "auto", 1.0, 0, {}) is None
+        ops.paged_attention_v1(out, q, kc, vc, H, 0.1, tables, lens, 16, 48, None, "auto", 1.0)
+        assert host.attend(at, out, q, kc, vc, H, 0.1, tables, lens, 16, 48, "auto", 1.0, 0, ops._WS) == 0
+    side.synchronize()

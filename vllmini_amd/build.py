@@ -27,6 +27,9 @@ native code at all: hipcc translation units compiled concurrently and linked int
                                                     per-wave timeline there).  Used by tests that force kernel modes,
                                                     scripts/ and scripts/bench_diag.py — never by the operators.
 
+  vllmini_amd/_C/_vmi_host.so                       csrc/host_ops.cpp: what ops.py does per call, for the plain cases, in native
+                                                    code over torch's C++ interface (the libraries above know nothing of torch).
+
 Every object is compiled once and shared by the libraries that hold it (pa_queue.hip twice: its bfloat16 / E5M2 rows are
 behind -DVMI_EXTRAS).  hipcc cross-compiles without a GPU, so this runs in the build container; the .so files are
 git-ignored but travel to the GPU box with the repo snapshot (the objects do not: .gpurunignore).
@@ -89,6 +92,10 @@ LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 SRC_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hip") for t in ("linear", "rglru", "latent", "state", "attention")]
 HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "softmax")]
 HYBRID_LIB_PATH = os.path.join(OUT_DIR, "libvmi_hybrid.so")
+
+# the operators' checks and calls in native code: an extension module over torch's C++ interface, loaded by _lib.py (no device code)
+SRC_HOST = os.path.join(CSRC, "host_ops.cpp")
+HOST_LIB_PATH = os.path.join(OUT_DIR, "_vmi_host.so")
 
 ARCH = "gfx950"
 # -ffp-contract=off: the fp16 p*v products must be rounded before the fp16 adds (reference
@@ -246,6 +253,38 @@ def build_hybrid(force: bool = False, verbose: bool = False) -> str:
     return HYBRID_LIB_PATH
 
 
+def host_is_stale() -> bool:
+    if not os.path.exists(HOST_LIB_PATH):
+        return True
+    t = os.path.getmtime(HOST_LIB_PATH)
+    return any(os.path.getmtime(d) > t for d in (SRC_HOST, os.path.join(INCLUDE, "vmi_paged_attention.h")))
+
+
+def build_host(force: bool = False, verbose: bool = False) -> str:
+    """_vmi_host.so: one C++ unit against the installed torch (~30 s)."""
+    os.makedirs(OUT_DIR, exist_ok=True)
+    if not force and os.path.exists(HOST_LIB_PATH) and not _have_objects():
+        return HOST_LIB_PATH
+    if force or host_is_stale():
+        import sysconfig
+
+        import torch
+
+        root, tmp = os.path.dirname(torch.__file__), HOST_LIB_PATH + ".tmp"
+        rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include",
+               f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
+               SRC_HOST, "-o", tmp, f"-L{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+        if verbose:
+            print(" ".join(cmd), file=sys.stderr)
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"g++ failed ({proc.returncode}): {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+        os.replace(tmp, HOST_LIB_PATH)
+    return HOST_LIB_PATH
+
+
 def _have_objects() -> bool:
     return os.path.isdir(OUT_DIR) and any(f.endswith(".o") for f in os.listdir(OUT_DIR))
 
@@ -260,6 +299,7 @@ def build(force: bool = False, verbose: bool = False, diag: bool = False, extras
     os.makedirs(OUT_DIR, exist_ok=True)
     build_layer(force, verbose)
     build_hybrid(force, verbose)
+    build_host(force, verbose)
     kinds = ["product"] + (["extras"] if (extras or diag) else []) + (["diag"] if diag else [])
     if not force and not _have_objects() and not any(is_stale(k) for k in kinds):
         return _lib_of(kinds[-1])

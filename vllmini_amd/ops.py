@@ -295,6 +295,13 @@ def paged_attention_v1(
     Reference: attention_kernels.cu:805-826 (host), :86-496 (kernel).  `_variant` (keyword only,
     not part of the reference surface) forces a work decomposition for tuning/tests.
     """
+    at = _lib.entries()
+    if at is not None and alibi_slopes is None and blocksparse_vert_stride == 1:
+        # the plain cases: checked and launched in native code (csrc/host_ops.cpp); None: not one of them
+        rc = _lib.host().attend(at, out, query, key_cache, value_cache, num_kv_heads, scale, block_tables, seq_lens, block_size, max_seq_len,
+                                kv_cache_dtype, kv_scale, _variant, _WS if _ws_enabled else None)
+        if rc is not None:
+            return _raise_native(rc) if rc else None
     args = _pa_common(out, query, key_cache, value_cache, num_kv_heads, scale, block_tables,
                       seq_lens, block_size, max_seq_len, alibi_slopes, kv_cache_dtype, kv_scale,
                       tp_rank, blocksparse_local_blocks, blocksparse_vert_stride,
@@ -483,6 +490,11 @@ def reshape_and_cache(
 
     Reference: cache_kernels.cu:256-281 (host), :152-207 (kernel).
     """
+    at = _lib.entries()
+    if at is not None:      # the plain cases: checked and launched in native code (csrc/host_ops.cpp); None: not one of them
+        rc = _lib.host().cache(at, key, value, key_cache, value_cache, slot_mapping, kv_cache_dtype, kv_scale)
+        if rc is not None:
+            return _raise_native(rc) if rc else None
     fp8 = _check_kv_cache_dtype(kv_cache_dtype)
     kshape = key.shape
     if len(kshape) != 3 or kshape != value.shape:
