@@ -99,6 +99,26 @@ VMI_LAYER_API int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, voi
 VMI_LAYER_API int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const void* gamma, const void* beta, float eps,
                                         void* out, int32_t M, int32_t E, int32_t device, void* stream);
 
+/* All layers of whole prompts, the launches of vmi_gpt2_embed_f16, then per layer vmi_gpt2_linear_f16 (norm, c_attn),
+ * vmi_gpt2_prompt_attention_f16, vmi_gpt2_linear_f16 (c_proj, residual), (norm, c_fc, GELU), (c_proj, residual), then vmi_gpt2_add_norm_f16 of
+ * the prompts' last rows, issued from one call: a prompt of a few dozen tokens takes the GPU less time than sixty calls take an interpreter.
+ * Everything as those entries take it; block_tables [num_layers][num_prompts][table_ld], layer l's weights in layers[l], matrices in
+ * w_layout 1.  x, qkv, attended, hidden: scratch of num_tokens rows of E, 3 E, E and 4 E halves, 16-byte aligned; out: [num_prompts, E]. */
+typedef struct {
+  const void *ln_1_g, *ln_1_b, *c_attn, *c_attn_b, *attn_proj, *attn_proj_b, *ln_2_g, *ln_2_b, *c_fc, *c_fc_b, *mlp_proj, *mlp_proj_b;
+} vmi_gpt2_layer_weights;
+typedef struct {
+  const vmi_gpt2_layer_weights* layers;
+  const void *wte, *wpe, *ln_f_g, *ln_f_b;
+  const int64_t *input_ids, *position_ids;
+  const int32_t *tiles, *block_tables, *last_rows;
+  void *x, *qkv, *attended, *hidden, *out, *key_cache, *value_cache;
+  int64_t kv_block_stride, kv_head_stride;
+  int32_t num_layers, num_heads, head_size, num_tokens, num_prompts, num_tiles, tile_rows, table_ld, block_size, device;
+  float eps, scale;
+} vmi_gpt2_prompts;
+VMI_LAYER_API int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream);
+
 /* Scheduler.sample_next_token (vllmini/scheduler.py:144-153: logits / temperature, top-k, softmax, one multinomial draw) for a
  * batch of rows in one launch: out[r] = the index drawn from softmax(top_k largest of logits[r, :] / temperature), the draw made by
  * inverse CDF over those top_k in descending order (ties: smaller index first) at uniform[r] in [0, 1) — the caller's random

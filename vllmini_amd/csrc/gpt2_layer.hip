@@ -918,6 +918,33 @@ int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const v
   return after_launch(who, prev, device);
 }
 
+int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream) {
+  using namespace vmi_layer;
+  static const char* who = "vmi_gpt2_prompts_f16";
+  if (!a || !a->layers || !a->out || !a->last_rows || !a->block_tables || a->num_layers <= 0 || a->num_prompts <= 0 || a->num_heads <= 0 ||
+      a->head_size <= 0 || a->table_ld <= 0) {
+    set_err(who, ": null pointer or non-positive size");
+    return VMI_LAYER_E_ARG;
+  }
+  const int T = a->num_tokens, E = a->num_heads * a->head_size, dev = a->device;
+  int rc = vmi_gpt2_embed_f16(a->input_ids, a->position_ids, a->wte, a->wpe, a->x, T, E, dev, stream);
+  for (int l = 0; l < a->num_layers && rc == VMI_LAYER_OK; ++l) {
+    const vmi_gpt2_layer_weights& w = a->layers[l];
+    auto linear = [&](const void* x, int K, const void* m, const void* b, const void* g, const void* beta, const void* res, void* y, int N, int epi) {
+      return vmi_gpt2_linear_f16(x, K, m, b, g, beta, a->eps, res, N, y, N, T, N, K, epi, 1, dev, stream);
+    };
+    if ((rc = linear(a->x, E, w.c_attn, w.c_attn_b, w.ln_1_g, w.ln_1_b, nullptr, a->qkv, 3 * E, VMI_LAYER_EPI_BIAS))) break;
+    if ((rc = vmi_gpt2_prompt_attention_f16(a->qkv, 3 * E, a->attended, E, a->tiles, a->num_tiles, a->tile_rows, a->num_heads, a->head_size, a->scale,
+                                            a->key_cache, a->value_cache, a->block_tables + (int64_t)l * a->num_prompts * a->table_ld, a->table_ld,
+                                            a->block_size, a->kv_block_stride, a->kv_head_stride, dev, stream)))
+      break;
+    if ((rc = linear(a->attended, E, w.attn_proj, w.attn_proj_b, nullptr, nullptr, a->x, a->x, E, VMI_LAYER_EPI_BIAS_RESIDUAL))) break;
+    if ((rc = linear(a->x, E, w.c_fc, w.c_fc_b, w.ln_2_g, w.ln_2_b, nullptr, a->hidden, 4 * E, VMI_LAYER_EPI_BIAS_GELU))) break;
+    rc = linear(a->hidden, 4 * E, w.mlp_proj, w.mlp_proj_b, nullptr, nullptr, a->x, a->x, E, VMI_LAYER_EPI_BIAS_RESIDUAL);
+  }
+  return rc ? rc : vmi_gpt2_add_norm_f16(a->x, nullptr, a->last_rows, a->ln_f_g, a->ln_f_b, a->eps, a->out, a->num_prompts, E, dev, stream);
+}
+
 int vmi_gpt2_argmax_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int64_t* out, int32_t device,
                         void* stream) {
   using namespace vmi_layer;

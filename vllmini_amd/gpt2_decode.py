@@ -86,9 +86,9 @@ class GPT2PagedDecoder:
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
     # prompts of more tokens in all take the vendor's products: by the GPU's time alone they are ahead from 400 tokens on (a layer's linears
-    # at 384 / 512 / 1024 / 1536 tokens 47 / 49 / 59 / 70 us, the decode step's kernels 46 / 51 / 77 / 109), but their eight launches a layer take the
-    # host 150 us where the five take 75, and that is what a call of so few tokens waits for: 1.96 against 1.12 ms at 1024, 2.02 against 1.54 at 1536
-    NATIVE_PROMPT_MAX_TOKENS = 1536
+    # at 384 / 512 / 1024 / 2048 tokens 47 / 49 / 59 / 80 us, the decode step's kernels 46 / 51 / 77 / 132), but their eight launches a layer take
+    # the host 150 us, and that is what a call of so few tokens waits for: 1.95 against 1.09 ms at 1024, 2.08 against 1.80 at 2048
+    NATIVE_PROMPT_MAX_TOKENS = 2048
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
@@ -142,6 +142,7 @@ class GPT2PagedDecoder:
         if not can_scatter:
             self.scatter_in_c_attn = False
         self._packed: Dict[str, gpt2_layer.PackedWeight] = {}
+        self._prompt_tensors = None
         if self.native_layers:
             gpt2_layer.load()
             # the block weights once more as the MFMA tiles the kernels stream (include/vmi_gpt2_layer.h, w_layout 1): weights
@@ -316,9 +317,9 @@ class GPT2PagedDecoder:
 
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
         """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
-        takes four launches (the decode step's linear kernels) up to NATIVE_PROMPT_MAX_TOKENS tokens, seven beyond: the vendor's
-        products, and one kernel for the residual add with the norm behind it."""
-        d, pool, dev, sd, pw, n = self.dims, self.pool, self.device, self.sd, self._packed, len(lens)
+        takes four launches (the decode step's linear kernels) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by one native call,
+        and seven beyond: the vendor's products, and one kernel for the residual add with the norm behind it."""
+        d, pool, dev, sd = self.dims, self.pool, self.device, self.sd
         H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
         if T == 0:
             raise RuntimeError("prefill_batch: a prompt needs at least one token")
@@ -339,27 +340,33 @@ class GPT2PagedDecoder:
         kinds = {np.dtype(np.int32): torch.int32, np.dtype(np.int64): torch.int64}
         up = {name: up[at[name]: at[name] + a.nbytes].view(kinds[a.dtype]).view(a.shape) for name, a in parts.items()}
 
-        x = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"])
-        native, add = self.native_layers and T <= self.NATIVE_PROMPT_MAX_TOKENS, None
+        if self.native_layers and T <= self.NATIVE_PROMPT_MAX_TOKENS:
+            weights, ends = self._prompt_weights()
+            h = gpt2_layer.prompts(weights, ends, up["ids"], up["pos"], up["last"], up["tiles"], tile_rows, up["tables"], pool.key_cache,
+                                   pool.value_cache, H, d.head_size, d.layer_norm_epsilon, self.scale)
+            return F.linear(h, sd["lm_head.weight"])
+        x, add = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"]), None
         for i in range(d.n_layer):
             p = f"transformer.h.{i}."
             ln_1, ln_2 = ((sd[f"{p}{k}.weight"], sd[f"{p}{k}.bias"], d.layer_norm_epsilon) for k in ("ln_1", "ln_2"))
-            if native:
-                qkv = gpt2_layer.linear(x, pw[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"], ln=ln_1)
-            else:
-                qkv = F.linear(gpt2_layer.add_norm(x, ln_1, add), sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
+            qkv = F.linear(gpt2_layer.add_norm(x, ln_1, add), sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
             a = gpt2_layer.prompt_attention(qkv, up["tiles"], tile_rows, pool.key_cache, pool.value_cache, up["tables"][i], H, self.scale)
-            if native:
-                gpt2_layer.linear(a, pw[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"], residual=x, out=x)
-                h = gpt2_layer.linear(x, pw[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True, ln=ln_2)
-                gpt2_layer.linear(h, pw[p + "mlp.c_proj.weight"], sd[p + "mlp.c_proj.bias"], residual=x, out=x)
-            else:
-                h = gpt2_layer.add_norm(x, ln_2, F.linear(a, sd[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"]))
-                add = self._mlp(h, p)
-        if add is not None:
-            x += add
+            h = gpt2_layer.add_norm(x, ln_2, F.linear(a, sd[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"]))
+            add = self._mlp(h, p)
+        x += add
         h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
         return F.linear(h, sd["lm_head.weight"])
+
+    def _prompt_weights(self):
+        """The tensors that gpt2_layer.prompts reads, looked up and checked once (like the packed matrices among them)."""
+        if self._prompt_tensors is None:
+            sd, names = self.sd, gpt2_layer.LAYER_WEIGHTS
+            keys = [f"transformer.h.{i}.{k}" for i in range(self.dims.n_layer) for k in names]
+            weights = [self._packed[k].tiles if k in self._packed else sd[k] for k in keys]
+            ends = [sd[f"transformer.{k}"] for k in ("wte.weight", "wpe.weight", "ln_f.weight", "ln_f.bias")]
+            gpt2_layer.check_weights([*weights, *ends], weights[0].device)
+            self._prompt_tensors = weights, ends
+        return self._prompt_tensors
 
     def _prefill_variant(self) -> int:
         """The work decomposition of the prefill launch.  Its "sequences" are the positions of a few prompts: thousands of short

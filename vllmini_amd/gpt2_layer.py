@@ -22,6 +22,17 @@ ABI_VERSION = 1
 EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_RESIDUAL, EPI_BIAS_KV_CACHE = 0, 1, 2, 3
 
 _vp, _i32, _i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
+
+
+class Prompts(ctypes.Structure):
+    """vmi_gpt2_prompts."""
+    _fields_ = [(n, t) for t, names in (
+        (_vp, "layers wte wpe ln_f_g ln_f_b input_ids position_ids tiles block_tables last_rows x qkv attended hidden out key_cache value_cache"),
+        (_i64, "kv_block_stride kv_head_stride"),
+        (_i32, "num_layers num_heads head_size num_tokens num_prompts num_tiles tile_rows table_ld block_size device"),
+        (ctypes.c_float, "eps scale")) for n in names.split()]
+
+
 SIGNATURES = {
     "vmi_gpt2_linear_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i64, _vp, _i64,
                                            _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
@@ -31,6 +42,7 @@ SIGNATURES = {
     "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
                                                      _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_add_norm_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i32, _i32, _i32, _vp]),
+    "vmi_gpt2_prompts_f16": (ctypes.c_int, [ctypes.POINTER(Prompts), _vp]),
     "vmi_gpt2_argmax_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_gpt2_sample_top_k_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, ctypes.c_float, _vp, _vp, _i32, _vp]),
     "vmi_gpt2_linear_kernel_name": (ctypes.c_char_p, [_i32, _i32, _i32, _i32, _i32]),
@@ -287,6 +299,47 @@ def prompt_attention(qkv: torch.Tensor, tiles: torch.Tensor, tile_rows: int, key
                                              block_table.data_ptr(), block_table.stride(0), PROMPT_BLOCK_SIZE, key_cache.stride(0),
                                              key_cache.stride(1), qkv.device.index or 0,
                                              torch.cuda.current_stream(qkv.device).cuda_stream))
+    return out
+
+
+# a layer's weights in the order of vmi_gpt2_layer_weights (matrices as pack_weight() lays them out)
+LAYER_WEIGHTS = ("ln_1.weight", "ln_1.bias", "attn.c_attn.weight", "attn.c_attn.bias", "attn.c_proj.weight", "attn.c_proj.bias", "ln_2.weight", "ln_2.bias",
+                 "mlp.c_fc.weight", "mlp.c_fc.bias", "mlp.c_proj.weight", "mlp.c_proj.bias")
+
+
+def check_weights(tensors, device: torch.device) -> None:
+    """What prompts() reads by address: half, contiguous, 16-byte aligned, on one device."""
+    for t in tensors:
+        if t.dtype != torch.float16 or not t.is_contiguous() or t.device != device or t.data_ptr() % 16:
+            raise RuntimeError("gpt2_layer.prompts: weights must be contiguous, aligned half tensors on the pool's device")
+
+
+def prompts(weights, ends, input_ids: torch.Tensor, position_ids: torch.Tensor, last_rows: torch.Tensor, tiles: torch.Tensor, tile_rows: int,
+            block_tables: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, num_heads: int, head_size: int, eps: float,
+            scale: float) -> torch.Tensor:
+    """All layers over whole prompts, issued from one native call: the normed last rows [prompts, E].  weights: the layers' tensors, LAYER_WEIGHTS
+    each, one layer behind the other; ends: wte, wpe, ln_f weight and bias (check_weights() has seen them all); the others as prompt_attention and
+    embed take them, block_tables [layers, prompts, blocks]."""
+    T, E, n, dev = input_ids.shape[0], num_heads * head_size, last_rows.shape[0], input_ids.device
+    layers = len(weights) // len(LAYER_WEIGHTS)
+    if input_ids.dtype != torch.int64 or position_ids.dtype != torch.int64 or position_ids.shape != (T,) or last_rows.dtype != torch.int32 \
+            or tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4 or block_tables.dtype != torch.int32 \
+            or tuple(block_tables.shape[:2]) != (layers, n) or any(not t.is_contiguous() or t.device != dev for t in (
+                input_ids, position_ids, last_rows, tiles, block_tables)):
+        raise RuntimeError("gpt2_layer.prompts: int64 ids and positions [T], int32 last rows, tiles [n, 4] and tables [layers, prompts, blocks]")
+    if key_cache.dtype != torch.float16 or value_cache.dtype != torch.float16 or key_cache.device != dev or value_cache.device != dev \
+            or tuple(key_cache.shape[1:]) != (num_heads, head_size // 8, PROMPT_BLOCK_SIZE, 8) \
+            or tuple(value_cache.shape[1:]) != (num_heads, head_size, PROMPT_BLOCK_SIZE) or not key_cache[0].is_contiguous() \
+            or not value_cache[0].is_contiguous() or key_cache.stride(0) != value_cache.stride(0):
+        raise RuntimeError("gpt2_layer.prompts: float16 caches in the reference layout [NB, H, D/8, 16, 8] / [NB, H, D, 16]")
+    work = torch.empty((T, 9 * E), dtype=torch.float16, device=dev)      # x, qkv, attended, hidden
+    out = torch.empty((n, E), dtype=torch.float16, device=dev)
+    at, w = work.data_ptr(), (ctypes.c_void_p * len(weights))(*[t.data_ptr() for t in weights])
+    a = Prompts(ctypes.addressof(w), *[t.data_ptr() for t in (*ends, input_ids, position_ids, tiles, block_tables, last_rows)],
+                at, at + 2 * T * E, at + 8 * T * E, at + 10 * T * E, out.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
+                key_cache.stride(0), key_cache.stride(1), layers, num_heads, head_size, T, n, tiles.shape[0], tile_rows, block_tables.shape[2],
+                PROMPT_BLOCK_SIZE, dev.index or 0, eps, scale)
+    _check(load().vmi_gpt2_prompts_f16(ctypes.byref(a), torch.cuda.current_stream(dev).cuda_stream))
     return out
 
 
