@@ -49,7 +49,7 @@ $(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_softmax.h
 
 layer: $(LAYER_LIB)
 
-$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp include/vmi_gpt2_layer.h
+$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp $(CSRC)/gpt2_rows.hpp include/vmi_gpt2_layer.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $< -o $@
 

@@ -526,3 +526,23 @@ def test_add_norm_is_the_add_and_the_layer_norm(M, E):
     rows = torch.tensor([M - 1, 0], dtype=torch.int32, device=dev)
     close(gl.add_norm(z, ln, rows=rows), z[rows.long()])
     assert torch.equal(z, x + y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (16, 48, 224), (17, 144, 288), (3, 2304, 768), (47, 768, 1056), (33, 320, 2048), (112, 768, 3072), (5, 80, 4096)])
+def test_few_rows_split_k_over_the_waves(M, N, K):
+    """rows_kernel where its waves have unequal parts of K, or none; row tiles that are not full; more of them than XCDs: against the module chain,
+    for every epilogue it has, both weight layouts to the same bits."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    x, w, b, res = (rnd(M, K + 8) * 1.5 + 0.3).half()[:, :K], (rnd(N, K) * 0.6 / K ** 0.5).half(), (rnd(N) * 0.1).half(), rnd(M, N).half()
+    ln = ((1 + 0.2 * rnd(K)).half(), (0.1 * rnd(K)).half(), 1e-5)
+    for kw in ({"ln": ln}, {"ln": ln, "gelu": True}, {"residual": res}):
+        if kw.get("ln") and K > 2048:
+            continue
+        got = gl.linear(x, w, b, **kw)
+        _close(got, _chain(x, w, b, kw.get("ln"), kw.get("gelu", False), kw.get("residual")), (M, N, K, sorted(kw)))
+        assert torch.equal(gl.linear(x, gl.pack_weight(w), b, **kw), got)

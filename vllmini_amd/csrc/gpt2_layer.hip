@@ -140,6 +140,60 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// A lane's four consecutive columns n .. n + 3 of row m on their way out; n0: the first column of their slab (scalar).  load() asks early for what
+// store() will need.
+struct Tail {
+  h16x4 bias, res;
+  int64_t slot;   // EPI 3: the row's cache slot, -1 where there is nothing to write
+  template <int EPI>
+  __device__ __forceinline__ void load(const LinearParams& p, int m, int n, int n0) {
+    bias = res = h16x4{0, 0, 0, 0};
+    if (p.bias != nullptr) bias = *reinterpret_cast<const h16x4*>(p.bias + n);
+    if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL)
+      if (m < p.M) res = *reinterpret_cast<const h16x4*>(p.res + (int64_t)m * p.ldr + n);
+    slot = -1;
+    if constexpr (EPI == VMI_LAYER_EPI_BIAS_KV_CACHE)
+      if (n0 >= p.qdim && m < p.M) slot = p.slots[m];
+  }
+  template <int EPI>
+  __device__ __forceinline__ void store(const LinearParams& p, const f32x4& acc, int m, int n, int n0) const {
+    h16x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (h16)(acc[r] + (float)bias[r]);   // the linear layer's own half output
+    if constexpr (EPI == VMI_LAYER_EPI_BIAS_GELU) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float v = (float)o[r];
+        o[r] = (h16)(0.5f * v * (1.f + erff(v * 0.70710678118654752440f)));
+      }
+    } else if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = (h16)((float)res[r] + (float)o[r]);
+    }
+    *reinterpret_cast<h16x4*>(p.y + (int64_t)m * p.ldy + n) = o;
+    if constexpr (EPI == VMI_LAYER_EPI_BIAS_KV_CACHE) {
+      // reshape_and_cache's copy (cache_kernels.cu:172-199) done by the producer: K[blk, h, d / 8, off, d % 8], V[blk, h, d, off];
+      // a slab of 16 columns lies inside one of q | k | v and inside one head (E and head_size are multiples of 16)
+      const int part = n0 / p.qdim;   // wave-uniform
+      if (part > 0 && slot >= 0) {    // (a negative slot is a padded token: skipped, cache_kernels.cu:165-169)
+        const int64_t blk = slot >> p.bs_shift;     // block sizes are powers of two (8 / 16 / 32)
+        const int off = (int)(slot & (p.bs - 1));
+        const int c0 = n0 - part * p.qdim, hh = c0 / p.hsize, d = c0 - hh * p.hsize + n - n0;   // (hh: wave-uniform)
+        const int64_t base = blk * p.kv_bstride + (int64_t)hh * p.kv_hstride;
+        if (part == 1) {
+          // (non-temporal, like the scatter kernel's stores: a token's 2-byte V pieces dirty one 128-byte line each, and lines
+          //  left dirty in L2 are written back under the attention launch that follows — profiles/r02b_call_pair_aftermath.md)
+          __builtin_nontemporal_store(o, reinterpret_cast<h16x4*>(p.kcache + base + (int64_t)(d >> 3) * p.bs * 8 + off * 8 + (d & 7)));
+        } else {
+          h16* dst = p.vcache + base + (int64_t)d * p.bs + off;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) __builtin_nontemporal_store(o[r], dst + (int64_t)r * p.bs);
+        }
+      }
+    }
+  }
+};
+
 // Order of the memory requests (they complete in order, so what is needed first is asked for first): the row tile, weight
 // chunk 0, [tile to LDS], weight chunks 1 .. NBUF - 1, [LayerNorm], the ring of chunks.  For K = 768 (NBUF = 2) and for
 // mlp.c_proj's K = 3072 over two waves (NBUF = 4) everything a wave will ever read is in flight before its first MFMA.
@@ -199,28 +253,13 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const LinearParams 
 #pragma unroll
     for (int j = 0; j < CH; ++j) wb[b][j] = u32x4{0u, 0u, 0u, 0u};
   if (nvalid) load_w(wb[0], wrow, wstep, ks0, ks1);
-  // residual values of this lane's outputs: asked for now, used in the epilogue
-  const int n = n0 + 4 * kc;
-  h16x4 rr[MT];
-  if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL) {
-#pragma unroll
-    for (int mi = 0; mi < MT; ++mi) {
-      const int m = m0 + mi * 16 + r16;
-      rr[mi] = h16x4{0, 0, 0, 0};
-      if (nvalid && m < p.M) rr[mi] = *reinterpret_cast<const h16x4*>(p.res + (int64_t)m * p.ldr + n);
-    }
-  }
-  // EPI 3: the rows' cache slots too — a load in the epilogue would wait for the stores in front of it (loads and stores share
+  // what this lane's outputs will need, asked for now: a load in the epilogue would wait for the stores in front of it (loads and stores share
   // vmcnt), one acknowledged round trip per row block
-  int64_t slot[MT];
-  if constexpr (EPI == VMI_LAYER_EPI_BIAS_KV_CACHE) {
+  const int n = n0 + 4 * kc;
+  Tail tail[MT];
 #pragma unroll
-    for (int mi = 0; mi < MT; ++mi) {
-      const int m = m0 + mi * 16 + r16;
-      slot[mi] = -1;
-      if (nvalid && n0 >= p.qdim && m < p.M) slot[mi] = p.slots[m];
-    }
-  }
+  for (int mi = 0; mi < MT; ++mi)
+    if (nvalid) tail[mi].template load<EPI>(p, m0 + mi * 16 + r16, n, n0);
   if constexpr (!LN) {
     // 3. tile to LDS (the few shapes whose rows are longer than XU * LPR units finish them here, one more round trip each)
 #pragma unroll
@@ -311,52 +350,10 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const LinearParams 
   if (!nvalid) return;
 
   // D[row = 4 * kc + r -> column n][col = r16 -> row m]
-  float bias[4] = {0.f, 0.f, 0.f, 0.f};
-  if (p.bias != nullptr) {
-    const h16x4 b = *reinterpret_cast<const h16x4*>(p.bias + n);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) bias[r] = (float)b[r];
-  }
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) {
     const int m = m0 + mi * 16 + r16;
-    if (m >= p.M) continue;
-    h16x4 o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = (h16)(acc[mi][r] + bias[r]);   // the linear layer's own half output
-    if constexpr (EPI == VMI_LAYER_EPI_BIAS_GELU) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = (float)o[r];
-        o[r] = (h16)(0.5f * v * (1.f + erff(v * 0.70710678118654752440f)));
-      }
-    } else if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (h16)((float)rr[mi][r] + (float)o[r]);
-    }
-    *reinterpret_cast<h16x4*>(p.y + (int64_t)m * p.ldy + n) = o;
-    if constexpr (EPI == VMI_LAYER_EPI_BIAS_KV_CACHE) {
-      // reshape_and_cache's copy (cache_kernels.cu:172-199) done by the producer: K[blk, h, d / 8, off, d % 8], V[blk, h, d, off];
-      // a slab of 16 columns lies inside one of q | k | v and inside one head (E and head_size are multiples of 16)
-      const int part = n0 / p.qdim;   // wave-uniform
-      if (part > 0) {
-        if (slot[mi] >= 0) {          // (a negative slot is a padded token: skipped, cache_kernels.cu:165-169)
-          const int64_t blk = slot[mi] >> p.bs_shift;     // block sizes are powers of two (8 / 16 / 32)
-          const int off = (int)(slot[mi] & (p.bs - 1));
-          const int c0 = n0 - part * p.qdim, hh = c0 / p.hsize, d = c0 - hh * p.hsize + 4 * kc;   // (hh: wave-uniform)
-          const int64_t base = blk * p.kv_bstride + (int64_t)hh * p.kv_hstride;
-          if (part == 1) {
-            // (non-temporal, like the scatter kernel's stores: a token's 2-byte V pieces dirty one 128-byte line each, and lines
-            //  left dirty in L2 are written back under the attention launch that follows — profiles/r02b_call_pair_aftermath.md)
-            __builtin_nontemporal_store(o, reinterpret_cast<h16x4*>(p.kcache + base + (int64_t)(d >> 3) * p.bs * 8 + off * 8 + (d & 7)));
-          } else {
-            h16* dst = p.vcache + base + (int64_t)d * p.bs + off;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) __builtin_nontemporal_store(o[r], dst + (int64_t)r * p.bs);
-          }
-        }
-      }
-    }
+    if (m < p.M) tail[mi].template store<EPI>(p, acc[mi], m, n, n0);
   }
 }
 
@@ -643,6 +640,7 @@ __global__ __launch_bounds__(SK_T) void sample_top_k_kernel(const h16* __restric
 }  // namespace vmi_layer
 
 #include "gpt2_prompt.hpp"
+#include "gpt2_rows.hpp"
 
 namespace vmi_layer {
 
@@ -713,6 +711,49 @@ static int launch(const LinearParams& p, const Shape& s, hipStream_t stream) {
     return VMI_LAYER_E_HIP;
   }
   return VMI_LAYER_OK;
+}
+
+// Whether a linear layer goes to rows_kernel: where its workgroups, one for 16 columns of 16 rows, are at most two a compute unit.  Beyond, every
+// further row tile reads the weights again behind the others (K 768 behind a norm, 37 rows: N 2304, 432 of them, 6.3 -> 5.6 us; N 3072, 576,
+// 6.7 -> 7.1), and linear_kernel's row tiles in LDS are ahead; with a long K sooner (K 3072, 96 rows, 288: 12.4 -> 9.7; 128, 384: 8.9 -> 9.7).
+static bool rows_pick(int M, int N, int K, bool ln, int epi) {
+  const int j = rows_steps(K);
+  if (!j || (K & 31) || (N & 15) || (int64_t)(N >> 4) * ((M + 15) >> 4) > (K < 1536 ? 512 : 383)) return false;
+  return ln ? j <= 8 && epi != VMI_LAYER_EPI_BIAS_RESIDUAL : epi == VMI_LAYER_EPI_BIAS_RESIDUAL;
+}
+
+template <int J>
+static int launch_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream) {
+  const dim3 grid(((p.N >> 4) + 7) / 8 * 8 * ((p.M + 15) >> 4)), block(64 * RK);
+  auto go = [&](auto fn) {
+    hipLaunchKernelGGL(fn, grid, block, 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return (int)VMI_LAYER_OK;
+    set_err("launch: ", hipGetErrorString(e));
+    return (int)VMI_LAYER_E_HIP;
+  };
+  if (!ln) return go(rows_kernel<J, false, VMI_LAYER_EPI_BIAS_RESIDUAL>);
+  if constexpr (J <= 8) {
+    switch (epi) {
+      case VMI_LAYER_EPI_BIAS: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS>);
+      case VMI_LAYER_EPI_BIAS_GELU: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS_GELU>);
+      default: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS_KV_CACHE>);
+    }
+  }
+  return VMI_LAYER_E_SHAPE;   // (rows_pick asks for none of these)
+}
+
+static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream) {
+  switch (rows_steps(p.K)) {
+    case 1: return launch_rows<1>(p, ln, epi, stream);
+    case 2: return launch_rows<2>(p, ln, epi, stream);
+    case 3: return launch_rows<3>(p, ln, epi, stream);
+    case 4: return launch_rows<4>(p, ln, epi, stream);
+    case 6: return launch_rows<6>(p, ln, epi, stream);
+    case 8: return launch_rows<8>(p, ln, epi, stream);
+    case 12: return launch_rows<12>(p, ln, epi, stream);
+    default: return launch_rows<16>(p, ln, epi, stream);
+  }
 }
 
 template <int D, int MI>
@@ -786,7 +827,9 @@ static int linear_common(const char* who, const void* x, int64_t ldx, const void
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (epilogue == VMI_LAYER_EPI_BIAS_KV_CACHE) s.nbuf = 2;   // (the four-chunk ring is built for bias / GELU / residual only)
   int rc;
-  if (s.bm == 32)   // (three 32-row tiles side by side in LDS means K <= 845: never with a split K range)
+  if (rows_pick(M, N, K, ln, epilogue))
+    rc = run_rows(p, ln, epilogue, st);
+  else if (s.bm == 32)   // (three 32-row tiles side by side in LDS means K <= 845: never with a split K range)
     rc = launch_le<32, 4, 1, 2>(p, s, ln, epilogue, st);
   else if (s.nw == 1)
     rc = launch_le<16, 1, 4, 2>(p, s, ln, epilogue, st);
