@@ -94,18 +94,30 @@ def test_linear_kinds(dtype, M, N, K):
         close(ops.linear(a, t, x2=b, float_out=(N, 1.0)), torch.cat([a, b], 1).double() @ W.T, dtype)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 16 * 3, 256), (2, 16 * 600, 288), (3, 16 * 514, 1024), (5, 32, 4096), (8, 16 * 1030, 320), (16, 16 * 258, 2080), (17, 16 * 512, 256),
+@pytest.mark.parametrize("M,N,K", [(1, 32, 32), (16, 96, 224), (17, 160, 288), (3, 2048, 1024), (50, 512, 1056), (64, 1024, 2048), (33, 64, 512)])
+def test_few_rows_behind_a_norm_split_k_over_the_waves(M, N, K):
+    """rows_kernel where its waves have unequal parts of K, or none; row tiles that are not full; several of them."""
+    _norm_products(M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16 * 530, 256), (2, 16 * 600, 288), (3, 16 * 514, 1024), (5, 32, 4096), (8, 16 * 1030, 320), (16, 16 * 258, 2080), (17, 16 * 512, 256),
                                    (12, 512, 4096), (32, 16 * 515, 1024), (31, 16 * 600, 2048)])
 def test_rows_behind_a_norm_stay_in_lds(M, N, K):
     """resident_kernel at the edges of what it deals out: rows over waves, k-steps over waves, slabs over workgroups (fewer, one more than a round,
-    several), one and two places for partial tiles; every epilogue against float64, the norm over fewer columns than there are."""
+    several), one and two places for partial tiles."""
     from vllmini_amd import hybrid_ops as ops
 
-    N = ops.pad32(N)
+    t = _norm_products(M, ops.pad32(N), K)
+    assert ops.linear_resident(M, t) and not ops.linear_resident(33, t)
+
+
+def _norm_products(M, N, K):
+    """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
+    from vllmini_amd import hybrid_ops as ops
+
     g = torch.Generator(device=dev()).manual_seed(M * K + N)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
     t = ops.MatrixTiles((rnd(N, K) / K ** 0.5).to(torch.bfloat16), torch.bfloat16, dense=True)
-    assert ops.linear_resident(M, t) and not ops.linear_resident(33, t)
     n, x, bias = K - 13, rnd(M + 2, K + 8)[:, :K] * 3 + 40, rnd(N)
     nw = torch.zeros(K, device=dev())
     nw[:n] = 1 + 0.5 * rnd(n)
@@ -123,6 +135,7 @@ def test_rows_behind_a_norm_stay_in_lds(M, N, K):
         split, rest = 16 * (N // 32), torch.empty((M, (N - 16 * (N // 32)) // 2), dtype=torch.bfloat16, device=dev())
         close(ops.linear(x[:M], t, norm=norm, glu=ops.SILU_UNIT, glu_from=split, glu_out=rest), y[:M, :split], torch.bfloat16)
         close(rest, F.silu(y[:M, split::2]) * y[:M, split + 1::2], torch.bfloat16, tol16=3e-2)
+    return t
 
 
 @pytest.mark.parametrize("dtype", BOTH)

@@ -473,6 +473,90 @@ static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
   return launched("vmi_hy_linear");
 }
 
+// Few rows behind a norm and few columns (bfloat16, one group): a workgroup owns 16 columns of 16 rows and its EIGHT waves take an eighth of K
+// each.  A wave needs its part of a row once, so x and the weights go straight from memory to registers in the matrix cores' layout, all of it
+// requested before the first wait; the norm happens on those registers once the waves' parts of a row's sums have met in LDS.  Bound by one
+// trip through memory and the launch.  1 / 12 rows (linear_kernel before; resident_kernel, whose workgroups first bring whole rows into LDS):
+// K 1024, N 2048 6.5 / 7.1 (5.6 / 6.8) -> 4.7 / 5.6 us, N 6144 10.0 / 11.1 (7.7 / 9.7) -> 6.7 / 8.4; K 2048, N 4096 14.1 / 16.2 -> 8.0 / 9.9; 32 rows, K 1024, N 2048
+// 9.5 (9.4) -> 6.1.  Without a norm linear_kernel's waves see x as early: level at K 1024, 4.7 against 5.4 -> 6.0 for 12 rows of 3072.
+template <int J, int EPI>   // at most J k-steps a wave
+__global__ __launch_bounds__(512, 2) void rows_kernel(const vmi_hy_linear_args p) {
+  constexpr int RK = 8;
+  __shared__ f32x4 red[RK - 1][64];
+  __shared__ float sums[RK][2][16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
+  // (the row tiles of 16 columns go to one XCD, which then reads their weights once)
+  const int RB = (p.M + 15) >> 4, SL = p.N >> 4;
+  const int slab = (int)(blockIdx.x / (8 * RB)) * 8 + (int)(blockIdx.x & 7), m = (int)(blockIdx.x >> 3) % RB * 16 + r16;
+  if (slab >= SL) return;
+  const int nks = p.K >> 5, per = (nks + RK - 1) / RK, k0 = wave * per, nk = min(per, nks - k0);   // (nk <= 0: no part of K is left for it)
+  // (steps past this wave's last read it again and meet nothing: no lane-wise condition around a load)
+  auto at = [&](int j) { return 32 * min(k0 + min(j, per - 1), nks - 1) + 8 * kc; };
+  const int mm = min(m, p.M - 1);
+  const float* row = static_cast<const float*>(p.x) + (int64_t)(p.rows ? p.rows[mm] : mm) * p.ldx;
+  f32x8 x[J], nw[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) x[j] = load8(row + at(j));
+  const float sh = p.rms ? 0.f : row[0];
+#pragma unroll
+  for (int j = 0; j < J; ++j) nw[j] = load8(p.norm_w + at(j));
+  const b16* wp = static_cast<const b16*>(p.w) + ((int64_t)slab * nks * 64 + lane) * 8;
+  b16x8 w[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) w[j] = load8(wp + (int64_t)(at(j) >> 5) * 512);
+  float s = 0.f, q = 0.f;
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (j < nk) {   // (scalar)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = at(j) + e < p.norm_n ? x[j][e] - sh : 0.f;
+        s += d;
+        q = fmaf(d, d, q);
+      }
+    }
+  s += __shfl_xor(s, 16, 64), q += __shfl_xor(q, 16, 64);
+  s += __shfl_xor(s, 32, 64), q += __shfl_xor(q, 32, 64);
+  if (kc == 0) sums[wave][0][r16] = s, sums[wave][1][r16] = q;
+  __syncthreads();
+  s = q = 0.f;
+#pragma unroll
+  for (int v = 0; v < RK; ++v) s += sums[v][0][r16], q += sums[v][1][r16];
+  const float ms = p.rms ? 0.f : s / (float)p.norm_n, mean = sh + ms;
+  const float rstd = 1.f / sqrtf(fmaxf(q / (float)p.norm_n - ms * ms, 0.f) + p.eps);
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (j < nk) {
+      f32x8 r;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[e] = (x[j][e] - mean) * rstd * nw[j][e];   // (the weight is zero past norm_n)
+      mma(acc, w[j], from_f32<b16>(r));
+    }
+  if (wave > 0) red[wave - 1][lane] = acc;
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int v = 0; v < RK - 1; ++v) acc += red[v][lane];
+  if (m < p.M) epilogue<b16, EPI>(p, acc, m, slab * 16 + 4 * kc, slab * 16, 0);
+}
+
+// Whether a product behind a norm goes to rows_kernel: every workgroup reads its rows again, so only while they are few, and fewer where a row is long
+// (K 2048, N 6144, 384 of them: 13.3 us here, 10.2 in resident_kernel; 32 rows, K 1024, N 8192, 1024: 13.8 and 12.7)
+static bool rows_fit(int M, int N, int K) {
+  return M <= 64 && K <= 2048 && (int64_t)(N >> 4) * ((M + 15) >> 4) <= (K <= 1024 ? 512 : 256);
+}
+
+template <int EPI>
+static int launch_rows(const vmi_hy_linear_args& p, hipStream_t st) {
+  const int per = ((p.K >> 5) + 7) / 8;
+  auto go = [&](auto fn) {
+    hipLaunchKernelGGL(fn, dim3(((p.N >> 4) + 7) / 8 * 8 * ((p.M + 15) >> 4)), dim3(512), 0, st, p);
+    return launched("vmi_hy_linear");
+  };
+  return per <= 1 ? go(rows_kernel<1, EPI>) : per <= 2 ? go(rows_kernel<2, EPI>) : per <= 4 ? go(rows_kernel<4, EPI>) : go(rows_kernel<8, EPI>);
+}
+
 template <typename T, int BM, int NW, int KS, int XK, int EPI>
 static int launch_linear(const vmi_hy_linear_args& p, hipStream_t st) {
   constexpr int KC = Chunk<T, BM, KS>::KC, LD = KC + 16 / (int)sizeof(T);
@@ -490,6 +574,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   // few rows: 16-row tiles; a layer with few columns splits K over the waves of a workgroup so that all compute units read
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
+    if (p.groups == 1 && rows_fit(p.M, p.N, p.K)) return launch_rows<EPI>(p, st);
     switch (p.groups == 1 ? resident_kind(p.M, p.N, p.K) : 0) {
       case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, XK, EPI>(p, st) : launch_resident<2, 8, 2, 2, XK, EPI>(p, st);
       case 3: return launch_resident<2, 8, 1, 2, XK, EPI>(p, st);
