@@ -53,6 +53,7 @@ typedef struct {
   const void* gate;
   void* y;
   void* y2;
+  void* normed;          /* X_NORM, bfloat16: room for [M][K] of the element type: the rows are normed there first (NULL: on their way into the product) */
   int64_t ldx, ldy, ldg, ldy2;
   int64_t x_gstride, y_gstride;   /* elements from one group to the next */
   int32_t M, N, K, groups;
@@ -61,6 +62,8 @@ typedef struct {
   int32_t x_kind, epilogue, dtype, device;
 } vmi_hy_linear_args;
 VMI_HY_API int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream);
+/* Whether a product of these sizes behind a norm is faster over rows normed beforehand (`normed`) */
+VMI_HY_API int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype);
 /* Whether a product of these sizes behind a norm keeps its rows in LDS: then it is ahead of a norm, a library product and what
  * follows it, at any number of rows it is built for. */
 VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype);

@@ -3,7 +3,7 @@
 // y = epilogue(prologue(x) . W^T), written for steps of few rows, where the weights are what has to be read: every wave owns 16
 // output columns and streams its weight tiles (one contiguous KiB per k-step of 32) straight into registers one or two chunks ahead; the
 // BM rows of x go through LDS in chunks of K, double-buffered, normalised / concatenated / rounded to the element type on their
-// way in, so no normalised copy of the residual stream is ever written.  KS > 1: the k-steps of a chunk are dealt over KS waves
+// way in, so few rows need no normalised copy of the residual stream (norm_first: when they are better written once).  KS > 1: the k-steps of a chunk are dealt over KS waves
 // whose partial tiles meet in LDS in a fixed order.  D[row = column n][col = row m]: a lane ends with 4 consecutive columns of
 // one row, so every epilogue works on vectors.
 #include <string>
@@ -547,6 +547,17 @@ static bool rows_fit(int M, int N, int K) {
   return M <= 64 && K <= 2048 && (int64_t)(N >> 4) * ((M + 15) >> 4) <= (K <= 1024 ? 512 : 256);
 }
 
+// Whether the rows behind a norm are better normed once, by a kernel of their own (3.3 us between two others), than in every workgroup of the product:
+// from 17 rows on, where the workgroups' share of that is 32 rows a column of tiles, except of a vocabulary's columns behind rows that stay in LDS;
+// from 9 on where a row is long and its columns few.  32 rows (in every workgroup -> once): K 1024, N 8192 15.0 -> 11.6 us; K 2048, N 4096 15.3 -> 12.2,
+// N 12288 22.4 -> 20.7, N 50272 52.3 -> 56.7; K 4096, N 4096 25.0 -> 18.3, N 12288 56.3 -> 35.5.  40: K 2048, N 12288 30.0 -> 21.8, K 4096, N 24576
+// 84.4 -> 54.4.  16: K 2048, N 8192 17.4 -> 14.6, N 24576 26.7 -> 27.0; K 4096, N 4096 19.3 -> 16.4; K 1024, N 8192 9.6 -> 10.5.  8: K 4096, N 8192 21.8 -> 21.4.
+static bool norm_first(int M, int N, int K) {
+  if (K < 1024 || rows_fit(M, N, K)) return false;
+  if (M > 16) return M > 32 || N < 24576 || resident_kind(M, N, K) == 0;
+  return M > 8 && K >= 2048 && N <= 4 * K;
+}
+
 template <int EPI>
 static int launch_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   const int per = ((p.K >> 5) + 7) / 8;
@@ -599,6 +610,9 @@ static int linear_kind(const vmi_hy_linear_args& p, hipStream_t st) {
   switch (p.x_kind * 8 + p.epilogue) {
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_STORE: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_STORE>(p, st);
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_RESIDUAL: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_RESIDUAL>(p, st);
+    case VMI_HY_X_ROWS * 8 + VMI_HY_E_FLOAT: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_FLOAT>(p, st);
+    case VMI_HY_X_ROWS * 8 + VMI_HY_E_GLU: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_GLU>(p, st);
+    case VMI_HY_X_ROWS * 8 + VMI_HY_E_STORE_GLU: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_STORE_GLU>(p, st);
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_GATED: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_GATED>(p, st);
     case VMI_HY_X_NORM * 8 + VMI_HY_E_STORE: return linear_shape<T, VMI_HY_X_NORM, VMI_HY_E_STORE>(p, st);
     case VMI_HY_X_NORM * 8 + VMI_HY_E_FLOAT: return linear_shape<T, VMI_HY_X_NORM, VMI_HY_E_FLOAT>(p, st);
@@ -623,13 +637,13 @@ __global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ 
   }
 }
 
-// one workgroup per row; a row of up to 4 * 4096 columns stays in registers between the three passes
+// one workgroup per row of x, or of its rows[t]; a row of up to 4 * 4096 columns stays in registers between the three passes
 template <typename T>
-__global__ __launch_bounds__(256) void add_norm_kernel(float* x, const T* add, int64_t ld_add, const float* norm_w, T* out, int n,
-                                                       int ld, float eps, int rms) {
+__global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, const int* rows, const T* add, int64_t ld_add,
+                                                       const float* norm_w, T* out, int n, int ld, float eps, int rms) {
   __shared__ float part[2][4];
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float* row = x + (int64_t)t * ld;
+  float* row = x + (rows ? rows[t] : t) * ldx;
   constexpr int MAXV = 8;
   f32x4 v[MAXV];
   float s = 0.f;
@@ -788,6 +802,10 @@ using namespace vmi_hybrid;
 
 extern "C" {
 
+int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups == 1 && norm_first(M, N, K);
+}
+
 int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
   return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && resident_kind(M, N, K) != 0;
 }
@@ -807,6 +825,13 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a->x_kind == VMI_HY_X_NORM && a->normed && a->dtype == VMI_HY_BF16) {
+    hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
+                       (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
+    vmi_hy_linear_args rows = *a;
+    rows.x = a->normed, rows.ldx = a->K, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;
+    return linear_kind<b16>(rows, st);
+  }
   return a->dtype == VMI_HY_BF16 ? linear_kind<b16>(*a, st) : linear_kind<float>(*a, st);
 }
 
@@ -829,10 +854,10 @@ int vmi_hy_add_norm(float* x, const void* add, int64_t ld_add, const float* norm
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == VMI_HY_BF16)
-    hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(T), dim3(256), 0, st, x, static_cast<const b16*>(add), ld_add, norm_w,
+    hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(T), dim3(256), 0, st, x, (int64_t)ld, nullptr, static_cast<const b16*>(add), ld_add, norm_w,
                        static_cast<b16*>(out), n, ld, eps, rms);
   else
-    hipLaunchKernelGGL(add_norm_kernel<float>, dim3(T), dim3(256), 0, st, x, static_cast<const float*>(add), ld_add, norm_w,
+    hipLaunchKernelGGL(add_norm_kernel<float>, dim3(T), dim3(256), 0, st, x, (int64_t)ld, nullptr, static_cast<const float*>(add), ld_add, norm_w,
                        static_cast<float*>(out), n, ld, eps, rms);
   return launched(who);
 }

@@ -43,7 +43,7 @@ def _struct(name, fields):
     return type(name, (ctypes.Structure,), {"_fields_": [(n, t) for t, names in fields for n in names.split()]})
 
 
-LinearArgs = _struct("LinearArgs", [(_vp, "x x2 rows norm_w w bias gate y y2"), (_i64, "ldx ldy ldg ldy2 x_gstride y_gstride"),
+LinearArgs = _struct("LinearArgs", [(_vp, "x x2 rows norm_w w bias gate y y2 normed"), (_i64, "ldx ldy ldg ldy2 x_gstride y_gstride"),
                                     (_i32, "M N K groups norm_n n_out n_split rms"), (_f32, "eps scale glu_alpha glu_up"),
                                     (_i32, "x_kind epilogue dtype device")])
 StepArgs = _struct("StepArgs", [(_vp, "tok_seq tok_pos tok_slot q_start q_len ctx state_slot flip table chunks chunk_start"),
@@ -66,6 +66,7 @@ GqaArgs = _struct("GqaArgs", [(_vp, "q cache out bias sink gate tiles partial"),
 
 SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
+    "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "vmi_hy_add_norm": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp]),
@@ -230,7 +231,10 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
         out = torch.empty((M, cols), dtype=odt, device=x.device)
     _need(out.dim() == 2 and out.shape[0] == M and out.shape[1] >= cols and out.stride(1) == 1 and out.dtype == odt
           and out.data_ptr() != x.data_ptr(), f"hybrid_ops.linear: out {tuple(out.shape)} {out.dtype} for {M} x {cols}")
-    a = LinearArgs(x=x.data_ptr(), x2=_ptr(x2), rows=_ptr(rows), norm_w=norm[0].data_ptr() if norm else None, w=w.tiles.data_ptr(),
+    normed = None
+    if norm is not None and lib.vmi_hy_linear_normed(M, N, K, w.groups, DTYPES[T]):
+        normed = torch.empty((M, K), dtype=T, device=x.device)
+    a = LinearArgs(x=x.data_ptr(), x2=_ptr(x2), normed=_ptr(normed), rows=_ptr(rows), norm_w=norm[0].data_ptr() if norm else None, w=w.tiles.data_ptr(),
                    bias=_ptr(bias), gate=_ptr(gate), y=out.data_ptr(), y2=_ptr(glu_out), ldx=x.stride(0), ldy=out.stride(0),
                    ldg=gate.stride(0) if gate is not None else 0, ldy2=glu_out.stride(0) if glu_out is not None else 0, x_gstride=x_gstride, y_gstride=y_gstride, M=M, N=N, K=K,
                    groups=w.groups, norm_n=norm[1] if norm else 0, n_out=float_out[0] if float_out else 0,
