@@ -1770,6 +1770,27 @@ def test_gqa_shared_tile_kernels_match_kernel_model(D):
         assert ran >= 3, (H, hkv, ran)
 
 
+@pytest.mark.parametrize("D,H,hkv", [(128, 32, 8), (64, 16, 2)])
+@pytest.mark.parametrize("B", [33, 64, 65, 96, 256, 257])
+def test_gqa_longest_sequences_first_changes_no_bit(B, D, H, hkv):
+    """The order of the workgroups: one and two a CU and more, up to the most sequences that are ranked and one past; lengths with ties, equal
+    ones and empty ones.  A sequence's row is what it is alone, where nothing is ranked."""
+    from vllmini_amd import ops
+
+    ids = [v for v, n in enumerate(ops.variant_names(), start=1) if n.startswith(f"d{D}_gq4_h1_w") and "_w1_" not in n and "pvm" not in n]
+    assert ids
+    rng = np.random.default_rng(B + D)
+    for lens in (rng.integers(0, 100, B).tolist(), [40] * B, [65 if i == B // 2 else 17 for i in range(B)]):
+        case = make_case(rng, B, H, D, lens, num_kv_heads=hkv, poison_tail=True)
+        for vid in ids:
+            got = run_hip(case, variant=vid, max_seq_len=max(lens))
+            if max(lens) > 65:
+                assert_close(got, run_model(case), f"B{B} variant {vid}", tight=True)
+            for i in {0, B // 2, B - 1, int(np.argmax(lens)), int(np.argmin(lens))}:
+                one = dict(case, **{k: case[k][i:i + 1] for k in ("q", "qbuf", "tables", "lens")})
+                assert np.array_equal(run_hip(one, variant=vid, max_seq_len=max(lens))[0], got[i]), (B, vid, i, lens[i])
+
+
 # ------------------------------------------------------------------------------------------------
 # float32 tensors: the (float, float) dispatch branch (x = 4)
 # ------------------------------------------------------------------------------------------------

@@ -295,6 +295,40 @@ __device__ __forceinline__ bool batch_is_ragged(int maxL, float sum, int B) { re
 // and the balanced kernel back to back, and each leaves at once unless the batch is its kind
 constexpr int QF_GATE_UNIFORM = 1 << 16;  // pa_v1_kernel: leave unless the batch has (nearly) equal lengths
 constexpr int QF_GATE_RAGGED = 1 << 17;   // pa_q_kernel: leave unless the batch is ragged
+// pa_v1_kernel, grouped-query, several waves: workgroups in the order of their sequences' lengths, longest first, of launches with more of them than
+// CUs (a workgroup of a long context holds half a CU's LDS or more for as long as that context lasts: one that comes late is what the launch then waits
+// for).  PAParams::alone != 0: all are on the chip at once, the first `alone` sequences' one a CU and the others' beside them; then the longest
+// stay alone, and of the rest, which go out first, the longest meet the shortest.  32 heads over 8 of 128, contexts U{1 .. longest}: 48 x 4096
+// 106.6 -> 85.6 us, 36 x 3000 68.9 -> 62.5, 60 x 2500 75.7 -> 64.7, 100 x 1500 72.3 -> 66.9, 200 x 800 77.0 -> 74.1; equal lengths leave at once (48 x 4096
+// 166 -> 152, which is TIGHT's).
+constexpr int QF_LONGEST_FIRST = 1 << 18;
+constexpr int LONGEST_FIRST_MAX_SEQS = 256;
+
+// The sequence of rank y when the launch's B (<= LONGEST_FIRST_MAX_SEQS) are sorted by length, longest first, ties in their order.  Every wave finds
+// it by itself, bit by bit, over keys that are distinct: no LDS, no barrier.  R: 64 sequences each
+template <int R>
+__device__ __forceinline__ int seq_of_rank(const int32_t* __restrict__ seq_lens, int B, int y, int lpad, int lane) {
+  int key[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int i = r * 64 + lane, l = seq_lens[i < B ? i : 0];
+    key[r] = i < B ? (l < 0 ? 0 : l > lpad ? lpad : l) * LONGEST_FIRST_MAX_SEQS + LONGEST_FIRST_MAX_SEQS - 1 - i : -1;
+  }
+  const int l0 = __builtin_amdgcn_readfirstlane(key[0]) / LONGEST_FIRST_MAX_SEQS;
+  bool other = false;
+#pragma unroll
+  for (int r = 0; r < R; ++r) other |= key[r] >= 0 && key[r] / LONGEST_FIRST_MAX_SEQS != l0;
+  if (__ballot(other) == 0) return y;
+  int v = 0;   // the largest value that more than y keys reach: the key of rank y
+  for (int bit = 31 - __builtin_clz(lpad * LONGEST_FIRST_MAX_SEQS + LONGEST_FIRST_MAX_SEQS - 1); bit >= 0; --bit) {
+    const int t = v | 1 << bit;
+    int n = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) n += __popcll(__ballot(key[r] >= t));
+    if (n > y) v = t;
+  }
+  return LONGEST_FIRST_MAX_SEQS - 1 - v % LONGEST_FIRST_MAX_SEQS;
+}
 
 // Workgroup barrier for waves that exchange data through LDS only.  __syncthreads() is a release/acquire fence at
 // workgroup scope plus s_barrier, and the fence makes every wave wait for ALL its outstanding global loads
@@ -352,6 +386,7 @@ struct PAParams {
   // balanced kernels (pa_queue.hpp) only: the grid is not (heads, seqs), so the batch size rides here;
   // q_flags = test / experiment knobs, 0 = automatic
   int32_t num_seqs;
+  int32_t alone;      // QF_LONGEST_FIRST: sequences whose workgroups come one a CU (0: not all are on the chip)
   int32_t q_flags;
   // fused append: bit 0 = do NOT store the rows (vmi_paged_attention_v1_newest_*: the attention takes the newest token from
   // key / value, the caller writes the cache itself — e.g. one reshape_and_cache for all the layers of a token)
@@ -387,7 +422,8 @@ struct PAParams {
 //
 // grid = (ceil(H / (HPW*HPT)), num_seqs[, partitions]), block = HPW*WPH*64.
 // LDS  = HPW*HPT * ( lpad*4 (logits) + 2*WPH*4 (max/sum exchange) + WPH*D*4 (partial out)
-//                    + (WPH > 1 ? lpad*2 : 0) (fp16 probabilities; in place over the logits when WPH = 1) ).
+//                    + (WPH > 1 ? lpad*2 : 0) (fp16 probabilities; in place over the logits when WPH = 1) );
+//        GQS with WPH > 1: HPW*HPT * ( max(lpad, WPH*D)*4 + 2*WPH*4 ), see TIGHT.
 // ----------------------------------------------------------------------------------------
 template <int D, int HPW, int WPH, int U, bool NT, bool LOADS_ONLY = false, bool PART = false, int BS = 16,
           bool LOCK = false, bool BF = false, int HPT = 1, bool APP = false, int UMAX = 0, int F8 = 0,
@@ -442,7 +478,14 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = wave / WPH;   // head slot
   const int sub = wave % WPH;  // wave within the slot
-  const int seq = blockIdx.y;
+  int seq = blockIdx.y;
+  if constexpr (GQS && WPH > 1 && !PART) {
+    if (p.q_flags & QF_LONGEST_FIRST) {
+      const int B = gridDim.y, alone = p.alone, beside = B - alone;
+      if (alone) seq = seq < beside ? alone - beside + seq : seq < alone ? seq - beside : B - 1 - (seq - alone);
+      seq = gridDim.y <= 64 ? seq_of_rank<1>(p.seq_lens, gridDim.y, seq, p.lpad, lane) : seq_of_rank<4>(p.seq_lens, gridDim.y, seq, p.lpad, lane);
+    }
+  }
 
   const int head0 = (blockIdx.x * HPW + hl) * HPT;
   // valid heads of this slot (wave-uniform).  With WPH > 1 the host guarantees H % (HPW*HPT) == 0, so every
@@ -484,16 +527,22 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int Lloc = (L < blk_hi * BS ? L : blk_hi * BS) - tok_lo;              // tokens in range (:134-136)
 
   float* smem_f = reinterpret_cast<float*>(smem);
-  float* logits0 = smem_f + (size_t)(hl * HPT) * p.lpad;                                    // + hh*lpad
-  float* red0 = smem_f + (size_t)HPW * HPT * p.lpad + (hl * HPT) * 2 * WPH;                 // + hh*2*WPH
-  float* osm0 = smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH + (size_t)(hl * HPT) * WPH * D;
+  // TIGHT (grouped-query, several waves): the logits' place holds everything, so that two workgroups of long contexts fit a CU.  A wave writes the
+  // probabilities of its own blocks over their logits (a block's 16-bit values in the first half of its place), and the partial outputs
+  // go there when all waves are through
+  constexpr bool TIGHT = GQS && WPH > 1;
+  const int lrow = TIGHT && p.lpad < WPH * D ? WPH * D : p.lpad;                            // a head's share of the logits' place
+  float* logits0 = smem_f + (size_t)(hl * HPT) * lrow;                                      // + hh*lpad
+  float* red0 = smem_f + (size_t)HPW * HPT * lrow + (hl * HPT) * 2 * WPH;                   // + hh*2*WPH
+  float* osm0 = TIGHT ? logits0 : smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH + (size_t)(hl * HPT) * WPH * D;
   // Probabilities as fp16 / bf16 bit patterns, written ONCE per token after the softmax (the V pass used to convert
   // exp * inv_sum again in every lane that met the token: D/8-fold redundant VALU work).  One wave per head: in
   // place over the fp32 values (a value is read before any lane overwrites it — see the normalise loop); WPH waves
   // per head: a region of their own behind the exchange buffers, because another wave may not have read yet.
-  const int ph_stride = WPH == 1 ? 2 * p.lpad : p.lpad;  // uint16 units between the heads of a slot
+  const int ph_stride = WPH == 1 || TIGHT ? 2 * p.lpad : p.lpad;  // uint16 units between the heads of a slot
+  auto ph_at = [](int t) { return TIGHT ? t + t / BS * BS : t; };  // where token t's probability lies
   uint16_t* ph0 =
-      WPH == 1 ? reinterpret_cast<uint16_t*>(logits0)
+      WPH == 1 || TIGHT ? reinterpret_cast<uint16_t*>(logits0)
                : reinterpret_cast<uint16_t*>(smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH +
                                              (size_t)HPW * HPT * WPH * D) + (size_t)(hl * HPT) * p.lpad;
 
@@ -1002,7 +1051,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
             const float e = lg[i];
             // in place (WPH == 1, i == t): the 64 lanes read fp32 values [t0, t0+64) and then write bytes
             // [2*t0, 2*t0+128), i.e. fp32 slots [t0/2, t0/2+32) — already consumed, or being read by this very access
-            ph[i] = i < Lloc ? to_elem<BF>(e * inv_sum[hh]) : (uint16_t)0;
+            ph[ph_at(i)] = i < Lloc ? to_elem<BF>(e * inv_sum[hh]) : (uint16_t)0;
           }
         }
       }
@@ -1031,7 +1080,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   #pragma unroll
             for (int hs = 0; hs < (F8 ? 2 : 1); ++hs)
               pa[hs] = (live && vm_n < HPT)
-                           ? *reinterpret_cast<const u32x4_alias*>(ph0 + vm_n * ph_stride + (tokb + 8 * hs - tok_lo))
+                           ? *reinterpret_cast<const u32x4_alias*>(ph0 + vm_n * ph_stride + ph_at(tokb + 8 * hs - tok_lo))
                            : zero4;
             uint16_t vnew16[VG * NL];
             bool patch = false;
@@ -1104,7 +1153,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   #pragma unroll
           for (int hh = 0; hh < HPT; ++hh) {
             if (valid(hh)) {
-              const uint16_t* php = ph0 + hh * ph_stride + (token0 - tok_lo);
+              const uint16_t* php = ph0 + hh * ph_stride + ph_at(token0 - tok_lo);
               if constexpr (APP && MASK) {  // the appended token lives in the sequence's last block -> final group only
                 if (b == lbA && hf == (offA >> 3) && (!GQS || hh == 0)) {
                   const int e = offA & 7;
@@ -1229,6 +1278,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
     }
   }
 
+  if constexpr (TIGHT) lds_barrier();  // (every wave has read its probabilities)
   if constexpr (FPV) {  // accM: column (lane & 15) = dim 16t + n, rows 4*(lane >> 4) + reg = head
     const int n = lane & 15, g4 = lane >> 4;
 #pragma unroll

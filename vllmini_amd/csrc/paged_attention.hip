@@ -1214,11 +1214,13 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
       return fail(VMI_E_VARIANT, "paged_attention_v1: variant %s would launch %lld workgroups; the split kernels need every "
                   "workgroup resident (at most %d on this device)", v.name, (long long)wgs, split_resident_wgs(head_size, v.HPT));
   }
-  const size_t lds = lds_of(v);
+  size_t lds = lds_of(v);
   if (lds > 160 * 1024)
     return fail(VMI_E_MAX_SEQ_LEN, "paged_attention_v1: max_seq_len=%d needs %zu B of LDS per "
                 "workgroup (variant %s), limit 163840 — paged_attention_v2 has no such limit", max_seq_len, lds,
                 v.name);
+  if (v.GQS && v.WPH > 1 && !v.XW)   // (TIGHT: what the kernel uses; the limit above stays the menu's)
+    lds = (size_t)v.HPW * v.HPT * ((size_t)std::max(lpad, v.WPH * v.D) * 4 + 2 * v.WPH * 4);
 
   DeviceGuard guard(device);
   hipError_t e = guard.err;
@@ -1258,6 +1260,7 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
   fill_sparse(p, bsp);
   p.num_seqs = num_seqs;
   p.q_flags = 0;
+  p.alone = 0;
   p.app_flags = (append && append_no_write) ? 1 : 0;
   g_last_variant = sparse_v ? 0 : variant;
   g_last_partner = 0;
@@ -1341,6 +1344,13 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
   if (partner) {
     p.q_flags |= QF_GATE_UNIFORM;
     g_last_partner = nvariants_v1() - g_stage_nvariants - g_split_nvariants - g_queue_nvariants + (int)(partner - g_queue_variants) + 1;
+  }
+
+  if (v.GQS && v.WPH > 1 && num_seqs <= LONGEST_FIRST_MAX_SEQS) {
+    const int per_seq = num_heads / (v.HPW * v.HPT), wgs = num_seqs * per_seq, cus = device_cus(device);
+    if (wgs > cus) p.q_flags |= QF_LONGEST_FIRST;
+    const int beside = wgs <= 2 * cus ? (wgs - cus + per_seq - 1) / per_seq : 0;
+    if (beside > 0 && 2 * beside <= num_seqs) p.alone = num_seqs - beside;
   }
 
   dim3 block(v.HPW * v.WPH * 64);
@@ -1551,6 +1561,7 @@ int launch_pa_v2(void* out, float* exp_sums, float* max_logits, void* tmp_out, c
   p.value_stride = 0;
   p.num_seqs = num_seqs;
   p.q_flags = 0;
+  p.alone = 0;
   p.app_flags = 0;
   p.kv_scale = kv_scale;
   fill_sparse(p, bsp);
