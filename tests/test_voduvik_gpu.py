@@ -111,14 +111,14 @@ def test_rows_behind_a_norm_stay_in_lds(M, N, K):
     assert ops.linear_resident(M, t) and not ops.linear_resident(33, t)
 
 
-@pytest.mark.parametrize("M,N,K", [(9, 32, 2080), (16, 8192, 2048), (12, 1024, 4064), (17, 16 * 513, 1024), (32, 4128, 2048), (33, 64, 4096), (47, 4128, 1024), (70, 256, 2048)])
+@pytest.mark.parametrize("M,N,K", [(9, 32, 4096), (16, 16384, 4096), (12, 1024, 4128), (17, 4128, 4096), (32, 8192, 4096), (33, 64, 4096), (47, 4128, 4128), (70, 256, 4096)])
 def test_rows_are_normed_once_before_the_product(M, N, K):
     """norm_first: at its borders, and kept to bfloat16 on one group (the same bound: one rounding of the normed rows either way)."""
     from vllmini_amd import hybrid_ops as ops
 
     asks = lambda m, n, k, groups=1, dtype=torch.bfloat16: bool(ops.load().vmi_hy_linear_normed(m, n, k, groups, ops.DTYPES[dtype]))      # noqa: E731
     assert asks(M, N, K) and not asks(M, N, K, 2) and not asks(M, N, K, 1, torch.float32)
-    assert not asks(8, N, K) and not asks(16, 4 * 2048 + 16, 2048) and not asks(32, 24576, 2048) and asks(32, 24576, 4096)
+    assert not asks(8, N, K) and not asks(16, 4 * 4096 + 16, 4096) and not asks(32, 8192, 4064) and asks(32, 24576, 4096)
     _norm_products(M, ops.pad32(N), K)
 
 

@@ -548,14 +548,14 @@ static bool rows_fit(int M, int N, int K) {
 }
 
 // Whether the rows behind a norm are better normed once, by a kernel of their own (3.3 us between two others), than in every workgroup of the product:
-// from 17 rows on, where the workgroups' share of that is 32 rows a column of tiles, except of a vocabulary's columns behind rows that stay in LDS;
-// from 9 on where a row is long and its columns few.  32 rows (in every workgroup -> once): K 1024, N 8192 15.0 -> 11.6 us; K 2048, N 4096 15.3 -> 12.2,
-// N 12288 22.4 -> 20.7, N 50272 52.3 -> 56.7; K 4096, N 4096 25.0 -> 18.3, N 12288 56.3 -> 35.5.  40: K 2048, N 12288 30.0 -> 21.8, K 4096, N 24576
-// 84.4 -> 54.4.  16: K 2048, N 8192 17.4 -> 14.6, N 24576 26.7 -> 27.0; K 4096, N 4096 19.3 -> 16.4; K 1024, N 8192 9.6 -> 10.5.  8: K 4096, N 8192 21.8 -> 21.4.
+// long rows, from 17 of them on, where the workgroups' share of that is 32 rows a column of tiles (except of a vocabulary's columns behind rows that stay
+// in LDS), from 9 on where the columns are few.  K 4096, in every workgroup -> once: 32 rows, N 4096 25.0 -> 18.3 us, N 12288 56.3 -> 35.5; 40, N 24576 84.4 ->
+// 54.4; 16, N 4096 19.3 -> 16.4, N 24576 50.7 -> 46.8; 8, N 8192 21.8 -> 21.4.  Shorter rows gain less than a launch costs a caller who records no graph
+// and waits for his own calls (6 us): 32 rows, K 2048, N 12288 22.4 -> 20.7, K 1024, N 8192 15.0 -> 11.6; a prompt of 35 tokens, width 1024, 1.00 -> 1.06 ms.
 static bool norm_first(int M, int N, int K) {
-  if (K < 1024 || rows_fit(M, N, K)) return false;
+  if (K < 4096 || rows_fit(M, N, K)) return false;
   if (M > 16) return M > 32 || N < 24576 || resident_kind(M, N, K) == 0;
-  return M > 8 && K >= 2048 && N <= 4 * K;
+  return M > 8 && N <= 4 * K;
 }
 
 template <int EPI>

@@ -19,6 +19,7 @@ StepLayout describes the tokens of one step to the latter ones.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 from typing import NamedTuple, Optional, Tuple
@@ -231,9 +232,7 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
         out = torch.empty((M, cols), dtype=odt, device=x.device)
     _need(out.dim() == 2 and out.shape[0] == M and out.shape[1] >= cols and out.stride(1) == 1 and out.dtype == odt
           and out.data_ptr() != x.data_ptr(), f"hybrid_ops.linear: out {tuple(out.shape)} {out.dtype} for {M} x {cols}")
-    normed = None
-    if norm is not None and lib.vmi_hy_linear_normed(M, N, K, w.groups, DTYPES[T]):
-        normed = torch.empty((M, K), dtype=T, device=x.device)
+    normed = torch.empty((M, K), dtype=T, device=x.device) if norm is not None and _normed_first(M, N, K, w.groups, T) else None
     a = LinearArgs(x=x.data_ptr(), x2=_ptr(x2), normed=_ptr(normed), rows=_ptr(rows), norm_w=norm[0].data_ptr() if norm else None, w=w.tiles.data_ptr(),
                    bias=_ptr(bias), gate=_ptr(gate), y=out.data_ptr(), y2=_ptr(glu_out), ldx=x.stride(0), ldy=out.stride(0),
                    ldg=gate.stride(0) if gate is not None else 0, ldy2=glu_out.stride(0) if glu_out is not None else 0, x_gstride=x_gstride, y_gstride=y_gstride, M=M, N=N, K=K,
@@ -244,6 +243,12 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
                    x_kind=kind, epilogue=epi, dtype=DTYPES[T], device=device)
     _check(lib.vmi_hy_linear(ctypes.byref(a), stream))
     return out
+
+
+@functools.lru_cache(maxsize=4096)
+def _normed_first(M: int, N: int, K: int, groups: int, dtype: torch.dtype) -> bool:
+    """Whether a product of these sizes behind a norm is faster over rows normed beforehand."""
+    return bool(load().vmi_hy_linear_normed(M, N, K, groups, DTYPES[dtype]))
 
 
 def linear_resident(M: int, w: MatrixTiles) -> bool:
