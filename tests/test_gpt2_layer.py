@@ -491,6 +491,51 @@ def test_prompt_attention_matches_plain_attention_and_leaves_reshape_and_caches_
         at += n
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,T", [(1, 64, 1200), (3, 64, 1217), (1, 128, 1263), (12, 64, 1249), (12, 64, 2900)])
+def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T):
+    """vmi_gpt2_prompts_f16 from 1200 rows on (tiles_kernel: 64 and 128 columns, rows and chunks left over) against its entries called one by one.
+    Both round in the same five places (normed rows, q / k / v, attention, hidden, stream); a sum in another order may fall on the other side,
+    2^-10 of a value each, and the two products behind one another pass that on."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev, E = torch.device("cuda:0"), H * D
+    g = torch.Generator(device=dev).manual_seed(T + E)
+    rnd = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).half()      # noqa: E731
+    lens = [16] * (T // 16 - 1) + [16 + T % 16]
+    w = {"ln_1": (1 + rnd(E, std=0.2), rnd(E, std=0.2)), "ln_2": (1 + rnd(E, std=0.2), rnd(E, std=0.2)), "ln_f": (1 + rnd(E, std=0.2), rnd(E, std=0.2))}
+    for name, n, k in (("c_attn", 3 * E, E), ("attn_proj", E, E), ("c_fc", 4 * E, E), ("mlp_proj", E, 4 * E)):
+        w[name] = (gl.pack_weight(rnd(n, k, std=k ** -0.5)), rnd(n, std=0.2))
+    wte, wpe = rnd(50, E), rnd(40, E)
+    ids = torch.randint(0, 50, (T,), generator=g, device=dev)
+    pos = torch.cat([torch.arange(n, device=dev) for n in lens])
+    last = (torch.tensor(lens, device=dev).cumsum(0) - 1).int()
+    per = [-(-n // 16) for n in lens]
+    table = torch.full((1, len(lens), max(per)), -1, dtype=torch.int32, device=dev)
+    at = 0
+    for i, n in enumerate(per):
+        table[0, i, :n] = torch.arange(at, at + n, device=dev)
+        at += n
+    kc, vc = rnd(at, H, D // 8, 16, 8), rnd(at, H, D, 16)
+    k2, v2 = kc.clone(), vc.clone()
+    rows = 64
+    tiles = torch.tensor([[i, sum(lens[:i]), a, n] for i, n in enumerate(lens) for a in range(0, n, rows)], dtype=torch.int32, device=dev)
+    flat = []
+    for name in ("ln_1", "c_attn", "attn_proj", "ln_2", "c_fc", "mlp_proj"):
+        flat += [getattr(w[name][0], "tiles", w[name][0]), w[name][1]]
+    got = gl.prompts(flat, (wte, wpe, *w["ln_f"]), ids, pos, last, tiles, rows, table, kc, vc, H, D, 1e-5, D ** -0.5)
+    x = gl.embed(ids, pos, wte, wpe)
+    qkv = gl.linear(x, *w["c_attn"], ln=(*w["ln_1"], 1e-5))
+    a = gl.prompt_attention(qkv, tiles, rows, k2, v2, table[0], H, D ** -0.5)
+    x = gl.linear(a, *w["attn_proj"], residual=x)
+    h = gl.linear(x, *w["c_fc"], gelu=True, ln=(*w["ln_2"], 1e-5))
+    x = gl.linear(h, *w["mlp_proj"], residual=x)
+    want = torch.nn.functional.layer_norm(x[last.long()].float(), (E,), w["ln_f"][0].float(), w["ln_f"][1].float(), 1e-5)
+    assert float((got.float() - want).abs().max()) <= 10 * 2.0 ** -10 * float(want.abs().max())
+    for new, old in ((kc, k2), (vc, v2)):
+        assert float((new.float() - old.float()).abs().max()) <= 4 * 2.0 ** -10 * float(old.abs().max())
+
+
 def test_prompt_tiles_cover_every_position_once():
     from vllmini_amd import gpt2_layer as gl
 

@@ -756,6 +756,31 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
   }
 }
 
+// Whether prompts of T rows take tiles_kernel behind norms of their own: from 1200 rows on the few-row kernels, which norm a row again for
+// every 16 columns, are behind (a layer's four products and its norms, width 768: 1024 rows 58 us there, 58 here; 1500 88 and 75; 2048 108 and 80)
+static bool many_rows(int T, int E) { return T >= 1200 && E % 64 == 0 && 4 * E <= 4608; }
+
+template <int MI, int NI, int PF>
+static int launch_tiles(const LinearParams& p, int epi, hipStream_t stream) {
+  auto go = [&](auto fn) {
+    hipLaunchKernelGGL(fn, dim3((p.M + 32 * MI - 1) / (32 * MI) * (p.N / (32 * NI))), dim3(256), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return (int)VMI_LAYER_OK;
+    set_err("launch: ", hipGetErrorString(e));
+    return (int)VMI_LAYER_E_HIP;
+  };
+  switch (epi) {
+    case VMI_LAYER_EPI_BIAS: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS>);
+    case VMI_LAYER_EPI_BIAS_GELU: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS_GELU>);
+    default: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS_RESIDUAL>);
+  }
+}
+// 64 x 128 where that is a tile for every compute unit, 64 x 64 (more of it in flight) where it is not: 2048 rows, N 768, K 3072 27.4 -> 25.8 us
+static int run_tiles(const LinearParams& p, int epi, hipStream_t stream) {
+  if (p.N % 128 == 0 && (int64_t)((p.M + 63) / 64) * (p.N / 128) >= 256) return launch_tiles<2, 4, 2>(p, epi, stream);
+  return launch_tiles<2, 2, 4>(p, epi, stream);
+}
+
 template <int D, int MI>
 static int launch_prompt(const PromptParams& p, int n_tiles, hipStream_t stream) {
   auto* fn = prompt_attention_kernel<D, MI>;
@@ -961,6 +986,29 @@ int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const v
   return after_launch(who, prev, device);
 }
 
+// packed weights, rows of K and N halves
+static int linear_tiles(const char* who, const void* x, const void* w, const void* bias, const void* res, void* y, int M, int N, int K, int epi,
+                        int device, hipStream_t st) {
+  using namespace vmi_layer;
+  if (!x || !w || !y || (epi == VMI_LAYER_EPI_BIAS_RESIDUAL && !res)) {
+    set_err(who, ": null pointer");
+    return VMI_LAYER_E_ARG;
+  }
+  if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 7)) {
+    set_err(who, ": needs 16-byte aligned rows of x and w, 8-byte aligned rows of y");
+    return VMI_LAYER_E_SHAPE;
+  }
+  LinearParams p{};
+  p.x = static_cast<const h16*>(x), p.ldx = K, p.w = static_cast<const h16*>(w), p.bias = static_cast<const h16*>(bias);
+  p.res = static_cast<const h16*>(res), p.ldr = N, p.y = static_cast<h16*>(y), p.ldy = N;
+  p.M = M, p.N = N, p.K = K, p.w_packed = 1;
+  int prev = -1;
+  if (int rc = with_device(who, device, &prev)) return rc;
+  const int rc = run_tiles(p, epi, st);
+  if (prev != device) (void)hipSetDevice(prev);
+  return rc;
+}
+
 int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream) {
   using namespace vmi_layer;
   static const char* who = "vmi_gpt2_prompts_f16";
@@ -971,9 +1019,19 @@ int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream) {
   }
   const int T = a->num_tokens, E = a->num_heads * a->head_size, dev = a->device;
   int rc = vmi_gpt2_embed_f16(a->input_ids, a->position_ids, a->wte, a->wpe, a->x, T, E, dev, stream);
+  bool many = many_rows(T, E);   // (norms of their own read their weights 16 bytes at a time)
+  for (int l = 0; l < a->num_layers; ++l)
+    for (const void* q : {a->layers[l].ln_1_g, a->layers[l].ln_1_b, a->layers[l].ln_2_g, a->layers[l].ln_2_b}) many = many && q && ((uintptr_t)q & 15) == 0;
   for (int l = 0; l < a->num_layers && rc == VMI_LAYER_OK; ++l) {
     const vmi_gpt2_layer_weights& w = a->layers[l];
     auto linear = [&](const void* x, int K, const void* m, const void* b, const void* g, const void* beta, const void* res, void* y, int N, int epi) {
+      if (many) {   // (`attended` holds the normed rows: the product behind a norm is through with them before the attention, or the layer's end)
+        if (g) {
+          if (int e = vmi_gpt2_add_norm_f16(const_cast<void*>(x), nullptr, nullptr, g, beta, a->eps, a->attended, T, E, dev, stream)) return e;
+          x = a->attended;
+        }
+        return linear_tiles(who, x, m, b, res, y, T, N, K, epi, dev, static_cast<hipStream_t>(stream));
+      }
       return vmi_gpt2_linear_f16(x, K, m, b, g, beta, a->eps, res, N, y, N, T, N, K, epi, 1, dev, stream);
     };
     if ((rc = linear(a->x, E, w.c_attn, w.c_attn_b, w.ln_1_g, w.ln_1_b, nullptr, a->qkv, 3 * E, VMI_LAYER_EPI_BIAS))) break;

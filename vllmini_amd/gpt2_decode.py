@@ -85,10 +85,10 @@ class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
-    # prompts of more tokens in all take the vendor's products: by the GPU's time alone they are ahead from 400 tokens on (a layer's linears
-    # at 384 / 512 / 1024 / 2048 tokens 47 / 49 / 59 / 80 us, the decode step's kernels 46 / 51 / 77 / 132), but their eight launches a layer take
-    # the host 150 us, and that is what a call of so few tokens waits for: 1.95 against 1.09 ms at 1024, 2.08 against 1.80 at 2048
-    NATIVE_PROMPT_MAX_TOKENS = 2048
+    # prompts of more tokens in all take the vendor's products: by the GPU's time alone they are ahead from 400 tokens on (a layer's linears at 512 /
+    # 1024 / 2048 / 4096 tokens 49 / 59 / 80 / 82 us, the native call's 51 / 58 / 80 / 130), but their eight launches a layer take the host 150 us, and that
+    # is what such a call waits for: 1.84 against 1.05 ms at 742 tokens, 1.96 / 1.37 at 1936, 2.18 / 2.06 at 4081, 2.30 / 2.35 at 5212
+    NATIVE_PROMPT_MAX_TOKENS = 4096
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
@@ -317,8 +317,8 @@ class GPT2PagedDecoder:
 
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
         """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
-        takes four launches (the decode step's linear kernels) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by one native call,
-        and seven beyond: the vendor's products, and one kernel for the residual add with the norm behind it."""
+        takes four or six launches (the decode step's linear kernels, or norms and tiles) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by
+        one native call, and seven beyond: the vendor's products, and one kernel for the residual add with the norm behind it."""
         d, pool, dev, sd = self.dims, self.pool, self.device, self.sd
         H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
         if T == 0:
