@@ -13,8 +13,8 @@ for what the operators are actually batched over:
   * around the two ops a decode step runs the block's linear layers on this build's own gfx950 kernels
     (`native_layers`, vllmini_amd/gpt2_layer.py -> csrc/gpt2_layer.hip): LayerNorm + c_attn, c_proj + residual,
     LayerNorm + c_fc + GELU, mlp.c_proj + residual — four launches per layer where the torch modules take eleven
-    (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt,
-    layer_norm, gelu), which prefill, the embeddings and lm_head always use.
+    (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt, layer_norm,
+    gelu), which lm_head always uses, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products.
 
 `reference_off_by_one=True` reproduces the reference caller's seq_lens (length BEFORE the new
 token, scheduler.py:96, so the newest token is not attended); the default attends to it.

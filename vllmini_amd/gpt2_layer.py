@@ -3,7 +3,8 @@
 Counterpart of the torch modules around the reference's call pair — ln_1 -> c_attn, c_proj + residual,
 ln_2 -> c_fc -> GELU -> c_proj + residual (vllmini/model/gpt2.py:14-15, 117-128, 130-135, GPT2Block.forward): one
 hand-written gfx950 kernel family (csrc/gpt2_layer.hip) that runs each linear layer of a decode step — LayerNorm in front,
-bias / GELU / residual add behind — as ONE launch.  `linear()` is the only operation; it has no torch fallback: a missing
+bias / GELU / residual add behind — as ONE launch; and prompts whole: attention that also writes the pages
+(csrc/gpt2_prompt.hpp), norms, and every launch of all layers from one call (`prompts()`).  There is no torch fallback: a missing
 library or an unsupported shape raises.
 """
 from __future__ import annotations
