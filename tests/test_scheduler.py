@@ -175,6 +175,29 @@ def test_a_request_that_can_never_fit_is_rejected_and_the_loop_goes_on():
     assert not sch.pending() and sorted(dec.pool.free_blocks) == list(range(8))
 
 
+def test_gpt2_prompts_past_the_block_table_are_rejected_and_bad_ids_leave_no_blocks_behind(monkeypatch):
+    """GPT2PagedDecoder.prefill_batch asks the pool before it looks at the tokens: a prompt that neither the block table nor the positions hold
+    is the pool's refusal, which the scheduler records; an id that no table holds is refused with every block given back."""
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+
+    dims = GPT2Dims(vocab_size=50, n_positions=128, n_embd=64, n_layer=2, n_head=1)
+    pool = PagedKVPool(24, 1, 64, 16, 10, 2, device="cpu", allocate_tensors=False)
+    dec = GPT2PagedDecoder(dims, random_state_dict(dims, torch.device("cpu")), pool)
+    dec.paged_prefill = dec.prompt_kernel = True      # (as on a HIP device; the launches themselves are stood in for)
+    monkeypatch.setattr(dec, "_whole_prompts", lambda ids, lens, tabs: torch.zeros((len(lens), 50)))
+    sch = BatchScheduler(dec, max_length=40, eos_token_id=EOS, sampler=sample_greedy)
+    big, small = sch.submit([7] * 200), sch.submit([1, 2, 3])
+    sch.step()
+    assert "blocks per layer" in sch.rejected[big] and list(sch.waiting) == [(small, [1, 2, 3])]
+    sch.step()
+    assert small in sch.active and len(pool.free_blocks) == 22
+    pool.free(small)
+    for bad in ([[1, 50]], [[1], [-51]], [[1] * 20, [1] * 140]):
+        with pytest.raises(IndexError):
+            dec.prefill_batch(list(range(100, 100 + len(bad))), bad)
+        assert len(pool.free_blocks) == 24 and not pool.allocated_blocks
+
+
 def test_out_of_blocks_drop_mode_is_the_reference_behaviour():
     # 2 layers, 16-token blocks: each sequence needs 2 blocks at prefill and 2 more at token 17
     dec = FakeDecoder(num_blocks=10, layers=2)

@@ -234,8 +234,6 @@ class GPT2PagedDecoder:
         d, pool, dev = self.dims, self.pool, self.device
         H, D, E = d.n_head, d.head_size, d.n_embd
         whole = self.paged_prefill and self.prompt_kernel
-        if whole:
-            ids_host = self._checked_ids(prompts, lens)
         done = []
         try:
             slots, tabs = [], []
@@ -244,7 +242,9 @@ class GPT2PagedDecoder:
                 slots.append(sl)
                 tabs.append(tb)
                 done.append(sid)
-        except RuntimeError:
+            # (behind the pool: what it refuses is a RuntimeError, which the scheduler turns into a rejected request)
+            ids_host = self._checked_ids(prompts, lens) if whole else None
+        except (RuntimeError, IndexError):
             for sid in done:       # all or nothing: the caller retries with a smaller group
                 pool.free(sid)
             raise
