@@ -185,6 +185,7 @@ def test_gpt2_prompts_past_the_block_table_are_rejected_and_bad_ids_leave_no_blo
     dec = GPT2PagedDecoder(dims, random_state_dict(dims, torch.device("cpu")), pool)
     dec.paged_prefill = dec.prompt_kernel = True      # (as on a HIP device; the launches themselves are stood in for)
     monkeypatch.setattr(dec, "_whole_prompts", lambda ids, lens, tabs: torch.zeros((len(lens), 50)))
+    monkeypatch.setattr(dec, "decode", lambda ids, tokens, **kw: (pool.decode_step_batch(ids), torch.zeros((len(ids), 50)))[1])
     sch = BatchScheduler(dec, max_length=40, eos_token_id=EOS, sampler=sample_greedy)
     big, small = sch.submit([7] * 200), sch.submit([1, 2, 3])
     sch.step()
