@@ -193,7 +193,7 @@ def test_gpt2_prompts_past_the_block_table_are_rejected_and_bad_ids_leave_no_blo
     sch.step()
     assert small in sch.active and len(pool.free_blocks) == 22
     pool.free(small)
-    for bad in ([[1, 50]], [[1], [-51]], [[1] * 20, [1] * 140]):
+    for bad in ([[1, 50]], [[1], [-51]], [[1] * 20, [1] * 140], [[1] * 200]):
         with pytest.raises(IndexError):
             dec.prefill_batch(list(range(100, 100 + len(bad))), bad)
         assert len(pool.free_blocks) == 24 and not pool.allocated_blocks

@@ -81,6 +81,11 @@ def random_state_dict(dims: GPT2Dims, device, dtype=torch.float16, seed: int = 0
     return sd
 
 
+class PromptTooLong(IndexError, RuntimeError):
+    """A prompt of more tokens than the model has positions: no row of the table for the last of them, and where the pool does not hold it either, the
+    pool's refusal, which callers know as a RuntimeError."""
+
+
 class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
@@ -238,7 +243,12 @@ class GPT2PagedDecoder:
         try:
             slots, tabs = [], []
             for sid, T in zip(seq_ids, lens):
-                _, sl, tb = pool.allocate_for_prefill(sid, T)                # slots [layers, T], table [layers, MB]
+                try:
+                    _, sl, tb = pool.allocate_for_prefill(sid, T)            # slots [layers, T], table [layers, MB]
+                except RuntimeError as e:
+                    if whole and T > self.sd["transformer.wpe.weight"].shape[0]:
+                        raise PromptTooLong(str(e)) from e
+                    raise
                 slots.append(sl)
                 tabs.append(tb)
                 done.append(sid)
@@ -312,7 +322,7 @@ class GPT2PagedDecoder:
         if len(ids) and (int(ids.min()) < 0 or int(ids.max()) >= V):
             raise IndexError(f"a token id is out of range (vocabulary of {V})")
         if max(lens) > P:
-            raise IndexError(f"a prompt of {max(lens)} tokens: the model has {P} positions")
+            raise PromptTooLong(f"a prompt of {max(lens)} tokens: the model has {P} positions")
         return ids
 
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
