@@ -536,6 +536,38 @@ def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H
         assert float((new.float() - old.float()).abs().max()) <= 4 * 2.0 ** -10 * float(old.abs().max())
 
 
+def test_what_the_prompt_kernels_read_by_address():
+    from vllmini_amd import gpt2_layer as gl
+
+    flat = torch.zeros(64, dtype=torch.float16)
+    off = -(flat.data_ptr() // 2) % 8
+    ok = flat[off: off + 16]
+    assert gl.takes_weights([ok, flat[off + 8: off + 24]])
+    for bad in (flat[off + 1: off + 17], flat[off + 4: off + 20], flat[off: off + 32: 2], ok.float(), ok.to("meta")):
+        assert not gl.takes_weights([ok, bad])
+
+
+def test_weights_of_other_shapes_or_places_are_not_read_by_address():
+    from vllmini_amd import gpt2_layer as gl
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+    from vllmini_amd.kv_pool import PagedKVPool
+
+    dims = GPT2Dims(vocab_size=50, n_positions=128, n_embd=64, n_layer=2, n_head=1)
+    dec = GPT2PagedDecoder(dims, random_state_dict(dims, torch.device("cpu")), PagedKVPool(24, 1, 64, 16, 10, 2, device="cpu", allocate_tensors=False))
+    dec.native_layers = True
+    assert dec._find_prompt_tensors()
+    weights, ends = dec._prompt_tensors
+    assert [tuple(t.shape) for t in ends] == [(50, 64), (128, 64), (64,), (64,)]
+    assert all(weights[12 + j] is dec.sd["transformer.h.1." + k] for j, k in enumerate(gl.LAYER_WEIGHTS))
+    for key, bad in (("ln_f.bias", torch.zeros(63).half()), ("h.1.attn.c_attn.bias", torch.zeros(64).half()), ("h.0.mlp.c_fc.weight", torch.zeros(64, 256).half()),
+                     ("wte.weight", torch.zeros(50, 72).half()), ("h.1.ln_2.weight", torch.zeros(65).half()[1:]), ("wpe.weight", torch.zeros(128, 64)), ("h.0.ln_1.bias", None)):
+        was = dec.sd["transformer." + key]
+        dec.sd["transformer." + key] = bad
+        assert not dec._find_prompt_tensors(), key
+        dec.sd["transformer." + key] = was
+    assert dec._find_prompt_tensors()
+
+
 def test_prompt_tiles_cover_every_position_once():
     from vllmini_amd import gpt2_layer as gl
 

@@ -267,3 +267,27 @@ def test_prompts_through_the_vendors_products_or_the_decode_kernels_give_the_sam
         assert 50 not in many.pool.allocated_blocks
         same = many.prefill_batch([51, 52], [[7, -1], [7, many.dims.vocab_size - 1]])
         assert torch.equal(same[0], same[1])
+
+
+def test_weights_that_lie_anywhere_take_the_operators_and_give_the_same_logits():
+    """One-dimensional weights as views into one flat buffer, at addresses of two bytes' alignment: the prompts go through paged_attention_v1
+    and torch's modules, as they do for everything the prompt kernels are not built for."""
+    from vllmini_amd.gpt2_decode import GPT2PagedDecoder
+
+    rng = np.random.default_rng(10)
+    prompts = [rng.integers(0, 500, n).tolist() for n in (40, 3)]
+    dims, plain = _model(num_blocks=100)
+    want = plain.prefill_batch([0, 1], prompts)
+    _, other = _model(num_blocks=100)
+    small = [k for k, t in other.sd.items() if t.dim() == 1]
+    flat = torch.empty(1 + sum(other.sd[k].numel() + 1 for k in small), dtype=torch.float16, device=_dev())
+    sd, at = dict(other.sd), 1
+    for k in small:
+        n = sd[k].numel()
+        flat[at: at + n] = sd[k]
+        sd[k] = flat[at: at + n]
+        at += n + 1
+    dec = GPT2PagedDecoder(dims, sd, other.pool)
+    assert plain.prompt_kernel and not dec.prompt_kernel
+    got = dec.prefill_batch([0, 1], prompts)
+    assert float((got.float() - want.float()).abs().max()) <= 2e-2 + 2e-2 * float(want.float().abs().max())

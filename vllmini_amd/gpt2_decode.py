@@ -147,7 +147,7 @@ class GPT2PagedDecoder:
         if not can_scatter:
             self.scatter_in_c_attn = False
         self._packed: Dict[str, gpt2_layer.PackedWeight] = {}
-        self._prompt_tensors = None
+        self._prompt_tensors = None                # what gpt2_layer.prompts reads
         if self.native_layers:
             gpt2_layer.load()
             # the block weights once more as the MFMA tiles the kernels stream (include/vmi_gpt2_layer.h, w_layout 1): weights
@@ -172,11 +172,35 @@ class GPT2PagedDecoder:
         # of 16 tokens, heads of 64 or 128; the operators otherwise, and where the caller wants no native layers
         self.prompt_kernel = self.paged_prefill and native_layers is not False and pool.device.type == "cuda" and wdt == torch.float16 \
             and pool.kv_cache_dtype == "auto" and pool.block_size == gpt2_layer.PROMPT_BLOCK_SIZE \
-            and dims.head_size in gpt2_layer.PROMPT_HEAD_SIZES and E <= gpt2_layer.ADD_NORM_MAX_WIDTH \
-            and all(state_dict[f"transformer.{k}.weight"].is_contiguous() for k in ("wte", "wpe"))
+            and dims.head_size in gpt2_layer.PROMPT_HEAD_SIZES and E <= gpt2_layer.ADD_NORM_MAX_WIDTH
+        if self.prompt_kernel:
+            self.prompt_kernel = self._find_prompt_tensors()
         if self.prompt_kernel:
             gpt2_layer.load()
         self.pad_batch_to = int(pad_batch_to)      # decode steps are laid out for the next multiple of this many rows (0: as they come)
+
+    def _find_prompt_tensors(self) -> bool:
+        """Looks up what gpt2_layer.prompts reads by address; False where a tensor's type, shape or place is not what the kernels take (torch's modules
+        then use it, or say what is wrong with it)."""
+        E, sd, rows = self.dims.n_embd, self.sd, {"c_attn": 3, "c_fc": 4}
+        want = {"wte.weight": (None, E), "wpe.weight": (None, E), "ln_f.weight": (E,), "ln_f.bias": (E,)}
+        for i in range(self.dims.n_layer):
+            for k in gpt2_layer.LAYER_WEIGHTS:
+                n = rows.get(k.split(".")[-2], 1) * E
+                matrix = k.endswith("weight") and "ln_" not in k
+                want[f"h.{i}.{k}"] = (n, 4 * E if k == "mlp.c_proj.weight" else E) if matrix else (n,)
+        for k, shape in want.items():
+            t = sd.get("transformer." + k)
+            if t is None or t.dim() != len(shape) or any(a not in (None, b) for a, b in zip(shape, t.shape)):
+                return False
+        got = {k: sd["transformer." + k] for k in want}
+        # (a layer's matrices are read packed, or by F.linear, which takes any layout)
+        if not gpt2_layer.takes_weights([t for k, t in got.items() if t.dim() == 1 or not k.startswith("h.")]):
+            return False
+        if self.native_layers:
+            flat = [self._packed["transformer." + k].tiles if "transformer." + k in self._packed else t for k, t in got.items()]
+            self._prompt_tensors = flat[4:], flat[:4]
+        return True
 
     # ---- pieces shared by prefill and decode --------------------------------------------------------
     def _ln(self, x, prefix):
@@ -351,7 +375,7 @@ class GPT2PagedDecoder:
         up = {name: up[at[name]: at[name] + a.nbytes].view(kinds[a.dtype]).view(a.shape) for name, a in parts.items()}
 
         if self.native_layers and T <= self.NATIVE_PROMPT_MAX_TOKENS:
-            weights, ends = self._prompt_weights()
+            weights, ends = self._prompt_tensors
             h = gpt2_layer.prompts(weights, ends, up["ids"], up["pos"], up["last"], up["tiles"], tile_rows, up["tables"], pool.key_cache,
                                    pool.value_cache, H, d.head_size, d.layer_norm_epsilon, self.scale)
             return F.linear(h, sd["lm_head.weight"])
@@ -366,17 +390,6 @@ class GPT2PagedDecoder:
         x += add
         h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
         return F.linear(h, sd["lm_head.weight"])
-
-    def _prompt_weights(self):
-        """The tensors that gpt2_layer.prompts reads, looked up and checked once (like the packed matrices among them)."""
-        if self._prompt_tensors is None:
-            sd, names = self.sd, gpt2_layer.LAYER_WEIGHTS
-            keys = [f"transformer.h.{i}.{k}" for i in range(self.dims.n_layer) for k in names]
-            weights = [self._packed[k].tiles if k in self._packed else sd[k] for k in keys]
-            ends = [sd[f"transformer.{k}"] for k in ("wte.weight", "wpe.weight", "ln_f.weight", "ln_f.bias")]
-            gpt2_layer.check_weights([*weights, *ends], weights[0].device)
-            self._prompt_tensors = weights, ends
-        return self._prompt_tensors
 
     def _prefill_variant(self) -> int:
         """The work decomposition of the prefill launch.  Its "sequences" are the positions of a few prompts: thousands of short

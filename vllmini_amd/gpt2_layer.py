@@ -308,18 +308,16 @@ LAYER_WEIGHTS = ("ln_1.weight", "ln_1.bias", "attn.c_attn.weight", "attn.c_attn.
                  "mlp.c_fc.weight", "mlp.c_fc.bias", "mlp.c_proj.weight", "mlp.c_proj.bias")
 
 
-def check_weights(tensors, device: torch.device) -> None:
-    """What prompts() reads by address: half, contiguous, 16-byte aligned, on one device."""
-    for t in tensors:
-        if t.dtype != torch.float16 or not t.is_contiguous() or t.device != device or t.data_ptr() % 16:
-            raise RuntimeError("gpt2_layer.prompts: weights must be contiguous, aligned half tensors on the pool's device")
+def takes_weights(tensors) -> bool:
+    """Whether prompts() and add_norm() can read these by address: half, contiguous, 16-byte aligned, on one device."""
+    return all(t.dtype == torch.float16 and t.is_contiguous() and t.device == tensors[0].device and t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def prompts(weights, ends, input_ids: torch.Tensor, position_ids: torch.Tensor, last_rows: torch.Tensor, tiles: torch.Tensor, tile_rows: int,
             block_tables: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor, num_heads: int, head_size: int, eps: float,
             scale: float) -> torch.Tensor:
     """All layers over whole prompts, issued from one native call: the normed last rows [prompts, E].  weights: the layers' tensors, LAYER_WEIGHTS
-    each, one layer behind the other; ends: wte, wpe, ln_f weight and bias (check_weights() has seen them all); the others as prompt_attention and
+    each, one layer behind the other; ends: wte, wpe, ln_f weight and bias (all such as takes_weights() allows); the others as prompt_attention and
     embed take them, block_tables [layers, prompts, blocks]."""
     T, E, n, dev = input_ids.shape[0], num_heads * head_size, last_rows.shape[0], input_ids.device
     layers = len(weights) // len(LAYER_WEIGHTS)
