@@ -199,6 +199,28 @@ def test_gpt2_prompts_past_the_block_table_are_rejected_and_bad_ids_leave_no_blo
         assert len(pool.free_blocks) == 24 and not pool.allocated_blocks
 
 
+def test_gpt2_prompts_that_fail_leave_no_blocks_behind(monkeypatch):
+    """prefill_batch of whole prompts is all or nothing whatever goes wrong: a library's error, a sequence given twice, no token at all."""
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+
+    dims = GPT2Dims(vocab_size=50, n_positions=128, n_embd=64, n_layer=2, n_head=1)
+    pool = PagedKVPool(24, 1, 64, 16, 10, 2, device="cpu", allocate_tensors=False)
+    dec = GPT2PagedDecoder(dims, random_state_dict(dims, torch.device("cpu")), pool)
+    dec.paged_prefill = dec.prompt_kernel = True
+    for ids, prompts in (([0, 0], [[1], [2]]), ([0], [[]]), ([0, 1], [[], []])):
+        with pytest.raises((ValueError, RuntimeError)):
+            dec.prefill_batch(ids, prompts)
+        assert len(pool.free_blocks) == 24 and not pool.allocated_blocks
+
+    def refuses(*_):
+        raise RuntimeError("launch: out of memory")
+
+    monkeypatch.setattr(dec, "_whole_prompts", refuses)
+    with pytest.raises(RuntimeError, match="out of memory"):
+        dec.prefill_batch([0, 1], [[1, 2], [3]])
+    assert len(pool.free_blocks) == 24 and not pool.allocated_blocks
+
+
 def test_out_of_blocks_drop_mode_is_the_reference_behaviour():
     # 2 layers, 16-token blocks: each sequence needs 2 blocks at prefill and 2 more at token 17
     dec = FakeDecoder(num_blocks=10, layers=2)

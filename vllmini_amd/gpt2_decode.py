@@ -276,14 +276,12 @@ class GPT2PagedDecoder:
                 slots.append(sl)
                 tabs.append(tb)
                 done.append(sid)
-            # (behind the pool: what it refuses is a RuntimeError, which the scheduler turns into a rejected request)
-            ids_host = self._checked_ids(prompts, lens) if whole else None
-        except (RuntimeError, IndexError):
+            if whole:      # (behind the pool: what it refuses is a RuntimeError, which the scheduler turns into a rejected request)
+                return self._whole_prompts(self._checked_ids(prompts, lens), lens, tabs)
+        except Exception:
             for sid in done:       # all or nothing: the caller retries with a smaller group
                 pool.free(sid)
             raise
-        if whole:
-            return self._whole_prompts(ids_host, lens, tabs)
         paged = self.paged_prefill
         slots_dev = torch.from_numpy(np.ascontiguousarray(np.concatenate(slots, axis=1))).to(dev)     # [layers, sum T]
         ids = torch.as_tensor([t for p in prompts for t in p], dtype=torch.long, device=dev)
