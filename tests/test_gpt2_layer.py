@@ -492,6 +492,41 @@ def test_prompt_attention_matches_plain_attention_and_leaves_reshape_and_caches_
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("D,tile_rows,lens,at", [(64, 64, [3, 50, 20], 30), (64, 64, [150], 149), (64, 64, [200], 64), (128, 64, [70], 1), (128, 128, [300], 190)])
+def test_prompt_attention_keeps_values_that_are_not_numbers_from_queries_that_do_not_see_them(D, tile_rows, lens, at, bad):
+    """A value of inf or NaN at one position (of the prompt that holds it) shows in the rows from that position on and in no other: the
+    rows in front of it, which share tiles with it, and the other prompts are what plain attention gives (bound as above)."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev, H, T = torch.device("cuda:0"), 2, sum(lens)
+    E, which = H * D, int(np.argmax(lens))
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    qkv = torch.randn((T, 3 * E), generator=g, device=dev).half()
+    first = sum(lens[:which])
+    qkv[first + at, 2 * E + D + 7] = bad                  # head 1, column 7
+    per = [-(-n // 16) for n in lens]
+    table = torch.full((len(lens), max(per)), -1, dtype=torch.int32, device=dev)
+    for i, n in enumerate(per):
+        table[i, :n] = torch.arange(sum(per[:i]), sum(per[:i]) + n, device=dev)
+    kc, vc = torch.zeros((sum(per), H, D // 8, 16, 8), device=dev).half(), torch.zeros((sum(per), H, D, 16), device=dev).half()
+    tiles = torch.tensor([[i, sum(lens[:i]), a, n] for i, n in enumerate(lens) for a in range(0, n, tile_rows)], dtype=torch.int32, device=dev)
+    out = gl.prompt_attention(qkv, tiles, tile_rows, kc, vc, table, H, D ** -0.5).view(T, H, D).double().cpu()
+    q, k, v = (qkv[:, i * E:(i + 1) * E].view(T, H, D).double().cpu() for i in range(3))
+    hit = torch.zeros(T, H, D, dtype=torch.bool)
+    hit[first + at: first + lens[which], 1, 7] = True
+    assert bool((~torch.isfinite(out))[hit].all()) and bool(torch.isfinite(out)[~hit].all())
+    v[first + at, 1, 7] = 0
+    for i, n in enumerate(lens):
+        a, b, c = (t[sum(lens[:i]): sum(lens[:i]) + n].transpose(0, 1) for t in (q, k, v))
+        w = torch.softmax((a @ b.transpose(1, 2).contiguous()) * D ** -0.5 + torch.full((n, n), float("-inf"), dtype=torch.float64).triu(1), dim=-1)
+        rows = slice(sum(lens[:i]), sum(lens[:i]) + n)
+        want, size = (w @ c).transpose(0, 1), (w @ c.abs()).transpose(0, 1)
+        ok = ((out[rows] - want).abs() <= 2 * 2.0 ** -11 * (size + want.abs())) | hit[rows]
+        assert bool(ok.all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,D,T", [(1, 64, 1200), (3, 64, 1217), (1, 128, 1263), (12, 64, 1249), (12, 64, 2900)])
 def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T):
     """vmi_gpt2_prompts_f16 from 1200 rows on (tiles_kernel: 64 and 128 columns, rows and chunks left over) against its entries called one by one.

@@ -58,6 +58,42 @@ __device__ __forceinline__ float over_kc(float v, F op) {
 constexpr int PKT = 64;      // keys of a tile: four pages of 16
 constexpr int PROMPT_BS = 16;
 
+// One query row by one wave over keys 0 .. q, with nothing but those in any sum: lanes share the keys for the scores and the columns for the values.  k: key
+// 0 of the head, its value E further on; kept for rows whose sums are NaN otherwise
+template <int D>
+__device__ void one_query(const h16* qrow, const h16* k, int64_t ld, int q, float scale2, h16* out, int E, int lane) {
+  auto score = [&](int key) {
+    float s = 0.f;
+    for (int d = 0; d < D; d += 8) {
+      const h16x8 a = *reinterpret_cast<const h16x8*>(qrow + d), b = *reinterpret_cast<const h16x8*>(k + key * ld + d);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s = fmaf((float)a[e], (float)b[e], s);
+    }
+    return s * scale2;
+  };
+  float mx = -1e30f;
+  for (int key = lane; key <= q; key += 64) mx = fmaxf(mx, score(key));
+#pragma unroll
+  for (int i = 1; i < 64; i <<= 1) mx = fmaxf(mx, __shfl_xor(mx, i, 64));
+  float sum = 0.f, o[D / 64];
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) o[i] = 0.f;
+  for (int key0 = 0; key0 <= q; key0 += 64) {
+    const int n = min(64, q + 1 - key0);
+    const float pr = lane < n ? (float)(h16)__builtin_amdgcn_exp2f(score(key0 + lane) - mx) : 0.f;
+    sum += pr;
+    for (int j = 0; j < n; ++j) {
+      const float pj = __shfl(pr, j, 64);
+#pragma unroll
+      for (int i = 0; i < D / 64; ++i) o[i] = fmaf(pj, (float)k[(key0 + j) * ld + E + lane + 64 * i], o[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 1; i < 64; i <<= 1) sum += __shfl_xor(sum, i, 64);
+#pragma unroll
+  for (int i = 0; i < D / 64; ++i) out[lane + 64 * i] = (h16)(o[i] / sum);
+}
+
 template <int D, int MI>
 __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptParams p) {
   constexpr int LD = D + 8, NK = D / 32, NT = D / 16, UPR = D / 8, U = PKT * UPR / 256;
@@ -186,6 +222,18 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) o[mi][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[mi][k], o[mi][nt], 0, 0, 0);
       }
+  }
+  // A key that a query does not see has a probability of 0, which times an infinite or NaN value is NaN in the matrix cores: a wave whose sums hold a NaN
+  // does its rows again, one by one, and leaves out what is masked.  (One add and compare a value, once: 24 prompts of up to 512 tokens as before)
+  float any = 0.f;
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) any += (o[mi][nt][0] + o[mi][nt][1]) + (o[mi][nt][2] + o[mi][nt][3]);
+  if (__ballot(any != any) != 0) {
+    const int last = min(w0 + 16 * MI, len);
+    for (int q = w0; q < last; ++q) one_query<D>(row0 + (int64_t)q * p.ld, row0 + E, p.ld, q, p.scale2, p.out + (int64_t)(tile.y + q) * p.ldo + h * D, E, lane);
+    return;
   }
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
