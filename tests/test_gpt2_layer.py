@@ -658,3 +658,25 @@ def test_few_rows_split_k_over_the_waves(M, N, K):
         got = gl.linear(x, w, b, **kw)
         _close(got, _chain(x, w, b, kw.get("ln"), kw.get("gelu", False), kw.get("residual")), (M, N, K, sorted(kw)))
         assert torch.equal(gl.linear(x, gl.pack_weight(w), b, **kw), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", [(1, 768), (17, 768), (33, 96), (5, 1056), (12, 2048), (200, 768), (700, 768), (640, 1024), (900, 224)])
+def test_the_norm_in_front_holds_rows_whose_mean_is_far_from_zero(M, K):
+    """Rows of mean 300 and deviation 0.5 (a half holds these to 0.25) through both kernels' norms: identity weights, so a result is one normed
+    value.  The sum and the squares are float32 sums of a few dozen terms a lane: the mean is off by at most 8 roundings (2^-24 of 300) and so is
+    the deviation, relatively; the result is rounded once to half (2^-11 of it)."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x = (torch.randn((M, K), generator=g, device=dev) * 0.5 + 300).half()
+    x[0] = (x[0].float() - 600).half()
+    gamma, beta = (1 + 0.2 * torch.randn(K, generator=g, device=dev)).half(), (0.1 * torch.randn(K, generator=g, device=dev)).half()
+    got = gl.linear(x, gl.pack_weight(torch.eye(K, device=dev).half()), torch.zeros(K, device=dev).half(), ln=(gamma, beta, 1e-5)).double()
+    d = x.double()
+    dev_, off = d.std(-1, unbiased=False, keepdim=True), d.mean(-1, keepdim=True).abs()
+    t = (d - d.mean(-1, keepdim=True)) / torch.sqrt(dev_ ** 2 + 1e-5) * gamma.double()
+    want = t + beta.double()
+    bound = 2.0 ** -11 * want.abs() + 8 * 2.0 ** -24 * (off / dev_ * gamma.double().abs() + t.abs()) + 2.0 ** -24
+    assert bool(((got - want).abs() <= 1.01 * bound).all()), float(((got - want).abs() / bound).max())

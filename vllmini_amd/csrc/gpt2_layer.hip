@@ -101,26 +101,35 @@ __device__ __forceinline__ void mma_chunk(f32x4 (&acc)[MT], const u32x4 (&wf)[CH
   }
 }
 
-// two elements of a row through LayerNorm's affine form: t = x * rstd - mean * rstd in fp32 straight from the half (v_fma_mix_f32),
-// y = t * gamma + beta in fp32 written as a half (v_fma_mixlo / mixhi_f16: one rounding, to nearest even) — 2 instructions per
-// element where conversions + fp32 math take 7
-__device__ __forceinline__ uint32_t ln_pair(uint32_t x2, uint32_t g2, uint32_t b2, float rstd, float nmr) {
-  float t0, t1;
+// LayerNorm's pieces, two elements of a row at a time, straight from the half (v_fma_mix_f32, v_dot2_f32_f16): x - mean ...
+__device__ __forceinline__ void ln_centred_pair(uint32_t x2, float neg_mean, float& d0, float& d1) {
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(d0) : "v"(x2), "v"(neg_mean));
+  asm("v_fma_mix_f32 %0, %1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d1) : "v"(x2), "v"(neg_mean));
+}
+// ... the affine form y = t * gamma + beta of t = (x - mean) * rstd in fp32, written as a half (v_fma_mixlo / mixhi_f16: one rounding, to nearest even) ...
+__device__ __forceinline__ uint32_t ln_affine_pair(float t0, float t1, uint32_t g2, uint32_t b2) {
   uint32_t y;
-  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(x2), "v"(rstd), "v"(nmr));
-  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(x2), "v"(rstd), "v"(nmr));
   asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[0,1,1]" : "=v"(y) : "v"(t0), "v"(g2), "v"(b2));
   asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[0,1,1] op_sel_hi:[0,1,1]" : "+v"(y) : "v"(t1), "v"(g2), "v"(b2));
   return y;
 }
-
-// s += x, q += x * x for the two halves of a dword, fp32 sums (v_dot2_f32_f16 would take half the instructions, but its sums
-// came out ~10 % off the fp32 ones on this data — measured, not used)
-__device__ __forceinline__ void ln_stats_pair(uint32_t x2, float& s, float& q) {
-  asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "+v"(s) : "v"(x2));
-  asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(s) : "v"(x2));
-  asm("v_fma_mix_f32 %0, %1, %1, %0 op_sel:[0,0,0] op_sel_hi:[1,1,0]" : "+v"(q) : "v"(x2));
-  asm("v_fma_mix_f32 %0, %1, %1, %0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "+v"(q) : "v"(x2));
+__device__ __forceinline__ uint32_t ln_pair(uint32_t x2, uint32_t g2, uint32_t b2, float rstd, float nmr) {   // (nmr = -mean * rstd)
+  float t0, t1;
+  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(x2), "v"(rstd), "v"(nmr));
+  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(x2), "v"(rstd), "v"(nmr));
+  return ln_affine_pair(t0, t1, g2, b2);
+}
+// ... s += x ...
+__device__ __forceinline__ void ln_sum_pair(uint32_t x2, float& s) {
+  s = __builtin_amdgcn_fdot2(__builtin_bit_cast(h16x2, x2), h16x2{1, 1}, s, false);
+}
+// ... and q += (x - mean)^2: a second pass over registers, because E[x^2] - mean^2 has no variance left in fp32 where a row's mean is a few hundred
+// deviations
+__device__ __forceinline__ void ln_square_pair(uint32_t x2, float neg_mean, float& q) {
+  float d0, d1;
+  ln_centred_pair(x2, neg_mean, d0, d1);
+  q = fmaf(d0, d0, q);
+  q = fmaf(d1, d1, q);
 }
 
 // sum over the LPR consecutive lanes that share a row: inside a row of 16 lanes on the DPP cross-lane paths (quad permutes, then
@@ -279,7 +288,7 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const LinearParams 
     __syncthreads();
   } else {
     // 3. LayerNorm on the values as they sit in registers (a row's K <= XU * LPR * 8, checked on the host): the LPR lanes of a
-    //    row add up the sum and the sum of squares (fp32; var = E[x^2] - mean^2), gamma / beta come back from LDS, and the tile is written ONCE,
+    //    row add up the sum, then the squares around the mean (fp32), gamma / beta come back from LDS, and the tile is written ONCE,
     //    normalised: y = (x - mean) * rstd * gamma + beta rounded to half — torch's layer_norm on half input
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -287,15 +296,20 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const LinearParams 
       if (u < 2 * upr) *reinterpret_cast<u32x4*>(gb + u * 8) = gv[i];
     }
     const float inv_k = 1.f / (float)p.K;
-    float s = 0.f, q = 0.f;   // sum and sum of squares in fp32, each element straight from its half: v_fma_mix_f32
+    float s[4] = {0.f, 0.f, 0.f, 0.f}, q[4] = {0.f, 0.f, 0.f, 0.f};   // (four chains of dependent adds side by side)
 #pragma unroll
     for (int i = 0; i < XU; ++i) {   // (units past the row are zeros)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) ln_stats_pair(xv[i][e], s, q);
+      for (int e = 0; e < 4; ++e) ln_sum_pair(xv[i][e], s[e]);
     }
-    const float mean = group_sum<LPR>(s) * inv_k;
-    const float var = fmaxf(group_sum<LPR>(q) * inv_k - mean * mean, 0.f);
-    const float rstd = rsqrtf(var + p.eps), nmr = -mean * rstd;
+    const float neg_mean = -group_sum<LPR>((s[0] + s[1]) + (s[2] + s[3])) * inv_k;
+#pragma unroll
+    for (int i = 0; i < XU; ++i)
+      if (xj + i * LPR < upr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ln_square_pair(xv[i][e], neg_mean, q[e]);
+      }
+    const float rstd = rsqrtf(group_sum<LPR>((q[0] + q[1]) + (q[2] + q[3])) * inv_k + p.eps), nmr = neg_mean * rstd;
     // 4. the other chunks of the ring
     if (nvalid) {
 #pragma unroll
