@@ -11,7 +11,7 @@
 #                   linear layers; one unit, part of `make` / `all`
 #   make hybrid     libvmi_hybrid.so (include/vmi_hybrid.h): the layers of decoders that mix recurrences, linear and
 #                   softmax attention; part of `make` / `all`
-# (_vmi_host.so, the operators' native call path over torch's C++ interface, needs torch's headers: `python -m vllmini_amd.build`)
+# (The operators run on these; `python -m vllmini_amd.build` adds _vmi_host.<python>.<torch>.so, their native call path, which needs torch's headers)
 HIPCC  ?= hipcc
 ARCH   ?= gfx950
 # -ffp-contract=off: the fp16 p*v products are rounded before the fp16 adds (the reference's rounding points)

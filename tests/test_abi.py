@@ -286,6 +286,35 @@ def test_no_cpu_fallback_ops_raise_on_host_tensors():
         ext.cache_ops.reshape_and_cache(a["q"], a["q"], a["kc"], a["vc"], torch.zeros(2, dtype=torch.int64), "auto", 1.0)
 
 
+def test_the_libraries_alone_are_enough_for_the_operators():
+    """What `make` builds, without the extension module for this interpreter and torch: the libraries load, with a warning, and the operators
+    make their checks in Python."""
+    import sys
+
+    from vllmini_amd import build
+
+    name = os.path.basename(build.HOST_LIB_PATH)
+    assert sys.implementation.cache_tag in name and torch.__version__ in name      # (another pair never loads it)
+    code = """
+import warnings, torch
+from vllmini_amd import _lib, build, ops
+build.HOST_LIB_PATH = build.OUT_DIR + "/_vmi_host.other.so"
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    assert _lib.load().vmi_target_arch() == b"gfx950" and _lib.host() is None and _lib.entries() is None
+assert [w.category for w in seen if "_vmi_host" in str(w.message)] == [RuntimeWarning]
+t = torch.zeros(2, 4, 64).half()
+try:
+    ops.reshape_and_cache(t, t, torch.zeros(8, 4, 8, 16, 8).half(), torch.zeros(8, 4, 64, 16).half(), torch.zeros(2).long(), "auto", 1.0)
+except RuntimeError as e:
+    assert "no CPU path" in str(e)
+else:
+    raise AssertionError
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=REPO)
+    assert r.returncode == 0, r.stderr
+
+
 def test_argument_validation_before_any_launch():
     import paged_attention_cuda as ext
 

@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 
 from . import build as _build
 
@@ -137,18 +138,21 @@ def lib_path() -> str:
 
 _HOST_ENTRIES = ("vmi_paged_attention_v1_f16", "vmi_paged_attention_v1_f16_variant", "vmi_paged_attention_v1_f16_ws", "vmi_paged_attention_v1_fp8",
                  "vmi_paged_attention_v1_fp8_ws", "vmi_reshape_and_cache_f16", "vmi_reshape_and_cache_fp8")
-_host = None         # module _vmi_host (csrc/host_ops.cpp)
+_host = None         # module _vmi_host (csrc/host_ops.cpp); False: this build has none
 
 
 def host():
-    """The native form of the operators' checks and calls.  Part of the build: missing, it raises."""
+    """The native form of the operators' checks and calls, or None where the libraries were built without it (`make`), or for another torch:
+    ops.py then checks and calls by itself, the same C entries, 5 us a call later."""
     global _host
     if _host is None:
         import torch  # noqa: F401  (the module links against its libraries)
 
         path = _build.HOST_LIB_PATH
         if not os.path.exists(path):
-            raise NativeLibraryError(f"{path} not found: build it with `python -m vllmini_amd.build` (or __graft_entry__.build()).")
+            warnings.warn(f"{path} not found (`python -m vllmini_amd.build` makes it): the operators' checks run in Python", RuntimeWarning, stacklevel=2)
+            _host = False
+            return None
         loader = importlib.machinery.ExtensionFileLoader("_vmi_host", path)
         try:
             module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_vmi_host", loader))
@@ -156,11 +160,11 @@ def host():
         except ImportError as e:
             raise NativeLibraryError(f"cannot load {path}: {e}") from e
         _host = module
-    return _host
+    return _host or None
 
 
 def entries():
-    """What _vmi_host's functions take first, for the library the calling context runs on; None while that is not loaded yet."""
+    """What _vmi_host's functions take first, for the library the calling context runs on; None while that is not loaded yet, or without _vmi_host."""
     lib = _active.get()
     if lib is None:
         lib = _product
@@ -192,7 +196,7 @@ def _open(path: str, signatures: dict, want_diag: int, want_extras: int = 0) -> 
     if lib.vmi_has_extras() != want_extras:
         raise NativeLibraryError(f"{path}: vmi_has_extras() = {lib.vmi_has_extras()}, expected {want_extras}")
     lib._vmi_has_extras = bool(want_extras)
-    lib._vmi_entries = host().bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES))
+    lib._vmi_entries = host() and host().bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _HOST_ENTRIES))
     return lib
 
 

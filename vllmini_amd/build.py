@@ -27,8 +27,9 @@ native code at all: hipcc translation units compiled concurrently and linked int
                                                     per-wave timeline there).  Used by tests that force kernel modes,
                                                     scripts/ and scripts/bench_diag.py — never by the operators.
 
-  vllmini_amd/_C/_vmi_host.so                       csrc/host_ops.cpp: what ops.py does per call, for the plain cases, in native
+  vllmini_amd/_C/_vmi_host.<python>.<torch>.so      csrc/host_ops.cpp: what ops.py does per call, for the plain cases, in native
                                                     code over torch's C++ interface (the libraries above know nothing of torch).
+                                                    Without it (`make`) ops.py's own checks and calls stand in for it.
 
 Every object is compiled once and shared by the libraries that hold it (pa_queue.hip twice: its bfloat16 / E5M2 rows are
 behind -DVMI_EXTRAS).  hipcc cross-compiles without a GPU, so this runs in the build container; the .so files are
@@ -36,6 +37,7 @@ git-ignored but travel to the GPU box with the repo snapshot (the objects do not
 """
 from __future__ import annotations
 
+import importlib.metadata
 import os
 import shutil
 import subprocess
@@ -95,7 +97,17 @@ HYBRID_LIB_PATH = os.path.join(OUT_DIR, "libvmi_hybrid.so")
 
 # the operators' checks and calls in native code: an extension module over torch's C++ interface, loaded by _lib.py (no device code)
 SRC_HOST = os.path.join(CSRC, "host_ops.cpp")
-HOST_LIB_PATH = os.path.join(OUT_DIR, "_vmi_host.so")
+
+
+def _torch_version() -> str:
+    try:
+        return importlib.metadata.version("torch")
+    except importlib.metadata.PackageNotFoundError:
+        return "none"
+
+
+# (for THIS interpreter and THIS torch, whose C++ interface it is compiled against: another pair has another name, and so never loads this one)
+HOST_LIB_PATH = os.path.join(OUT_DIR, f"_vmi_host.{sys.implementation.cache_tag}.torch-{_torch_version()}.so")
 
 ARCH = "gfx950"
 # -ffp-contract=off: the fp16 p*v products must be rounded before the fp16 adds (reference
@@ -261,7 +273,7 @@ def host_is_stale() -> bool:
 
 
 def build_host(force: bool = False, verbose: bool = False) -> str:
-    """_vmi_host.so: one C++ unit against the installed torch (~30 s)."""
+    """_vmi_host: one C++ unit against the installed torch (~30 s)."""
     os.makedirs(OUT_DIR, exist_ok=True)
     if not force and os.path.exists(HOST_LIB_PATH) and not _have_objects():
         return HOST_LIB_PATH
@@ -272,15 +284,17 @@ def build_host(force: bool = False, verbose: bool = False) -> str:
 
         root, tmp = os.path.dirname(torch.__file__), HOST_LIB_PATH + ".tmp"
         rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
-        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
-               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include",
-               f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-isystem{root}/include",
+               f"-isystem{root}/include/torch/csrc/api/include", f"-isystem{rocm}/include", f"-isystem{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
                SRC_HOST, "-o", tmp, f"-L{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10_hip", "-lc10"]
         if verbose:
             print(" ".join(cmd), file=sys.stderr)
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"g++ failed ({proc.returncode}): {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+        if proc.stderr:
+            print(proc.stderr, file=sys.stderr)
         os.replace(tmp, HOST_LIB_PATH)
     return HOST_LIB_PATH
 
