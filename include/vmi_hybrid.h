@@ -23,7 +23,7 @@ extern "C" {
 #endif
 
 #define VMI_HY_API __attribute__((visibility("default")))
-#define VMI_HYBRID_ABI_VERSION 2
+#define VMI_HYBRID_ABI_VERSION 3
 
 enum { VMI_HY_OK = 0, VMI_HY_E_ARG = 1, VMI_HY_E_SHAPE = 2, VMI_HY_E_HIP = 3 };
 enum { VMI_HY_BF16 = 0, VMI_HY_F32 = 1 };

@@ -292,6 +292,27 @@ def test_hybrid_library_exports_its_header_and_nothing_else():
     assert lib.vmi_hybrid_abi_version() == hybrid_ops.ABI_VERSION and lib.vmi_hybrid_target_arch() == b"gfx950"
 
 
+def test_the_structs_layouts_belong_to_their_version(tmp_path):
+    """A caller knows a struct by its version number alone: a field that comes or moves takes a new one (3: `normed` in vmi_hy_linear_args).  The sizes as
+    the C header has them, as the ctypes side has them, and as recorded for the version."""
+    from vllmini_amd import hybrid_ops as h
+
+    layouts = {2: {"linear_args": 184, "step": 112, "rglru_args": 136, "latent_prep_args": 88, "latent_attention_args": 80, "state_args": 216, "kv_prep_args": 64,
+                   "attention_args": 128}}
+    layouts[3] = {**layouts[2], "linear_args": 192}
+    src = open(os.path.join(REPO, "include", "vmi_hybrid.h")).read()
+    names = re.findall(r"^} vmi_hy_([a-z_]+);", src, flags=re.M)
+    (tmp_path / "s.c").write_text('#include <stdio.h>\n#include "vmi_hybrid.h"\nint main(void) {\n' + "".join(
+        f'printf("{n} %zu\\n", sizeof(vmi_hy_{n}));\n' for n in names) + "return 0; }\n")
+    subprocess.run(["gcc", "-I", os.path.join(REPO, "include"), str(tmp_path / "s.c"), "-o", str(tmp_path / "s")], check=True)
+    lines = subprocess.run([str(tmp_path / "s")], capture_output=True, text=True, check=True).stdout.split()
+    sizes = dict(zip(lines[::2], map(int, lines[1::2])))
+    assert sizes == layouts[h.ABI_VERSION]
+    py = {"linear_args": h.LinearArgs, "step": h.StepArgs, "rglru_args": h.RglruArgs, "latent_prep_args": h.PrepArgs, "latent_attention_args": h.AttentionArgs,
+          "state_args": h.StateArgs, "kv_prep_args": h.KvPrepArgs, "attention_args": h.GqaArgs}
+    assert {n: ctypes.sizeof(c) for n, c in py.items()} == sizes
+
+
 def test_hybrid_entries_refuse_bad_arguments_without_touching_a_device():
     from vllmini_amd import hybrid_ops as h
 

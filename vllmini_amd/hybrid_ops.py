@@ -28,7 +28,7 @@ import torch
 
 from . import build as _build
 
-ABI_VERSION = 2
+ABI_VERSION = 3
 DTYPES = {torch.bfloat16: 0, torch.float32: 1}
 X_ROWS, X_NORM, X_CONCAT = 0, 1, 2
 E_STORE, E_RESIDUAL, E_FLOAT, E_GLU, E_GATED, E_STORE_GLU = 0, 1, 2, 3, 4, 5
