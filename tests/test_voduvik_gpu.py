@@ -155,6 +155,29 @@ def _norm_products(M, N, K):
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+def test_products_that_are_not_built_are_refused(dtype):
+    """Inputs and epilogues that vmi_hy_linear has no kernel for: an error and nothing written, whether or not there is room for normed rows."""
+    import ctypes
+
+    from vllmini_amd import hybrid_ops as ops
+
+    M, N, K = 12, 64, 4096
+    lib, t = ops.load(), ops.MatrixTiles(torch.ones(N, K, dtype=dtype, device=dev()), dtype)
+    x, xt = torch.ones(M, K, device=dev()), torch.ones(M, K, dtype=dtype, device=dev())
+    nw, y, y2, normed = torch.ones(K, device=dev()), torch.full((M, N), 7.0, device=dev()), torch.full((M, N), 7.0, device=dev()), torch.full_like(xt, 7.0)
+    assert all(b.is_cuda for b in (t.tiles, x, xt, nw, y, y2, normed))
+    built = {0: {0, 1, 4}, 1: {0, 2, 3, 5}, 2: {2}}      # x_kind: epilogues
+    for kind, epi in ((a, b) for a in range(3) for b in range(6) if b not in built[a]):
+        for room in (None, normed):
+            a = ops.LinearArgs(x=(xt if kind == 0 else x).data_ptr(), x2=x.data_ptr(), norm_w=nw.data_ptr(), w=t.tiles.data_ptr(), gate=xt.data_ptr(), y=y.data_ptr(),
+                               y2=y2.data_ptr(), normed=None if room is None else room.data_ptr(), ldx=K, ldy=N, ldg=K, ldy2=N, M=M, N=N, K=K, groups=1, norm_n=K,
+                               n_out=N, n_split=32, eps=1e-5, scale=1.0, x_kind=kind, epilogue=epi, dtype=ops.DTYPES[dtype])
+            assert lib.vmi_hy_linear(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 1, (kind, epi)
+            assert b"not built" in lib.vmi_hybrid_last_error()
+    assert all(bool((b == 7.0).all()) for b in (y, y2, normed))
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("M", [3, 70])
 def test_linear_groups_and_head_gate(dtype, M):
     from vllmini_amd import hybrid_ops as ops

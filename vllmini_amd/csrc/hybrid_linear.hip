@@ -605,14 +605,22 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   return launch_linear<T, 64, 4, 1, XK, EPI>(p, st);
 }
 
+// rows that stand in p.x normed: what follows a norm
+static int linear_normed(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch (p.epilogue) {
+    case VMI_HY_E_STORE: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_STORE>(p, st);
+    case VMI_HY_E_FLOAT: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_FLOAT>(p, st);
+    case VMI_HY_E_GLU: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_GLU>(p, st);
+    case VMI_HY_E_STORE_GLU: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_STORE_GLU>(p, st);
+    default: return fail(VMI_HY_E_ARG, "vmi_hy_linear", "this combination of input and epilogue is not built");
+  }
+}
+
 template <typename T>
 static int linear_kind(const vmi_hy_linear_args& p, hipStream_t st) {
   switch (p.x_kind * 8 + p.epilogue) {
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_STORE: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_STORE>(p, st);
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_RESIDUAL: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_RESIDUAL>(p, st);
-    case VMI_HY_X_ROWS * 8 + VMI_HY_E_FLOAT: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_FLOAT>(p, st);
-    case VMI_HY_X_ROWS * 8 + VMI_HY_E_GLU: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_GLU>(p, st);
-    case VMI_HY_X_ROWS * 8 + VMI_HY_E_STORE_GLU: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_STORE_GLU>(p, st);
     case VMI_HY_X_ROWS * 8 + VMI_HY_E_GATED: return linear_shape<T, VMI_HY_X_ROWS, VMI_HY_E_GATED>(p, st);
     case VMI_HY_X_NORM * 8 + VMI_HY_E_STORE: return linear_shape<T, VMI_HY_X_NORM, VMI_HY_E_STORE>(p, st);
     case VMI_HY_X_NORM * 8 + VMI_HY_E_FLOAT: return linear_shape<T, VMI_HY_X_NORM, VMI_HY_E_FLOAT>(p, st);
@@ -825,12 +833,12 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a->x_kind == VMI_HY_X_NORM && a->normed && a->dtype == VMI_HY_BF16) {
+  if (a->x_kind == VMI_HY_X_NORM && a->normed && a->dtype == VMI_HY_BF16 && a->epilogue != VMI_HY_E_RESIDUAL && a->epilogue != VMI_HY_E_GATED) {
     hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
                        (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
     vmi_hy_linear_args rows = *a;
     rows.x = a->normed, rows.ldx = a->K, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;
-    return linear_kind<b16>(rows, st);
+    return linear_normed(rows, st);
   }
   return a->dtype == VMI_HY_BF16 ? linear_kind<b16>(*a, st) : linear_kind<float>(*a, st);
 }
