@@ -122,6 +122,26 @@ def test_rows_are_normed_once_before_the_product(M, N, K):
     _norm_products(M, ops.pad32(N), K)
 
 
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("M,N,K", [(12, 512, 4096), (12, 512, 512), (3, 64, 9216)])
+def test_columns_behind_the_norm_do_not_count(M, N, K, rms):
+    """The norm is over its first columns, wherever it happens (before the product, in rows_kernel, in linear_kernel): what the rows hold behind them
+    (the weight is zero there) changes no bit, and add_norm leaves them out of its mean too."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M + K)
+    n, x = K - 28, torch.randn(M, K, generator=g, device=dev())
+    t = ops.MatrixTiles((torch.randn(N, K, generator=g, device=dev()) / K ** 0.5).to(torch.bfloat16), torch.bfloat16)
+    nw = torch.zeros(K, device=dev())
+    nw[:n] = 1
+    clean, dirty = x.clone(), x.clone()
+    clean[:, n:], dirty[:, n:] = 0, 1000
+    a, b = (ops.linear(v, t, norm=(nw, n, 1e-5, rms)) for v in (clean, dirty))
+    assert torch.equal(a, b)
+    a, b = (ops.add_norm(v, None, (nw, n, 1e-5, rms), torch.bfloat16) for v in (clean, dirty))
+    assert torch.equal(a[:, :n], b[:, :n])
+
+
 @pytest.mark.parametrize("M,N,K", [(31, 16 * 1542, 1024), (32, 16 * 1536, 2048)])
 def test_many_columns_leave_the_rows_in_lds(M, N, K):
     _norm_products(M, N, K)

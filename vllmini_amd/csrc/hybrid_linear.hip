@@ -665,17 +665,18 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, co
     }
     return a;
   };
+  auto sum = [&](const f32x4& a, int k) {   // (of the n columns that are normed: what lies behind them may be anything)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s += k + e < n ? a[e] : 0.f;
+  };
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
     const int k = (tid + i * 256) * 4;
     v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (k < ld) v[i] = fetch(k);
-    s += v[i][0] + v[i][1] + v[i][2] + v[i][3];   // (padding columns are zeros)
+    sum(v[i], k);
   }
-  for (int k = (tid + MAXV * 256) * 4; k < ld; k += 1024) {
-    const f32x4 a = fetch(k);
-    s += a[0] + a[1] + a[2] + a[3];
-  }
+  for (int k = (tid + MAXV * 256) * 4; k < ld; k += 1024) sum(fetch(k), k);
   if (!out) return;
   float mean = 0.f;
   if (!rms) {
