@@ -53,7 +53,7 @@ typedef struct {
   const void* gate;
   void* y;
   void* y2;
-  void* normed;          /* X_NORM, bfloat16: room for [M][K] of the element type: the rows are normed there first (NULL: on their way into the product) */
+  void* normed;          /* X_NORM, bfloat16: 16-byte aligned room for [M][K] of the element type: the rows are normed there first (NULL: on their way into the product) */
   int64_t ldx, ldy, ldg, ldy2;
   int64_t x_gstride, y_gstride;   /* elements from one group to the next */
   int32_t M, N, K, groups;

@@ -322,6 +322,8 @@ def test_hybrid_entries_refuse_bad_arguments_without_touching_a_device():
     p = (ctypes.addressof(buf) + 15) & ~15
     a = h.LinearArgs(x=p, w=p, y=p, M=1, N=16, K=40, groups=1, ldx=40, ldy=16)
     assert lib.vmi_hy_linear(ctypes.byref(a), None) == 2 and b"K % 32" in lib.vmi_hybrid_last_error()
+    a = h.LinearArgs(x=p, w=p, y=p, norm_w=p, normed=p + 8, M=1, N=16, K=32, groups=1, ldx=32, ldy=16, norm_n=32, x_kind=1)
+    assert lib.vmi_hy_linear(ctypes.byref(a), None) == 2 and b"16-byte aligned" in lib.vmi_hybrid_last_error()
     assert lib.vmi_hy_rglru(ctypes.byref(h.RglruArgs()), ctypes.byref(h.StepArgs()), None) == 1
     assert lib.vmi_hy_latent_attention(ctypes.byref(h.AttentionArgs()), ctypes.byref(h.StepArgs()), None) == 1
     assert lib.vmi_hy_latent_prep(ctypes.byref(h.PrepArgs()), ctypes.byref(h.StepArgs()), None) == 1

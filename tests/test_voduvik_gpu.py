@@ -142,6 +142,31 @@ def test_columns_behind_the_norm_do_not_count(M, N, K, rms):
     assert torch.equal(a[:, :n], b[:, :n])
 
 
+@pytest.mark.parametrize("stride", [0, 4096])
+def test_groups_behind_a_norm_read_the_same_rows_normed_once_or_not(stride):
+    """vmi_hy_linear of two groups behind a norm: x_gstride means nothing there, with room for normed rows or without."""
+    import ctypes
+
+    from vllmini_amd import hybrid_ops as ops
+
+    M, N, K = 12, 64, 4096
+    g = torch.Generator(device=dev()).manual_seed(stride)
+    x, w = torch.randn(M, K, generator=g, device=dev()), torch.randn(2 * N, K, generator=g, device=dev()) / K ** 0.5
+    t = [ops.MatrixTiles(w[i * N:(i + 1) * N].to(torch.bfloat16), torch.bfloat16).tiles.flatten() for i in range(2)]
+    tiles, nw = torch.cat(t), torch.ones(K, device=dev())
+    normed = torch.full((M, K), 7.0, dtype=torch.bfloat16, device=dev())
+    got = []
+    for room in (None, normed.data_ptr()):
+        y = torch.zeros(M, 2 * N, dtype=torch.bfloat16, device=dev())
+        a = ops.LinearArgs(x=x.data_ptr(), norm_w=nw.data_ptr(), w=tiles.data_ptr(), y=y.data_ptr(), normed=room, ldx=K, ldy=2 * N, x_gstride=stride, y_gstride=N, M=M,
+                           N=N, K=K, groups=2, norm_n=K, eps=1e-5, x_kind=1, epilogue=0, dtype=ops.DTYPES[torch.bfloat16])
+        assert ops.load().vmi_hy_linear(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+        got.append(y)
+    h = torch.nn.functional.layer_norm(x.double(), (K,), nw.double(), None, 1e-5) @ w.to(torch.bfloat16).double().T
+    for y in got:
+        close(y, h, torch.bfloat16)
+
+
 @pytest.mark.parametrize("M,N,K", [(31, 16 * 1542, 1024), (32, 16 * 1536, 2048)])
 def test_many_columns_leave_the_rows_in_lds(M, N, K):
     _norm_products(M, N, K)

@@ -827,7 +827,8 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
     return fail(VMI_HY_E_ARG, who, "null pointer, non-positive size or unknown element type");
   if ((a->K & 31) || (a->N & 15) || (a->x_kind == VMI_HY_X_CONCAT && (a->K & 63)) || (a->ldx & 7) || (a->x_gstride & 7) ||
       (a->epilogue != VMI_HY_E_FLOAT && ((a->ldy & 3) || (a->y_gstride & 3))) || ((uintptr_t)a->x & 15) || ((uintptr_t)a->w & 15) ||
-      ((uintptr_t)a->y & 15) || (a->epilogue == VMI_HY_E_FLOAT && (a->n_out <= 0 || a->n_out > a->N || a->groups != 1)) ||
+      ((uintptr_t)a->y & 15) || ((uintptr_t)a->normed & 15) ||
+      (a->epilogue == VMI_HY_E_FLOAT && (a->n_out <= 0 || a->n_out > a->N || a->groups != 1)) ||
       (a->epilogue == VMI_HY_E_STORE_GLU && (a->n_split < 0 || a->n_split > a->N || (a->n_split & 15) || (a->ldy2 & 1) ||
                                              ((uintptr_t)a->y2 & 7) || a->groups != 1)))
     return fail(VMI_HY_E_SHAPE, who, "needs K % 32 == 0, N % 16 == 0 and 16-byte aligned rows");
@@ -838,7 +839,7 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
     hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
                        (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
     vmi_hy_linear_args rows = *a;
-    rows.x = a->normed, rows.ldx = a->K, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;
+    rows.x = a->normed, rows.ldx = a->K, rows.x_gstride = 0, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;   // (all groups read the same rows)
     return linear_normed(rows, st);
   }
   return a->dtype == VMI_HY_BF16 ? linear_kind<b16>(*a, st) : linear_kind<float>(*a, st);
