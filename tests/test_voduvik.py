@@ -335,6 +335,22 @@ def test_hybrid_entries_refuse_bad_arguments_without_touching_a_device():
     assert h.latent_row_tiles(1000, 4, torch.bfloat16) == 1
 
 
+def test_large_products_stay_with_the_library_unless_their_rows_stay_in_lds():
+    """dense(): 17 to 47 tokens and a large matrix go to the library, but for those behind a norm whose kernel keeps the rows in LDS; a product that
+    norms its rows first is not that kernel (17 tokens, 8192 x 4096)."""
+    from types import SimpleNamespace
+
+    from vllmini_amd import hybrid_layers, hybrid_ops as h
+
+    def of(N, K, groups=1, dtype=torch.bfloat16):
+        return SimpleNamespace(N=N, K=K, groups=groups, tiles=torch.empty(0, dtype=dtype))
+
+    assert not hybrid_layers.dense(32, of(22528, 2048), True) and hybrid_layers.dense(32, of(22528, 2048)) and not hybrid_layers.dense(17, of(24576, 4096), True)
+    for M, N, K in ((17, 8192, 4096), (18, 24560, 4096), (19, 24576, 4096)):
+        assert hybrid_layers.dense(M, of(N, K), True), (M, N, K)
+    assert not hybrid_layers.dense(16, of(8192, 4096), True) and h.linear_normed_first(17, of(8192, 4096)) and not h.linear_normed_first(17, of(8192, 4096, 2))
+
+
 def test_command_line_lists_models_and_parses_requests(capsys):
     from vllmini_amd.__main__ import _parser, main
 

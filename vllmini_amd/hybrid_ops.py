@@ -251,8 +251,13 @@ def _normed_first(M: int, N: int, K: int, groups: int, dtype: torch.dtype) -> bo
     return bool(load().vmi_hy_linear_normed(M, N, K, groups, DTYPES[dtype]))
 
 
+def linear_normed_first(M: int, w: MatrixTiles) -> bool:
+    """Whether linear(x, w, norm=...) of M rows norms them by a launch of their own."""
+    return _normed_first(M, w.N, w.K, w.groups, w.tiles.dtype)
+
+
 def linear_resident(M: int, w: MatrixTiles) -> bool:
-    """Whether linear(x, w, norm=...) of M rows keeps x in LDS."""
+    """Whether linear(x, w, norm=...) of M rows keeps x in LDS, unless it norms them first."""
     return w.groups == 1 and bool(load().vmi_hy_linear_resident(M, w.N, w.K, DTYPES[w.tiles.dtype]))
 
 
