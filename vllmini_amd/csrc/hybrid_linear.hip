@@ -666,8 +666,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, co
     return a;
   };
   auto sum = [&](const f32x4& a, int k) {   // (of the n columns that are normed: what lies behind them may be anything)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) s += k + e < n ? a[e] : 0.f;
+    s += (k < n ? a[0] : 0.f) + (k + 1 < n ? a[1] : 0.f) + (k + 2 < n ? a[2] : 0.f) + (k + 3 < n ? a[3] : 0.f);
   };
 #pragma unroll
   for (int i = 0; i < MAXV; ++i) {
