@@ -278,9 +278,9 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear
   }
 }
 
-// Steps of few rows whose x fits a compute unit's LDS (bfloat16, one group).  Such a product is the reading of its weights, so nothing but
+// Steps of few rows behind a norm whose x fits a compute unit's LDS (bfloat16, one group).  Such a product is the reading of its weights, so nothing but
 // that reading may take time:
-//   * a workgroup puts all rows of x into LDS once, normed / concatenated / rounded on the way: every wave has a share of a row and all of
+//   * a workgroup puts all rows of x into LDS once, normed and rounded on the way: every wave has a share of a row and all of
 //     its loads in flight; after that the walk over K has no barrier and no load but the weights';
 //   * then it walks over slabs of 16 columns, blockIdx, blockIdx + grid, ..: its W waves take a W-th of K each and the ring of weight
 //     tiles runs on across slabs; a slab's partial tiles meet in LDS (two places, one barrier a slab) and one wave, another each time,
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear
 // weights.  One row, K 4096: N 24576 57.4 -> 37.1 us (5.4 TB/s), N 8192 25.6 -> 17.1; K 1024: N 6144 10.1 -> 7.7, N 50272 30.6 -> 22.0; 16 rows, K 4096,
 // N 24576 67.6 -> 46.6; 32 rows, K 2048: N 22528 40.4 -> 29.9, N 50272 85.8 -> 51.9.  (Non-temporal loads of the weights: 36.5, but 77 against 74 us
 // for 412 MB and slower wherever they stay in the Infinity Cache.  16 waves a workgroup where there is one slab a compute unit: 9.9 -> 11.3.)
-template <int MT, int W, int PL, int CU, int XK, int EPI>
+template <int MT, int W, int PL, int CU, int EPI>
 __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_linear_args p, const int slabs) {
   constexpr int CS = 4, NB = CU > 1 ? 4 : 6;   // k-steps of a chunk, chunks of weights in registers (NB - 1 of them ahead)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -319,14 +319,14 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
   // x into LDS: wpr waves a row, rpp rows at a time
   const int M = p.M, upr = p.K >> 3;
   const int wpr = M == 1 ? W : M == 2 ? W / 2 : M <= 4 ? W / 4 : M <= 8 ? W / 8 : 1, rpp = W / wpr, sub = wave % wpr, step8 = 64 * wpr;
-  const int u0 = sub * 64 + lane, upl = (upr + step8 - 1) / step8;   // this lane's units of a row of its wave: u0, u0 + step8, ..
+  const int u0 = sub * 64 + lane;   // this lane's units of a row of its wave: u0, u0 + step8, ..
   auto row_at = [&](int round) { return min(round * rpp + wave / wpr, M - 1); };
   const int rounds = (M + rpp - 1) / rpp;
   auto open_ring = [&]() {
 #pragma unroll
     for (int b = 0; b < NB - 1; ++b) load_w(wb[b]);
   };
-  if constexpr (XK == VMI_HY_X_NORM) {
+  {
     constexpr int HOLD = CU > 1 ? 2 : 4;   // units of 8 columns a lane keeps; longer shares are read again
     f32x8 w[HOLD];
     f32x8 v[HOLD];
@@ -380,26 +380,6 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
         if (u0 + i * step8 < upr) put(v[i], w[i], u0 + i * step8);
       for (int u = u0 + HOLD * step8; u < upr; u += step8) put(load8(row + u * 8), load8(p.norm_w + u * 8), u);
       if (round + 1 < rounds) fetch(round + 1);
-    }
-  } else {
-    constexpr int HOLD = 4;
-    XUnit<b16, XK> v[HOLD];
-    int r0 = 0, i0 = 0;   // round and unit of the batch's first
-    for (int at = 0; at < rounds * upl; at += HOLD) {
-      int r = r0, i = i0;
-#pragma unroll
-      for (int h = 0; h < HOLD; ++h) {
-        v[h].load(p, row_at(r), 0, min(u0 + i * step8, upr - 1) * 8);
-        if (++i == upl) i = 0, ++r;
-      }
-      if (at == 0) open_ring();
-      r = r0, i = i0;
-#pragma unroll
-      for (int h = 0; h < HOLD; ++h) {   // (a clamped unit is written again with the same values)
-        *reinterpret_cast<b16x8*>(xs + row_at(r) * LD + min(u0 + i * step8, upr - 1) * 8) = v[h].finish(nullptr, 0, 0.f, 0.f);
-        if (++i == upl) i = 0, ++r;
-      }
-      r0 = r, i0 = i;
     }
   }
   __syncthreads();
@@ -463,9 +443,9 @@ static int resident_kind(int M, int N, int K) {
   return resident_lds(M, K, 8, 1) <= LDS_PER_CU ? 1 : 0;
 }
 
-template <int MT, int W, int PL, int CU, int XK, int EPI>   // CU workgroups a compute unit
+template <int MT, int W, int PL, int CU, int EPI>   // CU workgroups a compute unit
 static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
-  auto* fn = resident_kernel<MT, W, PL, CU, XK, EPI>;
+  auto* fn = resident_kernel<MT, W, PL, CU, EPI>;
   const size_t lds = resident_lds(p.M, p.K, W, PL);
   if (int rc = allow_lds(fn, lds, "vmi_hy_linear")) return rc;
   const int slabs = p.N / 16;
@@ -587,9 +567,9 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
     if (p.groups == 1 && rows_fit(p.M, p.N, p.K)) return launch_rows<EPI>(p, st);
     switch (p.groups == 1 ? resident_kind(p.M, p.N, p.K) : 0) {
-      case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, XK, EPI>(p, st) : launch_resident<2, 8, 2, 2, XK, EPI>(p, st);
-      case 3: return launch_resident<2, 8, 1, 2, XK, EPI>(p, st);
-      case 1: return p.M <= 16 ? launch_resident<1, 8, 1, 1, XK, EPI>(p, st) : launch_resident<2, 8, 1, 1, XK, EPI>(p, st);
+      case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, EPI>(p, st) : launch_resident<2, 8, 2, 2, EPI>(p, st);
+      case 3: return launch_resident<2, 8, 1, 2, EPI>(p, st);
+      case 1: return p.M <= 16 ? launch_resident<1, 8, 1, 1, EPI>(p, st) : launch_resident<2, 8, 1, 1, EPI>(p, st);
       default: break;
     }
   }
@@ -645,7 +625,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ 
   }
 }
 
-// one workgroup per row of x, or of its rows[t]; a row of up to 4 * 4096 columns stays in registers between the three passes
+// one workgroup per row of x, or of its rows[t]; a row of up to 8192 columns stays in registers between the three passes
 template <typename T>
 __global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, const int* rows, const T* add, int64_t ld_add,
                                                        const float* norm_w, T* out, int n, int ld, float eps, int rms) {
