@@ -579,6 +579,16 @@ def test_prompts_take_tiles_from_fewer_rows_the_wider_they_are(H, D, T):
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
 
 
+def test_how_many_tokens_one_native_call_takes_depends_on_the_width():
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+    from vllmini_amd.kv_pool import PagedKVPool
+
+    for E, most in ((64, 8192), (768, 4747), (1152, 2109)):
+        dims = GPT2Dims(vocab_size=8, n_positions=8, n_embd=E, n_layer=1, n_head=E // 64)
+        pool = PagedKVPool(4, dims.n_head, 64, 16, 4, 1, device="cpu", allocate_tensors=False)
+        assert GPT2PagedDecoder(dims, random_state_dict(dims, torch.device("cpu")), pool).NATIVE_PROMPT_MAX_TOKENS == most
+
+
 def test_what_the_prompt_kernels_read_by_address():
     from vllmini_amd import gpt2_layer as gl
 

@@ -90,10 +90,12 @@ class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
-    # prompts of more tokens in all take the vendor's products: by the GPU's time alone they are ahead from 400 tokens on (a layer's linears at 512 /
-    # 1024 / 2048 / 4096 tokens 49 / 59 / 80 / 82 us, the native call's 51 / 58 / 80 / 130), but their eight launches a layer take the host 150 us, and that
-    # is what such a call waits for: 1.84 against 1.05 ms at 742 tokens, 1.96 / 1.37 at 1936, 2.18 / 2.06 at 4081, 2.30 / 2.35 at 5212
-    NATIVE_PROMPT_MAX_TOKENS = 4096
+    # prompts of more tokens in all (times the width's square) take the vendor's products: by the GPU's time alone they are ahead from 400 tokens of width 768
+    # on, but their eight launches a layer take the host 150 us, and that is what such a call waits for.  12 layers of prompts of 128 tokens, native / vendor
+    # in us: width 512 8192 tokens 2065 / 2701; 768 5000 2296 / 2412, 6000 2818 / 2690; 896 2400 1873 / 1967, 4800 2846 / 2703; 1024 1536 1507 / 1942, 3000 2362 / 2218;
+    # 1152 1536 1756 / 1952, 3000 2737 / 2354
+    NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
+    NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
@@ -148,6 +150,7 @@ class GPT2PagedDecoder:
             self.scatter_in_c_attn = False
         self._packed: Dict[str, gpt2_layer.PackedWeight] = {}
         self._prompt_tensors = None                # what gpt2_layer.prompts reads
+        self.NATIVE_PROMPT_MAX_TOKENS = min(self.NATIVE_PROMPT_MAX_TOKENS, self.NATIVE_PROMPT_MAX_WORK // (E * E))
         if self.native_layers:
             gpt2_layer.load()
             # the block weights once more as the MFMA tiles the kernels stream (include/vmi_gpt2_layer.h, w_layout 1): weights
