@@ -64,8 +64,9 @@ typedef struct {
 VMI_HY_API int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream);
 /* Whether a product of these sizes behind a norm is faster over rows normed beforehand (`normed`) */
 VMI_HY_API int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype);
-/* Whether a product of these sizes behind a norm keeps its rows in LDS, given that they are normed on their way into it: then it is ahead of a norm, a
- * library product and what follows it.  Of sizes that vmi_hy_linear_normed names it says nothing. */
+/* Whether the rows of a product of these sizes behind a norm can stay in LDS, normed on their way there: then the product is ahead of a norm, a library
+ * product and what follows it, also at the sizes where another kernel that norms its rows itself is ahead still.  Of sizes that vmi_hy_linear_normed
+ * names it says nothing. */
 VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype);
 
 /* x[t, 0:width) = table[ids[t]] * scale (bfloat16 table of row length ld), zeros up to ld; float32 out */

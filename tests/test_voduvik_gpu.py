@@ -167,6 +167,22 @@ def test_groups_behind_a_norm_read_the_same_rows_normed_once_or_not(stride):
         close(y, h, torch.bfloat16)
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 6144, 3072), (12, 16 * 1026, 4096), (9, 16 * 1540, 4096), (17, 16 * 514, 256), (24, 8192, 1024), (32, 16384, 1536), (20, 16 * 1538, 3072),
+                                   (16, 16 * 1026, 512), (16, 16 * 2046, 544)])
+def test_rows_behind_a_norm_stay_in_lds_and_are_not_normed_first(M, N, K):
+    """resident_kernel where no rule stands in front of it: one workgroup a compute unit with one row tile and with two, and just past the lines at which
+    linear_kernel takes over."""
+    from vllmini_amd import hybrid_ops as ops
+
+    t = _norm_products(M, N, K)
+    assert ops.linear_resident(M, t) and not ops.linear_normed_first(M, t)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 16 * 1024, 512), (9, 16 * 2048, 256), (9, 16 * 3072, 512), (17, 16 * 512, 512), (25, 8192, 1024), (32, 16 * 1024, 992), (17, 16 * 1536, 1280)])
+def test_rows_that_could_stay_in_lds_but_are_few_and_short(M, N, K):
+    _norm_products(M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(31, 16 * 1542, 1024), (32, 16 * 1536, 2048)])
 def test_many_columns_leave_the_rows_in_lds(M, N, K):
     _norm_products(M, N, K)

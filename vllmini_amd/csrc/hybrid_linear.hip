@@ -443,6 +443,18 @@ static int resident_kind(int M, int N, int K) {
   return resident_lds(M, K, 8, 1) <= LDS_PER_CU ? 1 : 0;
 }
 
+// ... and where it does not pay: linear_kernel is as fast or faster on short rows while all of its workgroups are on the chip at once (up to
+// 1024 of 32 columns, 2048 to 3072 of 64; in between and beyond it takes another round).  linear_kernel / resident_kernel in us: 8 rows, K 256, N 12288 7.4 / 6.6, N 32768
+// 7.1 / 8.4; 16 rows, K 256, N 16384 7.9 / 8.4, N 32768 7.5 / 9.8, K 512, N 32768 10.5 / 10.4; 17 rows, K 512, N 8192 8.0 / 9.3, N 12288 13.6 / 9.6, N 24576 11.2 / 11.6; 32 rows, K 256, N 24576 8.2 / 12.8, K 768, N 16384
+// 10.8 / 12.9, K 1024 14.9 / 14.3, K 1280 17.1 / 18.8, K 1536 19.2 / 20.0, K 2048 27.6 / 22.8; N 8192, 17 and 32 rows, K 1024 10.8 / 10.4 and 11.0 / 11.7, K 1536 11.8 / 13.0 and
+// 12.1 / 14.0, K 2048 15.4 / 13.8 and 16.0 / 16.4 (a wave takes its share of K four k-steps at a time: multiples of 1024 leave none unused)
+static bool resident_pays(int M, int N, int K) {
+  const int wgs = (N >> 4) * ((M + 15) >> 4);
+  if ((wgs > 1024 && wgs < 2048) || wgs > 3072) return true;
+  if (M <= 16) return K > 512 || (M <= 8 && wgs <= 1024);
+  return wgs <= 1024 ? K % 1024 == 0 && K <= 2048 && M <= 24 : K == 1024 || K >= 1536;
+}
+
 template <int MT, int W, int PL, int CU, int EPI>   // CU workgroups a compute unit
 static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
   auto* fn = resident_kernel<MT, W, PL, CU, EPI>;
@@ -566,7 +578,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
     if (p.groups == 1 && rows_fit(p.M, p.N, p.K)) return launch_rows<EPI>(p, st);
-    switch (p.groups == 1 ? resident_kind(p.M, p.N, p.K) : 0) {
+    switch (p.groups == 1 && resident_pays(p.M, p.N, p.K) ? resident_kind(p.M, p.N, p.K) : 0) {
       case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, EPI>(p, st) : launch_resident<2, 8, 2, 2, EPI>(p, st);
       case 3: return launch_resident<2, 8, 1, 2, EPI>(p, st);
       case 1: return p.M <= 16 ? launch_resident<1, 8, 1, 1, EPI>(p, st) : launch_resident<2, 8, 1, 1, EPI>(p, st);

@@ -257,7 +257,7 @@ def linear_normed_first(M: int, w: MatrixTiles) -> bool:
 
 
 def linear_resident(M: int, w: MatrixTiles) -> bool:
-    """Whether linear(x, w, norm=...) of M rows keeps x in LDS, unless it norms them first."""
+    """Whether linear(x, w, norm=...) can keep M rows in LDS, unless it norms them first."""
     return w.groups == 1 and bool(load().vmi_hy_linear_resident(M, w.N, w.K, DTYPES[w.tiles.dtype]))
 
 
