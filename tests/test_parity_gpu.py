@@ -1791,6 +1791,27 @@ def test_gqa_longest_sequences_first_changes_no_bit(B, D, H, hkv):
                 assert np.array_equal(run_hip(one, variant=vid, max_seq_len=max(lens))[0], got[i]), (B, vid, i, lens[i])
 
 
+@pytest.mark.parametrize("D,H,hkv", [(128, 32, 8), (64, 16, 2)])
+@pytest.mark.parametrize("B", [33, 64, 65, 129, 256, 257])
+def test_gqa_long_launches_change_no_bit(B, D, H, hkv):
+    """The LONG form's launches (room for 2016 tokens: one or two workgroups a CU; more of them than the menu form's LDS holds) over lengths in many classes
+    and many of one class, empty ones and ones past the room: a sequence's row is what it is alone, where the menu's form runs."""
+    from vllmini_amd import ops
+
+    ids = [v for v, n in enumerate(ops.variant_names(), start=1) if n.startswith(f"d{D}_gq4_h1_w4") and "pvm" not in n]
+    assert ids
+    rng = np.random.default_rng(B * D)
+    spread = rng.integers(0, 300, B)
+    spread[rng.integers(0, B, 3)] = (0, 700, 33)
+    for lens in (spread.tolist(), rng.integers(32, 64, B).tolist(), [40] * B, [2016 if i == B - 1 else i % 70 for i in range(B)]):
+        case = make_case(rng, B, H, D, lens, num_kv_heads=hkv, poison_tail=True)
+        for vid in ids:
+            got = run_hip(case, variant=vid, max_seq_len=2016)
+            for i in {0, 1, B // 2, B - 2, B - 1, *np.argsort(lens, kind="stable")[[0, 1, -2, -1]].tolist()}:
+                one = dict(case, **{k: case[k][i:i + 1] for k in ("q", "qbuf", "tables", "lens")})
+                assert np.array_equal(run_hip(one, variant=vid, max_seq_len=2016)[0], got[i]), (B, vid, i, lens[i])
+
+
 # ------------------------------------------------------------------------------------------------
 # float32 tensors: the (float, float) dispatch branch (x = 4)
 # ------------------------------------------------------------------------------------------------

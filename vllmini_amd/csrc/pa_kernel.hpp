@@ -295,39 +295,60 @@ __device__ __forceinline__ bool batch_is_ragged(int maxL, float sum, int B) { re
 // and the balanced kernel back to back, and each leaves at once unless the batch is its kind
 constexpr int QF_GATE_UNIFORM = 1 << 16;  // pa_v1_kernel: leave unless the batch has (nearly) equal lengths
 constexpr int QF_GATE_RAGGED = 1 << 17;   // pa_q_kernel: leave unless the batch is ragged
-// pa_v1_kernel, grouped-query, several waves: workgroups in the order of their sequences' lengths, longest first, of launches with more of them than
-// CUs (a workgroup of a long context holds half a CU's LDS or more for as long as that context lasts: one that comes late is what the launch then waits
-// for).  PAParams::alone != 0: all are on the chip at once, the first `alone` sequences' one a CU and the others' beside them; then the longest
-// stay alone, and of the rest, which go out first, the longest meet the shortest.  32 heads over 8 of 128, contexts U{1 .. longest}: 48 x 4096
-// 106.6 -> 85.6 us, 36 x 3000 68.9 -> 62.5, 60 x 2500 75.7 -> 64.7, 100 x 1500 72.3 -> 66.9, 200 x 800 77.0 -> 74.1; equal lengths leave at once (48 x 4096
-// 166 -> 152, which is TIGHT's).
+// pa_v1_kernel, LONG: workgroups in the order of their sequences' lengths, longest first (a workgroup of a long context holds half a CU's LDS or more for as
+// long as that context lasts: one that comes late is what the launch then waits for).  PAParams::alone != 0: all are on the chip at once, the first
+// `alone` sequences' one a CU and the others' beside them; then the longest stay alone, and of the rest, which go out first, the longest meet the
+// shortest.  32 heads over 8 of 128, contexts U{1 .. longest}, as the menu's kernel -> LONG: 48 x 4096 106.6 -> 85.0 us, 48 x 2000 59.0 -> 44.8, 33 x 2000 57.4 -> 42.9, 64 x
+// 1000 33.8 -> 29.8.  By classes of lengths and places inside a class, 0.6 us a launch of 64 sequences less than a rank bit by bit over whole lengths.
 constexpr int QF_LONGEST_FIRST = 1 << 18;
 constexpr int LONGEST_FIRST_MAX_SEQS = 256;
 
-// The sequence of rank y when the launch's B (<= LONGEST_FIRST_MAX_SEQS) are sorted by length, longest first, ties in their order.  Every wave finds
-// it by itself, bit by bit, over keys that are distinct: no LDS, no barrier.  R: 64 sequences each
+// The sequence of rank y when the launch's B (<= LONGEST_FIRST_MAX_SEQS) are ordered by length in classes of an equal width (at most 64 of them), longest first, those
+// of a class in their order; len: its length.  Every wave finds it by itself, no LDS, no barrier: the class by its bits, then the lane
+// whose place among its class is the one that is left.  R: 64 sequences each
 template <int R>
-__device__ __forceinline__ int seq_of_rank(const int32_t* __restrict__ seq_lens, int B, int y, int lpad, int lane) {
-  int key[R];
+__device__ __forceinline__ int seq_of_rank(const int32_t* __restrict__ seq_lens, int B, int y, int lpad, int lane, int& len) {
+  int l[R], c[R];
+  const int shift = max(0, 26 - __builtin_clz(lpad));
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = r * 64 + lane, l = seq_lens[i < B ? i : 0];
-    key[r] = i < B ? (l < 0 ? 0 : l > lpad ? lpad : l) * LONGEST_FIRST_MAX_SEQS + LONGEST_FIRST_MAX_SEQS - 1 - i : -1;
-  }
-  const int l0 = __builtin_amdgcn_readfirstlane(key[0]) / LONGEST_FIRST_MAX_SEQS;
+  for (int r = 0; r < R; ++r) l[r] = seq_lens[min(r * 64 + lane, B - 1)];
+#pragma unroll
+  for (int r = 0; r < R; ++r) c[r] = r * 64 + lane < B ? min(max(l[r], 0), lpad) >> shift : -1;
+  auto at = [&](int seq) {
+    len = __builtin_amdgcn_readlane(l[0], seq & 63);
+#pragma unroll
+    for (int r = 1; r < R; ++r)
+      if (seq >> 6 == r) len = __builtin_amdgcn_readlane(l[r], seq & 63);
+    return seq;
+  };
+  const int c0 = __builtin_amdgcn_readfirstlane(c[0]);
   bool other = false;
 #pragma unroll
-  for (int r = 0; r < R; ++r) other |= key[r] >= 0 && key[r] / LONGEST_FIRST_MAX_SEQS != l0;
-  if (__ballot(other) == 0) return y;
-  int v = 0;   // the largest value that more than y keys reach: the key of rank y
-  for (int bit = 31 - __builtin_clz(lpad * LONGEST_FIRST_MAX_SEQS + LONGEST_FIRST_MAX_SEQS - 1); bit >= 0; --bit) {
-    const int t = v | 1 << bit;
+  for (int r = 0; r < R; ++r) other |= c[r] >= 0 && c[r] != c0;
+  if (__ballot(other) == 0) return at(y);
+  int v = 0, before = 0;   // the largest class that more than y sequences reach
+#pragma unroll
+  for (int bit = 32; bit > 0; bit >>= 1) {
     int n = 0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) n += __popcll(__ballot(key[r] >= t));
-    if (n > y) v = t;
+    for (int r = 0; r < R; ++r) n += __popcll(__ballot(c[r] >= (v | bit)));
+    if (n > y) v |= bit;
   }
-  return LONGEST_FIRST_MAX_SEQS - 1 - v % LONGEST_FIRST_MAX_SEQS;
+  uint64_t same[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    before += __popcll(__ballot(c[r] > v));
+    same[r] = __ballot(c[r] == v);
+  }
+  int left = y - before, seq = 0;   // places of its class in front of it
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int mine = __builtin_amdgcn_mbcnt_hi((uint32_t)(same[r] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same[r], 0u));
+    const uint64_t hit = __ballot(c[r] == v && mine == left);
+    if (hit) seq = r * 64 + __ffsll((unsigned long long)hit) - 1;
+    left -= __popcll(same[r]);   // (negative once it is found: no later one matches)
+  }
+  return at(seq);
 }
 
 // Workgroup barrier for waves that exchange data through LDS only.  __syncthreads() is a release/acquire fence at
@@ -423,11 +444,11 @@ struct PAParams {
 // grid = (ceil(H / (HPW*HPT)), num_seqs[, partitions]), block = HPW*WPH*64.
 // LDS  = HPW*HPT * ( lpad*4 (logits) + 2*WPH*4 (max/sum exchange) + WPH*D*4 (partial out)
 //                    + (WPH > 1 ? lpad*2 : 0) (fp16 probabilities; in place over the logits when WPH = 1) );
-//        GQS with WPH > 1: HPW*HPT * ( max(lpad, WPH*D)*4 + 2*WPH*4 ), see TIGHT.
+//        LONG: HPW*HPT * ( max(lpad, WPH*D)*4 + 2*WPH*4 ).
 // ----------------------------------------------------------------------------------------
 template <int D, int HPW, int WPH, int U, bool NT, bool LOADS_ONLY = false, bool PART = false, int BS = 16,
           bool LOCK = false, bool BF = false, int HPT = 1, bool APP = false, int UMAX = 0, int F8 = 0,
-          bool GQS = false, bool FPV = false, bool SPARSE = false>
+          bool GQS = false, bool FPV = false, bool SPARSE = false, bool LONG = false>
 // (second launch bound = minimum waves per SIMD.  The adaptive-depth kernels are the full-chip defaults: 12 waves
 //  per CU = 3 per SIMD that must ALL be resident, i.e. stay under 170 VGPRs — the fused-append form had drifted to 180
 //  and ran 173 us instead of 125.  Not applied elsewhere: on the big-tile kernels it only forces spills.)
@@ -478,12 +499,13 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = wave / WPH;   // head slot
   const int sub = wave % WPH;  // wave within the slot
-  int seq = blockIdx.y;
-  if constexpr (GQS && WPH > 1 && !PART) {
+  int seq = blockIdx.y, ranked_len = -1;
+  if constexpr (LONG) {
     if (p.q_flags & QF_LONGEST_FIRST) {
       const int B = gridDim.y, alone = p.alone, beside = B - alone;
       if (alone) seq = seq < beside ? alone - beside + seq : seq < alone ? seq - beside : B - 1 - (seq - alone);
-      seq = gridDim.y <= 64 ? seq_of_rank<1>(p.seq_lens, gridDim.y, seq, p.lpad, lane) : seq_of_rank<4>(p.seq_lens, gridDim.y, seq, p.lpad, lane);
+      seq = gridDim.y <= 64 ? seq_of_rank<1>(p.seq_lens, gridDim.y, seq, p.lpad, lane, ranked_len)
+                            : seq_of_rank<4>(p.seq_lens, gridDim.y, seq, p.lpad, lane, ranked_len);
     }
   }
 
@@ -505,7 +527,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
 
   // seq_len > max_seq_len overflows the logits buffer in the reference (undefined behaviour,
   // attention_kernels.cu:725-732); here the context is truncated to the LDS that was reserved.
-  int L = p.seq_lens[seq];
+  int L = LONG && (p.q_flags & QF_LONGEST_FIRST) ? ranked_len : p.seq_lens[seq];
   const int Lfull = L;
   // UMAX: 64 sequence lengths sampled evenly across this launch (requested now, used when the queue depth is chosen)
   int samp = 0;
@@ -527,22 +549,23 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int Lloc = (L < blk_hi * BS ? L : blk_hi * BS) - tok_lo;              // tokens in range (:134-136)
 
   float* smem_f = reinterpret_cast<float*>(smem);
-  // TIGHT (grouped-query, several waves): the logits' place holds everything, so that two workgroups of long contexts fit a CU.  A wave writes the
+  // LONG (grouped-query, several waves; which launches: launch_pa_v1): the logits' place holds everything, so that two workgroups of long contexts fit a CU, at
+  // the cost of a barrier and of the ranking (2 - 3 % of a launch that gains nothing by them).  A wave writes the
   // probabilities of its own blocks over their logits (a block's 16-bit values in the first half of its place), and the partial outputs
   // go there when all waves are through
-  constexpr bool TIGHT = GQS && WPH > 1;
-  const int lrow = TIGHT && p.lpad < WPH * D ? WPH * D : p.lpad;                            // a head's share of the logits' place
+  static_assert(!LONG || (GQS && WPH > 1 && !PART), "LONG: grouped-query, several waves, whole sequences");
+  const int lrow = LONG && p.lpad < WPH * D ? WPH * D : p.lpad;                            // a head's share of the logits' place
   float* logits0 = smem_f + (size_t)(hl * HPT) * lrow;                                      // + hh*lpad
   float* red0 = smem_f + (size_t)HPW * HPT * lrow + (hl * HPT) * 2 * WPH;                   // + hh*2*WPH
-  float* osm0 = TIGHT ? logits0 : smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH + (size_t)(hl * HPT) * WPH * D;
+  float* osm0 = LONG ? logits0 : smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH + (size_t)(hl * HPT) * WPH * D;
   // Probabilities as fp16 / bf16 bit patterns, written ONCE per token after the softmax (the V pass used to convert
   // exp * inv_sum again in every lane that met the token: D/8-fold redundant VALU work).  One wave per head: in
   // place over the fp32 values (a value is read before any lane overwrites it — see the normalise loop); WPH waves
   // per head: a region of their own behind the exchange buffers, because another wave may not have read yet.
-  const int ph_stride = WPH == 1 || TIGHT ? 2 * p.lpad : p.lpad;  // uint16 units between the heads of a slot
-  auto ph_at = [](int t) { return TIGHT ? t + t / BS * BS : t; };  // where token t's probability lies
+  const int ph_stride = WPH == 1 || LONG ? 2 * p.lpad : p.lpad;  // uint16 units between the heads of a slot
+  auto ph_at = [](int t) { return LONG ? t + t / BS * BS : t; };  // where token t's probability lies
   uint16_t* ph0 =
-      WPH == 1 || TIGHT ? reinterpret_cast<uint16_t*>(logits0)
+      WPH == 1 || LONG ? reinterpret_cast<uint16_t*>(logits0)
                : reinterpret_cast<uint16_t*>(smem_f + (size_t)HPW * HPT * p.lpad + HPW * HPT * 2 * WPH +
                                              (size_t)HPW * HPT * WPH * D) + (size_t)(hl * HPT) * p.lpad;
 
@@ -1278,7 +1301,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
     }
   }
 
-  if constexpr (TIGHT) lds_barrier();  // (every wave has read its probabilities)
+  if constexpr (LONG) lds_barrier();  // (every wave has read its probabilities)
   if constexpr (FPV) {  // accM: column (lane & 15) = dim 16t + n, rows 4*(lane >> 4) + reg = head
     const int n = lane & 15, g4 = lane >> 4;
 #pragma unroll
@@ -1475,6 +1498,7 @@ struct Variant {
                      //   caller-owned workspace; 0 = not a split kernel.  fn is a pa_split_kernel_t there
   pa_kernel_t fn_rounds;  // split kernels: the same kernel serving more items than are resident in rounds (nullptr: none)
   pa_kernel_t fn_app;     // balanced kernels: the append-read form of the same kernel (pa_queue.hpp APP; nullptr: none)
+  pa_kernel_t fn_long;    // grouped-query kernels of several waves: the same kernel, LONG (half the LDS, longest sequences first); others: nothing of use
 };
 
 typedef void (*pa_reduce_t)(h16*, const float*, const float*, const h16*, const int32_t*, int);
@@ -1498,23 +1522,27 @@ typedef void (*pa_reduce_t)(h16*, const float*, const float*, const h16*, const 
 #define VMI_ROW_F8G(NAME, D, BS, HPW, WPH, U, HPT)  /* fp8 pages, grouped-query sharing, fp16 query */              \
   {NAME, D, BS, HPW, WPH, U, true, HPT, false,                                                                     \
    (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, false, HPT, false, 0, VMI_F8_FMT, true>, 0, \
-   0, 0, VMI_F8_FMT, true},
+   0, 0, VMI_F8_FMT, true, false, false, false, false, false, 0, nullptr, nullptr,                                  \
+   (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, false, HPT, false, 0, VMI_F8_FMT, true, false, false, (WPH > 1)>},
 #define VMI_ROW_F8GP(NAME, D, BS, HPW, WPH, U, HPT)  /* ... and P.V on the matrix cores too (opt-in "_pvm") */      \
   {NAME, D, BS, HPW, WPH, U, true, HPT, false,                                                                           \
    (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, false, HPT, false, 0, VMI_F8_FMT, true, true>, 0, \
-   0, 0, VMI_F8_FMT, true, true},
+   0, 0, VMI_F8_FMT, true, true, false, false, false, false, 0, nullptr, nullptr,                                   \
+   (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, false, HPT, false, 0, VMI_F8_FMT, true, true, false, (WPH > 1)>},
 #define VMI_ROW_F8(NAME, D, BS, HPW, WPH, U, NT, LOCK, HPT, UMAX) \
   VMI_ROW_F8B(NAME, D, BS, HPW, WPH, U, NT, LOCK, HPT, UMAX, false)
 // grouped-query rows: HPT query heads of one KV head per wave, each tile loaded once
 #define VMI_ROW_G(NAME, D, BS, HPW, WPH, U, NT, LOCK, BF, HPT)                                                     \
   {NAME, D, BS, HPW, WPH, U, (bool)(NT), HPT, BF,                                                                  \
    (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, (bool)(NT), false, false, BS, LOCK, BF, HPT, VMI_APP, 0, false, true>, \
-   0, 0, 0, false, true},
+   0, 0, 0, false, true, false, false, false, false, false, 0, nullptr, nullptr,                                    \
+   (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, (bool)(NT), false, false, BS, LOCK, BF, HPT, VMI_APP, 0, false, true, false, false, (WPH > 1)>},
 // ... and with the probabilities x V contraction on the matrix cores as well (opt-in, "_pvm" names)
 #define VMI_ROW_GP(NAME, D, BS, HPW, WPH, U, BF, HPT)                                                              \
   {NAME, D, BS, HPW, WPH, U, true, HPT, BF,                                                                        \
    (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, BF, HPT, VMI_APP, 0, false, true, true>, \
-   0, 0, 0, false, true, true},
+   0, 0, 0, false, true, true, false, false, false, false, 0, nullptr, nullptr,                                     \
+   (pa_kernel_t)pa_v1_kernel<D, HPW, WPH, U, true, false, false, BS, false, BF, HPT, VMI_APP, 0, false, true, true, false, (WPH > 1)>},
 #define VMI_ROW(NAME, D, BS, HPW, WPH, U, NT, LO, LOCK, BF, HPT) \
   VMI_ROW_A(NAME, D, BS, HPW, WPH, U, NT, LO, LOCK, BF, HPT, 0)
 

@@ -1219,8 +1219,21 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
     return fail(VMI_E_MAX_SEQ_LEN, "paged_attention_v1: max_seq_len=%d needs %zu B of LDS per "
                 "workgroup (variant %s), limit 163840 — paged_attention_v2 has no such limit", max_seq_len, lds,
                 v.name);
-  if (v.GQS && v.WPH > 1 && !v.XW)   // (TIGHT: what the kernel uses; the limit above stays the menu's)
-    lds = (size_t)v.HPW * v.HPT * ((size_t)std::max(lpad, v.WPH * v.D) * 4 + 2 * v.WPH * 4);
+  // Grouped queries, several waves: the LONG form (pa_kernel.hpp; the limit above stays the menu's) of launches of more workgroups than CUs, where
+  //   * they are not all on the chip at once by the menu form's LDS: half of it brings more of them there, and what is left over starts with the shortest; or
+  //   * they are one or two a CU, so that it matters which ones share it, and long enough for the 0.6 - 1.4 us of ranking (of looking, where all are equal).
+  // Elsewhere that is what the launch loses: 32 heads over 8 of 128, contexts equal / U{1 .. longest} / the first longest and the others an eighth of it, menu form ->
+  // LONG in us: 48 x 4000 157 -> 145 / 102 -> 81 / 65 -> 67; 48 x 1000 39.5 -> 39.9 / 32.8 -> 27.2 / 24.5 -> 24.1; 48 x 500 24.5 -> 24.8 / 19.8 -> 18.1 / 16.8 -> 16.5;
+  // 48 x 100 11.9 -> 12.4 / 11.6 -> 11.7 / 10.1 -> 10.7; 96 x 500 41.2 -> 41.5 / 31.7 -> 31.7 / 19.7 -> 21.9. 16 over 2 of 64: 256 x 2000 134 -> 83 / 122 -> 70 / 64 -> 67; 200 x 1000 (two
+  // a CU either way) 44.3 -> 46.3 / 40.9 -> 39.9 / 35.9 -> 38.4; 32 over 8 of 64, 48 x 2000 42.4 -> 43.8 / 36.3 -> 32.3 / 29.0 -> 30.0
+  bool go_long = false;
+  if (v.GQS && v.WPH > 1 && !v.XW && !bsp) {
+    const int64_t wgs = (int64_t)num_seqs * (num_heads / (v.HPW * v.HPT)), cus = device_cus(device);
+    go_long = wgs > cus && (wgs > (int64_t)(160 * 1024 / lds) * cus ||
+                            (wgs <= 2 * cus && num_seqs <= LONGEST_FIRST_MAX_SEQS && (int64_t)max_seq_len * v.D * v.D >= 6000000));
+    if (go_long) lds = (size_t)v.HPW * v.HPT * ((size_t)std::max(lpad, v.WPH * v.D) * 4 + 2 * v.WPH * 4);
+  }
+  const pa_kernel_t fn = split_rounds ? v.fn_rounds : go_long ? v.fn_long : v.fn;
 
   DeviceGuard guard(device);
   hipError_t e = guard.err;
@@ -1228,7 +1241,7 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
   if (lds > 48 * 1024) {
     // (set on every such launch: the attribute is per device and the library may be driven from several host threads —
     //  remembering "already granted" in the variant table was a data race; the call costs about a microsecond)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_rounds ? v.fn_rounds : v.fn),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(MaxDynamicSharedMemorySize)");
   }
@@ -1346,9 +1359,9 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
     g_last_partner = nvariants_v1() - g_stage_nvariants - g_split_nvariants - g_queue_nvariants + (int)(partner - g_queue_variants) + 1;
   }
 
-  if (v.GQS && v.WPH > 1 && num_seqs <= LONGEST_FIRST_MAX_SEQS) {
+  if (go_long && num_seqs <= LONGEST_FIRST_MAX_SEQS) {
     const int per_seq = num_heads / (v.HPW * v.HPT), wgs = num_seqs * per_seq, cus = device_cus(device);
-    if (wgs > cus) p.q_flags |= QF_LONGEST_FIRST;
+    p.q_flags |= QF_LONGEST_FIRST;
     const int beside = wgs <= 2 * cus ? (wgs - cus + per_seq - 1) / per_seq : 0;
     if (beside > 0 && 2 * beside <= num_seqs) p.alone = num_seqs - beside;
   }
@@ -1368,7 +1381,7 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
     }
     const int hpg = v.HPW * v.HPT;  // heads per workgroup
     dim3 grid((num_heads + hpg - 1) / hpg, ns, 1);
-    hipLaunchKernelGGL(v.fn, grid, block, lds, static_cast<hipStream_t>(stream), ps);
+    hipLaunchKernelGGL(fn, grid, block, lds, static_cast<hipStream_t>(stream), ps);
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "paged_attention_v1 launch");
   }
