@@ -266,6 +266,8 @@ class GPT2PagedDecoder:
         d, pool, dev = self.dims, self.pool, self.device
         H, D, E = d.n_head, d.head_size, d.n_embd
         whole = self.paged_prefill and self.prompt_kernel
+        if whole:      # (in front of the pool's arrays, which push the token objects out of the cache: 13 000 tokens 110 us)
+            ids_host = np.fromiter(itertools.chain.from_iterable(prompts), dtype=np.int64, count=sum(lens))
         done = []
         try:
             slots, tabs = [], []
@@ -280,7 +282,7 @@ class GPT2PagedDecoder:
                 tabs.append(tb)
                 done.append(sid)
             if whole:      # (behind the pool: what it refuses is a RuntimeError, which the scheduler turns into a rejected request)
-                return self._whole_prompts(self._checked_ids(prompts, lens), lens, tabs)
+                return self._whole_prompts(self._check_tokens(ids_host, lens), lens, tabs)
         except Exception:
             for sid in done:       # all or nothing: the caller retries with a smaller group
                 pool.free(sid)
@@ -338,11 +340,10 @@ class GPT2PagedDecoder:
         last = torch.from_numpy(starts[1:] - 1).to(dev)
         return F.linear(self._ln(x[last], "transformer.ln_f"), self.sd["lm_head.weight"])
 
-    def _checked_ids(self, prompts, lens) -> np.ndarray:
-        """The prompts' tokens in one row, as an index would take them: a negative one counts from the end, others past the tables are
-        refused (no kernel checks them)."""
+    def _check_tokens(self, ids: np.ndarray, lens) -> np.ndarray:
+        """The prompts' tokens as an index would take them: a negative one counts from the end, others past the tables are refused (no kernel checks
+        them)."""
         V, P = self.sd["transformer.wte.weight"].shape[0], self.sd["transformer.wpe.weight"].shape[0]
-        ids = np.fromiter(itertools.chain.from_iterable(prompts), dtype=np.int64, count=sum(lens))
         ids[ids < 0] += V
         if len(ids) and (int(ids.min()) < 0 or int(ids.max()) >= V):
             raise IndexError(f"a token id is out of range (vocabulary of {V})")
