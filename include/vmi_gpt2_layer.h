@@ -102,7 +102,7 @@ VMI_LAYER_API int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t*
 /* All layers of whole prompts, the launches of vmi_gpt2_embed_f16, then per layer vmi_gpt2_linear_f16 (norm, c_attn),
  * vmi_gpt2_prompt_attention_f16, vmi_gpt2_linear_f16 (c_proj, residual), (norm, c_fc, GELU), (c_proj, residual), then vmi_gpt2_add_norm_f16 of
  * the prompts' last rows, issued from one call: a prompt of a few dozen tokens takes the GPU less time than sixty calls take an interpreter.
- * (Of many tokens, T times E from 320 000 on, vmi_gpt2_add_norm_f16 and products of tiles stand for the linears behind norms.)
+ * (Of many tokens, T times E from 390 000 on, vmi_gpt2_add_norm_f16 and products of tiles stand for the linears behind norms.)
  * Everything as those entries take it; block_tables [num_layers][num_prompts][table_ld], layer l's weights in layers[l], matrices in
  * w_layout 1.  x, qkv, attended, hidden: scratch of num_tokens rows of E, 3 E, E and 4 E halves, 16-byte aligned; out: [num_prompts, E]. */
 typedef struct {

@@ -572,10 +572,10 @@ def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,D,T", [(1, 64, 5003), (3, 64, 1667), (1, 128, 2517), (12, 64, 417), (16, 64, 313), (9, 128, 278), (18, 64, 1201)])
+@pytest.mark.parametrize("H,D,T", [(1, 64, 6099), (3, 64, 2035), (1, 128, 3049), (12, 64, 508), (16, 64, 381), (9, 128, 339), (18, 64, 1201)])
 def test_prompts_take_tiles_from_fewer_rows_the_wider_they_are(H, D, T):
-    """As above just past the line between the two, T E = 320 000, at widths from 64 to 1152."""
-    assert 320000 <= T * H * D
+    """As above just past the line between the two, T E = 390 000, at widths from 64 to 1152."""
+    assert 390000 <= T * H * D
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
 
 

@@ -772,8 +772,9 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
 
 // Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
 // are ahead while rows times width are few: 12 layers of prompts of 128 tokens in us, few-row kernels / tiles, width 256 1024 tokens 490 / 546, 1536 635 / 616;
-// 512 512 541 / 606, 640 684 / 635; 768 384 725 / 759, 512 802 / 799, 1024 1145 / 945; 1024 256 821 / 907, 384 1106 / 969, 1000 2157 / 1206; 1152 256 1063 / 1043.
-static bool many_rows(int T, int E) { return (int64_t)T * E >= 320000 && E % 64 == 0 && 4 * E <= 4608; }
+// 512 512 541 / 606, 640 684 / 635; 768 384 725 / 759, 512 802 / 799, 1024 1145 / 945; 1024 256 821 / 907, 384 1106 / 969, 1000 2157 / 1206; 1152 256 1063 / 1043,
+// 384 1251 / 1091.  (At the line itself they are level at 768, and tiles some per cent ahead at other widths.)
+static bool many_rows(int T, int E) { return (int64_t)T * E >= 390000 && E % 64 == 0 && 4 * E <= 4608; }
 
 template <int MI, int NI, int PF>
 static int launch_tiles(const LinearParams& p, int epi, hipStream_t stream) {
