@@ -855,10 +855,11 @@ def serve_measure(args, dev, rank=0, requests=None, note_extra=""):
                     f"(mean {np.mean([len(p) for p in prompts]):.0f}), outputs geometric (mean {np.mean(new):.0f}), prompt + output "
                     f"<= {max_length}; seed 17",
            "note": "BatchScheduler (vllmini_amd/scheduler.py) over GPT2PagedDecoder, random-init GPT-2 small, real prefills (several "
-                   "prompts per call, their causal attention ONE paged_attention_v1 launch per layer) and decode steps through the operators; "
+                   "prompts per call, their causal attention ONE launch per layer: over whole prompts, or paged_attention_v1 over their positions for fp8 "
+                   "pages) and decode steps through the operators; "
                    "host_us_per_step = the scheduler's and pool's Python per decode step (bookkeeping, staging, the graph launch) apart "
                    "from gpu_wait_us_per_step, the time it then waits for the sampled ids, and from admit_s, the admission of queued "
-                   "requests (prefill_s = the prefill calls in it: host-bound torch launches); all of it is inside wall_s" + note_extra}
+                   "requests (prefill_s = the prefill calls in it); all of it is inside wall_s" + note_extra}
     del sch, warm, dec, pool
     torch.cuda.empty_cache()
     return rec
