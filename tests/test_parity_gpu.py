@@ -1812,6 +1812,51 @@ def test_gqa_long_launches_change_no_bit(B, D, H, hkv):
                 assert np.array_equal(run_hip(one, variant=vid, max_seq_len=2016)[0], got[i]), (B, vid, i, lens[i])
 
 
+@pytest.mark.parametrize("pages", ["auto", "fp8"])
+def test_gqa_long_launches_over_byte_pages_and_with_the_fused_append(pages):
+    """The LONG form of the kernels over fp8 pages and of the fused append: a sequence's row is what it is alone, and the append leaves the bytes and
+    the rows of reshape_and_cache + paged_attention_v1."""
+    from vllmini_amd import cache_ops, ops
+
+    dev, B, H, G, D = torch.device("cuda:0"), 65, 32, 8, 128
+    g = torch.Generator(device=dev).manual_seed(7)
+    lens = torch.randint(1, 300, (B,), generator=g, device=dev).to(torch.int32)
+    lens[3], lens[64] = 700, 1
+    per, tables, at = ((lens + 15) // 16).tolist(), torch.full((B, 44), -1, dtype=torch.int32), 0
+    order = torch.randperm(sum(per), generator=torch.Generator().manual_seed(3)).to(torch.int32)
+    for i, n in enumerate(per):
+        tables[i, :n] = order[at: at + n]
+        at += n
+    tables, NB = tables.to(dev), at
+    qkv = torch.randn((B, (H + 2 * G) * D), generator=g, device=dev).half()
+    q, k, v = qkv[:, : H * D].view(B, H, D), qkv[:, H * D: (H + G) * D].view(B, G, D), qkv[:, (H + G) * D:].view(B, G, D)
+    if pages == "fp8":
+        kc, vc = (torch.randint(0, 64, s, generator=g, device=dev, dtype=torch.uint8) for s in ((NB, G, D // 16, 16, 16), (NB, G, D, 16)))
+        prefix, refs = f"fp8_d{D}_bs16_gq", 0
+    else:
+        kc, vc = (torch.randn(s, generator=g, device=dev).half() for s in ((NB, G, D // 8, 16, 8), (NB, G, D, 16)))
+        prefix, refs = f"d{D}_gq", 0
+    slots = (tables[torch.arange(B, device=dev), (lens.long() - 1) // 16].long() * 16 + (lens.long() - 1) % 16)
+    for vid, name in enumerate(ops.variant_names(), start=1):
+        if not name.startswith(prefix) or "_h1_w" not in name or "_h1_w1_" in name or "gq7" in name or "gq3" in name or "gq8" in name:
+            continue
+        a, b = kc.clone(), vc.clone()
+        cache_ops.reshape_and_cache(k, v, a, b, slots, pages, 1.0)
+        run = lambda i: ops.paged_attention_v1(out[i], q[i], a, b, G, D ** -0.5, tables[i], lens[i], 16, 2016, None, pages, 1.0, _variant=vid)      # noqa: E731
+        out = torch.empty((B, H, D), dtype=torch.float16, device=dev)
+        run(slice(0, B))
+        rows = out.clone()
+        for i in range(B):
+            run(slice(i, i + 1))
+        assert torch.equal(out, rows), name
+        if pages == "auto":
+            a2, b2, fused = kc.clone(), vc.clone(), torch.empty_like(out)
+            ops.paged_attention_v1_append(fused, q, k, v, a2, b2, G, D ** -0.5, tables, lens, 16, 2016, _variant=vid)
+            assert torch.equal(fused.view(torch.int16), rows.view(torch.int16)) and torch.equal(a2, a) and torch.equal(b2, b), name
+        refs += 1
+    assert refs >= (2 if pages == "fp8" else 4)
+
+
 # ------------------------------------------------------------------------------------------------
 # float32 tensors: the (float, float) dispatch branch (x = 4)
 # ------------------------------------------------------------------------------------------------
