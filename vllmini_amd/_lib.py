@@ -143,7 +143,7 @@ _host = None         # module _vmi_host (csrc/host_ops.cpp); False: this build h
 
 def host():
     """The native form of the operators' checks and calls, or None where the libraries were built without it (`make`), or for another torch:
-    ops.py then checks and calls by itself, the same C entries, 5 us a call later."""
+    ops.py then checks and calls by itself, the same C entries, 5 us later for the two calls of a step."""
     global _host
     if _host is None:
         import torch  # noqa: F401  (the module links against its libraries)
