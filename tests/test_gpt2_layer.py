@@ -679,6 +679,14 @@ def test_few_rows_split_k_over_the_waves(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 2320, 768), (70, 2320, 768), (90, 2320, 768), (123, 2320, 768), (40, 3088, 1152), (50, 2064, 2048), (200, 784, 768), (20, 48, 4608),
+                                   (9, 256, 1504)])
+def test_few_rows_of_several_slabs_a_workgroup(M, N, K):
+    """norm_rows_kernel with 2, 3, 4 and 6 slabs a workgroup and rows_kernel with two, the last workgroup's not all there; K that its waves do not divide evenly."""
+    test_few_rows_split_k_over_the_waves(M, N, K)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,K", [(1, 768), (17, 768), (33, 96), (5, 1056), (12, 2048), (200, 768), (700, 768), (640, 1024), (900, 224)])
 def test_the_norm_in_front_holds_rows_whose_mean_is_far_from_zero(M, K):
     """Rows of mean 300 and deviation 0.5 (a half holds these to 0.25) through both kernels' norms: identity weights, so a result is one normed

@@ -727,47 +727,94 @@ static int launch(const LinearParams& p, const Shape& s, hipStream_t stream) {
   return VMI_LAYER_OK;
 }
 
-// Whether a linear layer goes to rows_kernel: where its workgroups, one for 16 columns of 16 rows, are at most two a compute unit.  Beyond, every
-// further row tile reads the weights again behind the others (K 768 behind a norm, 37 rows: N 2304, 432 of them, 6.3 -> 5.6 us; N 3072, 576,
-// 6.7 -> 7.1), and linear_kernel's row tiles in LDS are ahead; with a long K sooner (K 3072, 96 rows, 288: 12.4 -> 9.7; 128, 384: 8.9 -> 9.7).
-static bool rows_pick(int M, int N, int K, bool ln, int epi) {
-  const int j = rows_steps(K);
-  if (!j || (K & 31) || (N & 15) || (int64_t)(N >> 4) * ((M + 15) >> 4) > (K < 1536 ? 512 : 383)) return false;
-  return ln ? j <= 8 && epi != VMI_LAYER_EPI_BIAS_RESIDUAL : epi == VMI_LAYER_EPI_BIAS_RESIDUAL;
+// Slabs of 16 columns a workgroup of few rows takes: as few as leave one workgroup a compute unit (256), at most `most`
+static int rows_slabs(int M, int N, int most) {
+  const int rb = (M + 15) >> 4;
+  for (int ns : {1, 2, 3, 4, 6})
+    if (ns >= most || (int64_t)(((N >> 4) + ns - 1) / ns) * rb <= 256) return ns < most ? ns : most;
+  return most;
+}
+static int rows_most(int K, bool ln) {   // (the weights of NS slabs wait in registers)
+  const int per = ((K >> 5) + 7) / 8;
+  if (!ln) return (K >> 5) <= 96 ? 2 : 1;
+  return per <= 4 ? 6 : per <= 6 ? 4 : 3;
 }
 
-template <int J>
-static int launch_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream) {
-  const dim3 grid(((p.N >> 4) + 7) / 8 * 8 * ((p.M + 15) >> 4)), block(64 * RK);
-  auto go = [&](auto fn) {
-    hipLaunchKernelGGL(fn, grid, block, 0, stream, p);
-    const hipError_t e = hipGetLastError();
-    if (e == hipSuccess) return (int)VMI_LAYER_OK;
-    set_err("launch: ", hipGetErrorString(e));
-    return (int)VMI_LAYER_E_HIP;
-  };
-  if (!ln) return go(rows_kernel<J, false, VMI_LAYER_EPI_BIAS_RESIDUAL>);
-  if constexpr (J <= 8) {
-    switch (epi) {
-      case VMI_LAYER_EPI_BIAS: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS>);
-      case VMI_LAYER_EPI_BIAS_GELU: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS_GELU>);
-      default: return go(rows_kernel<J, true, VMI_LAYER_EPI_BIAS_KV_CACHE>);
+// Whether a linear layer goes to the kernels of gpt2_rows.hpp.  Behind a norm, while its workgroups are on the chip at once: up to 768 columns four a
+// compute unit, beyond one.  linear_kernel / these, us: K 768, N 3072 192 rows (384 workgroups) 9.3 / 7.4, 320 (640) 9.6 / 9.8, 384 (768) 14.1 / 9.9, 512 (1024) 14.3 / 12.1;
+// K 512, N 2048 512 rows (704) 8.1 / 7.7; K 1024, N 4096 64 rows (172) 7.9 / 5.7, 96 (258) 9.0 / 10.6, 160 (430) 14.3 / 10.8, 256 (688) 16.1 / 15.4; K 1152, N 3456
+// 64 rows (216) 9.3 / 6.3, 128 (432) 9.8 / 10.8.  Without one their reading of x is what grows: K 768, N 768 512 rows (768) 4.8 / 4.7, K 1152, N 1152 256 rows
+// (576) 6.6 / 6.3, 320 (720) 6.7 / 7.5, K 4096, N 1024 128 rows (512) 11.4 / 10.1, 160 (640) 11.4 / 13.5, K 4608, N 1152 128 rows (576) 14.2 / 13.7
+static bool rows_pick(int M, int N, int K, bool ln, int epi) {
+  if ((K & 31) || (N & 15) || K > (ln ? MAX_K_LN : MAX_K) || ln == (epi == VMI_LAYER_EPI_BIAS_RESIDUAL)) return false;
+  const int ns = rows_slabs(M, N, rows_most(K, ln));
+  return (int64_t)(((N >> 4) + ns - 1) / ns) * ((M + 15) >> 4) <= (K <= 768 ? 1024 : ln ? 256 : 576);
+}
+
+static int launch_rows(void (*fn)(LinearParams), const LinearParams& p, int ns, int threads, size_t lds, hipStream_t stream) {
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) {
+      set_err("hipFuncSetAttribute: ", hipGetErrorString(e));
+      return VMI_LAYER_E_HIP;
     }
   }
-  return VMI_LAYER_E_SHAPE;   // (rows_pick asks for none of these)
+  // (a multiple of 8 column blocks: the row tiles of one then go to one XCD, which reads their weights once)
+  const int nb = ((p.N >> 4) + ns - 1) / ns;
+  hipLaunchKernelGGL(fn, dim3((nb + 7) / 8 * 8, (p.M + 15) >> 4), dim3(threads), lds, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return VMI_LAYER_OK;
+  set_err("launch: ", hipGetErrorString(e));
+  return VMI_LAYER_E_HIP;
+}
+
+template <int J, int EPI>
+static int launch_norm_rows(const LinearParams& p, int ns, hipStream_t stream) {
+  auto go = [&](auto fn) { return launch_rows(fn, p, ns, 64 * NORM_RW, norm_rows_lds(p.K, ns), stream); };
+  if (ns == 1) return go(norm_rows_kernel<J, 1, EPI>);
+  if (ns == 2) return go(norm_rows_kernel<J, 2, EPI>);
+  if (ns == 3) return go(norm_rows_kernel<J, 3, EPI>);
+  if constexpr (J <= 6)
+    if (ns == 4) return go(norm_rows_kernel<J, 4, EPI>);
+  if constexpr (J <= 4)
+    if (ns == 6) return go(norm_rows_kernel<J, 6, EPI>);
+  return VMI_LAYER_E_SHAPE;   // (rows_slabs asks for no other)
+}
+
+template <int RW, int J>
+static int launch_plain_rows(const LinearParams& p, int ns, hipStream_t stream) {
+  if (ns == 1) return launch_rows(rows_kernel<RW, J, 1>, p, 1, 64 * RW, (size_t)RW * rows_stride(J, 1), stream);
+  if constexpr (J <= 6)
+    if (ns == 2) return launch_rows(rows_kernel<RW, J, 2>, p, 2, 64 * RW, (size_t)RW * rows_stride(J, 2), stream);
+  return VMI_LAYER_E_SHAPE;
+}
+
+template <int EPI>
+static int run_norm_rows(const LinearParams& p, int ns, hipStream_t stream) {
+  const int per = ((p.K >> 5) + NORM_RW - 1) / NORM_RW;
+  if (per <= 1) return launch_norm_rows<1, EPI>(p, ns, stream);
+  if (per <= 2) return launch_norm_rows<2, EPI>(p, ns, stream);
+  if (per <= 3) return launch_norm_rows<3, EPI>(p, ns, stream);
+  if (per <= 4) return launch_norm_rows<4, EPI>(p, ns, stream);
+  return per <= 6 ? launch_norm_rows<6, EPI>(p, ns, stream) : launch_norm_rows<8, EPI>(p, ns, stream);
 }
 
 static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream) {
-  switch (rows_steps(p.K)) {
-    case 1: return launch_rows<1>(p, ln, epi, stream);
-    case 2: return launch_rows<2>(p, ln, epi, stream);
-    case 3: return launch_rows<3>(p, ln, epi, stream);
-    case 4: return launch_rows<4>(p, ln, epi, stream);
-    case 6: return launch_rows<6>(p, ln, epi, stream);
-    case 8: return launch_rows<8>(p, ln, epi, stream);
-    case 12: return launch_rows<12>(p, ln, epi, stream);
-    default: return launch_rows<16>(p, ln, epi, stream);
+  const int ns = rows_slabs(p.M, p.N, rows_most(p.K, ln)), nks = p.K >> 5;
+  if (ln) {
+    switch (epi) {
+      case VMI_LAYER_EPI_BIAS: return run_norm_rows<VMI_LAYER_EPI_BIAS>(p, ns, stream);
+      case VMI_LAYER_EPI_BIAS_GELU: return run_norm_rows<VMI_LAYER_EPI_BIAS_GELU>(p, ns, stream);
+      default: return run_norm_rows<VMI_LAYER_EPI_BIAS_KV_CACHE>(p, ns, stream);
+    }
   }
+  if (nks <= 8) return launch_plain_rows<4, 2>(p, ns, stream);
+  if (nks <= 16) return launch_plain_rows<4, 4>(p, ns, stream);
+  if (nks <= 24) return launch_plain_rows<4, 6>(p, ns, stream);
+  if (nks <= 32) return launch_plain_rows<8, 4>(p, ns, stream);
+  if (nks <= 48) return launch_plain_rows<8, 6>(p, ns, stream);
+  if (nks <= 64) return launch_plain_rows<16, 4>(p, ns, stream);
+  return nks <= 96 ? launch_plain_rows<16, 6>(p, ns, stream) : launch_plain_rows<16, 9>(p, ns, stream);
 }
 
 // Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
