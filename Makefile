@@ -36,14 +36,14 @@ DEPS   := $(wildcard $(CSRC)/*.hpp) $(wildcard $(CSRC)/*.inc) include/vmi_paged_
 LAYER_LIB := $(OUTDIR)/libvmi_gpt2_layer.so
 
 HYBRID_LIB := $(OUTDIR)/libvmi_hybrid.so
-HYBRID_UNITS := hybrid_linear hybrid_rglru hybrid_latent hybrid_state hybrid_attention
+HYBRID_UNITS := hybrid_linear hybrid_rows hybrid_rglru hybrid_latent hybrid_state hybrid_attention
 HYBRID_SRCS := $(HYBRID_UNITS:%=$(CSRC)/%.hip)
 
 all: $(LIB) $(LAYER_LIB) $(HYBRID_LIB) oracle
 
 hybrid: $(HYBRID_LIB)
 
-$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_softmax.hpp include/vmi_hybrid.h
+$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_linear.hpp $(CSRC)/hybrid_softmax.hpp include/vmi_hybrid.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $(HYBRID_SRCS) -o $@
 

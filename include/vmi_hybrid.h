@@ -68,6 +68,9 @@ VMI_HY_API int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t
  * product and what follows it, also at the sizes where another kernel that norms its rows itself is ahead still.  Of sizes that vmi_hy_linear_normed
  * names it says nothing. */
 VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype);
+/* Whether a product of these sizes behind a norm (one that vmi_hy_linear_normed names) keeps its normed rows in registers: then it is ahead of a norm, a
+ * library product and what follows it as well. */
+VMI_HY_API int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype);
 
 /* x[t, 0:width) = table[ids[t]] * scale (bfloat16 table of row length ld), zeros up to ld; float32 out */
 VMI_HY_API int vmi_hy_embed(const int64_t* ids, const void* table, float* x, int32_t T, int32_t width, int32_t ld, int32_t vocab,

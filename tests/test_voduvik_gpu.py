@@ -188,6 +188,42 @@ def test_many_columns_leave_the_rows_in_lds(M, N, K):
     _norm_products(M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K", [(7, 16 * 515, 1024), (33, 16 * 387, 1024), (17, 16 * 389, 1024), (64, 16 * 130, 1024), (40, 16 * 510, 1024), (3, 16 * 257, 2048), (31, 16 * 129, 2048),
+                                   (18, 16 * 259, 1536), (50, 16 * 129, 768), (70, 16 * 255, 512), (90, 16 * 85, 256), (21, 16 * 200, 96), (35, 16 * 330, 992)])
+def test_few_rows_behind_a_norm_take_several_slabs_a_workgroup(M, N, K):
+    """norm_rows_kernel with two to six slabs of 16 columns a workgroup, the last workgroup's not all there, for every length of a row it is built for, shared
+    out evenly and not."""
+    from vllmini_amd import hybrid_ops as ops
+
+    assert not ops.linear_normed_first(M, _norm_products(M, ops.pad32(N), K))
+
+
+@pytest.mark.parametrize("M,N,K", [(9, 16 * 513, 2048), (16, 16 * 1030, 2048), (32, 16 * 770, 2048), (33, 16 * 400, 2048), (64, 16 * 514, 2048), (50, 16 * 770, 1024), (12, 16 * 258, 4096),
+                                   (40, 16 * 514, 4096)])
+def test_rows_normed_once_are_held_in_registers(M, N, K):
+    """held_rows_kernel: one and two row tiles, row blocks, slabs that the workgroups do not share evenly, several chunks of K a slab and one."""
+    from vllmini_amd import hybrid_ops as ops
+
+    assert ops.linear_normed_first(M, _norm_products(M, ops.pad32(N), K))
+
+
+@pytest.mark.parametrize("M", [1, 16, 33, 64])
+@pytest.mark.parametrize("N,K", [(48, 32), (16 * 130, 128), (32, 224), (16 * 133, 480), (16 * 131, 992), (64, 1024), (16 * 129, 2016), (32, 2080), (96, 3072), (32, 4064), (48, 4576), (32, 4640),
+                                 (16 * 130, 4640), (48, 9248)])
+def test_few_rows_as_they_are(M, N, K):
+    """plain_rows_kernel: K in one chunk a wave and in several, waves with unequal parts or none, one and two row tiles a workgroup; the rows of a wider matrix."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M * K + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    N = ops.pad32(N)
+    w = (rnd(N, K) / K ** 0.5).to(torch.bfloat16)
+    t, x, bias, base = ops.MatrixTiles(w, torch.bfloat16), rnd(M, K + 8).to(torch.bfloat16)[:, :K], rnd(N), rnd(M, N)
+    y = x.double() @ w.double().T
+    close(ops.linear(x, t, bias=bias), y + bias, torch.bfloat16)
+    close(ops.linear(x, t, residual=True, out=base.clone()), base.double() + y, torch.bfloat16, tol16=1e-3)
+
+
 def _norm_products(M, N, K):
     """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
     from vllmini_amd import hybrid_ops as ops

@@ -9,6 +9,7 @@
 #include <string>
 
 #include "hybrid_common.hpp"
+#include "hybrid_linear.hpp"
 
 namespace vmi_hybrid {
 
@@ -67,55 +68,6 @@ struct XUnit<T, VMI_HY_X_CONCAT> {
   }
   __device__ __forceinline__ V8<T> finish(const float*, int, float, float) const { return from_f32<T>(v); }
 };
-
-// Four consecutive columns n .. n + 3 of row m, accumulated, on their way out.  n0: the first column of their tile (scalar)
-template <typename T, int EPI>
-__device__ __forceinline__ void epilogue(const vmi_hy_linear_args& p, const f32x4& acc, int m, int n, int n0, int grp) {
-  const int64_t yoff = (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride;
-  if constexpr (EPI == VMI_HY_E_STORE) {
-    f32x4 b = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (p.bias) b = *reinterpret_cast<const f32x4*>(p.bias + n);
-    V4<T> o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = (T)(acc[r] + b[r]);
-    *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
-  } else if constexpr (EPI == VMI_HY_E_RESIDUAL) {
-    f32x4* y = reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + yoff + n);
-    *y = *y + acc;
-  } else if constexpr (EPI == VMI_HY_E_FLOAT) {
-    float* y = static_cast<float*>(p.y) + yoff + n;
-    if (n + 4 <= p.n_out && (p.ldy & 3) == 0) {
-      *reinterpret_cast<f32x4*>(y) = acc * p.scale;
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < p.n_out) y[r] = acc[r] * p.scale;
-    }
-  } else if constexpr (EPI == VMI_HY_E_GLU) {
-    typename Elem<T>::v2 o;
-    o[0] = (T)glu(acc[0], acc[1], p.scale, p.glu_alpha, p.glu_up);
-    o[1] = (T)glu(acc[2], acc[3], p.scale, p.glu_alpha, p.glu_up);
-    *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y) + yoff + (n >> 1)) = o;
-  } else if constexpr (EPI == VMI_HY_E_STORE_GLU) {
-    if (n0 < p.n_split) {
-      V4<T> o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (T)acc[r];
-      *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
-    } else {
-      typename Elem<T>::v2 o;
-      o[0] = (T)glu(acc[0], acc[1], p.scale, p.glu_alpha, p.glu_up);
-      o[1] = (T)glu(acc[2], acc[3], p.scale, p.glu_alpha, p.glu_up);
-      *reinterpret_cast<typename Elem<T>::v2*>(static_cast<T*>(p.y2) + (int64_t)m * p.ldy2 + ((n - p.n_split) >> 1)) = o;
-    }
-  } else {   // VMI_HY_E_GATED
-    const float g = sigmoid((float)static_cast<const T*>(p.gate)[(int64_t)m * p.ldg + grp]);
-    V4<T> o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = (T)(acc[r] * g);
-    *reinterpret_cast<V4<T>*>(static_cast<T*>(p.y) + yoff + n) = o;
-  }
-}
 
 template <typename T, int BM, int NW, int KS, int XK, int EPI>
 __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear_args p) {
@@ -465,99 +417,15 @@ static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
   return launched("vmi_hy_linear");
 }
 
-// Few rows behind a norm and few columns (bfloat16, one group): a workgroup owns 16 columns of 16 rows and its EIGHT waves take an eighth of K
-// each.  A wave needs its part of a row once, so x and the weights go straight from memory to registers in the matrix cores' layout, all of it
-// requested before the first wait; the norm happens on those registers once the waves' parts of a row's sums have met in LDS.  Bound by one
-// trip through memory and the launch.  1 / 12 rows (linear_kernel before; resident_kernel, whose workgroups first bring whole rows into LDS):
-// K 1024, N 2048 6.5 / 7.1 (5.6 / 6.8) -> 4.7 / 5.6 us, N 6144 10.0 / 11.1 (7.7 / 9.7) -> 6.7 / 8.4; K 2048, N 4096 14.1 / 16.2 -> 8.0 / 9.9; 32 rows, K 1024, N 2048
-// 9.5 (9.4) -> 6.1.  Without a norm linear_kernel's waves see x as early: level at K 1024, 4.7 against 5.4 -> 6.0 for 12 rows of 3072.
-template <int J, int EPI>   // at most J k-steps a wave
-__global__ __launch_bounds__(512, 2) void rows_kernel(const vmi_hy_linear_args p) {
-  constexpr int RK = 8;
-  __shared__ f32x4 red[RK - 1][64];
-  __shared__ float sums[RK][2][16];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
-  // (the row tiles of 16 columns go to one XCD, which then reads their weights once)
-  const int RB = (p.M + 15) >> 4, SL = p.N >> 4;
-  const int slab = (int)(blockIdx.x / (8 * RB)) * 8 + (int)(blockIdx.x & 7), m = (int)(blockIdx.x >> 3) % RB * 16 + r16;
-  if (slab >= SL) return;
-  const int nks = p.K >> 5, per = (nks + RK - 1) / RK, k0 = wave * per, nk = min(per, nks - k0);   // (nk <= 0: no part of K is left for it)
-  // (steps past this wave's last read it again and meet nothing: no lane-wise condition around a load)
-  auto at = [&](int j) { return 32 * min(k0 + min(j, per - 1), nks - 1) + 8 * kc; };
-  const int mm = min(m, p.M - 1);
-  const float* row = static_cast<const float*>(p.x) + (int64_t)(p.rows ? p.rows[mm] : mm) * p.ldx;
-  f32x8 x[J], nw[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) x[j] = load8(row + at(j));
-  const float sh = p.rms ? 0.f : row[0];
-#pragma unroll
-  for (int j = 0; j < J; ++j) nw[j] = load8(p.norm_w + at(j));
-  const b16* wp = static_cast<const b16*>(p.w) + ((int64_t)slab * nks * 64 + lane) * 8;
-  b16x8 w[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) w[j] = load8(wp + (int64_t)(at(j) >> 5) * 512);
-  float s = 0.f, q = 0.f;
-#pragma unroll
-  for (int j = 0; j < J; ++j)
-    if (j < nk) {   // (scalar)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float d = at(j) + e < p.norm_n ? x[j][e] - sh : 0.f;
-        s += d;
-        q = fmaf(d, d, q);
-      }
-    }
-  s += __shfl_xor(s, 16, 64), q += __shfl_xor(q, 16, 64);
-  s += __shfl_xor(s, 32, 64), q += __shfl_xor(q, 32, 64);
-  if (kc == 0) sums[wave][0][r16] = s, sums[wave][1][r16] = q;
-  __syncthreads();
-  s = q = 0.f;
-#pragma unroll
-  for (int v = 0; v < RK; ++v) s += sums[v][0][r16], q += sums[v][1][r16];
-  const float ms = p.rms ? 0.f : s / (float)p.norm_n, mean = sh + ms;
-  const float rstd = 1.f / sqrtf(fmaxf(q / (float)p.norm_n - ms * ms, 0.f) + p.eps);
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < J; ++j)
-    if (j < nk) {
-      f32x8 r;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = (x[j][e] - mean) * rstd * nw[j][e];   // (the weight is zero past norm_n)
-      mma(acc, w[j], from_f32<b16>(r));
-    }
-  if (wave > 0) red[wave - 1][lane] = acc;
-  __syncthreads();
-  if (wave > 0) return;
-#pragma unroll
-  for (int v = 0; v < RK - 1; ++v) acc += red[v][lane];
-  if (m < p.M) epilogue<b16, EPI>(p, acc, m, slab * 16 + 4 * kc, slab * 16, 0);
-}
-
-// Whether a product behind a norm goes to rows_kernel: every workgroup reads its rows again, so only while they are few, and fewer where a row is long
-// (K 2048, N 6144, 384 of them: 13.3 us here, 10.2 in resident_kernel; 32 rows, K 1024, N 8192, 1024: 13.8 and 12.7)
-static bool rows_fit(int M, int N, int K) {
-  return M <= 64 && K <= 2048 && (int64_t)(N >> 4) * ((M + 15) >> 4) <= (K <= 1024 ? 512 : 256);
-}
-
-// Whether the rows behind a norm are better normed once, by a kernel of their own (3.3 us between two others), than in every workgroup of the product:
+// Whether the rows behind a norm are better normed once, by a kernel of their own (2.8 us between two others), than in every workgroup of the product:
 // long rows, from 17 of them on, where the workgroups' share of that is 32 rows a column of tiles (except of a vocabulary's columns behind rows that stay
 // in LDS), from 9 on where the columns are few.  K 4096, in every workgroup -> once: 32 rows, N 4096 25.0 -> 18.3 us, N 12288 56.3 -> 35.5; 40, N 24576 84.4 ->
 // 54.4; 16, N 4096 19.3 -> 16.4, N 24576 50.7 -> 46.8; 8, N 8192 21.8 -> 21.4.  Shorter rows gain less than a launch costs a caller who records no graph
 // and waits for his own calls (6 us): 32 rows, K 2048, N 12288 22.4 -> 20.7, K 1024, N 8192 15.0 -> 11.6; a prompt of 35 tokens, width 1024, 1.00 -> 1.06 ms.
 static bool norm_first(int M, int N, int K) {
-  if (K < 4096 || rows_fit(M, N, K)) return false;
+  if (K < 4096) return false;
   if (M > 16) return M > 32 || N < 24576 || resident_kind(M, N, K) == 0;
   return M > 8 && N <= 4 * K;
-}
-
-template <int EPI>
-static int launch_rows(const vmi_hy_linear_args& p, hipStream_t st) {
-  const int per = ((p.K >> 5) + 7) / 8;
-  auto go = [&](auto fn) {
-    hipLaunchKernelGGL(fn, dim3(((p.N >> 4) + 7) / 8 * 8 * ((p.M + 15) >> 4)), dim3(512), 0, st, p);
-    return launched("vmi_hy_linear");
-  };
-  return per <= 1 ? go(rows_kernel<1, EPI>) : per <= 2 ? go(rows_kernel<2, EPI>) : per <= 4 ? go(rows_kernel<4, EPI>) : go(rows_kernel<8, EPI>);
 }
 
 template <typename T, int BM, int NW, int KS, int XK, int EPI>
@@ -576,8 +444,11 @@ template <typename T, int XK, int EPI>
 static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   // few rows: 16-row tiles; a layer with few columns splits K over the waves of a workgroup so that all compute units read
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
+  constexpr bool PLAIN = sizeof(T) == 2 && XK == VMI_HY_X_ROWS && (EPI == VMI_HY_E_STORE || EPI == VMI_HY_E_RESIDUAL || EPI == VMI_HY_E_GATED);
+  if constexpr (PLAIN)
+    if (plain_rows_fit(p.M)) return launch_plain_rows(p, st);
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
-    if (p.groups == 1 && rows_fit(p.M, p.N, p.K)) return launch_rows<EPI>(p, st);
+    if (p.groups == 1 && norm_rows_fit(p.M, p.N, p.K)) return launch_norm_rows(p, st);
     switch (p.groups == 1 && resident_pays(p.M, p.N, p.K) ? resident_kind(p.M, p.N, p.K) : 0) {
       case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, EPI>(p, st) : launch_resident<2, 8, 2, 2, EPI>(p, st);
       case 3: return launch_resident<2, 8, 1, 2, EPI>(p, st);
@@ -585,13 +456,15 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
       default: break;
     }
   }
-  if (p.M <= 32) {
-    const int64_t wgs = slabs * ((p.M + 15) / 16);
-    if (wgs >= 2048) return launch_linear<T, 16, 4, 1, XK, EPI>(p, st);
-    if (wgs >= 400 || p.K < 256) return launch_linear<T, 16, 2, 2, XK, EPI>(p, st);
-    if constexpr (sizeof(T) == 2)
-      if (wgs < 192 && p.K >= 1024) return launch_linear<T, 16, 1, 8, XK, EPI>(p, st);
-    return launch_linear<T, 16, 1, 4, XK, EPI>(p, st);
+  if constexpr (!PLAIN) {
+    if (p.M <= 32) {
+      const int64_t wgs = slabs * ((p.M + 15) / 16);
+      if (wgs >= 2048) return launch_linear<T, 16, 4, 1, XK, EPI>(p, st);
+      if (wgs >= 400 || p.K < 256) return launch_linear<T, 16, 2, 2, XK, EPI>(p, st);
+      if constexpr (sizeof(T) == 2)
+        if (wgs < 192 && p.K >= 1024) return launch_linear<T, 16, 1, 8, XK, EPI>(p, st);
+      return launch_linear<T, 16, 1, 4, XK, EPI>(p, st);
+    }
   }
   if (p.M <= 96 || slabs / 4 * ((p.M + 63) / 64) < 256) return launch_linear<T, 32, 4, 1, XK, EPI>(p, st);
   return launch_linear<T, 64, 4, 1, XK, EPI>(p, st);
@@ -599,6 +472,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
 
 // rows that stand in p.x normed: what follows a norm
 static int linear_normed(const vmi_hy_linear_args& p, hipStream_t st) {
+  if (p.groups == 1 && held_rows_pay(p.M, p.N, p.K)) return launch_held_rows(p, st);
   switch (p.epilogue) {
     case VMI_HY_E_STORE: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_STORE>(p, st);
     case VMI_HY_E_FLOAT: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_FLOAT>(p, st);
@@ -803,11 +677,15 @@ using namespace vmi_hybrid;
 extern "C" {
 
 int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype) {
-  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups == 1 && norm_first(M, N, K);
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups == 1 && (norm_first(M, N, K) || (K <= 2048 && held_rows_pay(M, N, K)));
 }
 
 int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
   return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && resident_kind(M, N, K) != 0;
+}
+
+int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && K <= 2048 && held_rows_pay(M, N, K);
 }
 
 int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
@@ -827,7 +705,8 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (a->x_kind == VMI_HY_X_NORM && a->normed && a->dtype == VMI_HY_BF16 && a->epilogue != VMI_HY_E_RESIDUAL && a->epilogue != VMI_HY_E_GATED) {
-    hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
+    if (launch_norm_few(*a, st) != VMI_HY_OK)
+      hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
                        (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
     vmi_hy_linear_args rows = *a;
     rows.x = a->normed, rows.ldx = a->K, rows.x_gstride = 0, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;   // (all groups read the same rows)

@@ -1,0 +1,497 @@
+// Products of few rows in bfloat16 (include/vmi_hybrid.h): the waves of a workgroup take a part of K each.
+//
+// A launch of this kind is a chain of latencies, so what is on the chip is counted: rows come from memory as whole lines and change into the matrix
+// cores' layout (16 rows x 64 bytes) in LDS; all arguments are asked for at once (`need`: left to itself the compiler asks branch by branch, a trip to
+// memory each); what the epilogue adds to is asked for in front of everything.  The waves' partial tiles meet in LDS; one wave a tile adds them in
+// the order of K and stores.
+#include "hybrid_linear.hpp"
+
+namespace vmi_hybrid {
+
+template <class V>
+__device__ __forceinline__ void need(const V& v) {
+  asm volatile("" ::"s"(v));
+}
+
+template <int EPI>
+__device__ __forceinline__ void need_args(const vmi_hy_linear_args& p) {
+  need(p.x), need(p.w), need(p.y), need(p.ldx), need(p.ldy), need(p.M), need(p.N), need(p.K);
+  if constexpr (EPI == VMI_HY_E_STORE) need(p.bias);
+  if constexpr (EPI == VMI_HY_E_GATED) need(p.gate), need(p.ldg);
+  if constexpr (EPI == VMI_HY_E_GLU || EPI == VMI_HY_E_STORE_GLU) need(p.scale), need(p.glu_alpha), need(p.glu_up);
+  if constexpr (EPI == VMI_HY_E_STORE_GLU) need(p.y2), need(p.ldy2), need(p.n_split);
+  if constexpr (EPI == VMI_HY_E_FLOAT) need(p.scale), need(p.n_out);
+}
+
+constexpr int plain_stride(int J, int MT) { return MT * 16 * (64 * J + 16); }   // bytes of LDS a wave
+
+// Rows as they are.  A workgroup owns 16 columns of 16 MT rows of a group; a wave brings its own part of K of the rows through its own part of the
+// LDS, chunks of J k-steps, so nothing but the sum at the end waits for another wave.  NB chunks of weights in registers.  The order of the requests is the
+// order of their use (they complete in order): rows of a chunk, then the weights NB - 1 chunks on.  NB = 1: a wave's part is one chunk.
+template <int RW, int J, int MT, int NB, int EPI>
+__global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_hy_linear_args p) {
+  constexpr int LDB = 64 * J + 16, STRIDE = plain_stride(J, MT);
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [RW][STRIDE]
+  need_args<EPI>(p), need(p.x_gstride), need(p.y_gstride);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int slab = blockIdx.x, m0 = blockIdx.y * 16 * MT, grp = blockIdx.z;
+  if (slab * 16 >= p.N) return;
+  const int nks = p.K >> 5, per = (nks + RW - 1) / RW, k0 = wave * per, nk = min(per, nks - k0);   // (nk <= 0: no part of K is left for it)
+  const int nch = (per + J - 1) / J, rows = p.M - m0;
+  const int m = m0 + (MT == 1 ? 0 : wave * 16) + r16, n = slab * 16 + 4 * kc;   // (what this wave stores, if it does)
+  const bool stores = wave < MT && m < p.M;
+  [[maybe_unused]] f32x4 before = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (EPI == VMI_HY_E_RESIDUAL)
+    if (stores) before = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.y) + (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride + n);
+
+  const b16* xp = static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride;
+  const b16* wp = static_cast<const b16*>(p.w) + (((int64_t)grp * (p.N >> 4) + slab) * nks * 64 + lane) * 8;
+  b16x8 x[MT][J], w[NB][J];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+    for (int i = 0; i < J; ++i) x[mi][i] = zero8<b16>();
+  // (16 rows of 4 J units of 16 bytes; units past the row are its last one and meet nothing; 64 units that lie past M altogether stay away)
+  auto load_x = [&](int c) {
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+      for (int i = 0; i < J; ++i)
+        if (mi * 16 + 64 * i / (4 * J) < rows) {   // (scalar)
+          const int u = lane + 64 * i, r = u / (4 * J), col = min(4 * (k0 + c * J) + u % (4 * J), 4 * nks - 1);
+          x[mi][i] = load8(xp + (int64_t)min(m0 + mi * 16 + r, p.M - 1) * p.ldx + col * 8);
+        }
+  };
+  auto load_w = [&](b16x8(&dst)[J], int c) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) dst[j] = load8(wp + (int64_t)min(k0 + min(c * J + j, per - 1), nks - 1) * 512);
+  };
+  load_x(0);
+#pragma unroll
+  for (int b = 0; b < (NB > 1 ? NB - 1 : 1); ++b) load_w(w[b], b);
+  unsigned char* mine = smem + wave * STRIDE;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto chunk = [&](int c, b16x8(&cur)[J], b16x8(&last)[J]) {
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+      for (int i = 0; i < J; ++i) {
+        const int u = lane + 64 * i;
+        *reinterpret_cast<b16x8*>(mine + (mi * 16 + u / (4 * J)) * LDB + u % (4 * J) * 16) = x[mi][i];
+      }
+    if constexpr (NB > 1) {
+      if (c + 1 < nch) load_x(c + 1);
+      load_w(last, c + NB - 1);   // (past the end: a tile again, a cache hit)
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's LDS accesses happen in order: only the compiler has to keep them)
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      if (c * J + j < nk) {   // (scalar)
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], *reinterpret_cast<const b16x8*>(mine + (mi * 16 + r16) * LDB + 64 * j + 16 * kc));
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  for (int c = 0; c < nch; c += NB) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      if (c + b < nch) chunk(c + b, w[b], w[(b + NB - 1) % NB]);
+  }
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) *reinterpret_cast<f32x4*>(mine + mi * 1024 + lane * 16) = acc[mi];
+  __syncthreads();
+  if (!stores) return;
+  const unsigned char* at = smem + (MT == 1 ? 0 : wave) * 1024 + lane * 16;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+  for (int v = 1; v < RW; ++v) sum += *reinterpret_cast<const f32x4*>(at + v * STRIDE);
+  if constexpr (EPI == VMI_HY_E_RESIDUAL)
+    *reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride + n) = before + sum;
+  else
+    epilogue<b16, EPI>(p, sum, m, n, slab * 16, grp);
+}
+
+// Rows of the element type over many columns, 16 MT of them: eight waves hold an eighth of K of all rows each, in registers and in the matrix cores' layout,
+// and the workgroup walks over slabs of 16 columns, blockIdx, blockIdx + grid, ..; the ring of weight tiles runs on across slabs.  NCH chunks of 4 k-steps are a
+// wave's part of a slab, NB chunks are in registers.  A slab's partial tiles meet in LDS (two places, one barrier a slab); another wave each time adds a
+// tile's in the order of K and stores.
+constexpr size_t HELD_LDS = 2 * 8 * 1024;   // ... a row tile
+
+template <int NCH, int MT, int NB, int EPI>
+__global__ __launch_bounds__(512, 2) void held_rows_kernel(const vmi_hy_linear_args p, const int slabs) {
+  constexpr int W = 8, CS = 4;
+  static_assert(NB % NCH == 0, "a chunk's place in its slab follows from its place in the ring");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [2][W][MT][1024]
+  need_args<EPI>(p), need(slabs);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int m0 = blockIdx.y * 16 * MT, nks = p.K >> 5, kpw = (nks + W - 1) / W, k0 = wave * kpw, nk = min(kpw, nks - k0);
+  if ((int)blockIdx.x >= slabs) return;
+  b16x8 x[NCH * CS][MT], wb[NB][CS];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) {
+    const b16* row = static_cast<const b16*>(p.x) + (int64_t)min(m0 + mi * 16 + r16, p.M - 1) * p.ldx + 8 * kc;
+#pragma unroll
+    for (int j = 0; j < NCH * CS; ++j) x[j][mi] = load8(row + 32 * min(k0 + min(j, kpw - 1), nks - 1));
+  }
+  const b16* wp = static_cast<const b16*>(p.w) + lane * 8;
+  int ls = blockIdx.x;   // the slab to load from next
+  auto load_w = [&](b16x8(&dst)[CS], int c) {
+    const b16* at = wp + (int64_t)ls * nks * 512;
+#pragma unroll
+    for (int j = 0; j < CS; ++j) dst[j] = load8(at + (int64_t)min(k0 + min(c * CS + j, kpw - 1), nks - 1) * 512);
+    if (c == NCH - 1 && ls + (int)gridDim.x < slabs) ls += gridDim.x;   // (past the last: that one again, a cache hit)
+  };
+#pragma unroll
+  for (int b = 0; b < NB - 1; ++b) load_w(wb[b], b % NCH);
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int total = (slabs - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * NCH;
+  int i = 0, slab = blockIdx.x;
+  for (int t = 0; t < total; t += NB) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (t + b >= total) break;
+      load_w(wb[(b + NB - 1) % NB], (b + NB - 1) % NCH);
+#pragma unroll
+      for (int j = 0; j < CS; ++j)
+        if (b % NCH * CS + j < nk) {   // (scalar)
+#pragma unroll
+          for (int mi = 0; mi < MT; ++mi) mma(acc[mi], wb[b][j], x[b % NCH * CS + j][mi]);
+        }
+      if (b % NCH < NCH - 1) continue;
+      unsigned char* to = smem + (i & 1) * W * MT * 1024;
+#pragma unroll
+      for (int mi = 0; mi < MT; ++mi) {
+        *reinterpret_cast<f32x4*>(to + (wave * MT + mi) * 1024 + lane * 16) = acc[mi];
+        acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      __syncthreads();   // (two places: who still adds up slab i has not passed the barrier of slab i + 1)
+      const int mi = (wave - i * MT) & (W - 1);
+      if (mi < MT) {
+        f32x4 sum = *reinterpret_cast<const f32x4*>(to + mi * 1024 + lane * 16);
+#pragma unroll
+        for (int v = 1; v < W; ++v) sum += *reinterpret_cast<const f32x4*>(to + (v * MT + mi) * 1024 + lane * 16);
+        const int m = m0 + mi * 16 + r16;
+        if (m < p.M) epilogue<b16, EPI>(p, sum, m, slab * 16 + 4 * kc, slab * 16, 0);
+      }
+      ++i;
+      slab += gridDim.x;
+    }
+  }
+}
+
+inline size_t norm_rows_lds(int K, int rw, int ns) { return (size_t)16 * (K * 2 + 16) + (size_t)rw * ns * 1024; }
+
+// Rows behind a norm (float32).  Half a wave owns a row, so its statistics meet inside the wave: mean first, then the squares around it, on registers.  A
+// workgroup takes NS slabs of 16 columns, as many as leave one workgroup a compute unit: two of them share its load paths and vector units.
+// J: at most that many k-steps a wave, and half as many 16-byte units of a row a lane.
+template <int RW, int J, int NS, bool FULL, int EPI>
+__global__ __launch_bounds__(64 * RW, RW / 4) void norm_rows_kernel(const vmi_hy_linear_args p) {
+  constexpr int LPR = 4 * RW, U = 2 * J;   // lanes a row, 16-byte units of a row a lane
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // rows [16][2 K + 16 bytes], then the partial tiles [RW][NS][1024]
+  need_args<EPI>(p), need(p.rows), need(p.norm_w), need(p.norm_n), need(p.rms), need(p.eps);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int SL = p.N >> 4, slab = blockIdx.x * NS, m = blockIdx.y * 16 + r16;
+  if (slab >= SL) return;
+  const int nks = FULL ? RW * J : p.K >> 5, per = FULL ? J : (nks + RW - 1) / RW, k0 = wave * per, nk = FULL ? J : min(per, nks - k0);
+  auto step = [&](int j) { return FULL ? k0 + j : min(k0 + min(j, per - 1), nks - 1); };
+  auto row_sum = [](float v) {
+#pragma unroll
+    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+  };
+  const int units = nks * 8, l = lane % LPR, xr = (wave * 64 + lane) / LPR, mm = min((int)blockIdx.y * 16 + xr, p.M - 1);
+  // (what lies past a row, or past a wave's last k-step, is that last one again and meets nothing: no lane-wise condition around a load)
+  auto unit = [&](int i) { return (FULL ? l + LPR * i : min(l + LPR * i, units - 1)) * 4; };
+  const float* row = static_cast<const float*>(p.x) + (int64_t)(p.rows ? p.rows[mm] : mm) * p.ldx;
+  f32x4 x[U], g[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) x[i] = *reinterpret_cast<const f32x4*>(row + unit(i));
+#pragma unroll
+  for (int i = 0; i < U; ++i) g[i] = *reinterpret_cast<const f32x4*>(p.norm_w + unit(i));
+  b16x8 w[NS][J];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const b16* wp = static_cast<const b16*>(p.w) + ((int64_t)min(slab + s, SL - 1) * nks * 64 + lane) * 8;
+#pragma unroll
+    for (int j = 0; j < J; ++j) w[s][j] = load8(wp + (int64_t)step(j) * 512);
+  }
+  // (only the first norm_n columns are normed: what lies behind them may be anything, and comes out as zeros)
+  auto clear_behind = [&]() {
+    if (p.norm_n < p.K) {   // (scalar)
+#pragma unroll
+      for (int i = 0; i < U; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[i][e] = (l + LPR * i) * 4 + e < p.norm_n ? x[i][e] : 0.f;
+    }
+  };
+  auto there = [&](int i) { return FULL || l + LPR * i < units; };
+  const float inv = 1.f / (float)p.norm_n;
+  clear_behind();
+  if (!p.rms) {
+    float s4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (there(i)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s4[e] += x[i][e];
+      }
+    const float mean = row_sum((s4[0] + s4[1]) + (s4[2] + s4[3])) * inv;
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[i][e] -= mean;
+    clear_behind();
+  }
+  float q4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < U; ++i)
+    if (there(i)) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q4[e] = fmaf(x[i][e], x[i][e], q4[e]);
+    }
+  const float rstd = 1.f / sqrtf(row_sum((q4[0] + q4[1]) + (q4[2] + q4[3])) * inv + p.eps);
+  const int ldb = (FULL ? 64 * RW * J : p.K * 2) + 16;
+#pragma unroll
+  for (int i = 0; i < U; ++i)
+    if (there(i)) {
+      b16x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (b16)(x[i][e] * rstd * g[i][e]);
+      *reinterpret_cast<b16x4*>(smem + xr * ldb + unit(i) * 2) = v;
+    }
+  __syncthreads();
+  f32x4 acc[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+    if (j < nk) {   // (scalar)
+      const b16x8 v = *reinterpret_cast<const b16x8*>(smem + r16 * ldb + 64 * (k0 + j) + 16 * kc);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) mma(acc[s], w[s][j], v);
+    }
+  unsigned char* parts = smem + 16 * ldb;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) *reinterpret_cast<f32x4*>(parts + (wave * NS + s) * 1024 + lane * 16) = acc[s];
+  __syncthreads();
+  const int s = NS == 1 ? 0 : wave;   // the slab this wave stores
+  if (wave >= NS || slab + s >= SL || m >= p.M) return;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(parts + s * 1024 + lane * 16);
+#pragma unroll
+  for (int v = 1; v < RW; ++v) sum += *reinterpret_cast<const f32x4*>(parts + (v * NS + s) * 1024 + lane * 16);
+  epilogue<b16, EPI>(p, sum, m, (slab + s) * 16 + 4 * kc, (slab + s) * 16, 0);
+}
+
+// out[t] = the norm of x[rows[t]] in the element type, a workgroup a row; everything asked for at once, U 16-byte units a thread (K <= 2048 U).  Few rows stand
+// between two products here, and what counts is how soon the second one starts: 4.1 us of a chain of launches with a row's weight asked for behind its statistics, 2.8 so
+template <int U>
+__global__ __launch_bounds__(512) void norm_few_kernel(const vmi_hy_linear_args p) {
+  need(p.x), need(p.ldx), need(p.rows), need(p.norm_w), need(p.normed), need(p.norm_n), need(p.K), need(p.eps), need(p.rms);
+  __shared__ float part[2][8];
+  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const float* row = static_cast<const float*>(p.x) + (int64_t)(p.rows ? p.rows[t] : t) * p.ldx;
+  f32x4 v[U], w[U];
+#pragma unroll
+  for (int i = 0; i < U; ++i) v[i] = *reinterpret_cast<const f32x4*>(row + min((tid + i * 512) * 4, p.K - 4));
+#pragma unroll
+  for (int i = 0; i < U; ++i) w[i] = *reinterpret_cast<const f32x4*>(p.norm_w + min((tid + i * 512) * 4, p.K - 4));
+  auto clear_behind = [&]() {   // (the columns that are normed: what lies behind them may be anything)
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] = (tid + i * 512) * 4 + e < p.norm_n ? v[i][e] : 0.f;
+  };
+  auto all = [&](float s, float(&at)[8]) {
+    s = wave_sum(s);
+    if (lane == 0) at[wave] = s;
+    __syncthreads();
+    return ((at[0] + at[1]) + (at[2] + at[3])) + ((at[4] + at[5]) + (at[6] + at[7]));
+  };
+  const float inv = 1.f / (float)p.norm_n;
+  clear_behind();
+  if (!p.rms) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < U; ++i) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+    const float mean = all(s, part[0]) * inv;
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] -= mean;
+    clear_behind();
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < U; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q = fmaf(v[i][e], v[i][e], q);
+  const float rstd = 1.f / sqrtf(all(q, part[1]) * inv + p.eps);
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    const int k = (tid + i * 512) * 4;
+    b16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (b16)(v[i][e] * rstd * w[i][e]);
+    if (k < p.K) *reinterpret_cast<b16x4*>(static_cast<b16*>(p.normed) + (int64_t)t * p.K + k) = o;
+  }
+}
+
+// ---- which, and how -------------------------------------------------------------------------------------------------------------
+
+template <typename F>
+static int launch(F* fn, const vmi_hy_linear_args& p, dim3 grid, int threads, size_t lds, hipStream_t st) {
+  if (int rc = allow_lds(fn, lds, "vmi_hy_linear")) return rc;
+  hipLaunchKernelGGL(fn, grid, dim3(threads), lds, st, p);
+  return launched("vmi_hy_linear");
+}
+// (a multiple of 8 column blocks: the row tiles of one then go to one XCD, which reads their weights once)
+static unsigned blocks8(int n) { return (unsigned)(n + 7) / 8 * 8; }
+
+int launch_norm_few(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch ((p.K + 2047) / 2048) {
+    case 1: return launch(norm_few_kernel<1>, p, dim3(p.M), 512, 0, st);
+    case 2: return launch(norm_few_kernel<2>, p, dim3(p.M), 512, 0, st);
+    case 3:
+    case 4: return launch(norm_few_kernel<4>, p, dim3(p.M), 512, 0, st);
+    default: return -1;   // (longer rows: add_norm_kernel)
+  }
+}
+
+// Slabs a workgroup of norm_rows_kernel takes: as few as leave one workgroup a compute unit; 0: the kernel is not built for these sizes, or they are more than
+// that.  Up to 1024 columns, and 1536 and 2048, whose rows a workgroup's 16 waves share without a remainder (else the addresses cost the registers: 7.5 -> 14.5 us).
+static int norm_slabs(int M, int N, int K) {
+  const int nks = K >> 5, rb = (M + 15) >> 4;
+  if (nks > 32 && nks != 48 && nks != 64) return 0;
+  for (int ns : {1, 2, 3, 4, 6}) {
+    if (ns > 2 && nks > 32) break;
+    if ((ns == 3 || ns == 6) && nks != 32) continue;
+    if ((int64_t)(((N >> 4) + ns - 1) / ns) * rb <= 256) return ns;
+  }
+  return 0;
+}
+// rows_kernel's forerunner (an eighth of K a wave, rows in the matrix cores' layout), resident_kernel or linear_kernel, whichever was ahead / norm_rows_kernel, in a graph of such
+// launches, us: K 1024, N 2048 1 / 12 / 32 / 40 rows 4.7 / 5.6 / 6.0 / 8.6 -> 4.2 / 4.4 / 4.5 / 4.8, N 6144 6.5 / 8.2 / 11.2 / 18.5 -> 5.2 / 5.3 / 5.6 / 6.5, N 10240 8.1 / 9.9 / 13.8
+// (32) -> 6.4 / 6.3 / 7.1; K 2048, N 4096 7.7 / 9.8 / 15.3 (32) -> 7.1 / 7.5 / 8.5.  More than a workgroup a compute unit: K 1024, N 10240, 40 rows 11.5 here, 11.0 in held_rows_kernel.
+bool norm_rows_fit(int M, int N, int K) { return norm_slabs(M, N, K) > 0; }
+
+template <int RW, int J, bool FULL, int EPI>
+static int norm_rows_of(const vmi_hy_linear_args& p, int ns, hipStream_t st) {
+  auto go = [&](auto* fn) { return launch(fn, p, dim3(blocks8(((p.N >> 4) + ns - 1) / ns), (p.M + 15) >> 4), 64 * RW, norm_rows_lds(p.K, RW, ns), st); };
+  if (ns == 1) return go(norm_rows_kernel<RW, J, 1, FULL, EPI>);
+  if (ns == 2) return go(norm_rows_kernel<RW, J, 2, FULL, EPI>);
+  if constexpr (RW == 8) {
+    if (ns == 4) return go(norm_rows_kernel<RW, J, 4, FULL, EPI>);
+    if constexpr (J == 4 && FULL) {
+      if (ns == 3) return go(norm_rows_kernel<RW, J, 3, FULL, EPI>);
+      if (ns == 6) return go(norm_rows_kernel<RW, J, 6, FULL, EPI>);
+    }
+  }
+  return fail(VMI_HY_E_ARG, "vmi_hy_linear", "not built");   // (norm_slabs names no other)
+}
+
+template <int EPI>
+static int norm_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
+  const int nks = p.K >> 5, ns = norm_slabs(p.M, p.N, p.K);
+  if (nks == 64) return norm_rows_of<16, 4, true, EPI>(p, ns, st);
+  if (nks == 48) return norm_rows_of<16, 3, true, EPI>(p, ns, st);
+  if (nks == 32) return norm_rows_of<8, 4, true, EPI>(p, ns, st);
+  if (nks == 24) return norm_rows_of<8, 3, true, EPI>(p, ns, st);
+  if (nks == 16) return norm_rows_of<8, 2, true, EPI>(p, ns, st);
+  if (nks == 8) return norm_rows_of<8, 1, true, EPI>(p, ns, st);
+  return nks <= 16 ? norm_rows_of<8, 2, false, EPI>(p, ns, st) : norm_rows_of<8, 4, false, EPI>(p, ns, st);
+}
+
+int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch (p.epilogue) {
+    case VMI_HY_E_STORE: return norm_rows_epi<VMI_HY_E_STORE>(p, st);
+    case VMI_HY_E_FLOAT: return norm_rows_epi<VMI_HY_E_FLOAT>(p, st);
+    case VMI_HY_E_GLU: return norm_rows_epi<VMI_HY_E_GLU>(p, st);
+    default: return norm_rows_epi<VMI_HY_E_STORE_GLU>(p, st);
+  }
+}
+
+// Whether rows that have been normed by a launch of their own go to held_rows_kernel: its waves' parts of K are whole chunks (a condition around a chunk's products costs the
+// ring).  Up to 2048 columns they are normed for it: 9 and more of them, which resident_kernel's workgroups would norm all each, over too many columns for norm_rows_kernel; at 4096 where
+// norm_first says so.  Both launches, us, the forerunners / now: K 2048, N 12288 8 / 12 / 32 / 40 rows 14.9 / 17.8 / 21.6 / 41.8 -> 14.9 / 15.0 / 17.3 / 17.2,
+// N 20480 19.0 / 22.3 / 26.8 / 47.8 -> 19.9 / 19.9 / 22.2 / 23.5, N 50272 39.4 / 42.3 / 50.4 / 95.1 -> 41.3 / 41.6 / 45.7 / 48.8; K 4096, N 8192 12 / 32 / 40 rows 20.4 / 24.0 / 30.1 -> 18.5 / 23.0 /
+// 22.9, N 24576 32 / 40 rows 50.1 / 48.4 -> 45.4 / 46.9, N 50272 100.5 / 112.4 -> 86.3 / 90.6; K 1024, N 50272 40 rows 49.5 -> 22.1
+bool held_rows_pay(int M, int N, int K) {
+  if (M < 9 || M > 64 || norm_slabs(M, N, K) > 0) return false;
+  return K == 2048 || K == 4096 || (K == 1024 && M > 32);
+}
+
+template <int NCH, int MT, int NB, int EPI>
+static int held_rows_of(const vmi_hy_linear_args& p, hipStream_t st) {
+  auto* fn = held_rows_kernel<NCH, MT, NB, EPI>;
+  const int slabs = p.N >> 4, rb = (p.M + 16 * MT - 1) / (16 * MT), most = 256 / rb / 8 * 8;   // (one workgroup a compute unit in all)
+  if (int rc = allow_lds(fn, HELD_LDS * MT, "vmi_hy_linear")) return rc;
+  hipLaunchKernelGGL(fn, dim3(slabs < most ? blocks8(slabs) : most, rb), dim3(512), HELD_LDS * MT, st, p, slabs);
+  return launched("vmi_hy_linear");
+}
+
+template <int EPI>
+static int held_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch (p.K * 4 + (p.M > 16 ? 2 : 1)) {
+    case 1024 * 4 + 2: return held_rows_of<1, 2, 6, EPI>(p, st);
+    case 2048 * 4 + 1: return held_rows_of<2, 1, 6, EPI>(p, st);
+    case 2048 * 4 + 2: return held_rows_of<2, 2, 6, EPI>(p, st);
+    case 4096 * 4 + 1: return held_rows_of<4, 1, 4, EPI>(p, st);
+    case 4096 * 4 + 2: return held_rows_of<4, 2, 4, EPI>(p, st);
+    default: return fail(VMI_HY_E_ARG, "vmi_hy_linear", "not built");   // (held_rows_pay names no other)
+  }
+}
+
+int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch (p.epilogue) {
+    case VMI_HY_E_STORE: return held_rows_epi<VMI_HY_E_STORE>(p, st);
+    case VMI_HY_E_FLOAT: return held_rows_epi<VMI_HY_E_FLOAT>(p, st);
+    case VMI_HY_E_GLU: return held_rows_epi<VMI_HY_E_GLU>(p, st);
+    default: return held_rows_epi<VMI_HY_E_STORE_GLU>(p, st);
+  }
+}
+
+// linear_kernel / plain_rows_kernel, in a graph of such launches, us: K 1024, N 1024 1 / 16 / 32 / 64 rows 3.7 / 4.0 / 4.1 / 6.4 -> 2.9 / 3.1 / 3.1 / 3.2, K 3072, N 1024 4.8 / 5.4 / 5.5 / 13.0 ->
+// 3.8 / 4.4 / 4.5 / 4.6, K 8192, N 2048 10.7 / 13.3 / 14.2 / 44.5 -> 10.1 / 12.5 / 12.3 / 15.2, K 4096, N 4096 10.1 / 11.3 / 12.4 / 24.6 -> 8.1 / 9.0 / 10.7 / 17.1, K 12288, N 4096 20.8 / 22.5 / 27.9 /
+// 65.2 -> 20.0 / 21.6 / 25.3 / 41.4; 8 groups of K 128, N 512 3.7 / 3.9 / 4.0 / 3.4 -> 2.3 / 2.4 / 2.5 / 2.6, of K 512, N 128 4.0 / 4.5 / 4.5 / 5.1 -> 2.5 / 2.7 / 2.7 / 2.7.  Of more rows there are tiles.
+bool plain_rows_fit(int M) { return M <= 64; }
+
+// Row tiles share a workgroup (and its weights) once there are more workgroups than compute units.  Waves and k-steps a wave by the length of K: four to nine
+// k-steps a wave keep all of its part in flight; past 4608 columns chunks follow each other.
+template <int EPI>
+static int plain_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
+  const int nks = p.K >> 5, slabs = p.N >> 4;
+  auto go = [&](auto* fn, int rw, int j, int mt) {
+    return launch(fn, p, dim3(blocks8(slabs), (p.M + 16 * mt - 1) / (16 * mt), p.groups), 64 * rw, (size_t)rw * plain_stride(j, mt), st);
+  };
+  if ((int64_t)slabs * p.groups * ((p.M + 15) >> 4) <= 256 || p.M <= 16) {
+    if (nks <= 4) return go(plain_rows_kernel<4, 1, 1, 1, EPI>, 4, 1, 1);
+    if (nks <= 8) return go(plain_rows_kernel<4, 2, 1, 1, EPI>, 4, 2, 1);
+    if (nks <= 16) return go(plain_rows_kernel<4, 4, 1, 1, EPI>, 4, 4, 1);
+    if (nks <= 32) return go(plain_rows_kernel<8, 4, 1, 1, EPI>, 8, 4, 1);
+    if (nks <= 64) return go(plain_rows_kernel<8, 8, 1, 1, EPI>, 8, 8, 1);
+    if (nks <= 96) return go(plain_rows_kernel<16, 6, 1, 1, EPI>, 16, 6, 1);
+    if (nks <= 128) return go(plain_rows_kernel<16, 8, 1, 1, EPI>, 16, 8, 1);
+    if (nks <= 144) return go(plain_rows_kernel<16, 9, 1, 1, EPI>, 16, 9, 1);
+    return go(plain_rows_kernel<8, 8, 1, 3, EPI>, 8, 8, 1);
+  }
+  if (nks <= 4) return go(plain_rows_kernel<4, 1, 2, 1, EPI>, 4, 1, 2);
+  if (nks <= 8) return go(plain_rows_kernel<4, 2, 2, 1, EPI>, 4, 2, 2);
+  if (nks <= 16) return go(plain_rows_kernel<4, 4, 2, 1, EPI>, 4, 4, 2);
+  if (nks <= 32) return go(plain_rows_kernel<8, 4, 2, 1, EPI>, 8, 4, 2);
+  if (nks <= 64) return go(plain_rows_kernel<16, 4, 2, 1, EPI>, 16, 4, 2);
+  return go(plain_rows_kernel<16, 4, 2, 2, EPI>, 16, 4, 2);
+}
+
+int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
+  switch (p.epilogue) {
+    case VMI_HY_E_STORE: return plain_rows_epi<VMI_HY_E_STORE>(p, st);
+    case VMI_HY_E_RESIDUAL: return plain_rows_epi<VMI_HY_E_RESIDUAL>(p, st);
+    default: return plain_rows_epi<VMI_HY_E_GATED>(p, st);
+  }
+}
+
+}  // namespace vmi_hybrid

@@ -36,10 +36,13 @@ DENSE_MIN_TOKENS_LARGE, DENSE_LARGE = 17, 32 << 20
 
 
 def dense(tokens: int, w: MatrixTiles, normed: bool = False) -> bool:
-    """normed: the product stands behind a norm, and a kernel that keeps its rows in LDS (linear_resident, where they are not normed by a launch of their
-    own first) is ahead of the vendor's with a launch in front and one behind: 32 tokens, 22528 x 2048 29.9 us against 5.5 + 25.3 + 5.7."""
-    return tokens >= DENSE_MIN_TOKENS or (tokens >= DENSE_MIN_TOKENS_LARGE and w.N * w.K >= DENSE_LARGE
-                                          and not (normed and ops.linear_resident(tokens, w) and not ops.linear_normed_first(tokens, w)))
+    """normed: the product stands behind a norm, and a kernel that keeps its rows in registers (linear_held) or, where they are not normed by a launch of
+    their own first, in LDS (linear_resident) is ahead of the vendor's with a launch in front and one behind: 32 tokens, 22528 x 2048 24 us against 5.5 + 25.3 + 5.7."""
+    if tokens >= DENSE_MIN_TOKENS:
+        return True
+    if tokens < DENSE_MIN_TOKENS_LARGE or w.N * w.K < DENSE_LARGE:
+        return False
+    return not (normed and (ops.linear_held if ops.linear_normed_first(tokens, w) else ops.linear_resident)(tokens, w))
 
 
 def float_product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -69,6 +69,7 @@ SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
+    "vmi_hy_linear_held": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "vmi_hy_add_norm": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp]),
     "vmi_hy_merge": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _f32, _i32, _i32, _vp]),
@@ -259,6 +260,11 @@ def linear_normed_first(M: int, w: MatrixTiles) -> bool:
 def linear_resident(M: int, w: MatrixTiles) -> bool:
     """Whether linear(x, w, norm=...) can keep M rows in LDS, unless it norms them first."""
     return w.groups == 1 and bool(load().vmi_hy_linear_resident(M, w.N, w.K, DTYPES[w.tiles.dtype]))
+
+
+def linear_held(M: int, w: MatrixTiles) -> bool:
+    """Whether linear(x, w, norm=...), which norms M rows first, keeps them in registers then."""
+    return w.groups == 1 and bool(load().vmi_hy_linear_held(M, w.N, w.K, DTYPES[w.tiles.dtype]))
 
 
 def embed(ids: torch.Tensor, table: torch.Tensor, width: int, scale: float) -> torch.Tensor:
