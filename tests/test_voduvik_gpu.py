@@ -417,6 +417,22 @@ def test_recurrence_decodes_like_it_prefills_and_skips_padding_rows(dtype):
     assert torch.equal(k.state[B], untouched)
 
 
+@pytest.mark.parametrize("width,blocks,taps,B", [(96, 1, 4, 1), (2560, 10, 4, 16), (2112, 3, 4, 70), (1536, 2, 4, 33), (288, 9, 6, 40), (4096, 16, 4, 70)])
+def test_single_tokens_share_a_gate_block_over_waves_and_workgroups(width, blocks, taps, B):
+    """rglru_step_kernel with one, two and four tiles of channels a workgroup (the last one's not all there), blocks of fewer and more channels than its waves take at
+    a time, beside rglru_tile_kernel where there are more tiles: two steps, whose tokens come in another order than their entries in the second."""
+    k = _Rglru(width, blocks, taps, torch.bfloat16, slots=B)
+    seqs = [k.inputs(2, 90 + i) for i in range(B)]
+    for t in range(2):
+        order = list(range(B)) if t == 0 else list(range(B))[::-1]
+        step = layout([1] * B, [t] * B, [[0]] * B, 64, flips=[t & 1] * B, pos_slots=False)
+        step.fields["tok_seq"].copy_(i32(order))
+        step.fields["q_start"].copy_(i32(order))
+        got = k.run(torch.cat([seqs[i][2][t:t + 1] for i in order]), step)
+        for at, i in enumerate(order):
+            close(got[at], k.plain(*seqs[i][:2])[t], torch.bfloat16, tol32=1e-4, tol16=3e-2)
+
+
 def test_recurrence_keeps_a_long_memory_in_fp32():
     """Decays near one: after a thousand tokens without input the first token's trace is still there, to fp32 accuracy."""
     k = _Rglru(64, 2, 1, torch.bfloat16, slots=1)

@@ -93,6 +93,12 @@ __device__ __forceinline__ float glu(float g, float u, float limit, float alpha,
 }
 __device__ __forceinline__ float silu(float z) { return z * sigmoid(z); }
 
+// Asks for a kernel argument now (all of them in front of a kernel: one trip to memory; the compiler asks for them branch by branch, a trip each)
+template <class V>
+__device__ __forceinline__ void need(const V& v) {
+  asm volatile("" ::"s"(v));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -354,6 +354,158 @@ __global__ __launch_bounds__(256) void rglru_finish_kernel(const vmi_hy_rglru_ar
   store_out8<T>(p, t, c, o, to_f32<T>(load8(static_cast<const T*>(p.yx) + (int64_t)t * p.ldx + c)));
 }
 
+// A step of single tokens, bfloat16.  A workgroup takes 16 tokens x NO tiles of 16 channels of one gate block; its eight waves share the block's channels, the k of
+// the gate products: a lane convolves eight channels of one token, which is the products' operand as it stands, so nothing goes through LDS but the partial products
+// and the workgroup's own channels.  Tokens are their entries, so what the tables say of a token is asked for at once.  Bound by three trips through memory
+// (tables, states and tails, results) and the launch; rglru_tile_kernel's workgroups, 64 channels each, left most of the chip idle.  Blocks of
+// 256, width 1024, 1 / 12 / 64 tokens 5.7 / 6.7 / 6.9 -> 4.3 / 4.6 / 5.3 us, width 4096, 1 / 12 / 64 5.7 / 7.7 / 8.4 -> 4.4 / 5.3 / 6.8.
+template <int NO, int TAPS>   // TAPS = 0: any number of taps
+__global__ __launch_bounds__(512, 2) void rglru_step_kernel(const vmi_hy_rglru_args p, const vmi_hy_step s) {
+  constexpr int RW = 8, LDU = NO * 16 + 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  f32x4* part = reinterpret_cast<f32x4*>(smem);                     // [RW][NO][2][64]
+  b16* own = reinterpret_cast<b16*>(part + RW * NO * 2 * 64);       // [16][LDU]: this workgroup's channels behind the convolution
+  need(p.yx), need(p.out), need(p.conv_w), need(p.conv_b), need(p.gates), need(p.gate_b), need(p.decay), need(p.state), need(p.tail), need(p.ldx), need(p.ldo), need(p.width),
+      need(p.blocks), need(s.tok_seq), need(s.ctx), need(s.state_slot), need(s.flip), need(s.T), need(s.B);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int taps = TAPS ? TAPS : p.taps, nt = taps - 1;
+  const int bw = p.width / p.blocks, nks = bw >> 5, tiles = bw >> 4, ng = (tiles + NO - 1) / NO;
+  const int blk = blockIdx.x / ng, o0 = blockIdx.x % ng * NO, t0 = blockIdx.y * 16, rows = min(16, s.T - t0);
+  struct Row {
+    int seq, ctx, slot, flip;
+  };
+  auto row_of = [&](int m) {
+    const int t = t0 + min(m, rows - 1), e = min(t, s.B - 1);
+    Row r{s.tok_seq[t], s.ctx[e], s.state_slot[e], s.flip[e]};
+    if (r.seq >= 0 && r.seq != e) r.ctx = s.ctx[r.seq], r.slot = s.state_slot[r.seq], r.flip = s.flip[r.seq];   // (tokens in another order than entries)
+    return r;
+  };
+  const b16* yx = static_cast<const b16*>(p.yx);
+  const b16* tail = static_cast<const b16*>(p.tail);
+  const int t = t0 + min(r16, rows - 1);
+
+  // what needs no table: this lane's inputs and weights of its wave's first k-step, the gates' tiles, what the results need
+  auto channel = [&](int ks) { return blk * bw + 32 * min(ks, nks - 1) + 8 * kc; };
+  V8<b16> x = load8(yx + (int64_t)t * p.ldx + p.width + channel(wave));
+  const b16* gp = static_cast<const b16*>(p.gates) + (int64_t)blk * bw * bw + lane * 8;
+  const int64_t gsz = (int64_t)p.blocks * bw * bw;
+  b16x8 gr[NO], gi[NO];
+  auto load_gates = [&](int ks) {
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      const int64_t at = ((int64_t)min(o0 + o, tiles - 1) * nks + min(ks, nks - 1)) * 512;
+      gr[o] = load8(gp + at), gi[o] = load8(gp + gsz + at);
+    }
+  };
+  const Row mine = row_of(r16);
+  f32x8 cw[TAPS ? TAPS : 1], cb = load8(p.conv_b + channel(wave));
+  if constexpr (TAPS > 0) {
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) cw[j] = load8(p.conv_w + (int64_t)j * p.width + channel(wave));
+  }
+  load_gates(wave);
+  const bool ends = wave < NO && o0 + wave < tiles;   // whether this wave finishes a tile, and which of its channels this lane does
+  const int c = blk * bw + min(o0 + wave, tiles - 1) * 16 + 4 * kc;
+  f32x4 br, bi, dec, S0;
+  b16x4 y;
+  if (ends) {
+    br = *reinterpret_cast<const f32x4*>(p.gate_b + c);
+    bi = *reinterpret_cast<const f32x4*>(p.gate_b + p.width + c);
+    dec = *reinterpret_cast<const f32x4*>(p.decay + c);
+    y = *reinterpret_cast<const b16x4*>(yx + (int64_t)t * p.ldx + c);
+  }
+  const bool live = mine.seq >= 0;
+  const b16* old = tail + ((int64_t)mine.slot * 2 + mine.flip) * nt * p.width;
+  if (ends) S0 = *reinterpret_cast<const f32x4*>(p.state + (int64_t)mine.slot * p.width + c);
+
+  f32x4 ar[NO], ai[NO];
+#pragma unroll
+  for (int o = 0; o < NO; ++o) ar[o] = ai[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ks = wave; ks < nks; ks += RW) {
+    const int ch = channel(ks);
+    f32x8 acc;
+    if constexpr (TAPS > 0) {
+      if (ks > wave) {
+        x = load8(yx + (int64_t)t * p.ldx + p.width + ch);
+        cb = load8(p.conv_b + ch);
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) cw[j] = load8(p.conv_w + (int64_t)j * p.width + ch);
+        load_gates(ks);
+      }
+      b16x8 v[TAPS];
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) v[j] = load8(old + (int64_t)j * p.width + ch);
+      v[TAPS - 1] = x;
+      acc = cb;
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        const bool on = mine.ctx >= TAPS - 1 - j;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(cw[j][e], on ? (float)v[j][e] : 0.f, acc[e]);
+      }
+    } else {
+      if (ks > wave) load_gates(ks);
+      acc = load8(p.conv_b + ch);
+      for (int j = 0; j < taps; ++j) {
+        const b16x8 v = load8(j < nt ? old + (int64_t)j * p.width + ch : yx + (int64_t)t * p.ldx + p.width + ch);
+        const f32x8 w = load8(p.conv_w + (int64_t)j * p.width + ch);
+        const bool on = mine.ctx >= nt - j;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(w[e], on ? (float)v[e] : 0.f, acc[e]);
+      }
+    }
+    const b16x8 u = live ? from_f32<b16>(acc) : zero8<b16>();
+    const int k = 32 * ks + 8 * kc - o0 * 16;
+    if (k >= 0 && k < NO * 16) *reinterpret_cast<b16x8*>(own + r16 * LDU + k) = u;
+#pragma unroll
+    for (int o = 0; o < NO; ++o) mma(ar[o], gr[o], u), mma(ai[o], gi[o], u);
+  }
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    part[((wave * NO + o) * 2) * 64 + lane] = ar[o];
+    part[((wave * NO + o) * 2 + 1) * 64 + lane] = ai[o];
+  }
+  // the convolution's tail, into its other half
+  for (int u = tid; u < rows * nt * 2 * NO; u += 512) {
+    const int k = u % (2 * NO), e = u / (2 * NO) % nt, m = u / (2 * NO) / nt, ch = blk * bw + o0 * 16 + k * 8;
+    const Row r = row_of(m);
+    if (r.seq < 0 || o0 * 16 + k * 8 >= bw) continue;
+    const int64_t at = ((int64_t)r.slot * 2 + r.flip) * nt * p.width + ch, to = ((int64_t)r.slot * 2 + (r.flip ^ 1)) * nt * p.width + ch;
+    const int pos = r.ctx + 1 - nt + e;   // the position this entry stands for
+    V8<b16> v = zero8<b16>();
+    if (e == nt - 1) v = load8(yx + (int64_t)(t0 + m) * p.ldx + p.width + ch);
+    else if (pos >= 0) v = load8(tail + at + (int64_t)(e + 1) * p.width);
+    *reinterpret_cast<V8<b16>*>(static_cast<b16*>(p.tail) + to + (int64_t)e * p.width) = v;
+  }
+  __syncthreads();
+  if (!ends || r16 >= rows) return;
+  f32x4 sr = part[(wave * 2) * 64 + lane], si = part[(wave * 2 + 1) * 64 + lane];
+#pragma unroll
+  for (int w = 1; w < RW; ++w) sr += part[((w * NO + wave) * 2) * 64 + lane], si += part[((w * NO + wave) * 2 + 1) * 64 + lane];
+  const b16x4 u = *reinterpret_cast<const b16x4*>(own + r16 * LDU + wave * 16 + 4 * kc);
+  f32x4 S;
+  b16x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float la = dec[e] * sigmoid(sr[e] + br[e]), a = exp_hw(la);
+    const float b = __builtin_amdgcn_sqrtf(one_minus_exp(-2.f * la, a * a)) * sigmoid(si[e] + bi[e]) * (float)u[e];
+    S[e] = fmaf(a, mine.ctx > 0 ? S0[e] : 0.f, b);
+    o[e] = live ? (b16)(S[e] * gelu_tanh((float)y[e])) : (b16)0.f;
+  }
+  *reinterpret_cast<b16x4*>(static_cast<b16*>(p.out) + (int64_t)(t0 + r16) * p.ldo + c) = o;
+  if (live) *reinterpret_cast<f32x4*>(p.state + (int64_t)mine.slot * p.width + c) = S;
+}
+
+template <int NO>
+static int launch_step(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream_t st) {
+  auto* fn = p.taps == 4 ? rglru_step_kernel<NO, 4> : rglru_step_kernel<NO, 0>;
+  const size_t lds = (size_t)8 * NO * 2 * 1024 + (size_t)16 * (NO * 16 + 8) * 2;
+  if (int rc = allow_lds(fn, lds, "vmi_hy_rglru")) return rc;
+  const int tiles = p.width / p.blocks / 16;
+  hipLaunchKernelGGL(fn, dim3(p.blocks * ((tiles + NO - 1) / NO), (s.T + 15) / 16), dim3(512), lds, st, p, s);
+  return launched("vmi_hy_rglru");
+}
+
 template <typename T, int BM, int TAPS>
 static int launch_tile(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream_t st) {
   auto* fn = rglru_tile_kernel<T, BM, TAPS>;
@@ -365,7 +517,15 @@ static int launch_tile(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStre
 
 template <typename T>
 static int run_rglru(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream_t st) {
-  if (p.single) return p.taps == 4 ? launch_tile<T, 16, 4>(p, s, st) : launch_tile<T, 16, 0>(p, s, st);
+  if constexpr (sizeof(T) == 2) {
+    // as few tiles a workgroup as leave one of them a compute unit, each convolves all of its block's channels; past four, rglru_tile_kernel's 64 channels beside rows in
+    // LDS are as good (width 2048, 256 tokens, 2048 tiles 10.2 us, here 11.2; width 4096, 64 tokens, 1024 tiles 8.4 and 6.8)
+    const int64_t n = (int64_t)(p.width / 16) * ((s.T + 15) / 16);
+    if (p.single && n <= 1024) return n <= 256 ? launch_step<1>(p, s, st) : n <= 512 ? launch_step<2>(p, s, st) : launch_step<4>(p, s, st);
+  }
+  if (p.single) {
+    return p.taps == 4 ? launch_tile<T, 16, 4>(p, s, st) : launch_tile<T, 16, 0>(p, s, st);
+  }
   if (int rc = p.taps == 4 ? launch_tile<T, 64, 4>(p, s, st) : launch_tile<T, 64, 0>(p, s, st)) return rc;
   if (!p.spans) return VMI_HY_OK;
   hipLaunchKernelGGL(rglru_carry_kernel, dim3((p.width + 63) / 64, s.B), dim3(64), 0, st, p, s);

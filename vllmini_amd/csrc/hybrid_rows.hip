@@ -8,11 +8,6 @@
 
 namespace vmi_hybrid {
 
-template <class V>
-__device__ __forceinline__ void need(const V& v) {
-  asm volatile("" ::"s"(v));
-}
-
 template <int EPI>
 __device__ __forceinline__ void need_args(const vmi_hy_linear_args& p) {
   need(p.x), need(p.w), need(p.y), need(p.ldx), need(p.ldy), need(p.M), need(p.N), need(p.K);
