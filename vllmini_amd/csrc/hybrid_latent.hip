@@ -22,6 +22,8 @@ inline size_t attention_lds(int D) {
 template <typename T, int KT, int RT, int NT, int U, bool EXACT>
 __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attention_kernel(const vmi_hy_latent_attention_args p, const vmi_hy_step s) {
   constexpr int R = 16 * RT, TPK = 256 / KT, PAD = pad_of<T>(), LDP = KT + PAD, SW = KT / 16;   // SW waves score
+  need(p.tiles), need(p.q), need(p.cache), need(p.out), need(p.partial), need(p.heads), need(p.rank), need(p.splits), need(p.scale), need(s.ctx), need(s.q_len),
+      need(s.q_start), need(s.table), need(s.table_ld), need(s.page_size), need(s.T);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr bool QREG = EXACT && RT == 1 && sizeof(T) == 2;
   const int D = EXACT ? U * TPK * 8 : p.rank + p.rot, LDK = D + PAD;
@@ -71,9 +73,11 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
 #pragma unroll
     for (int k = 0; k < QK; ++k) qr[k] = load8(static_cast<const T*>(p.q) + (grow0 + min(r16, nrows - 1)) * D + k * 32 + 8 * kc);
   } else {
+    // (rows past the last one repeat it and are not stored; eight units a thread in flight together)
+#pragma unroll 8
     for (int u = tid; u < R * (D >> 3); u += 256) {
       const int m = u / (D >> 3), k = (u - m * (D >> 3)) * 8;
-      *reinterpret_cast<V8<T>*>(qs + m * LDK + k) = m < nrows ? load8(static_cast<const T*>(p.q) + (grow0 + m) * D + k) : zero8<T>();
+      *reinterpret_cast<V8<T>*>(qs + m * LDK + k) = load8(static_cast<const T*>(p.q) + (grow0 + min(m, nrows - 1)) * D + k);
     }
   }
 
@@ -230,6 +234,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s) {
   extern __shared__ float cs[];   // [rot_n / 2][2]
   __shared__ float part[4];
+  need(p.proj), need(p.q), need(p.cache), need(p.norm_w), need(p.freq), need(p.ldp), need(p.heads), need(p.dim), need(p.rot), need(p.rank), need(p.rot_n), need(p.rank_n),
+      need(p.eps), need(s.tok_seq), need(s.tok_pos), need(s.tok_slot);
   const int t = blockIdx.x, tid = threadIdx.x, half = p.rot_n >> 1, hd = p.dim + p.rot, D = p.rank + p.rot;
   const int seq = s.tok_seq[t];
   const int64_t slot = s.tok_slot[t];

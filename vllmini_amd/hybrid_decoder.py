@@ -83,6 +83,8 @@ class HybridDecoder:
         if n_tiles > 128:
             return 1
         max_keys = min(max_keys, kind.chunk) if kind.chunk else max_keys
+        if max_keys <= 2 * self.KEY_TILE:      # (a second tile costs 2 us, the sum over splits 3)
+            return 1
         want = min(self.FILL_WORKGROUPS[row_tiles] // max(n_tiles, 1), -(-max_keys // self.KEY_TILE))
         fit = (256 << 20) // max(1, T * kind.rep * kind.sets * (kind.width + 2) * 4)       # (bytes of the partial results)
         n = 1
@@ -117,7 +119,8 @@ class HybridDecoder:
         plans = []
         for kind in self._kinds:
             rep, longest = kind.rep, int(counts.max()) * kind.rep
-            rt = kind.row_tiles(4 if longest > 32 else 2 if longest > 16 else 1, self.model.dtype)
+            # single tokens: a row tile each, however many heads a token has (one token of 32 heads, 1000 keys in 8 splits 16.1 -> 13.1 us; 256 tokens level)
+            rt = kind.row_tiles(4 if longest > 32 else 2 if longest > 16 else 1, self.model.dtype) if counts.max() > 1 else 1
             per = -(-(counts * rep) // (16 * rt))
             ent = np.repeat(np.arange(b), per)
             first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * 16 * rt
