@@ -99,10 +99,16 @@ VMI_LAYER_API int vmi_gpt2_prompt_attention_f16(const void* qkv, int64_t ld, voi
 VMI_LAYER_API int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const void* gamma, const void* beta, float eps,
                                         void* out, int32_t M, int32_t E, int32_t device, void* stream);
 
+/* y [M, N] = epilogue(x [M, K] w^T + bias) in tiles of many rows (w: w_layout 1, epilogue VMI_LAYER_EPI_BIAS, _BIAS_GELU or _BIAS_RESIDUAL with
+ * res [M, N], which may be y): for hundreds of rows and more, where vmi_gpt2_linear_f16's few-row kernels read the weights for every row tile.
+ * Rows contiguous, x and w 16-byte aligned, y, res and bias 8-byte, N % 16 == 0, K % 64 == 0, x below 4 GiB. */
+VMI_LAYER_API int vmi_gpt2_linear_tiles_f16(const void* x, const void* w, const void* bias, const void* res, void* y, int32_t M, int32_t N, int32_t K,
+                                            int32_t epilogue, int32_t device, void* stream);
+
 /* All layers of whole prompts, the launches of vmi_gpt2_embed_f16, then per layer vmi_gpt2_linear_f16 (norm, c_attn),
  * vmi_gpt2_prompt_attention_f16, vmi_gpt2_linear_f16 (c_proj, residual), (norm, c_fc, GELU), (c_proj, residual), then vmi_gpt2_add_norm_f16 of
  * the prompts' last rows, issued from one call: a prompt of a few dozen tokens takes the GPU less time than sixty calls take an interpreter.
- * (Of many tokens, T times E from 390 000 on, vmi_gpt2_add_norm_f16 and products of tiles stand for the linears behind norms.)
+ * (Of many tokens, T times E from 390 000 at E = 64 to 160 000 at E = 1152, vmi_gpt2_add_norm_f16 and vmi_gpt2_linear_tiles_f16 stand for the linears.)
  * Everything as those entries take it; block_tables [num_layers][num_prompts][table_ld], layer l's weights in layers[l], matrices in
  * w_layout 1.  x, qkv, attended, hidden: scratch of num_tokens rows of E, 3 E, E and 4 E halves, 16-byte aligned; out: [num_prompts, E]. */
 typedef struct {

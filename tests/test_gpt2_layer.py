@@ -706,3 +706,44 @@ def test_the_norm_in_front_holds_rows_whose_mean_is_far_from_zero(M, K):
     want = t + beta.double()
     bound = 2.0 ** -11 * want.abs() + 8 * 2.0 ** -24 * (off / dev_ * gamma.double().abs() + t.abs()) + 2.0 ** -24
     assert bool(((got - want).abs() <= 1.01 * bound).all()), float(((got - want).abs() / bound).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (17, 80, 128), (300, 3088, 320), (1063, 5408, 192), (770, 5392, 128), (1442, 6160, 128), (641, 5920, 576), (323, 5424, 832),
+                                   (481, 5392, 64), (130, 5472, 768), (129, 5552, 1984), (2100, 768, 3072)])
+def test_products_of_many_rows_in_tiles(M, N, K):
+    """tiles_kernel, all nine tiles of its list (128 x 256, 128 x 192, 96 x 256, 96 x 192, 96 x 128, 128 x 128, 64 x 128, and K in two halves 64 x 128 and 64 x 64): rows and
+    columns left over, one chunk of K, an odd number of them, halves of unequal length; every epilogue, the residual in place."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    x, w, b, res = (rnd(M, K) * 1.5 + 0.3).half(), (rnd(N, K) * 0.6 / K ** 0.5).half(), (rnd(N) * 0.1).half(), rnd(M, N).half()
+    for bias, kw in ((None, {}), (b, {"gelu": True}), (b, {"residual": res})):
+        _close(gl.linear_tiles(x, gl.pack_weight(w), bias, **kw), _chain(x, w, bias, None, kw.get("gelu", False), kw.get("residual")), (M, N, K, sorted(kw)))
+
+
+@pytest.mark.gpu
+def test_gelu_of_every_half():
+    """The exact GELU of all 65536 halves, as biases under rows of zeros: within half a unit in the last place of v Phi(v) in 64 bits, up to the float's own error
+    (2^-11 of a unit, some twenty roundings); infinity stays, minus infinity
+    (times a zero) and NaN are NaN, as 0.5 v (1 + erf) has them."""
+    from vllmini_amd import gpt2_layer as gl
+
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    x = torch.zeros((1, 64), dtype=torch.float16, device="cuda:0")
+    w = gl.pack_weight(torch.zeros((4096, 64), dtype=torch.float16, device="cuda:0"))
+    got = torch.cat([gl.linear(x, w, part.cuda(), gelu=True)[0] for part in v.split(4096)]).cpu()
+    fin, d = torch.isfinite(v), v.double()
+    want = d * torch.special.ndtr(d)
+    unit = 2.0 ** (want.abs().clamp_min(2.0 ** -14).log2().floor() - 10)
+    assert bool((((got.double() - want) / unit).abs()[fin] <= 0.5 + 2.0 ** -11).all())
+    assert bool((got[v == float("inf")] == float("inf")).all()) and bool(got[~fin & (v != float("inf"))].isnan().all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,T", [(12, 64, 391), (14, 64, 179), (18, 64, 139), (6, 128, 400), (8, 64, 587)])
+def test_prompts_take_tiles_from_fewer_rows_still_past_a_width_of_768(H, D, T):
+    """As test_prompts_of_many_rows_..., just past the lines T E = 300 000 up to a width of 768 and 160 000 beyond."""
+    test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)

@@ -149,6 +149,19 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// v Phi(v), the exact GELU, of a half's value: Phi(-|v|) = 2^P(|v|), P least squares for log2 Phi(-t) on [0, 6] (weights 1 / (2e-8 + 5e-8 t^3), P(0) = -1), falling without
+// end beyond.  15 instructions where erff takes both its branches: at 2100 rows, N 3072, K 768, whose workgroups have a compute unit each and nothing to hide an epilogue
+// behind, the product 32 -> 21 us (17 without GELU).  Of all halves 333 come out closer to the exact value than 0.5 v (1 + erff) does (up to 2.7 units in the last
+// place off below -3, where 1 + erff cancels) and none further; infinities and NaN as there.
+__device__ __forceinline__ float gelu(float v) {
+  const float t = fabsf(v);
+  float p = -2.5964232e-08f;
+  for (float c : {7.884347e-07f, -1.0245299e-05f, 7.2435578e-05f, -2.6644077e-04f, -2.6124299e-05f, 6.9771572e-03f, -5.2460529e-02f, -4.5921496e-01f, -1.1511048f, -1.f})
+    p = fmaf(p, t, c);
+  const float q = __builtin_amdgcn_exp2f(p);
+  return v * (v >= 0.f ? 1.f - q : q);
+}
+
 // A lane's four consecutive columns n .. n + 3 of row m on their way out; n0: the first column of their slab (scalar).  load() asks early for what
 // store() will need.
 struct Tail {
@@ -156,8 +169,15 @@ struct Tail {
   int64_t slot;   // EPI 3: the row's cache slot, -1 where there is nothing to write
   template <int EPI>
   __device__ __forceinline__ void load(const LinearParams& p, int m, int n, int n0) {
-    bias = res = h16x4{0, 0, 0, 0};
-    if (p.bias != nullptr) bias = *reinterpret_cast<const h16x4*>(p.bias + n);
+    bias = load_bias(p, n);
+    load_row<EPI>(p, m, n, n0);
+  }
+  static __device__ __forceinline__ h16x4 load_bias(const LinearParams& p, int n) {
+    return p.bias != nullptr ? *reinterpret_cast<const h16x4*>(p.bias + n) : h16x4{0, 0, 0, 0};
+  }
+  template <int EPI>
+  __device__ __forceinline__ void load_row(const LinearParams& p, int m, int n, int n0) {
+    res = h16x4{0, 0, 0, 0};
     if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL)
       if (m < p.M) res = *reinterpret_cast<const h16x4*>(p.res + (int64_t)m * p.ldr + n);
     slot = -1;
@@ -171,10 +191,7 @@ struct Tail {
     for (int r = 0; r < 4; ++r) o[r] = (h16)(acc[r] + (float)bias[r]);   // the linear layer's own half output
     if constexpr (EPI == VMI_LAYER_EPI_BIAS_GELU) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = (float)o[r];
-        o[r] = (h16)(0.5f * v * (1.f + erff(v * 0.70710678118654752440f)));
-      }
+      for (int r = 0; r < 4; ++r) o[r] = (h16)gelu((float)o[r]);
     } else if constexpr (EPI == VMI_LAYER_EPI_BIAS_RESIDUAL) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) o[r] = (h16)((float)res[r] + (float)o[r]);
@@ -818,30 +835,35 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
 }
 
 // Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
-// are ahead while rows times width are few: 12 layers of prompts of 128 tokens in us, few-row kernels / tiles, width 256 1024 tokens 490 / 546, 1536 635 / 616;
-// 512 512 541 / 606, 640 684 / 635; 768 384 725 / 759, 512 802 / 799, 1024 1145 / 945; 1024 256 821 / 907, 384 1106 / 969, 1000 2157 / 1206; 1152 256 1063 / 1043,
-// 384 1251 / 1091.  (At the line itself they are level at 768, and tiles some per cent ahead at other widths.)
-static bool many_rows(int T, int E) { return (int64_t)T * E >= 390000 && E % 64 == 0 && 4 * E <= 4608; }
+// are ahead while rows are few, and the wider the rows the sooner they fall behind: 4 layers of prompts of 128 tokens in us, few-row kernels / tiles, width 256 1200
+// tokens 163 / 173, 1500 185 / 183; 512 500 151 / 179, 600 201 / 190; 640 400 205 / 201, 500 218 / 204; 768 350 199 / 214, 400 222 / 215; 896 150 208 / 209, 250 231 / 213;
+// 1024 150 207 / 218, 200 237 / 222, 300 319 / 235; 1152 100 185 / 233, 150 243 / 236, 300 367 / 264.
+static bool many_rows(int T, int E) { return (int64_t)T * E >= (E > 768 ? 160000 : E > 384 ? 300000 : 390000) && E % 64 == 0 && 4 * E <= 4608; }
 
-template <int MI, int NI, int PF>
-static int launch_tiles(const LinearParams& p, int epi, hipStream_t stream) {
-  auto go = [&](auto fn) {
-    hipLaunchKernelGGL(fn, dim3((p.M + 32 * MI - 1) / (32 * MI) * (p.N / (32 * NI))), dim3(256), 0, stream, p);
-    const hipError_t e = hipGetLastError();
-    if (e == hipSuccess) return (int)VMI_LAYER_OK;
-    set_err("launch: ", hipGetErrorString(e));
-    return (int)VMI_LAYER_E_HIP;
-  };
-  switch (epi) {
-    case VMI_LAYER_EPI_BIAS: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS>);
-    case VMI_LAYER_EPI_BIAS_GELU: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS_GELU>);
-    default: return go(tiles_kernel<MI, NI, PF, VMI_LAYER_EPI_BIAS_RESIDUAL>);
-  }
+template <int I, int EPI>
+static int launch_tiles(const LinearParams& p, hipStream_t stream) {
+  constexpr vmi_tiles::Tile T = vmi_tiles::TILES[I];
+  auto* fn = tiles_kernel<T.mi, T.ni, T.ks, T.prio, EPI>;
+  constexpr size_t lds = vmi_tiles::tiles_lds<T.mi, T.ni, T.ks>();
+  static_assert(lds <= 64 * 1024, "no leave needed for the LDS");
+  hipLaunchKernelGGL(fn, dim3(vmi_tiles::tiles_grid(T, p.M, p.N)), dim3(256 * T.ks), lds, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return VMI_LAYER_OK;
+  set_err("launch: ", hipGetErrorString(e));
+  return VMI_LAYER_E_HIP;
 }
-// 64 x 128 where that is a tile for every compute unit, 64 x 64 (more of it in flight) where it is not: 2048 rows, N 768, K 3072 27.4 -> 25.8 us
+template <int EPI, int I = 0>
+static int run_tile(int i, const LinearParams& p, hipStream_t stream) {
+  if constexpr (I < vmi_tiles::NTILES) return i == I ? launch_tiles<I, EPI>(p, stream) : run_tile<EPI, I + 1>(i, p, stream);
+  return VMI_LAYER_E_SHAPE;
+}
 static int run_tiles(const LinearParams& p, int epi, hipStream_t stream) {
-  if (p.N % 128 == 0 && (int64_t)((p.M + 63) / 64) * (p.N / 128) >= 256) return launch_tiles<2, 4, 2>(p, epi, stream);
-  return launch_tiles<2, 2, 4>(p, epi, stream);
+  const int i = vmi_tiles::tiles_pick(p.M, p.N, p.K);
+  switch (epi) {
+    case VMI_LAYER_EPI_BIAS: return run_tile<VMI_LAYER_EPI_BIAS>(i, p, stream);
+    case VMI_LAYER_EPI_BIAS_GELU: return run_tile<VMI_LAYER_EPI_BIAS_GELU>(i, p, stream);
+    default: return run_tile<VMI_LAYER_EPI_BIAS_RESIDUAL>(i, p, stream);
+  }
 }
 
 template <int D, int MI>
@@ -1049,16 +1071,17 @@ int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t* rows, const v
   return after_launch(who, prev, device);
 }
 
-// packed weights, rows of K and N halves
-static int linear_tiles(const char* who, const void* x, const void* w, const void* bias, const void* res, void* y, int M, int N, int K, int epi,
-                        int device, hipStream_t st) {
+int vmi_gpt2_linear_tiles_f16(const void* x, const void* w, const void* bias, const void* res, void* y, int32_t M, int32_t N, int32_t K, int32_t epilogue,
+                              int32_t device, void* stream) {
   using namespace vmi_layer;
-  if (!x || !w || !y || (epi == VMI_LAYER_EPI_BIAS_RESIDUAL && !res)) {
-    set_err(who, ": null pointer");
+  static const char* who = "vmi_gpt2_linear_tiles_f16";
+  if (!x || !w || !y || (epilogue == VMI_LAYER_EPI_BIAS_RESIDUAL && !res) || M <= 0 || N <= 0 || K <= 0 ||
+      (epilogue != VMI_LAYER_EPI_BIAS && epilogue != VMI_LAYER_EPI_BIAS_GELU && epilogue != VMI_LAYER_EPI_BIAS_RESIDUAL)) {
+    set_err(who, ": null pointer, non-positive size or unknown epilogue");
     return VMI_LAYER_E_ARG;
   }
-  if (((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 7)) {
-    set_err(who, ": needs 16-byte aligned rows of x and w, 8-byte aligned rows of y");
+  if ((N & 15) || !vmi_tiles::tiles_fit(M, K, K) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)y & 7) || ((uintptr_t)bias & 7) || ((uintptr_t)res & 7)) {
+    set_err(who, ": needs N % 16 == 0, K % 64 == 0, x below 4 GiB, x and w aligned to 16 bytes, y, res and bias to 8");
     return VMI_LAYER_E_SHAPE;
   }
   LinearParams p{};
@@ -1067,7 +1090,7 @@ static int linear_tiles(const char* who, const void* x, const void* w, const voi
   p.M = M, p.N = N, p.K = K, p.w_packed = 1;
   int prev = -1;
   if (int rc = with_device(who, device, &prev)) return rc;
-  const int rc = run_tiles(p, epi, st);
+  const int rc = run_tiles(p, epilogue, static_cast<hipStream_t>(stream));
   if (prev != device) (void)hipSetDevice(prev);
   return rc;
 }
@@ -1093,7 +1116,7 @@ int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream) {
           if (int e = vmi_gpt2_add_norm_f16(const_cast<void*>(x), nullptr, nullptr, g, beta, a->eps, a->attended, T, E, dev, stream)) return e;
           x = a->attended;
         }
-        return linear_tiles(who, x, m, b, res, y, T, N, K, epi, dev, static_cast<hipStream_t>(stream));
+        return vmi_gpt2_linear_tiles_f16(x, m, b, res, y, T, N, K, epi, dev, stream);
       }
       return vmi_gpt2_linear_f16(x, K, m, b, g, beta, a->eps, res, N, y, N, T, N, K, epi, 1, dev, stream);
     };

@@ -18,6 +18,7 @@
 // a launch in front in 2-byte pieces.  24 prompts of up to 512 tokens (6 146 in all), 12 heads of 64, a layer: 205.6 + 30.2 -> 23.4 us; one
 // prompt of 37: 5.1 + 3.2 -> 3.9 us.
 #pragma once
+#include "mfma_tiles.hpp"
 
 namespace vmi_layer {
 
@@ -308,94 +309,42 @@ __global__ __launch_bounds__(256) void add_norm_kernel(h16* __restrict__ x, cons
   }
 }
 
-// Linear layers of many rows, packed weights: tiles of 32 MI rows and 32 NI columns a workgroup, four waves, 2 x 2.
-//
-// Both operands go through LDS in the matrix cores' own order (a KiB holds a lane's 16 bytes at 16 x lane): packed weights lie that way in
-// memory; of x a wave fetches eight rows' 128 bytes at a time, whole lines (a fragment's gather of 16 rows x 64 bytes takes the
-// addresses four times as long: 12.6 -> 11.9 us at 128 x 128 x 768), and puts them down swizzled.  A chunk is 64 columns of K, requested PF chunks
-// ahead into registers; two buffers, one barrier a chunk.  Bound by LDS and the barrier a chunk (a tile of 64 x 128 takes 0.5 us of it): 40 % of
-// the matrix cores at 8192 rows, where the vendor's kernels reach 60 %, but bias, GELU and residual ride along and one native call issues all.
-// c_attn / c_proj / c_fc / mlp.c_proj of width 768 in us, the few-row kernels -> these: 1500 rows 17 / 10 / 22 / 39 -> 15 / 10 / 20 / 25; 2048 rows 21 / 11 / 28
-// / 47 -> 18 / 10 / 21 / 26; 4096 rows 38 / 20 / 51 / 89 -> 29 / 16 / 40 / 40 (vendor 20 / 12 / 24 / 26, with 150 us of the host a layer).
-constexpr int TKC = 2;   // k-steps (of 32) of a chunk
-
-template <int MI, int NI, int PF, int EPI>
-__global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
-  constexpr int XT = 2 * MI * TKC, WT = 2 * NI * TKC, TILES = XT + WT;   // fragments (KiB) of a chunk
-  constexpr int U = TILES / 4;                                           // of them a wave fetches
-  static_assert(TKC == 2 && XT % 4 == 0 && WT % 4 == 0, "fragments divide over four waves");
-  __shared__ __attribute__((aligned(16))) h16 smem[2][TILES][512];
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kc = lane >> 4, r16 = lane & 15, wm = wave & 1, wn = wave >> 1;
-  // workgroups go to the eight dies in turn: each die takes whole columns of tiles, whose weights it then reads once
-  const int TM = (p.M + 32 * MI - 1) / (32 * MI), all = (int)gridDim.x, die = (int)blockIdx.x & 7;
-  const int tile = die * (all >> 3) + min(die, all & 7) + ((int)blockIdx.x >> 3);
-  const int m0 = tile % TM * 32 * MI, s0 = tile / TM * 2 * NI;   // first row, first slab
-  const int nks = p.K >> 5;
-  // fetch f of a chunk: x first (rows 8 f .. 8 f + 7, 128 bytes each, whole lines: lane 8 r + c brings 16 bytes c of row r), then w (fragment
-  // f - XT, as it lies); this wave does f = wave, wave + 4, ..  The eight lanes of a row write eight fragment rows kc: row r of piece c lies at
-  // r ^ c of its sixteen, so that neither they nor the readers of a fragment meet in a bank
-  const int r8 = lane >> 3, c8 = lane & 7;
-  const h16* src[U];
-  int dst[U];
+// Linear layers of many rows, packed weights (mfma_tiles.hpp): bias, GELU or the residual add on a lane's four columns of a row, the rounding points of the few-row
+// kernels.  The bias is asked for at the start, residuals too where a tile leaves the registers, else a slab's together at the end.
+template <int MI, int NI, int KS, bool PRIO, int EPI>
+__global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const LinearParams p) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  constexpr bool EARLY = MI * NI <= 24 && !PRIO;
+  const int kc = (threadIdx.x & 63) >> 4;
+  h16x4 bias[NI];
+  Tail tail[NI][MI];
+  auto ask = [&](int n, int m, int s) {
 #pragma unroll
-  for (int i = 0; i < U; ++i) {
-    const int f = wave + 4 * i;
-    if (4 * i < XT) {
-      src[i] = p.x + (int64_t)min(m0 + f * 8 + r8, p.M - 1) * p.ldx + 8 * c8;
-      dst[i] = (f >> 1) * 1024 + (f & 1) * 64 + c8 * 128 + (r8 ^ c8) * 8;
-    } else {
-      src[i] = p.w + (((int64_t)(s0 + (f - XT) / TKC) * nks + (f - XT) % TKC) * 64 + lane) * 8;
-      dst[i] = f * 512 + lane * 8;
-    }
-  }
-  h16x8 st[PF][U];
-  auto load = [&](int k, h16x8 (&to)[U]) {   // (past the end: the last chunk again)
-    const int at = min(k, nks - TKC);
-#pragma unroll
-    for (int i = 0; i < U; ++i) to[i] = *reinterpret_cast<const h16x8*>(src[i] + (int64_t)at * (4 * i < XT ? 32 : 512));
+    for (int i = 0; i < MI; ++i) tail[n][i].template load_row<EPI>(p, m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16);
   };
-  f32x4 acc[MI][NI];
+  vmi_tiles::tiles_product<vmi_tiles::Half, MI, NI, KS, PRIO>(
+      p.x, p.ldx, p.w, p.M, p.N, p.K, smem,
+      [&](int m, int s, int SL) {
 #pragma unroll
-  for (int mi = 0; mi < MI; ++mi)
+        for (int n = 0; n < NI; ++n) bias[n] = Tail::load_bias(p, min(s + n, SL - 1) * 16 + 4 * kc);
+        if constexpr (EARLY) {
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int n = 0; n < NI; ++n)
+            if (s + n < SL) ask(n, m, s);   // (scalar)
+        }
+      },
+      [&](const f32x4(&acc)[NI][MI], int m, int s, int SL) {
 #pragma unroll
-  for (int i = 0; i < PF; ++i) load(i * TKC, st[i]);
-  for (int kk = 0; kk < nks; kk += PF * TKC) {
+        for (int n = 0; n < NI; ++n) {
+          if (s + n >= SL) break;   // (scalar)
+          if constexpr (!EARLY) ask(n, m, s);
 #pragma unroll
-    for (int q = 0; q < PF; ++q) {
-      const int k = kk + q * TKC;
-      if (k >= nks) break;
-      h16* to = smem[q & 1][0];
-#pragma unroll
-      for (int i = 0; i < U; ++i) *reinterpret_cast<h16x8*>(to + dst[i]) = st[q][i];
-      load(k + PF * TKC, st[q]);
-      __syncthreads();   // (two buffers: the writes of the next chunk go where the last one was read, which every wave has left behind)
-#pragma unroll
-      for (int j = 0; j < TKC; ++j) {
-        h16x8 xf[MI], wf[NI];
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) xf[mi] = *reinterpret_cast<const h16x8*>(to + ((wm * MI + mi) * TKC + j) * 512 + (kc * 16 + (r16 ^ (4 * j + kc))) * 8);
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) wf[ni] = *reinterpret_cast<const h16x8*>(to + (XT + (wn * NI + ni) * TKC + j) * 512 + lane * 8);
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-          for (int ni = 0; ni < NI; ++ni) acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[ni], xf[mi], acc[mi][ni], 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int mi = 0; mi < MI; ++mi) {
-    const int m = m0 + (wm * MI + mi) * 16 + r16;
-    if (m >= p.M) continue;
-    Tail tail[NI];
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) tail[ni].template load<EPI>(p, m, (s0 + wn * NI + ni) * 16 + 4 * kc, (s0 + wn * NI + ni) * 16);
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) tail[ni].template store<EPI>(p, acc[mi][ni], m, (s0 + wn * NI + ni) * 16 + 4 * kc, (s0 + wn * NI + ni) * 16);
-  }
+          for (int i = 0; i < MI; ++i) {
+            tail[n][i].bias = bias[n];
+            if (m + 16 * i < p.M) tail[n][i].template store<EPI>(p, acc[n][i], m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16);
+          }
+        }
+      });
 }
 
 }  // namespace vmi_layer

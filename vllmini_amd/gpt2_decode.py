@@ -14,7 +14,7 @@ for what the operators are actually batched over:
     (`native_layers`, vllmini_amd/gpt2_layer.py -> csrc/gpt2_layer.hip): LayerNorm + c_attn, c_proj + residual,
     LayerNorm + c_fc + GELU, mlp.c_proj + residual — four launches per layer where the torch modules take eleven
     (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt, layer_norm,
-    gelu), which lm_head always uses, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products.
+    gelu), which lm_head always uses, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products but c_fc.
 
 `reference_off_by_one=True` reproduces the reference caller's seq_lens (length BEFORE the new
 token, scheduler.py:96, so the newest token is not attended); the default attends to it.
@@ -90,10 +90,10 @@ class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
-    # prompts of more tokens in all (times the width's square) take the vendor's products: by the GPU's time alone they are ahead from 400 tokens of width 768
-    # on, but their eight launches a layer take the host 150 us, and that is what such a call waits for.  12 layers of prompts of 128 tokens, native / vendor
-    # in us: width 512 8192 tokens 2065 / 2701; 768 5000 2296 / 2412, 6000 2818 / 2690; 896 2400 1873 / 1967, 4800 2846 / 2703; 1024 1536 1507 / 1942, 3000 2362 / 2218;
-    # 1152 1536 1756 / 1952, 3000 2737 / 2354
+    # prompts of more tokens in all (times the width's square) take the vendor's products but for c_fc with its GELU: by the GPU's time alone they are level from
+    # some 2500 tokens of width 768 on, but their seven launches a layer take the host 150 us, and that is what a call of fewer waits for.  12 layers of prompts of
+    # 128 tokens, native / vendor in us: width 512 4000 tokens 1743 / 2138, 8000 2666 / 2795; 768 1000 1126 / 1847, 3000 1916 / 1981, 5000 2561 / 2544, 6000 2963 / 2910;
+    # 1024 1500 1666 / 1879, 2600 2165 / 2109; 1152 1500 1806 / 1864, 2100 2267 / 2125
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
     NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
@@ -354,7 +354,8 @@ class GPT2PagedDecoder:
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
         """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
         takes four or six launches (the decode step's linear kernels, or norms and tiles) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by
-        one native call, and seven beyond: the vendor's products, and one kernel for the residual add with the norm behind it."""
+        one native call, and six beyond: the vendor's products around one of this build's tiles for c_fc and its GELU (4 layers of 6300 tokens, width 768, 807 us
+        with F.gelu behind the vendor's, 747 so), and one kernel for the residual add with the norm behind it."""
         d, pool, dev, sd = self.dims, self.pool, self.device, self.sd
         H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
         if T == 0:
@@ -381,6 +382,7 @@ class GPT2PagedDecoder:
             h = gpt2_layer.prompts(weights, ends, up["ids"], up["pos"], up["last"], up["tiles"], tile_rows, up["tables"], pool.key_cache,
                                    pool.value_cache, H, d.head_size, d.layer_norm_epsilon, self.scale)
             return F.linear(h, sd["lm_head.weight"])
+        tiles = self.native_layers and d.n_embd % 64 == 0 and T * d.n_embd < 1 << 31
         x, add = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"]), None
         for i in range(d.n_layer):
             p = f"transformer.h.{i}."
@@ -388,7 +390,11 @@ class GPT2PagedDecoder:
             qkv = F.linear(gpt2_layer.add_norm(x, ln_1, add), sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
             a = gpt2_layer.prompt_attention(qkv, up["tiles"], tile_rows, pool.key_cache, pool.value_cache, up["tables"][i], H, self.scale)
             h = gpt2_layer.add_norm(x, ln_2, F.linear(a, sd[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"]))
-            add = self._mlp(h, p)
+            if tiles:
+                h = gpt2_layer.linear_tiles(h, self._packed[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True)
+                add = F.linear(h, sd[p + "mlp.c_proj.weight"], sd[p + "mlp.c_proj.bias"])
+            else:
+                add = self._mlp(h, p)
         x += add
         h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
         return F.linear(h, sd["lm_head.weight"])

@@ -42,6 +42,7 @@ SIGNATURES = {
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
                                                      _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
+    "vmi_gpt2_linear_tiles_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_add_norm_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_prompts_f16": (ctypes.c_int, [ctypes.POINTER(Prompts), _vp]),
     "vmi_gpt2_argmax_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
@@ -154,6 +155,30 @@ def linear(x: torch.Tensor, weight, bias: Optional[torch.Tensor] = None, *,
                                  M, N, K, epi, int(packed), x.device.index or 0, stream)
     if rc != 0:
         raise RuntimeError(lib.vmi_gpt2_layer_last_error().decode("utf-8", "replace"))
+    return out
+
+
+def linear_tiles(x: torch.Tensor, weight: PackedWeight, bias: Optional[torch.Tensor] = None, *, gelu: bool = False,
+                 residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """linear() for hundreds of rows and more (rows and residual contiguous, K a multiple of 64, no norm in front): a new tensor."""
+    lib = load()
+    if x.device.type != "cuda":
+        raise RuntimeError("gpt2_layer.linear_tiles: there is no CPU path")
+    if gelu and residual is not None:
+        raise RuntimeError("gpt2_layer.linear_tiles: gelu and residual are alternative epilogues")
+    if not isinstance(weight, PackedWeight) or weight.tiles.device != x.device:
+        raise RuntimeError("gpt2_layer.linear_tiles: a packed weight on x's device")
+    if x.dim() != 2 or x.dtype != torch.float16 or x.shape[1] != weight.shape[1] or not x.is_contiguous():
+        raise RuntimeError("gpt2_layer.linear_tiles: x half [M, K], contiguous")
+    M, (N, K) = x.shape[0], weight.shape
+    for t, shape, what in ((bias, (N,), "bias [N]"), (residual, (M, N), "residual [M, N]")):
+        if t is not None and (t.dtype != torch.float16 or t.shape != shape or not t.is_contiguous() or t.device != x.device):
+            raise RuntimeError(f"gpt2_layer.linear_tiles: {what} half, contiguous, on x's device")
+    out = torch.empty((M, N), dtype=torch.float16, device=x.device)
+    epi = EPI_BIAS_GELU if gelu else EPI_BIAS_RESIDUAL if residual is not None else EPI_BIAS
+    _check(lib.vmi_gpt2_linear_tiles_f16(x.data_ptr(), weight.tiles.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                         residual.data_ptr() if residual is not None else None, out.data_ptr(), M, N, K, epi, x.device.index or 0,
+                                         torch.cuda.current_stream(x.device).cuda_stream))
     return out
 
 
