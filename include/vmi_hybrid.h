@@ -62,6 +62,10 @@ typedef struct {
   int32_t x_kind, epilogue, dtype, device;
 } vmi_hy_linear_args;
 VMI_HY_API int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream);
+/* The same for bfloat16 rows by the hundred (x_kind X_ROWS, one group, K % 64 == 0, epilogue E_GLU or E_STORE_GLU), in tiles of the matrix cores */
+VMI_HY_API int vmi_hy_linear_tiles(const vmi_hy_linear_args* a, void* stream);
+/* Whether it takes such a product (rows of K elements one behind the other) and is ahead of a library product and vmi_hy_glu behind it */
+VMI_HY_API int32_t vmi_hy_linear_tiles_pay(int32_t M, int32_t N, int32_t K, int32_t n_split, int32_t dtype);
 /* Whether a product of these sizes behind a norm is faster over rows normed beforehand (`normed`) */
 VMI_HY_API int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype);
 /* Whether the rows of a product of these sizes behind a norm can stay in LDS, normed on their way there: then the product is ahead of a norm, a library

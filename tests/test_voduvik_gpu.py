@@ -251,6 +251,43 @@ def _norm_products(M, N, K):
     return t
 
 
+@pytest.mark.parametrize("M,N,K,split", [(1, 16, 64, 0), (17, 96, 128, 32), (300, 3088, 320, 16), (1063, 5408, 192, 5408 - 32), (770, 5392, 128, 0), (1442, 6160, 128, 4096), (641, 5920, 576, 48),
+                                         (323, 5424, 832, 0), (481, 5392, 64, 2048), (130, 5472, 768, 0), (129, 5552, 1984, 64), (2100, 768, 3072, 256)])
+def test_many_rows_in_tiles_with_the_gated_unit_behind(M, N, K, split):
+    """vmi_hy_linear_tiles, all nine tiles: rows and columns left over, one chunk of K, an odd number of them, halves of unequal length; the line between columns as they
+    are and gated ones inside tiles; outputs that are columns of wider tensors, whose others stay as they were."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M + N + K)
+    x, w = (torch.randn(*s, generator=g, device=dev()) for s in ((M, K), (N, K)))
+    N = ops.pad32(N)
+    t = ops.MatrixTiles(w / K ** 0.5, torch.bfloat16, dense=True)
+    x = torch.cat([x, x], 1).to(torch.bfloat16)[:, K:]
+    y = x.double() @ t.dense.double().T
+    for unit in (ops.SILU_UNIT, ops.GatedUnit.clamped(0.7)):
+        wide = torch.full((M, (N - split) // 2 + 24), 7.0, dtype=torch.bfloat16, device=dev())
+        out = ops.linear_tiles(x, t, unit, split, wide[:, 8:-16])
+        a, b = y[:, split::2].clamp(max=unit.limit), y[:, split + 1::2].clamp(-unit.limit, unit.limit)
+        # (half a unit of bfloat16, and float32 sums of K products: 1e-3 is far more than those)
+        want = a * torch.sigmoid(unit.alpha * a) * (b + unit.up)
+        assert bool(((wide[:, 8:-16].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all())
+        assert bool((wide[:, :8] == 7).all()) and bool((wide[:, -16:] == 7).all())
+        if split:
+            assert out.shape == (M, split) and bool(((out.double() - y[:, :split]).abs() <= 2.0 ** -8 * y[:, :split].abs() + 1e-3).all())
+
+
+def test_many_rows_in_tiles_refuse_what_is_not_built():
+    from vllmini_amd import hybrid_ops as ops
+
+    x, t = torch.zeros((64, 128), dtype=torch.bfloat16, device=dev()), ops.MatrixTiles(torch.zeros((64, 128), device=dev()), torch.bfloat16)
+    for bad in (lambda: ops.linear_tiles(x.float(), t, ops.SILU_UNIT), lambda: ops.linear_tiles(x[:, :96], t, ops.SILU_UNIT), lambda: ops.linear_tiles(x, t, ops.SILU_UNIT, 8),
+                lambda: ops.linear_tiles(x[:, :96], ops.MatrixTiles(torch.zeros((64, 96), device=dev()), torch.bfloat16), ops.SILU_UNIT),
+                lambda: ops.linear_tiles(x, t, ops.SILU_UNIT, 32, x[:, :32]), lambda: ops.linear_tiles(x, ops.MatrixTiles(torch.zeros((64, 128), device=dev()), torch.float32), ops.SILU_UNIT)):
+        with pytest.raises(RuntimeError):
+            bad()
+    assert not ops.linear_tiles_pay(300, ops.MatrixTiles(torch.zeros((64, 96)), torch.bfloat16)) and not ops.linear_tiles_pay(300, ops.MatrixTiles(torch.zeros((64, 128)), torch.float32))
+
+
 @pytest.mark.parametrize("dtype", BOTH)
 def test_products_that_are_not_built_are_refused(dtype):
     """Inputs and epilogues that vmi_hy_linear has no kernel for: an error and nothing written, whether or not there is room for normed rows."""

@@ -149,6 +149,13 @@ constexpr Tile TILES[] = {{8, 4, 1, false, .90f, .83f}, {8, 3, 1, false, .77f, .
                           {8, 2, 1, false, .50f, .50f}, {4, 2, 1, false, .44f, .30f}, {4, 2, 2, false, .39f, .34f}, {4, 1, 2, false, .27f, .22f}};
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 
+// us, as the chip's tiles are dealt
+inline float tiles_cost(int i, int M, int N, int K) {
+  const Tile& t = TILES[i];
+  const int64_t n = (int64_t)((M + 16 * t.mi - 1) / (16 * t.mi)) * ((N + 64 * t.ni - 1) / (64 * t.ni)), share = (n + 255) / 256;
+  return (share == 1 ? t.alone : share * t.beside) * ((float)(K >> 6) + (t.ks == 2 ? 9.5f : 6.f));
+}
+
 // The tile whose largest share of a compute unit ends first: so many tiles one behind the other, each 64 columns of K at a time and as long as 6 such at its ends (9.5
 // where two halves meet).  On average 0.5 per cent behind the best of the list over those 258 products, 11 at most.  (us, 128 x 256 / 128 x 192 / 96 x 256 / 64 x 128: 2770
 // rows, N 2048, K 6144 86 / 69 / 75 / 89, of 176 / 242 / 232 / 704 tiles; 2100 rows, N 768, K 768 16 / 13 / 13 / 7.)
@@ -156,9 +163,7 @@ inline int tiles_pick(int M, int N, int K) {
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < NTILES; ++i) {
-    const Tile& t = TILES[i];
-    const int64_t n = (int64_t)((M + 16 * t.mi - 1) / (16 * t.mi)) * ((N + 64 * t.ni - 1) / (64 * t.ni)), share = (n + 255) / 256;
-    const float cost = (share == 1 ? t.alone : share * t.beside) * ((float)(K >> 6) + (t.ks == 2 ? 9.5f : 6.f));
+    const float cost = tiles_cost(i, M, N, K);
     if (i == 0 || cost < least) best = i, least = cost;
   }
   return best;

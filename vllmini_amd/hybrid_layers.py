@@ -18,7 +18,7 @@ What a decoder asks of a mixer: page_rows() and state_shapes(), the cache tensor
 The residual stream is float32 (`Residual`).  Steps of few tokens run on the streaming kernels with everything fused around the
 products (norm in front, gated unit / head gate / residual add behind); from DENSE_MIN_TOKENS tokens on (from DENSE_MIN_TOKENS_LARGE
 for matrices of DENSE_LARGE elements, unless the kernel behind a norm can keep its rows in LDS) the products go to the vendor library (F.linear, as the prefill of the GPT-2 decoder does)
-with one elementwise kernel between two of them.
+with one elementwise kernel between two of them, those with a gated unit behind them to tiles of this build's own where these are ahead (gated_product).
 """
 from __future__ import annotations
 
@@ -269,6 +269,15 @@ class RGLRU:
         res.branch_out(o, self.w_o, step)
 
 
+def gated_product(h: torch.Tensor, w: MatrixTiles, unit: GatedUnit, split: int = 0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """h W^T of many rows, the columns from `split` on through the gated unit (into `out`); the columns below, or with split = 0 the unit's."""
+    if ops.linear_tiles_pay(h.shape[0], w, split):
+        return ops.linear_tiles(h, w, unit, split, out)
+    proj = F.linear(h, w.dense)
+    gated = ops.glu(proj[:, split:], unit, out=out)
+    return proj if split else gated
+
+
 class ClampedGLU:
     """gate, up [ff, E], down [E, ff]."""
 
@@ -282,7 +291,7 @@ class ClampedGLU:
 
     def run(self, res: Residual, step: StepLayout) -> None:
         if dense(step.T, self.w_in, True):
-            h = ops.glu(F.linear(res.normed(self.norm), self.w_in.dense), self.unit)
+            h = gated_product(res.normed(self.norm), self.w_in, self.unit)
         else:
             h = ops.linear(res.settle(), self.w_in, norm=self.norm.args, glu=self.unit)
         res.branch_out(h, self.w_out, step)
@@ -510,9 +519,8 @@ class ParallelBlock:
         T, m = step.T, self.n_mix
         rows = torch.empty((T, m + self.ff), dtype=self.dtype, device=res.x.device)      # [mixer cores | gated unit]
         if dense(T, self.w_in, True):
-            proj = F.linear(res.normed(self.norm), self.w_in.dense)
-            if self.ff:
-                ops.glu(proj[:, self.n_in:], self.unit, out=rows[:, m:])
+            h = res.normed(self.norm)
+            proj = gated_product(h, self.w_in, self.unit, self.n_in, rows[:, m:]) if self.ff else F.linear(h, self.w_in.dense)
         else:
             proj = ops.linear(res.settle(), self.w_in, norm=self.norm.args, **(
                 {"glu": self.unit, "glu_from": self.n_in, "glu_out": rows[:, m:]} if self.ff else {}))

@@ -67,6 +67,8 @@ GqaArgs = _struct("GqaArgs", [(_vp, "q cache out bias sink gate tiles partial"),
 
 SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
+    "vmi_hy_linear_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
+    "vmi_hy_linear_tiles_pay": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_held": (_i32, [_i32, _i32, _i32, _i32]),
@@ -244,6 +246,36 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
                    x_kind=kind, epilogue=epi, dtype=DTYPES[T], device=device)
     _check(lib.vmi_hy_linear(ctypes.byref(a), stream))
     return out
+
+
+def linear_tiles(x: torch.Tensor, w: MatrixTiles, unit: GatedUnit, split: int = 0, glu_out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The product of hundreds of bfloat16 rows and more (K a multiple of 64): columns from `split` on, interleaved (gate, up), through the gated unit into glu_out
+    [M, (N - split) / 2] (default: a new tensor), those below it as they are into a new tensor.  Returns the latter, or with split = 0 the former."""
+    device, stream = _on(x)
+    M, N, K = int(x.shape[0]), w.N, w.K
+    _need(w.groups == 1 and w.tiles.dtype == torch.bfloat16 and w.tiles.device == x.device, "hybrid_ops.linear_tiles: one bfloat16 matrix on x's device")
+    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, f"hybrid_ops.linear_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
+    _need(0 <= split <= N and split % 16 == 0, "hybrid_ops.linear_tiles: split")
+    if glu_out is None:
+        glu_out = torch.empty((M, (N - split) // 2), dtype=x.dtype, device=x.device)
+    _need(glu_out.dim() == 2 and glu_out.shape == (M, (N - split) // 2) and glu_out.stride(1) == 1 and glu_out.dtype == x.dtype and glu_out.device == x.device,
+          "hybrid_ops.linear_tiles: glu_out")
+    y = torch.empty((M, split), dtype=x.dtype, device=x.device) if split else glu_out
+    a = LinearArgs(x=x.data_ptr(), w=w.tiles.data_ptr(), y=y.data_ptr(), y2=glu_out.data_ptr(), ldx=x.stride(0), ldy=y.stride(0), ldy2=glu_out.stride(0), M=M, N=N, K=K,
+                   groups=1, n_split=split, scale=unit.limit, glu_alpha=unit.alpha, glu_up=unit.up, x_kind=X_ROWS, epilogue=E_STORE_GLU if split else E_GLU,
+                   dtype=DTYPES[x.dtype], device=device)
+    _check(load().vmi_hy_linear_tiles(ctypes.byref(a), stream))
+    return y
+
+
+def linear_tiles_pay(M: int, w: MatrixTiles, split: int = 0) -> bool:
+    """Whether linear_tiles takes M contiguous rows and is ahead of the vendor's product and glu() behind it."""
+    return w.groups == 1 and _tiles_pay(M, w.N, w.K, split, w.tiles.dtype)
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles_pay(M: int, N: int, K: int, split: int, dtype: torch.dtype) -> bool:
+    return bool(load().vmi_hy_linear_tiles_pay(M, N, K, split, DTYPES[dtype]))
 
 
 @functools.lru_cache(maxsize=4096)
