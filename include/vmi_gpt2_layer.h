@@ -76,6 +76,10 @@ VMI_LAYER_API int vmi_gpt2_linear_qkv_cache_f16(const void* x, int64_t ldx, cons
  * (torch.argmax's tie rule; row stride ld elements, any alignment). */
 VMI_LAYER_API int vmi_gpt2_embed_f16(const int64_t* input_ids, const int64_t* position_ids, const void* wte, const void* wpe,
                                      void* out, int32_t num_tokens, int32_t hidden, int32_t device, void* stream);
+/* What a step's launches read: head_bytes (a multiple of 16) from `host`, pinned memory, to the same place in `dev`, behind them the first `used` of `ld` whole numbers
+ * (int32) of each of `rows` rows; and ids_out[0:n] = ids[0:n].  16-byte aligned; the host memory is read when the launch runs. */
+VMI_LAYER_API int vmi_gpt2_step_inputs(const void* host, void* dev, int64_t head_bytes, int32_t rows, int32_t ld, int32_t used, const int64_t* ids, int64_t* ids_out,
+                                       int32_t n, int32_t device, void* stream);
 VMI_LAYER_API int vmi_gpt2_argmax_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int64_t* out,
                                       int32_t device, void* stream);
 

@@ -76,6 +76,10 @@ VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32
  * library product and what follows it as well. */
 VMI_HY_API int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype);
 
+/* What a step's launches read: `bytes` (a multiple of 16) from `host`, pinned memory, to `dev`; and ids_out[0:n] = ids[0:n].  16-byte aligned; the host memory
+ * is read when the launch runs. */
+VMI_HY_API int vmi_hy_step_inputs(const void* host, void* dev, int64_t bytes, const int64_t* ids, int64_t* ids_out, int32_t n, int32_t device, void* stream);
+
 /* x[t, 0:width) = table[ids[t]] * scale (bfloat16 table of row length ld), zeros up to ld; float32 out */
 VMI_HY_API int vmi_hy_embed(const int64_t* ids, const void* table, float* x, int32_t T, int32_t width, int32_t ld, int32_t vocab,
                             float scale, int32_t device, void* stream);

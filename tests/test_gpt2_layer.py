@@ -747,3 +747,28 @@ def test_gelu_of_every_half():
 def test_prompts_take_tiles_from_fewer_rows_still_past_a_width_of_768(H, D, T):
     """As test_prompts_of_many_rows_..., just past the lines T E = 300 000 up to a width of 768 and 160 000 beyond."""
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head,rows,ld,used,n", [(0, 0, 0, 0, 1), (16, 3, 5, 5, 0), (4080, 1, 64, 1, 0), (4096, 384, 64, 13, 32), (48, 7, 9, 0, 300), (1 << 20, 1000, 33, 32, 5)])
+def test_a_steps_inputs_go_where_its_launches_read_them(head, rows, ld, used, n):
+    """step_inputs: the head, the columns that count and the ids arrive, everything else stays; the pinned memory may be written again after wait()."""
+    from vllmini_amd import gpt2_layer as gl
+    from vllmini_amd.staging import PinnedBuffer
+
+    dev = torch.device("cuda:0")
+    buf, size = PinnedBuffer(head + rows * ld * 4 + 16), head + rows * ld * 4 + 16
+    ids = torch.arange(100, 100 + n, device=dev)
+    for turn in (1, 2):
+        buf.wait()
+        buf.tensor.copy_(torch.randint(0, 255, (size,), dtype=torch.uint8, generator=torch.Generator().manual_seed(turn)))
+        to, out = torch.full((size,), 255, dtype=torch.uint8, device=dev), torch.full((n + 2,), -1, dtype=torch.int64, device=dev)
+        gl.step_inputs(buf, to, head, rows, ld, used, ids if n else None, out)
+        want = torch.full((size,), 255, dtype=torch.uint8)
+        want[:head] = buf.tensor[:head]
+        want[head:head + rows * ld * 4].view(rows, ld * 4)[:, : used * 4] = buf.tensor[head:head + rows * ld * 4].view(rows, ld * 4)[:, : used * 4]
+        assert torch.equal(to.cpu(), want) and out.tolist() == [*range(100, 100 + n), -1, -1]
+    with pytest.raises(RuntimeError):
+        gl.step_inputs(buf, to, head + 32, rows, ld, used, None, out)
+    with pytest.raises(RuntimeError):
+        gl.step_inputs(buf, to, head, rows, ld, used, ids.int() if n else out.int(), out)

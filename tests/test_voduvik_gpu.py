@@ -59,6 +59,22 @@ def layout(counts, ctx, tables, page, slots=None, flips=None, pos_slots=True):
                           int((ctx + counts).max()))
 
 
+@pytest.mark.parametrize("ints,n", [(4, 1), (1028, 0), (1 << 15, 300)])
+def test_a_steps_inputs_arrive(ints, n):
+    from vllmini_amd import hybrid_ops as ops
+    from vllmini_amd.staging import PinnedBuffer
+
+    buf, ids = PinnedBuffer(4 * ints + 64), torch.arange(7, 7 + n, device=dev())
+    for turn in (1, 2):
+        buf.wait()
+        buf.tensor.copy_(torch.randint(0, 255, buf.tensor.shape, dtype=torch.uint8, generator=torch.Generator().manual_seed(turn)))
+        to, out = torch.zeros(ints, dtype=torch.int32, device=dev()), torch.full((n + 2,), -1, dtype=torch.int64, device=dev())
+        ops.step_inputs(buf, to, ids, out)
+        assert torch.equal(to.cpu(), buf.tensor[: 4 * ints].view(torch.int32)) and out.tolist() == [*range(7, 7 + n), -1, -1]
+    with pytest.raises(RuntimeError):
+        ops.step_inputs(buf, torch.zeros(ints + 20, dtype=torch.int32, device=dev()), ids, out)
+
+
 # ---- linear layers ---------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("M", [1, 5, 17, 40, 130])

@@ -23,6 +23,7 @@
 
 #include <string>
 
+#include "step_inputs.hpp"
 #include "vmi_gpt2_layer.h"
 
 namespace vmi_layer {
@@ -996,6 +997,20 @@ static int after_launch(const char* who, int prev, int32_t device) {
     return VMI_LAYER_E_HIP;
   }
   return VMI_LAYER_OK;
+}
+
+int vmi_gpt2_step_inputs(const void* host, void* dev, int64_t head_bytes, int32_t rows, int32_t ld, int32_t used, const int64_t* ids, int64_t* ids_out, int32_t n,
+                         int32_t device, void* stream) {
+  using namespace vmi_layer;
+  const vmi_step::Inputs p{static_cast<const char*>(host), static_cast<char*>(dev), head_bytes, rows, ld, used, n, ids, ids_out};
+  if (!vmi_step::inputs_fit(p)) {
+    g_err = "vmi_gpt2_step_inputs: null pointer, a size out of range, or memory that is not aligned to 16 bytes";
+    return VMI_LAYER_E_ARG;
+  }
+  int prev = -1;
+  if (int rc = with_device("vmi_gpt2_step_inputs", device, &prev)) return rc;
+  vmi_step::launch_inputs(p, static_cast<hipStream_t>(stream));
+  return after_launch("vmi_gpt2_step_inputs", prev, device);
 }
 
 int vmi_gpt2_embed_f16(const int64_t* input_ids, const int64_t* position_ids, const void* wte, const void* wpe, void* out,

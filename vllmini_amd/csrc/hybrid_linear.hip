@@ -10,6 +10,7 @@
 
 #include "hybrid_common.hpp"
 #include "hybrid_linear.hpp"
+#include "step_inputs.hpp"
 
 namespace vmi_hybrid {
 
@@ -713,6 +714,16 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
     return linear_normed(rows, st);
   }
   return a->dtype == VMI_HY_BF16 ? linear_kind<b16>(*a, st) : linear_kind<float>(*a, st);
+}
+
+int vmi_hy_step_inputs(const void* host, void* dev_to, int64_t bytes, const int64_t* ids, int64_t* ids_out, int32_t n, int32_t device, void* stream) {
+  static const char* who = "vmi_hy_step_inputs";
+  const vmi_step::Inputs p{static_cast<const char*>(host), static_cast<char*>(dev_to), bytes, 0, 0, 0, n, ids, ids_out};
+  if (!vmi_step::inputs_fit(p)) return fail(VMI_HY_E_ARG, who, "null pointer, a size out of range, or memory that is not aligned to 16 bytes");
+  DeviceScope dev(device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  vmi_step::launch_inputs(p, static_cast<hipStream_t>(stream));
+  return launched(who);
 }
 
 int vmi_hy_embed(const int64_t* ids, const void* table, float* x, int32_t T, int32_t width, int32_t ld, int32_t vocab, float scale,

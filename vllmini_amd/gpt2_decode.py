@@ -35,6 +35,7 @@ import torch.nn.functional as F
 
 from . import cache_ops, gpt2_layer, ops
 from .kv_pool import PagedKVPool
+from .staging import PinnedBuffer
 
 
 @dataclasses.dataclass(frozen=True)
@@ -483,15 +484,15 @@ class GPT2PagedDecoder:
         cur = self._sets.get(B)
         if cur is None:
             L, MB, dev = self.dims.n_layer, self.pool.max_blocks_per_seq, self.device
-            # tables, slots, lengths and positions live in ONE device buffer (8-byte aligned sections, typed views): a step
-            # uploads them with one copy instead of four (4 x ~4 us of copy kernels per token: 3 % of a batch-1 token)
+            # tables, slots, lengths and positions live in ONE device buffer (16-byte aligned sections, typed views): a step
+            # uploads them with one launch or copy instead of four (4 x ~4 us of copy kernels per token: 3 % of a batch-1 token)
             sections = (("slots", (L, B), torch.int64), ("position_ids", (B,), torch.int64),
-                        ("tables", (L, B, MB), torch.int32), ("seq_lens", (B,), torch.int32))
+                        ("seq_lens", (B,), torch.int32), ("tables", (L, B, MB), torch.int32))
             offs, total = {}, 0
             for name, shape, dt in sections:
                 nbytes = int(np.prod(shape)) * torch.empty((), dtype=dt).element_size()
                 offs[name] = (total, nbytes)
-                total += (nbytes + 7) // 8 * 8
+                total += (nbytes + 15) // 16 * 16
 
             def views(buf):
                 return {name: buf[offs[name][0]:offs[name][0] + offs[name][1]].view(dt).view(shape) for name, shape, dt in sections}
@@ -507,10 +508,10 @@ class GPT2PagedDecoder:
             # of GPU work, ran 3.06 ms that way).  From pinned memory the copy is truly asynchronous and the host
             # prepares step i+1 while the GPU runs step i; a buffer is reused only after its own copy has executed.
             if dev.type == "cuda":
-                cur["stage_buf"] = [torch.empty(total, dtype=torch.uint8, pin_memory=True) for _ in range(2)]
-                cur["stage"] = [{k: v.numpy() for k, v in views(b).items()} for b in cur["stage_buf"]]
-                cur["stage_ev"] = [None, None]
+                cur["stage_buf"] = [PinnedBuffer(total) for _ in range(2)]
+                cur["stage"] = [{k: v.numpy() for k, v in views(b.tensor).items()} for b in cur["stage_buf"]]
                 cur["stage_i"] = 0
+                cur["head"] = offs["tables"][0]
             self._sets[B] = cur
         self._cur = cur
         self._static = cur["static"]
@@ -537,6 +538,7 @@ class GPT2PagedDecoder:
         positions = np.fromiter((self.pool.seq_len(s) for s in seq_ids), dtype=np.int64, count=B)  # scheduler.py:81
         tables, slots, ctx = self.pool.decode_step_batch(seq_ids)
         lens = ctx - 1 if self.reference_off_by_one else ctx
+        ids = None
         host = {"tables": tables, "slots": slots, "seq_lens": lens.astype(np.int32), "position_ids": positions}
         if cur["stage"] is None:
             for k, a in host.items():
@@ -547,8 +549,8 @@ class GPT2PagedDecoder:
                     pad.fill_(-1 if k in ("tables", "slots") else 0)
         else:
             i = cur["stage_i"]
-            if cur["stage_ev"][i] is not None:
-                cur["stage_ev"][i].synchronize()          # this set's previous uploads have run
+            buf = cur["stage_buf"][i]
+            buf.wait()                                    # this set's previous uploads have run
             sg = cur["stage"][i]
             sg["tables"][:, :B] = tables
             sg["slots"][:, :B] = slots
@@ -559,10 +561,15 @@ class GPT2PagedDecoder:
                 sg["slots"][:, B:] = -1
                 sg["seq_lens"][B:] = 0
                 sg["position_ids"][B:] = 0
-            cur["meta"].copy_(cur["stage_buf"][i], non_blocking=True)
-            ev = torch.cuda.Event()
-            ev.record()
-            cur["stage_ev"][i] = ev
+            if self.native_layers:      # (one launch: the columns of the tables that count, and the tokens where they are a tensor beside them)
+                if isinstance(input_ids, torch.Tensor) and input_ids.device == st["input_ids"].device and input_ids.dtype == torch.long \
+                        and input_ids.shape == (B,) and input_ids.is_contiguous():
+                    ids = input_ids
+                used = min(-(-max(int(ctx.max()), 1) // self.pool.block_size), tables.shape[2])
+                gpt2_layer.step_inputs(buf, cur["meta"], cur["head"], self.dims.n_layer * Bp, tables.shape[2], used, ids, st["input_ids"])
+            else:
+                cur["meta"].copy_(buf.tensor, non_blocking=True)
+                buf.read()
             cur["stage_i"] = i ^ 1
         # the lengths are known here on the host: let the library's heuristic see the batch's true longest and mean
         # length (a ragged batch gets the many-waves-per-head decomposition, vmi_paged_attention_v1_pick_variant_hint)
@@ -587,7 +594,9 @@ class GPT2PagedDecoder:
                                 for_append="read" if self.deferred_scatter else self.fused_append):
             st["variant"] = 0
         ids_dst = st["input_ids"][:B]
-        if isinstance(input_ids, torch.Tensor):
+        if ids is not None:
+            pass                                          # (they are there)
+        elif isinstance(input_ids, torch.Tensor):
             ids_dst.copy_(input_ids.to(torch.long), non_blocking=True)
         else:
             ids_dst.copy_(torch.as_tensor(list(input_ids), dtype=torch.long), non_blocking=True)

@@ -18,6 +18,7 @@ import numpy as np
 import torch
 
 from . import build as _build
+from .staging import PinnedBuffer
 
 ABI_VERSION = 1
 EPI_BIAS, EPI_BIAS_GELU, EPI_BIAS_RESIDUAL, EPI_BIAS_KV_CACHE = 0, 1, 2, 3
@@ -40,6 +41,7 @@ SIGNATURES = {
     "vmi_gpt2_linear_qkv_cache_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i64, _i32, _i32, _i32,
                                                      _vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
+    "vmi_gpt2_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp]),
     "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
                                                      _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_linear_tiles_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
@@ -231,6 +233,19 @@ def linear_qkv_cache(x: torch.Tensor, weight, bias: Optional[torch.Tensor], key_
 def _check(rc: int) -> None:
     if rc != 0:
         raise RuntimeError(load().vmi_gpt2_layer_last_error().decode("utf-8", "replace"))
+
+
+def step_inputs(host: PinnedBuffer, dev: torch.Tensor, head: int, rows: int, ld: int, used: int, ids: Optional[torch.Tensor], ids_out: torch.Tensor) -> None:
+    """The first `head` bytes of `host` into `dev`, behind them the first `used` of the `ld` int32 of each of `rows` rows; ids (if any) into the start of ids_out."""
+    if not dev.is_contiguous() or min(host.tensor.numel(), dev.numel() * dev.element_size()) < head + rows * ld * 4:
+        raise RuntimeError("gpt2_layer.step_inputs: host and device memory hold the head and the rows")
+    if ids is not None and not (ids.dtype == ids_out.dtype == torch.int64 and ids.is_contiguous() and ids_out.is_contiguous() and ids.device == dev.device == ids_out.device
+                                and ids.numel() <= ids_out.numel()):
+        raise RuntimeError("gpt2_layer.step_inputs: int64 ids beside what they are copied to")
+    with torch.cuda.device(dev.device):
+        _check(load().vmi_gpt2_step_inputs(host.tensor.data_ptr(), dev.data_ptr(), head, rows, ld, used, ids.data_ptr() if ids is not None else None, ids_out.data_ptr(),
+                                           ids.numel() if ids is not None else 0, dev.device.index or 0, torch.cuda.current_stream(dev.device).cuda_stream))
+        host.read()
 
 
 def embed(input_ids: torch.Tensor, position_ids: torch.Tensor, wte: torch.Tensor, wpe: torch.Tensor,

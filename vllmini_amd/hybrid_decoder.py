@@ -19,6 +19,7 @@ import torch
 from . import hybrid_ops as ops
 from .hybrid_layers import AttentionPlan, ClampedGLU, ConcatProjection, Head, LatentAttention, ParallelBlock, QueryTiling, Residual, RGLRU
 from .kv_pool import PagedKVPool
+from .staging import PinnedBuffer
 
 
 @dataclasses.dataclass
@@ -73,7 +74,7 @@ class HybridDecoder:
             self._slots.append((*(next(ip) for _ in r.mixer.page_rows()), *(next(st) for _ in r.mixer.state_shapes())))
         self._kinds: List[QueryTiling] = sorted({r.mixer.tiling() for r in model.runs} - {None})
         self.tap: Optional[List[torch.Tensor]] = None  # set to a list: the residual stream after every layer run is appended to it
-        self._stage: List[list] = []                   # pinned staging buffers: [tensor, event]
+        self._stage: List[PinnedBuffer] = []           # what steps are uploaded from
         self._stage_i = 0
         self._sets: Dict[tuple, dict] = {}             # captured decode steps
 
@@ -145,27 +146,28 @@ class HybridDecoder:
             total += (len(v) + 3) // 4 * 4
         return sec, offs, total, plans
 
-    def _upload(self, sec, offs, total: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """The sections into device memory with one asynchronous copy from pinned memory (a ring of four staging buffers)."""
-        if out is None:
-            out = torch.empty(total, dtype=torch.int32, device=self.device)
+    def _staged(self, sec, offs, total: int) -> PinnedBuffer:
+        """The sections in pinned memory (a ring of four buffers)."""
         if len(self._stage) < 4:
-            self._stage.append([torch.empty(max(total, 1 << 14), dtype=torch.int32, pin_memory=True), None])
+            self._stage.append(PinnedBuffer(4 * max(total, 1 << 14)))
             i = len(self._stage) - 1
         else:
             i = self._stage_i = (self._stage_i + 1) % 4
-        buf, ev = self._stage[i]
-        if ev is not None:
-            ev.synchronize()                    # its previous copy has run
-        if buf.numel() < total:
-            buf = self._stage[i][0] = torch.empty(2 * total, dtype=torch.int32, pin_memory=True)
-        host = buf.numpy()
+        buf = self._stage[i]
+        buf.wait()                              # what reads its previous contents has run
+        if buf.tensor.numel() < 4 * total:
+            buf = self._stage[i] = PinnedBuffer(8 * total)
+        host = buf.tensor.numpy().view(np.int32)
         for name, v in sec.items():
             host[offs[name][0]: offs[name][0] + len(v)] = v
-        out.copy_(buf[:total], non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record()
-        self._stage[i][1] = ev
+        return buf
+
+    def _upload(self, sec, offs, total: int) -> torch.Tensor:
+        """The sections into new device memory with one asynchronous copy."""
+        buf = self._staged(sec, offs, total)
+        out = torch.empty(total, dtype=torch.int32, device=self.device)
+        out.copy_(buf.tensor[: 4 * total].view(torch.int32), non_blocking=True)
+        buf.read()
         return out
 
     def _views(self, dev: torch.Tensor, offs, B: int, table_ld: int, plans):
@@ -303,8 +305,7 @@ class HybridDecoder:
         if hit is None:
             hit = self._sets[key] = {"meta": torch.zeros(total, dtype=torch.int32, device=self.device),
                                      "ids": torch.zeros(Bp, dtype=torch.int64, device=self.device), "graph": None}
-        self._upload(sec, offs, total, hit["meta"])
-        hit["ids"][:B].copy_(ids, non_blocking=True)
+        ops.step_inputs(self._staged(sec, offs, total), hit["meta"], ids.expand(B).contiguous(), hit["ids"])
         if hit["graph"] is None:
             v, plan = self._views(hit["meta"], offs, Bp, MB, plans)
             layout = ops.StepLayout(v, Bp, Bp, self.pool.block_size, True, False, 1, bucket)

@@ -27,6 +27,7 @@ from typing import NamedTuple, Optional, Tuple
 import torch
 
 from . import build as _build
+from .staging import PinnedBuffer
 
 ABI_VERSION = 3
 DTYPES = {torch.bfloat16: 0, torch.float32: 1}
@@ -72,6 +73,7 @@ SIGNATURES = {
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_held": (_i32, [_i32, _i32, _i32, _i32]),
+    "vmi_hy_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "vmi_hy_add_norm": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp]),
     "vmi_hy_merge": (ctypes.c_int, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _f32, _f32, _i32, _i32, _vp]),
@@ -297,6 +299,18 @@ def linear_resident(M: int, w: MatrixTiles) -> bool:
 def linear_held(M: int, w: MatrixTiles) -> bool:
     """Whether linear(x, w, norm=...), which norms M rows first, keeps them in registers then."""
     return w.groups == 1 and bool(load().vmi_hy_linear_held(M, w.N, w.K, DTYPES[w.tiles.dtype]))
+
+
+def step_inputs(host: PinnedBuffer, dev: torch.Tensor, ids: torch.Tensor, ids_out: torch.Tensor) -> None:
+    """What `host` holds into all of `dev`, ids into the start of ids_out."""
+    device, stream = _on(dev)
+    nbytes = dev.numel() * dev.element_size()
+    _need(dev.is_contiguous() and host.tensor.numel() >= nbytes, "hybrid_ops.step_inputs: pinned memory of at least dev's size")
+    _need(ids.dtype == ids_out.dtype == torch.int64 and ids.is_contiguous() and ids_out.is_contiguous() and ids.device == dev.device == ids_out.device
+          and ids.numel() <= ids_out.numel(), "hybrid_ops.step_inputs: int64 ids beside what they are copied to")
+    with torch.cuda.device(dev.device):
+        _check(load().vmi_hy_step_inputs(host.tensor.data_ptr(), dev.data_ptr(), nbytes, ids.data_ptr(), ids_out.data_ptr(), ids.numel(), device, stream))
+        host.read()
 
 
 def embed(ids: torch.Tensor, table: torch.Tensor, width: int, scale: float) -> torch.Tensor:
