@@ -6,7 +6,8 @@
 namespace vmi_hybrid {
 
 // Columns below n_split as they are, the others, interleaved (gate, up), through the gated unit: what a product and an elementwise launch behind it (a
-// write and a read of 2 N bytes a row) took.
+// write and a read of 2 N bytes a row) took, and what they give: gate and up are rounded on their way into the unit, so what a prompt comes to does not hang on
+// which side tiles_pay finds ahead for the tokens that happen to share its step.
 template <int MI, int NI, int KS, bool PRIO>
 __global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const vmi_hy_linear_args p) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -18,8 +19,12 @@ __global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const vmi_hy_linear_
         for (int n = 0; n < NI; ++n) {
           if (s + n >= SL) break;   // (scalar)
 #pragma unroll
-          for (int i = 0; i < MI; ++i)
-            if (m + 16 * i < p.M) epilogue<b16, VMI_HY_E_STORE_GLU>(p, acc[n][i], m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16, 0);
+          for (int i = 0; i < MI; ++i) {
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = (float)(b16)acc[n][i][r];
+            if (m + 16 * i < p.M) epilogue<b16, VMI_HY_E_STORE_GLU>(p, v, m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16, 0);
+          }
         }
       });
 }
