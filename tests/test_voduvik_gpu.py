@@ -667,6 +667,24 @@ def test_whole_prompt_and_the_stream_after_every_run(name, dtype):
         close(a, b, dtype, tol32=1e-4, tol16=8e-2)
 
 
+def test_ids_come_from_the_host_from_the_device_or_from_both():
+    """Prompts as lists, tensors of the host, tensors of the device, mixed in one step: the same logits; what is no token is refused as it was."""
+    name = sorted(cases.CONFIGS)[0]
+    a, b, c = ([int(t) for t in cases.tokens(cases.CONFIGS[name], n, s)] for n, s in ((7, 1), (1, 2), (20, 3)))
+    got = []
+    for form in (lambda k, t: t, lambda k, t: torch.tensor(t), lambda k, t: torch.tensor(t).to(dev()), lambda k, t: t if k == 1 else torch.tensor(t, dtype=torch.int32).to(dev())):
+        d = decoder(name, torch.bfloat16)
+        for k in range(3):
+            d.pool.open(k)
+        got.append(d.step([0, 1, 2], [form(k, t) for k, t in enumerate((a, b, c))]))
+        got.append(d.decode([0, 1, 2], [5, 6, 7] if len(got) % 4 == 1 else torch.tensor([5, 6, 7]), use_graph=len(got) > 4))
+    for g, h in zip(got[2:], got):
+        assert torch.equal(g, h)
+    for bad, kind in (([[d.model.vocab_size]], ValueError), ([[-1]], ValueError), ([[1 << 70]], RuntimeError), ([[]], IndexError)):
+        with pytest.raises(kind):
+            d.step([0], bad)
+
+
 @pytest.mark.parametrize("name", sorted(cases.CONFIGS))
 def test_many_tokens_take_the_dense_path_to_the_same_logits(name, monkeypatch):
     from vllmini_amd import hybrid_layers

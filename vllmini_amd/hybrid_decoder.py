@@ -11,6 +11,7 @@ Every layer RUN has its own cache / state: a layer inside a loop keeps one per p
 from __future__ import annotations
 
 import dataclasses
+import itertools
 from typing import Dict, List, Optional, Sequence, Union
 
 import numpy as np
@@ -197,23 +198,36 @@ class HybridDecoder:
             return None
         return m.head.run(res.settle(), rows)
 
-    def _ids(self, tokens: Sequence) -> torch.Tensor:
-        """The step's token ids on the device; host ids are range-checked here."""
+    def _host_ids(self, tokens) -> np.ndarray:
+        try:
+            ids = np.fromiter((int(x) for x in tokens), dtype=np.int64)
+        except OverflowError as e:
+            raise RuntimeError(str(e)) from e
+        if len(ids) and (int(ids.min()) < 0 or int(ids.max()) >= self.model.vocab_size):
+            raise ValueError(f"token id out of range (vocabulary of {self.model.vocab_size})")
+        return ids
+
+    def _ids(self, tokens: Sequence) -> Union[torch.Tensor, np.ndarray]:
+        """The step's token ids: a device tensor, or an array where none of them are on the device yet (they go up with the step's layout: a copy off pageable memory
+        would wait for all that is queued on the stream, and what the host does behind it for the GPU).  Host ids are range-checked here."""
         parts, host = [], []
+
+        def flush():
+            ids = self._host_ids(itertools.chain.from_iterable(host))
+            host.clear()
+            if len(ids):
+                parts.append(ids)
+
         for t in tokens:
             if isinstance(t, torch.Tensor) and t.is_cuda:
-                if host:
-                    parts.append(torch.tensor(host, dtype=torch.int64))
-                    host = []
+                flush()
                 parts.append(t.reshape(-1).to(torch.int64))
             else:
-                host.extend(int(x) for x in t)
-        if host:
-            parts.append(torch.tensor(host, dtype=torch.int64))
-        for t in parts:
-            if not t.is_cuda and t.numel() and (int(t.min()) < 0 or int(t.max()) >= self.model.vocab_size):
-                raise ValueError(f"token id out of range (vocabulary of {self.model.vocab_size})")
-        return torch.cat([t.to(self.device, non_blocking=True) for t in parts]) if len(parts) > 1 else parts[0].to(self.device)
+                host.append(t)
+        flush()
+        if len(parts) <= 1:
+            return parts[0]
+        return torch.cat([t if isinstance(t, torch.Tensor) else torch.from_numpy(t).to(self.device) for t in parts])
 
     @torch.no_grad()
     def step(self, seq_ids: Sequence[int], tokens: Sequence, want: Optional[Sequence[Sequence[int]]] = None) -> Optional[torch.Tensor]:
@@ -231,7 +245,7 @@ class HybridDecoder:
             rows = np.asarray([int(s) + int(k) for s, w in zip(starts, want) for k in w], dtype=np.int64)
         return self._run(seq_ids, counts, self._ids(tokens), rows)
 
-    def _run(self, seq_ids: Sequence[int], counts: np.ndarray, ids: torch.Tensor, rows: np.ndarray) -> Optional[torch.Tensor]:
+    def _run(self, seq_ids: Sequence[int], counts: np.ndarray, ids: Union[torch.Tensor, np.ndarray], rows: np.ndarray) -> Optional[torch.Tensor]:
         T, B, starts = int(counts.sum()), len(counts), np.cumsum(counts) - counts
         if T > 65535:
             raise ValueError("a step holds at most 65535 tokens")
@@ -239,7 +253,13 @@ class HybridDecoder:
         keys = int((a["ctx"] + counts).max())
         ld = -(-keys // self.pool.block_size)
         sec, offs, total, plans = self._layout(a, counts, rows, T, B, ld, keys)
+        if isinstance(ids, np.ndarray):
+            sec["ids"] = ids.view(np.int32)
+            offs["ids"] = (total, 2 * len(ids))
+            total += (2 * len(ids) + 3) // 4 * 4
         v, plan = self._views(self._upload(sec, offs, total), offs, B, ld, plans)
+        if "ids" in v:
+            ids = v.pop("ids").view(torch.int64)
         spans = bool((starts // ops.ROW_TILE != (starts + counts - 1) // ops.ROW_TILE).any())
         layout = ops.StepLayout(v, T, B, self.pool.block_size, bool((counts == 1).all()), spans, int(counts.max()), keys)
         return self._forward(ids, layout, plan, v["rows"] if len(rows) else None)
@@ -292,6 +312,8 @@ class HybridDecoder:
         ids = input_ids.reshape(-1).to(self.device, torch.int64) if isinstance(input_ids, torch.Tensor) else self._ids([list(input_ids)])
         if not use_graph:
             return self._run(seq_ids, np.ones(B, dtype=np.int64), ids, np.arange(B))
+        if isinstance(ids, np.ndarray):
+            ids = torch.from_numpy(ids).to(self.device)
         Bp, MB = self._padded(B), self.pool.max_blocks_per_seq
         counts = np.ones(B, dtype=np.int64)
         a = self.pool.append(seq_ids, counts)
