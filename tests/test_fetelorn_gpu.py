@@ -225,6 +225,26 @@ def test_many_states_take_two_column_tiles_a_workgroup(kind):
     close(got[7], alone, torch.float32, tol32=1e-5)
 
 
+@pytest.mark.parametrize("kind", ["retention", "delta"])
+@pytest.mark.parametrize("B", [4, 5, 6, 9, 17, 33])
+def test_walks_of_every_length_start_in_turn(kind, B):
+    """state_scan_kernel's order of entries, 64 workgroups each (4: as they come, 5 and 6: two workgroups a compute unit, 9: three, 17: two column tiles each, 33: as they come
+    again): lengths all over, some of them equal, each sequence as it comes out alone."""
+    k, want = (retention_case(8, 128, 128, 64, (0.9, 0.5, 0.99, 1.0, 0.8, 0.97, 0.3, 0.999), torch.float32, B) if kind == "retention" else
+               delta_case(8, 4, 128, 128, 4, torch.float32, B))
+    rng = np.random.default_rng(B)
+    lens = [int(n) for n in rng.integers(1, 70, B)]
+    lens[-1] = lens[0]
+    seqs = [k.inputs(n, 100 + i) for i, n in enumerate(lens)]
+    got = k.run([torch.cat([s[1][j] for s in seqs]) for j in range(3)], layout(lens, [0] * B, [[0]] * B, 64, pos_slots=False)).split(lens)
+    states = k.held[0].clone()
+    close(got[0], want(seqs[0][0]), torch.float32, tol32=5e-5)
+    for i, n in enumerate(lens):
+        alone = k.run(seqs[i][1], layout([n], [0], [[0]], 64, slots=[i], pos_slots=False))
+        close(got[i], alone, torch.float32, tol32=1e-5)
+        close(states[i], k.held[0][i], torch.float32, tol32=1e-5)
+
+
 def test_delta_rule_survives_decays_that_leave_nothing():
     k, want = delta_case(2, 1, 32, 32, 4, torch.float32, rate=6.0, bias=8.0)
     _portions(k, want, 40, [[40], [17, 2, 21], [1] * 40], [1, 0, 3])

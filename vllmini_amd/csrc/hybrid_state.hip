@@ -397,17 +397,35 @@ __global__ __launch_bounds__(256) void state_prep_kernel(const vmi_hy_state_args
   }
 }
 
-// NT: 16-row tiles of the state, dealt over RS waves.  One workgroup: CT tiles of 16 value columns of one (entry, head)
-template <int KIND, int NT, int RS, int CT>
-__global__ __launch_bounds__(64 * RS, CT > 1 && NT <= 8 ? 2 : 1) void state_scan_kernel(const vmi_hy_state_args p, const vmi_hy_step s) {
-  constexpr int NW = NT / RS, DEPTH = NW <= 2 && CT == 1 ? 3 : 2;   // tiles of a wave, chunks of operands in registers
+// The entry of this workgroup's place in the grid where more workgroups are launched than there are compute units, of up to 32 entries: the `first` longest ones, which fill the
+// chip, come shortest of them first, and behind them the others, longest first.  A compute unit that gets a second workgroup gets it in the order of the first ones, so the
+// longest walks, which everything else waits for, keep theirs to themselves: side by side two take 0.93 us a chunk each, one alone 0.63.
+__device__ __forceinline__ int entry_in_turn(const vmi_hy_step& s, int first, int lane) {
+  const int len = lane < s.B ? s.q_len[lane] : -1;
+  int rank = 0;   // longer ones, and equal ones in front
+  for (int j = 0; j < s.B; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane) ? 1 : 0;
+  }
+  const int at = (int)blockIdx.y < first ? first - 1 - (int)blockIdx.y : (int)blockIdx.y;
+  return __builtin_ctzll(__ballot(lane < s.B && rank == at));
+}
+
+// NT: 16-row tiles of the state, dealt over RS waves.  One workgroup: CT tiles of 16 value columns of one (entry, head); CU of them a compute unit
+template <int KIND, int NT, int RS, int CT, int CU>
+__global__ __launch_bounds__(64 * RS, CU) void state_scan_kernel(const vmi_hy_state_args p, const vmi_hy_step s, const int first) {
   constexpr bool DELTA = KIND == VMI_HY_DELTA;
+  // A chunk's operands are some 1.8 us away (every chunk is a page of its own), a chunk takes 0.6: what bounds a walk is how many of them are asked for ahead, and with operands
+  // behind one address register each and accumulators among the other registers as many fit as it takes.  Heads of 128, retention / delta rule, us, before (three ahead, a
+  // compute unit's workgroups as they come) -> now: 1 x 1500 rows, 8 heads 70 / 93 -> 59 / 80, 6 x up to 1500 88 / 118 -> 61 / 84, 9 x 400 34 / 51 -> 30 / 37; 16 heads, 3 x 1000
+  // 55 / 72 -> 42 / 57, 12 x 400 59 / 80 -> 46 / 64, 5 x 700 51 / 71 -> 52 / 70.
+  constexpr int NW = NT / RS, DEPTH = NW > 2 || CT > 1 ? 2 : CU > 2 ? DELTA ? 2 : 3 : DELTA ? 3 : 4;   // tiles of a wave, chunks of operands in registers
   constexpr int EW = 4 / RS;                             // elements of a lane's four that a wave finishes of o
   __shared__ f32x4 reda[DELTA ? 2 : 1][CT][DELTA ? RS : 1][64];
   __shared__ float redo[2][CT][RS][4][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
   // (heads vary fastest: the column blocks of one head, which read the same operands, then share an XCD's L2)
-  const int h = blockIdx.x % p.heads, col0 = (int)(blockIdx.x / p.heads) * 16 * CT, e = blockIdx.y;
+  const int h = blockIdx.x % p.heads, col0 = (int)(blockIdx.x / p.heads) * 16 * CT, e = first ? entry_in_turn(s, first, lane) : (int)blockIdx.y;
   const Portion r = portion(s, e);
   if (r.len <= 0) return;
   constexpr int dim = NT * 16;
@@ -429,23 +447,25 @@ __global__ __launch_bounds__(64 * RS, CT > 1 && NT <= 8 ? 2 : 1) void state_scan
     f32x4 w[DELTA ? NW : 1], q[NW], k[NW], d[NW], u[CT];
     float b[EW];
   };
-  const int row = r16 * dim + 16 * ct0 + 4 * kc, col = r16 * CH + 4 * kc;
+  const uint32_t row = (uint32_t)(r16 * dim + 4 * kc) * 4, col = (uint32_t)(r16 * CH + 4 * kc) * 4;
+  // a lane's bytes behind a place that all lanes share: one address register an operand, none to keep for later chunks
+  auto four = [](const float* at, uint32_t lane_at) { return *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(at) + lane_at); };
   // (no branch stands in a chunk: every path issues the same loads and stores, so the waits count them exactly)
   auto load = [&](Operands& o, int c) {
     const float* at = base + min(c, nch - 1) * step;   // (past the end: the last one again)
 #pragma unroll
     for (int t = 0; t < NW; ++t) {
-      if constexpr (DELTA) o.w[t] = *reinterpret_cast<const f32x4*>(at + sc.w + row + 16 * t);
-      o.q[t] = *reinterpret_cast<const f32x4*>(at + sc.q + row + 16 * t);
+      if constexpr (DELTA) o.w[t] = four(at + sc.w + 16 * (ct0 + t), row);
+      o.q[t] = four(at + sc.q + 16 * (ct0 + t), row);
     }
 #pragma unroll
-    for (int j = 0; j < CT; ++j) o.u[j] = *reinterpret_cast<const f32x4*>(at + sc.u + (col0 + 16 * j) * CH + col);
+    for (int j = 0; j < CT; ++j) o.u[j] = four(at + sc.u + (col0 + 16 * j) * CH, col);
 #pragma unroll
-    for (int i = 0; i < EW; ++i) o.b[i] = at[sc.b + col + wave + RS * i];
+    for (int i = 0; i < EW; ++i) o.b[i] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(at + sc.b + wave + RS * i) + col);
 #pragma unroll
     for (int t = 0; t < NW; ++t) {
-      o.d[t] = *reinterpret_cast<const f32x4*>(at + sc.d + 16 * (ct0 + t) + 4 * kc);
-      o.k[t] = *reinterpret_cast<const f32x4*>(at + sc.k + 16 * (ct0 + t) * CH + col);
+      o.d[t] = four(at + sc.d + 16 * (ct0 + t), (uint32_t)kc * 16);
+      o.k[t] = four(at + sc.k + 16 * (ct0 + t) * CH, col);
     }
   };
   f32x4 part[CT];                           // this wave's part of the last chunk's o
@@ -458,7 +478,8 @@ __global__ __launch_bounds__(64 * RS, CT > 1 && NT <= 8 ? 2 : 1) void state_scan
       for (int x = 0; x < 4; ++x) redo[c & 1][j][wave][x][lane] = part[j][x];
   };
   auto finish = [&](int c) {                // the elements wave, wave + RS, .. of every lane's four of chunk c - 1
-    float* out = base + max(c - 1, 0) * step + sc.o + 4 * kc * p.vdim + col0 + r16;
+    float* out = base + max(c - 1, 0) * step + sc.o + col0;
+    const uint32_t lane_at = (uint32_t)(4 * kc * p.vdim + r16) * 4;
 #pragma unroll
     for (int j = 0; j < CT; ++j)
 #pragma unroll
@@ -467,7 +488,7 @@ __global__ __launch_bounds__(64 * RS, CT > 1 && NT <= 8 ? 2 : 1) void state_scan
         float y = redo[c & 1][j][0][x][lane];
 #pragma unroll
         for (int w = 1; w < RS; ++w) y += redo[c & 1][j][w][x][lane];
-        out[x * p.vdim + 16 * j] = y;       // (c = 0: zeros, which the next chunk overwrites)
+        *reinterpret_cast<float*>(reinterpret_cast<char*>(out + x * p.vdim + 16 * j) + lane_at) = y;       // (c = 0: zeros, which the next chunk overwrites)
       }
   };
   auto chunk = [&](Operands& o, int c) {
@@ -738,12 +759,17 @@ template <int KIND, int NT>
 static void launch_scan(const vmi_hy_state_args& p, const vmi_hy_step& s, hipStream_t st) {
   constexpr int RS = NT % 4 == 0 ? 4 : 2;
   const int tiles = p.vdim / 16;   // (even: vdim is a multiple of 32)
-  // states enough for the chip: a workgroup takes two column tiles, which halves what is read per column
-  if (NT <= 16 && (int64_t)p.heads * tiles * s.B >= 1024)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(state_scan_kernel<KIND, NT, RS, NT <= 16 ? 2 : 1>), dim3(p.heads * (tiles / 2), s.B), dim3(64 * RS), 0,
-                       st, p, s);
-  else
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(state_scan_kernel<KIND, NT, RS, 1>), dim3(p.heads * tiles, s.B), dim3(64 * RS), 0, st, p, s);
+  const int each = p.heads * tiles;
+  // states enough for the chip: a workgroup takes two column tiles, which halves what is read per column.  More than two workgroups a compute unit: registers for three
+  constexpr int TWO = NT <= 8 ? 2 : 1, CT = NT <= 16 ? 2 : 1, THREE = NT <= 8 ? 3 : 1;
+  auto go = [&](auto* fn, int wgs) {
+    // (what entry_in_turn asks for; past 32 entries, which are short then, finding one's place takes longer than it gives: 60 entries of up to 100 rows 38 -> 43 us)
+    const int first = s.B <= 32 && (int64_t)wgs * s.B > 256 ? (wgs > 256 ? 1 : 256 / wgs) : 0;
+    hipLaunchKernelGGL(fn, dim3(wgs, s.B), dim3(64 * RS), 0, st, p, s, first);
+  };
+  if (NT <= 16 && (int64_t)each * s.B >= 1024) go(state_scan_kernel<KIND, NT, RS, CT, TWO>, each / 2);
+  else if (NT <= 8 && (int64_t)each * s.B > 512) go(state_scan_kernel<KIND, NT, RS, 1, THREE>, each);
+  else go(state_scan_kernel<KIND, NT, RS, 1, TWO>, each);
 }
 
 template <typename T, int KIND>
