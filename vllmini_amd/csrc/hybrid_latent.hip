@@ -19,9 +19,14 @@ inline size_t attention_lds(int D) {
 // RT row tiles, NT value tiles (of 16 columns) per wave, U 16-byte-element units of a cache row per thread
 // EXACT: a row has exactly that many (its length is known to the compiler: loops over it unroll, and with one row tile the query
 // stays in registers, which leaves LDS for a second workgroup)
-template <typename T, int KT, int RT, int NT, int U, bool EXACT>
-__global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attention_kernel(const vmi_hy_latent_attention_args p, const vmi_hy_step s) {
-  constexpr int R = 16 * RT, TPK = 256 / KT, PAD = pad_of<T>(), LDP = KT + PAD, SW = KT / 16;   // SW waves score
+// W waves.  Several row tiles take eight: a tile of 64 keys is some 1200 vector instructions, 72 reads of LDS and as many products behind them in each of four waves, and one wave a
+// SIMD waits for every one of them; two share them, with few enough registers each that no accumulator has to be moved to be scaled.  Four waves -> eight, rows of 576, 16 heads:
+// 1 x 1024 tokens 116 -> 82 us, 4 x up to 1024 164 -> 121; 8 heads, 12 x up to 300 49 -> 33; 30 x up to 40 24 -> 14.  (Row group rg of wave 4 rg + kg scores the 16 keys kg.)
+template <typename T, int KT, int RT, int NT, int U, bool EXACT, int W>
+__global__ __launch_bounds__(64 * W, EXACT && (RT == 1 || W == 8) ? 2 : 1) void latent_attention_kernel(const vmi_hy_latent_attention_args p, const vmi_hy_step s) {
+  constexpr int R = 16 * RT, TH = 64 * W, TPK = TH / KT, PAD = pad_of<T>(), LDP = KT + PAD, SW = KT / 16;   // SW key groups are scored
+  constexpr int RG = W / 4, RTS = RT / RG;   // row groups, row tiles of one
+  static_assert(W == 4 || (W == 8 && SW == 4 && RT % 2 == 0), "four key groups, one or two row groups");
   need(p.tiles), need(p.q), need(p.cache), need(p.out), need(p.partial), need(p.heads), need(p.rank), need(p.splits), need(p.scale), need(s.ctx), need(s.q_len),
       need(s.q_start), need(s.table), need(s.table_ld), need(s.page_size), need(s.T);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -32,6 +37,7 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
   T* ps = qs + (QREG ? 0 : (size_t)R * LDK);       // [R][LDP]
   float* sx = reinterpret_cast<float*>(ps + (size_t)R * LDP);   // [4][R]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int kg = RG > 1 ? wave & 3 : wave, rg = RG > 1 ? wave >> 2 : 0;   // (scalar)
   const int e = p.tiles[2 * blockIdx.x], r0 = p.tiles[2 * blockIdx.x + 1], split = blockIdx.y;
   if (e < 0) return;
   const int H = p.heads, ctx = s.ctx[e];
@@ -41,7 +47,7 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
   const int kv_end = ctx + (r0 + nrows - 1) / H + 1;
   const int nkt = (kv_end + KT - 1) / KT, tps = (nkt + p.splits - 1) / p.splits;
   const int kt0 = split * tps, kt1 = min(nkt, kt0 + tps);
-  const int n16 = p.rank >> 4, d0 = (int)blockIdx.z * (NT * 4);   // this workgroup's value tiles: d0 + wave + 4 nt
+  const int n16 = p.rank >> 4, d0 = (int)blockIdx.z * (NT * W);   // this workgroup's value tiles: d0 + wave + W nt
   float* part = p.partial ? p.partial + ((int64_t)split * s.T * H + grow0) * (p.rank + 2) : nullptr;
   if (kt0 >= kt1) {   // (splits > 1 only: split 0 always has keys)
     if (blockIdx.z == 0 && tid < nrows) {
@@ -75,14 +81,14 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
   } else {
     // (rows past the last one repeat it and are not stored; eight units a thread in flight together)
 #pragma unroll 8
-    for (int u = tid; u < R * (D >> 3); u += 256) {
+    for (int u = tid; u < R * (D >> 3); u += TH) {
       const int m = u / (D >> 3), k = (u - m * (D >> 3)) * 8;
       *reinterpret_cast<V8<T>*>(qs + m * LDK + k) = load8(static_cast<const T*>(p.q) + (grow0 + min(m, nrows - 1)) * D + k);
     }
   }
 
   f32x4 o[RT][NT];
-  float mrun[RT][4], lrun[RT][4];
+  float mrun[RT][4], lrun[RTS][4];   // (lrun: of the rows that this wave scores)
   int lim[RT][4];   // last key row m sees
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -91,7 +97,7 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       mrun[rt][r] = -1e30f;
-      lrun[rt][r] = 0.f;
+      if (rt < RTS) lrun[rt][r] = 0.f;
       lim[rt][r] = ctx + (r0 + rt * 16 + 4 * kc + r) / H;
     }
   }
@@ -106,12 +112,12 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
       next_page = tab[key_of(min(kt + 2, kt1 - 1)) / s.page_size];
     }
     __syncthreads();
-    f32x4 sc[RT];
+    f32x4 sc[RTS];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) sc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int rt = 0; rt < RTS; ++rt) sc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (SW == 4 || wave < SW) {
-      const T* krow = ks + (wave * 16 + r16) * LDK + 8 * kc;
-      const T* qrow = qs + r16 * LDK + 8 * kc;
+      const T* krow = ks + (kg * 16 + r16) * LDK + 8 * kc;
+      const T* qrow = qs + (rg * RTS * 16 + r16) * LDK + 8 * kc;
       if constexpr (QREG) {
         f32x4 odd = f32x4{0.f, 0.f, 0.f, 0.f};   // (two chains of sums)
 #pragma unroll
@@ -122,24 +128,24 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
         for (int k = 0; k < U * TPK * 8; k += 32) {
           const V8<T> kf = load8(krow + k);
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt) mma(sc[rt], load8(qrow + rt * 16 * LDK + k), kf);
+          for (int rt = 0; rt < RTS; ++rt) mma(sc[rt], load8(qrow + rt * 16 * LDK + k), kf);
         }
       } else {
 #pragma unroll 2
         for (int k = 0; k < D; k += 32) {
           const V8<T> kf = load8(krow + k);
 #pragma unroll
-          for (int rt = 0; rt < RT; ++rt) mma(sc[rt], load8(qrow + rt * 16 * LDK + k), kf);
+          for (int rt = 0; rt < RTS; ++rt) mma(sc[rt], load8(qrow + rt * 16 * LDK + k), kf);
         }
       }
-      const int key = kt * KT + wave * 16 + r16;
+      const int key = kt * KT + kg * 16 + r16;
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
+      for (int rt = 0; rt < RTS; ++rt) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          sc[rt][r] = key <= lim[rt][r] ? sc[rt][r] * sc2 : -INFINITY;   // (keys past kv_end are past every row's limit)
+          sc[rt][r] = key <= (rg ? lim[RT - RTS + rt][r] : lim[rt][r]) ? sc[rt][r] * sc2 : -INFINITY;   // (keys past kv_end are past every row's limit)
           const float v = max16(sc[rt][r]);
-          if (r16 == 0) sx[wave * R + rt * 16 + 4 * kc + r] = v;
+          if (r16 == 0) sx[kg * R + (rg * RTS + rt) * 16 + 4 * kc + r] = v;
         }
       }
     }
@@ -159,12 +165,17 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
         const float mn = fmaxf(mrun[rt][r], mx[r]);
         alpha[rt][r] = exp2_hw(mrun[rt][r] - mn);
         mrun[rt][r] = mn;
-        if (SW == 4 || wave < SW) {
-          const T pr = (T)exp2_hw(sc[rt][r] - mn);
-          lrun[rt][r] = fmaf(lrun[rt][r], alpha[rt][r], (float)pr);   // (what is summed is what multiplies the values)
-          ps[(rt * 16 + 4 * kc + r) * LDP + wave * 16 + r16] = pr;
-        }
       }
+    }
+    if (SW == 4 || wave < SW) {
+#pragma unroll
+      for (int rt = 0; rt < RTS; ++rt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const T pr = (T)exp2_hw(sc[rt][r] - (rg ? mrun[RT - RTS + rt][r] : mrun[rt][r]));
+          lrun[rt][r] = fmaf(lrun[rt][r], rg ? alpha[RT - RTS + rt][r] : alpha[rt][r], (float)pr);   // (what is summed is what multiplies the values)
+          ps[((rg * RTS + rt) * 16 + 4 * kc + r) * LDP + kg * 16 + r16] = pr;
+        }
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -180,7 +191,7 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
       for (int rt = 0; rt < RT; ++rt) pf[rt] = load8(ps + (rt * 16 + r16) * LDP + k + 8 * kc);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const int dt = min(d0 + wave + 4 * nt, n16 - 1);   // (past the last one: computed, not stored)
+        const int dt = min(d0 + wave + W * nt, n16 - 1);   // (past the last one: computed, not stored)
         const V8<T> vf = column8(ks, LDK, k + 8 * kc, dt * 16, r16);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) mma(o[rt][nt], pf[rt], vf);
@@ -191,11 +202,11 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
 
   // the rows' sums: over the 16 keys a lane group held, then over the waves
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
+  for (int rt = 0; rt < RTS; ++rt)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float v = sum16(lrun[rt][r]);
-      if (r16 == 0) sx[wave * R + rt * 16 + 4 * kc + r] = v;
+      if (r16 == 0) sx[kg * R + (rg * RTS + rt) * 16 + 4 * kc + r] = v;
     }
   __syncthreads();
 #pragma unroll
@@ -210,14 +221,14 @@ __global__ __launch_bounds__(256, EXACT && RT == 1 ? 2 : 1) void latent_attentio
         T* out = static_cast<T*>(p.out) + (grow0 + m) * p.rank + r16;
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          const int dt = d0 + wave + 4 * nt;
+          const int dt = d0 + wave + W * nt;
           if (dt < n16) out[dt * 16] = (T)(o[rt][nt][r] * inv);
         }
       } else {
         float* out = part + (int64_t)m * (p.rank + 2);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-          const int dt = d0 + wave + 4 * nt;
+          const int dt = d0 + wave + W * nt;
           if (dt < n16) out[dt * 16 + r16] = o[rt][nt][r];
         }
         if (blockIdx.z == 0 && wave == 0 && r16 == 0) {
@@ -312,12 +323,13 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_pr
 
 template <typename T, int KT, int RT, int NT, int U, bool EXACT = false>
 static int launch_attention(const vmi_hy_latent_attention_args& p, const vmi_hy_step& s, hipStream_t st) {
-  auto* fn = latent_attention_kernel<T, KT, RT, NT, U, EXACT>;
+  constexpr int W = RT > 1 ? 8 : 4;   // (NT and U are those of four waves)
+  auto* fn = latent_attention_kernel<T, KT, RT, NT * 4 / W, U * 4 / W, EXACT, W>;
   const int D = p.rank + p.rot;
   const size_t lds = attention_lds<T, KT, RT>(D) - (EXACT && RT == 1 && sizeof(T) == 2 ? (size_t)16 * (D + pad_of<T>()) * sizeof(T) : 0);
   if (int rc = allow_lds(fn, lds, "vmi_hy_latent_attention")) return rc;
   const int zb = ((p.rank >> 4) + 4 * NT - 1) / (4 * NT);
-  hipLaunchKernelGGL(fn, dim3(p.n_tiles, p.splits, zb), dim3(256), lds, st, p, s);
+  hipLaunchKernelGGL(fn, dim3(p.n_tiles, p.splits, zb), dim3(64 * W), lds, st, p, s);
   if (p.splits > 1)
     launch_combine<T>(Combine{p.partial, p.out, nullptr, s.tok_seq, (int64_t)p.heads * p.rank, 0, s.T, p.heads, p.rank, p.splits}, st);
   return launched("vmi_hy_latent_attention");
@@ -325,7 +337,7 @@ static int launch_attention(const vmi_hy_latent_attention_args& p, const vmi_hy_
 
 template <typename T, int KT, int RT>
 static int attention_width(const vmi_hy_latent_attention_args& p, const vmi_hy_step& s, hipStream_t st) {
-  const int units = (p.rank + p.rot + 2048 / KT - 1) / (2048 / KT);   // of 8 elements of a cache row, per thread
+  const int units = (p.rank + p.rot + 2048 / KT - 1) / (2048 / KT);   // of 8 elements of a cache row, per thread of four waves
   if (p.rank <= 128 && units <= 8) return launch_attention<T, KT, RT, 2, 8>(p, s, st);
   if (p.rank <= 256 && units <= 12) return launch_attention<T, KT, RT, 4, 12>(p, s, st);
   if constexpr (sizeof(T) == 2 && KT == 64)
