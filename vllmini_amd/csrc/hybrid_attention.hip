@@ -262,13 +262,15 @@ inline size_t gqa_rows_lds(int dim, int vdim, int rep, bool bias) {
   return ((size_t)64 * (dim + vdim + 8) + (size_t)64 * 72) * 2 + (bias ? (size_t)rep * bias_window(64, 64, rep) * 4 : 0);
 }
 
-// NK k-steps (of 32) of a query row, NV value tiles (of 16 columns)
-template <int NK, int NV, int U>
+// NK k-steps (of 32) of a query row, NV value tiles (of 16 columns): at most that many, or (EXACT) just that many, so that no condition stands between a read of LDS and the product
+// behind it and they overlap: a branch a product, a bias and a mask each waited for its own read (heads of 128, 8 over 2 of them, 1 x 1500 rows 84 -> 53 us, 6 x up to 1500 91 -> 63;
+// 16 over 4, 32 x up to 200 33 -> 25)
+template <int NK, int NV, int U, bool EXACT>
 __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vmi_hy_attention_args p, const vmi_hy_step s) {
   constexpr int R = 64, KT = 64, LDP = KT + 8;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int dim = p.dim, vdim = p.vdim, LDK = dim + vdim + 8;
+  const int dim = EXACT ? 32 * NK : p.dim, vdim = EXACT ? 16 * NV : p.vdim, LDK = dim + vdim + 8;
   b16* ks = reinterpret_cast<b16*>(smem);          // [64][LDK]
   b16* ps = ks + (size_t)KT * LDK + wave * 16 * LDP;   // [16][LDP], this wave's
   float* bl = reinterpret_cast<float*>(ks + (size_t)KT * LDK + 64 * LDP);
@@ -313,6 +315,17 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
     __syncthreads();
     const int key0 = kt * KT;
     if (key0 <= lim1 && key0 + KT > low0) {
+      float bias[4][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias[r][j] = 0.f;
+      if (keys.bn) {   // (all of them at once, in front of the products: one condition a tile)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bias[r][j] = bl[boff[r] - 16 * j];
+      }
       f32x4 sc[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -320,25 +333,25 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
         const b16* krow = ks + (j * 16 + r16) * LDK + 8 * kc;
 #pragma unroll
         for (int k = 0; k < NK; ++k)
-          if (NK <= 4 || k < nk) mma(sc[j], qr[k], k < nk ? load8(krow + 32 * k) : zero8<b16>());
+          if (EXACT || NK <= 4 || k < nk) mma(sc[j], qr[k], EXACT || k < nk ? load8(krow + 32 * k) : zero8<b16>());
       }
       const bool whole = key0 + KT - 1 <= lim0 && key0 >= low1;
-      f32x4 mx;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float v = -INFINITY;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float b = keys.bn ? bl[boff[r] - 16 * j] : 0.f;
-          sc[j][r] = fmaf(sc[j][r], sc2, b);
-          if (!whole) {
+        for (int j = 0; j < 4; ++j) sc[j][r] = fmaf(sc[j][r], sc2, bias[r][j]);
+      if (!whole) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
             const int key = key0 + j * 16 + r16;
             sc[j][r] = key <= lim[r] && key >= low[r] ? sc[j][r] : -INFINITY;
           }
-          v = fmaxf(v, sc[j][r]);
-        }
-        mx[r] = max16(v);
       }
+      f32x4 mx;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx[r] = max16(fmaxf(fmaxf(sc[0][r], sc[1][r]), fmaxf(sc[2][r], sc[3][r])));
       float alpha[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -362,7 +375,7 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
         const b16x8 pf = load8(ps + r16 * LDP + k + 8 * kc);
 #pragma unroll
         for (int nt = 0; nt < NV; ++nt)
-          if (nt < n16) mma(o[nt], pf, column8(ks, LDK, k + 8 * kc, dim + nt * 16, r16));
+          if (EXACT || nt < n16) mma(o[nt], pf, column8(ks, LDK, k + 8 * kc, dim + nt * 16, r16));
       }
     }
     __syncthreads();
@@ -379,12 +392,12 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
       b16* out = static_cast<b16*>(p.out) + t * p.ldo + (int64_t)h * vdim + r16;
 #pragma unroll
       for (int nt = 0; nt < NV; ++nt)
-        if (nt < n16) out[nt * 16] = (b16)(o[nt][r] * inv);
+        if (EXACT || nt < n16) out[nt * 16] = (b16)(o[nt][r] * inv);
     } else {
       float* out = q.part(p, s, m);
 #pragma unroll
       for (int nt = 0; nt < NV; ++nt)
-        if (nt < n16) out[nt * 16 + r16] = o[nt][r];
+        if (EXACT || nt < n16) out[nt * 16 + r16] = o[nt][r];
       if (r16 == 0) {
         out[vdim] = mrun[r];
         out[vdim + 1] = l;
@@ -443,9 +456,9 @@ static int launch_gqa(const vmi_hy_attention_args& p, const vmi_hy_step& s, hipS
   return launched_gqa<T>(p, s, st);
 }
 
-template <int NK, int NV, int U>
+template <int NK, int NV, int U, bool EXACT = false>
 static int launch_gqa_rows(const vmi_hy_attention_args& p, const vmi_hy_step& s, hipStream_t st) {
-  auto* fn = gqa_rows_kernel<NK, NV, U>;
+  auto* fn = gqa_rows_kernel<NK, NV, U, EXACT>;
   const size_t lds = gqa_rows_lds(p.dim, p.vdim, p.heads / p.kv_heads, p.bias != nullptr);
   if (int rc = allow_lds(fn, lds, "vmi_hy_attention")) return rc;
   hipLaunchKernelGGL(fn, dim3(p.n_tiles, p.splits, p.kv_heads), dim3(256), lds, st, p, s);
@@ -476,6 +489,7 @@ static int run_gqa(const vmi_hy_attention_args& p, const vmi_hy_step& s, hipStre
     return fail(VMI_HY_E_ARG, "vmi_hy_attention", "row_tiles is what vmi_hy_attention_row_tiles returns");
   if constexpr (sizeof(T) == 2) {
     if (p.row_tiles == 4) {
+      if (p.dim == 128 && p.vdim == 128) return launch_gqa_rows<4, 8, 8, true>(p, s, st);
       if (p.dim <= 128 && p.vdim <= 128) return launch_gqa_rows<4, 8, 8>(p, s, st);
       return launch_gqa_rows<8, 16, 16>(p, s, st);
     }
