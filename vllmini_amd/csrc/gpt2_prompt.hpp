@@ -118,6 +118,12 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
     }
   };
   load(0);
+  // the pages of the workgroup's own positions, asked for now: behind its last tile each of them was a trip to memory that nothing else was left to hide
+  int page[MI][U];
+#pragma unroll
+  for (int m = 0; m < MI; ++m)
+#pragma unroll
+    for (int i = 0; i < U; ++i) page[m][i] = table[min(q0 + m * PKT + (tid + 256 * i) / (16 * UPR) * PROMPT_BS, len - 1) / PROMPT_BS];
   const int w0 = q0 + wave * 16 * MI;   // this wave's first position
   h16x8 qf[MI][NK];
 #pragma unroll
@@ -148,11 +154,14 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
     if (kt + 1 < nkt) load(kt + 1);
     __syncthreads();   // (the writes of tile kt + 1 go where tile kt - 1 was read, which every wave has left behind)
     if (key0 >= q0) {   // this workgroup's own positions: four pages into the cache
+      int64_t at_page[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) at_page[i] = (MI > 1 && key0 > q0 ? page[MI - 1][i] : page[0][i]) * p.bstride + h * p.hstride;
 #pragma unroll
       for (int i = 0; i < U; ++i) {
         const int u = tid + 256 * i, pg = u / (16 * UPR), off = u & 15, d8 = (u >> 4) % UPR, pos = key0 + pg * PROMPT_BS;
         if (pos + off < len)
-          *reinterpret_cast<h16x8*>(p.kcache + table[pos / PROMPT_BS] * p.bstride + h * p.hstride + (d8 * PROMPT_BS + off) * 8) =
+          *reinterpret_cast<h16x8*>(p.kcache + at_page[i] + (d8 * PROMPT_BS + off) * 8) =
               *reinterpret_cast<const h16x8*>(ks + (pg * PROMPT_BS + off) * LD + d8 * 8);
       }
 #pragma unroll
@@ -161,7 +170,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
         const int at = pg * PROMPT_BS + half * 8;
         const h16x8 v = join(column4(vs, LD, at, nt * 16, r16), column4(vs, LD, at + 4, nt * 16, r16));
         if (pos < len) {
-          h16* dst = p.vcache + table[pos / PROMPT_BS] * p.bstride + h * p.hstride + (nt * 16 + r16) * PROMPT_BS + half * 8;
+          h16* dst = p.vcache + at_page[i] + (nt * 16 + r16) * PROMPT_BS + half * 8;
           if (pos + 8 <= len) {
             *reinterpret_cast<h16x8*>(dst) = v;
           } else {   // the prompt ends inside: slots behind it are not this prompt's to write
