@@ -49,7 +49,7 @@ $(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_linear.hp
 
 layer: $(LAYER_LIB)
 
-$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp $(CSRC)/gpt2_rows.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp include/vmi_gpt2_layer.h
+$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp $(CSRC)/gpt2_rows.hpp $(CSRC)/gpt2_head.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp include/vmi_gpt2_layer.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $< -o $@
 

@@ -109,6 +109,12 @@ VMI_LAYER_API int vmi_gpt2_add_norm_f16(void* x, const void* add, const int32_t*
 VMI_LAYER_API int vmi_gpt2_linear_tiles_f16(const void* x, const void* w, const void* bias, const void* res, void* y, int32_t M, int32_t N, int32_t K,
                                             int32_t epilogue, int32_t device, void* stream);
 
+/* logits [M][ld] (N columns) = norm(x [M, K], row m at x[rows[m]] or, rows NULL, x[m]) w^T for few rows: w packed tiles (w_layout 1) of ceil(N / 16) slabs, zeros past
+ * N; gamma and beta [K] (both NULL: no norm).  vmi_gpt2_head_fits: whether so many rows of K halves are taken. */
+VMI_LAYER_API int32_t vmi_gpt2_head_fits(int32_t M, int32_t K);
+VMI_LAYER_API int vmi_gpt2_head_f16(const void* x, int64_t ldx, const int32_t* rows, const void* gamma, const void* beta, float eps, const void* w, void* logits, int64_t ld,
+                                    int32_t M, int32_t N, int32_t K, int32_t device, void* stream);
+
 /* All layers of whole prompts, the launches of vmi_gpt2_embed_f16, then per layer vmi_gpt2_linear_f16 (norm, c_attn),
  * vmi_gpt2_prompt_attention_f16, vmi_gpt2_linear_f16 (c_proj, residual), (norm, c_fc, GELU), (c_proj, residual), then vmi_gpt2_add_norm_f16 of
  * the prompts' last rows, issued from one call: a prompt of a few dozen tokens takes the GPU less time than sixty calls take an interpreter.

@@ -772,3 +772,27 @@ def test_a_steps_inputs_go_where_its_launches_read_them(head, rows, ld, used, n)
         gl.step_inputs(buf, to, head + 32, rows, ld, used, None, out)
     with pytest.raises(RuntimeError):
         gl.step_inputs(buf, to, head, rows, ld, used, ids.int() if n else out.int(), out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,V,E", [(1, 50257, 768), (16, 50257, 768), (15, 33000, 32), (16, 1003, 1152), (5, 15, 416), (16, 4096, 384), (3, 32784, 1536), (2, 100001, 64), (9, 70001, 800)])
+@pytest.mark.parametrize("norm", [True, False])
+def test_logits_of_few_rows(M, V, E, norm):
+    """head(): fewer slabs than waves and several a wave, the last one cut, one to three chunks of K, rows with a stride, an odd number of columns."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + V + E)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    x, w = (rnd(M, E + 8) * 2 + 0.5).half()[:, :E], (rnd(V, E) / E ** 0.5).half()
+    ln = ((1 + 0.2 * rnd(E)).half(), (0.1 * rnd(E)).half(), 1e-5) if norm else None
+    assert gl.head_fits(M, E)
+    got = gl.head(x, gl.pack_head(w), ln)
+    h = torch.nn.functional.layer_norm(x.float(), (E,), ln[0].float(), ln[1].float(), 1e-5).half() if norm else x
+    want = h.double() @ w.double().T
+    # half a unit in the last place of the result, the float32 sum, and (norm) rows that round the other way: one in thousands of them, 2^-10 of its product
+    bound = 2.0 ** -11 * want.abs() + 2.0 ** -20 * E ** 0.5 + (2.0 ** -10 * 4 / E ** 0.5 if norm else 0) + 2.0 ** -24
+    assert got.shape == (M, V) and bool(((got.double() - want).abs() <= 1.01 * bound).all()), float(((got.double() - want).abs() / bound).max())
+    assert not gl.head_fits(17, E) and not gl.head_fits(M, 1568)
+    with pytest.raises(RuntimeError):
+        gl.head(x.float(), gl.pack_head(w), ln)

@@ -87,7 +87,7 @@ EXTRAS_LIB_PATH = os.path.join(OUT_DIR, "libvmi_paged_attention_extras.so")
 # the decode harness's own library (include/vmi_gpt2_layer.h): the GPT-2 block's linear layers — one unit, no shared objects,
 # not part of the operators' boundary; loaded by vllmini_amd/gpt2_layer.py only
 SRC_LAYER = os.path.join(CSRC, "gpt2_layer.hip")
-HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(CSRC, "gpt2_rows.hpp"), os.path.join(CSRC, "mfma_tiles.hpp"), os.path.join(CSRC, "step_inputs.hpp"), os.path.join(INCLUDE, "vmi_gpt2_layer.h")]
+HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(CSRC, "gpt2_rows.hpp"), os.path.join(CSRC, "gpt2_head.hpp"), os.path.join(CSRC, "mfma_tiles.hpp"), os.path.join(CSRC, "step_inputs.hpp"), os.path.join(INCLUDE, "vmi_gpt2_layer.h")]
 LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 
 # the layers of decoders that mix recurrences, linear and softmax attention (include/vmi_hybrid.h), loaded by hybrid_ops.py only

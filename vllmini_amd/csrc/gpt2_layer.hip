@@ -673,6 +673,7 @@ __global__ __launch_bounds__(SK_T) void sample_top_k_kernel(const h16* __restric
 
 #include "gpt2_prompt.hpp"
 #include "gpt2_rows.hpp"
+#include "gpt2_head.hpp"
 
 namespace vmi_layer {
 
@@ -1108,6 +1109,33 @@ int vmi_gpt2_linear_tiles_f16(const void* x, const void* w, const void* bias, co
   const int rc = run_tiles(p, epilogue, static_cast<hipStream_t>(stream));
   if (prev != device) (void)hipSetDevice(prev);
   return rc;
+}
+
+int32_t vmi_gpt2_head_fits(int32_t M, int32_t K) {
+  using namespace vmi_layer;
+  return M > 0 && M <= 16 && K >= 32 && (K & 31) == 0 && K <= HEAD_MAX_K;
+}
+
+int vmi_gpt2_head_f16(const void* x, int64_t ldx, const int32_t* rows, const void* gamma, const void* beta, float eps, const void* w, void* logits, int64_t ld, int32_t M,
+                      int32_t N, int32_t K, int32_t device, void* stream) {
+  using namespace vmi_layer;
+  static const char* who = "vmi_gpt2_head_f16";
+  if (!x || !w || !logits || (gamma == nullptr) != (beta == nullptr) || N <= 0 || N > (1 << 24) || ld < N || ldx < K) {
+    set_err(who, ": null pointer or a size out of range");
+    return VMI_LAYER_E_ARG;
+  }
+  if (!vmi_gpt2_head_fits(M, K) || (ldx & 7) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) || ((uintptr_t)gamma & 15) || ((uintptr_t)beta & 15)) {
+    set_err(who, ": needs at most 16 rows, K % 32 == 0 and at most 1536, rows and weights aligned to 16 bytes");
+    return VMI_LAYER_E_SHAPE;
+  }
+  const HeadParams p{static_cast<const h16*>(x), ldx, rows, static_cast<const h16*>(gamma), static_cast<const h16*>(beta), eps, static_cast<const h16*>(w),
+                     static_cast<h16*>(logits), ld, M, N, K};
+  int prev = -1;
+  if (int rc = with_device(who, device, &prev)) return rc;
+  const int SL = (N + 15) >> 4, wgs = (SL + HEAD_RW - 1) / HEAD_RW;
+  auto* fn = gamma ? head_kernel<true> : head_kernel<false>;
+  hipLaunchKernelGGL(fn, dim3(wgs < 256 ? wgs : 256), dim3(64 * HEAD_RW), head_lds(K), static_cast<hipStream_t>(stream), p);
+  return after_launch(who, prev, device);
 }
 
 int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream) {

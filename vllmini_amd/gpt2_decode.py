@@ -14,7 +14,7 @@ for what the operators are actually batched over:
     (`native_layers`, vllmini_amd/gpt2_layer.py -> csrc/gpt2_layer.hip): LayerNorm + c_attn, c_proj + residual,
     LayerNorm + c_fc + GELU, mlp.c_proj + residual — four launches per layer where the torch modules take eleven
     (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt, layer_norm,
-    gelu), which lm_head always uses, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products but c_fc.
+    gelu), which lm_head uses for more than 16 rows, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products but c_fc.
 
 `reference_off_by_one=True` reproduces the reference caller's seq_lens (length BEFORE the new
 token, scheduler.py:96, so the newest token is not attended); the default attends to it.
@@ -181,6 +181,12 @@ class GPT2PagedDecoder:
             self.prompt_kernel = self._find_prompt_tensors()
         if self.prompt_kernel:
             gpt2_layer.load()
+        # the vocabulary's weight once more for steps and prompts of few rows (gpt2_layer.head): 77 MB for GPT-2 small
+        head, ends = state_dict.get("lm_head.weight"), [state_dict.get(f"transformer.ln_f.{k}") for k in ("weight", "bias")]
+        self._head = None
+        if self.native_layers and gpt2_layer.head_fits(1, E) and head is not None and head.dim() == 2 and head.shape[1] == E and gpt2_layer.takes_weights([head]) \
+                and all(t is not None and t.shape == (E,) for t in ends) and gpt2_layer.takes_weights(ends):
+            self._head = gpt2_layer.pack_head(head)
         self.pad_batch_to = int(pad_batch_to)      # decode steps are laid out for the next multiple of this many rows (0: as they come)
 
     def _find_prompt_tensors(self) -> bool:
@@ -210,6 +216,13 @@ class GPT2PagedDecoder:
     def _ln(self, x, prefix):
         return F.layer_norm(x, (self.dims.n_embd,), self.sd[prefix + ".weight"], self.sd[prefix + ".bias"],
                             self.dims.layer_norm_epsilon)
+
+    def _logits(self, x, normed: bool):
+        """lm_head of rows x, behind the final norm unless they are normed."""
+        if self._head is not None and gpt2_layer.head_fits(x.shape[0], x.shape[1]):
+            sd, p = self.sd, "transformer.ln_f."
+            return gpt2_layer.head(x, self._head, None if normed else (sd[p + "weight"], sd[p + "bias"], self.dims.layer_norm_epsilon))
+        return F.linear(x if normed else self._ln(x, "transformer.ln_f"), self.sd["lm_head.weight"])
 
     def _mlp(self, x, p):                                      # gpt2.py:117-128 (nn.GELU = exact erf form)
         h = F.linear(x, self.sd[p + "mlp.c_fc.weight"], self.sd[p + "mlp.c_fc.bias"])
@@ -382,7 +395,7 @@ class GPT2PagedDecoder:
             weights, ends = self._prompt_tensors
             h = gpt2_layer.prompts(weights, ends, up["ids"], up["pos"], up["last"], up["tiles"], tile_rows, up["tables"], pool.key_cache,
                                    pool.value_cache, H, d.head_size, d.layer_norm_epsilon, self.scale)
-            return F.linear(h, sd["lm_head.weight"])
+            return self._logits(h, True)
         tiles = self.native_layers and d.n_embd % 64 == 0 and T * d.n_embd < 1 << 31
         x, add = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"]), None
         for i in range(d.n_layer):
@@ -398,7 +411,7 @@ class GPT2PagedDecoder:
                 add = self._mlp(h, p)
         x += add
         h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
-        return F.linear(h, sd["lm_head.weight"])
+        return self._logits(h, True)
 
     def _prefill_variant(self) -> int:
         """The work decomposition of the prefill launch.  Its "sequences" are the positions of a few prompts: thousands of short
@@ -476,7 +489,7 @@ class GPT2PagedDecoder:
             cache_ops.reshape_and_cache(rows[:, E:2 * E].view(d.n_layer * B, d.n_head, d.head_size),
                                         rows[:, 2 * E:].view(d.n_layer * B, d.n_head, d.head_size),
                                         pool.key_cache, pool.value_cache, st["slots"].view(-1), pool.kv_cache_dtype, pool.kv_scale)
-        return F.linear(self._ln(x, "transformer.ln_f"), self.sd["lm_head.weight"])   # [B, V]
+        return self._logits(x, False)   # [B, V]
 
     def _ensure_static(self, B: int) -> dict:
         """The static device buffers, pinned staging buffers and captured graphs of batch size B (kept per size: a serving

@@ -41,6 +41,8 @@ SIGNATURES = {
     "vmi_gpt2_linear_qkv_cache_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i64, _i32, _i32, _i32,
                                                      _vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
+    "vmi_gpt2_head_fits": (_i32, [_i32, _i32]),
+    "vmi_gpt2_head_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp]),
     "vmi_gpt2_prompt_attention_f16": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, ctypes.c_float, _vp, _vp,
                                                      _vp, _i32, _i32, _i64, _i64, _i32, _vp]),
@@ -233,6 +235,39 @@ def linear_qkv_cache(x: torch.Tensor, weight, bias: Optional[torch.Tensor], key_
 def _check(rc: int) -> None:
     if rc != 0:
         raise RuntimeError(load().vmi_gpt2_layer_last_error().decode("utf-8", "replace"))
+
+
+def pack_head(weight: torch.Tensor) -> PackedWeight:
+    """A vocabulary's weight [V, E] for head(): packed, zero rows up to a multiple of 16."""
+    V, E = weight.shape
+    padded = torch.zeros(((V + 15) // 16 * 16, E), dtype=weight.dtype, device=weight.device)
+    padded[:V] = weight
+    packed = PackedWeight(padded)
+    packed.shape = (V, E)
+    return packed
+
+
+def head_fits(rows: int, width: int) -> bool:
+    """Whether head() takes that many rows."""
+    return bool(load().vmi_gpt2_head_fits(rows, width))
+
+
+def head(x: torch.Tensor, weight: PackedWeight, ln: Optional[Tuple[torch.Tensor, torch.Tensor, float]] = None) -> torch.Tensor:
+    """Logits [M, V] of few rows x [M, E] behind the final norm (None: as they are), weight from pack_head()."""
+    lib = load()
+    if x.device.type != "cuda":
+        raise RuntimeError("gpt2_layer.head: there is no CPU path")
+    (V, E), M = weight.shape, x.shape[0]
+    if x.dim() != 2 or x.dtype != torch.float16 or x.shape[1] != E or x.stride(1) != 1 or weight.tiles.device != x.device or weight.tiles.numel() < (V + 15) // 16 * 16 * E:
+        raise RuntimeError("gpt2_layer.head: x half [M, E], unit column stride, and pack_head()'s weight beside it")
+    if ln is not None:
+        for t in ln[:2]:
+            if t.dtype != torch.float16 or t.shape != (E,) or not t.is_contiguous() or t.device != x.device:
+                raise RuntimeError("gpt2_layer.head: the norm's weight and bias half [E], contiguous, on x's device")
+    out = torch.empty((M, V), dtype=torch.float16, device=x.device)
+    _check(lib.vmi_gpt2_head_f16(x.data_ptr(), x.stride(0), None, ln[0].data_ptr() if ln else None, ln[1].data_ptr() if ln else None, ln[2] if ln else 0.0,
+                                 weight.tiles.data_ptr(), out.data_ptr(), V, M, V, E, x.device.index or 0, torch.cuda.current_stream(x.device).cuda_stream))
+    return out
 
 
 def step_inputs(host: PinnedBuffer, dev: torch.Tensor, head: int, rows: int, ld: int, used: int, ids: Optional[torch.Tensor], ids_out: torch.Tensor) -> None:
