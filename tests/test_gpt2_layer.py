@@ -796,3 +796,32 @@ def test_logits_of_few_rows(M, V, E, norm):
     assert not gl.head_fits(17, E) and not gl.head_fits(M, 1568)
     with pytest.raises(RuntimeError):
         gl.head(x.float(), gl.pack_head(w), ln)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,ctx", [(32, 100), (16, 200), (1, 800), (4, 300), (12, 250)])
+def test_steps_read_their_pages_past_the_caches_with_the_same_results(B, ctx, monkeypatch):
+    """_past_caches: where a step takes another variant than the operators would, it is the same split of a head over waves without a temporal load, and logits and caches
+    agree (to the bit where a wave takes its blocks one by one in both)."""
+    from vllmini_amd import ops
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+    from vllmini_amd.kv_pool import PagedKVPool
+
+    dims, dev = GPT2Dims(vocab_size=200, n_layer=2), torch.device("cuda:0")
+    sd = random_state_dict(dims, dev)
+    names, got = ops.variant_names(), []
+    for past in (True, False):
+        if not past:
+            monkeypatch.setattr(GPT2PagedDecoder, "_past_caches", lambda self, variant, B: variant)
+        pool = PagedKVPool(B * dims.n_layer * 64 + 8, dims.n_head, dims.head_size, 16, 64, dims.n_layer, device=dev, max_seqs=B, multi_block_prefill=True)
+        d = GPT2PagedDecoder(dims, sd, pool)
+        d.prefill_batch(list(range(B)), [[(7 * s + j) % 200 for j in range(ctx - s % 5)] for s in range(B)])
+        out = [d.decode(list(range(B)), torch.full((B,), 3 + i, device=dev), use_graph=True).clone() for i in range(3)]
+        got.append((names[d._static["variant"] - 1], out, pool.key_cache.clone(), pool.value_cache.clone()))
+    (a, x, ka, va), (b, y, kb, vb) = got
+    if a != b:
+        assert a.endswith("_u1_nt1") and b.endswith("_nt0") and a.rsplit("_u", 1)[0] == b.rsplit("_u", 1)[0]
+    if a.replace("nt1", "nt0") == b.replace("nt1", "nt0"):
+        assert all(torch.equal(p, q) for p, q in zip(x, y)) and torch.equal(ka, kb) and torch.equal(va, vb)
+    for p, q in zip(x, y):
+        assert float((p.float() - q.float()).norm() / q.float().norm()) <= 2e-3

@@ -27,6 +27,7 @@ from __future__ import annotations
 import dataclasses
 import itertools
 import math
+import re
 from typing import Dict, List, Optional, Sequence
 
 import numpy as np
@@ -150,6 +151,7 @@ class GPT2PagedDecoder:
         if not can_scatter:
             self.scatter_in_c_attn = False
         self._packed: Dict[str, gpt2_layer.PackedWeight] = {}
+        self._cold: Optional[Dict[int, tuple]] = None
         self._prompt_tensors = None                # what gpt2_layer.prompts reads
         self.NATIVE_PROMPT_MAX_TOKENS = min(self.NATIVE_PROMPT_MAX_TOKENS, self.NATIVE_PROMPT_MAX_WORK // (E * E))
         if self.native_layers:
@@ -539,6 +541,21 @@ class GPT2PagedDecoder:
         m = self.pad_batch_to
         return B if not m or B % m == 0 else (B // m + 1) * m
 
+    def _past_caches(self, variant: int, B: int) -> int:
+        """The same split of heads over waves with non-temporal loads of the pages.  The operators' choice for a small batch is temporal, measured on pages that the call before has read;
+        a step reads other pages in every layer, and all layers' weights go through the caches in between.  12 layers of 12 heads of 64, a step in us: 32 sequences of up to 128
+        tokens 339 -> 327, 20 of 200 326 -> 315, 13 of 300 325 -> 317, 8 of 600 334 -> 316, 4 of 900 348 -> 333, 1 of 900 332 -> 323.  Two blocks a wave at once stay where fewer than
+        16 waves a head and few heads leave them to: 4 of 400 312 against 316, 1 of 300 289 against 291."""
+        if self._cold is None:
+            names = ops.variant_names() if self.pool.kv_cache_dtype == "auto" and self.dims.head_size == 64 and self.pool.block_size == 16 else []
+            at, self._cold = {n: i + 1 for i, n in enumerate(names)}, {}
+            for n in at:
+                m = re.fullmatch(r"(d64_h1_w(\d+))_u(\d+)_nt0", n)
+                if m and f"{m[1]}_u1_nt1" in at:
+                    self._cold[at[n]] = at[f"{m[1]}_u1_nt1"], int(m[2]) < 16 and int(m[3]) > 1
+        to, many_only = self._cold.get(variant, (variant, False))
+        return variant if many_only and B * self.dims.n_head < 128 else to
+
     def stage_step(self, seq_ids: Sequence[int], input_ids) -> dict:
         """Host bookkeeping for one step + ONE upload of all of it into the static device buffers.  With pad_batch_to the
         step is laid out for the next multiple of it: the padding rows are empty sequences (length 0: the attention writes
@@ -590,6 +607,7 @@ class GPT2PagedDecoder:
                                          self.pool.block_size, mean_seq_len=max(int(lens.sum()) // Bp, 1),
                                          bf16=self.pool.key_cache.dtype == torch.bfloat16,
                                          fp8={"auto": False, "fp8_e5m2": "e5m2"}.get(self.pool.kv_cache_dtype, True))
+        st["variant"] = self._past_caches(st["variant"], Bp)
         # few sequences x long contexts: with the wrapper's workspace the library spreads a head over several workgroups
         # (ops.pick_variant(workspace=True) names a split kernel, "_x<waves>", exactly where the default entry would run one)
         # (only when the launch WILL carry a workspace: the wrapper's switch is on and one exists for this stream — none is
