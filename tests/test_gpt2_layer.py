@@ -793,7 +793,7 @@ def test_logits_of_few_rows(M, V, E, norm):
     # half a unit in the last place of the result, the float32 sum, and (norm) rows that round the other way: one in thousands of them, 2^-10 of its product
     bound = 2.0 ** -11 * want.abs() + 2.0 ** -20 * E ** 0.5 + (2.0 ** -10 * 4 / E ** 0.5 if norm else 0) + 2.0 ** -24
     assert got.shape == (M, V) and bool(((got.double() - want).abs() <= 1.01 * bound).all()), float(((got.double() - want).abs() / bound).max())
-    assert not gl.head_fits(17, E) and not gl.head_fits(M, 1568)
+    assert gl.HEAD_MAX_ROWS == 16 and not gl.head_fits(17, E) and not gl.head_fits(M, 1568)
     with pytest.raises(RuntimeError):
         gl.head(x.float(), gl.pack_head(w), ln)
 

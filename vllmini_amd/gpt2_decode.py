@@ -221,7 +221,7 @@ class GPT2PagedDecoder:
 
     def _logits(self, x, normed: bool):
         """lm_head of rows x, behind the final norm unless they are normed."""
-        if self._head is not None and gpt2_layer.head_fits(x.shape[0], x.shape[1]):
+        if self._head is not None and 0 < x.shape[0] <= gpt2_layer.HEAD_MAX_ROWS:
             sd, p = self.sd, "transformer.ln_f."
             return gpt2_layer.head(x, self._head, None if normed else (sd[p + "weight"], sd[p + "bias"], self.dims.layer_norm_epsilon))
         return F.linear(x if normed else self._ln(x, "transformer.ln_f"), self.sd["lm_head.weight"])

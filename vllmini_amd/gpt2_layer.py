@@ -247,8 +247,11 @@ def pack_head(weight: torch.Tensor) -> PackedWeight:
     return packed
 
 
+HEAD_MAX_ROWS = 16
+
+
 def head_fits(rows: int, width: int) -> bool:
-    """Whether head() takes that many rows."""
+    """Whether head() takes that many rows of that width."""
     return bool(load().vmi_gpt2_head_fits(rows, width))
 
 
