@@ -114,7 +114,7 @@ typedef struct {
   const int32_t* q_start;    /* [B] first token of the entry's portion */
   const int32_t* q_len;      /* [B] */
   const int32_t* ctx;        /* [B] tokens before the portion */
-  const int32_t* state_slot; /* [B] */
+  const int32_t* state_slot; /* [B]; anything in an entry without tokens, as in its q_start, q_len, ctx and flip where every portion is one token */
   const int32_t* flip;       /* [B] which half of the convolution tail holds the inputs before the portion (0 / 1) */
   const int32_t* table;      /* [B, table_ld] pages */
   const int32_t* chunks;     /* [n_chunks][2]: (entry, first row inside its portion) of every run of up to 16 rows */

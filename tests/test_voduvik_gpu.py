@@ -475,6 +475,32 @@ def test_recurrence_decodes_like_it_prefills_and_skips_padding_rows(dtype):
     assert torch.equal(k.state[B], untouched)
 
 
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("width,blocks,taps", [(96, 3, 4), (1536, 2, 4), (288, 9, 6)])
+def test_entries_of_padding_rows_name_no_state(dtype, width, blocks, taps):
+    """Single tokens among padding rows whose entries hold a slot, a context and a flip that are none: zeros come out, and no state and no tail is read or written for them."""
+    k = _Rglru(width, blocks, taps, dtype, slots=4)
+    from vllmini_amd import hybrid_ops as ops
+
+    at = [1, 4, 18]      # rows of the three sequences, of twenty
+    seqs = [k.inputs(2, 70 + i) for i in range(3)]
+    for t in range(2):
+        step = layout([1] * 20, [-1] * 20, [[0]] * 20, 64, slots=[-1 - 1000 * i for i in range(20)], flips=[-5] * 20, pos_slots=False)
+        f = dict(step.fields)
+        f["tok_seq"] = torch.full_like(f["tok_seq"], -1)
+        for i, row in enumerate(at):
+            f["tok_seq"][row], f["ctx"][row], f["state_slot"][row], f["flip"][row] = row, t, i, t & 1
+        yx = torch.full((20, 2 * k.layer.width), float("nan"), dtype=dtype, device=dev())
+        for i, row in enumerate(at):
+            yx[row] = seqs[i][2][t]
+        tail = k.tail[3].clone()
+        got = k.run(yx, ops.StepLayout(f, 20, 20, 64, True, False, 1, t + 1))
+        for i, row in enumerate(at):
+            close(got[row], k.plain(*seqs[i][:2])[t], dtype, tol32=1e-4, tol16=3e-2)
+        assert not got[[r for r in range(20) if r not in at]].any()
+        assert bool((k.state[3] == 7).all()) and torch.equal(k.tail[3], tail)
+
+
 @pytest.mark.parametrize("width,blocks,taps,B", [(96, 1, 4, 1), (2560, 10, 4, 16), (2112, 3, 4, 70), (1536, 2, 4, 33), (288, 9, 6, 40), (4096, 16, 4, 70)])
 def test_single_tokens_share_a_gate_block_over_waves_and_workgroups(width, blocks, taps, B):
     """rglru_step_kernel with one, two and four tiles of channels a workgroup (the last one's not all there), blocks of fewer and more channels than its waves take at

@@ -376,6 +376,7 @@ __global__ __launch_bounds__(512, 2) void rglru_step_kernel(const vmi_hy_rglru_a
     const int t = t0 + min(m, rows - 1), e = min(t, s.B - 1);
     Row r{s.tok_seq[t], s.ctx[e], s.state_slot[e], s.flip[e]};
     if (r.seq >= 0 && r.seq != e) r.ctx = s.ctx[r.seq], r.slot = s.state_slot[r.seq], r.flip = s.flip[r.seq];   // (tokens in another order than entries)
+    if (r.seq < 0) r.ctx = r.slot = r.flip = 0;   // (a padding row's entry may hold anything: it reads the first state and stores none)
     return r;
   };
   const b16* yx = static_cast<const b16*>(p.yx);
