@@ -351,6 +351,17 @@ def test_large_products_stay_with_the_library_unless_their_rows_stay_in_lds():
     assert not hybrid_layers.dense(16, of(8192, 4096), True) and h.linear_normed_first(17, of(8192, 4096)) and not h.linear_normed_first(17, of(8192, 4096, 2))
 
 
+def test_products_behind_a_norm_of_few_rows_and_columns_share_one_kernel_whatever_their_width():
+    """Up to 2048 columns, up to 64 rows, one workgroup a compute unit with one slab of 16 columns each: no width among them goes to kernels for more."""
+    from vllmini_amd import hybrid_ops as h
+
+    for K in range(32, 2049, 32):
+        for M in (1, 12, 16, 17, 33, 47, 64):
+            for N in (32, 512, 16 * (256 // -(-M // 16))):
+                assert h.load().vmi_hy_linear_slabs(M, N, K, 0) > 0 and not h.load().vmi_hy_linear_normed(M, N, K, 1, 0), (M, N, K)
+    assert h.load().vmi_hy_linear_slabs(12, 512, 2080, 0) == h.load().vmi_hy_linear_slabs(12, 512, 1024, 1) == h.load().vmi_hy_linear_slabs(12, 512, 1000, 0) == 0
+
+
 def test_command_line_lists_models_and_parses_requests(capsys):
     from vllmini_amd.__main__ import _parser, main
 

@@ -204,14 +204,17 @@ def test_many_columns_leave_the_rows_in_lds(M, N, K):
     _norm_products(M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(7, 16 * 515, 1024), (33, 16 * 387, 1024), (17, 16 * 389, 1024), (64, 16 * 130, 1024), (40, 16 * 510, 1024), (3, 16 * 257, 2048), (31, 16 * 129, 2048),
-                                   (18, 16 * 259, 1536), (50, 16 * 129, 768), (70, 16 * 255, 512), (90, 16 * 85, 256), (21, 16 * 200, 96), (35, 16 * 330, 992)])
-def test_few_rows_behind_a_norm_take_several_slabs_a_workgroup(M, N, K):
-    """norm_rows_kernel with two to six slabs of 16 columns a workgroup, the last workgroup's not all there, for every length of a row it is built for, shared
+@pytest.mark.parametrize("M,N,K,slabs", [(7, 16 * 515, 1024, 3), (33, 16 * 387, 1024, 6), (17, 16 * 389, 1024, 4), (64, 16 * 130, 1024, 3), (40, 16 * 510, 1024, 6), (3, 16 * 257, 2048, 2),
+                                         (31, 16 * 129, 2048, 2), (18, 16 * 254, 1536, 2), (5, 16 * 99, 1536, 1), (50, 16 * 129, 768, 4), (40, 16 * 254, 512, 4), (90, 16 * 85, 256, 4),
+                                         (21, 16 * 200, 96, 2), (35, 16 * 330, 992, 4), (9, 16 * 255, 1056, 1), (20, 16 * 201, 1152, 2), (33, 16 * 77, 1280, 1), (64, 16 * 127, 1792, 2),
+                                         (1, 16 * 511, 1888, 2), (47, 32, 2016, 1)])
+def test_few_rows_behind_a_norm_take_several_slabs_a_workgroup(M, N, K, slabs):
+    """norm_rows_kernel with one to six slabs of 16 columns a workgroup, the last workgroup's not all there, for every length of a row it is built for, shared
     out evenly and not."""
     from vllmini_amd import hybrid_ops as ops
 
-    assert not ops.linear_normed_first(M, _norm_products(M, ops.pad32(N), K))
+    w = _norm_products(M, ops.pad32(N), K)
+    assert ops.linear_slabs(M, w) == slabs and not ops.linear_normed_first(M, w)
 
 
 @pytest.mark.parametrize("M,N,K", [(9, 16 * 513, 2048), (16, 16 * 1030, 2048), (32, 16 * 770, 2048), (33, 16 * 400, 2048), (64, 16 * 514, 2048), (50, 16 * 770, 1024), (12, 16 * 258, 4096),

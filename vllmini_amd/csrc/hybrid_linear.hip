@@ -449,7 +449,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   if constexpr (PLAIN)
     if (plain_rows_fit(p.M)) return launch_plain_rows(p, st);
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
-    if (p.groups == 1 && norm_rows_fit(p.M, p.N, p.K)) return launch_norm_rows(p, st);
+    if (p.groups == 1 && norm_slabs(p.M, p.N, p.K)) return launch_norm_rows(p, st);
     switch (p.groups == 1 && resident_pays(p.M, p.N, p.K) ? resident_kind(p.M, p.N, p.K) : 0) {
       case 2: return p.M <= 16 ? launch_resident<1, 8, 2, 2, EPI>(p, st) : launch_resident<2, 8, 2, 2, EPI>(p, st);
       case 3: return launch_resident<2, 8, 1, 2, EPI>(p, st);
@@ -683,6 +683,10 @@ int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, in
 
 int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
   return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && resident_kind(M, N, K) != 0;
+}
+
+int32_t vmi_hy_linear_slabs(int32_t M, int32_t N, int32_t K, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && (K & 31) == 0 && (N & 15) == 0 ? norm_slabs(M, N, K) : 0;
 }
 
 int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype) {

@@ -55,7 +55,7 @@ __device__ __forceinline__ void epilogue(const vmi_hy_linear_args& p, const f32x
 }
 
 // Products of few rows in bfloat16 (hybrid_rows.hip).  Each is built for what its rule names
-bool norm_rows_fit(int M, int N, int K);   // behind a norm, one group
+int norm_slabs(int M, int N, int K);   // behind a norm, one group: 0 where it is not
 int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool held_rows_pay(int M, int N, int K);   // of the element type behind a norm of their own, one group
 int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st);

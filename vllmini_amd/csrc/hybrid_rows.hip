@@ -357,10 +357,10 @@ int launch_norm_few(const vmi_hy_linear_args& p, hipStream_t st) {
 }
 
 // Slabs a workgroup of norm_rows_kernel takes: as few as leave one workgroup a compute unit; 0: the kernel is not built for these sizes, or they are more than
-// that.  Up to 1024 columns, and 1536 and 2048, whose rows a workgroup's 16 waves share without a remainder (else the addresses cost the registers: 7.5 -> 14.5 us).
-static int norm_slabs(int M, int N, int K) {
+// that.  Rows of up to 2048 columns; past 1024 sixteen waves share one, whose registers hold two slabs.
+int norm_slabs(int M, int N, int K) {
   const int nks = K >> 5, rb = (M + 15) >> 4;
-  if (nks > 32 && nks != 48 && nks != 64) return 0;
+  if (nks > 64) return 0;
   for (int ns : {1, 2, 3, 4, 6}) {
     if (ns > 2 && nks > 32) break;
     if ((ns == 3 || ns == 6) && nks != 32) continue;
@@ -370,8 +370,8 @@ static int norm_slabs(int M, int N, int K) {
 }
 // rows_kernel's forerunner (an eighth of K a wave, rows in the matrix cores' layout), resident_kernel or linear_kernel, whichever was ahead / norm_rows_kernel, in a graph of such
 // launches, us: K 1024, N 2048 1 / 12 / 32 / 40 rows 4.7 / 5.6 / 6.0 / 8.6 -> 4.2 / 4.4 / 4.5 / 4.8, N 6144 6.5 / 8.2 / 11.2 / 18.5 -> 5.2 / 5.3 / 5.6 / 6.5, N 10240 8.1 / 9.9 / 13.8
-// (32) -> 6.4 / 6.3 / 7.1; K 2048, N 4096 7.7 / 9.8 / 15.3 (32) -> 7.1 / 7.5 / 8.5.  More than a workgroup a compute unit: K 1024, N 10240, 40 rows 11.5 here, 11.0 in held_rows_kernel.
-bool norm_rows_fit(int M, int N, int K) { return norm_slabs(M, N, K) > 0; }
+// (32) -> 6.4 / 6.3 / 7.1; K 2048, N 4096 7.7 / 9.8 / 15.3 (32) -> 7.1 / 7.5 / 8.5.  Of widths in between (K 1152 to 1920, the forerunner's sizes), 1 / 12 / 32 / 47 rows: K 1152, N 2048 6.1 / 7.9 / 8.5 / 14.2 -> 5.6 / 5.7 / 5.8 /
+// 6.6; K 1280, N 4096 6.5 / 8.1 / 10.5 (32) -> 5.9 / 5.9 / 6.8; K 1792, N 512 6.2 / 8.1 / 8.7 / 8.7 -> 5.5 / 5.7 / 5.9 / 5.9; K 1920, N 4096 7.4 / 9.1 / 12.7 (32) -> 6.4 / 6.5 / 7.5.  More than a workgroup a compute unit: K 1024, N 10240, 40 rows 11.5 here, 11.0 in held_rows_kernel.
 
 template <int RW, int J, bool FULL, int EPI>
 static int norm_rows_of(const vmi_hy_linear_args& p, int ns, hipStream_t st) {
@@ -397,6 +397,7 @@ static int norm_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
   if (nks == 24) return norm_rows_of<8, 3, true, EPI>(p, ns, st);
   if (nks == 16) return norm_rows_of<8, 2, true, EPI>(p, ns, st);
   if (nks == 8) return norm_rows_of<8, 1, true, EPI>(p, ns, st);
+  if (nks > 32) return norm_rows_of<16, 4, false, EPI>(p, ns, st);
   return nks <= 16 ? norm_rows_of<8, 2, false, EPI>(p, ns, st) : norm_rows_of<8, 4, false, EPI>(p, ns, st);
 }
 

@@ -72,6 +72,7 @@ SIGNATURES = {
     "vmi_hy_linear_tiles_pay": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
+    "vmi_hy_linear_slabs": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_held": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
@@ -294,6 +295,11 @@ def linear_normed_first(M: int, w: MatrixTiles) -> bool:
 def linear_resident(M: int, w: MatrixTiles) -> bool:
     """Whether linear(x, w, norm=...) can keep M rows in LDS, unless it norms them first."""
     return w.groups == 1 and bool(load().vmi_hy_linear_resident(M, w.N, w.K, DTYPES[w.tiles.dtype]))
+
+
+def linear_slabs(M: int, w: MatrixTiles) -> int:
+    """Slabs of 16 columns a workgroup takes where linear(x, w, norm=...) runs in the kernel for few rows and few columns; 0: in another one."""
+    return load().vmi_hy_linear_slabs(M, w.N, w.K, DTYPES[w.tiles.dtype]) if w.groups == 1 else 0
 
 
 def linear_held(M: int, w: MatrixTiles) -> bool:
