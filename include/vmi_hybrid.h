@@ -75,6 +75,8 @@ VMI_HY_API int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32
 /* How many slabs of 16 columns a workgroup takes where a product of these sizes behind a norm (one that vmi_hy_linear_normed does not name) runs in the kernel
  * for few rows and few columns; 0: in another one */
 VMI_HY_API int32_t vmi_hy_linear_slabs(int32_t M, int32_t N, int32_t K, int32_t dtype);
+/* Whether a product of rows as they are, with what is stored, added or gated behind it, runs in the kernel for few rows */
+VMI_HY_API int32_t vmi_hy_linear_plain(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype);
 /* Whether a product of these sizes behind a norm (one that vmi_hy_linear_normed names) keeps its normed rows in registers: then it is ahead of a norm, a
  * library product and what follows it as well. */
 VMI_HY_API int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype);

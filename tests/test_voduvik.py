@@ -362,6 +362,20 @@ def test_products_behind_a_norm_of_few_rows_and_columns_share_one_kernel_whateve
     assert h.load().vmi_hy_linear_slabs(12, 512, 2080, 0) == h.load().vmi_hy_linear_slabs(12, 512, 1024, 1) == h.load().vmi_hy_linear_slabs(12, 512, 1000, 0) == 0
 
 
+def test_products_of_few_rows_over_many_columns_read_their_rows_once():
+    """The kernel whose every workgroup brings the rows again is for a workgroup a compute unit, or for rows that are few or short."""
+    from vllmini_amd import hybrid_ops as h
+
+    plain = h.load().vmi_hy_linear_plain
+    for K in (128, 512, 1024, 2048, 4096, 4608):
+        assert all(plain(M, 16 * (256 // g), K, g, 0) for M in (1, 16, 32, 64) for g in (1, 8))
+        assert plain(16, 8192, K, 1, 0) and not plain(65, 512, K, 1, 0)
+    for M, N, K, groups in ((47, 16384, 2048, 1), (24, 16384, 1280, 1), (64, 8192, 768, 1), (16, 16384, 4096, 1), (32, 6144, 4096, 1), (1, 6144, 5120, 1), (16, 1024, 5120, 1), (64, 16384, 128, 1),
+                            (64, 128, 512, 64), (47, 512, 128, 64), (64, 128, 256, 128)):
+        assert not plain(M, N, K, groups, 0), (M, N, K, groups)
+    assert plain(47, 576, 128, 64, 0) and plain(64, 6144, 12288, 1, 0) and not plain(1, 512, 128, 1, 1)
+
+
 def test_command_line_lists_models_and_parses_requests(capsys):
     from vllmini_amd.__main__ import _parser, main
 

@@ -228,9 +228,10 @@ def test_rows_normed_once_are_held_in_registers(M, N, K):
 
 @pytest.mark.parametrize("M", [1, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(48, 32), (16 * 130, 128), (32, 224), (16 * 133, 480), (16 * 131, 992), (64, 1024), (16 * 129, 2016), (32, 2080), (96, 3072), (32, 4064), (48, 4576), (32, 4640),
-                                 (16 * 130, 4640), (48, 9248)])
+                                 (16 * 130, 4640), (48, 9248), (16 * 386, 96), (16 * 258, 1056), (16 * 514, 2080), (16 * 386, 8224)])
 def test_few_rows_as_they_are(M, N, K):
-    """plain_rows_kernel: K in one chunk a wave and in several, waves with unequal parts or none, one and two row tiles a workgroup; the rows of a wider matrix."""
+    """plain_rows_kernel: K in one chunk a wave and in several, waves with unequal parts or none, one and two row tiles a workgroup; the rows of a wider matrix; linear_kernel past
+    the line between them."""
     from vllmini_amd import hybrid_ops as ops
 
     g = torch.Generator(device=dev()).manual_seed(M * K + N)

@@ -447,7 +447,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
   constexpr bool PLAIN = sizeof(T) == 2 && XK == VMI_HY_X_ROWS && (EPI == VMI_HY_E_STORE || EPI == VMI_HY_E_RESIDUAL || EPI == VMI_HY_E_GATED);
   if constexpr (PLAIN)
-    if (plain_rows_fit(p.M)) return launch_plain_rows(p, st);
+    if (plain_rows_fit(p.M, p.N, p.K, p.groups)) return launch_plain_rows(p, st);
   if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_NORM) {
     if (p.groups == 1 && norm_slabs(p.M, p.N, p.K)) return launch_norm_rows(p, st);
     switch (p.groups == 1 && resident_pays(p.M, p.N, p.K) ? resident_kind(p.M, p.N, p.K) : 0) {
@@ -457,15 +457,13 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
       default: break;
     }
   }
-  if constexpr (!PLAIN) {
-    if (p.M <= 32) {
-      const int64_t wgs = slabs * ((p.M + 15) / 16);
-      if (wgs >= 2048) return launch_linear<T, 16, 4, 1, XK, EPI>(p, st);
-      if (wgs >= 400 || p.K < 256) return launch_linear<T, 16, 2, 2, XK, EPI>(p, st);
-      if constexpr (sizeof(T) == 2)
-        if (wgs < 192 && p.K >= 1024) return launch_linear<T, 16, 1, 8, XK, EPI>(p, st);
-      return launch_linear<T, 16, 1, 4, XK, EPI>(p, st);
-    }
+  if (p.M <= 32) {
+    const int64_t wgs = slabs * ((p.M + 15) / 16);
+    if (wgs >= 2048) return launch_linear<T, 16, 4, 1, XK, EPI>(p, st);
+    if (wgs >= 400 || p.K < 256) return launch_linear<T, 16, 2, 2, XK, EPI>(p, st);
+    if constexpr (sizeof(T) == 2)
+      if (wgs < 192 && p.K >= 1024) return launch_linear<T, 16, 1, 8, XK, EPI>(p, st);
+    return launch_linear<T, 16, 1, 4, XK, EPI>(p, st);
   }
   if (p.M <= 96 || slabs / 4 * ((p.M + 63) / 64) < 256) return launch_linear<T, 32, 4, 1, XK, EPI>(p, st);
   return launch_linear<T, 64, 4, 1, XK, EPI>(p, st);
@@ -687,6 +685,10 @@ int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
 
 int32_t vmi_hy_linear_slabs(int32_t M, int32_t N, int32_t K, int32_t dtype) {
   return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && (K & 31) == 0 && (N & 15) == 0 ? norm_slabs(M, N, K) : 0;
+}
+
+int32_t vmi_hy_linear_plain(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups > 0 && plain_rows_fit(M, N, K, groups);
 }
 
 int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype) {

@@ -59,7 +59,7 @@ int norm_slabs(int M, int N, int K);   // behind a norm, one group: 0 where it i
 int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool held_rows_pay(int M, int N, int K);   // of the element type behind a norm of their own, one group
 int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st);
-bool plain_rows_fit(int M);   // of the element type
+bool plain_rows_fit(int M, int N, int K, int groups);   // of the element type
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st);
 int launch_norm_few(const vmi_hy_linear_args& p, hipStream_t st);   // p.normed = the norm of p.x
 

@@ -453,7 +453,23 @@ int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 // linear_kernel / plain_rows_kernel, in a graph of such launches, us: K 1024, N 1024 1 / 16 / 32 / 64 rows 3.7 / 4.0 / 4.1 / 6.4 -> 2.9 / 3.1 / 3.1 / 3.2, K 3072, N 1024 4.8 / 5.4 / 5.5 / 13.0 ->
 // 3.8 / 4.4 / 4.5 / 4.6, K 8192, N 2048 10.7 / 13.3 / 14.2 / 44.5 -> 10.1 / 12.5 / 12.3 / 15.2, K 4096, N 4096 10.1 / 11.3 / 12.4 / 24.6 -> 8.1 / 9.0 / 10.7 / 17.1, K 12288, N 4096 20.8 / 22.5 / 27.9 /
 // 65.2 -> 20.0 / 21.6 / 25.3 / 41.4; 8 groups of K 128, N 512 3.7 / 3.9 / 4.0 / 3.4 -> 2.3 / 2.4 / 2.5 / 2.6, of K 512, N 128 4.0 / 4.5 / 4.5 / 5.1 -> 2.5 / 2.7 / 2.7 / 2.7.  Of more rows there are tiles.
-bool plain_rows_fit(int M) { return M <= 64; }
+// Every workgroup brings the rows again, so past one slab a compute unit (256) it is ahead only while the rows are few or short: K 2048, N 16384 1 / 32 / 64 rows 13.6 / 13.8 / 16.2 -> 12.7 / 16.8 / 30.8,
+// N 50272 42.8 (1) -> 35.0; K 4096, N 8192 8 / 24 / 64 14.2 / 14.0 / 20.7 -> 13.7 / 15.2 / 28.5, N 16384 16 rows 22.9 -> 24.8; K 512, N 16384 32 rows 7.1 -> 6.1, N 8192 64 rows 5.5 -> 6.0; K 128, N 50272 32
+// rows 10.5 -> 7.7; 32 / 64 groups of K 128, N 512 47 rows 4.2 / 5.3 -> 4.1 / 5.9 and, linear_kernel's nine column blocks of a group padded to sixteen, N 576 5.0 / 8.0 -> 4.4 / 6.5; 64 of K 256, N 128 4.5 -> 3.7.  Past 4608 columns
+// chunks follow each other: K 5120, N 6144 1 / 32 / 64 rows 12.6 / 15.1 / 22.0 -> 14.7 / 18.5 / 29.6, N 1024 16 rows 7.1 -> 7.6 (K 6144 7.9 -> 7.8, N 2048 8.5 -> 8.6), N 4096 10.4 -> 9.9; K 12288, N 6144 64 rows 66 -> 57.
+bool plain_rows_fit(int M, int N, int K, int groups) {
+  const int64_t slabs = (int64_t)(N >> 4) * groups;
+  if (M > 64) return false;
+  if (K > 4608) {
+    if (M > 32) return slabs <= (K > 8192 ? 384 : 256);
+    return slabs <= 256 && (slabs * ((M + 15) >> 4) >= 192 || (slabs <= 96 && K % 2048 == 0));   // (fewer: linear_kernel's eight waves are level, and ahead where a chunk is not whole)
+  }
+  if (M <= 16) return K <= 2048 || slabs <= 512;
+  if (M <= 32) return K <= 256 || slabs <= (K <= 512 ? 1024 : K <= 1024 ? 512 : 256);
+  const int blocks = (N + 63) >> 6, launched = blocks < 8 ? blocks : (blocks + 7) / 8 * 8;
+  if (groups > 1 && K <= 128) return slabs <= 1280 || launched * 2 >= blocks * 3;
+  return slabs <= (groups > 1 && K <= 256 ? 512 : K <= 512 ? 384 : 256);
+}
 
 // Row tiles share a workgroup (and its weights) once there are more workgroups than compute units.  Waves and k-steps a wave by the length of K: four to nine
 // k-steps a wave keep all of its part in flight; past 4608 columns chunks follow each other.
