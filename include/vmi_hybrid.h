@@ -80,6 +80,8 @@ VMI_HY_API int32_t vmi_hy_linear_plain(int32_t M, int32_t N, int32_t K, int32_t 
 /* Whether a product of these sizes behind a norm (one that vmi_hy_linear_normed names) keeps its normed rows in registers: then it is ahead of a norm, a
  * library product and what follows it as well. */
 VMI_HY_API int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype);
+/* Whether rows that are normed first are kept in registers, ahead of a library product or not; stored: what leaves the product is stored as it is */
+VMI_HY_API int32_t vmi_hy_linear_holds(int32_t M, int32_t N, int32_t K, int32_t stored, int32_t dtype);
 
 /* What a step's launches read: `bytes` (a multiple of 16) from `host`, pinned memory, to `dev`; and ids_out[0:n] = ids[0:n].  16-byte aligned; the host memory
  * is read when the launch runs. */

@@ -362,6 +362,19 @@ def test_products_behind_a_norm_of_few_rows_and_columns_share_one_kernel_whateve
     assert h.load().vmi_hy_linear_slabs(12, 512, 2080, 0) == h.load().vmi_hy_linear_slabs(12, 512, 1024, 1) == h.load().vmi_hy_linear_slabs(12, 512, 1000, 0) == 0
 
 
+def test_rows_normed_once_are_held_at_every_multiple_of_1024_columns():
+    """Whole chunks of K a wave are what the kernel that holds its rows in registers asks for, and few columns of long rows are left to kernels that share a slab's K out."""
+    from vllmini_amd import hybrid_ops as h
+
+    held, normed = h.load().vmi_hy_linear_held, h.load().vmi_hy_linear_normed
+    for K in (1024, 2048, 3072):
+        assert held(40, 50272, K, 0) and normed(40, 50272, K, 1, 0) and not held(65, 50272, K, 0) and not held(8, 50272, K, 0)
+    assert held(33, 512, 3072, 0) and held(9, 50272, 2048, 0) and not held(32, 50272, 3072, 0) and not held(40, 50272, 2560, 0) and not held(40, 50272, 4096, 0)
+    rows = h.load().vmi_hy_linear_holds
+    for M, N, stored, want in ((16, 4096, 1, 0), (16, 6144, 1, 1), (32, 8192, 1, 0), (32, 12288, 0, 1), (40, 512, 1, 0), (40, 512, 0, 1), (64, 4096, 1, 1)):
+        assert rows(M, N, 4096, stored, 0) == want, (M, N, stored)
+
+
 def test_products_of_few_rows_over_many_columns_read_their_rows_once():
     """The kernel whose every workgroup brings the rows again is for a workgroup a compute unit, or for rows that are few or short."""
     from vllmini_amd import hybrid_ops as h

@@ -218,7 +218,7 @@ def test_few_rows_behind_a_norm_take_several_slabs_a_workgroup(M, N, K, slabs):
 
 
 @pytest.mark.parametrize("M,N,K", [(9, 16 * 513, 2048), (16, 16 * 1030, 2048), (32, 16 * 770, 2048), (33, 16 * 400, 2048), (64, 16 * 514, 2048), (50, 16 * 770, 1024), (12, 16 * 258, 4096),
-                                   (40, 16 * 514, 4096)])
+                                   (40, 16 * 514, 4096), (33, 32, 3072), (50, 16 * 258, 3072), (40, 16 * 34, 3072), (64, 16 * 514, 3072), (16, 16 * 386, 4096), (32, 16 * 770, 4096)])
 def test_rows_normed_once_are_held_in_registers(M, N, K):
     """held_rows_kernel: one and two row tiles, row blocks, slabs that the workgroups do not share evenly, several chunks of K a slab and one."""
     from vllmini_amd import hybrid_ops as ops

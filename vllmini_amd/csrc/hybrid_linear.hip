@@ -471,7 +471,7 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
 
 // rows that stand in p.x normed: what follows a norm
 static int linear_normed(const vmi_hy_linear_args& p, hipStream_t st) {
-  if (p.groups == 1 && held_rows_pay(p.M, p.N, p.K)) return launch_held_rows(p, st);
+  if (p.groups == 1 && held_rows_pay(p.M, p.N, p.K, p.epilogue == VMI_HY_E_STORE)) return launch_held_rows(p, st);
   switch (p.epilogue) {
     case VMI_HY_E_STORE: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_STORE>(p, st);
     case VMI_HY_E_FLOAT: return linear_shape<b16, VMI_HY_X_ROWS, VMI_HY_E_FLOAT>(p, st);
@@ -676,7 +676,7 @@ using namespace vmi_hybrid;
 extern "C" {
 
 int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype) {
-  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups == 1 && (norm_first(M, N, K) || (K <= 2048 && held_rows_pay(M, N, K)));
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && groups == 1 && (norm_first(M, N, K) || (K < 4096 && held_rows_pay(M, N, K, false)));
 }
 
 int32_t vmi_hy_linear_resident(int32_t M, int32_t N, int32_t K, int32_t dtype) {
@@ -692,7 +692,11 @@ int32_t vmi_hy_linear_plain(int32_t M, int32_t N, int32_t K, int32_t groups, int
 }
 
 int32_t vmi_hy_linear_held(int32_t M, int32_t N, int32_t K, int32_t dtype) {
-  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && K <= 2048 && held_rows_pay(M, N, K);
+  return K < 4096 && vmi_hy_linear_holds(M, N, K, 0, dtype);
+}
+
+int32_t vmi_hy_linear_holds(int32_t M, int32_t N, int32_t K, int32_t stored, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && held_rows_pay(M, N, K, stored != 0);
 }
 
 int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {

@@ -57,7 +57,7 @@ __device__ __forceinline__ void epilogue(const vmi_hy_linear_args& p, const f32x
 // Products of few rows in bfloat16 (hybrid_rows.hip).  Each is built for what its rule names
 int norm_slabs(int M, int N, int K);   // behind a norm, one group: 0 where it is not
 int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st);
-bool held_rows_pay(int M, int N, int K);   // of the element type behind a norm of their own, one group
+bool held_rows_pay(int M, int N, int K, bool stored);   // of the element type behind a norm of their own, one group; stored: as they are
 int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool plain_rows_fit(int M, int N, int K, int groups);   // of the element type
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st);

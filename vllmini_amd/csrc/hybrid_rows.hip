@@ -410,14 +410,17 @@ int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   }
 }
 
-// Whether rows that have been normed by a launch of their own go to held_rows_kernel: its waves' parts of K are whole chunks (a condition around a chunk's products costs the
-// ring).  Up to 2048 columns they are normed for it: 9 and more of them, which resident_kernel's workgroups would norm all each, over too many columns for norm_rows_kernel; at 4096 where
-// norm_first says so.  Both launches, us, the forerunners / now: K 2048, N 12288 8 / 12 / 32 / 40 rows 14.9 / 17.8 / 21.6 / 41.8 -> 14.9 / 15.0 / 17.3 / 17.2,
-// N 20480 19.0 / 22.3 / 26.8 / 47.8 -> 19.9 / 19.9 / 22.2 / 23.5, N 50272 39.4 / 42.3 / 50.4 / 95.1 -> 41.3 / 41.6 / 45.7 / 48.8; K 4096, N 8192 12 / 32 / 40 rows 20.4 / 24.0 / 30.1 -> 18.5 / 23.0 /
-// 22.9, N 24576 32 / 40 rows 50.1 / 48.4 -> 45.4 / 46.9, N 50272 100.5 / 112.4 -> 86.3 / 90.6; K 1024, N 50272 40 rows 49.5 -> 22.1
-bool held_rows_pay(int M, int N, int K) {
+// Whether rows that have been normed by a launch of their own go to held_rows_kernel: 9 to 64 of them, whose waves' parts of K are whole chunks, K % 1024 == 0 (a condition around a chunk's products
+// costs the ring), up to the 4096 that registers hold.  Below 4096 columns they are normed for it, where norm_rows_kernel does not take them and resident_kernel, whose workgroups would norm all each, is behind or takes no more than 32; at 4096 norm_first
+// norms them anyway, and a workgroup walks a slab of that length alone: with few slabs the waves of plain_rows_kernel (or linear_kernel, with what it stores gated) end sooner.  Both launches, us, weights not in the
+// Infinity Cache, the other kernels / this one: K 2048, N 12288 8 / 12 / 32 / 40 rows 14.9 / 17.8 / 21.6 / 41.8 -> 14.9 / 15.0 / 17.3 / 17.2, N 20480 19.0 / 22.3 / 26.8 / 47.8 -> 19.9 / 19.9 / 22.2 / 23.5, N 50272 39.4 / 42.3 / 50.4 /
+// 95.1 -> 41.3 / 41.6 / 45.7 / 48.8; K 1024, N 50272 40 rows 49.5 -> 22.1; K 3072, 33 / 47 / 64 rows, N 512 26.2 / 27.2 / 31.7 -> 12.6 / 12.6 / 13.7,
+// N 4096 27.9 / 28.8 / 33.4 -> 14.3 / 14.7 / 16.4, N 24576 57.5 / 57.0 / 58.2 -> 35.2 / 37.2 / 39.0 (9 to 32 rows stay with resident_kernel, which is behind too from N 2048 on: N 6144 16 rows 17.7, 14.3 here); K 4096, N 4096 12.3 / 13.9 / 17.9 -> 13.3 / 17.6 / 16.5 (40 rows gated 27.5 -> 16.9), N 6144 17.9 / 21.1 / 27.7 -> 16.2 / 20.2 / 20.0, N 8192 19.0 / 22.5 /
+// 28.7 -> 19.1 / 23.1 / 23.0, N 12288 26.6 / 30.4 / 32.8 -> 23.7 / 28.4 / 28.8, N 50272 85.3 / 97.0 / 108 -> 85.5 / 83.2 / 87.7; with weights in that cache N 6144 32 rows 15.5 -> 18.5.
+bool held_rows_pay(int M, int N, int K, bool stored) {
   if (M < 9 || M > 64 || norm_slabs(M, N, K) > 0) return false;
-  return K == 2048 || K == 4096 || (K == 1024 && M > 32);
+  if (K == 4096) return M <= 16 ? N >= 6144 : M <= 32 ? N >= 12288 : N >= 4096 || !stored;
+  return K == 2048 || ((K == 1024 || K == 3072) && M > 32);
 }
 
 template <int NCH, int MT, int NB, int EPI>
@@ -435,6 +438,8 @@ static int held_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
     case 1024 * 4 + 2: return held_rows_of<1, 2, 6, EPI>(p, st);
     case 2048 * 4 + 1: return held_rows_of<2, 1, 6, EPI>(p, st);
     case 2048 * 4 + 2: return held_rows_of<2, 2, 6, EPI>(p, st);
+    case 3072 * 4 + 1: return held_rows_of<3, 1, 6, EPI>(p, st);
+    case 3072 * 4 + 2: return held_rows_of<3, 2, 6, EPI>(p, st);
     case 4096 * 4 + 1: return held_rows_of<4, 1, 4, EPI>(p, st);
     case 4096 * 4 + 2: return held_rows_of<4, 2, 4, EPI>(p, st);
     default: return fail(VMI_HY_E_ARG, "vmi_hy_linear", "not built");   // (held_rows_pay names no other)

@@ -74,6 +74,7 @@ SIGNATURES = {
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_slabs": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_plain": (_i32, [_i32, _i32, _i32, _i32, _i32]),
+    "vmi_hy_linear_holds": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_held": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp]),
     "vmi_hy_embed": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
