@@ -594,6 +594,15 @@ def test_latent_attention_over_pages(dtype, H, rank, rot, page):
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("H,rank,rot", [(3, 32, 32), (2, 160, 32), (1, 512, 64), (2, 608, 32)])
+def test_parts_of_any_number_add_up(dtype, H, rank, rot):
+    """combine_kernel: groups of 4, 8 and 16 parts, whole and not, up to all 128; parts without keys (of the short contexts most); one wave of columns and several."""
+    for sp in (2, 4, 5, 8, 9, 16, 17, 64, 65, 128):
+        got, want = _attend(dtype, H, rank, rot, [1, 1, 2], [40, 700, 8300], 64, 1, sp, seed=sp)
+        close(got, want, dtype, tol32=2e-5, tol16=1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 def test_latent_attention_sees_the_far_key_and_never_the_next_one(dtype):
     """One score stands out: at the very first token, at page borders, at the query's own position — and one past it, where it must
     not be seen."""

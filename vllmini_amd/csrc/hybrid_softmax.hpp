@@ -56,31 +56,37 @@ struct Combine {
   int T, heads, width, splits;
 };
 
-// out[row] = sum over splits of 2^(m_s - m) part_s / sum of 2^(m_s - m) l_s (times sigmoid(gate)); one workgroup per (token, head).  Bound by its trips through
-// memory: the parts beside their weights and two columns a thread took 1 to 1.7 us off the latent attention of 12 to 32 tokens (4 splits, 8 heads, 13.7 -> 12.0).
-template <typename T>
-__global__ __launch_bounds__(256) void combine_kernel(const Combine p) {
+// out[row] = sum over splits of 2^(m_s - m) part_s / sum of 2^(m_s - m) l_s (times sigmoid(gate)); one workgroup per (token, head), two columns a thread.  Bound by its
+// trips through memory: AHEAD parts are asked for beside their weights, and the following ones AHEAD at a time, all of them without a condition (parts past the last are
+// that one again, with a weight of zero): a condition a part waits for each of them.
+template <typename T, int AHEAD>
+__global__ __launch_bounds__(512) void combine_kernel(const Combine p) {
   need(p.partial), need(p.out), need(p.gate), need(p.tok_seq), need(p.ldo), need(p.ldg), need(p.T), need(p.heads), need(p.width), need(p.splits);
-  const int64_t row = blockIdx.x, n = (int64_t)p.T * p.heads;
+  static_assert(128 % AHEAD == 0, "the weights end with a group of parts");
   const int t = (int)(blockIdx.x / (unsigned)p.heads), h = (int)(blockIdx.x - (unsigned)t * p.heads), seq = p.tok_seq[t];
   const int ld = p.width + 2;
-  __shared__ float wt[128];   // weight of every part (at most 128 of them)
-  const float* first = p.partial + row * ld;
-  // (two columns a thread; the values of the first AHEAD parts are asked for beside the weights)
-  constexpr int AHEAD = 16;
-  auto pair = [&](int i, int k) { return *reinterpret_cast<const f32x2*>(first + i * n * ld + k); };
-  f32x2 ahead[AHEAD];
+  __shared__ float wt[128];   // weight of every part (at most 128 of them), zeros behind them
+  const char* first = reinterpret_cast<const char*>(p.partial + (int64_t)blockIdx.x * ld);
+  const int64_t each = (int64_t)p.T * p.heads * ld * 4;
+  auto ask = [&](f32x2(&v)[AHEAD], int i0, int k) {
+    const uint32_t at = (uint32_t)min(k, p.width - 2) * 4;
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i)
-    if (i < p.splits) ahead[i] = pair(i, min(2 * (int)threadIdx.x, p.width - 2));   // (scalar)
-  if (seq < 0) return;
+    for (int i = 0; i < AHEAD; ++i) v[i] = *reinterpret_cast<const f32x2*>(first + min(i0 + i, p.splits - 1) * each + at);
+  };
+  auto ask_weights = [&](int i) { return *reinterpret_cast<const f32x2*>(first + min((int)(threadIdx.x & 63) + i, p.splits - 1) * each + (uint32_t)p.width * 4); };
+  f32x2 v[AHEAD], ml[2];
+  ml[0] = ask_weights(0);
+  ask(v, 0, 2 * (int)threadIdx.x);
+  if (p.splits > 64) ml[1] = ask_weights(64);
+  T gate = (T)0.f;
+  if (p.gate) gate = static_cast<const T*>(p.gate)[t * p.ldg + h];
   if (threadIdx.x < 64) {
     float m[2], l[2], top = -1e30f, sum = 0.f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int i = threadIdx.x + 64 * j;
-      m[j] = i < p.splits ? first[i * n * ld + p.width] : -1e30f;
-      l[j] = i < p.splits ? first[i * n * ld + p.width + 1] : 0.f;
+      const bool there = (int)threadIdx.x + 64 * j < p.splits;
+      m[j] = there ? ml[j][0] : -1e30f;
+      l[j] = there ? ml[j][1] : 0.f;
       top = fmaxf(top, m[j]);
     }
 #pragma unroll
@@ -91,23 +97,23 @@ __global__ __launch_bounds__(256) void combine_kernel(const Combine p) {
       sum += m[j] * l[j];
     }
     sum = wave_sum(sum);
-    const float g = p.gate ? sigmoid((float)static_cast<const T*>(p.gate)[t * p.ldg + h]) : 1.f;
+    const float g = p.gate ? sigmoid((float)gate) : 1.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) wt[threadIdx.x + 64 * j] = m[j] / sum * g;
+    for (int j = 0; j < 2; ++j) wt[threadIdx.x + 64 * j] = threadIdx.x + 64 * j < p.splits ? m[j] / sum * g : 0.f;
   }
   __syncthreads();
+  if (seq < 0) return;   // (here: in front, the parts would wait for it)
   for (int k = 2 * threadIdx.x; k < p.width; k += 2 * blockDim.x) {
     f32x2 a = f32x2{0.f, 0.f};
-    auto add = [&](int i, const f32x2& v) {
-      const float w = wt[i];
+    for (int i0 = 0; i0 < p.splits; i0 += AHEAD) {
+      if (i0 > 0 || k >= 2 * (int)blockDim.x) ask(v, i0, k);
 #pragma unroll
-      for (int e = 0; e < 2; ++e) a[e] = fmaf(w, w != 0.f ? v[e] : 0.f, a[e]);   // (a part without keys holds whatever was there)
-    };
+      for (int i = 0; i < AHEAD; ++i) {
+        const float w = wt[i0 + i];
 #pragma unroll
-    for (int i = 0; i < AHEAD; ++i)
-      if (i < p.splits) add(i, k < 2 * (int)blockDim.x ? ahead[i] : pair(i, k));
-#pragma unroll 8
-    for (int i = AHEAD; i < p.splits; ++i) add(i, pair(i, k));
+        for (int e = 0; e < 2; ++e) a[e] = fmaf(w, w != 0.f ? v[i][e] : 0.f, a[e]);   // (a part without keys holds whatever was there)
+      }
+    }
     T* out = static_cast<T*>(p.out) + (int64_t)t * p.ldo + (int64_t)h * p.width + k;
     typename Elem<T>::v2 o;
     o[0] = (T)a[0], o[1] = (T)a[1];
@@ -118,7 +124,9 @@ __global__ __launch_bounds__(256) void combine_kernel(const Combine p) {
 
 template <typename T>
 inline void launch_combine(const Combine& p, hipStream_t st) {
-  hipLaunchKernelGGL(combine_kernel<T>, dim3((int64_t)p.T * p.heads), dim3(p.width > 256 ? 256 : p.width > 128 ? 128 : 64), 0, st, p);
+  const int threads = p.width >= 1024 ? 512 : (p.width + 127) / 128 * 64;
+  auto* fn = p.splits <= 4 ? combine_kernel<T, 4> : p.splits <= 8 ? combine_kernel<T, 8> : combine_kernel<T, 16>;
+  hipLaunchKernelGGL(fn, dim3((int64_t)p.T * p.heads), dim3(threads), 0, st, p);
 }
 
 }  // namespace vmi_hybrid
