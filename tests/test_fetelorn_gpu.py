@@ -358,6 +358,15 @@ def test_attention_over_pages_and_chunks(dtype, H, G, dim, vdim, chunk, page):
                 close(got, want, dtype, tol32=3e-5, tol16=1.5e-2)
 
 
+@pytest.mark.parametrize("dim", range(32, 257, 32))
+def test_heads_whose_values_are_as_wide_as_their_keys(dim):
+    """gqa_rows_kernel without a condition a product: every width it is built for, beside one column tile more of values, which takes the form with them."""
+    for counts, ctx in (([1], [0]), ([70, 1, 2], [0, 99, 62])):
+        for vdim in (dim, dim + 32 if dim < 256 else 224):
+            got, want = _attend(torch.bfloat16, 6, 2, dim, vdim, 100, counts, ctx, 64, 4, 2)
+            close(got, want, torch.bfloat16, tol16=1.5e-2)
+
+
 @pytest.mark.parametrize("parts", [(), ("bias",), ("sink",), ("gate",)])
 def test_attention_without_some_of_its_parts(parts):
     for rt, dtype in ((1, torch.float32), (4, torch.bfloat16)):

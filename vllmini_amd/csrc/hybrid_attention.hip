@@ -264,7 +264,7 @@ inline size_t gqa_rows_lds(int dim, int vdim, int rep, bool bias) {
 
 // NK k-steps (of 32) of a query row, NV value tiles (of 16 columns): at most that many, or (EXACT) just that many, so that no condition stands between a read of LDS and the product
 // behind it and they overlap: a branch a product, a bias and a mask each waited for its own read (heads of 128, 8 over 2 of them, 1 x 1500 rows 84 -> 53 us, 6 x up to 1500 91 -> 63;
-// 16 over 4, 32 x up to 200 33 -> 25)
+// 16 over 4, 32 x up to 200 33 -> 25; 16 over 4, 4 x up to 1000 rows, heads of 32 / 64 / 96 / 192 / 256 57 / 62 / 66 / 166 / 183 -> 32 / 34 / 51 / 92 / 126)
 template <int NK, int NV, int U, bool EXACT>
 __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vmi_hy_attention_args p, const vmi_hy_step s) {
   constexpr int R = 64, KT = 64, LDP = KT + 8;
@@ -489,7 +489,18 @@ static int run_gqa(const vmi_hy_attention_args& p, const vmi_hy_step& s, hipStre
     return fail(VMI_HY_E_ARG, "vmi_hy_attention", "row_tiles is what vmi_hy_attention_row_tiles returns");
   if constexpr (sizeof(T) == 2) {
     if (p.row_tiles == 4) {
-      if (p.dim == 128 && p.vdim == 128) return launch_gqa_rows<4, 8, 8, true>(p, s, st);
+      if (p.dim == p.vdim) {
+        switch (p.dim) {
+          case 32: return launch_gqa_rows<1, 2, 2, true>(p, s, st);
+          case 64: return launch_gqa_rows<2, 4, 4, true>(p, s, st);
+          case 96: return launch_gqa_rows<3, 6, 6, true>(p, s, st);
+          case 128: return launch_gqa_rows<4, 8, 8, true>(p, s, st);
+          case 160: return launch_gqa_rows<5, 10, 10, true>(p, s, st);
+          case 192: return launch_gqa_rows<6, 12, 12, true>(p, s, st);
+          case 224: return launch_gqa_rows<7, 14, 14, true>(p, s, st);
+          case 256: return launch_gqa_rows<8, 16, 16, true>(p, s, st);
+        }
+      }
       if (p.dim <= 128 && p.vdim <= 128) return launch_gqa_rows<4, 8, 8>(p, s, st);
       return launch_gqa_rows<8, 16, 16>(p, s, st);
     }
