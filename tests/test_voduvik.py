@@ -6,6 +6,7 @@ import ctypes
 import os
 import re
 import subprocess
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -349,6 +350,22 @@ def test_large_products_stay_with_the_library_unless_their_rows_stay_in_lds():
     for M, N, K in ((17, 8192, 4096), (18, 24560, 4096), (19, 24576, 4096)):
         assert hybrid_layers.dense(M, of(N, K), True), (M, N, K)
     assert not hybrid_layers.dense(16, of(8192, 4096), True) and h.linear_normed_first(17, of(8192, 4096)) and not h.linear_normed_first(17, of(8192, 4096, 2))
+
+
+@pytest.mark.parametrize("heads,row,tokens,keys,tiles", [(16, 576, 256, 4000, 1), (32, 576, 1, 1000, 1), (32, 576, 16, 400, 1), (32, 576, 16, 4000, 2), (32, 576, 64, 1000, 2), (32, 576, 128, 400, 1), (32, 576, 256, 400, 2),
+                                                         (128, 576, 1, 4000, 1), (128, 576, 16, 400, 1), (128, 576, 16, 4000, 4), (128, 576, 256, 1000, 4), (32, 544, 16, 1000, 2), (64, 288, 16, 1000, 1)])
+def test_single_tokens_take_a_row_tile_each_while_they_or_their_keys_are_few(heads, row, tokens, keys, tiles):
+    """The tiles of a step of single tokens, of latent attention; grouped queries of as many rows take as many as fit, however many tokens there are."""
+    from vllmini_amd.hybrid_decoder import HybridDecoder
+    from vllmini_amd.hybrid_layers import QueryTiling
+
+    d, at = object.__new__(HybridDecoder), np.arange(tokens)
+    d.model = SimpleNamespace(dtype=torch.bfloat16)
+    d._kinds = [QueryTiling("latent", heads, 1, row, sizes=(row,)), QueryTiling("grouped", heads, 1, 128, sizes=(128, 128))]
+    a = {"entry": at, "pos": at, "slots": [at], "ctx": np.full(tokens, keys - 1), "state_slot": at, "parity": at * 0, "tables": np.zeros((1, tokens, 1), dtype=np.int32)}
+    _, _, _, plans = d._layout(a, np.ones(tokens, dtype=np.int64), at, tokens, tokens, 1, keys)
+    assert [p[0] for p in plans] == [tiles, 4 if heads > 16 else 1]
+    assert plans[0][2] == tokens * -(-heads // (16 * tiles))
 
 
 def test_products_behind_a_norm_of_few_rows_and_columns_share_one_kernel_whatever_their_width():

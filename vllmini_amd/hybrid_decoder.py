@@ -120,9 +120,8 @@ class HybridDecoder:
         put("rows", max(len(rows), 1), rows, 0)
         plans = []
         for kind in self._kinds:
-            rep, longest = kind.rep, int(counts.max()) * kind.rep
-            # single tokens: a row tile each, however many heads a token has (one token of 32 heads, 1000 keys in 8 splits 16.1 -> 13.1 us; 256 tokens level)
-            rt = kind.row_tiles(4 if longest > 32 else 2 if longest > 16 else 1, self.model.dtype) if counts.max() > 1 else 1
+            rep, longest = kind.rep, int(counts.max())
+            rt = 1 if longest == 1 and kind.one_row_tile(B, max_keys) else kind.row_tiles(longest, self.model.dtype)
             per = -(-(counts * rep) // (16 * rt))
             ent = np.repeat(np.arange(b), per)
             first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * 16 * rt

@@ -74,8 +74,23 @@ class QueryTiling(NamedTuple):
     chunk: int = 0
     sizes: Tuple[int, ...] = ()
 
-    def row_tiles(self, want: int, dtype: torch.dtype) -> int:
+    def row_tiles(self, longest: int, dtype: torch.dtype) -> int:
+        """Of 16 rows each, a workgroup's: as many as an entry's `longest` portion fills."""
+        want = 4 if longest * self.rep > 32 else 2 if longest * self.rep > 16 else 1
         return (ops.latent_row_tiles if self.kernel == "latent" else ops.attention_row_tiles)(*self.sizes, want, dtype)
+
+    def one_row_tile(self, entries: int, keys: int) -> bool:
+        """Whether single tokens of more than 16 rows take a row tile a workgroup, in the latent kernel: more of them fill the chip sooner, but each walks all keys, so that is for few
+        of them or few keys.  Rows of 576, as many tiles as a token fills / one each, us: 32 heads, 1 token behind 1000 keys 12.3 / 11.9, 16 behind 400 17.5 / 16.3, behind 4000 31.7 / 38.0, 64 behind 1000 30.4 / 38.2, 128 behind
+        400 31.6 / 26.4 (two splits / none), 256 behind 400 34.7 / 44.8; 128 heads, 1 behind 400 and 4000 16.4 / 11.6 and 25.3 / 21.6, 16 behind 400 and 4000 27.1 / 24.9 and 57.9 / 97.3, 64 behind 400 44.1 / 44.5, 256 behind 1000 180 / 326.  One tile's
+        query stays in registers where a row is 576 long; of others a long one waits in LDS: 32 heads of 544, 16 tokens behind 1000 keys 20.7 / 26.8.  (Over 864 steps of 24 to 128 heads, 1 to 256 tokens and 60 to 4000 keys 0.2 per cent behind the better
+        side in the mean.)  Grouped queries take as many as fit: 128 heads of 128 over one, 256 tokens behind 1000 keys 50.7 / 152."""
+        if self.kernel != "latent" or self.rep <= 16:
+            return False
+        tiles, row = entries * -(-self.rep // 16), self.sizes[0]
+        small = self.rep <= 32 or (row > 320 and row != 576)
+        most = 1 << 14 if small else 1 << 17 if keys <= 512 else 1 << 16
+        return tiles <= 512 and ((128 < tiles <= 256 and keys <= 512) or tiles * keys <= most)
 
 
 class AttentionPlan(NamedTuple):
