@@ -226,15 +226,17 @@ def test_many_states_take_two_column_tiles_a_workgroup(kind):
 
 
 @pytest.mark.parametrize("kind", ["retention", "delta"])
+@pytest.mark.parametrize("longest", [70, 260])
 @pytest.mark.parametrize("B", [4, 5, 6, 9, 17, 33])
-def test_walks_of_every_length_start_in_turn(kind, B):
-    """state_scan_kernel's order of entries, 64 workgroups each (4: as they come, 5 and 6: two workgroups a compute unit, 9: three, 17: two column tiles each, 33: as they come
-    again): lengths all over, some of them equal, each sequence as it comes out alone."""
+def test_walks_of_every_length_start_in_turn(kind, B, longest):
+    """state_scan_kernel's order of entries, 64 workgroups each (up to 260 rows 4: as they come, 5 and 6: two workgroups a compute unit, 9: three, 17: two column tiles each, 33: as they come
+    again; up to 70: all as they come): lengths all over, some of them equal, each sequence as it comes out alone."""
     k, want = (retention_case(8, 128, 128, 64, (0.9, 0.5, 0.99, 1.0, 0.8, 0.97, 0.3, 0.999), torch.float32, B) if kind == "retention" else
                delta_case(8, 4, 128, 128, 4, torch.float32, B))
     rng = np.random.default_rng(B)
-    lens = [int(n) for n in rng.integers(1, 70, B)]
+    lens = [int(n) for n in rng.integers(1, longest, B)]
     lens[-1] = lens[0]
+    assert (sum(lens) > 64 * B) == (longest > 70)
     seqs = [k.inputs(n, 100 + i) for i, n in enumerate(lens)]
     got = k.run([torch.cat([s[1][j] for s in seqs]) for j in range(3)], layout(lens, [0] * B, [[0]] * B, 64, pos_slots=False)).split(lens)
     states = k.held[0].clone()
@@ -243,6 +245,20 @@ def test_walks_of_every_length_start_in_turn(kind, B):
         alone = k.run(seqs[i][1], layout([n], [0], [[0]], 64, slots=[i], pos_slots=False))
         close(got[i], alone, torch.float32, tol32=1e-5)
         close(states[i], k.held[0][i], torch.float32, tol32=1e-5)
+
+
+@pytest.mark.parametrize("dim,vdim,heads,B", [(96, 192, 8, 3), (96, 64, 4, 40), (512, 64, 2, 3), (256, 128, 8, 5)])
+@pytest.mark.parametrize("kind", ["retention", "delta"])
+def test_states_of_every_shape_walk_alike_in_company_and_alone(kind, dim, vdim, heads, B):
+    """Three and more row tiles a wave, in turn and as they come, one column tile a workgroup and two."""
+    k, want = (retention_case(heads, dim, vdim, dim // 2, (0.9, 0.97, 0.5, 0.99) * (heads // 4) or (0.9, 0.97), torch.float32, B) if kind == "retention" else
+               delta_case(heads, heads // 2, dim, vdim, 4, torch.float32, B))
+    lens = [1 + (53 * i) % 230 for i in range(1, B + 1)]
+    seqs = [k.inputs(n, 200 + i) for i, n in enumerate(lens)]
+    got = k.run([torch.cat([s[1][j] for s in seqs]) for j in range(3)], layout(lens, [0] * B, [[0]] * B, 64, pos_slots=False)).split(lens)
+    close(got[0], want(seqs[0][0]), torch.float32, tol32=5e-5)
+    for i in range(0, B, 7):
+        close(got[i], k.run(seqs[i][1], layout([lens[i]], [0], [[0]], 64, slots=[i], pos_slots=False)), torch.float32, tol32=1e-5)
 
 
 def test_delta_rule_survives_decays_that_leave_nothing():

@@ -411,21 +411,22 @@ __device__ __forceinline__ int entry_in_turn(const vmi_hy_step& s, int first, in
   return __builtin_ctzll(__ballot(lane < s.B && rank == at));
 }
 
-// NT: 16-row tiles of the state, dealt over RS waves.  One workgroup: CT tiles of 16 value columns of one (entry, head); CU of them a compute unit
-template <int KIND, int NT, int RS, int CT, int CU>
+// NT: 16-row tiles of the state, dealt over RS waves.  One workgroup: CT tiles of 16 value columns of one (entry, head); CU of them a compute unit.  FAR: chunks are
+// asked for further ahead; TURN: entries may come in turn
+template <int KIND, int NT, int RS, int CT, int CU, bool FAR, bool TURN>
 __global__ __launch_bounds__(64 * RS, CU) void state_scan_kernel(const vmi_hy_state_args p, const vmi_hy_step s, const int first) {
   constexpr bool DELTA = KIND == VMI_HY_DELTA;
   // A chunk's operands are some 1.8 us away (every chunk is a page of its own), a chunk takes 0.6: what bounds a walk is how many of them are asked for ahead, and with operands
   // behind one address register each and accumulators among the other registers as many fit as it takes.  Heads of 128, retention / delta rule, us, before (three ahead, a
-  // compute unit's workgroups as they come) -> now: 1 x 1500 rows, 8 heads 70 / 93 -> 59 / 80, 6 x up to 1500 88 / 118 -> 61 / 84, 9 x 400 34 / 51 -> 30 / 37; 16 heads, 3 x 1000
-  // 55 / 72 -> 42 / 57, 12 x 400 59 / 80 -> 46 / 64, 5 x 700 51 / 71 -> 52 / 70.
-  constexpr int NW = NT / RS, DEPTH = NW > 2 || CT > 1 ? 2 : CU > 2 ? DELTA ? 2 : 3 : DELTA ? 3 : 4;   // tiles of a wave, chunks of operands in registers
+  // compute unit's workgroups as they come) -> FAR and in turn: 1 x 1500 rows, 8 heads 70 / 93 -> 59 / 80, 6 x up to 1500 88 / 118 -> 61 / 84, 9 x 400 34 / 51 -> 30 / 37; 16 heads, 3 x 1000
+  // 55 / 72 -> 42 / 57, 12 x 400 59 / 80 -> 46 / 64, 5 x 700 51 / 71 -> 52 / 70.  (launch_scan: which walks they are not for)
+  constexpr int NW = NT / RS, DEPTH = NW > 2 || CT > 1 ? 2 : !FAR ? 3 : CU > 2 ? DELTA ? 2 : 3 : DELTA ? 3 : 4;   // tiles of a wave, chunks of operands in registers
   constexpr int EW = 4 / RS;                             // elements of a lane's four that a wave finishes of o
   __shared__ f32x4 reda[DELTA ? 2 : 1][CT][DELTA ? RS : 1][64];
   __shared__ float redo[2][CT][RS][4][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
   // (heads vary fastest: the column blocks of one head, which read the same operands, then share an XCD's L2)
-  const int h = blockIdx.x % p.heads, col0 = (int)(blockIdx.x / p.heads) * 16 * CT, e = first ? entry_in_turn(s, first, lane) : (int)blockIdx.y;
+  const int h = blockIdx.x % p.heads, col0 = (int)(blockIdx.x / p.heads) * 16 * CT, e = TURN && first ? entry_in_turn(s, first, lane) : (int)blockIdx.y;
   const Portion r = portion(s, e);
   if (r.len <= 0) return;
   constexpr int dim = NT * 16;
@@ -447,25 +448,28 @@ __global__ __launch_bounds__(64 * RS, CU) void state_scan_kernel(const vmi_hy_st
     f32x4 w[DELTA ? NW : 1], q[NW], k[NW], d[NW], u[CT];
     float b[EW];
   };
-  const uint32_t row = (uint32_t)(r16 * dim + 4 * kc) * 4, col = (uint32_t)(r16 * CH + 4 * kc) * 4;
-  // a lane's bytes behind a place that all lanes share: one address register an operand, none to keep for later chunks
-  auto four = [](const float* at, uint32_t lane_at) { return *reinterpret_cast<const f32x4*>(reinterpret_cast<const char*>(at) + lane_at); };
+  const int row = r16 * dim + 4 * kc + (FAR ? 0 : 16 * ct0), col = r16 * CH + 4 * kc;
+  const uint32_t row_bytes = (uint32_t)row * 4, col_bytes = (uint32_t)col * 4;
+  // FAR: a lane's elements behind a place that all lanes share: one address register an operand, none to keep for later chunks
+  auto word = [](const float* shared, uint32_t lane_at) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(shared) + lane_at); };
+  auto four = [&](const float* shared, uint32_t lane_at) { return *reinterpret_cast<const f32x4*>(word(shared, lane_at)); };
   // (no branch stands in a chunk: every path issues the same loads and stores, so the waits count them exactly)
   auto load = [&](Operands& o, int c) {
     const float* at = base + min(c, nch - 1) * step;   // (past the end: the last one again)
 #pragma unroll
     for (int t = 0; t < NW; ++t) {
-      if constexpr (DELTA) o.w[t] = four(at + sc.w + 16 * (ct0 + t), row);
-      o.q[t] = four(at + sc.q + 16 * (ct0 + t), row);
+      if constexpr (DELTA) o.w[t] = FAR ? four(at + sc.w + 16 * (ct0 + t), row_bytes) : *reinterpret_cast<const f32x4*>(at + sc.w + row + 16 * t);
+      o.q[t] = FAR ? four(at + sc.q + 16 * (ct0 + t), row_bytes) : *reinterpret_cast<const f32x4*>(at + sc.q + row + 16 * t);
     }
 #pragma unroll
-    for (int j = 0; j < CT; ++j) o.u[j] = four(at + sc.u + (col0 + 16 * j) * CH, col);
+    for (int j = 0; j < CT; ++j)
+      o.u[j] = FAR ? four(at + sc.u + (col0 + 16 * j) * CH, col_bytes) : *reinterpret_cast<const f32x4*>(at + sc.u + (col0 + 16 * j) * CH + col);
 #pragma unroll
-    for (int i = 0; i < EW; ++i) o.b[i] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(at + sc.b + wave + RS * i) + col);
+    for (int i = 0; i < EW; ++i) o.b[i] = FAR ? *word(at + sc.b + wave + RS * i, col_bytes) : at[sc.b + col + wave + RS * i];
 #pragma unroll
     for (int t = 0; t < NW; ++t) {
-      o.d[t] = four(at + sc.d + 16 * (ct0 + t), (uint32_t)kc * 16);
-      o.k[t] = four(at + sc.k + 16 * (ct0 + t) * CH, col);
+      o.d[t] = FAR ? four(at + sc.d + 16 * (ct0 + t), (uint32_t)kc * 16) : *reinterpret_cast<const f32x4*>(at + sc.d + 16 * (ct0 + t) + 4 * kc);
+      o.k[t] = FAR ? four(at + sc.k + 16 * (ct0 + t) * CH, col_bytes) : *reinterpret_cast<const f32x4*>(at + sc.k + 16 * (ct0 + t) * CH + col);
     }
   };
   f32x4 part[CT];                           // this wave's part of the last chunk's o
@@ -478,7 +482,7 @@ __global__ __launch_bounds__(64 * RS, CU) void state_scan_kernel(const vmi_hy_st
       for (int x = 0; x < 4; ++x) redo[c & 1][j][wave][x][lane] = part[j][x];
   };
   auto finish = [&](int c) {                // the elements wave, wave + RS, .. of every lane's four of chunk c - 1
-    float* out = base + max(c - 1, 0) * step + sc.o + col0;
+    float* out = base + max(c - 1, 0) * step + sc.o + (FAR ? col0 : 4 * kc * p.vdim + col0 + r16);
     const uint32_t lane_at = (uint32_t)(4 * kc * p.vdim + r16) * 4;
 #pragma unroll
     for (int j = 0; j < CT; ++j)
@@ -488,7 +492,8 @@ __global__ __launch_bounds__(64 * RS, CU) void state_scan_kernel(const vmi_hy_st
         float y = redo[c & 1][j][0][x][lane];
 #pragma unroll
         for (int w = 1; w < RS; ++w) y += redo[c & 1][j][w][x][lane];
-        *reinterpret_cast<float*>(reinterpret_cast<char*>(out + x * p.vdim + 16 * j) + lane_at) = y;       // (c = 0: zeros, which the next chunk overwrites)
+        if constexpr (FAR) *reinterpret_cast<float*>(reinterpret_cast<char*>(out + x * p.vdim + 16 * j) + lane_at) = y;       // (c = 0: zeros, which the next chunk overwrites)
+        else out[x * p.vdim + 16 * j] = y;
       }
   };
   auto chunk = [&](Operands& o, int c) {
@@ -760,16 +765,25 @@ static void launch_scan(const vmi_hy_state_args& p, const vmi_hy_step& s, hipStr
   constexpr int RS = NT % 4 == 0 ? 4 : 2;
   const int tiles = p.vdim / 16;   // (even: vdim is a multiple of 32)
   const int each = p.heads * tiles;
-  // states enough for the chip: a workgroup takes two column tiles, which halves what is read per column.  More than two workgroups a compute unit: registers for three
-  constexpr int TWO = NT <= 8 ? 2 : 1, CT = NT <= 16 ? 2 : 1, THREE = NT <= 8 ? 3 : 1;
-  auto go = [&](auto* fn, int wgs) {
-    // (what entry_in_turn asks for; past 32 entries, which are short then, finding one's place takes longer than it gives: 60 entries of up to 100 rows 38 -> 43 us)
-    const int first = s.B <= 32 && (int64_t)wgs * s.B > 256 ? (wgs > 256 ? 1 : 256 / wgs) : 0;
-    hipLaunchKernelGGL(fn, dim3(wgs, s.B), dim3(64 * RS), 0, st, p, s, first);
-  };
-  if (NT <= 16 && (int64_t)each * s.B >= 1024) go(state_scan_kernel<KIND, NT, RS, CT, TWO>, each / 2);
-  else if (NT <= 8 && (int64_t)each * s.B > 512) go(state_scan_kernel<KIND, NT, RS, 1, THREE>, each);
-  else go(state_scan_kernel<KIND, NT, RS, 1, TWO>, each);
+  constexpr int TWO = NT <= 8 ? 2 : 1, CT = NT <= 16 ? 2 : 1, THREE = NT <= 8 ? 3 : 1, PAIR = CT > 1 ? TWO : 1;
+  // Walks of more than four chunks on average.  Shorter ones have no use for a chunk further ahead, nor for an order of entries, which every workgroup reads all lengths for first, a trip to memory: 8 heads of 128, 30 x up to 40 rows
+  // 32.1 us as they come, 36.4 in turn, 4 x 64 15.3, 16.1; of 512, 30 x up to 40 344, 390; longer ones: 12 x up to 300, 96 x 192 76, 67.  Past 32 entries, which are short, it never gives (60 of up to 100 rows 38, 43), with states
+  // of 512 rows neither (12 x up to 100 223, 236).
+  const bool far = s.T > 64 * s.B;
+  // Tiles of more than two a wave, or two column tiles: their operands leave registers for two chunks however they are addressed, and one register an operand is behind then (of 512, 4 x up to 1000 760 -> 800 us; 96 x 192, 1 x 3000
+  // 164 -> 182) but where it lets a second workgroup on a compute unit (96 x 192, 4 x up to 1000 100 -> 96)
+  constexpr bool FAR = NT / RS <= 2;
+  auto turn = [&](int wgs) { return NT <= 16 && far && s.B <= 32 && (int64_t)wgs * s.B > 256 ? (wgs > 256 ? 1 : 256 / wgs) : 0; };   // (what entry_in_turn asks for)
+  auto go = [&](auto* fn, int wgs) { hipLaunchKernelGGL(fn, dim3(wgs, s.B), dim3(64 * RS), 0, st, p, s, turn(wgs)); };
+  if constexpr (NT <= 16) {
+    // states enough for the chip: a workgroup takes two column tiles, which halves what is read per column.  More than two workgroups a compute unit: registers for three
+    if ((int64_t)each * s.B >= 1024)
+      return turn(each / 2) ? go(state_scan_kernel<KIND, NT, RS, CT, PAIR, false, true>, each / 2) : go(state_scan_kernel<KIND, NT, RS, CT, PAIR, false, false>, each / 2);
+    if (NT <= 8 && (int64_t)each * s.B > 512) return go(state_scan_kernel<KIND, NT, RS, 1, THREE, true, true>, each);
+    if (NT <= 8 && (FAR ? far : (int64_t)each * s.B > 256)) return go(state_scan_kernel<KIND, NT, RS, 1, TWO, true, true>, each);
+    if (turn(each)) return go(state_scan_kernel<KIND, NT, RS, 1, 1, false, true>, each);
+  }
+  go(state_scan_kernel<KIND, NT, RS, 1, 1, false, false>, each);
 }
 
 template <typename T, int KIND>
