@@ -143,6 +143,8 @@ VMI_LAYER_API int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream);
 VMI_LAYER_API int vmi_gpt2_sample_top_k_f16(const void* logits, int64_t ld, int32_t num_rows, int32_t vocab, int32_t top_k,
                                             float temperature, const float* uniform, int64_t* out, int32_t device, void* stream);
 
+/* How many slabs of 16 columns a workgroup takes where vmi_gpt2_linear_f16 runs this shape in its kernels for few rows; 0: in tiles */
+VMI_LAYER_API int32_t vmi_gpt2_linear_slabs(int32_t M, int32_t N, int32_t K, int32_t has_ln, int32_t epilogue);
 /* The tile vmi_gpt2_linear_f16 cuts this shape into ("bm32_nw4_ks1_r2_ln_gelu"), for records; NULL if refused.  (Steps of few rows
  * may run undivided, an eighth of K a wave, instead.) */
 VMI_LAYER_API const char* vmi_gpt2_linear_kernel_name(int32_t M, int32_t N, int32_t K, int32_t has_ln, int32_t epilogue);

@@ -72,6 +72,20 @@ def test_layer_picks_for_the_gpt2_small_decode_step():
     assert gl.kernel_name(64, 768, 768, False, gl.EPI_BIAS_RESIDUAL) == "bm16_nw4_ks1_r2_residual"
 
 
+def test_linears_of_few_rows_past_1536_columns_count_the_rounds_of_a_die():
+    """Where a workgroup has a compute unit to itself, the kernels for few rows end when the die with the most column blocks does: three of its rounds are behind one of tiles, two are level, and as the widths go these lie at
+    other numbers of rows."""
+    from vllmini_amd import gpt2_layer as gl
+
+    def slabs(M, N, K, ln=False, epi=None):
+        return gl.load().vmi_gpt2_linear_slabs(M, N, K, int(ln), gl.EPI_BIAS_RESIDUAL if epi is None else epi)
+
+    for N, K, few, tiles in ((640, 2560, 336, 352), (576, 2304, 336, 352), (896, 3584, 144, 160), (704, 2816, 320, 352)):
+        assert slabs(few, N, K) and not slabs(tiles, N, K), (N, K)
+    assert slabs(448, 640, 2560) == 2 and slabs(384, 768, 3072) == 2 and slabs(128, 1152, 4608) == 1 and not slabs(160, 1152, 4608)
+    assert slabs(512, 3072, 768, True, gl.EPI_BIAS_GELU) == 6 and slabs(512, 768, 768) == 2 and not slabs(1040, 768, 768) and not slabs(8, 768, 768, True)
+
+
 # ---- GPU ---------------------------------------------------------------------------------------------------------------
 
 def _chain(x, w, b, ln=None, gelu=False, residual=None):
@@ -659,7 +673,7 @@ def test_add_norm_is_the_add_and_the_layer_norm(M, E):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (16, 48, 224), (17, 144, 288), (3, 2304, 768), (47, 768, 1056), (33, 320, 2048), (112, 768, 3072), (5, 80, 4096)])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (16, 48, 224), (17, 144, 288), (3, 2304, 768), (47, 768, 1056), (33, 320, 2048), (112, 768, 3072), (5, 80, 4096), (1, 832, 3328), (17, 48, 3616), (64, 96, 4128), (352, 640, 2560)])
 def test_few_rows_split_k_over_the_waves(M, N, K):
     """rows_kernel where its waves have unequal parts of K, or none; row tiles that are not full; more of them than XCDs: against the module chain,
     for every epilogue it has, both weight layouts to the same bits."""

@@ -760,15 +760,21 @@ static int rows_most(int K, bool ln) {   // (the weights of NS slabs wait in reg
   return per <= 4 ? 6 : per <= 6 ? 4 : 3;
 }
 
-// Whether a linear layer goes to the kernels of gpt2_rows.hpp.  Behind a norm, while its workgroups are on the chip at once: up to 768 columns four a
-// compute unit, beyond one.  linear_kernel / these, us: K 768, N 3072 192 rows (384 workgroups) 9.3 / 7.4, 320 (640) 9.6 / 9.8, 384 (768) 14.1 / 9.9, 512 (1024) 14.3 / 12.1;
-// K 512, N 2048 512 rows (704) 8.1 / 7.7; K 1024, N 4096 64 rows (172) 7.9 / 5.7, 96 (258) 9.0 / 10.6, 160 (430) 14.3 / 10.8, 256 (688) 16.1 / 15.4; K 1152, N 3456
+// Whether a linear layer goes to the kernels of gpt2_rows.hpp: as many workgroups as they were measured ahead of, or level with, linear_kernel.  Behind a norm up to 1024 where rows are at most 768 columns (two rounds: six slabs at K 768 take 74 KB of LDS,
+// two workgroups a compute unit), beyond one round.  linear_kernel / these, us: K 768, N 3072 192 rows (384 workgroups) 10.1 / 7.9, 288 (576) 10.3 / 10.1, 352 (704) 15.4 / 10.1, 512 (1024) 15.5 / 12.2, N 2304 352 (528) 9.3 / 9.5,
+// 448 (672) 9.4 / 9.5, 512 (768) 13.7 / 9.7; K 512, N 2048 256 (352) 8.2 / 6.4, 512 (704) 9.4 / 8.3; K 1024, N 4096 64 rows (172) 7.9 / 5.7, 96 (258) 9.0 / 10.6, 160 (430) 14.3 / 10.8, 256 (688) 16.1 / 15.4; K 1152, N 3456
 // 64 rows (216) 9.3 / 6.3, 128 (432) 9.8 / 10.8.  Without one their reading of x is what grows: K 768, N 768 512 rows (768) 4.8 / 4.7, K 1152, N 1152 256 rows
-// (576) 6.6 / 6.3, 320 (720) 6.7 / 7.5, K 4096, N 1024 128 rows (512) 11.4 / 10.1, 160 (640) 11.4 / 13.5, K 4608, N 1152 128 rows (576) 14.2 / 13.7
+// (576) 6.6 / 6.3, 320 (720) 6.7 / 7.5.  Past 1536 columns sixteen waves and their rows have a compute unit to themselves, and column blocks go to the dies in turn, so what counts is how many rounds the fullest of them makes, against linear_kernel's of 16 rows
+// x 64 columns: K 2560, N 640 320 rows (2 and 1) 8.9 / 8.7, 352 (3 and 1) 8.8 / 11.4, 448 (3 and 2) 15.3 / 11.9; K 3072, N 768 160 (1 and 1) 8.8 / 5.6, 320 (2 and 1) 9.0 / 9.1, 384 (3 and 2) 15.4 / 12.2; K 3584, N 896 128 (2 and 1) 11.9 / 9.6,
+// 160 (3 and 1) 12.0 / 12.9; K 4608, N 1152 128 (3 and 1) 14.3 / 13.6.
 static bool rows_pick(int M, int N, int K, bool ln, int epi) {
   if ((K & 31) || (N & 15) || K > (ln ? MAX_K_LN : MAX_K) || ln == (epi == VMI_LAYER_EPI_BIAS_RESIDUAL)) return false;
   const int ns = rows_slabs(M, N, rows_most(K, ln));
-  return (int64_t)(((N >> 4) + ns - 1) / ns) * ((M + 15) >> 4) <= (K <= 768 ? 1024 : ln ? 256 : 576);
+  const int nb = ((N >> 4) + ns - 1) / ns, rb = (M + 15) >> 4;
+  if ((int64_t)nb * rb > (K <= 768 ? 1024 : ln ? 256 : 576)) return false;
+  if (ln || K <= 1536) return true;
+  const int rounds = ((nb + 7) / 8 * rb + 31) / 32, theirs = (int)(((int64_t)((N + 63) >> 6) * rb + 255) / 256);
+  return rounds <= (K > 4096 ? 3 : 2) * theirs;
 }
 
 static int launch_rows(void (*fn)(LinearParams), const LinearParams& p, int ns, int threads, size_t lds, hipStream_t stream) {
@@ -834,7 +840,9 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
   if (nks <= 32) return launch_plain_rows<8, 4>(p, ns, stream);
   if (nks <= 48) return launch_plain_rows<8, 6>(p, ns, stream);
   if (nks <= 64) return launch_plain_rows<16, 4>(p, ns, stream);
-  return nks <= 96 ? launch_plain_rows<16, 6>(p, ns, stream) : launch_plain_rows<16, 9>(p, ns, stream);
+  if (nks <= 96) return launch_plain_rows<16, 6>(p, ns, stream);
+  if (nks <= 112) return launch_plain_rows<16, 7>(p, ns, stream);
+  return nks <= 128 ? launch_plain_rows<16, 8>(p, ns, stream) : launch_plain_rows<16, 9>(p, ns, stream);
 }
 
 // Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
@@ -1206,6 +1214,11 @@ int vmi_gpt2_sample_top_k_f16(const void* logits, int64_t ld, int32_t num_rows, 
   hipLaunchKernelGGL(sample_top_k_kernel, dim3(num_rows), dim3(SK_T), 0, static_cast<hipStream_t>(stream),
                      static_cast<const h16*>(logits), ld, vocab, top_k, 1.f / temperature, uniform, out);
   return after_launch("vmi_gpt2_sample_top_k_f16", prev, device);
+}
+
+int32_t vmi_gpt2_linear_slabs(int32_t M, int32_t N, int32_t K, int32_t has_ln, int32_t epilogue) {
+  using namespace vmi_layer;
+  return M > 0 && N > 0 && K > 0 && rows_pick(M, N, K, has_ln != 0, epilogue) ? rows_slabs(M, N, rows_most(K, has_ln != 0)) : 0;
 }
 
 const char* vmi_gpt2_linear_kernel_name(int32_t M, int32_t N, int32_t K, int32_t has_ln, int32_t epilogue) {

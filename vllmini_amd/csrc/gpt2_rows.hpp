@@ -134,7 +134,8 @@ __global__ __launch_bounds__(64 * NORM_RW, 2) void norm_rows_kernel(const Linear
 constexpr int rows_stride(int J, int NS) { return 16 * (64 * J + 16) > NS * 1024 ? 16 * (64 * J + 16) : NS * 1024; }   // bytes of LDS a wave
 
 // Rows that are multiplied as they are, with the residual behind: a wave brings its own part of K of the 16 rows through its own part of the LDS, no other
-// wave waits for it.  RW waves, at most J k-steps each: six a wave where that is possible (K 768 over 4 / 8 waves: 2.36 / 2.51 us; K 3072 over 8 / 16: 4.38 / 4.08)
+// wave waits for it.  RW waves, at most J k-steps each: six a wave where that is possible (K 768 over 4 / 8 waves: 2.36 / 2.51 us; K 3072 over 8 / 16: 4.38 / 4.08),
+// as few more as there are past 3072 columns (a step that a wave does not have is read all the same: K 4096, N 1024 1 / 16 rows nine a wave 5.3 / 6.0, eight 4.7 / 5.1)
 template <int RW, int J, int NS>
 __global__ __launch_bounds__(64 * RW, RW / 4) void rows_kernel(const LinearParams p) {
   constexpr int EPI = VMI_LAYER_EPI_BIAS_RESIDUAL, LDB = 64 * J + 16, STRIDE = rows_stride(J, NS);

@@ -41,6 +41,7 @@ SIGNATURES = {
     "vmi_gpt2_linear_qkv_cache_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i64, _i32, _i32, _i32,
                                                      _vp, _vp, _vp, _i32, _i32, _i32, _i64, _i64, _i32, _vp]),
     "vmi_gpt2_embed_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp]),
+    "vmi_gpt2_linear_slabs": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_gpt2_head_fits": (_i32, [_i32, _i32]),
     "vmi_gpt2_head_f16": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_step_inputs": (ctypes.c_int, [_vp, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp]),
