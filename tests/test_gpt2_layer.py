@@ -7,6 +7,7 @@ import ctypes
 import os
 import re
 import subprocess
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -70,6 +71,30 @@ def test_layer_picks_for_the_gpt2_small_decode_step():
     assert gl.kernel_name(1, 768, 3072, False, gl.EPI_BIAS_RESIDUAL) == "bm16_nw1_ks4_r2_residual"
     assert gl.kernel_name(64, 768, 3072, False, gl.EPI_BIAS_RESIDUAL) == "bm16_nw1_ks4_r2_residual"
     assert gl.kernel_name(64, 768, 768, False, gl.EPI_BIAS_RESIDUAL) == "bm16_nw4_ks1_r2_residual"
+
+
+@pytest.mark.parametrize("L,E,mb", [(4, 768, 134), (12, 768, 247), (12, 256, 45)])
+def test_pages_go_past_the_caches_where_they_and_the_weights_leave_them(L, E, mb):
+    """The rule of a decode step, in the sizes of GPT-2 and smaller: by the tokens whose pages no longer fit beside the weights."""
+    from vllmini_amd import ops
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder
+
+    def holds(numel):
+        return SimpleNamespace(numel=lambda: numel, element_size=lambda: 2)
+
+    d, names = object.__new__(GPT2PagedDecoder), ops.variant_names()
+    d.dims, d._cold = GPT2Dims(n_embd=E, n_head=E // 64, n_layer=L), None
+    d.pool = SimpleNamespace(key_cache=torch.empty(0, dtype=torch.float16), kv_cache_dtype="auto", block_size=16)
+    d._step_weights = GPT2PagedDecoder.step_weights({"lm_head.weight": holds(50257 * E), "transformer.wte.weight": holds(50257 * E), "transformer.wpe.weight": holds(1024 * E), **{f"transformer.h.{i}": holds(12 * E * E) for i in range(L)}})
+    assert abs(d._step_weights / 1e6 - mb) < 2
+    fits = ((248 << 20) - d._step_weights) // (4 * L * E)
+    assert not d._pages_leave_the_cache(fits) and d._pages_leave_the_cache(fits + 1)
+    at = {n: i + 1 for i, n in enumerate(names)}
+    for name, B, to in (("d64_h1_w16_u2_nt0", 1, "d64_h1_w16_u1_nt1"), ("d64_h1_w8_u1_nt0", 32, "d64_h1_w8_u1_nt1"), ("d64_h1_w4_u2_nt0", 1, "d64_h1_w4_u2_nt0"), ("d64_h1_w4_u2_nt0", 48, "d64_h1_w4_u1_nt1"),
+                        ("d64_h1_w8_u1_nt1", 64, "d64_h1_w8_u1_nt1")):
+        assert names[d._past_caches(at[name], B) - 1] == to
+    d._step_weights = (256 << 20) + 1
+    assert names[d._past_caches(at["d64_h1_w4_u2_nt0"], 48) - 1] == "d64_h1_w4_u2_nt0" and names[d._past_caches(at["d64_h1_w16_u2_nt0"], 48) - 1] == "d64_h1_w16_u1_nt1"
 
 
 def test_linears_of_few_rows_past_1536_columns_count_the_rounds_of_a_die():
@@ -813,10 +838,10 @@ def test_logits_of_few_rows(M, V, E, norm):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,ctx", [(32, 100), (16, 200), (1, 800), (4, 300), (12, 250)])
-def test_steps_read_their_pages_past_the_caches_with_the_same_results(B, ctx, monkeypatch):
-    """_past_caches: where a step takes another variant than the operators would, it is the same split of a head over waves without a temporal load, and logits and caches
-    agree (to the bit where a wave takes its blocks one by one in both)."""
+@pytest.mark.parametrize("B,ctx,switch", [(32, 100, False), (16, 200, True), (1, 800, True), (4, 300, False), (12, 250, True)])
+def test_steps_read_their_pages_past_the_caches_with_the_same_results(B, ctx, switch, monkeypatch):
+    """_past_caches, in a cache that holds the weights and nothing else: where a step takes another variant than the operators would (where two blocks a wave and few heads are not left to them, nor pages non-temporal as they
+    are), it is the same split of a head over waves without a temporal load, and logits and caches agree (to the bit where a wave takes its blocks one by one in both)."""
     from vllmini_amd import ops
     from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
     from vllmini_amd.kv_pool import PagedKVPool
@@ -829,10 +854,12 @@ def test_steps_read_their_pages_past_the_caches_with_the_same_results(B, ctx, mo
             monkeypatch.setattr(GPT2PagedDecoder, "_past_caches", lambda self, variant, B: variant)
         pool = PagedKVPool(B * dims.n_layer * 64 + 8, dims.n_head, dims.head_size, 16, 64, dims.n_layer, device=dev, max_seqs=B, multi_block_prefill=True)
         d = GPT2PagedDecoder(dims, sd, pool)
+        monkeypatch.setattr(d, "INFINITY_CACHE", d._step_weights)
         d.prefill_batch(list(range(B)), [[(7 * s + j) % 200 for j in range(ctx - s % 5)] for s in range(B)])
         out = [d.decode(list(range(B)), torch.full((B,), 3 + i, device=dev), use_graph=True).clone() for i in range(3)]
         got.append((names[d._static["variant"] - 1], out, pool.key_cache.clone(), pool.value_cache.clone()))
     (a, x, ka, va), (b, y, kb, vb) = got
+    assert (a != b) == switch, (a, b)
     if a != b:
         assert a.endswith("_u1_nt1") and b.endswith("_nt0") and a.rsplit("_u", 1)[0] == b.rsplit("_u", 1)[0]
     if a.replace("nt1", "nt0") == b.replace("nt1", "nt0"):

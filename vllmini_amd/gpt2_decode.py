@@ -98,6 +98,7 @@ class GPT2PagedDecoder:
     # 1024 1500 1666 / 1879, 2600 2165 / 2109; 1152 1500 1806 / 1864, 2100 2267 / 2125
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
     NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
+    INFINITY_CACHE = 248 << 20        # bytes of the last cache in front of the memory, 256 MiB, that a step's activations and logits leave
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
@@ -152,6 +153,7 @@ class GPT2PagedDecoder:
             self.scatter_in_c_attn = False
         self._packed: Dict[str, gpt2_layer.PackedWeight] = {}
         self._cold: Optional[Dict[int, tuple]] = None
+        self._step_weights = self.step_weights(state_dict)
         self._prompt_tensors = None                # what gpt2_layer.prompts reads
         self.NATIVE_PROMPT_MAX_TOKENS = min(self.NATIVE_PROMPT_MAX_TOKENS, self.NATIVE_PROMPT_MAX_WORK // (E * E))
         if self.native_layers:
@@ -541,11 +543,15 @@ class GPT2PagedDecoder:
         m = self.pad_batch_to
         return B if not m or B % m == 0 else (B // m + 1) * m
 
+    @staticmethod
+    def step_weights(state_dict) -> int:
+        """Bytes of weights that every step reads (of the embeddings a row a token)."""
+        return sum(t.numel() * t.element_size() for k, t in state_dict.items() if k not in ("transformer.wte.weight", "transformer.wpe.weight"))
+
     def _past_caches(self, variant: int, B: int) -> int:
         """The same split of heads over waves with non-temporal loads of the pages.  The operators' choice for a small batch is temporal, measured on pages that the call before has read;
-        a step reads other pages in every layer, and all layers' weights go through the caches in between.  12 layers of 12 heads of 64, a step in us: 32 sequences of up to 128
-        tokens 339 -> 327, 20 of 200 326 -> 315, 13 of 300 325 -> 317, 8 of 600 334 -> 316, 4 of 900 348 -> 333, 1 of 900 332 -> 323.  Two blocks a wave at once stay where fewer than
-        16 waves a head and few heads leave them to: 4 of 400 312 against 316, 1 of 300 289 against 291."""
+        a step reads other pages in every layer, and all layers' weights go through the caches in between.  Two blocks a wave at once stay where fewer than
+        16 waves a head and few heads leave them to, or the weights alone leave the cache: 12 layers of 12 heads of 64, 4 of 400 312 against 316, 1 of 300 289 against 291; of 16 heads, 8 of 200 347, 358."""
         if self._cold is None:
             names = ops.variant_names() if self.pool.kv_cache_dtype == "auto" and self.dims.head_size == 64 and self.pool.block_size == 16 else []
             at, self._cold = {n: i + 1 for i, n in enumerate(names)}, {}
@@ -554,7 +560,15 @@ class GPT2PagedDecoder:
                 if m and f"{m[1]}_u1_nt1" in at:
                     self._cold[at[n]] = at[f"{m[1]}_u1_nt1"], int(m[2]) < 16 and int(m[3]) > 1
         to, many_only = self._cold.get(variant, (variant, False))
-        return variant if many_only and B * self.dims.n_head < 128 else to
+        return variant if many_only and (B * self.dims.n_head < 128 or self._step_weights > self.INFINITY_CACHE) else to
+
+    def _pages_leave_the_cache(self, tokens: int) -> bool:
+        """Whether a step's weights and the pages of so many tokens in all are more than the last cache holds: then pages that go past it leave it to the weights, and while they are not, all of it is still there
+        from the step before.  Steps in us, temporal / past the caches: 4 layers of width 768 (134 MB of weights), 16 sequences of 300 (59 MB) 114 / 118, of 900 (176 MB) 142 / 133; 6 layers, 12 of 300 (162 + 66 MB)
+        151 / 160, of 500 (+ 110) 168 / 165, of 900 195 / 179; 12 layers (247 MB), 1 of 900 321 / 307, 8 of 900 363 / 322, 32 of 300 365 / 331; 12 layers of 256 (45 MB), 32 of 500 (195 MB) 251 / 254, of 900 302 / 281.  Over 250 steps of 2 to 24 layers, widths
+        of 256 to 1024, they meet at 244 to 256 MiB in all (12 layers of 768, 1 of 500, 265 MB: 299 / 285); weights of more are level with either, up to 3 per cent ahead past the caches."""
+        page = 2 * self.dims.n_layer * self.dims.n_embd * self.pool.key_cache.element_size()
+        return self._step_weights + tokens * page > self.INFINITY_CACHE
 
     def stage_step(self, seq_ids: Sequence[int], input_ids) -> dict:
         """Host bookkeeping for one step + ONE upload of all of it into the static device buffers.  With pad_batch_to the
@@ -607,7 +621,8 @@ class GPT2PagedDecoder:
                                          self.pool.block_size, mean_seq_len=max(int(lens.sum()) // Bp, 1),
                                          bf16=self.pool.key_cache.dtype == torch.bfloat16,
                                          fp8={"auto": False, "fp8_e5m2": "e5m2"}.get(self.pool.kv_cache_dtype, True))
-        st["variant"] = self._past_caches(st["variant"], Bp)
+        if self._pages_leave_the_cache(int(lens.sum())):
+            st["variant"] = self._past_caches(st["variant"], Bp)
         # few sequences x long contexts: with the wrapper's workspace the library spreads a head over several workgroups
         # (ops.pick_variant(workspace=True) names a split kernel, "_x<waves>", exactly where the default entry would run one)
         # (only when the launch WILL carry a workspace: the wrapper's switch is on and one exists for this stream — none is
