@@ -838,6 +838,17 @@ def test_logits_of_few_rows(M, V, E, norm):
 
 
 @pytest.mark.gpu
+def test_logits_of_a_vocabulary_of_more_than_sixteen_million():
+    from vllmini_amd import gpt2_layer as gl
+
+    dev, V = torch.device("cuda:0"), (1 << 24) + 37
+    g = torch.Generator(device=dev).manual_seed(7)
+    x, w = torch.randn((2, 32), generator=g, device=dev).half(), torch.randn((V, 32), generator=g, device=dev, dtype=torch.float16)
+    got, want = gl.head(x, gl.pack_head(w)), (w.float() @ x.float().T).T
+    assert got.shape == (2, V) and bool(((got.float() - want).abs() <= 2.0 ** -10 * want.abs() + 1e-4).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,ctx,switch", [(32, 100, False), (16, 200, True), (1, 800, True), (4, 300, False), (12, 250, True)])
 def test_steps_read_their_pages_past_the_caches_with_the_same_results(B, ctx, switch, monkeypatch):
     """_past_caches, in a cache that holds the weights and nothing else: where a step takes another variant than the operators would (where two blocks a wave and few heads are not left to them, nor pages non-temporal as they

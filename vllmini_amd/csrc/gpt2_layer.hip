@@ -1129,7 +1129,7 @@ int vmi_gpt2_head_f16(const void* x, int64_t ldx, const int32_t* rows, const voi
                       int32_t N, int32_t K, int32_t device, void* stream) {
   using namespace vmi_layer;
   static const char* who = "vmi_gpt2_head_f16";
-  if (!x || !w || !logits || (gamma == nullptr) != (beta == nullptr) || N <= 0 || N > (1 << 24) || ld < N || ldx < K) {
+  if (!x || !w || !logits || (gamma == nullptr) != (beta == nullptr) || N <= 0 || N > INT32_MAX - 16 * HEAD_RW * 256 || ld < N || ldx < K) {
     set_err(who, ": null pointer or a size out of range");
     return VMI_LAYER_E_ARG;
   }
