@@ -838,6 +838,27 @@ def test_logits_of_few_rows(M, V, E, norm):
 
 
 @pytest.mark.gpu
+def test_the_vocabulary_is_kept_once_more_unless_the_caller_declines():
+    from vllmini_amd.gpt2_decode import GPT2Dims, GPT2PagedDecoder, random_state_dict
+    from vllmini_amd.kv_pool import PagedKVPool
+
+    dims, dev = GPT2Dims(vocab_size=203, n_layer=2), torch.device("cuda:0")
+    sd, got = random_state_dict(dims, dev), []
+    for native_head in (None, True, False):
+        pool = PagedKVPool(64, dims.n_head, dims.head_size, 16, 8, dims.n_layer, device=dev, max_seqs=2)
+        d = GPT2PagedDecoder(dims, sd, pool, native_head=native_head)
+        assert (d._head is None) == (native_head is False)
+        d.prefill_batch([0, 1], [list(range(20)), list(range(5, 12))])
+        got.append(d.decode([0, 1], [1, 2]))
+    assert torch.equal(got[0], got[1])
+    _close(got[2], got[0], "torch's lm_head beside gpt2_layer.head")
+    odd = {**sd, "lm_head.weight": sd["lm_head.weight"].t().contiguous().t()}
+    with pytest.raises(RuntimeError, match="native_head"):
+        GPT2PagedDecoder(dims, odd, pool, native_head=True)
+    assert GPT2PagedDecoder(dims, odd, pool)._head is None
+
+
+@pytest.mark.gpu
 def test_logits_of_a_vocabulary_of_more_than_sixteen_million():
     from vllmini_amd import gpt2_layer as gl
 

@@ -104,7 +104,7 @@ class GPT2PagedDecoder:
     def __init__(self, dims: GPT2Dims, state_dict: Dict[str, torch.Tensor], pool: PagedKVPool,
                  reference_off_by_one: bool = False, fused_append: bool = False, native_layers: Optional[bool] = None,
                  scatter_in_c_attn: Optional[bool] = None, deferred_scatter: bool = False, pad_batch_to: int = 0,
-                 paged_prefill: Optional[bool] = None):
+                 paged_prefill: Optional[bool] = None, native_head: Optional[bool] = None):
         assert pool.num_layers == dims.n_layer and pool.num_heads == dims.n_head
         assert pool.head_size == dims.head_size
         self.dims, self.sd, self.pool = dims, state_dict, pool
@@ -185,12 +185,14 @@ class GPT2PagedDecoder:
             self.prompt_kernel = self._find_prompt_tensors()
         if self.prompt_kernel:
             gpt2_layer.load()
-        # the vocabulary's weight once more for steps and prompts of few rows (gpt2_layer.head): 77 MB for GPT-2 small
+        # the vocabulary's weight once more for steps and prompts of few rows (gpt2_layer.head): 77 MB for GPT-2 small.  native_head: None = where it applies; True insists (RuntimeError otherwise); False = lm_head as a
+        # torch module whatever the rows, and no second copy
         head, ends = state_dict.get("lm_head.weight"), [state_dict.get(f"transformer.ln_f.{k}") for k in ("weight", "bias")]
-        self._head = None
-        if self.native_layers and gpt2_layer.head_fits(1, E) and head is not None and head.dim() == 2 and head.shape[1] == E and gpt2_layer.takes_weights([head]) \
-                and all(t is not None and t.shape == (E,) for t in ends) and gpt2_layer.takes_weights(ends):
-            self._head = gpt2_layer.pack_head(head)
+        can_head = self.native_layers and gpt2_layer.head_fits(1, E) and head is not None and head.dim() == 2 and head.shape[1] == E and gpt2_layer.takes_weights([head]) \
+            and all(t is not None and t.shape == (E,) for t in ends) and gpt2_layer.takes_weights(ends)
+        if native_head and not can_head:
+            raise RuntimeError("native_head needs native_layers and an lm_head and a final norm of the hidden size, half, contiguous and 16-byte aligned")
+        self._head = gpt2_layer.pack_head(head) if can_head and native_head is not False else None
         self.pad_batch_to = int(pad_batch_to)      # decode steps are laid out for the next multiple of this many rows (0: as they come)
 
     def _find_prompt_tensors(self) -> bool:
