@@ -97,6 +97,52 @@ def test_pages_go_past_the_caches_where_they_and_the_weights_leave_them(L, E, mb
     assert names[d._past_caches(at["d64_h1_w4_u2_nt0"], 48) - 1] == "d64_h1_w4_u2_nt0" and names[d._past_caches(at["d64_h1_w16_u2_nt0"], 48) - 1] == "d64_h1_w16_u1_nt1"
 
 
+def test_pinned_memory_that_cannot_be_waited_for_is_not_given_back(monkeypatch):
+    """PinnedBuffer: a launch may still read what nobody holds any more.  Waited for where that is possible; while a stream of the thread is captured, and where waiting fails, the memory is kept until its event says that the launch has run."""
+    from vllmini_amd import staging
+
+    class Event:
+        waited, done, fails = 0, False, False
+
+        def record(self):
+            pass
+
+        def synchronize(self):
+            if self.fails:
+                raise RuntimeError("not now")
+            Event.waited += 1
+
+        def query(self):
+            return self.done
+
+    empty = torch.empty
+    monkeypatch.setattr(staging.torch, "empty", lambda n, dtype, pin_memory: empty(n, dtype=dtype))
+    monkeypatch.setattr(staging.torch.cuda, "Event", Event)
+    capturing = [False]
+    monkeypatch.setattr(staging.torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+
+    def dropped(fails, captured):
+        b = staging.PinnedBuffer(64)
+        b.read()
+        event, at = b._read, b.tensor.data_ptr()
+        event.fails, capturing[0] = fails, captured
+        del b
+        capturing[0] = False
+        return event, at
+
+    assert not staging._kept
+    dropped(False, False)
+    assert Event.waited == 1 and not staging._kept
+    for fails, captured in ((True, False), (False, True)):
+        event, at = dropped(fails, captured)
+        assert Event.waited == 1 and [t.data_ptr() for _, t in staging._kept] == [at]
+        staging.PinnedBuffer(64)
+        assert len(staging._kept) == 1
+        event.done = True
+        staging.PinnedBuffer(64)
+        assert not staging._kept
+
+
 def test_linears_of_few_rows_past_1536_columns_count_the_rounds_of_a_die():
     """Where a workgroup has a compute unit to itself, the kernels for few rows end when the die with the most column blocks does: three of its rounds are behind one of tiles, two are level, and as the widths go these lie at
     other numbers of rows."""

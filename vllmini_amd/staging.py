@@ -1,9 +1,11 @@
 """Pinned host memory that launches read by its address."""
 from __future__ import annotations
 
-from typing import Optional
+from typing import List, Optional, Tuple
 
 import torch
+
+_kept: List[Tuple[torch.cuda.Event, torch.Tensor]] = []      # what could not be waited for when its buffer went, until it has been read
 
 
 class PinnedBuffer:
@@ -11,8 +13,10 @@ class PinnedBuffer:
     kernel's reads it does not, so this does: the memory is written again (wait()) or given back only once the last launch told of (read()) has run."""
 
     def __init__(self, nbytes: int):
-        self.tensor = torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
         self._read: Optional[torch.cuda.Event] = None
+        if _kept and not torch.cuda.is_current_stream_capturing():
+            _kept[:] = [k for k in _kept if not k[0].query()]
+        self.tensor = torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
 
     def wait(self) -> None:
         if self._read is not None:
@@ -24,7 +28,12 @@ class PinnedBuffer:
         self._read.record()
 
     def __del__(self):
+        if self._read is None:
+            return
         try:
-            self.wait()
-        except Exception:       # (the interpreter or the runtime is on its way out: so is the memory)
+            if not torch.cuda.is_current_stream_capturing():      # (a wait would end the capture)
+                return self.wait()
+        except Exception:       # (the runtime is on its way out, or does not let us wait here)
             pass
+        if _kept is not None:      # (a module being torn down)
+            _kept.append((self._read, self.tensor))
