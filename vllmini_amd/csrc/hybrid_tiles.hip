@@ -31,7 +31,7 @@ __global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const vmi_hy_linear_
 
 // Whether tiles of our own with the unit behind them end sooner than the library's product and the unit in a launch of its own.  Ours are ahead where the
 // library's tiles of 256 x 256 leave part of the chip idle or rows are few, behind where they fill it (they take 0.74 of ours' time then).  Both sides as their tiles share
-// the chip out; the library's fitted to 80 products of 48 to 8192 rows, K 1024 to 4096, N 6144 to 24576, 9 per cent off in the mean, and the rule's picks within 0.6 per
+// the chip out; the library's (hipBLASLt as PyTorch 2.10.0+rocm7.0 loads it: another version may move the line, never the result) fitted to 80 products of 48 to 8192 rows, K 1024 to 4096, N 6144 to 24576, 9 per cent off in the mean, and the rule's picks within 0.6 per
 // cent of the better side in the mean, 11 at most.  Library + unit / ours in us, cold weights: K 1024, N 6144 all gated 300 rows 14.9 / 10.4, 1500 36.6 / 24.3, 4500
 // 65.8 / 65.3; K 2048, N 20480, 12288 of them gated, 100 rows 34.4 / 27.0, 1500 113 / 129, 3200 301 / 257, 8192 530 / 639; K 4096, N 24576 48 49.4 / 44.6, 2400 387 / 440.
 static bool tiles_pay(int M, int N, int K, int n_split) {
