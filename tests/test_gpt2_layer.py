@@ -810,6 +810,31 @@ def test_products_of_many_rows_in_tiles(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(771, 7584, 256), (1090, 5408, 192), (1650, 7184, 128), (1732, 6800, 64), (1369, 4368, 256), (1360, 4368, 320), (2122, 2832, 384), (1361, 4400, 192),
+                                   (521, 7184, 128), (515, 7184, 64), (2101, 2064, 3072), (257, 7344, 128), (259, 7312, 64), (260, 6544, 512), (259, 6608, 832), (258, 6544, 448),
+                                   (197, 7184, 128), (193, 7056, 64), (194, 6992, 256), (130, 6560, 832), (195, 7136, 640), (193, 7152, 192), (70, 5456, 256), (68, 5456, 576),
+                                   (66, 5520, 640), (66, 5968, 192), (65, 5648, 128), (66, 5520, 64), (1, 160, 512), (7, 32, 64), (11, 16, 128), (1, 32, 192), (40, 272, 320)])
+def test_every_tile_with_every_number_of_chunks_left(M, N, K):
+    """tiles_kernel, each tile of its list with each remainder of K's chunks of 64 by the two or four that it has in flight, rows and columns left over.  A chunk that is none adds
+    nothing where the last one holds an infinity: the row that has one is infinite or, where the weight is zero, NaN, and no other row is touched."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    x, w, b, res = (rnd(M, K) * 1.5 + 0.3).half(), (rnd(N, K) * 0.6 / K ** 0.5).half(), (rnd(N) * 0.1).half(), rnd(M, N).half()
+    packed = gl.pack_weight(w)
+    for bias, kw in ((None, {}), (b, {"gelu": True}), (b, {"residual": res})):
+        _close(gl.linear_tiles(x, packed, bias, **kw), _chain(x, w, bias, None, kw.get("gelu", False), kw.get("residual")), (M, N, K, sorted(kw)))
+    before, row = gl.linear_tiles(x, packed), M // 2
+    x[row, -1] = float("inf")
+    after = gl.linear_tiles(x, packed)
+    rest = torch.arange(M, device=dev) != row
+    assert torch.equal(after[rest], before[rest])
+    assert torch.equal(after[row], torch.where(w[:, -1] == 0, float("nan"), torch.sign(w[:, -1]) * float("inf")).half()) or bool((w[:, -1] == 0).any())
+
+
+@pytest.mark.gpu
 def test_gelu_of_every_half():
     """The exact GELU of all 65536 halves, as biases under rows of zeros: within half a unit in the last place of v Phi(v) in 64 bits, up to the float's own error
     (2^-11 of a unit, some twenty roundings); infinity stays, minus infinity

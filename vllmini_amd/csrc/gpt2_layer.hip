@@ -854,10 +854,8 @@ static bool many_rows(int T, int E) { return (int64_t)T * E >= (E > 768 ? 160000
 template <int I, int EPI>
 static int launch_tiles(const LinearParams& p, hipStream_t stream) {
   constexpr vmi_tiles::Tile T = vmi_tiles::TILES[I];
-  auto* fn = tiles_kernel<T.mi, T.ni, T.ks, T.prio, EPI>;
-  constexpr size_t lds = vmi_tiles::tiles_lds<T.mi, T.ni, T.ks>();
-  static_assert(lds <= 64 * 1024, "no leave needed for the LDS");
-  hipLaunchKernelGGL(fn, dim3(vmi_tiles::tiles_grid(T, p.M, p.N)), dim3(256 * T.ks), lds, stream, p);
+  auto* fn = tiles_kernel<T.mi, T.ni, T.d, EPI>;
+  hipLaunchKernelGGL(fn, dim3(vmi_tiles::tiles_grid(T, p.M, p.N)), dim3(256), 0, stream, p);
   const hipError_t e = hipGetLastError();
   if (e == hipSuccess) return VMI_LAYER_OK;
   set_err("launch: ", hipGetErrorString(e));

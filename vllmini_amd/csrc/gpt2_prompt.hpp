@@ -320,10 +320,9 @@ __global__ __launch_bounds__(256) void add_norm_kernel(h16* __restrict__ x, cons
 
 // Linear layers of many rows, packed weights (mfma_tiles.hpp): bias, GELU or the residual add on a lane's four columns of a row, the rounding points of the few-row
 // kernels.  The bias is asked for at the start, residuals too where a tile leaves the registers, else a slab's together at the end.
-template <int MI, int NI, int KS, bool PRIO, int EPI>
-__global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const LinearParams p) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  constexpr bool EARLY = MI * NI <= 24 && !PRIO;
+template <int MI, int NI, int D, int EPI>
+__global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
+  constexpr bool EARLY = MI * NI <= 12;
   const int kc = (threadIdx.x & 63) >> 4;
   h16x4 bias[NI];
   Tail tail[NI][MI];
@@ -331,8 +330,8 @@ __global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const LinearParams p
 #pragma unroll
     for (int i = 0; i < MI; ++i) tail[n][i].template load_row<EPI>(p, m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16);
   };
-  vmi_tiles::tiles_product<vmi_tiles::Half, MI, NI, KS, PRIO>(
-      p.x, p.ldx, p.w, p.M, p.N, p.K, smem,
+  vmi_tiles::tiles_product<vmi_tiles::Half, MI, NI, D>(
+      p.x, p.ldx, p.w, p.M, p.N, p.K,
       [&](int m, int s, int SL) {
 #pragma unroll
         for (int n = 0; n < NI; ++n) bias[n] = Tail::load_bias(p, min(s + n, SL - 1) * 16 + 4 * kc);

@@ -8,12 +8,11 @@ namespace vmi_hybrid {
 // Columns below n_split as they are, the others, interleaved (gate, up), through the gated unit: what a product and an elementwise launch behind it (a
 // write and a read of 2 N bytes a row) took, and what they give: gate and up are rounded on their way into the unit, so what a prompt comes to does not hang on
 // which side tiles_pay finds ahead for the tokens that happen to share its step.
-template <int MI, int NI, int KS, bool PRIO>
-__global__ __launch_bounds__(256 * KS, 2) void tiles_kernel(const vmi_hy_linear_args p) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+template <int MI, int NI, int D>
+__global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args p) {
   const int kc = (threadIdx.x & 63) >> 4;
-  vmi_tiles::tiles_product<vmi_tiles::Bf16, MI, NI, KS, PRIO>(
-      p.x, p.ldx, p.w, p.M, p.N, p.K, smem, [](int, int, int) {},
+  vmi_tiles::tiles_product<vmi_tiles::Bf16, MI, NI, D>(
+      p.x, p.ldx, p.w, p.M, p.N, p.K, [](int, int, int) {},
       [&](const f32x4(&acc)[NI][MI], int m, int s, int SL) {
 #pragma unroll
         for (int n = 0; n < NI; ++n) {
@@ -54,9 +53,7 @@ static int launch_tiles(int pick, const vmi_hy_linear_args& p, hipStream_t st) {
   if constexpr (I < vmi_tiles::NTILES) {
     if (pick != I) return launch_tiles<I + 1>(pick, p, st);
     constexpr vmi_tiles::Tile T = vmi_tiles::TILES[I];
-    constexpr size_t lds = vmi_tiles::tiles_lds<T.mi, T.ni, T.ks>();
-    static_assert(lds <= 64 * 1024, "no leave needed for the LDS");
-    hipLaunchKernelGGL((tiles_kernel<T.mi, T.ni, T.ks, T.prio>), dim3(vmi_tiles::tiles_grid(T, p.M, p.N)), dim3(256 * T.ks), lds, st, p);
+    hipLaunchKernelGGL((tiles_kernel<T.mi, T.ni, T.d>), dim3(vmi_tiles::tiles_grid(T, p.M, p.N)), dim3(256), 0, st, p);
     return launched("vmi_hy_linear_tiles");
   }
   return fail(VMI_HY_E_SHAPE, "vmi_hy_linear_tiles", "no such tile");

@@ -1,18 +1,20 @@
 // Products of many rows, y = x W^T, in 16-bit elements: x as rows, W as the tiles the linear layers pack ([N / 16][K / 32][64 lanes][8]).
 //
 // A workgroup's tile is 16 MI rows x 64 NI columns; four waves own 16 NI columns each and ALL of its rows.  So a wave's weights are nobody else's: they go from
-// memory straight to registers as they lie, one contiguous KiB a k-step, 64 columns of K ahead.  x goes through LDS: whole 128-byte lines in, through registers, two
-// buffers and one barrier per 64 columns of K; 16-byte piece c of row r lies at c ^ (r & 7) of its line, so that eight consecutive lanes, eight rows of one piece, meet in no
-// bank.  KS = 2: two groups of four waves take half of K each (few tiles, long K), their results meet in LDS.
+// memory straight to registers as they lie, one contiguous KiB a k-step.  x goes from memory straight into LDS (buffer loads that end there), whole 128-byte lines, a place of 64
+// columns of K a chunk; 16-byte piece c of row r lies at c ^ (r & 7) of its line, so that the lanes of one read meet in no bank.  D places are in flight, D - 1 chunks ahead, with
+// one barrier a chunk, and requests, reads of x and products are dealt over the chunk's steps one by one.
 //
-// Bound by the matrix cores' and the waves' issue together, 4.1 to 5 TFLOP/s a compute unit (the card 1.24 PFLOP/s at 8192^3, the vendor's kernels 1.34; both operands in LDS, 2 x 2
-// waves: 0.82), and by how the tiles share the chip out (tiles_pick).  2770 rows, N 12288, K 2048 131 us (vendor 132 - 138), N 2048, K 6144 69 (68 - 76), N 2048, K 2048 29
-// (27); 4500 rows, N 10240, K 1024 106 (81 - 109); 3200 rows, N 20480, K 2048 240 (270 - 290); 6300 rows, N 3072, K 768 43 (40 - 49): level, and what follows
-// a product (bias, GELU, gated unit, residual) rides along.  Two row groups of four waves over one tile (256 x 256, weights from L1 a second time): 0.83 of it.  32x32x16
-// matrix instructions: 0.95.  Tiles of 192 and 256 rows in one wave's registers spill.
+// What bounds it: tiles that have a compute unit to themselves the latency of memory, so those stay four chunks deep (300 rows, N 2048, K 6144 23.8 -> 19.3 us, the vendor's
+// kernels 28.5; 700 rows, N 768, K 3072 14.6 -> 11.8; 120 rows, N 2304, K 768 6.5 -> 4.9); a full chip L2 and the matrix cores at the clock that their power leaves (2773 rows, N 12288,
+// K 2048: 2.0 GHz, 47 per cent of their cycles): the order of tiles took 0.67 GB of misses in L2 to 0.41 there (143 -> 139 us, vendor 135 - 143; N 2048, K 6144 69 -> 63, 73) and 6146
+// rows, N 3072, K 768 with GELU from 52 to 40.  x through registers, two buffers: 18 per cent behind on average over 454 products, a quarter below 300 rows.  Taken back: eight
+// waves over 256 x 256 or 192 x 256 with both operands in LDS (level with these at 2773 rows, 0.97 of them at 8192^3), the same in four waves of 128 x 128 (level); a
+// workgroup for several tiles, which asks for the next one's first chunks behind the present one's last (within 2 per cent); K over two groups of waves (behind four chunks ahead).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace vmi_tiles {
 
@@ -27,138 +29,148 @@ struct Bf16 {
   static __device__ __forceinline__ f32x4 mma(const v8& a, const v8& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 
-template <int MI, int NI, int KS>
-constexpr size_t tiles_lds() {
-  const size_t x = (size_t)KS * 2 * 16 * MI * 128, parts = KS == 2 ? (size_t)16 * MI * 64 * NI * 4 : 0;
-  return x > parts ? x : parts;
-}
-
 // The product of this workgroup's tile; early(m, s, SL) asks for what finish will read, behind the first requests of the product; finish(acc, m, s, SL) gets a lane's results, acc[n][i] = columns 16 (s + n) + 4 (lane / 16) .. + 3 of row m + 16 i, and does not look at
 // slabs from SL or rows from M on.  K % 64 == 0, N % 16 == 0, x and ldx 16-byte aligned, a matrix of x below 4 GiB.
-template <class H, int MI, int NI, int KS, bool PRIO, class Early, class Finish>
-__device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const void* w, int M, int N, int K, unsigned char* smem, Early&& early, Finish&& finish) {
+template <class H, int MI, int NI, int D, class Early, class Finish>
+__device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const void* w, int M, int N, int K, Early&& early, Finish&& finish) {
   using V8 = typename H::v8;
+  static_assert(D >= 2 && D <= 4, "a place a chunk, by name");
   constexpr int BM = 16 * MI, BN = 64 * NI, ST = BM * 128, XU = BM * 8 / 256;   // 16-byte pieces of x a thread brings
-  const int tid = threadIdx.x & 255, lane = tid & 63, kc = lane >> 4, r16 = lane & 15;
-  const int g = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned char* xs = smem + g * 2 * ST;
-  const int SL = N >> 4, NB = (N + BN - 1) / BN, MB = (M + BM - 1) / BM;
-  // workgroups go to the eight dies in turn: each die takes a run of whole columns of tiles, whose weights it then reads once
+  constexpr int AHEAD = 4, STEPS = 2 * MI, ASKS = XU + 2 * NI, PER = (ASKS + STEPS - 1) / STEPS;
+  static_assert(STEPS >= AHEAD, "fragments of one chunk");
+  // (arrays by name: only so does the compiler know that a read of one does not wait for what is on its way into another)
+  __shared__ __attribute__((aligned(1024))) unsigned char xs0[ST], xs1[ST], xs2[D > 2 ? ST : 1], xs3[D > 3 ? ST : 1];
+  unsigned char* const xs[4] = {xs0, xs1, xs2, xs3};
+  const int tid = threadIdx.x, lane = tid & 63, kc = lane >> 4, r16 = lane & 15, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int SL = N >> 4, NB = (N + BN - 1) / BN, MB = (M + BM - 1) / BM, nkb = K >> 6;
+  // workgroups go to the eight dies in turn: each die takes a run of tiles, 1024 rows of x down and then the next columns, so that the tiles of a die that are under way
+  // together share their rows and weights in its L2
+  constexpr int DOWN = 1024 / BM;
   const int all = NB * MB, die = (int)blockIdx.x & 7, tile = die * (all >> 3) + min(die, all & 7) + ((int)blockIdx.x >> 3);
-  const int m0 = tile % MB * BM, s0 = tile / MB * 4 * NI + wave * NI;
-  const int nkb = K >> 6, per = (nkb + KS - 1) / KS, k0 = g * per, k1 = min(nkb, k0 + per);
-  // (rows past the last, slabs past the last and steps past the end are those again: no lane-wise condition around a load)
-  const char* xb = static_cast<const char*>(x);
-  uint32_t xo[XU];
+  const int band = tile / (DOWN * NB), in = tile - band * DOWN * NB, rows = min(DOWN, MB - band * DOWN), col = in / rows;
+  const int m0 = (band * DOWN + in - col * rows) * BM, s0 = col * 4 * NI + wave * NI;
+  // (rows past the last, slabs past the last and chunks past the end are those again: no lane-wise condition around a load)
+  const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(x), 0, -1, 0x20000);
+  uint32_t xo[XU], wo[NI];
 #pragma unroll
   for (int i = 0; i < XU; ++i) xo[i] = (uint32_t)min(m0 + (tid >> 3) + 32 * i, M - 1) * (uint32_t)(ldx * 2) + (uint32_t)((tid & 7) ^ ((tid >> 3) & 7)) * 16;
-  const char* wb[NI];
+  const int first = min(s0, SL - 1);
+  const __amdgpu_buffer_rsrc_t wb =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(w)) + (int64_t)first * (K >> 5) * 1024, 0, -1, 0x20000);
 #pragma unroll
-  for (int n = 0; n < NI; ++n) wb[n] = static_cast<const char*>(w) + (int64_t)min(s0 + n, SL - 1) * (K >> 5) * 1024;
-  V8 xr[XU], wr[2][2][NI];
-  auto load_x = [&](int kb) {
-    const uint32_t at = (uint32_t)min(kb, nkb - 1) * 128;
-#pragma unroll
-    for (int i = 0; i < XU; ++i) xr[i] = *reinterpret_cast<const V8*>(xb + (xo[i] + at));
-  };
-  auto load_w = [&](V8(&to)[2][NI], int kb) {
-    const int k = min(kb, nkb - 1);
-#pragma unroll
-    for (int n = 0; n < NI; ++n)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) to[j][n] = *reinterpret_cast<const V8*>(wb[n] + k * 2048 + (uint32_t)(j * 1024 + lane * 16));
-  };
-  auto put_x = [&](int s) {
-#pragma unroll
-    for (int i = 0; i < XU; ++i) *reinterpret_cast<V8*>(xs + s * ST + i * 4096 + tid * 16) = xr[i];
+  for (int n = 0; n < NI; ++n) wo[n] = (uint32_t)(min(s0 + n, SL - 1) - first) * (uint32_t)(K >> 5) * 1024;
+  V8 wr[D][2][NI], f[AHEAD];
+  // request i of chunk kb, which goes to place d: x first, which every wave waits for
+  auto ask = [&](int i, int d, int kb) {
+    if (i < XU) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, (__attribute__((address_space(3))) void*)(xs[d] + i * 4096 + wave * 1024), 16, xo[i], kb * 128, 0, 0);
+    } else if (i < ASKS) {
+      const int n = (i - XU) >> 1, j = (i - XU) & 1;
+      wr[d][j][n] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(wb, lane * 16 + j * 1024, wo[n] + (uint32_t)kb * 2048, 0));
+    }
   };
   const int frag = r16 * 128 + ((kc ^ (r16 & 7)) * 16);
+  auto read = [&](const unsigned char* from, int q) { return *reinterpret_cast<const V8*>(from + (frag ^ (q / MI * 64)) + q % MI * 2048); };
   f32x4 acc[NI][MI];
 #pragma unroll
   for (int n = 0; n < NI; ++n)
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[n][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  load_x(k0);
-  load_w(wr[0], k0);
-  put_x(0);
-  load_x(k0 + 1);
-  if (KS == 1 || g == 0) early(m0 + r16, s0, SL);
-  __syncthreads();
-  auto chunk = [&](int kb, int s, V8(&cur)[2][NI], V8(&nxt)[2][NI]) {
-    load_w(nxt, kb + 1);
-    put_x(s ^ 1);   // (every wave has passed the barrier behind its reads of that buffer)
-    load_x(kb + 2);
-    V8 f[2][MI];
+  // The x of the next chunk is there for every wave: this one has waited for all it asked for before that chunk's weights, the BEHIND whole chunks after those left out
+  // (s_waitcnt counts in order; the barrier is the plain one, a fence would wait for all of x that is on its way)
+  auto x_landed = [](auto behind) {
+    constexpr int V = decltype(behind)::value * ASKS + 2 * NI;
+    static_assert(V < 64, "vmcnt has six bits");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (V & 15) | (V >> 4 << 14));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+  for (int d = 0; d < D - 1; ++d)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) f[j][i] = *reinterpret_cast<const V8*>(xs + s * ST + (frag ^ (j * 64)) + i * 2048);
-    if (KS == 1 || kb < k1) {   // (scalar: an odd number of chunks)
-      if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
+    for (int i = 0; i < ASKS; ++i) ask(i, d, min(d, nkb - 1));
+  early(m0 + r16, s0, SL);
+  x_landed(std::integral_constant<int, D - 2>{});
+  // The chunk in place d, and chunk kb on its way into the place of the one before (whose readers have all passed the barrier): steps of one fragment of x, which was asked
+  // for AHEAD steps before, against the wave's NI of W, and its share of the requests.  A chunk that is none is zeros, x and W
+  auto chunk = [&](auto more, int d, int kb, bool on) {
+    auto fragment = [&](int q) {
+      const V8 v = read(xs[d], q);
+      return on ? v : V8{};
+    };
+    if (!on) {   // (scalar)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int n = 0; n < NI; ++n) acc[n][i] = H::mma(cur[j][n], f[j][i], acc[n][i]);
-      if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
+        for (int n = 0; n < NI; ++n) wr[d][j][n] = V8{};
     }
-    // requests, then x on, then the fragments three ahead of the products that take them
-    __builtin_amdgcn_sched_group_barrier(0x020, 2 * NI, 0);
-    __builtin_amdgcn_sched_group_barrier(0x200, XU, 0);
-    __builtin_amdgcn_sched_group_barrier(0x020, XU, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
 #pragma unroll
-    for (int i = 0; i < 2 * MI - 3; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, NI, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    for (int q = 0; q < AHEAD; ++q) f[q] = fragment(q);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < STEPS; ++q) {
+      if constexpr (decltype(more)::value) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) ask(q * PER + i, (d + D - 1) % D, kb);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < NI; ++n) acc[n][q % MI] = H::mma(wr[d][q / MI][n], f[q % AHEAD], acc[n][q % MI]);
+      if (q + AHEAD < STEPS) f[q % AHEAD] = fragment(q + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, 3 * NI, 0);
-    __syncthreads();
   };
-  for (int i = 0; i < per; i += 2) {
-    chunk(k0 + i, 0, wr[0], wr[1]);
-    if (i + 1 < per) chunk(k0 + i + 1, 1, wr[1], wr[0]);
-  }
-  if constexpr (KS == 2) {
-    f32x4* part = reinterpret_cast<f32x4*>(smem) + wave * NI * MI * 64 + lane;
-    if (g == 1) {
+  constexpr std::true_type asking{};
+  constexpr std::false_type asked{};
+  int c = 0;
+  for (; c + D < nkb; c += D) {
 #pragma unroll
-      for (int n = 0; n < NI; ++n)
-#pragma unroll
-        for (int i = 0; i < MI; ++i) part[(n * MI + i) * 64] = acc[n][i];
+    for (int d = 0; d < D; ++d) {
+      chunk(asking, d, min(c + d + D - 1, nkb - 1), true);
+      x_landed(std::integral_constant<int, D - 2>{});
     }
-    __syncthreads();
-    if (g == 1) return;
-#pragma unroll
-    for (int n = 0; n < NI; ++n)
-#pragma unroll
-      for (int i = 0; i < MI; ++i) acc[n][i] += part[(n * MI + i) * 64];
+  }
+  // the last D places, 1 to D of them chunks (without a branch around a product, whose accumulators would change registers)
+  chunk(asking, 0, nkb - 1, true);
+  x_landed(std::integral_constant<int, D - 2>{});
+  chunk(asked, 1, 0, c + 1 < nkb);
+  if constexpr (D > 2) {
+    x_landed(std::integral_constant<int, D - 3>{});
+    chunk(asked, 2, 0, c + 2 < nkb);
+  }
+  if constexpr (D > 3) {
+    x_landed(std::integral_constant<int, 0>{});
+    chunk(asked, 3, 0, c + 3 < nkb);
   }
   finish(acc, m0 + r16, s0, SL);
 }
 
 // ---- which tile -----------------------------------------------------------------------------------------------------------------
 struct Tile {
-  int mi, ni, ks;
-  bool prio;            // the products at a raised wave priority: ahead where waves of two workgroups share a compute unit's matrix cores
+  int mi, ni, d;
   float alone, beside;  // us per 64 columns of K: one workgroup a compute unit, and a workgroup's share of a full one
+  float ends;           // ... as many of which its ends take
 };
-// fitted to 258 products of 100 to 8192 rows, N 512 to 24576, K 768 to 12288
-constexpr Tile TILES[] = {{8, 4, 1, false, .90f, .83f}, {8, 3, 1, false, .77f, .76f}, {6, 4, 1, true, .85f, .61f}, {6, 3, 1, false, .64f, .51f}, {6, 2, 1, false, .47f, .42f},
-                          {8, 2, 1, false, .50f, .50f}, {4, 2, 1, false, .44f, .30f}, {4, 2, 2, false, .39f, .34f}, {4, 1, 2, false, .27f, .22f}};
+// fitted to 459 products of 33 to 8192 rows, N 256 to 24576, K 256 to 12288
+constexpr Tile TILES[] = {{8, 4, 2, .695f, .687f, 7.8f}, {8, 3, 2, .908f, .582f, 5.3f}, {8, 3, 4, .657f, .601f, 5.9f}, {6, 3, 2, .561f, .473f, 4.7f},
+                          {6, 3, 4, .485f, .695f, 8.0f}, {6, 2, 2, .439f, .354f, 3.8f}, {6, 2, 4, .357f, .399f, 5.6f}, {4, 2, 2, .380f, .268f, 3.8f},
+                          {4, 2, 4, .288f, .291f, 6.1f}, {4, 1, 4, .184f, .182f, 5.2f}, {2, 1, 2, .320f, .133f, 2.5f}, {2, 1, 4, .131f, .104f, 5.1f}};
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 
 // us, as the chip's tiles are dealt
 inline float tiles_cost(int i, int M, int N, int K) {
   const Tile& t = TILES[i];
   const int64_t n = (int64_t)((M + 16 * t.mi - 1) / (16 * t.mi)) * ((N + 64 * t.ni - 1) / (64 * t.ni)), share = (n + 255) / 256;
-  return (share == 1 ? t.alone : share * t.beside) * ((float)(K >> 6) + (t.ks == 2 ? 9.5f : 6.f));
+  const int chunks = ((K >> 6) + t.d - 1) / t.d * t.d;
+  return 2.f + (share == 1 ? t.alone : share * t.beside) * ((float)chunks + t.ends);
 }
 
-// The tile whose largest share of a compute unit ends first: so many tiles one behind the other, each 64 columns of K at a time and as long as 6 such at its ends (9.5
-// where two halves meet).  On average 0.5 per cent behind the best of the list over those 258 products, 11 at most.  (us, 128 x 256 / 128 x 192 / 96 x 256 / 64 x 128: 2770
-// rows, N 2048, K 6144 86 / 69 / 75 / 89, of 176 / 242 / 232 / 704 tiles; 2100 rows, N 768, K 768 16 / 13 / 13 / 7.)
+// The tile whose largest share of a compute unit ends first: so many tiles one behind the other, each 64 columns of K at a time and as long as `ends` such at its ends.  On
+// average 0.6 per cent behind the best of the list over those 459 products, 14 at most.  (us, 128 x 256 / 128 x 192, four chunks / 96 x 128, four / 32 x 64, four: 2773 rows, N 2048,
+// K 6144 81 / 63 / 75 / 190; 300 rows, the same 70 / 46 / 34 / 23 and 64 x 64 19.)
 inline int tiles_pick(int M, int N, int K) {
   int best = 0;
   float least = 0.f;
