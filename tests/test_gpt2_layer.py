@@ -810,10 +810,11 @@ def test_products_of_many_rows_in_tiles(M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(771, 7584, 256), (1090, 5408, 192), (1650, 7184, 128), (1732, 6800, 64), (1369, 4368, 256), (1360, 4368, 320), (2122, 2832, 384), (1361, 4400, 192),
-                                   (521, 7184, 128), (515, 7184, 64), (2101, 2064, 3072), (257, 7344, 128), (259, 7312, 64), (260, 6544, 512), (259, 6608, 832), (258, 6544, 448),
-                                   (197, 7184, 128), (193, 7056, 64), (194, 6992, 256), (130, 6560, 832), (195, 7136, 640), (193, 7152, 192), (70, 5456, 256), (68, 5456, 576),
-                                   (66, 5520, 640), (66, 5968, 192), (65, 5648, 128), (66, 5520, 64), (1, 160, 512), (7, 32, 64), (11, 16, 128), (1, 32, 192), (40, 272, 320)])
+@pytest.mark.parametrize("M,N,K", [(2029, 6544, 768), (2024, 6576, 704), (2507, 7216, 256), (2517, 7216, 192), (1859, 3232, 512), (866, 6624, 832), (963, 5920, 1152),
+                                   (1375, 4368, 448), (2026, 4400, 128), (2068, 4368, 64), (321, 7536, 128), (354, 6800, 64), (269, 6544, 512), (263, 6688, 832),
+                                   (257, 6544, 1152), (259, 6576, 448), (769, 7600, 128), (778, 7568, 64), (391, 6560, 1536), (386, 6560, 1216), (195, 7088, 128),
+                                   (193, 7056, 64), (199, 7008, 256), (132, 6624, 576), (130, 6736, 640), (194, 7136, 192), (70, 5456, 512), (67, 5456, 576), (66, 5968, 640),
+                                   (68, 5536, 448), (1, 32, 384), (8, 16, 64), (5, 32, 512), (1, 112, 576), (1, 160, 1152), (16, 16, 448), (1, 160, 64), (40, 272, 320)])
 def test_every_tile_with_every_number_of_chunks_left(M, N, K):
     """tiles_kernel, each tile of its list with each remainder of K's chunks of 64 by the two or four that it has in flight, rows and columns left over.  A chunk that is none adds
     nothing where the last one holds an infinity: the row that has one is infinite or, where the weight is zero, NaN, and no other row is touched."""

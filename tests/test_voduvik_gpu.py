@@ -301,6 +301,42 @@ def test_many_rows_in_tiles_with_the_gated_unit_behind(M, N, K, split):
             assert out.shape == (M, split) and bool(((out.double() - y[:, :split]).abs() <= 2.0 ** -8 * y[:, :split].abs() + 1e-3).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(2029, 6560, 768), (2507, 7232, 256), (1859, 3232, 512), (963, 5920, 1152), (2026, 4416, 128), (321, 7552, 128), (269, 6560, 512),
+                                   (257, 6560, 1152), (769, 7616, 128), (391, 6560, 1536), (195, 7104, 128), (199, 7008, 256), (130, 6752, 640), (70, 5472, 512),
+                                   (66, 5984, 640), (1, 32, 384), (5, 32, 512), (1, 160, 1152), (1, 160, 64)])
+def test_products_of_many_rows_alone(M, N, K):
+    """vmi_hy_product_tiles, each of its tiles: rows, columns and chunks of K left over, rows of a wider tensor; in bfloat16 with a bias in 32 bits (half a unit of the result) and in
+    32 bits (K products summed in another order).  Beside the result nothing is written."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M + N + K)
+    x, w, b = (torch.randn(*s, generator=g, device=dev()) for s in ((M, 2 * K), (N, K), (N,)))
+    t = ops.MatrixTiles(w / K ** 0.5, torch.bfloat16, dense=True)
+    x = x.to(torch.bfloat16)[:, K:]
+    y = x.double() @ t.dense.double().T
+    err = 2.0 ** -24 * K ** 0.5 * 8 * (x.double().abs() @ t.dense.double().abs().T) / K ** 0.5
+    got = ops.product_tiles(x, t, float_out=True)
+    assert got.dtype == torch.float32 and bool(((got.double() - y).abs() <= err + 1e-6).all())
+    for bias in (None, b):
+        want = y if bias is None else y + b.double()
+        got = ops.product_tiles(x, t, bias)
+        assert got.dtype == torch.bfloat16 and bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-6).all())
+
+
+def test_products_of_many_rows_alone_refuse_what_is_not_built():
+    from vllmini_amd import hybrid_ops as ops
+
+    x, t = torch.zeros((64, 128), dtype=torch.bfloat16, device=dev()), ops.MatrixTiles(torch.zeros((64, 128), device=dev()), torch.bfloat16)
+    odd = ops.MatrixTiles(torch.zeros((64, 96), device=dev()), torch.bfloat16)
+    wide = torch.zeros((64, 136), dtype=torch.bfloat16, device=dev())
+    for bad in (lambda: ops.product_tiles(x.float(), t), lambda: ops.product_tiles(x[:, :96], t), lambda: ops.product_tiles(x[:, :96], odd), lambda: ops.product_tiles(wide[:, 4:132], t),
+                lambda: ops.product_tiles(x, t, torch.zeros(64, dtype=torch.bfloat16, device=dev())), lambda: ops.product_tiles(x, t, torch.zeros(64, device=dev()), True),
+                lambda: ops.product_tiles(torch.zeros((64, 132), dtype=torch.bfloat16, device=dev())[:, :128], t), lambda: ops.product_tiles(x, t, torch.zeros(32, device=dev()))):
+        with pytest.raises(RuntimeError):
+            bad()
+    assert ops.product_tiles_pay(x, t) and not ops.product_tiles_pay(x[:, :96], odd) and not ops.product_tiles_pay(wide[:, 4:132], t) and not ops.product_tiles_pay(x.float(), t)
+
+
 def test_many_rows_in_tiles_refuse_what_is_not_built():
     from vllmini_amd import hybrid_ops as ops
 

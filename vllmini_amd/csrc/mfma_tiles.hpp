@@ -135,16 +135,14 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
   }
   // the last D places, 1 to D of them chunks (without a branch around a product, whose accumulators would change registers)
   chunk(asking, 0, nkb - 1, true);
-  x_landed(std::integral_constant<int, D - 2>{});
-  chunk(asked, 1, 0, c + 1 < nkb);
-  if constexpr (D > 2) {
-    x_landed(std::integral_constant<int, D - 3>{});
-    chunk(asked, 2, 0, c + 2 < nkb);
-  }
-  if constexpr (D > 3) {
-    x_landed(std::integral_constant<int, 0>{});
-    chunk(asked, 3, 0, c + 3 < nkb);
-  }
+  auto rest = [&](auto dd) {
+    constexpr int d = decltype(dd)::value;
+    if constexpr (d < D) {
+      x_landed(std::integral_constant<int, (d < D ? D - 1 - d : 0)>{});
+      chunk(asked, d, 0, c + d < nkb);
+    }
+  };
+  rest(std::integral_constant<int, 1>{}), rest(std::integral_constant<int, 2>{}), rest(std::integral_constant<int, 3>{});
   finish(acc, m0 + r16, s0, SL);
 }
 
@@ -154,10 +152,11 @@ struct Tile {
   float alone, beside;  // us per 64 columns of K: one workgroup a compute unit, and a workgroup's share of a full one
   float ends;           // ... as many of which its ends take
 };
-// fitted to 459 products of 33 to 8192 rows, N 256 to 24576, K 256 to 12288
-constexpr Tile TILES[] = {{8, 4, 2, .695f, .687f, 7.8f}, {8, 3, 2, .908f, .582f, 5.3f}, {8, 3, 4, .657f, .601f, 5.9f}, {6, 3, 2, .561f, .473f, 4.7f},
-                          {6, 3, 4, .485f, .695f, 8.0f}, {6, 2, 2, .439f, .354f, 3.8f}, {6, 2, 4, .357f, .399f, 5.6f}, {4, 2, 2, .380f, .268f, 3.8f},
-                          {4, 2, 4, .288f, .291f, 6.1f}, {4, 1, 4, .184f, .182f, 5.2f}, {2, 1, 2, .320f, .133f, 2.5f}, {2, 1, 4, .131f, .104f, 5.1f}};
+// fitted to 1080 products of 33 to 8192 rows, N 256 to 45 056, K 256 to 16 384, weights in the last cache and not
+constexpr Tile TILES[] = {{8, 4, 2, .836f, .727f, 6.9f}, {8, 3, 2, .884f, .594f, 5.5f}, {8, 3, 4, .630f, .715f, 7.7f}, {6, 3, 2, .680f, .483f, 4.4f},
+                          {6, 2, 2, .545f, .375f, 3.0f}, {6, 2, 4, .431f, .581f, 5.0f}, {8, 2, 2, .590f, .445f, 3.8f}, {8, 2, 4, .448f, 1.009f, 9.9f},
+                          {4, 2, 2, .452f, .312f, 2.4f}, {4, 2, 4, .336f, .354f, 4.6f}, {4, 1, 4, .177f, .192f, 6.3f}, {2, 1, 2, .240f, .165f, 1.3f},
+                          {2, 1, 4, .148f, .129f, 5.1f}};
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 
 // us, as the chip's tiles are dealt
@@ -169,7 +168,7 @@ inline float tiles_cost(int i, int M, int N, int K) {
 }
 
 // The tile whose largest share of a compute unit ends first: so many tiles one behind the other, each 64 columns of K at a time and as long as `ends` such at its ends.  On
-// average 0.6 per cent behind the best of the list over those 459 products, 14 at most.  (us, 128 x 256 / 128 x 192, four chunks / 96 x 128, four / 32 x 64, four: 2773 rows, N 2048,
+// average 0.7 per cent behind the best of the list over those products.  (us, 128 x 256 / 128 x 192, four chunks / 96 x 128, four / 32 x 64, four: 2773 rows, N 2048,
 // K 6144 81 / 63 / 75 / 190; 300 rows, the same 70 / 46 / 34 / 23 and 64 x 64 19.)
 inline int tiles_pick(int M, int N, int K) {
   int best = 0;

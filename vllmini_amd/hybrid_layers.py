@@ -17,8 +17,8 @@ What a decoder asks of a mixer: page_rows() and state_shapes(), the cache tensor
 
 The residual stream is float32 (`Residual`).  Steps of few tokens run on the streaming kernels with everything fused around the
 products (norm in front, gated unit / head gate / residual add behind); from DENSE_MIN_TOKENS tokens on (from DENSE_MIN_TOKENS_LARGE
-for matrices of DENSE_LARGE elements, unless the kernel behind a norm can keep its rows in LDS) the products go to the vendor library (F.linear, as the prefill of the GPT-2 decoder does)
-with one elementwise kernel between two of them, those with a gated unit behind them to tiles of this build's own where these are ahead (gated_product).
+for matrices of DENSE_LARGE elements, unless the kernel behind a norm can keep its rows in LDS) the products go to tiles of this build's own, with the gated unit
+where one stands behind them, or to the vendor library where that is ahead (product, gated_product), with one elementwise kernel between two of them.
 """
 from __future__ import annotations
 
@@ -48,6 +48,13 @@ def dense(tokens: int, w: MatrixTiles, normed: bool = False) -> bool:
 def float_product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x W^T as float32, whatever the operands' type."""
     return torch.mm(x, w.t()) if x.dtype == torch.float32 else torch.mm(x, w.t(), out_dtype=torch.float32)
+
+
+def product(x: torch.Tensor, w: MatrixTiles, bias: Optional[torch.Tensor] = None, dense_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x W^T (+ bias: float32 for the tiles, the element type for the vendor's) of many rows: in tiles of this build's own where they are ahead of the vendor's product."""
+    if ops.product_tiles_pay(x, w):
+        return ops.product_tiles(x, w, bias)
+    return F.linear(x, w.dense, dense_bias)
 
 
 class Norm:
@@ -141,13 +148,13 @@ class Residual:
                   dense_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """norm(x) W^T (+ bias) in the element type."""
         if dense(step.T, w, True):
-            return F.linear(self.normed(norm), w.dense, dense_bias)
+            return product(self.normed(norm), w, bias, dense_bias)
         return ops.linear(self.settle(), w, norm=norm.args, bias=bias)
 
     def branch_out(self, o: torch.Tensor, w: MatrixTiles, step: StepLayout) -> None:
         """x += o W^T."""
         if dense(step.T, w):
-            self.pending = F.linear(o, w.dense)
+            self.pending = product(o, w)
         else:
             ops.linear(o, w, residual=True, out=self.settle())
 
@@ -323,7 +330,8 @@ class ConcatProjection:
     def run(self, res: Residual, x0: torch.Tensor) -> None:
         x = res.settle()
         if dense(x.shape[0], self.w):
-            res.x = float_product(ops.concat(x, x0, res.dtype), self.w.dense)      # (the stream stays float32)
+            both = ops.concat(x, x0, res.dtype)                                    # (the stream stays float32)
+            res.x = ops.product_tiles(both, self.w, float_out=True) if ops.product_tiles_pay(both, self.w) else float_product(both, self.w.dense)
         else:
             res.x = ops.linear(x, self.w, x2=x0, float_out=(x.shape[1], 1.0))
 
@@ -535,7 +543,7 @@ class ParallelBlock:
         rows = torch.empty((T, m + self.ff), dtype=self.dtype, device=res.x.device)      # [mixer cores | gated unit]
         if dense(T, self.w_in, True):
             h = res.normed(self.norm)
-            proj = gated_product(h, self.w_in, self.unit, self.n_in, rows[:, m:]) if self.ff else F.linear(h, self.w_in.dense)
+            proj = gated_product(h, self.w_in, self.unit, self.n_in, rows[:, m:]) if self.ff else product(h, self.w_in)
         else:
             proj = ops.linear(res.settle(), self.w_in, norm=self.norm.args, **(
                 {"glu": self.unit, "glu_from": self.n_in, "glu_out": rows[:, m:]} if self.ff else {}))
@@ -546,12 +554,12 @@ class ParallelBlock:
         at, branches = 0, []
         for w in self.w_out[:2]:
             o = rows[:, at:at + w.K]
-            branches.append(F.linear(o, w.dense) if dense(T, w) else ops.linear(o, w))
+            branches.append(product(o, w) if dense(T, w) else ops.linear(o, w))
             at += w.K
         add = None
         if self.ff:
             if dense(T, self.w_out[2]):
-                add = F.linear(rows[:, m:], self.w_out[2].dense)
+                add = product(rows[:, m:], self.w_out[2])
             else:
                 ops.linear(rows[:, m:], self.w_out[2], residual=True, out=res.settle())
         self.mixer.merge(res, branches, add)

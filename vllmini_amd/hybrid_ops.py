@@ -70,6 +70,8 @@ SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_linear_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_linear_tiles_pay": (_i32, [_i32, _i32, _i32, _i32, _i32]),
+    "vmi_hy_product_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
+    "vmi_hy_product_tiles_pay": (_i32, [_i32, _i32, _i32, ctypes.c_int64, _i32]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_slabs": (_i32, [_i32, _i32, _i32, _i32]),
@@ -281,6 +283,31 @@ def linear_tiles_pay(M: int, w: MatrixTiles, split: int = 0) -> bool:
 @functools.lru_cache(maxsize=4096)
 def _tiles_pay(M: int, N: int, K: int, split: int, dtype: torch.dtype) -> bool:
     return bool(load().vmi_hy_linear_tiles_pay(M, N, K, split, DTYPES[dtype]))
+
+
+def product_tiles(x: torch.Tensor, w: MatrixTiles, bias: Optional[torch.Tensor] = None, float_out: bool = False) -> torch.Tensor:
+    """x W^T (+ bias, float32) of tens of bfloat16 rows and more (K a multiple of 64, rows of x aligned to 16 bytes), a new tensor [M, N] of bfloat16 or, float_out, of float32."""
+    device, stream = _on(x)
+    M, N, K = int(x.shape[0]), w.N, w.K
+    _need(w.groups == 1 and w.tiles.dtype == torch.bfloat16 and w.tiles.device == x.device, "hybrid_ops.product_tiles: one bfloat16 matrix on x's device")
+    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, f"hybrid_ops.product_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
+    _need(bias is None or (not float_out and bias.dtype == torch.float32 and bias.numel() >= N and bias.is_contiguous() and bias.device == x.device),
+          "hybrid_ops.product_tiles: bias float32 [N], with a result in bfloat16")
+    y = torch.empty((M, N), dtype=torch.float32 if float_out else x.dtype, device=x.device)
+    a = LinearArgs(x=x.data_ptr(), w=w.tiles.data_ptr(), bias=_ptr(bias), y=y.data_ptr(), ldx=x.stride(0), ldy=N, M=M, N=N, K=K, groups=1, n_out=N, scale=1.0,
+                   x_kind=X_ROWS, epilogue=E_FLOAT if float_out else E_STORE, dtype=DTYPES[x.dtype], device=device)
+    _check(load().vmi_hy_product_tiles(ctypes.byref(a), stream))
+    return y
+
+
+def product_tiles_pay(x: torch.Tensor, w: MatrixTiles) -> bool:
+    """Whether product_tiles takes these rows and is ahead of the vendor's product."""
+    return w.groups == 1 and x.dtype == w.tiles.dtype and x.data_ptr() % 16 == 0 and _product_pays(x.shape[0], w.N, w.K, x.stride(0), w.tiles.dtype)
+
+
+@functools.lru_cache(maxsize=4096)
+def _product_pays(M: int, N: int, K: int, ldx: int, dtype: torch.dtype) -> bool:
+    return bool(load().vmi_hy_product_tiles_pay(M, N, K, ldx, DTYPES[dtype]))
 
 
 @functools.lru_cache(maxsize=4096)
