@@ -269,6 +269,22 @@ def test_prompts_through_the_vendors_products_or_the_decode_kernels_give_the_sam
         assert torch.equal(same[0], same[1])
 
 
+def test_prompts_past_one_native_call_in_tiles_or_the_vendors_products_give_the_same_logits():
+    """prefill_batch past NATIVE_PROMPT_MAX_TOKENS on either side of OWN_PRODUCTS_MAX_WORK, against the native call: the same five roundings a layer, sums in another order."""
+    rng = np.random.default_rng(11)
+    prompts = [rng.integers(0, 500, n).tolist() for n in (70, 1, 128, 16, 101)]
+    _, native = _model(num_blocks=400)
+    ref = native.prefill_batch(list(range(len(prompts))), prompts).float()
+    for most in (0, 10 ** 12):
+        _, many = _model(num_blocks=400)
+        many.NATIVE_PROMPT_MAX_TOKENS, many.OWN_PRODUCTS_MAX_WORK = 0, most
+        got = many.prefill_batch(list(range(len(prompts))), prompts).float()
+        assert float((got - ref).abs().max()) <= 2e-2 + 2e-2 * float(ref.abs().max()), most
+        for a, b in ((many.pool.key_cache, native.pool.key_cache), (many.pool.value_cache, native.pool.value_cache)):
+            used = sorted(x for i in range(len(prompts)) for x in native.pool.allocated_blocks[i])
+            assert float((a[used].float() - b[used].float()).abs().max()) <= 2e-2 * float(b[used].float().abs().max())
+
+
 def test_weights_that_lie_anywhere_take_the_operators_and_give_the_same_logits():
     """One-dimensional weights as views into one flat buffer, at addresses of two bytes' alignment: the prompts go through paged_attention_v1
     and torch's modules, as they do for everything the prompt kernels are not built for."""

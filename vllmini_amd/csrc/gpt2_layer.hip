@@ -846,10 +846,10 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
 }
 
 // Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
-// are ahead while rows are few, and the wider the rows the sooner they fall behind: 4 layers of prompts of 128 tokens in us, few-row kernels / tiles, width 256 1200
-// tokens 163 / 173, 1500 185 / 183; 512 500 151 / 179, 600 201 / 190; 640 400 205 / 201, 500 218 / 204; 768 350 199 / 214, 400 222 / 215; 896 150 208 / 209, 250 231 / 213;
-// 1024 150 207 / 218, 200 237 / 222, 300 319 / 235; 1152 100 185 / 233, 150 243 / 236, 300 367 / 264.
-static bool many_rows(int T, int E) { return (int64_t)T * E >= (E > 768 ? 160000 : E > 384 ? 300000 : 390000) && E % 64 == 0 && 4 * E <= 4608; }
+// are ahead while rows are few, and the wider the rows the sooner they fall behind; six launches a layer for four are what narrow ones wait for.  12 layers of prompts of 100 tokens
+// in us, few-row kernels / tiles, width 256 1600 tokens 541 / 605; 512 500 437 / 496, 600 579 / 508; 768 300 526 / 554, 350 588 / 584, 400 658 / 580; 1024 130 649 / 614, 160
+// 658 / 637, 200 730 / 634; 1152 130 703 / 706, 160 779 / 723.
+static bool many_rows(int T, int E) { return (int64_t)T * E >= (E > 768 ? 150000 : E > 640 ? 270000 : E > 384 ? 300000 : 390000) && E % 64 == 0 && 4 * E <= 4608; }
 
 template <int I, int EPI>
 static int launch_tiles(const LinearParams& p, hipStream_t stream) {

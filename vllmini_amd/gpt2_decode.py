@@ -14,7 +14,7 @@ for what the operators are actually batched over:
     (`native_layers`, vllmini_amd/gpt2_layer.py -> csrc/gpt2_layer.hip): LayerNorm + c_attn, c_proj + residual,
     LayerNorm + c_fc + GELU, mlp.c_proj + residual — four launches per layer where the torch modules take eleven
     (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt, layer_norm,
-    gelu), which lm_head uses for more than 16 rows, and prompts past NATIVE_PROMPT_MAX_TOKENS for their products but c_fc.
+    gelu), which lm_head uses for more than 16 rows, and prompts past OWN_PRODUCTS_MAX_WORK for their products but c_fc.
 
 `reference_off_by_one=True` reproduces the reference caller's seq_lens (length BEFORE the new
 token, scheduler.py:96, so the newest token is not attended); the default attends to it.
@@ -92,12 +92,13 @@ class GPT2PagedDecoder:
     """Prefill + batched decode of GPT-2 over a PagedKVPool, calling the two hot-path ops."""
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
-    # prompts of more tokens in all (times the width's square) take the vendor's products but for c_fc with its GELU: by the GPU's time alone they are level from
-    # some 2500 tokens of width 768 on, but their seven launches a layer take the host 150 us, and that is what a call of fewer waits for.  12 layers of prompts of
-    # 128 tokens, native / vendor in us: width 512 4000 tokens 1743 / 2138, 8000 2666 / 2795; 768 1000 1126 / 1847, 3000 1916 / 1981, 5000 2561 / 2544, 6000 2963 / 2910;
-    # 1024 1500 1666 / 1879, 2600 2165 / 2109; 1152 1500 1806 / 1864, 2100 2267 / 2125
+    # prompts of more tokens in all (times the width's square) issue their launches from here: the native call saves the host 150 us, which is what a call of fewer waits for.
+    # Their products are tiles of this build's own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond.  12
+    # layers of prompts of 100 tokens, tiles / vendor in us: width 256 8000 tokens 1485 / 2541, 512 1681 / 2570; 768 5000 1764 / 2187, 6000 2147 / 2357, 8000 2623 / 2787; 1024
+    # 4000 2084 / 2164, 5000 2522 / 2352, 7000 4024 / 3140; 1152 4000 2579 / 2691, 7000 3736 / 3791
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
     NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
+    OWN_PRODUCTS_MAX_WORK = 50 * 10 ** 8
     INFINITY_CACHE = 248 << 20        # bytes of the last cache in front of the memory, 256 MiB, that a step's activations and logits leave
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
@@ -374,8 +375,8 @@ class GPT2PagedDecoder:
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
         """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
         takes four or six launches (the decode step's linear kernels, or norms and tiles) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by
-        one native call, and six beyond: the vendor's products around one of this build's tiles for c_fc and its GELU (4 layers of 6300 tokens, width 768, 807 us
-        with F.gelu behind the vendor's, 747 so), and one kernel for the residual add with the norm behind it."""
+        one native call, and the same six issued from here beyond; past OWN_PRODUCTS_MAX_WORK the vendor's products around one of this build's tiles for c_fc and its GELU, and one
+        kernel for the residual add with the norm behind it."""
         d, pool, dev, sd = self.dims, self.pool, self.device, self.sd
         H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
         if T == 0:
@@ -403,19 +404,27 @@ class GPT2PagedDecoder:
                                    pool.value_cache, H, d.head_size, d.layer_norm_epsilon, self.scale)
             return self._logits(h, True)
         tiles = self.native_layers and d.n_embd % 64 == 0 and T * d.n_embd < 1 << 31
-        x, add = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"]), None
+        own = tiles and T * d.n_embd ** 2 <= self.OWN_PRODUCTS_MAX_WORK
+        x, add, pw = gpt2_layer.embed(up["ids"], up["pos"], sd["transformer.wte.weight"], sd["transformer.wpe.weight"]), None, self._packed
         for i in range(d.n_layer):
             p = f"transformer.h.{i}."
             ln_1, ln_2 = ((sd[f"{p}{k}.weight"], sd[f"{p}{k}.bias"], d.layer_norm_epsilon) for k in ("ln_1", "ln_2"))
-            qkv = F.linear(gpt2_layer.add_norm(x, ln_1, add), sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
+            h = gpt2_layer.add_norm(x, ln_1, add)
+            qkv = gpt2_layer.linear_tiles(h, pw[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"]) if own else F.linear(h, sd[p + "attn.c_attn.weight"], sd[p + "attn.c_attn.bias"])
             a = gpt2_layer.prompt_attention(qkv, up["tiles"], tile_rows, pool.key_cache, pool.value_cache, up["tables"][i], H, self.scale)
+            if own:
+                x = gpt2_layer.linear_tiles(a, pw[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"], residual=x)
+                h = gpt2_layer.linear_tiles(gpt2_layer.add_norm(x, ln_2), pw[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True)
+                x = gpt2_layer.linear_tiles(h, pw[p + "mlp.c_proj.weight"], sd[p + "mlp.c_proj.bias"], residual=x)
+                continue
             h = gpt2_layer.add_norm(x, ln_2, F.linear(a, sd[p + "attn.c_proj.weight"], sd[p + "attn.c_proj.bias"]))
             if tiles:
-                h = gpt2_layer.linear_tiles(h, self._packed[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True)
+                h = gpt2_layer.linear_tiles(h, pw[p + "mlp.c_fc.weight"], sd[p + "mlp.c_fc.bias"], gelu=True)
                 add = F.linear(h, sd[p + "mlp.c_proj.weight"], sd[p + "mlp.c_proj.bias"])
             else:
                 add = self._mlp(h, p)
-        x += add
+        if add is not None:
+            x += add
         h = gpt2_layer.add_norm(x, (sd["transformer.ln_f.weight"], sd["transformer.ln_f.bias"], d.layer_norm_epsilon), rows=up["last"])
         return self._logits(h, True)
 
