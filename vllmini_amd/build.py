@@ -77,6 +77,7 @@ SOURCES = [*CORE, SRC_ABSENT, *EXTRAS]                        # every unit of th
 HDR = os.path.join(CSRC, "pa_kernel.hpp")
 HDR_QUEUE = os.path.join(CSRC, "pa_queue.hpp")
 HDR_SPLIT = os.path.join(CSRC, "pa_split.hpp")
+HDR_LANES = os.path.join(CSRC, "lane_ops.hpp")                # (shared by all three libraries)
 HDRS_HOST = [os.path.join(CSRC, "pa_host.hpp"), os.path.join(CSRC, "pa_cache_fp8.hpp")]
 INCLUDE = os.path.join(REPO_ROOT, "include")
 OUT_DIR = os.path.join(PKG_DIR, "_C")
@@ -87,12 +88,12 @@ EXTRAS_LIB_PATH = os.path.join(OUT_DIR, "libvmi_paged_attention_extras.so")
 # the decode harness's own library (include/vmi_gpt2_layer.h): the GPT-2 block's linear layers — one unit, no shared objects,
 # not part of the operators' boundary; loaded by vllmini_amd/gpt2_layer.py only
 SRC_LAYER = os.path.join(CSRC, "gpt2_layer.hip")
-HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(CSRC, "gpt2_rows.hpp"), os.path.join(CSRC, "gpt2_head.hpp"), os.path.join(CSRC, "mfma_tiles.hpp"), os.path.join(CSRC, "step_inputs.hpp"), os.path.join(INCLUDE, "vmi_gpt2_layer.h")]
+HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(CSRC, "gpt2_rows.hpp"), os.path.join(CSRC, "gpt2_head.hpp"), os.path.join(CSRC, "mfma_tiles.hpp"), os.path.join(CSRC, "step_inputs.hpp"), HDR_LANES, os.path.join(INCLUDE, "vmi_gpt2_layer.h")]
 LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 
 # the layers of decoders that mix recurrences, linear and softmax attention (include/vmi_hybrid.h), loaded by hybrid_ops.py only
 SRC_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hip") for t in ("linear", "rows", "tiles", "rglru", "latent", "state", "attention")]
-HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "linear", "softmax")] + [os.path.join(CSRC, f"{t}.hpp") for t in ("mfma_tiles", "step_inputs")]
+HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "linear", "softmax")] + [os.path.join(CSRC, f"{t}.hpp") for t in ("mfma_tiles", "step_inputs", "lane_ops")]
 HYBRID_LIB_PATH = os.path.join(OUT_DIR, "libvmi_hybrid.so")
 
 # the operators' checks and calls in native code: an extension module over torch's C++ interface, loaded by _lib.py (no device code)
@@ -142,7 +143,7 @@ def _units_of(kind: str):
 
 
 def _deps(kind: str = "product") -> list[str]:
-    return [*(s for s, _ in _units_of(kind)), *TABLES, HDR, HDR_QUEUE, HDR_SPLIT, *HDRS_HOST,
+    return [*(s for s, _ in _units_of(kind)), *TABLES, HDR, HDR_QUEUE, HDR_SPLIT, HDR_LANES, *HDRS_HOST,
             os.path.join(INCLUDE, "vmi_paged_attention.h"), os.path.join(INCLUDE, "vmi_paged_attention_extras.h"),
             os.path.join(INCLUDE, "vmi_paged_attention_diag.h"),
             os.path.abspath(__file__)]

@@ -23,6 +23,7 @@
 
 #include <string>
 
+#include "lane_ops.hpp"
 #include "step_inputs.hpp"
 #include "vmi_gpt2_layer.h"
 
@@ -134,7 +135,7 @@ __device__ __forceinline__ void ln_square_pair(uint32_t x2, float neg_mean, floa
 }
 
 // sum over the LPR consecutive lanes that share a row: inside a row of 16 lanes on the DPP cross-lane paths (quad permutes, then
-// the half-row and row mirrors: each a VALU operand modifier, no LDS round trip), beyond that through ds_bpermute
+// the half-row and row mirrors: each a VALU operand modifier, no LDS round trip), beyond that rows and halves change places
 template <int CTRL>
 __device__ __forceinline__ float dpp_get(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -145,8 +146,9 @@ __device__ __forceinline__ float group_sum(float v) {
   if constexpr (LPR >= 4) v += dpp_get<0x4E>(v);    // quad_perm [2,3,0,1]
   if constexpr (LPR >= 8) v += dpp_get<0x141>(v);   // row_half_mirror: lane i <-> 7 - i of each 8
   if constexpr (LPR >= 16) v += dpp_get<0x140>(v);  // row_mirror: lane i <-> 15 - i of each 16
-#pragma unroll
-  for (int o = 16; o < LPR; o <<= 1) v += __shfl_xor(v, o, 64);
+  auto add = [](float a, float b) { return a + b; };
+  if constexpr (LPR >= 32) v = vmi_lanes::across16(v, add);
+  if constexpr (LPR >= 64) v = vmi_lanes::across32(v, add);
   return v;
 }
 
@@ -490,9 +492,7 @@ __device__ __forceinline__ float sk_value(uint32_t key) {
   return (float)__builtin_bit_cast(h16, b);
 }
 __device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return vmi_lanes::over_lanes<64>(v, [](int a, int b) { return a + b; });
 }
 
 // The row sits in registers as packed 16-bit value keys, eight consecutive elements (one 16-byte load from the first aligned

@@ -23,8 +23,7 @@ __device__ __forceinline__ void need(const T& v) {
 
 // sum over 32 lanes
 __device__ __forceinline__ float half_wave_sum(float v) {
-  v = group_sum<16>(v);
-  return v + __shfl_xor(v, 16, 64);
+  return group_sum<32>(v);
 }
 
 // where a wave's weight tiles lie: k-step t of a slab is `step` halves behind k-step 0 (packed tiles, or rows as stored)

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lane_ops.hpp"
 #include "vmi_hybrid.h"
 
 namespace vmi_hybrid {
@@ -99,11 +100,7 @@ __device__ __forceinline__ void need(const V& v) {
   asm volatile("" ::"s"(v));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return vmi_lanes::sum_over<64>(v); }
 
 // ---- host ------------------------------------------------------------------------------------------------------------------
 int fail(int code, const char* who, const char* what);

@@ -193,11 +193,7 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void norm_rows_kernel(const vmi_hy
   if (slab >= SL) return;
   const int nks = FULL ? RW * J : p.K >> 5, per = FULL ? J : (nks + RW - 1) / RW, k0 = wave * per, nk = FULL ? J : min(per, nks - k0);
   auto step = [&](int j) { return FULL ? k0 + j : min(k0 + min(j, per - 1), nks - 1); };
-  auto row_sum = [](float v) {
-#pragma unroll
-    for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-  };
+  auto row_sum = [](float v) { return vmi_lanes::sum_over<LPR>(v); };
   const int units = nks * 8, l = lane % LPR, xr = (wave * 64 + lane) / LPR, mm = min((int)blockIdx.y * 16 + xr, p.M - 1);
   // (what lies past a row, or past a wave's last k-step, is that last one again and meets nothing: no lane-wise condition around a load)
   auto unit = [&](int i) { return (FULL ? l + LPR * i : min(l + LPR * i, units - 1)) * 4; };

@@ -89,8 +89,7 @@ __global__ __launch_bounds__(512) void combine_kernel(const Combine p) {
       l[j] = there ? ml[j][1] : 0.f;
       top = fmaxf(top, m[j]);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+    top = vmi_lanes::max_over<64>(top);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       m[j] = l[j] > 0.f ? exp2_hw(m[j] - top) : 0.f;   // (a part without keys holds no values)

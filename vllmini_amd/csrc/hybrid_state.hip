@@ -235,8 +235,7 @@ __global__ __launch_bounds__(256) void state_prep_kernel(const vmi_hy_state_args
       for (int c = 8 * l16; c < dim; c += 128)
 #pragma unroll
         for (int x = 0; x < 8; ++x) a = fmaf(q[c + x], q[c + x], a), b = fmaf(k[c + x], k[c + x], b);
-#pragma unroll
-      for (int o = 8; o > 0; o >>= 1) a += __shfl_xor(a, o, 64), b += __shfl_xor(b, o, 64);
+      a = vmi_lanes::sum_over<16>(a), b = vmi_lanes::sum_over<16>(b);
       a = 1.f / sqrtf((a + 1e-6f) * (float)p.dim_n);
       b = 1.f / sqrtf(b + 1e-6f);
       for (int c = 8 * l16; c < dim; c += 128)
@@ -252,8 +251,7 @@ __global__ __launch_bounds__(256) void state_prep_kernel(const vmi_hy_state_args
       dl[c] = exp_hw(G);
       deepest = fminf(deepest, G);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) deepest = fminf(deepest, __shfl_xor(deepest, o, 64));
+    deepest = vmi_lanes::over_lanes<64>(deepest, [](float a, float b) { return fminf(a, b); });
     if (lane == 0) most[wave] = deepest;
     __syncthreads();
     const bool little = fminf(fminf(most[0], most[1]), fminf(most[2], most[3])) >= -LITTLE_DECAY;
@@ -589,8 +587,7 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const vmi_hy_state_
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss = fmaf(v[e], v[e], ss);
   }
-#pragma unroll
-  for (int m = 8; m > 0; m >>= 1) ss += __shfl_xor(ss, m, 64);
+  ss = vmi_lanes::sum_over<16>(ss);
   const float r = 1.f / sqrtf(ss / (float)p.vdim_n + p.eps);
   for (int k = l * 4; k < vdim; k += 64) {
     const f32x4 v = *reinterpret_cast<const f32x4*>(o + k);

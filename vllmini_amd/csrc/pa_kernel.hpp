@@ -20,6 +20,8 @@
 #include <float.h>
 #include <type_traits>
 
+#include "lane_ops.hpp"
+
 namespace vmi {
 
 typedef _Float16 h16;
@@ -238,25 +240,10 @@ struct PV8 {
   }
 };
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-  return v;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-  return v;
-}
-
+__device__ __forceinline__ float wave_max(float v) { return vmi_lanes::max_over<64>(v); }
+__device__ __forceinline__ float wave_sum(float v) { return vmi_lanes::sum_over<64>(v); }
 __device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const int o = __shfl_xor(v, m);
-    v = v > o ? v : o;
-  }
-  return v;
+  return vmi_lanes::over_lanes<64>(v, [](int a, int b) { return a > b ? a : b; });
 }
 
 // Batch statistics that every wave of a launch computes for itself from the same seq_lens (clamped to [0, lpad]), in
@@ -927,8 +914,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
               float acc = accv[0];
   #pragma unroll
               for (int i = 1; i < NL; ++i) acc += accv[i];
-  #pragma unroll
-              for (int m = BS; m < 64; m <<= 1) acc += __shfl_xor(acc, m);  // lanes holding the same token
+              acc = vmi_lanes::sum_above<BS>(acc);  // lanes holding the same token
               float qk = p.scale * acc;
               qk += (slope[hh] != 0.f) ? slope[hh] * (float)(token - L + 1) : 0.f;
               if (lane < BS) logits0[hh * p.lpad + token - tok_lo] = masked ? 0.f : qk;
@@ -993,8 +979,8 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
     }
 
     if constexpr (QK_MFMA) {  // per-head maxima live in lanes (lane & 15) = head: fold the 4 row groups, then hand out
-      qmaxB = fmaxf(qmaxB, __shfl_xor(qmaxB, 16));
-      qmaxB = fmaxf(qmaxB, __shfl_xor(qmaxB, 32));
+      auto larger = [](float a, float b) { return fmaxf(a, b); };
+      qmaxB = vmi_lanes::across32(vmi_lanes::across16(qmaxB, larger), larger);
   #pragma unroll
       for (int hh = 0; hh < HPT; ++hh) qk_max[hh] = __shfl(qmaxB, hh);
     }
@@ -1294,10 +1280,7 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
 #pragma unroll
     for (int hh = 0; hh < HPT; ++hh) {
 #pragma unroll
-      for (int i = 0; i < NL; ++i) {
-#pragma unroll
-        for (int m = 1; m < UPR; m <<= 1) acc[hh][i] += __shfl_xor(acc[hh][i], m);
-      }
+      for (int i = 0; i < NL; ++i) acc[hh][i] = vmi_lanes::sum_quad<UPR>(acc[hh][i]);
     }
   }
 

@@ -466,8 +466,7 @@ __global__ void __launch_bounds__(256, (US >= 4 || (UQ >= 4 && !F8) || D > 64) ?
             acc = accv[0];
 #pragma unroll
             for (int i = 1; i < NL; ++i) acc += accv[i];
-            acc += __shfl_xor(acc, 16);
-            acc += __shfl_xor(acc, 32);
+            acc = vmi_lanes::sum_above<16>(acc);
           }
           float qk = p.scale * acc;
           qk += (slope != 0.f) ? slope * (float)(token - L + 1) : 0.f;
@@ -707,9 +706,7 @@ __global__ void __launch_bounds__(256, (US >= 4 || (UQ >= 4 && !F8) || D > 64) ?
 
       // the two lanes of a row hold its 8-token groups
 #pragma unroll
-      for (int i = 0; i < NL; ++i)
-#pragma unroll
-        for (int mm = 1; mm < UPR; mm <<= 1) acc[i] += __shfl_xor(acc[i], mm);
+      for (int i = 0; i < NL; ++i) acc[i] = vmi_lanes::sum_quad<UPR>(acc[i]);
       if constexpr (TEAM) {
         if (hf == 0) {
 #pragma unroll

@@ -283,8 +283,7 @@ __global__ void __launch_bounds__(256, split_wgs_per_cu(D, HPT, ROUNDS)) pa_spli
               float a = accv[0];
 #pragma unroll
               for (int i = 1; i < NL; ++i) a += accv[i];
-              a += __shfl_xor(a, 16);
-              a += __shfl_xor(a, 32);
+              a = vmi_lanes::sum_above<16>(a);
               float qk = p.scale * a;
               qk += (slope[hh] != 0.f) ? slope[hh] * (float)(token - L + 1) : 0.f;
               if (lane < BS) lg0[hh * wtok + idx * BS + tk] = masked ? 0.f : qk;
@@ -323,8 +322,8 @@ __global__ void __launch_bounds__(256, split_wgs_per_cu(D, HPT, ROUNDS)) pa_spli
     VMI_SSTAMP(3);
 
     if constexpr (QKM) {  // per-head maxima live in lanes (lane & 15) = head: fold the four row groups, then hand out
-      qmaxB = fmaxf(qmaxB, __shfl_xor(qmaxB, 16));
-      qmaxB = fmaxf(qmaxB, __shfl_xor(qmaxB, 32));
+      auto larger = [](float a, float b) { return fmaxf(a, b); };
+      qmaxB = vmi_lanes::across32(vmi_lanes::across16(qmaxB, larger), larger);
 #pragma unroll
       for (int hh = 0; hh < HPT; ++hh) qk_max[hh] = __shfl(qmaxB, hh);
     }
@@ -466,9 +465,7 @@ __global__ void __launch_bounds__(256, split_wgs_per_cu(D, HPT, ROUNDS)) pa_spli
 #pragma unroll
     for (int hh = 0; hh < HPT; ++hh)
 #pragma unroll
-      for (int i = 0; i < NL; ++i)
-#pragma unroll
-        for (int mm = 1; mm < UPR; mm <<= 1) acc[hh][i] += __shfl_xor(acc[hh][i], mm);  // the 8-token groups of a row held by other lanes
+      for (int i = 0; i < NL; ++i) acc[hh][i] = vmi_lanes::sum_quad<UPR>(acc[hh][i]);  // the 8-token groups of a row held by other lanes
   }
   VMI_SSTAMP(6);
 
