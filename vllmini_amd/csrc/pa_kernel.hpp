@@ -240,6 +240,12 @@ struct PV8 {
   }
 };
 
+// asks for a kernel argument now
+template <class T>
+__device__ __forceinline__ void need(const T& v) {
+  asm volatile("" ::"s"(v));
+}
+
 __device__ __forceinline__ float wave_max(float v) { return vmi_lanes::max_over<64>(v); }
 __device__ __forceinline__ float wave_sum(float v) { return vmi_lanes::sum_over<64>(v); }
 __device__ __forceinline__ int wave_max_i(int v) {
@@ -486,6 +492,10 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hl = wave / WPH;   // head slot
   const int sub = wave % WPH;  // wave within the slot
+  // (several waves per head: a launch is a chain of latencies; left to itself the compiler asks for arguments branch by branch, a trip to memory each)
+  if constexpr (WPH > 1)
+    need(p.out), need(p.q), need(p.kc), need(p.vc), need(p.block_tables), need(p.seq_lens), need(p.alibi), need(p.num_heads), need(p.num_kv_heads), need(p.scale),
+        need(p.max_blocks_per_seq), need(p.q_stride), need(p.kv_block_stride), need(p.kv_head_stride), need(p.lpad), need(p.q_flags);
   int seq = blockIdx.y, ranked_len = -1;
   if constexpr (LONG) {
     if (p.q_flags & QF_LONGEST_FIRST) {
@@ -511,6 +521,31 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   const int blk_lo = PART ? part * PBLK : 0;  // first block of my range (:126-127)
   int bt_sg = 0;  // which 64-entry slice of my blocks is in bt_reg
   int32_t bt_reg = (blk_lo + sub + lane * WPH < p.max_blocks_per_seq) ? bt[blk_lo + sub + lane * WPH] : 0;
+
+  // ---- per head: tile offset inside a block, ALiBi slope, this lane's q chunks (one per K load), asked for beside the table ----
+  const int c4 = lane / BS;  // chunk-within-load
+  const int tk = lane % BS;  // token-within-block
+  const bool tail_ok = (TAIL == 64) || lane < TAIL;  // this lane takes part in the last load of a tile
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  const int qpk = p.num_heads == p.num_kv_heads ? 1 : p.num_heads / p.num_kv_heads;
+  int64_t hoff[HPT];
+  float slope[HPT];
+  u32x4 qreg[HPT][NL][F8 ? 2 : 1];  // the EPU dims of q that face this lane's chunk of each K load
+#pragma unroll
+  for (int hh = 0; hh < HPT; ++hh) {
+    const int head = head0 + (valid(hh) ? hh : 0);
+    hoff[hh] = (int64_t)(qpk == 1 ? head : head / qpk) * p.kv_head_stride + lane * EPU;
+    slope[hh] = p.alibi ? p.alibi[head] : 0.f;
+    const h16* qp = p.q + (int64_t)seq * p.q_stride + (int64_t)head * D;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+#pragma unroll
+      for (int w = 0; w < (F8 ? 2 : 1); ++w)
+        qreg[hh][i][w] = (i < NL - 1 || tail_ok)
+                             ? *reinterpret_cast<const u32x4*>(qp + (CPL * i + c4) * EPU + 8 * w)
+                             : zero4;
+    }
+  }
 
   // seq_len > max_seq_len overflows the logits buffer in the reference (undefined behaviour,
   // attention_kernels.cu:725-732); here the context is truncated to the LDS that was reserved.
@@ -572,12 +607,6 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
   }
   VMI_STAMP(1);
 
-  // ---- per head: tile offset inside a block, ALiBi slope, this lane's q chunks (one per K load) ----
-  const int c4 = lane / BS;  // chunk-within-load
-  const int tk = lane % BS;  // token-within-block
-  const bool tail_ok = (TAIL == 64) || lane < TAIL;  // this lane takes part in the last load of a tile
-  const u32x4 zero4 = {0u, 0u, 0u, 0u};
-  const int qpk = p.num_heads / p.num_kv_heads;
   // SPARSE (attention_kernels.cu:209-254, 385-393): cache block b is attended when the sparse block holding its first
   // token is "remote" — on this head's vertical stripe — or "local" — within local_blocks of the query's sparse block.
   // The attended blocks are listed up front (ablk, below) and the passes walk that list, so the loads in flight are
@@ -594,25 +623,6 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
     const int kb = b * BS / p.bs_block_size;  // :235
     return ((kb + bs_off) % p.bs_vert_stride == 0) || (kb > q_bs - p.bs_local_blocks);
   };
-  int64_t hoff[HPT];
-  float slope[HPT];
-  u32x4 qreg[HPT][NL][F8 ? 2 : 1];  // the EPU dims of q that face this lane's chunk of each K load
-#pragma unroll
-  for (int hh = 0; hh < HPT; ++hh) {
-    const int head = head0 + (valid(hh) ? hh : 0);
-    hoff[hh] = (int64_t)(head / qpk) * p.kv_head_stride + lane * EPU;
-    slope[hh] = p.alibi ? p.alibi[head] : 0.f;
-    const h16* qp = p.q + (int64_t)seq * p.q_stride + (int64_t)head * D;
-#pragma unroll
-    for (int i = 0; i < NL; ++i) {
-#pragma unroll
-      for (int w = 0; w < (F8 ? 2 : 1); ++w)
-        qreg[hh][i][w] = (i < NL - 1 || tail_ok)
-                             ? *reinterpret_cast<const u32x4*>(qp + (CPL * i + c4) * EPU + 8 * w)
-                             : zero4;
-    }
-  }
-
   // ---- fused append (APP): this step's key/value rows, in the lane map of the K / V tiles.  They are patched
   //      into the page registers where the attention meets position Lfull-1; whatever bytes the cache holds there
   //      at that moment (old, or already the writer workgroup's) are never used. ----
@@ -931,6 +941,10 @@ __global__ void __launch_bounds__(HPW* WPH * 64, (UMAX > 0 && WPH == 1) ? 3 : 1)
     // Latency regime (small batches): when everything this wave owns fits ONE register group, the V pages are
     // requested together with the K pages (into the idle second buffer), so K and V cost one memory round trip
     // between them instead of two in a row.
+    // q was asked for beside the table entries, which the first page load waits for.  Said here, on every path: where a path seemed to leave q in flight (a wave
+    // may have no blocks), the compiler waited behind the first barrier, where it takes those registers again, for ALL loads,
+    // and the softmax began when the V pages were there.
+    if constexpr (WPH > 1) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     const bool single = (ngroups == 1);  // wave-uniform (and workgroup-uniform under LOCK)
     if (single) {
       load_group(ra, p.kc, 0);
