@@ -190,6 +190,28 @@ CUTS = [[70], [15, 2, 16, 3, 1, 1, 17, 2, 9], [1] * 5 + [2, 31, 1, 2]]
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("kind,heads,dim,vdim", [("retention", 2, 128, 128), ("delta", 2, 128, 128), ("retention", 1, 300, 96), ("delta", 4, 32, 288)])
+def test_a_token_of_many_states_is_that_of_few(dtype, kind, heads, dim, vdim):
+    """From 1 MiB of states a launch on they go past the caches: the same bits, in outputs and states, as in launches of fewer."""
+    B = 10
+    args = (heads, dim, vdim, 0, (0.9, 0.99, 0.5, 0.7)[:heads]) if kind == "retention" else (heads, 1, dim, vdim, 4)
+    k = (retention_case if kind == "retention" else delta_case)(*args, dtype, slots=B + 1)[0]
+    g = torch.Generator().manual_seed(dim)
+    k.held = [torch.randn(t.shape, generator=g).to(t.dtype).to(dev()) for t in k.held]
+    many, few = [t.clone() for t in k.held], [t.clone() for t in k.held]
+    size = many[0][0].numel() * 4
+    assert many[0].dtype == torch.float32 and B * size >= 1 << 20 > 5 * size
+    inputs, slots, ctx = k.inputs(B, 3)[1], [3, 1, 0, 10, 7, 5, 6, 4, 8, 9], [4, 0, 9, 9, 1, 2, 30, 7, 7, 1]
+    step = lambda at: layout([1] * len(at), [ctx[i] for i in at], [[0]] * len(at), 64, [slots[i] for i in at], [0] * len(at), pos_slots=False)  # noqa: E731
+    k.held = many
+    got = k.run(inputs, step(range(B)))
+    k.held = few
+    want = torch.cat([k.run([t[at.start:at.stop] for t in inputs], step(at)) for at in (range(0, 5), range(5, 10))])
+    assert torch.equal(got, want) and all(torch.equal(a, b) for a, b in zip(many, few))
+    assert not torch.equal(many[0][slots[0]], many[0][2]) and torch.isfinite(got.float()).all()
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("heads,dim,vdim,rot,decay", [(1, 10, 33, 10, (1.0,)), (3, 20, 24, 12, (0.5, 0.01, 0.999)), (2, 64, 160, 36, (0.9, 0.99)),
                                                       (2, 150, 40, 2, (0.7, 0.95)), (1, 300, 96, 300, (0.98,)), (4, 96, 16, 0, (0.0, 0.3, 0.6, 0.9))])
 def test_retention_over_portions_of_every_size(dtype, heads, dim, vdim, rot, decay):

@@ -614,8 +614,12 @@ inline int step_rows(int dim, int slice) {
   return (dim + groups - 1) / groups;
 }
 
-// one token of one (entry, head), a slice of the value columns.  RPT: state rows a thread holds (at most)
-template <typename T, int KIND, int RPT>
+// one token of one (entry, head), a slice of the value columns.  RPT: state rows a thread holds (at most).  FAR: the states go past the caches both ways.  A step
+// reads and writes each once, and until the next step reads it again all layers' weights and states go by: kept, they leave the last cache nothing to
+// hold weights with.  Width 2048, 32 sequences (33 MB of states a launch): this kernel 16.9 -> 14.2 us, and beside it the products of 84 MB 22.2 -> 19.8,
+// the logits' 51.0 -> 44.4; whole answers of 32 sequences 10.66 -> 9.85 ms, of 8 8.33 -> 7.93, of one 7.33 -> 7.21; width 1024, 32 / 4 5.97 / 4.78 -> 5.62 / 4.62.  Only the
+// stores past the caches: 17.2 us, and nothing for the products.
+template <typename T, int KIND, int RPT, bool FAR>
 __global__ __launch_bounds__(256) void state_step_kernel(const vmi_hy_state_args p, const vmi_hy_step s, const int slice) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int dim = p.dim, tid = threadIdx.x, h = blockIdx.x, e = blockIdx.y, c0 = (int)blockIdx.z * slice;
@@ -640,7 +644,10 @@ __global__ __launch_bounds__(256) void state_step_kernel(const vmi_hy_state_args
   for (int i = 0; i < RPT; ++i) {
     const int row = grp + i * groups;
     S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (have && mine && row < dim) S[i] = *reinterpret_cast<const f32x4*>(st + (int64_t)row * p.vdim);
+    if (have && mine && row < dim) {
+      const f32x4* at = reinterpret_cast<const f32x4*>(st + (int64_t)row * p.vdim);
+      S[i] = FAR ? __builtin_nontemporal_load(at) : *at;
+    }
   }
   float beta = 1.f;
   if constexpr (KIND == VMI_HY_DELTA) {
@@ -720,7 +727,9 @@ __global__ __launch_bounds__(256) void state_step_kernel(const vmi_hy_state_args
         S[i][x] = fmaf(k, u[x], S[i][x]);
         part[x] = fmaf(S[i][x], q, part[x]);
       }
-      *reinterpret_cast<f32x4*>(st + (int64_t)row * p.vdim) = S[i];
+      f32x4* to = reinterpret_cast<f32x4*>(st + (int64_t)row * p.vdim);
+      if constexpr (FAR) __builtin_nontemporal_store(S[i], to);
+      else *to = S[i];
     }
   }
   const float o = gather(part);
@@ -743,18 +752,25 @@ static void launch_norm_gate(const vmi_hy_state_args& p, const vmi_hy_step& s, h
   hipLaunchKernelGGL(head_norm_gate_kernel<T>, dim3(((int64_t)s.T * p.heads + 15) / 16), dim3(256), 0, st, p, s);
 }
 
-template <typename T, int KIND>
-static int run_step(const vmi_hy_state_args& p, const vmi_hy_step& s, hipStream_t st) {
+template <typename T, int KIND, bool FAR>
+static int run_step_of(const vmi_hy_state_args& p, const vmi_hy_step& s, hipStream_t st) {
   const int slice = step_slice(p.dim, p.vdim), rows = step_rows(p.dim, slice);
   const dim3 grid(p.heads, s.B, (p.vdim + slice - 1) / slice);
   const size_t lds = (size_t)(3 * p.dim + 2 * slice + 1024 + 8) * sizeof(float);
-  if (rows <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 4>), grid, dim3(256), lds, st, p, s, slice);
-  else if (rows <= 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 8>), grid, dim3(256), lds, st, p, s, slice);
-  else if (rows <= 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 16>), grid, dim3(256), lds, st, p, s, slice);
-  else if (rows <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 32>), grid, dim3(256), lds, st, p, s, slice);
+  if (rows <= 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 4, FAR>), grid, dim3(256), lds, st, p, s, slice);
+  else if (rows <= 8) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 8, FAR>), grid, dim3(256), lds, st, p, s, slice);
+  else if (rows <= 16) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 16, FAR>), grid, dim3(256), lds, st, p, s, slice);
+  else if (rows <= 32) hipLaunchKernelGGL(HIP_KERNEL_NAME(state_step_kernel<T, KIND, 32, FAR>), grid, dim3(256), lds, st, p, s, slice);
   else return fail(VMI_HY_E_SHAPE, "vmi_hy_state", "heads this large are not built");
   if (slice < p.vdim) launch_norm_gate<T>(p, s, st);
   return launched("vmi_hy_state");
+}
+
+// Past the caches from 1 MiB of states a launch on.  All kernels of a step, 8 layers, kept / past the caches, us: width 512 (165 MB of weights: everything stays in the last cache), 1 sequence (0.25 MiB a launch)
+// 3731 / 3760, 4 (1) 3870 / 3887, 16 (4) 4044 / 4013, 32 4275 / 4205, 64 5980 / 5520; width 1024, 2 (1 MiB) 4622 / 4582; width 2048, 1 (1 MiB) 7331 / 7213.
+template <typename T, int KIND>
+static int run_step(const vmi_hy_state_args& p, const vmi_hy_step& s, hipStream_t st) {
+  return (int64_t)s.B * p.heads * p.dim * p.vdim * 4 >= 1 << 20 ? run_step_of<T, KIND, true>(p, s, st) : run_step_of<T, KIND, false>(p, s, st);
 }
 
 template <int KIND, int NT>
