@@ -111,70 +111,98 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
 // Rows of the element type over many columns, 16 MT of them: eight waves hold an eighth of K of all rows each, in registers and in the matrix cores' layout,
 // and the workgroup walks over slabs of 16 columns, blockIdx, blockIdx + grid, ..; the ring of weight tiles runs on across slabs.  NCH chunks of 4 k-steps are a
 // wave's part of a slab, NB chunks are in registers.  A slab's partial tiles meet in LDS (two places, one barrier a slab); another wave each time adds a
-// tile's in the order of K and stores.
+// tile's in the order of K and stores.  Nothing in the walk depends on a condition but its end and the stores: the compiler counts loads
+// in flight, and where paths meet that differ in them it waits for all.  With sizes and ends it could not see, the ring ran empty every three slabs.  Norm and
+// product, us, before -> without conditions: K 2048, N 12288 9 / 32 / 47 rows 15.5 / 18.0 / 19.0 -> 14.2 / 16.7 / 17.2, N 20480 20.8 / 23.2 / 25.6 -> 19.4 / 22.3 / 24.1, N 6144 32
+// rows 13.9 -> 12.5; K 3072, N 6144 47 rows 17.6 -> 15.6; K 1024, N 24576 18.5 -> 16.7.  (84 MB alone, nothing computed: 15.2.)
 constexpr size_t HELD_LDS = 2 * 8 * 1024;   // ... a row tile
 
 template <int NCH, int MT, int NB, int EPI>
 __global__ __launch_bounds__(512, 2) void held_rows_kernel(const vmi_hy_linear_args p, const int slabs) {
-  constexpr int W = 8, CS = 4;
+  constexpr int W = 8, CS = 4, KS = NCH * CS, NKS = W * KS;   // k-steps of a wave, of a slab: K = 1024 NCH
   static_assert(NB % NCH == 0, "a chunk's place in its slab follows from its place in the ring");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [2][W][MT][1024]
   need_args<EPI>(p), need(slabs);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int m0 = blockIdx.y * 16 * MT, nks = p.K >> 5, kpw = (nks + W - 1) / W, k0 = wave * kpw, nk = min(kpw, nks - k0);
+  const int m0 = blockIdx.y * 16 * MT, k0 = wave * KS;
   if ((int)blockIdx.x >= slabs) return;
-  b16x8 x[NCH * CS][MT], wb[NB][CS];
+  b16x8 x[KS][MT], wb[NB][CS];
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) {
-    const b16* row = static_cast<const b16*>(p.x) + (int64_t)min(m0 + mi * 16 + r16, p.M - 1) * p.ldx + 8 * kc;
+    const b16* row = static_cast<const b16*>(p.x) + (int64_t)min(m0 + mi * 16 + r16, p.M - 1) * p.ldx + 8 * kc + 32 * k0;
 #pragma unroll
-    for (int j = 0; j < NCH * CS; ++j) x[j][mi] = load8(row + 32 * min(k0 + min(j, kpw - 1), nks - 1));
+    for (int j = 0; j < KS; ++j) x[j][mi] = load8(row + 32 * j);
   }
-  const b16* wp = static_cast<const b16*>(p.w) + lane * 8;
+  __builtin_amdgcn_sched_barrier(0);   // (requests in the order of their use, also where the compiler would turn them round: they complete in order)
   int ls = blockIdx.x;   // the slab to load from next
   auto load_w = [&](b16x8(&dst)[CS], int c) {
-    const b16* at = wp + (int64_t)ls * nks * 512;
+    // (past the last slab: 16 bytes of it for all lanes, which meet nothing; a condition around a load makes every wait a wait for all)
+    const bool past = ls >= slabs;
+    const b16* at = static_cast<const b16*>(p.w) + ((int64_t)(past ? (int)blockIdx.x : ls) * NKS + k0 + c * CS) * 512 + (past ? 0 : lane * 8);
 #pragma unroll
-    for (int j = 0; j < CS; ++j) dst[j] = load8(at + (int64_t)min(k0 + min(c * CS + j, kpw - 1), nks - 1) * 512);
-    if (c == NCH - 1 && ls + (int)gridDim.x < slabs) ls += gridDim.x;   // (past the last: that one again, a cache hit)
+    for (int j = 0; j < CS; ++j) dst[j] = load8(at + j * 512);
+    __builtin_amdgcn_sched_barrier(0);
+    if (c == NCH - 1) ls += gridDim.x;
   };
 #pragma unroll
   for (int b = 0; b < NB - 1; ++b) load_w(wb[b], b % NCH);
-  f32x4 acc[MT];
-#pragma unroll
-  for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int total = (slabs - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * NCH;
   int i = 0, slab = blockIdx.x;
-  for (int t = 0; t < total; t += NB) {
+  // a slab whose first chunk is in place B0 of the ring; more: its chunks' successors are asked for
+  auto walk = [&](auto b0, bool more) {
+    constexpr int B0 = decltype(b0)::value;
+    f32x4 acc[MT];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (t + b >= total) break;
-      load_w(wb[(b + NB - 1) % NB], (b + NB - 1) % NCH);
+    for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (more) load_w(wb[(B0 + c + NB - 1) % NB], (c + NB - 1) % NCH);
 #pragma unroll
       for (int j = 0; j < CS; ++j)
-        if (b % NCH * CS + j < nk) {   // (scalar)
 #pragma unroll
-          for (int mi = 0; mi < MT; ++mi) mma(acc[mi], wb[b][j], x[b % NCH * CS + j][mi]);
-        }
-      if (b % NCH < NCH - 1) continue;
-      unsigned char* to = smem + (i & 1) * W * MT * 1024;
-#pragma unroll
-      for (int mi = 0; mi < MT; ++mi) {
-        *reinterpret_cast<f32x4*>(to + (wave * MT + mi) * 1024 + lane * 16) = acc[mi];
-        acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      __syncthreads();   // (two places: who still adds up slab i has not passed the barrier of slab i + 1)
-      const int mi = (wave - i * MT) & (W - 1);
-      if (mi < MT) {
-        f32x4 sum = *reinterpret_cast<const f32x4*>(to + mi * 1024 + lane * 16);
-#pragma unroll
-        for (int v = 1; v < W; ++v) sum += *reinterpret_cast<const f32x4*>(to + (v * MT + mi) * 1024 + lane * 16);
-        const int m = m0 + mi * 16 + r16;
-        if (m < p.M) epilogue<b16, EPI>(p, sum, m, slab * 16 + 4 * kc, slab * 16, 0);
-      }
-      ++i;
-      slab += gridDim.x;
+        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], wb[B0 + c][j], x[c * CS + j][mi]);
     }
+    unsigned char* to = smem + (i & 1) * W * MT * 1024;
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) *reinterpret_cast<f32x4*>(to + (wave * MT + mi) * 1024 + lane * 16) = acc[mi];
+    __syncthreads();   // (two places: who still adds up slab i has not passed the barrier of slab i + 1)
+    const int mi = (wave - i * MT) & (W - 1);
+    if (mi < MT) {
+      f32x4 sum = *reinterpret_cast<const f32x4*>(to + mi * 1024 + lane * 16);
+#pragma unroll
+      for (int v = 1; v < W; ++v) sum += *reinterpret_cast<const f32x4*>(to + (v * MT + mi) * 1024 + lane * 16);
+      const int m = m0 + mi * 16 + r16;
+      if (m < p.M) epilogue<b16, EPI>(p, sum, m, slab * 16 + 4 * kc, slab * 16, 0);
+    }
+    ++i;
+    slab += gridDim.x;
+  };
+  // Whole rounds of the ring, then what is left, which the ring holds.  One way out of the loop: any other joins the way back in the compiler's eyes
+  // (a return as well), and then the places of the ring are in an unknown order and a third of the waits are waits for all.
+  constexpr int ROUND = NB / NCH;
+  static_assert((ROUND <= 3 || ROUND == 6) && (ROUND - 1) * NCH <= NB - 1, "the slabs behind the last round are in the ring");
+  for (; slab + (ROUND - 1) * (int)gridDim.x < slabs;) {
+    walk(std::integral_constant<int, 0>{}, true);
+    if constexpr (ROUND > 1) walk(std::integral_constant<int, NCH % NB>{}, true);
+    if constexpr (ROUND > 2) walk(std::integral_constant<int, 2 * NCH % NB>{}, true);
+    if constexpr (ROUND > 3) walk(std::integral_constant<int, 3 * NCH % NB>{}, true);
+    if constexpr (ROUND > 4) walk(std::integral_constant<int, 4 * NCH % NB>{}, true);
+    if constexpr (ROUND > 5) walk(std::integral_constant<int, 5 * NCH % NB>{}, true);
+  }
+  if constexpr (ROUND > 1) {
+    if (slab >= slabs) return;
+    walk(std::integral_constant<int, 0>{}, false);
+  }
+  if constexpr (ROUND > 2) {
+    if (slab >= slabs) return;
+    walk(std::integral_constant<int, NCH % NB>{}, false);
+  }
+  if constexpr (ROUND > 3) {
+    if (slab >= slabs) return;
+    walk(std::integral_constant<int, 2 * NCH % NB>{}, false);
+    if (slab >= slabs) return;
+    walk(std::integral_constant<int, 3 * NCH % NB>{}, false);
+    if (slab >= slabs) return;
+    walk(std::integral_constant<int, 4 * NCH % NB>{}, false);
   }
 }
 
