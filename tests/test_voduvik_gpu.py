@@ -226,6 +226,14 @@ def test_rows_normed_once_are_held_in_registers(M, N, K):
     assert ops.linear_normed_first(M, _norm_products(M, ops.pad32(N), K))
 
 
+@pytest.mark.parametrize("M,K,wgs,slabs", [(3, 1024, 512, (4, 5, 6, 7, 8)), (16, 2048, 256, (3, 4, 5, 6)), (5, 2048, 512, (2, 3, 4)), (1, 4096, 512, (1, 2)), (20, 1024, 512, (2, 4, 5, 6, 7)),
+                                           (32, 2048, 256, (2, 3, 4, 5)), (50, 1024, 128, (4, 5, 6, 7, 8, 9)), (40, 3072, 128, (1, 2, 3, 4))])
+def test_every_number_of_slabs_behind_the_rings_last_round(M, K, wgs, slabs):
+    """resident_kernel and held_rows_kernel over whole chunks of K: `slabs` of a workgroup's are all that the longest walks have, one workgroup's; the others' are one less."""
+    for n in slabs:
+        _norm_products(M, 16 * (wgs * (n - 1) + 2), K)
+
+
 @pytest.mark.parametrize("M", [1, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(48, 32), (16 * 130, 128), (32, 224), (16 * 133, 480), (16 * 131, 992), (64, 1024), (16 * 129, 2016), (32, 2080), (96, 3072), (32, 4064), (48, 4576), (32, 4640),
                                  (16 * 130, 4640), (48, 9248), (16 * 386, 96), (16 * 258, 1056), (16 * 514, 2080), (16 * 386, 8224)])

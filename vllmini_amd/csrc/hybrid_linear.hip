@@ -243,9 +243,15 @@ __global__ __launch_bounds__(NW* KS * 64) void linear_kernel(const vmi_hy_linear
 // weights.  One row, K 4096: N 24576 57.4 -> 37.1 us (5.4 TB/s), N 8192 25.6 -> 17.1; K 1024: N 6144 10.1 -> 7.7, N 50272 30.6 -> 22.0; 16 rows, K 4096,
 // N 24576 67.6 -> 46.6; 32 rows, K 2048: N 22528 40.4 -> 29.9, N 50272 85.8 -> 51.9.  (Non-temporal loads of the weights: 36.5, but 77 against 74 us
 // for 412 MB and slower wherever they stay in the Infinity Cache.  16 waves a workgroup where there is one slab a compute unit: 9.9 -> 11.3.)
-template <int MT, int W, int PL, int CU, int EPI>
+// NCH > 0: rows of 1024 NCH columns, NCH whole chunks a wave.  Then nothing in the walk depends on a condition but its end and the stores: the compiler counts loads in
+// flight, and where paths meet that differ in them it waits for all of them, every NB chunks.  General form -> this one, weights not in the Infinity Cache, us: K 4096, N 4096 1 / 4 / 8
+// rows 11.1 / 12.5 / 14.8 -> 8.8 / 11.0 / 13.1, N 8192 16.7 / 17.8 / 21.2 -> 14.5 / 16.8 / 20.1, N 24576 38.5 / 39.0 / 43.1 -> 37.1 / 38.4 / 41.9, N 50272 72.9 -> 71.8; K 2048, N 12288 1 / 16 rows 13.8 / 15.4 -> 11.8 /
+// 14.4, N 50272 40.3 / 44.8 -> 37.8 / 43.3; K 1024, N 50272 22.3 / 23.1 -> 20.6 / 22.0.  (201 and 412 MB alone, nothing computed: 34.5 and 70.)
+template <int MT, int W, int PL, int CU, int EPI, int NCH = 0>
 __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_linear_args p, const int slabs) {
   constexpr int CS = 4, NB = CU > 1 ? 4 : 6;   // k-steps of a chunk, chunks of weights in registers (NB - 1 of them ahead)
+  constexpr int KS = NCH * CS;                 // k-steps of a wave
+  if constexpr (NCH > 0) need(p.x), need(p.ldx), need(p.rows), need(p.norm_w), need(p.norm_n), need(p.rms), need(p.eps), need(p.w), need(p.y), need(p.ldy), need(p.M), need(p.N), need(p.K);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int LD = p.K + 8, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
   f32x4* red = reinterpret_cast<f32x4*>(smem);                         // [PL][W - 1][MT][64]
@@ -257,6 +263,16 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
   b16x8 wb[NB][CS];
   const b16* wp = static_cast<const b16*>(p.w) + lane * 8;
   int ls = blockIdx.x, lc = 0;   // the chunk to load next: slab and chunk of it
+  // whole chunks: chunk c of slab ls.  Past the last slab 16 bytes of one for all lanes, which meet nothing; requests stay in the order of their use
+  [[maybe_unused]] auto load_whole = [&](b16x8(&dst)[CS], int c) {
+    const bool past = ls >= slabs;
+    const b16* at = static_cast<const b16*>(p.w) + ((int64_t)(past ? (int)blockIdx.x : ls) * (W * KS) + wave * KS + c * CS) * 512 + (past ? 0 : lane * 8);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < CS; ++j) dst[j] = load8(at + j * 512);
+    __builtin_amdgcn_sched_barrier(0);
+    if (c == NCH - 1) ls += gridDim.x;
+  };
   auto load_w = [&](b16x8(&dst)[CS]) {
     const b16* at = wp + (int64_t)ls * nks * 512;
 #pragma unroll
@@ -277,7 +293,10 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
   const int rounds = (M + rpp - 1) / rpp;
   auto open_ring = [&]() {
 #pragma unroll
-    for (int b = 0; b < NB - 1; ++b) load_w(wb[b]);
+    for (int b = 0; b < NB - 1; ++b) {
+      if constexpr (NCH > 0) load_whole(wb[b], b % NCH);
+      else load_w(wb[b]);
+    }
   };
   {
     constexpr int HOLD = CU > 1 ? 2 : 4;   // units of 8 columns a lane keeps; longer shares are read again
@@ -296,7 +315,7 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
 #pragma unroll
     for (int i = 0; i < HOLD; ++i) w[i] = load8(p.norm_w + min(u0 + i * step8, upr - 1) * 8);
     open_ring();   // (behind the first loads of x, so that waiting for those leaves the weights in flight)
-    for (int round = 0; round < rounds; ++round) {
+    auto one_round = [&](int round) {
       float s = 0.f, q = 0.f;
       auto sums = [&](const f32x8& x, int u) {
 #pragma unroll
@@ -332,7 +351,15 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
       for (int i = 0; i < HOLD; ++i)
         if (u0 + i * step8 < upr) put(v[i], w[i], u0 + i * step8);
       for (int u = u0 + HOLD * step8; u < upr; u += step8) put(load8(row + u * 8), load8(p.norm_w + u * 8), u);
-      if (round + 1 < rounds) fetch(round + 1);
+    };
+    // (by itself: with the following ones, whose rows come behind the weights, it would wait for those; and what came in front of the weights is there, whichever lanes use it)
+    constexpr int RING = (NB - 1) * CS;
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (RING & 15) | (RING >> 4 << 14));   // vmcnt(RING)
+    one_round(0);
+    for (int round = 1; round < rounds; ++round) {
+      fetch(round);
+      one_round(round);
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
     }
   }
   __syncthreads();
@@ -344,17 +371,7 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
   int slab = blockIdx.x, c = 0, i = 0;   // of the chunk to multiply next; slabs done
-  auto step = [&](b16x8(&cur)[CS], b16x8(&nxt)[CS]) {
-    load_w(nxt);
-#pragma unroll
-    for (int j = 0; j < CS; ++j) {
-      const int kk = c * CS + j, k = wave * kpw + kk;
-      if (kk < kpw && k < nks) {   // (scalar)
-#pragma unroll
-        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], load8(xa[mi] + k * 32));
-      }
-    }
-    if (++c < nch) return;
+  auto meet = [&]() {   // a slab's partial tiles
     f32x4* to = red + (PL > 1 ? (i & 1) * (W - 1) * MT * 64 : 0);
     const int behind = (wave - i) & (W - 1);   // 0: the wave that adds up; the others' places in their order behind it
 #pragma unroll
@@ -371,14 +388,64 @@ __global__ __launch_bounds__(64 * W, 2 * CU) void resident_kernel(const vmi_hy_l
       acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     if constexpr (PL == 1) __syncthreads();
-    c = 0;
     ++i;
     slab += gridDim.x;
   };
-  for (int t = 0; t < total; t += NB) {
+  [[maybe_unused]] auto step = [&](b16x8(&cur)[CS], b16x8(&nxt)[CS]) {
+    load_w(nxt);
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      if (t + b < total) step(wb[b], wb[(b + NB - 1) % NB]);
+    for (int j = 0; j < CS; ++j) {
+      const int kk = c * CS + j, k = wave * kpw + kk;
+      if (kk < kpw && k < nks) {   // (scalar)
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], load8(xa[mi] + k * 32));
+      }
+    }
+    if (++c < nch) return;
+    meet();
+    c = 0;
+  };
+  if constexpr (NCH == 0) {
+    for (int t = 0; t < total; t += NB) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        if (t + b < total) step(wb[b], wb[(b + NB - 1) % NB]);
+    }
+  } else {
+    // a slab whose first chunk is in place B0 of the ring; more: its chunks' successors are asked for
+    auto walk = [&](auto b0, bool more) {
+      constexpr int B0 = decltype(b0)::value;
+#pragma unroll
+      for (int n = 0; n < NCH; ++n) {
+        if (more) load_whole(wb[(B0 + n + NB - 1) % NB], (n + NB - 1) % NCH);
+#pragma unroll
+        for (int j = 0; j < CS; ++j)
+#pragma unroll
+          for (int mi = 0; mi < MT; ++mi) mma(acc[mi], wb[B0 + n][j], load8(xa[mi] + (wave * KS + n * CS + j) * 32));
+      }
+      meet();
+    };
+    constexpr int ROUND = NB / NCH;   // slabs the ring goes round in
+    static_assert(NB % NCH == 0 && ROUND <= 4, "a chunk's place in its slab follows from its place in the ring");
+    // whole rounds, then what is left, which the ring holds; one way out of the loop, since any other joins the way back in the compiler's eyes
+    for (; slab + (ROUND - 1) * (int)gridDim.x < slabs;) {
+      walk(std::integral_constant<int, 0>{}, true);
+      if constexpr (ROUND > 1) walk(std::integral_constant<int, NCH % NB>{}, true);
+      if constexpr (ROUND > 2) walk(std::integral_constant<int, 2 * NCH % NB>{}, true);
+      if constexpr (ROUND > 3) walk(std::integral_constant<int, 3 * NCH % NB>{}, true);
+    }
+    if constexpr (ROUND > 1) {
+      if (slab >= slabs) return;
+      walk(std::integral_constant<int, 0>{}, false);
+    }
+    if constexpr (ROUND > 2) {
+      if (slab >= slabs) return;
+      walk(std::integral_constant<int, NCH % NB>{}, false);
+    }
+    if constexpr (ROUND > 3) {
+      if (slab >= slabs) return;
+      walk(std::integral_constant<int, 2 * NCH % NB>{}, false);
+    }
   }
 }
 
@@ -411,6 +478,13 @@ static bool resident_pays(int M, int N, int K) {
 template <int MT, int W, int PL, int CU, int EPI>   // CU workgroups a compute unit
 static int launch_resident(const vmi_hy_linear_args& p, hipStream_t st) {
   auto* fn = resident_kernel<MT, W, PL, CU, EPI>;
+  if constexpr (CU == 2) {   // (longer rows of 17 and more do not leave room for two workgroups)
+    if (p.K == 1024) fn = resident_kernel<MT, W, PL, CU, EPI, 1>;
+    if constexpr (MT == 1) {
+      if (p.K == 2048) fn = resident_kernel<MT, W, PL, CU, EPI, 2>;
+      if (p.K == 4096) fn = resident_kernel<MT, W, PL, CU, EPI, 4>;
+    }
+  }
   const size_t lds = resident_lds(p.M, p.K, W, PL);
   if (int rc = allow_lds(fn, lds, "vmi_hy_linear")) return rc;
   const int slabs = p.N / 16;
