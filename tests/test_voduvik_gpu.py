@@ -252,6 +252,23 @@ def test_few_rows_as_they_are(M, N, K):
     close(ops.linear(x, t, residual=True, out=base.clone()), base.double() + y, torch.bfloat16, tol16=1e-3)
 
 
+@pytest.mark.parametrize("K", [6144, 8192, 12288])
+@pytest.mark.parametrize("M,slabs", [(1, 3), (2, 512), (3, 130), (8, 514), (9, 66), (16, 384), (17, 96), (32, 128), (50, 6)])
+def test_rows_as_they_are_over_whole_chunks(M, slabs, K):
+    """plain_rows_kernel's form for waves of whole chunks, with requests for two, eight and sixteen rows, and linear_kernel past its line; gated by a column as well."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M * K + slabs)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    N = 16 * slabs
+    w = (rnd(ops.pad32(N), K) / K ** 0.5).to(torch.bfloat16)
+    t, x, bias, base, gate = ops.MatrixTiles(w, torch.bfloat16), rnd(M, K + 8).to(torch.bfloat16)[:, :K], rnd(len(w)), rnd(M, len(w)), rnd(M, 1).to(torch.bfloat16)
+    y = x.double() @ w.double().T
+    close(ops.linear(x, t, bias=bias), y + bias, torch.bfloat16)
+    close(ops.linear(x, t, residual=True, out=base.clone()), base.double() + y, torch.bfloat16, tol16=1e-3)
+    close(ops.linear(x, t, gate=gate), y * torch.sigmoid(gate.double()), torch.bfloat16)
+
+
 def _norm_products(M, N, K):
     """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
     from vllmini_amd import hybrid_ops as ops

@@ -23,7 +23,11 @@ constexpr int plain_stride(int J, int MT) { return MT * 16 * (64 * J + 16); }   
 // Rows as they are.  A workgroup owns 16 columns of 16 MT rows of a group; a wave brings its own part of K of the rows through its own part of the
 // LDS, chunks of J k-steps, so nothing but the sum at the end waits for another wave.  NB chunks of weights in registers.  The order of the requests is the
 // order of their use (they complete in order): rows of a chunk, then the weights NB - 1 chunks on.  NB = 1: a wave's part is one chunk.
-template <int RW, int J, int MT, int NB, int EPI>
+// NCH > 0: NCH whole chunks a wave, K = 32 RW J NCH, all of whose requests are written out, NB chunks of rows and of weights on their way: with sizes and ends the compiler could
+// not see it waited for all of them at every chunk.  XI: requests for the rows of a chunk (2 XI rows at most).  Before -> now, weights not in the Infinity Cache, us: K 6144, N 1024 1 / 16 / 32
+// rows 7.9 / 9.7 / 9.4 -> 6.5 / 8.8 / 8.6, N 2048 32 rows 10.2 -> 9.4, N 4096 1 / 16 12.4 / 14.1 -> 11.1 / 13.1; K 8192, N 2048 32 rows 12.5 -> 11.4, N 4096 1 / 16 16.4 / 17.9 -> 14.5 / 16.3; K 12288,
+// N 1024 12.0 / 16.0 -> 11.0 / 14.7, N 4096 21.9 / 23.8 -> 20.3 / 22.6 (101 MB, 5.0 TB/s).
+template <int RW, int J, int MT, int NB, int EPI, int NCH = 0, int XI = J>
 __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_hy_linear_args p) {
   constexpr int LDB = 64 * J + 16, STRIDE = plain_stride(J, MT);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [RW][STRIDE]
@@ -41,58 +45,90 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
 
   const b16* xp = static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride;
   const b16* wp = static_cast<const b16*>(p.w) + (((int64_t)grp * (p.N >> 4) + slab) * nks * 64 + lane) * 8;
-  b16x8 x[MT][J], w[NB][J];
-#pragma unroll
-  for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-    for (int i = 0; i < J; ++i) x[mi][i] = zero8<b16>();
-  // (16 rows of 4 J units of 16 bytes; units past the row are its last one and meet nothing; 64 units that lie past M altogether stay away)
-  auto load_x = [&](int c) {
-#pragma unroll
-    for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-      for (int i = 0; i < J; ++i)
-        if (mi * 16 + 64 * i / (4 * J) < rows) {   // (scalar)
-          const int u = lane + 64 * i, r = u / (4 * J), col = min(4 * (k0 + c * J) + u % (4 * J), 4 * nks - 1);
-          x[mi][i] = load8(xp + (int64_t)min(m0 + mi * 16 + r, p.M - 1) * p.ldx + col * 8);
-        }
-  };
-  auto load_w = [&](b16x8(&dst)[J], int c) {
-#pragma unroll
-    for (int j = 0; j < J; ++j) dst[j] = load8(wp + (int64_t)min(k0 + min(c * J + j, per - 1), nks - 1) * 512);
-  };
-  load_x(0);
-#pragma unroll
-  for (int b = 0; b < (NB > 1 ? NB - 1 : 1); ++b) load_w(w[b], b);
   unsigned char* mine = smem + wave * STRIDE;
   f32x4 acc[MT];
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto chunk = [&](int c, b16x8(&cur)[J], b16x8(&last)[J]) {
+  if constexpr (NCH > 0) {
+    static_assert(MT == 1, "one row tile");
+    b16x8 xc[NB][XI], wc[NB][J];
+    const int u0 = 4 * k0 + lane % (4 * J), r0 = lane / (4 * J);   // (request i of a chunk: rows r0 + 2 i)
+    static_assert(4 * J == 32, "two rows a request");
+    const b16* xr[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) xr[i] = xp + (int64_t)min(m0 + r0 + 2 * i, p.M - 1) * p.ldx + u0 * 8;
+    const b16* wr = wp + (int64_t)k0 * 512;
+    auto ask = [&](int b, int c) {   // (in the order of their use, which is the order they come in)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < XI; ++i) xc[b][i] = load8(xr[i] + c * (32 * J));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < J; ++j) wc[b][j] = load8(wr + (c * J + j) * 512);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int b = 0; b < NB; ++b) ask(b, b);
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+#pragma unroll
+      for (int i = 0; i < XI; ++i) *reinterpret_cast<b16x8*>(mine + (r0 + 2 * i) * LDB + lane % (4 * J) * 16) = xc[c % NB][i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's LDS accesses happen in order: only the compiler has to keep them)
+#pragma unroll
+      for (int j = 0; j < J; ++j) mma(acc[0], wc[c % NB][j], *reinterpret_cast<const b16x8*>(mine + r16 * LDB + 64 * j + 16 * kc));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (c + NB < NCH) ask(c % NB, c + NB);
+    }
+  } else {
+    b16x8 x[MT][J], w[NB][J];
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi)
 #pragma unroll
-      for (int i = 0; i < J; ++i) {
-        const int u = lane + 64 * i;
-        *reinterpret_cast<b16x8*>(mine + (mi * 16 + u / (4 * J)) * LDB + u % (4 * J) * 16) = x[mi][i];
+      for (int i = 0; i < J; ++i) x[mi][i] = zero8<b16>();
+    // (16 rows of 4 J units of 16 bytes; units past the row are its last one and meet nothing; 64 units that lie past M altogether stay away)
+    auto load_x = [&](int c) {
+#pragma unroll
+      for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int i = 0; i < J; ++i)
+          if (mi * 16 + 64 * i / (4 * J) < rows) {   // (scalar)
+            const int u = lane + 64 * i, r = u / (4 * J), col = min(4 * (k0 + c * J) + u % (4 * J), 4 * nks - 1);
+            x[mi][i] = load8(xp + (int64_t)min(m0 + mi * 16 + r, p.M - 1) * p.ldx + col * 8);
+          }
+    };
+    auto load_w = [&](b16x8(&dst)[J], int c) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) dst[j] = load8(wp + (int64_t)min(k0 + min(c * J + j, per - 1), nks - 1) * 512);
+    };
+    load_x(0);
+#pragma unroll
+    for (int b = 0; b < (NB > 1 ? NB - 1 : 1); ++b) load_w(w[b], b);
+    auto chunk = [&](int c, b16x8(&cur)[J], b16x8(&last)[J]) {
+#pragma unroll
+      for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int i = 0; i < J; ++i) {
+          const int u = lane + 64 * i;
+          *reinterpret_cast<b16x8*>(mine + (mi * 16 + u / (4 * J)) * LDB + u % (4 * J) * 16) = x[mi][i];
+        }
+      if constexpr (NB > 1) {
+        if (c + 1 < nch) load_x(c + 1);
+        load_w(last, c + NB - 1);   // (past the end: a tile again, a cache hit)
       }
-    if constexpr (NB > 1) {
-      if (c + 1 < nch) load_x(c + 1);
-      load_w(last, c + NB - 1);   // (past the end: a tile again, a cache hit)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's LDS accesses happen in order: only the compiler has to keep them)
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (c * J + j < nk) {   // (scalar)
+#pragma unroll
+          for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], *reinterpret_cast<const b16x8*>(mine + (mi * 16 + r16) * LDB + 64 * j + 16 * kc));
+        }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    for (int c = 0; c < nch; c += NB) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        if (c + b < nch) chunk(c + b, w[b], w[(b + NB - 1) % NB]);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's LDS accesses happen in order: only the compiler has to keep them)
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-      if (c * J + j < nk) {   // (scalar)
-#pragma unroll
-        for (int mi = 0; mi < MT; ++mi) mma(acc[mi], cur[j], *reinterpret_cast<const b16x8*>(mine + (mi * 16 + r16) * LDB + 64 * j + 16 * kc));
-      }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  };
-  for (int c = 0; c < nch; c += NB) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-      if (c + b < nch) chunk(c + b, w[b], w[(b + NB - 1) % NB]);
   }
 #pragma unroll
   for (int mi = 0; mi < MT; ++mi) *reinterpret_cast<f32x4*>(mine + mi * 1024 + lane * 16) = acc[mi];
@@ -486,9 +522,14 @@ int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 // N 50272 42.8 (1) -> 35.0; K 4096, N 8192 8 / 24 / 64 14.2 / 14.0 / 20.7 -> 13.7 / 15.2 / 28.5, N 16384 16 rows 22.9 -> 24.8; K 512, N 16384 32 rows 7.1 -> 6.1, N 8192 64 rows 5.5 -> 6.0; K 128, N 50272 32
 // rows 10.5 -> 7.7; 32 / 64 groups of K 128, N 512 47 rows 4.2 / 5.3 -> 4.1 / 5.9 and, linear_kernel's nine column blocks of a group padded to sixteen, N 576 5.0 / 8.0 -> 4.4 / 6.5; 64 of K 256, N 128 4.5 -> 3.7.  Past 4608 columns
 // chunks follow each other: K 5120, N 6144 1 / 32 / 64 rows 12.6 / 15.1 / 22.0 -> 14.7 / 18.5 / 29.6, N 1024 16 rows 7.1 -> 7.6 (K 6144 7.9 -> 7.8, N 2048 8.5 -> 8.6), N 4096 10.4 -> 9.9; K 12288, N 6144 64 rows 66 -> 57.
+// Whole chunks (a form of its own, see plain_rows_kernel) keep more on their way: linear_kernel / here, K 6144, N 2048 1 / 16 rows 9.9 / 10.9 -> 7.8 / 9.5, N 6144 18.2 / 22.1 -> 16.3 / 20.8, N 8192 1 / 8 /
+// 16 rows 22.2 / 22.5 / 22.8 -> 19.9 / 20.7 / 23.6; K 8192, N 2048 11.0 / 14.0 -> 8.5 / 11.6, N 8192 28.2 / 28.1 -> 26.1 / 28.4; K 12288, N 2048 14.3 / 18.4 -> 11.7 / 16.0, N 6144 32.2 / 38.8 -> 30.4 / 37.3.
+static bool whole_chunks(int K) { return K == 6144 || K == 8192 || K == 12288; }
+
 bool plain_rows_fit(int M, int N, int K, int groups) {
   const int64_t slabs = (int64_t)(N >> 4) * groups;
   if (M > 64) return false;
+  if (whole_chunks(K) && M <= 16) return slabs <= (M <= 8 ? 512 : 384);
   if (K > 4608) {
     if (M > 32) return slabs <= (K > 8192 ? 384 : 256);
     return slabs <= 256 && (slabs * ((M + 15) >> 4) >= 192 || (slabs <= 96 && K % 2048 == 0));   // (fewer: linear_kernel's eight waves are level, and ahead where a chunk is not whole)
@@ -517,6 +558,16 @@ static int plain_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
     if (nks <= 96) return go(plain_rows_kernel<16, 6, 1, 1, EPI>, 16, 6, 1);
     if (nks <= 128) return go(plain_rows_kernel<16, 8, 1, 1, EPI>, 16, 8, 1);
     if (nks <= 144) return go(plain_rows_kernel<16, 9, 1, 1, EPI>, 16, 9, 1);
+    auto whole = [&](auto chunks) {   // (requests for rows: 2, 8 or 16 of them)
+      constexpr int NCH = decltype(chunks)::value;
+      if (p.M <= 2) return go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 1>, 8, 8, 1);
+      if (p.M <= 8) return go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 4>, 8, 8, 1);
+      return go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 8>, 8, 8, 1);
+    };
+    if (whole_chunks(p.K)) {
+      if (p.K == 6144) return whole(std::integral_constant<int, 3>{});
+      return p.K == 8192 ? whole(std::integral_constant<int, 4>{}) : whole(std::integral_constant<int, 6>{});
+    }
     return go(plain_rows_kernel<8, 8, 1, 3, EPI>, 8, 8, 1);
   }
   if (nks <= 4) return go(plain_rows_kernel<4, 1, 2, 1, EPI>, 4, 1, 2);
