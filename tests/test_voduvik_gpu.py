@@ -269,6 +269,29 @@ def test_rows_as_they_are_over_whole_chunks(M, slabs, K):
     close(ops.linear(x, t, gate=gate), y * torch.sigmoid(gate.double()), torch.bfloat16)
 
 
+@pytest.mark.parametrize("groups,K,N,pad", [(2, 64, 32, 0), (3, 128, 512, 64), (16, 192, 96, 8), (5, 512, 128, 16), (4, 96, 64, 0), (2, 320, 4096, 0)])
+@pytest.mark.parametrize("M", [65, 130, 400, 1100])
+def test_groups_of_many_rows(groups, K, N, pad, M):
+    """group_tiles_kernel, linear_kernel beside its line (few columns more or less, K no whole chunks of 64): groups whose columns of x overlap, stored
+    with a bias and gated, into columns of a wider matrix."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M * K + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    step, wide = K // 2 + pad, N + 32
+    w = (rnd(groups, N, K) / K ** 0.5).to(torch.bfloat16)
+    t, x = ops.MatrixTiles(w, torch.bfloat16), rnd(M, (groups - 1) * step + K + 8).to(torch.bfloat16)
+    gate, bias = rnd(M, groups).to(torch.bfloat16), rnd(N)
+    cols = torch.stack([x[:, i * step:i * step + K] for i in range(groups)]).double()
+    want = torch.bmm(cols, w.double().transpose(1, 2).contiguous())      # [groups, M, N]
+    for kind in ("bias", "gate"):
+        out = torch.full((M, groups * wide), 7.0, dtype=torch.bfloat16, device=dev())
+        ops.linear(x, t, x_gstride=step, y_gstride=wide, out=out, **({"bias": bias} if kind == "bias" else {"gate": gate}))
+        y = out.view(M, groups, wide)
+        close(y[..., :N].transpose(0, 1), want + bias if kind == "bias" else want * torch.sigmoid(gate.double()).T[..., None], torch.bfloat16)
+        assert (y[..., N:] == 7).all()
+
+
 def _norm_products(M, N, K):
     """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
     from vllmini_amd import hybrid_ops as ops

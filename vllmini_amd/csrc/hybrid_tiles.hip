@@ -46,6 +46,49 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args 
       });
 }
 
+// Products of a group of matrices, a group a y of the grid, each with its own columns of x and of y (the per-head products of latent attention, of low ranks)
+template <int MI, int NI, int D, int EPI>
+__global__ __launch_bounds__(256, 2) void group_tiles_kernel(const vmi_hy_linear_args p) {
+  const int kc = (threadIdx.x & 63) >> 4, grp = blockIdx.y;
+  vmi_tiles::tiles_product<vmi_tiles::Bf16, MI, NI, D>(
+      static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride, p.ldx, static_cast<const b16*>(p.w) + (int64_t)grp * p.N * p.K, p.M, p.N, p.K, [](int, int, int) {},
+      [&](const f32x4(&acc)[NI][MI], int m, int s, int SL) {
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+          if (s + n >= SL) break;   // (scalar)
+#pragma unroll
+          for (int i = 0; i < MI; ++i)
+            if (m + 16 * i < p.M) epilogue<b16, EPI>(p, acc[n][i], m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16, grp);
+        }
+      });
+}
+
+// Whether a group's products go to tiles: whole chunks of K, what the tiles' loads are aligned to, and more rows than plain_rows_kernel takes.  linear_kernel / tiles, us: 16 groups of K 128, N
+// 512 97 / 300 / 900 / 2773 rows 4.0 / 5.3 / 12.1 / 28.7 -> 3.5 / 5.2 / 10.0 / 24.4, of K 512, N 128 4.7 / 5.3 / 9.7 / 27.6 -> 3.8 / 5.4 / 8.4 / 18.9; 32 groups, 2773 rows 51 / 44 -> 45 / 30; 2 of
+// K 192, N 4096 900 13.2 -> 10.9.  (All ten groups below 65 rows: 2.4 - 2.9 -> 2.9 - 3.8.)  Not where tiles of 64 x 64 are just more than the chip has compute units for: 200 rows, 16 groups of K 128, N 512 4.6 / 4.9; 300,
+// 2 of K 192, N 4096 6.3 / 6.8; 500, 32 of K 512, N 128 11.6 / 12.0.
+bool group_tiles_fit(const vmi_hy_linear_args& p) {
+  const int64_t results = (int64_t)p.M * p.N * p.groups;
+  return p.groups > 1 && p.groups < 65536 && p.M > 64 && (results < 1300000 || results >= 2600000) && (p.N & 15) == 0 && (p.ldx & 7) == 0 && (p.x_gstride & 7) == 0 && p.x_gstride >= 0 && ((uintptr_t)p.x & 15) == 0 &&
+         ((uintptr_t)p.w & 15) == 0 && vmi_tiles::tiles_fit(p.M, p.K, p.ldx);
+}
+
+template <int EPI, int I = 0>
+static int launch_group_tiles_of(int pick, const vmi_hy_linear_args& p, hipStream_t st) {
+  if constexpr (I < vmi_tiles::NTILES) {
+    if (pick != I) return launch_group_tiles_of<EPI, I + 1>(pick, p, st);
+    constexpr vmi_tiles::Tile T = vmi_tiles::TILES[I];
+    hipLaunchKernelGGL((group_tiles_kernel<T.mi, T.ni, T.d, EPI>), dim3(vmi_tiles::tiles_grid(T, p.M, p.N), p.groups), dim3(256), 0, st, p);
+    return launched("vmi_hy_linear");
+  }
+  return fail(VMI_HY_E_SHAPE, "vmi_hy_linear", "no such tile");
+}
+
+int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
+  const int pick = vmi_tiles::tiles_pick(p.M, p.N, p.K, p.groups);
+  return p.epilogue == VMI_HY_E_STORE ? launch_group_tiles_of<VMI_HY_E_STORE>(pick, p, st) : launch_group_tiles_of<VMI_HY_E_GATED>(pick, p, st);
+}
+
 // Whether tiles of our own end sooner than the library's product (hipBLASLt as PyTorch 2.10.0+rocm7.0 loads it: another version may move the line, never the result beyond the
 // order of a sum).  Measured in bfloat16, 48 to 6000 rows, weights that leave the last cache between two products from K 2048 on and others that stay.
 //

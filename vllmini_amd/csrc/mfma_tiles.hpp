@@ -160,9 +160,9 @@ constexpr Tile TILES[] = {{8, 4, 2, .836f, .727f, 6.9f}, {8, 3, 2, .884f, .594f,
 constexpr int NTILES = sizeof(TILES) / sizeof(TILES[0]);
 
 // us, as the chip's tiles are dealt
-inline float tiles_cost(int i, int M, int N, int K) {
+inline float tiles_cost(int i, int M, int N, int K, int groups) {
   const Tile& t = TILES[i];
-  const int64_t n = (int64_t)((M + 16 * t.mi - 1) / (16 * t.mi)) * ((N + 64 * t.ni - 1) / (64 * t.ni)), share = (n + 255) / 256;
+  const int64_t n = (int64_t)((M + 16 * t.mi - 1) / (16 * t.mi)) * ((N + 64 * t.ni - 1) / (64 * t.ni)) * groups, share = (n + 255) / 256;
   const int chunks = ((K >> 6) + t.d - 1) / t.d * t.d;
   return 2.f + (share == 1 ? t.alone : share * t.beside) * ((float)chunks + t.ends);
 }
@@ -170,11 +170,11 @@ inline float tiles_cost(int i, int M, int N, int K) {
 // The tile whose largest share of a compute unit ends first: so many tiles one behind the other, each 64 columns of K at a time and as long as `ends` such at its ends.  On
 // average 0.7 per cent behind the best of the list over those products.  (us, 128 x 256 / 128 x 192, four chunks / 96 x 128, four / 32 x 64, four: 2773 rows, N 2048,
 // K 6144 81 / 63 / 75 / 190; 300 rows, the same 70 / 46 / 34 / 23 and 64 x 64 19.)
-inline int tiles_pick(int M, int N, int K) {
+inline int tiles_pick(int M, int N, int K, int groups = 1) {
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < NTILES; ++i) {
-    const float cost = tiles_cost(i, M, N, K);
+    const float cost = tiles_cost(i, M, N, K, groups);
     if (i == 0 || cost < least) best = i, least = cost;
   }
   return best;
