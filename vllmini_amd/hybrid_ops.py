@@ -27,6 +27,7 @@ from typing import NamedTuple, Optional, Tuple
 import torch
 
 from . import build as _build
+from .ops import _stream_of
 from .staging import PinnedBuffer
 
 ABI_VERSION = 3
@@ -138,9 +139,10 @@ def _check(rc: int) -> None:
         raise RuntimeError(load().vmi_hybrid_last_error().decode("utf-8", "replace"))
 
 
-def _need(cond: bool, what: str) -> None:
+def _need(cond: bool, what) -> None:
+    """what: the message, or what makes it (one with sizes in it took as long as a launch)"""
     if not cond:
-        raise RuntimeError(what)
+        raise RuntimeError(what if isinstance(what, str) else what())
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -148,9 +150,9 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _on(t: torch.Tensor) -> Tuple[int, int]:
-    _need(t.device.type == "cuda", "hybrid_ops: there is no CPU path")
-    idx = t.device.index if t.device.index is not None else torch.cuda.current_device()
-    return idx, torch.cuda.current_stream(t.device).cuda_stream
+    _need(t.is_cuda, "hybrid_ops: there is no CPU path")
+    idx = t.get_device()
+    return idx, _stream_of(idx)   # (torch.cuda.current_stream makes a Stream of it: 2 us a call, 60 calls a prompt)
 
 
 def pad32(n: int) -> int:
@@ -220,7 +222,7 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
     K, N = w.K, w.N
     span = (w.groups - 1) * x_gstride + (K // 2 if kind == X_CONCAT else K)
     _need(x.dim() == 2 and x.stride(1) == 1 and x.shape[1] >= span and x.dtype == (T if kind == X_ROWS else torch.float32),
-          f"hybrid_ops.linear: x {tuple(x.shape)} {x.dtype} does not hold {w.groups} x {K} columns")
+          lambda: f"hybrid_ops.linear: x {tuple(x.shape)} {x.dtype} does not hold {w.groups} x {K} columns")
     if x2 is not None:
         _need(x2.shape == x.shape and x2.stride() == x.stride() and x2.dtype == torch.float32 and x2.device == x.device,
               "hybrid_ops.linear: x2 must match x")
@@ -241,7 +243,7 @@ def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, 
     if out is None:
         out = torch.empty((M, cols), dtype=odt, device=x.device)
     _need(out.dim() == 2 and out.shape[0] == M and out.shape[1] >= cols and out.stride(1) == 1 and out.dtype == odt
-          and out.data_ptr() != x.data_ptr(), f"hybrid_ops.linear: out {tuple(out.shape)} {out.dtype} for {M} x {cols}")
+          and out.data_ptr() != x.data_ptr(), lambda: f"hybrid_ops.linear: out {tuple(out.shape)} {out.dtype} for {M} x {cols}")
     normed = torch.empty((M, K), dtype=T, device=x.device) if norm is not None and _normed_first(M, N, K, w.groups, T) else None
     a = LinearArgs(x=x.data_ptr(), x2=_ptr(x2), normed=_ptr(normed), rows=_ptr(rows), norm_w=norm[0].data_ptr() if norm else None, w=w.tiles.data_ptr(),
                    bias=_ptr(bias), gate=_ptr(gate), y=out.data_ptr(), y2=_ptr(glu_out), ldx=x.stride(0), ldy=out.stride(0),
@@ -261,7 +263,7 @@ def linear_tiles(x: torch.Tensor, w: MatrixTiles, unit: GatedUnit, split: int = 
     device, stream = _on(x)
     M, N, K = int(x.shape[0]), w.N, w.K
     _need(w.groups == 1 and w.tiles.dtype == torch.bfloat16 and w.tiles.device == x.device, "hybrid_ops.linear_tiles: one bfloat16 matrix on x's device")
-    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, f"hybrid_ops.linear_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
+    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, lambda: f"hybrid_ops.linear_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
     _need(0 <= split <= N and split % 16 == 0, "hybrid_ops.linear_tiles: split")
     if glu_out is None:
         glu_out = torch.empty((M, (N - split) // 2), dtype=x.dtype, device=x.device)
@@ -290,7 +292,7 @@ def product_tiles(x: torch.Tensor, w: MatrixTiles, bias: Optional[torch.Tensor] 
     device, stream = _on(x)
     M, N, K = int(x.shape[0]), w.N, w.K
     _need(w.groups == 1 and w.tiles.dtype == torch.bfloat16 and w.tiles.device == x.device, "hybrid_ops.product_tiles: one bfloat16 matrix on x's device")
-    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, f"hybrid_ops.product_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
+    _need(x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[1] == K and x.stride(1) == 1, lambda: f"hybrid_ops.product_tiles: x {tuple(x.shape)} {x.dtype} is not rows of {K}")
     _need(bias is None or (not float_out and bias.dtype == torch.float32 and bias.numel() >= N and bias.is_contiguous() and bias.device == x.device),
           "hybrid_ops.product_tiles: bias float32 [N], with a result in bfloat16")
     y = torch.empty((M, N), dtype=torch.float32 if float_out else x.dtype, device=x.device)
