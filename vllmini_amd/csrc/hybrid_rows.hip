@@ -476,7 +476,7 @@ int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 // Infinity Cache, the other kernels / this one: K 2048, N 12288 8 / 12 / 32 / 40 rows 14.9 / 17.8 / 21.6 / 41.8 -> 14.9 / 15.0 / 17.3 / 17.2, N 20480 19.0 / 22.3 / 26.8 / 47.8 -> 19.9 / 19.9 / 22.2 / 23.5, N 50272 39.4 / 42.3 / 50.4 /
 // 95.1 -> 41.3 / 41.6 / 45.7 / 48.8; K 1024, N 50272 40 rows 49.5 -> 22.1; K 3072, 33 / 47 / 64 rows, N 512 26.2 / 27.2 / 31.7 -> 12.6 / 12.6 / 13.7,
 // N 4096 27.9 / 28.8 / 33.4 -> 14.3 / 14.7 / 16.4, N 24576 57.5 / 57.0 / 58.2 -> 35.2 / 37.2 / 39.0 (9 to 32 rows stay with resident_kernel, which is behind too from N 2048 on: N 6144 16 rows 17.7, 14.3 here); K 4096, N 4096 12.3 / 13.9 / 17.9 -> 13.3 / 17.6 / 16.5 (40 rows gated 27.5 -> 16.9), N 6144 17.9 / 21.1 / 27.7 -> 16.2 / 20.2 / 20.0, N 8192 19.0 / 22.5 /
-// 28.7 -> 19.1 / 23.1 / 23.0, N 12288 26.6 / 30.4 / 32.8 -> 23.7 / 28.4 / 28.8, N 50272 85.3 / 97.0 / 108 -> 85.5 / 83.2 / 87.7; with weights in that cache N 6144 32 rows 15.5 -> 18.5.
+// 28.7 -> 19.1 / 23.1 / 23.0 (the walk with its conditions; without them K 1024 to 3072 end 3 to 10 per cent sooner), N 12288 26.6 / 30.4 / 32.8 -> 23.7 / 28.4 / 28.8, N 50272 85.3 / 97.0 / 108 -> 85.5 / 83.2 / 87.7; with weights in that cache N 6144 32 rows 15.5 -> 18.5.
 bool held_rows_pay(int M, int N, int K, bool stored) {
   if (M < 9 || M > 64 || norm_slabs(M, N, K) > 0) return false;
   if (K == 4096) return M <= 16 ? N >= 6144 : M <= 32 ? N >= 12288 : N >= 4096 || !stored;
@@ -518,7 +518,7 @@ int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 // linear_kernel / plain_rows_kernel, in a graph of such launches, us: K 1024, N 1024 1 / 16 / 32 / 64 rows 3.7 / 4.0 / 4.1 / 6.4 -> 2.9 / 3.1 / 3.1 / 3.2, K 3072, N 1024 4.8 / 5.4 / 5.5 / 13.0 ->
 // 3.8 / 4.4 / 4.5 / 4.6, K 8192, N 2048 10.7 / 13.3 / 14.2 / 44.5 -> 10.1 / 12.5 / 12.3 / 15.2, K 4096, N 4096 10.1 / 11.3 / 12.4 / 24.6 -> 8.1 / 9.0 / 10.7 / 17.1, K 12288, N 4096 20.8 / 22.5 / 27.9 /
 // 65.2 -> 20.0 / 21.6 / 25.3 / 41.4; 8 groups of K 128, N 512 3.7 / 3.9 / 4.0 / 3.4 -> 2.3 / 2.4 / 2.5 / 2.6, of K 512, N 128 4.0 / 4.5 / 4.5 / 5.1 -> 2.5 / 2.7 / 2.7 / 2.7.  Of more rows there are tiles.
-// Every workgroup brings the rows again, so past one slab a compute unit (256) it is ahead only while the rows are few or short: K 2048, N 16384 1 / 32 / 64 rows 13.6 / 13.8 / 16.2 -> 12.7 / 16.8 / 30.8,
+// (K 8192 and 12288 before whole chunks had a form of their own: below.)  Every workgroup brings the rows again, so past one slab a compute unit (256) it is ahead only while the rows are few or short: K 2048, N 16384 1 / 32 / 64 rows 13.6 / 13.8 / 16.2 -> 12.7 / 16.8 / 30.8,
 // N 50272 42.8 (1) -> 35.0; K 4096, N 8192 8 / 24 / 64 14.2 / 14.0 / 20.7 -> 13.7 / 15.2 / 28.5, N 16384 16 rows 22.9 -> 24.8; K 512, N 16384 32 rows 7.1 -> 6.1, N 8192 64 rows 5.5 -> 6.0; K 128, N 50272 32
 // rows 10.5 -> 7.7; 32 / 64 groups of K 128, N 512 47 rows 4.2 / 5.3 -> 4.1 / 5.9 and, linear_kernel's nine column blocks of a group padded to sixteen, N 576 5.0 / 8.0 -> 4.4 / 6.5; 64 of K 256, N 128 4.5 -> 3.7.  Past 4608 columns
 // chunks follow each other: K 5120, N 6144 1 / 32 / 64 rows 12.6 / 15.1 / 22.0 -> 14.7 / 18.5 / 29.6, N 1024 16 rows 7.1 -> 7.6 (K 6144 7.9 -> 7.8, N 2048 8.5 -> 8.6), N 4096 10.4 -> 9.9; K 12288, N 6144 64 rows 66 -> 57.

@@ -7,7 +7,7 @@ namespace vmi_hybrid {
 
 // STORE_GLU: columns below n_split as they are, the others, interleaved (gate, up), through the gated unit: what a product and an elementwise launch behind it (a
 // write and a read of 2 N bytes a row) took, and what they give: gate and up are rounded on their way into the unit, so what a prompt comes to does not hang on
-// which side tiles_pay finds ahead for the tokens that happen to share its step.  STORE, FLOAT: a product alone, with the bias in 32 bits, in bfloat16 or as it is.
+// whether the tokens that happen to share its step are enough for tiles.  STORE, FLOAT: a product alone, with the bias in 32 bits, in bfloat16 or as it is.
 template <int MI, int NI, int D, int EPI>
 __global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args p) {
   const int kc = (threadIdx.x & 63) >> 4;
