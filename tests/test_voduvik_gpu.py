@@ -292,6 +292,20 @@ def test_groups_of_many_rows(groups, K, N, pad, M):
         assert (y[..., N:] == 7).all()
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 9, 16, 17])
+@pytest.mark.parametrize("N,K", [(48, 64), (128, 448), (16 * 30, 1024), (96, 1984), (64, 2112), (16 * 70, 4608), (32, 6144), (16 * 20, 8192), (48, 12288), (64, 10240)])
+def test_few_rows_side_by_side(M, N, K):
+    """plain_rows_kernel over two float32 halves: waves whose parts lie in one and in both, K in one chunk a wave and in several, linear_kernel past its lines; some of the columns, scaled."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M * K + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    a, b, w = rnd(M, K // 2 + 8)[:, :K // 2], rnd(M, K // 2 + 8)[:, :K // 2], (rnd(ops.pad32(N), K) / K ** 0.5).to(torch.bfloat16)
+    want = torch.cat([a, b], 1).to(torch.bfloat16).double() @ w.double().T
+    got = ops.linear(a, ops.MatrixTiles(w, torch.bfloat16), x2=b, float_out=(N - 3, 0.5))
+    close(got, 0.5 * want[:, :N - 3], torch.bfloat16, tol16=1e-5)      # (products of 16 bits are exact in 32: what is left is the order of a float32 sum)
+
+
 def _norm_products(M, N, K):
     """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
     from vllmini_amd import hybrid_ops as ops

@@ -520,6 +520,8 @@ static int linear_shape(const vmi_hy_linear_args& p, hipStream_t st) {
   // few rows: 16-row tiles; a layer with few columns splits K over the waves of a workgroup so that all compute units read
   const int64_t slabs = (int64_t)(p.N / 16) * p.groups;
   constexpr bool PLAIN = sizeof(T) == 2 && XK == VMI_HY_X_ROWS && (EPI == VMI_HY_E_STORE || EPI == VMI_HY_E_RESIDUAL || EPI == VMI_HY_E_GATED);
+  if constexpr (sizeof(T) == 2 && XK == VMI_HY_X_CONCAT && EPI == VMI_HY_E_FLOAT)
+    if (p.groups == 1 && concat_rows_fit(p.M, p.N, p.K)) return launch_concat_rows(p, st);
   if constexpr (PLAIN && EPI != VMI_HY_E_RESIDUAL)
     if (group_tiles_fit(p)) return launch_group_tiles(p, st);
   if constexpr (PLAIN)

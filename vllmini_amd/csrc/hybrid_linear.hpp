@@ -61,6 +61,8 @@ bool held_rows_pay(int M, int N, int K, bool stored);   // of the element type b
 int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool plain_rows_fit(int M, int N, int K, int groups);   // of the element type
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st);
+bool concat_rows_fit(int M, int N, int K);   // float32 rows side by side, FLOAT, one group
+int launch_concat_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool group_tiles_fit(const vmi_hy_linear_args& p);   // STORE or GATED, of the element type, many rows (hybrid_tiles.hip)
 int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st);
 int launch_norm_few(const vmi_hy_linear_args& p, hipStream_t st);   // p.normed = the norm of p.x

@@ -27,11 +27,19 @@ constexpr int plain_stride(int J, int MT) { return MT * 16 * (64 * J + 16); }   
 // not see it waited for all of them at every chunk.  XI: requests for the rows of a chunk (2 XI rows at most).  Before -> now, weights not in the Infinity Cache, us: K 6144, N 1024 1 / 16 / 32
 // rows 7.9 / 9.7 / 9.4 -> 6.5 / 8.8 / 8.6, N 2048 32 rows 10.2 -> 9.4, N 4096 1 / 16 12.4 / 14.1 -> 11.1 / 13.1; K 8192, N 2048 32 rows 12.5 -> 11.4, N 4096 1 / 16 16.4 / 17.9 -> 14.5 / 16.3; K 12288,
 // N 1024 12.0 / 16.0 -> 11.0 / 14.7, N 4096 21.9 / 23.8 -> 20.3 / 22.6 (101 MB, 5.0 TB/s).
-template <int RW, int J, int MT, int NB, int EPI, int NCH = 0, int XI = J>
+// XK = VMI_HY_X_CONCAT: rows of x and x2 side by side, float32, rounded on their way into LDS (half of K is whole units, and of whole chunks a wave's part lies in one).
+template <int RW, int J, int MT, int NB, int EPI, int NCH = 0, int XI = J, int XK = VMI_HY_X_ROWS>
 __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_hy_linear_args p) {
+  constexpr bool CAT = XK == VMI_HY_X_CONCAT;
+  using XT = std::conditional_t<CAT, float, b16>;
+  auto rounded = [](const V8<XT>& v) {
+    if constexpr (CAT) return from_f32<b16>(v);
+    else return v;
+  };
   constexpr int LDB = 64 * J + 16, STRIDE = plain_stride(J, MT);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [RW][STRIDE]
   need_args<EPI>(p), need(p.x_gstride), need(p.y_gstride);
+  if constexpr (CAT) need(p.x2);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
   const int slab = blockIdx.x, m0 = blockIdx.y * 16 * MT, grp = blockIdx.z;
   if (slab * 16 >= p.N) return;
@@ -43,7 +51,8 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
   if constexpr (EPI == VMI_HY_E_RESIDUAL)
     if (stores) before = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p.y) + (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride + n);
 
-  const b16* xp = static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride;
+  const XT* xp = static_cast<const XT*>(p.x) + (int64_t)grp * p.x_gstride;
+  [[maybe_unused]] const XT* x2p = CAT ? static_cast<const XT*>(p.x2) - (p.K >> 1) : nullptr;   // (column c of the second half: x2p[c])
   const b16* wp = static_cast<const b16*>(p.w) + (((int64_t)grp * (p.N >> 4) + slab) * nks * 64 + lane) * 8;
   unsigned char* mine = smem + wave * STRIDE;
   f32x4 acc[MT];
@@ -51,12 +60,13 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
   for (int mi = 0; mi < MT; ++mi) acc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
   if constexpr (NCH > 0) {
     static_assert(MT == 1, "one row tile");
-    b16x8 xc[NB][XI], wc[NB][J];
+    V8<XT> xc[NB][XI];
+    b16x8 wc[NB][J];
     const int u0 = 4 * k0 + lane % (4 * J), r0 = lane / (4 * J);   // (request i of a chunk: rows r0 + 2 i)
     static_assert(4 * J == 32, "two rows a request");
-    const b16* xr[XI];
+    const XT* xr[XI];
 #pragma unroll
-    for (int i = 0; i < XI; ++i) xr[i] = xp + (int64_t)min(m0 + r0 + 2 * i, p.M - 1) * p.ldx + u0 * 8;
+    for (int i = 0; i < XI; ++i) xr[i] = (CAT && wave >= RW / 2 ? x2p : xp) + (int64_t)min(m0 + r0 + 2 * i, p.M - 1) * p.ldx + u0 * 8;
     const b16* wr = wp + (int64_t)k0 * 512;
     auto ask = [&](int b, int c) {   // (in the order of their use, which is the order they come in)
       __builtin_amdgcn_sched_barrier(0);
@@ -72,7 +82,7 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
 #pragma unroll
-      for (int i = 0; i < XI; ++i) *reinterpret_cast<b16x8*>(mine + (r0 + 2 * i) * LDB + lane % (4 * J) * 16) = xc[c % NB][i];
+      for (int i = 0; i < XI; ++i) *reinterpret_cast<b16x8*>(mine + (r0 + 2 * i) * LDB + lane % (4 * J) * 16) = rounded(xc[c % NB][i]);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wave's LDS accesses happen in order: only the compiler has to keep them)
 #pragma unroll
       for (int j = 0; j < J; ++j) mma(acc[0], wc[c % NB][j], *reinterpret_cast<const b16x8*>(mine + r16 * LDB + 64 * j + 16 * kc));
@@ -80,11 +90,12 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
       if (c + NB < NCH) ask(c % NB, c + NB);
     }
   } else {
-    b16x8 x[MT][J], w[NB][J];
+    V8<XT> x[MT][J];
+    b16x8 w[NB][J];
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi)
 #pragma unroll
-      for (int i = 0; i < J; ++i) x[mi][i] = zero8<b16>();
+      for (int i = 0; i < J; ++i) x[mi][i] = zero8<XT>();
     // (16 rows of 4 J units of 16 bytes; units past the row are its last one and meet nothing; 64 units that lie past M altogether stay away)
     auto load_x = [&](int c) {
 #pragma unroll
@@ -93,7 +104,7 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
         for (int i = 0; i < J; ++i)
           if (mi * 16 + 64 * i / (4 * J) < rows) {   // (scalar)
             const int u = lane + 64 * i, r = u / (4 * J), col = min(4 * (k0 + c * J) + u % (4 * J), 4 * nks - 1);
-            x[mi][i] = load8(xp + (int64_t)min(m0 + mi * 16 + r, p.M - 1) * p.ldx + col * 8);
+            x[mi][i] = load8((CAT && 16 * col >= p.K ? x2p : xp) + (int64_t)min(m0 + mi * 16 + r, p.M - 1) * p.ldx + col * 8);
           }
     };
     auto load_w = [&](b16x8(&dst)[J], int c) {
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
 #pragma unroll
         for (int i = 0; i < J; ++i) {
           const int u = lane + 64 * i;
-          *reinterpret_cast<b16x8*>(mine + (mi * 16 + u / (4 * J)) * LDB + u % (4 * J) * 16) = x[mi][i];
+          *reinterpret_cast<b16x8*>(mine + (mi * 16 + u / (4 * J)) * LDB + u % (4 * J) * 16) = rounded(x[mi][i]);
         }
       if constexpr (NB > 1) {
         if (c + 1 < nch) load_x(c + 1);
@@ -576,6 +587,30 @@ static int plain_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
   if (nks <= 32) return go(plain_rows_kernel<8, 4, 2, 1, EPI>, 8, 4, 2);
   if (nks <= 64) return go(plain_rows_kernel<16, 4, 2, 1, EPI>, 16, 4, 2);
   return go(plain_rows_kernel<16, 4, 2, 2, EPI>, 16, 4, 2);
+}
+
+// linear_kernel / here, us, weights not in the Infinity Cache: K 512, N 256 1 / 16 rows 3.5 / 4.4 -> 2.1 / 2.4, K 2048, N 1024 4.5 / 5.8 -> 3.3 / 4.1, N 4096 7.5 / 10.3 -> 5.7 / 6.7; K 4096, N 2048 8.3 / 12.0 -> 6.4 / 8.9; K 8192, N
+// 4096 1 / 8 19.0 / 25.0 -> 15.2 / 16.7, K 12288, N 6144 34.9 / 46.6 -> 31.5 / 38.3.  (Past 16 rows linear_kernel, as before.)
+bool concat_rows_fit(int M, int N, int K) {
+  if (M > 16) return false;
+  return whole_chunks(K) ? M <= 8 && N <= 16 * 512 : K <= 4608 && plain_rows_fit(M, N, K, 1);   // (registers hold four requests of float32 rows three chunks ahead, not eight)
+}
+
+int launch_concat_rows(const vmi_hy_linear_args& p, hipStream_t st) {
+  constexpr int EPI = VMI_HY_E_FLOAT, XK = VMI_HY_X_CONCAT;
+  const int nks = p.K >> 5;
+  auto go = [&](auto* fn, int rw, int j) { return launch(fn, p, dim3(blocks8(p.N >> 4), 1, 1), 64 * rw, (size_t)rw * plain_stride(j, 1), st); };
+  if (nks <= 16) return go(plain_rows_kernel<4, 4, 1, 1, EPI, 0, 4, XK>, 4, 4);
+  if (nks <= 32) return go(plain_rows_kernel<8, 4, 1, 1, EPI, 0, 4, XK>, 8, 4);
+  if (nks <= 64) return go(plain_rows_kernel<8, 8, 1, 1, EPI, 0, 8, XK>, 8, 8);
+  if (nks <= 96) return go(plain_rows_kernel<16, 6, 1, 1, EPI, 0, 6, XK>, 16, 6);
+  if (nks <= 144) return go(plain_rows_kernel<16, 9, 1, 1, EPI, 0, 9, XK>, 16, 9);
+  auto whole = [&](auto chunks) {
+    constexpr int NCH = decltype(chunks)::value;
+    return p.M <= 2 ? go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 1, XK>, 8, 8) : go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 4, XK>, 8, 8);
+  };
+  if (p.K == 6144) return whole(std::integral_constant<int, 3>{});
+  return p.K == 8192 ? whole(std::integral_constant<int, 4>{}) : whole(std::integral_constant<int, 6>{});
 }
 
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
