@@ -93,7 +93,7 @@ class GPT2PagedDecoder:
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
     # prompts of more tokens in all (times the width's square) issue their launches from here: the native call saves the host 150 us, which is what a call of fewer waits for.
-    # Their products are tiles of this build's own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond.  12
+    # Their products are tiles of our own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond.  12
     # layers of prompts of 100 tokens, tiles / vendor in us: width 256 8000 tokens 1485 / 2541, 512 1681 / 2570; 768 5000 1764 / 2187, 6000 2147 / 2357, 8000 2623 / 2787; 1024
     # 4000 2084 / 2164, 5000 2522 / 2352, 7000 4024 / 3140; 1152 4000 2579 / 2691, 7000 3736 / 3791
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
@@ -375,7 +375,7 @@ class GPT2PagedDecoder:
     def _whole_prompts(self, ids: np.ndarray, lens: List[int], tabs) -> torch.Tensor:
         """prefill_batch over prompt_attention: what its launches read goes up in one asynchronous copy, and around the attention a layer
         takes four or six launches (the decode step's linear kernels, or norms and tiles) up to NATIVE_PROMPT_MAX_TOKENS tokens, all of them issued by
-        one native call, and the same six issued from here beyond; past OWN_PRODUCTS_MAX_WORK the vendor's products around one of this build's tiles for c_fc and its GELU, and one
+        one native call, and the same six issued from here beyond; past OWN_PRODUCTS_MAX_WORK the vendor's products around one of our own tiles for c_fc and its GELU, and one
         kernel for the residual add with the norm behind it."""
         d, pool, dev, sd = self.dims, self.pool, self.device, self.sd
         H, T, mbe = d.n_head, len(ids), -(-max(lens) // pool.block_size)
