@@ -38,6 +38,7 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
   constexpr int BM = 16 * MI, BN = 64 * NI, ST = BM * 128, XU = BM * 8 / 256;   // 16-byte pieces of x a thread brings
   constexpr int AHEAD = 4, STEPS = 2 * MI, ASKS = XU + 2 * NI, PER = (ASKS + STEPS - 1) / STEPS;
   static_assert(STEPS >= AHEAD, "fragments of one chunk");
+  static_assert(PER == 1, "a barrier of the scheduler between any two requests of the walk");
   // (arrays by name: only so does the compiler know that a read of one does not wait for what is on its way into another)
   __shared__ __attribute__((aligned(1024))) unsigned char xs0[ST], xs1[ST], xs2[D > 2 ? ST : 1], xs3[D > 3 ? ST : 1];
   unsigned char* const xs[4] = {xs0, xs1, xs2, xs3};
@@ -88,10 +89,15 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
+  // (the counts above are of requests in this order, and to the scheduler requests into LDS and into registers have nothing to do with each other)
 #pragma unroll
-  for (int d = 0; d < D - 1; ++d)
+  for (int d = 0; d < D - 1; ++d) {
 #pragma unroll
-    for (int i = 0; i < ASKS; ++i) ask(i, d, min(d, nkb - 1));
+    for (int i = 0; i < ASKS; ++i) {
+      ask(i, d, min(d, nkb - 1));
+      if (i == XU - 1 || i == ASKS - 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
   early(m0 + r16, s0, SL);
   x_landed(std::integral_constant<int, D - 2>{});
   // The chunk in place d, and chunk kb on its way into the place of the one before (whose readers have all passed the barrier): steps of one fragment of x, which was asked
