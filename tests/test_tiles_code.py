@@ -1,8 +1,10 @@
 """What mfma_tiles.hpp relies on and no result shows: the code that the compiler makes of it (CPU: hipcc compiles for gfx950 without one)."""
 import os
 import re
+import struct
 import subprocess
 
+import msgpack
 import pytest
 
 from vllmini_amd import build
@@ -44,3 +46,51 @@ def test_requests_of_a_tile_go_out_in_the_order_that_its_waits_count(strategy, t
         chunk = "X" * (mi // 2) + "W" * (2 * ni)
         assert parts[0] == chunk * (d - 1), (mi, ni, d, parts[0])
         assert parts[1:] == [chunk] * (d + 1) + [""] * (d - 1), (mi, ni, d, parts)
+
+
+def _code_objects(path):
+    """The gfx950 code objects of a library built here."""
+    data, at = open(path, "rb").read(), 0
+    while (at := data.find(b"__CLANG_OFFLOAD_BUNDLE__", at)) >= 0:
+        p = at + 32
+        for _ in range(struct.unpack_from("<Q", data, at + 24)[0]):
+            offset, size, n = struct.unpack_from("<QQQ", data, p)
+            if b"gfx950" in data[p + 24: p + 24 + n]:
+                yield data[at + offset: at + offset + size]
+            p += 24 + n
+        at += 24
+
+
+def _kernels(obj):
+    """Its kernels as the metadata note lists them."""
+    sections, (step, n) = struct.unpack_from("<Q", obj, 0x28)[0], struct.unpack_from("<HH", obj, 0x3A)
+    for i in range(n):
+        kind, offset, size = (struct.unpack_from(f, obj, sections + i * step + a)[0] for f, a in (("<I", 4), ("<Q", 24), ("<Q", 32)))
+        if kind == 7:      # SHT_NOTE; its records: sizes of name and content, type
+            while size > 0:
+                a, b, t = struct.unpack_from("<III", obj, offset)
+                if t == 32:
+                    return msgpack.unpackb(obj[offset + 12 + (a + 3) // 4 * 4:][:b])["amdhsa.kernels"]
+                used = 12 + (a + 3) // 4 * 4 + (b + 3) // 4 * 4
+                offset, size = offset + used, size - used
+    return []
+
+
+@pytest.mark.parametrize("lib,kinds", [(build.LAYER_LIB_PATH, 3), (build.HYBRID_LIB_PATH, 5)])
+def test_every_tile_keeps_its_registers_and_its_scalars(lib, kinds, tmp_path):
+    """What the cost of a tile is fitted to: no instance of a tile keeps values in scratch memory, and none asks for weights lane by lane because an offset is no scalar."""
+    objdump = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(build._hipcc()))), "llvm", "bin", "llvm-objdump")
+    seen = 0
+    for obj in _code_objects(lib):
+        tiles = {k[".name"]: k for k in _kernels(obj) if "tiles_kernelILi" in k[".name"]}
+        if not tiles:
+            continue
+        (tmp_path / "code").write_bytes(obj)
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(tmp_path / "code")], capture_output=True, text=True, check=True).stdout
+        code = {m.group(1): part for part in re.split(r"\n(?=[0-9a-f]{16} <)", text) if (m := re.match(r"[0-9a-f]{16} <(\w+)>:", part))}
+        for name, k in tiles.items():
+            assert k[".private_segment_fixed_size"] == k[".vgpr_spill_count"] == k[".sgpr_spill_count"] == 0, name
+            walk = code[name][: code[name].rfind("s_barrier")]
+            assert "s_barrier" in walk and "execnz" not in walk and "scratch_" not in walk, name
+        seen += len(tiles)
+    assert seen == 13 * kinds      # (the list of tiles, a launch of each for every kind of end)

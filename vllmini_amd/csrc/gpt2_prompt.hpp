@@ -319,10 +319,10 @@ __global__ __launch_bounds__(256) void add_norm_kernel(h16* __restrict__ x, cons
 }
 
 // Linear layers of many rows, packed weights (mfma_tiles.hpp): bias, GELU or the residual add on a lane's four columns of a row, the rounding points of the few-row
-// kernels.  The bias is asked for at the start, residuals too where a tile leaves the registers, else a slab's together at the end.
+// kernels.  The bias is asked for at the start, residuals too, each where a tile leaves the registers for it, else a slab's together at the end.
 template <int MI, int NI, int D, int EPI>
 __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
-  constexpr bool EARLY = MI * NI <= 12;
+  constexpr bool EARLY = MI * NI <= 12, EARLY_BIAS = MI * NI <= 24 || EPI == VMI_LAYER_EPI_BIAS;
   const int kc = (threadIdx.x & 63) >> 4;
   h16x4 bias[NI];
   Tail tail[NI][MI];
@@ -333,8 +333,10 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
   vmi_tiles::tiles_product<vmi_tiles::Half, MI, NI, D>(
       p.x, p.ldx, p.w, p.M, p.N, p.K,
       [&](int m, int s, int SL) {
+        if constexpr (EARLY_BIAS) {
 #pragma unroll
-        for (int n = 0; n < NI; ++n) bias[n] = Tail::load_bias(p, min(s + n, SL - 1) * 16 + 4 * kc);
+          for (int n = 0; n < NI; ++n) bias[n] = Tail::load_bias(p, min(s + n, SL - 1) * 16 + 4 * kc);
+        }
         if constexpr (EARLY) {
 #pragma unroll
           for (int n = 0; n < NI; ++n)
@@ -345,6 +347,7 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
 #pragma unroll
         for (int n = 0; n < NI; ++n) {
           if (s + n >= SL) break;   // (scalar)
+          if constexpr (!EARLY_BIAS) bias[n] = Tail::load_bias(p, (s + n) * 16 + 4 * kc);
           if constexpr (!EARLY) ask(n, m, s);
 #pragma unroll
           for (int i = 0; i < MI; ++i) {

@@ -48,7 +48,8 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
   // together share their rows and weights in its L2
   constexpr int DOWN = 1024 / BM;
   const int all = NB * MB, die = (int)blockIdx.x & 7, tile = die * (all >> 3) + min(die, all & 7) + ((int)blockIdx.x >> 3);
-  const int band = tile / (DOWN * NB), in = tile - band * DOWN * NB, rows = min(DOWN, MB - band * DOWN), col = in / rows;
+  // (a division leaves a scalar's value in a vector register: said here, or the compiler may keep what follows from it there, and ask for weights lane by lane)
+  const int band = __builtin_amdgcn_readfirstlane(tile / (DOWN * NB)), in = tile - band * DOWN * NB, rows = min(DOWN, MB - band * DOWN), col = __builtin_amdgcn_readfirstlane(in / rows);
   const int m0 = (band * DOWN + in - col * rows) * BM, s0 = col * 4 * NI + wave * NI;
   // (rows past the last, slabs past the last and chunks past the end are those again: no lane-wise condition around a load)
   const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(x), 0, -1, 0x20000);
