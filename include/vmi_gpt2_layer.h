@@ -135,6 +135,8 @@ typedef struct {
   float eps, scale;
 } vmi_gpt2_prompts;
 VMI_LAYER_API int vmi_gpt2_prompts_f16(const vmi_gpt2_prompts* a, void* stream);
+/* Whether it takes the products of num_tokens tokens in all to tiles behind norms of their own (0: the few-row kernels) */
+VMI_LAYER_API int32_t vmi_gpt2_prompts_in_tiles(int32_t num_tokens, int32_t hidden);
 
 /* Scheduler.sample_next_token (vllmini/scheduler.py:144-153: logits / temperature, top-k, softmax, one multinomial draw) for a
  * batch of rows in one launch: out[r] = the index drawn from softmax(top_k largest of logits[r, :] / temperature), the draw made by

@@ -860,6 +860,31 @@ def test_prompts_take_tiles_from_fewer_rows_still_past_a_width_of_768(H, D, T):
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
 
 
+LINES = [(128, 4800), (192, 3200), (256, 1760), (320, 912), (384, 768), (448, 656), (512, 576), (576, 448), (640, 400), (704, 368), (768, 336), (832, 144), (896, 144), (960, 128),
+         (1024, 128), (1088, 112), (1152, 112)]      # width, the most tokens that the few-row kernels are measured ahead or level for
+
+
+def test_prompts_take_tiles_where_the_few_row_kernels_fall_behind():
+    """The rule against both sides as measured: the line, and points of either side that a line over T E alone has got wrong."""
+    from vllmini_amd import gpt2_layer as gl
+
+    tiles = gl.load().vmi_gpt2_prompts_in_tiles
+    for E, T in LINES:
+        assert not tiles(T, E) and tiles(T + 16, E), (E, T)
+    for T, E in ((1600, 256), (2400, 192), (4000, 128), (120, 960), (124, 1024), (100, 1152)):
+        assert not tiles(T, E), (T, E)
+    for T, E in ((1100, 320), (850, 384), (500, 576), (450, 640), (160, 832), (130, 960), (130, 1024), (128, 1088)):
+        assert tiles(T, E), (T, E)
+    assert not tiles(8192, 64) and not tiles(4000, 800) and not tiles(4000, 1216) and not tiles(0, 768)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,T", [(E, T + d) for E, T in LINES if E in (192, 256, 512, 640, 768, 896, 1024, 1152) for d in (0, 1)])
+def test_prompts_on_both_sides_of_the_line_to_tiles(E, T):
+    """As test_prompts_of_many_rows_..., where the kernels change."""
+    test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(E // 64, 64, T)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("head,rows,ld,used,n", [(0, 0, 0, 0, 1), (16, 3, 5, 5, 0), (4080, 1, 64, 1, 0), (4096, 384, 64, 13, 32), (48, 7, 9, 0, 300), (1 << 20, 1000, 33, 32, 5)])
 def test_a_steps_inputs_go_where_its_launches_read_them(head, rows, ld, used, n):

@@ -845,11 +845,19 @@ static int run_rows(const LinearParams& p, bool ln, int epi, hipStream_t stream)
   return nks <= 128 ? launch_plain_rows<16, 8>(p, ns, stream) : launch_plain_rows<16, 9>(p, ns, stream);
 }
 
-// Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every tile, so they
-// are ahead while rows are few, and the wider the rows the sooner they fall behind; six launches a layer for four are what narrow ones wait for.  12 layers of prompts of 100 tokens
-// in us, few-row kernels / tiles, width 256 1600 tokens 541 / 605; 512 500 437 / 496, 600 579 / 508; 768 300 526 / 554, 350 588 / 584, 400 658 / 580; 1024 130 649 / 614, 160
-// 658 / 637, 200 730 / 634; 1152 130 703 / 706, 160 779 / 723.
-static bool many_rows(int T, int E) { return (int64_t)T * E >= (E > 768 ? 150000 : E > 640 ? 270000 : E > 384 ? 300000 : 390000) && E % 64 == 0 && 4 * E <= 4608; }
+// Whether prompts of T rows take tiles_kernel behind norms of their own.  The few-row kernels read their weights and norm their rows again for every 16 rows, and
+// take a step up where the 16 x 16 blocks of a product of E columns no longer fit the compute units at so many each: two past E = 768, four up to there; from that
+// step on tiles are ahead.  Narrower models wait for launches, six a layer for four, so their lines lie further out.
+// 12 layers of prompts of 100 tokens, few-row kernels / tiles in us, on both sides of each line:
+//   E 1152  T 112 574 / 687, 120 680 / 704, 136 699 / 707, 152 776 / 712     E 1088  T 112 596 / 683, 120 713 / 694      E 1024  T 128 507 / 616, 129 663 / 615
+//   E  960  T 128 497 / 609, 129 673 / 608     E 896  T 144 555 / 586, 152 640 / 598     E 832  T 144 528 / 576, 152 624 / 588
+//   E  768  T 336 524 / 566, 344 584 / 571     E 704  T 368 533 / 541, 384 576 / 542     E 640  T 400 541 / 535, 408 591 / 541     E 576  T 448 510 / 504, 456 557 / 521
+//   E  512  T 576 498 / 531, 592 580 / 506     E 448  T 656 497 / 535, 680 577 / 522     E 384  T 752 525 / 531, 776 532 / 518     E 320  T 896 530 / 534, 928 544 / 545, 1064 569 / 564
+//   E  256  T 1752 648 / 718, 1800 753 / 725   E 192  T 2728 797 / 913, 3248 969 / 921   E 128  T 4592 1032 / 1052, 5096 1095 / 1094
+static bool many_rows(int T, int E) {
+  const int64_t blocks = (int64_t)(E >> 4) * ((T + 15) >> 4);
+  return blocks > (E > 768 ? 512 : E > 512 ? 1024 : E > 256 ? 1152 : E > 192 ? 1760 : 2400) && E % 64 == 0 && 4 * E <= 4608;
+}
 
 template <int I, int EPI>
 static int launch_tiles(const LinearParams& p, hipStream_t stream) {
@@ -1117,6 +1125,8 @@ int vmi_gpt2_linear_tiles_f16(const void* x, const void* w, const void* bias, co
   if (prev != device) (void)hipSetDevice(prev);
   return rc;
 }
+
+int32_t vmi_gpt2_prompts_in_tiles(int32_t T, int32_t hidden) { return T > 0 && hidden > 0 && vmi_layer::many_rows(T, hidden); }
 
 int32_t vmi_gpt2_head_fits(int32_t M, int32_t K) {
   using namespace vmi_layer;

@@ -50,6 +50,7 @@ SIGNATURES = {
     "vmi_gpt2_linear_tiles_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_add_norm_f16": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp, ctypes.c_float, _vp, _i32, _i32, _i32, _vp]),
     "vmi_gpt2_prompts_f16": (ctypes.c_int, [ctypes.POINTER(Prompts), _vp]),
+    "vmi_gpt2_prompts_in_tiles": (_i32, [_i32, _i32]),
     "vmi_gpt2_argmax_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_gpt2_sample_top_k_f16": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, ctypes.c_float, _vp, _vp, _i32, _vp]),
     "vmi_gpt2_linear_kernel_name": (ctypes.c_char_p, [_i32, _i32, _i32, _i32, _i32]),
