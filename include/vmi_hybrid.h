@@ -66,6 +66,8 @@ VMI_HY_API int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream);
 VMI_HY_API int vmi_hy_linear_tiles(const vmi_hy_linear_args* a, void* stream);
 /* Whether it takes such a product (rows of K elements one behind the other) and is ahead of a library product and vmi_hy_glu behind it */
 VMI_HY_API int32_t vmi_hy_linear_tiles_pay(int32_t M, int32_t N, int32_t K, int32_t n_split, int32_t dtype);
+/* Whether it does for any number of rows below 4 GiB: then a library product of this matrix is never asked for */
+VMI_HY_API int32_t vmi_hy_linear_tiles_only(int32_t N, int32_t K, int32_t n_split, int32_t dtype);
 /* A product of such rows alone: epilogue E_STORE (bias or none) or E_FLOAT */
 VMI_HY_API int vmi_hy_product_tiles(const vmi_hy_linear_args* a, void* stream);
 /* Whether it takes such a product (rows of x ldx elements apart) and is ahead of a library product */

@@ -314,6 +314,20 @@ def test_the_structs_layouts_belong_to_their_version(tmp_path):
     assert {n: ctypes.sizeof(c) for n, c in py.items()} == sizes
 
 
+def test_gated_products_go_to_tiles_but_where_the_library_is_ahead():
+    """The rule against both sides as measured: in the mean of its sizes the library with the unit behind it is ahead in two places past K 7168 only."""
+    from vllmini_amd import hybrid_ops as h
+
+    pay, only = h.load().vmi_hy_linear_tiles_pay, h.load().vmi_hy_linear_tiles_only
+    for M, N, K in ((420, 20480, 8192), (1200, 8192, 16384), (742, 16384, 8192), (76, 2048, 16384), (61, 2816, 8192), (55, 1152, 8960)):
+        assert not pay(M, N, K, 0, h.DTYPES[torch.bfloat16]), (M, N, K)
+    for M, N, K in ((300, 6144, 1024), (4500, 6144, 1024), (948, 40960, 4096), (64, 2048, 6144), (420, 20512, 8192), (300, 16384, 8192), (2773, 8192, 8192), (130, 2048, 16384)):
+        assert pay(M, N, K, 0, h.DTYPES[torch.bfloat16]), (M, N, K)
+    for split in (0, 4096):
+        assert only(20480, 4096, split, 0) and not only(20480, 8192, split, 0) and not only(20480, 4096, split, 1) and not only(20480, 96, split, 0)
+    assert not only(4096, 4096, 4096, 0) and not pay(1 << 20, 4096, 2048, 0, 0) and not pay(0, 4096, 2048, 0, 0)
+
+
 def test_hybrid_entries_refuse_bad_arguments_without_touching_a_device():
     from vllmini_amd import hybrid_ops as h
 

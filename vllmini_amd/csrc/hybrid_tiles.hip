@@ -90,10 +90,7 @@ int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
 }
 
 // Whether tiles of our own end sooner than the library's product (hipBLASLt as PyTorch 2.10.0+rocm7.0 loads it: another version may move the line, never the result beyond the
-// order of a sum).  Measured in bfloat16, 48 to 6000 rows, weights that leave the last cache between two products from K 2048 on and others that stay.
-//
-// With the gated unit behind them always: of 160 pairs (library and unit in a launch of its own / ours) K 1024 to 4096, N 6144 to 45 056, 0.87 of the time in the mean, 1.16 at most.  us: K
-// 1024, N 6144 all gated 300 rows 13.0 / 8.5, 1200 26 / 21, 4500 66 / 58; K 2048, N 20480, 12288 of them gated, 140 rows 35 / 31, 948 98 / 94, 2400 268 / 201.
+// order of a sum).  Measured in bfloat16, weights that leave the last cache between two products from K 2048 on and others that stay.
 //
 // Alone 0.89 in the mean of 502, and not where whole tiles of 256 columns fill the chip more than once (N 2048, K 6144: 2400 rows 74 / 70, 4500 103 / 115; N 4096, K 2048
 // 948 24 / 22, 2400 41 / 46; past K 4096 whatever N is), where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4),
@@ -104,6 +101,19 @@ static bool product_pays(int M, int N, int K) {
   if (K >= 2048 && results >= 5600000 && (whole || K >= 4096)) return false;
   if (K >= 3072 && (least <= 128 || (whole && N >= 2048 && results >= 1050000 && results < 2400000))) return false;
   return K < 16384;
+}
+
+// With the gated unit behind them (library and unit in a launch of its own / ours), 1930 pairs of 48 to 12 000 rows, K 512 to 16 384, N 1024 to 45 056: ours 0.86 of
+// the time (K below 2048 0.74, 4096 0.85, 7168 0.90, beyond 0.95).  By K, results, and whether columns are whole tiles of 256, ours are ahead or level in
+// every class but two past K 7168.  Where few of the smallest tiles walk a long K each 1.13 of 12 (76 rows, N 2048, K 16384 38 / 51), and where the library's largest
+// tiles go round once, more than a third full, 1.03 of 86 (420 rows, N 20480, K 8192 142 / 174; 1200, 8192, 16384 275 / 328).
+// What is left is single pairs that no size explains: below K 4096 8 of 927 are more than 5 per cent behind (1.11 at most), below 7168 45 of 450 (1.22; 6000 rows,
+// N 40960, K 4096 1493 / 1712), beyond 76 of 455 (1.24), beside more of the like that are as far ahead (948, 40960, 4096 363 / 297).
+// us: K 1024, N 6144 all gated 300 rows 13.0 / 8.5, 4500 66 / 58; K 2048, N 20480, 12288 of them gated, 140 rows 35 / 31, 2400 268 / 201.
+static bool gated_whatever_rows(int K) { return K < 7168; }
+static bool gated_pays(int M, int N, int K) {
+  const int64_t results = (int64_t)M * N, least = (int64_t)((M + 31) / 32) * ((N + 63) / 64);
+  return gated_whatever_rows(K) || (least > 128 && !(N % 256 == 0 && results >= 6000000 && results < 15000000));
 }
 
 template <int EPI, int I = 0>
@@ -123,9 +133,15 @@ using namespace vmi_hybrid;
 
 extern "C" {
 
-int32_t vmi_hy_linear_tiles_pay(int32_t M, int32_t N, int32_t K, int32_t n_split, int32_t dtype) {
-  return dtype == VMI_HY_BF16 && M > 0 && N > 0 && K > 0 && n_split >= 0 && n_split < N && ((N | n_split) & 15) == 0 && vmi_tiles::tiles_fit(M, K, K);
+static bool linear_tiles_fit(int32_t N, int32_t K, int32_t n_split, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && N > 0 && K > 0 && n_split >= 0 && n_split < N && ((N | n_split) & 15) == 0 && (K & 63) == 0;
 }
+
+int32_t vmi_hy_linear_tiles_pay(int32_t M, int32_t N, int32_t K, int32_t n_split, int32_t dtype) {
+  return M > 0 && linear_tiles_fit(N, K, n_split, dtype) && vmi_tiles::tiles_fit(M, K, K) && gated_pays(M, N, K);
+}
+
+int32_t vmi_hy_linear_tiles_only(int32_t N, int32_t K, int32_t n_split, int32_t dtype) { return linear_tiles_fit(N, K, n_split, dtype) && gated_whatever_rows(K); }
 
 int vmi_hy_linear_tiles(const vmi_hy_linear_args* a, void* stream) {
   static const char* who = "vmi_hy_linear_tiles";

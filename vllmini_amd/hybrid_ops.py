@@ -71,6 +71,7 @@ SIGNATURES = {
     "vmi_hy_linear": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_linear_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_linear_tiles_pay": (_i32, [_i32, _i32, _i32, _i32, _i32]),
+    "vmi_hy_linear_tiles_only": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_product_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_product_tiles_pay": (_i32, [_i32, _i32, _i32, ctypes.c_int64, _i32]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
@@ -285,6 +286,11 @@ def linear_tiles_pay(M: int, w: MatrixTiles, split: int = 0) -> bool:
 @functools.lru_cache(maxsize=4096)
 def _tiles_pay(M: int, N: int, K: int, split: int, dtype: torch.dtype) -> bool:
     return bool(load().vmi_hy_linear_tiles_pay(M, N, K, split, DTYPES[dtype]))
+
+
+def linear_tiles_only(N: int, K: int, split: int, dtype: torch.dtype) -> bool:
+    """Whether that holds for an [N, K] matrix whatever the rows, below 4 GiB of them."""
+    return bool(load().vmi_hy_linear_tiles_only(N, K, split, DTYPES[dtype]))
 
 
 def product_tiles(x: torch.Tensor, w: MatrixTiles, bias: Optional[torch.Tensor] = None, float_out: bool = False) -> torch.Tensor:
