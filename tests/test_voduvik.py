@@ -328,6 +328,18 @@ def test_gated_products_go_to_tiles_but_where_the_library_is_ahead():
     assert not only(4096, 4096, 4096, 0) and not pay(1 << 20, 4096, 2048, 0, 0) and not pay(0, 4096, 2048, 0, 0)
 
 
+@pytest.mark.parametrize("width,dtype,kept", [(64, torch.bfloat16, False), (96, torch.bfloat16, True), (64, torch.float32, True), (7168, torch.bfloat16, True)])
+def test_gated_matrices_keep_the_librarys_layout_only_where_it_is_asked_for(width, dtype, kept):
+    from vllmini_amd import hybrid_layers as hl
+
+    w = torch.randn((48, width), generator=torch.Generator().manual_seed(width))
+    for m in (hl.gated_matrix(w, dtype), hl.gated_matrix(w, dtype, 16)):
+        assert (m.dense is not None) == kept and (m.N, m.K) == (64, width)
+    norm = hl.Norm(torch.ones(width), width, 1e-5)
+    ff = hl.ClampedGLU(width=width, limit=7.0, norm=norm, gate=w, up=w, down=w.t(), dtype=dtype)
+    assert (ff.w_in.dense is not None) == kept and ff.w_out.dense is not None
+
+
 def test_hybrid_entries_refuse_bad_arguments_without_touching_a_device():
     from vllmini_amd import hybrid_ops as h
 

@@ -399,6 +399,23 @@ def test_products_of_many_rows_alone_refuse_what_is_not_built():
     assert ops.product_tiles_pay(x, t) and not ops.product_tiles_pay(x[:, :96], odd) and not ops.product_tiles_pay(wide[:, 4:132], t) and not ops.product_tiles_pay(x.float(), t)
 
 
+@pytest.mark.parametrize("split", [0, 64])
+def test_gated_rows_past_what_one_launch_takes_go_in_parts(split, monkeypatch):
+    """Without the vendor's layout rows of 4 GiB and more are cut in two until a launch takes them: the same bits."""
+    from vllmini_amd import hybrid_layers as hl, hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(split)
+    w, x = hl.gated_matrix(torch.randn((192, 128), generator=g, device=dev()) / 11, torch.bfloat16, split), torch.randn((333, 128), generator=g, device=dev()).to(torch.bfloat16)
+    runs, pay = [], ops.linear_tiles_pay
+    assert w.dense is None
+    for most in (10 ** 9, 50):
+        monkeypatch.setattr(ops, "linear_tiles_pay", lambda M, w, split=0: M <= most and pay(M, w, split))
+        out = torch.zeros((333, 200), dtype=torch.bfloat16, device=dev())[:, 8:8 + (192 - split) // 2]
+        runs.append((hl.gated_product(x, w, ops.SILU_UNIT, split, out), hl.gated_product(x, w, ops.SILU_UNIT, split), out))
+    assert all(torch.equal(a, b) for a, b in zip(*runs)) and bool(runs[0][2].any())
+    assert hl.gated_product(x[:0], w, ops.SILU_UNIT, split).shape == (0, split or 96)
+
+
 def test_many_rows_in_tiles_refuse_what_is_not_built():
     from vllmini_amd import hybrid_ops as ops
 

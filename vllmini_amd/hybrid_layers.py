@@ -291,10 +291,21 @@ class RGLRU:
         res.branch_out(o, self.w_o, step)
 
 
+def gated_matrix(weight: torch.Tensor, dtype: torch.dtype, split: int = 0) -> MatrixTiles:
+    """The matrix of a gated_product; with the vendor's layout beside the tiles only where that product may be asked for (201 MB a matrix of 24576 x 4096)."""
+    N, K = (pad32(n) for n in weight.shape)
+    return MatrixTiles(weight, dtype, dense=dtype != torch.bfloat16 or not ops.linear_tiles_only(N, K, split, dtype))
+
+
 def gated_product(h: torch.Tensor, w: MatrixTiles, unit: GatedUnit, split: int = 0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """h W^T of many rows, the columns from `split` on through the gated unit (into `out`); the columns below, or with split = 0 the unit's."""
     if ops.linear_tiles_pay(h.shape[0], w, split):
         return ops.linear_tiles(h, w, unit, split, out)
+    if w.dense is None:      # (rows of 4 GiB and more: in two)
+        M = h.shape[0]
+        cuts = ((0, M // 2), (M // 2, M)) if M > 1 else ()
+        parts = [gated_product(h[a:b], w, unit, split, None if out is None else out[a:b]) for a, b in cuts] or [h.new_empty((0, split or w.N // 2))]
+        return out if out is not None and not split else torch.cat(parts)
     proj = F.linear(h, w.dense)
     gated = ops.glu(proj[:, split:], unit, out=out)
     return proj if split else gated
@@ -308,7 +319,7 @@ class ClampedGLU:
         E, ff = pad32(width), gate.shape[0]
         self.unit, self.norm = GatedUnit.clamped(limit), norm
         fp = pad32(ff)
-        self.w_in = MatrixTiles(interleaved(gate, up, E), dtype, dense=True)
+        self.w_in = gated_matrix(interleaved(gate, up, E), dtype)
         self.w_out = MatrixTiles(spread(spread(down, 1, torch.arange(ff), fp), 0, torch.arange(width), E), dtype, dense=True)
 
     def run(self, res: Residual, step: StepLayout) -> None:
@@ -524,7 +535,7 @@ class ParallelBlock:
         self.ff = 0 if gate is None else pad32(gate.shape[0])
         tail = [] if gate is None else [padded_rows(padded_rows(down, self.ff, 1), E)]
         outs = [padded_rows(w, E) for w in mixer.outs]
-        self.w_in = MatrixTiles(rows if gate is None else torch.cat([rows, interleaved(gate, up, E)]), dtype, dense=True)
+        self.w_in = MatrixTiles(rows, dtype, dense=True) if gate is None else gated_matrix(torch.cat([rows, interleaved(gate, up, E)]), dtype, self.n_in)
         groups = [[*outs, *tail]] if len(outs) == 1 else [[w] for w in (*outs, *tail)]
         self.w_out = [MatrixTiles(torch.cat(g, dim=1), dtype, dense=True) for g in groups]
         del mixer.in_weight, mixer.outs      # (they live on in the tiles)
