@@ -72,6 +72,8 @@ VMI_HY_API int32_t vmi_hy_linear_tiles_only(int32_t N, int32_t K, int32_t n_spli
 VMI_HY_API int vmi_hy_product_tiles(const vmi_hy_linear_args* a, void* stream);
 /* Whether it takes such a product (rows of x ldx elements apart) and is ahead of a library product */
 VMI_HY_API int32_t vmi_hy_product_tiles_pay(int32_t M, int32_t N, int32_t K, int64_t ldx, int32_t dtype);
+/* The place in their list of the tile that a product of these sizes takes; -1: tiles do not take it, or, of a group of matrices, leave it to the kernels of few rows */
+VMI_HY_API int32_t vmi_hy_tiles_pick(int32_t M, int32_t N, int32_t K, int32_t groups);
 /* Whether a product of these sizes behind a norm is faster over rows normed beforehand (`normed`) */
 VMI_HY_API int32_t vmi_hy_linear_normed(int32_t M, int32_t N, int32_t K, int32_t groups, int32_t dtype);
 /* Whether the rows of a product of these sizes behind a norm can stay in LDS, normed on their way there: then the product is ahead of a norm, a library

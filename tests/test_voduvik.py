@@ -328,6 +328,17 @@ def test_gated_products_go_to_tiles_but_where_the_library_is_ahead():
     assert not only(4096, 4096, 4096, 0) and not pay(1 << 20, 4096, 2048, 0, 0) and not pay(0, 4096, 2048, 0, 0)
 
 
+def test_groups_go_to_tiles_but_where_all_run_at_once_over_a_short_k():
+    """The rule against both sides as measured."""
+    from vllmini_amd import hybrid_ops as h
+
+    pick = h.load().vmi_hy_tiles_pick
+    for M, N, K, groups in ((2260, 128, 512, 8), (879, 128, 512, 16), (366, 128, 512, 32), (1312, 160, 448, 10), (1628, 96, 192, 16), (900, 4096, 192, 2), (97, 512, 128, 16)):
+        assert pick(M, N, K, groups) >= 0, (M, N, K, groups)
+    for M, N, K, groups in ((177, 512, 128, 32), (354, 2048, 64, 4), (1365, 1024, 128, 2), (220, 4096, 192, 2), (864, 256, 64, 12), (1100, 512, 128, 3), (64, 512, 128, 16), (300, 512, 96, 16), (300, 520, 128, 16)):
+        assert pick(M, N, K, groups) == -1, (M, N, K, groups)
+
+
 @pytest.mark.parametrize("width,dtype,kept", [(64, torch.bfloat16, False), (96, torch.bfloat16, True), (64, torch.float32, True), (7168, torch.bfloat16, True)])
 def test_gated_matrices_keep_the_librarys_layout_only_where_it_is_asked_for(width, dtype, kept):
     from vllmini_amd import hybrid_layers as hl

@@ -63,14 +63,20 @@ __global__ __launch_bounds__(256, 2) void group_tiles_kernel(const vmi_hy_linear
       });
 }
 
-// Whether a group's products go to tiles: whole chunks of K, what the tiles' loads are aligned to, and more rows than plain_rows_kernel takes.  linear_kernel / tiles, us: 16 groups of K 128, N
-// 512 97 / 300 / 900 / 2773 rows 4.0 / 5.3 / 12.1 / 28.7 -> 3.5 / 5.2 / 10.0 / 24.4, of K 512, N 128 4.7 / 5.3 / 9.7 / 27.6 -> 3.8 / 5.4 / 8.4 / 18.9; 32 groups, 2773 rows 51 / 44 -> 45 / 30; 2 of
-// K 192, N 4096 900 13.2 -> 10.9.  (All ten groups below 65 rows: 2.4 - 2.9 -> 2.9 - 3.8.)  Not where tiles of 64 x 64 are just more than the chip has compute units for: 200 rows, 16 groups of K 128, N 512 4.6 / 4.9; 300,
-// 2 of K 192, N 4096 6.3 / 6.8; 500, 32 of K 512, N 128 11.6 / 12.0.
+// Whether a group's products go to tiles: whole chunks of K, what the tiles' loads are aligned to, and more rows than plain_rows_kernel takes (all of ten groups below 65
+// rows: 2.4 - 2.9 -> 2.9 - 3.8 us).  Not where K is four chunks at most and all tiles run at once, 64 rows or more each: nothing is beside a tile's ends then, and
+// linear_kernel deals the rows finer.  Both over 246 products of 19 groups (2 to 64 matrices, K 64 to 512, N 64 to 4096, 65 to 4500 rows): this rule 0.1 per cent
+// behind the better side in the mean, 4 at most; tiles always 1.2 and 14.  linear_kernel / tiles, us: 16 groups of K 128, N 512 97 / 300 / 900 / 2773 rows 4.0 / 5.3 / 12.1 / 28.7 -> 3.5 / 5.2 / 10.0
+// / 24.4; of K 512, N 128 879 / 2773 8.8 / 27.6 -> 7.2 / 18.9; 8 of K 512, N 128 2260 11.1 -> 8.4; 2 of K 192, N 4096 900 13.2 -> 10.9.  Where the rule declines: 32 of K 128, N 512 177 rows 5.5 / 6.2; 4 of
+// K 64, N 2048 354 5.4 / 6.2; 2 of K 192, N 4096 220 5.4 / 6.0.
+static bool group_tiles_ahead(int M, int N, int K, int groups) {
+  if (M <= 64) return false;
+  const vmi_tiles::Tile& t = vmi_tiles::TILES[vmi_tiles::tiles_pick(M, N, K, groups)];
+  return !(K <= 256 && t.mi >= 4 && (int64_t)vmi_tiles::tiles_grid(t, M, N) * groups <= 256);
+}
 bool group_tiles_fit(const vmi_hy_linear_args& p) {
-  const int64_t results = (int64_t)p.M * p.N * p.groups;
-  return p.groups > 1 && p.groups < 65536 && p.M > 64 && (results < 1300000 || results >= 2600000) && (p.N & 15) == 0 && (p.ldx & 7) == 0 && (p.x_gstride & 7) == 0 && p.x_gstride >= 0 && ((uintptr_t)p.x & 15) == 0 &&
-         ((uintptr_t)p.w & 15) == 0 && vmi_tiles::tiles_fit(p.M, p.K, p.ldx);
+  return p.groups > 1 && p.groups < 65536 && (p.N & 15) == 0 && (p.ldx & 7) == 0 && (p.x_gstride & 7) == 0 && p.x_gstride >= 0 && ((uintptr_t)p.x & 15) == 0 &&
+         ((uintptr_t)p.w & 15) == 0 && vmi_tiles::tiles_fit(p.M, p.K, p.ldx) && group_tiles_ahead(p.M, p.N, p.K, p.groups);
 }
 
 template <int EPI, int I = 0>
@@ -142,6 +148,11 @@ int32_t vmi_hy_linear_tiles_pay(int32_t M, int32_t N, int32_t K, int32_t n_split
 }
 
 int32_t vmi_hy_linear_tiles_only(int32_t N, int32_t K, int32_t n_split, int32_t dtype) { return linear_tiles_fit(N, K, n_split, dtype) && gated_whatever_rows(K); }
+
+int32_t vmi_hy_tiles_pick(int32_t M, int32_t N, int32_t K, int32_t groups) {
+  if (M <= 0 || N <= 0 || K <= 0 || groups <= 0 || (N & 15) || !vmi_tiles::tiles_fit(M, K, K)) return -1;
+  return groups == 1 || group_tiles_ahead(M, N, K, groups) ? vmi_tiles::tiles_pick(M, N, K, groups) : -1;
+}
 
 int vmi_hy_linear_tiles(const vmi_hy_linear_args* a, void* stream) {
   static const char* who = "vmi_hy_linear_tiles";

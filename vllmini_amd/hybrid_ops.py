@@ -74,6 +74,7 @@ SIGNATURES = {
     "vmi_hy_linear_tiles_only": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_product_tiles": (ctypes.c_int, [ctypes.POINTER(LinearArgs), _vp]),
     "vmi_hy_product_tiles_pay": (_i32, [_i32, _i32, _i32, ctypes.c_int64, _i32]),
+    "vmi_hy_tiles_pick": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_normed": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_linear_resident": (_i32, [_i32, _i32, _i32, _i32]),
     "vmi_hy_linear_slabs": (_i32, [_i32, _i32, _i32, _i32]),
