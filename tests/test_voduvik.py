@@ -328,6 +328,17 @@ def test_gated_products_go_to_tiles_but_where_the_library_is_ahead():
     assert not only(4096, 4096, 4096, 0) and not pay(1 << 20, 4096, 2048, 0, 0) and not pay(0, 4096, 2048, 0, 0)
 
 
+def test_products_alone_go_to_tiles_but_where_the_library_is_ahead():
+    """The rule against both sides as measured."""
+    from vllmini_amd import hybrid_ops as h
+
+    pay = lambda M, N, K: h.load().vmi_hy_product_tiles_pay(M, N, K, K, h.DTYPES[torch.bfloat16])      # noqa: E731
+    for M, N, K in ((7455, 2048, 1024), (5251, 3072, 1536), (3985, 6400, 1728), (4000, 6400, 1024), (4500, 2048, 6144), (2400, 4096, 2048), (64, 2048, 6144), (300, 4096, 8192), (48, 64, 16384)):
+        assert not pay(M, N, K), (M, N, K)
+    for M, N, K in ((3719, 2048, 1024), (3564, 2048, 1024), (7455, 2080, 1024), (5274, 1792, 768), (2300, 2048, 2048), (2400, 2080, 3072), (1300, 2048, 6144), (48, 512, 512)):
+        assert pay(M, N, K), (M, N, K)
+
+
 def test_groups_go_to_tiles_but_where_all_run_at_once_over_a_short_k():
     """The rule against both sides as measured."""
     from vllmini_amd import hybrid_ops as h
