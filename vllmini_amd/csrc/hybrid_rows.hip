@@ -509,7 +509,6 @@ static int held_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
     case 1024 * 4 + 2: return held_rows_of<1, 2, 6, EPI>(p, st);
     case 2048 * 4 + 1: return held_rows_of<2, 1, 6, EPI>(p, st);
     case 2048 * 4 + 2: return held_rows_of<2, 2, 6, EPI>(p, st);
-    case 3072 * 4 + 1: return held_rows_of<3, 1, 6, EPI>(p, st);
     case 3072 * 4 + 2: return held_rows_of<3, 2, 6, EPI>(p, st);
     case 4096 * 4 + 1: return held_rows_of<4, 1, 4, EPI>(p, st);
     case 4096 * 4 + 2: return held_rows_of<4, 2, 4, EPI>(p, st);
