@@ -306,6 +306,20 @@ def test_few_rows_side_by_side(M, N, K):
     close(got, 0.5 * want[:, :N - 3], torch.bfloat16, tol16=1e-5)      # (products of 16 bits are exact in 32: what is left is the order of a float32 sum)
 
 
+@pytest.mark.parametrize("K", [10240, 14336, 16384])
+@pytest.mark.parametrize("M,slabs", [(1, 3), (2, 512), (8, 130), (9, 66), (16, 384), (17, 96)])
+def test_rows_as_they_are_over_every_number_of_whole_chunks(M, slabs, K):
+    """As above over the other multiples of 2048 up to 16 384; two float32 halves side by side too."""
+    from vllmini_amd import hybrid_ops as ops
+
+    test_rows_as_they_are_over_whole_chunks(M, slabs, K)
+    g = torch.Generator(device=dev()).manual_seed(M + K)
+    a, b, w = (torch.randn(*s, generator=g, device=dev()) for s in ((M, K // 2), (M, K // 2), (16 * slabs + 16 * (slabs & 1), K)))
+    w = (w / K ** 0.5).to(torch.bfloat16)
+    want = torch.cat([a, b], 1).to(torch.bfloat16).double() @ w.double().T
+    close(ops.linear(a, ops.MatrixTiles(w, torch.bfloat16), x2=b, float_out=(16 * slabs, 1.0)), want[:, :16 * slabs], torch.bfloat16, tol16=1e-5)
+
+
 def _norm_products(M, N, K):
     """Every epilogue behind a norm against float64, the norm over fewer columns than there are; returns the weights."""
     from vllmini_amd import hybrid_ops as ops

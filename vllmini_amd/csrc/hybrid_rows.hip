@@ -534,7 +534,22 @@ int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 // chunks follow each other: K 5120, N 6144 1 / 32 / 64 rows 12.6 / 15.1 / 22.0 -> 14.7 / 18.5 / 29.6, N 1024 16 rows 7.1 -> 7.6 (K 6144 7.9 -> 7.8, N 2048 8.5 -> 8.6), N 4096 10.4 -> 9.9; K 12288, N 6144 64 rows 66 -> 57.
 // Whole chunks (a form of its own, see plain_rows_kernel) keep more on their way: linear_kernel / here, K 6144, N 2048 1 / 16 rows 9.9 / 10.9 -> 7.8 / 9.5, N 6144 18.2 / 22.1 -> 16.3 / 20.8, N 8192 1 / 8 /
 // 16 rows 22.2 / 22.5 / 22.8 -> 19.9 / 20.7 / 23.6; K 8192, N 2048 11.0 / 14.0 -> 8.5 / 11.6, N 8192 28.2 / 28.1 -> 26.1 / 28.4; K 12288, N 2048 14.3 / 18.4 -> 11.7 / 16.0, N 6144 32.2 / 38.8 -> 30.4 / 37.3.
-static bool whole_chunks(int K) { return K == 6144 || K == 8192 || K == 12288; }
+// Every K of whole chunks for eight waves has it; of the others (us, the form that waits for all loads at every chunk, or linear_kernel past its line / here) K 10240, N 2048 1 / 8 / 16 rows
+// 12.5 / 14.0 / 16.1 -> 10.3 / 12.5 / 14.5, N 8192 1 / 8 32.2 / 32.8 -> 30.2 / 31.6; K 14336, N 2048 16.2 / 18.1 / 21.0 -> 13.6 / 16.4 / 18.7; K 16384, N 4096 28.4 / 29.1 / 30.2 -> 25.9 / 26.8 / 28.8,
+// N 7168 44.5 / 45.3 / 46.1 -> 44.0 / 47.0 / 46.0, N 8192 50.4 / 51.0 / 51.5 -> 49.8 / 51.3 / 51.4.  (Longer ones are not measured.)
+static bool whole_chunks(int K) { return K % 2048 == 0 && K >= 6144 && K <= 16384; }
+
+template <class F>
+static int with_chunks(int K, F&& launch_with) {   // K: whole_chunks
+  switch (K >> 11) {
+    case 3: return launch_with(std::integral_constant<int, 3>{});
+    case 4: return launch_with(std::integral_constant<int, 4>{});
+    case 5: return launch_with(std::integral_constant<int, 5>{});
+    case 6: return launch_with(std::integral_constant<int, 6>{});
+    case 7: return launch_with(std::integral_constant<int, 7>{});
+    default: return launch_with(std::integral_constant<int, 8>{});
+  }
+}
 
 bool plain_rows_fit(int M, int N, int K, int groups) {
   const int64_t slabs = (int64_t)(N >> 4) * groups;
@@ -574,10 +589,7 @@ static int plain_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
       if (p.M <= 8) return go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 4>, 8, 8, 1);
       return go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 8>, 8, 8, 1);
     };
-    if (whole_chunks(p.K)) {
-      if (p.K == 6144) return whole(std::integral_constant<int, 3>{});
-      return p.K == 8192 ? whole(std::integral_constant<int, 4>{}) : whole(std::integral_constant<int, 6>{});
-    }
+    if (whole_chunks(p.K)) return with_chunks(p.K, whole);
     return go(plain_rows_kernel<8, 8, 1, 3, EPI>, 8, 8, 1);
   }
   if (nks <= 4) return go(plain_rows_kernel<4, 1, 2, 1, EPI>, 4, 1, 2);
@@ -589,7 +601,7 @@ static int plain_rows_epi(const vmi_hy_linear_args& p, hipStream_t st) {
 }
 
 // linear_kernel / here, us, weights not in the Infinity Cache: K 512, N 256 1 / 16 rows 3.5 / 4.4 -> 2.1 / 2.4, K 2048, N 1024 4.5 / 5.8 -> 3.3 / 4.1, N 4096 7.5 / 10.3 -> 5.7 / 6.7; K 4096, N 2048 8.3 / 12.0 -> 6.4 / 8.9; K 8192, N
-// 4096 1 / 8 19.0 / 25.0 -> 15.2 / 16.7, K 12288, N 6144 34.9 / 46.6 -> 31.5 / 38.3.  (Past 16 rows linear_kernel, as before.)
+// 4096 1 / 8 19.0 / 25.0 -> 15.2 / 16.7, K 12288, N 6144 34.9 / 46.6 -> 31.5 / 38.3; K 10240, N 5120 26.2 / 36.7 -> 23.5 / 29.4, K 16384, N 8192 53.8 / 65.7 -> 51.0 / 55.0.  (Past 16 rows linear_kernel, as before.)
 bool concat_rows_fit(int M, int N, int K) {
   if (M > 16) return false;
   return whole_chunks(K) ? M <= 8 && N <= 16 * 512 : K <= 4608 && plain_rows_fit(M, N, K, 1);   // (registers hold four requests of float32 rows three chunks ahead, not eight)
@@ -608,8 +620,7 @@ int launch_concat_rows(const vmi_hy_linear_args& p, hipStream_t st) {
     constexpr int NCH = decltype(chunks)::value;
     return p.M <= 2 ? go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 1, XK>, 8, 8) : go(plain_rows_kernel<8, 8, 1, 3, EPI, NCH, 4, XK>, 8, 8);
   };
-  if (p.K == 6144) return whole(std::integral_constant<int, 3>{});
-  return p.K == 8192 ? whole(std::integral_constant<int, 4>{}) : whole(std::integral_constant<int, 6>{});
+  return with_chunks(p.K, whole);
 }
 
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
