@@ -29,6 +29,7 @@ extern "C" {
 #define VMI_LAYER_API
 #endif
 
+/* The layouts of the structs below and the arguments of the entries that are there; an entry that comes leaves it, and a caller finds a library without it by its name */
 #define VMI_GPT2_LAYER_ABI_VERSION 1
 
 enum {

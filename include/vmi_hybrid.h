@@ -23,6 +23,7 @@ extern "C" {
 #endif
 
 #define VMI_HY_API __attribute__((visibility("default")))
+/* The layouts of the structs below and the arguments of the entries that are there; an entry that comes leaves it, and a caller finds a library without it by its name */
 #define VMI_HYBRID_ABI_VERSION 3
 
 enum { VMI_HY_OK = 0, VMI_HY_E_ARG = 1, VMI_HY_E_SHAPE = 2, VMI_HY_E_HIP = 3 };

@@ -293,6 +293,27 @@ def test_hybrid_library_exports_its_header_and_nothing_else():
     assert lib.vmi_hybrid_abi_version() == hybrid_ops.ABI_VERSION and lib.vmi_hybrid_target_arch() == b"gfx950"
 
 
+@pytest.mark.parametrize("module,error", [("hybrid_ops", "HybridLibraryError"), ("gpt2_layer", "LayerLibraryError")])
+def test_a_library_of_older_sources_is_named_with_what_to_do(module, error, monkeypatch, tmp_path):
+    """One of the same version that lacks an entry which came since (its struct layouts are right), and one of another version."""
+    import importlib
+
+    from vllmini_amd import build
+
+    m = importlib.import_module(f"vllmini_amd.{module}")
+    version = next(n for n in m.SIGNATURES if n.endswith("abi_version"))
+    late = sorted(set(m.SIGNATURES) - {version})
+    for left_out, number, words in ((late[-1], m.ABI_VERSION, f"does not export {late[-1]}"), (None, m.ABI_VERSION + 1, f"expected {m.ABI_VERSION}")):
+        src, lib = tmp_path / f"{number}.c", tmp_path / f"{number}.so"
+        src.write_text("".join(f"int {n}(void) {{ return {number if n == version else 0}; }}\n" for n in m.SIGNATURES if n != left_out))
+        subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+        monkeypatch.setattr(build, "HYBRID_LIB_PATH" if module == "hybrid_ops" else "LAYER_LIB_PATH", str(lib))
+        monkeypatch.setattr(m, "_lib", None)
+        with pytest.raises(getattr(m, error), match=words) as e:
+            m.load()
+        assert "python -m vllmini_amd.build" in str(e.value) and str(lib) in str(e.value)
+
+
 def test_the_structs_layouts_belong_to_their_version(tmp_path):
     """A caller knows a struct by its version number alone: a field that comes or moves takes a new one (3: `normed` in vmi_hy_linear_args).  The sizes as
     the C header has them, as the ctypes side has them, and as recorded for the version."""

@@ -85,10 +85,10 @@ def load() -> ctypes.CDLL:
                     try:
                         fn = getattr(lib, name)
                     except AttributeError as e:
-                        raise LayerLibraryError(f"{path} does not export {name}") from e
+                        raise LayerLibraryError(f"{path} does not export {name}: it is of older sources, build it with `python -m vllmini_amd.build` (or `make layer`)") from e
                     fn.restype, fn.argtypes = restype, argtypes
                 if lib.vmi_gpt2_layer_abi_version() != ABI_VERSION:
-                    raise LayerLibraryError(f"{path}: ABI {lib.vmi_gpt2_layer_abi_version()}, expected {ABI_VERSION}")
+                    raise LayerLibraryError(f"{path}: ABI {lib.vmi_gpt2_layer_abi_version()}, expected {ABI_VERSION}: build it with `python -m vllmini_amd.build` (or `make layer`)")
                 _lib = lib
     return _lib
 

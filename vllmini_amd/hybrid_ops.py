@@ -128,10 +128,10 @@ def load() -> ctypes.CDLL:
                     try:
                         fn = getattr(lib, name)
                     except AttributeError as e:
-                        raise HybridLibraryError(f"{path} does not export {name}") from e
+                        raise HybridLibraryError(f"{path} does not export {name}: it is of older sources, build it with `python -m vllmini_amd.build` (or `make hybrid`)") from e
                     fn.restype, fn.argtypes = restype, argtypes
                 if lib.vmi_hybrid_abi_version() != ABI_VERSION:
-                    raise HybridLibraryError(f"{path}: ABI {lib.vmi_hybrid_abi_version()}, expected {ABI_VERSION}")
+                    raise HybridLibraryError(f"{path}: ABI {lib.vmi_hybrid_abi_version()}, expected {ABI_VERSION}: build it with `python -m vllmini_amd.build` (or `make hybrid`)")
                 _lib = lib
     return _lib
 
