@@ -14,6 +14,8 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from tests import tile_cases
+
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -797,8 +799,8 @@ def test_the_norm_in_front_holds_rows_whose_mean_is_far_from_zero(M, K):
 @pytest.mark.parametrize("M,N,K", [(1, 16, 64), (17, 80, 128), (300, 3088, 320), (1063, 5408, 192), (770, 5392, 128), (1442, 6160, 128), (641, 5920, 576), (323, 5424, 832),
                                    (481, 5392, 64), (130, 5472, 768), (129, 5552, 1984), (2100, 768, 3072)])
 def test_products_of_many_rows_in_tiles(M, N, K):
-    """tiles_kernel, all nine tiles of its list (128 x 256, 128 x 192, 96 x 256, 96 x 192, 96 x 128, 128 x 128, 64 x 128, and K in two halves 64 x 128 and 64 x 64): rows and
-    columns left over, one chunk of K, an odd number of them, halves of unequal length; every epilogue, the residual in place."""
+    """tiles_kernel: rows and columns left over, one chunk of K, two, an odd number of them and many; every epilogue.  (Which tile runs is the rule's: test_each_tile_by_itself goes
+    through their list.)"""
     from vllmini_amd import gpt2_layer as gl
 
     dev = torch.device("cuda:0")
@@ -816,14 +818,15 @@ def test_products_of_many_rows_in_tiles(M, N, K):
                                    (193, 7056, 64), (199, 7008, 256), (132, 6624, 576), (130, 6736, 640), (194, 7136, 192), (70, 5456, 512), (67, 5456, 576), (66, 5968, 640),
                                    (68, 5536, 448), (1, 32, 384), (8, 16, 64), (5, 32, 512), (1, 112, 576), (1, 160, 1152), (16, 16, 448), (1, 160, 64), (40, 272, 320)])
 def test_every_tile_with_every_number_of_chunks_left(M, N, K):
-    """tiles_kernel, each tile of its list with each remainder of K's chunks of 64 by the two or four that it has in flight, rows and columns left over.  A chunk that is none adds
-    nothing where the last one holds an infinity: the row that has one is infinite or, where the weight is zero, NaN, and no other row is touched."""
+    """tiles_kernel, rows, columns and chunks of K left over, fewer chunks than are in flight among them.  A chunk that is none adds nothing where the last one holds an infinity: the row that
+    has one is infinite or, where the weight is zero, NaN, and no other row is touched."""
     from vllmini_amd import gpt2_layer as gl
 
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(M + N + K)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
     x, w, b, res = (rnd(M, K) * 1.5 + 0.3).half(), (rnd(N, K) * 0.6 / K ** 0.5).half(), (rnd(N) * 0.1).half(), rnd(M, N).half()
+    w[N // 3, -1] = 0
     packed = gl.pack_weight(w)
     for bias, kw in ((None, {}), (b, {"gelu": True}), (b, {"residual": res})):
         _close(gl.linear_tiles(x, packed, bias, **kw), _chain(x, w, bias, None, kw.get("gelu", False), kw.get("residual")), (M, N, K, sorted(kw)))
@@ -832,7 +835,16 @@ def test_every_tile_with_every_number_of_chunks_left(M, N, K):
     after = gl.linear_tiles(x, packed)
     rest = torch.arange(M, device=dev) != row
     assert torch.equal(after[rest], before[rest])
-    assert torch.equal(after[row], torch.where(w[:, -1] == 0, float("nan"), torch.sign(w[:, -1]) * float("inf")).half()) or bool((w[:, -1] == 0).any())
+    want = torch.where(w[:, -1] == 0, float("nan"), torch.sign(w[:, -1]) * float("inf")).half()
+    assert bool(((after[row] == want) | (after[row].isnan() & want.isnan())).all()) and bool(after[row, N // 3].isnan())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,left", tile_cases.places())
+def test_each_tile_by_itself(tile, left):
+    """As above, the tile of the list with so many chunks of K left behind two rounds of its walk or more: the size is looked up, so the tile runs whatever the costs it is picked by."""
+    M, N, K, _ = tile_cases.size_for(tile, left)
+    test_every_tile_with_every_number_of_chunks_left(M, N, K)
 
 
 @pytest.mark.gpu

@@ -7,6 +7,7 @@ import subprocess
 import msgpack
 import pytest
 
+from tests import tile_cases
 from vllmini_amd import build
 
 PROBE = """
@@ -93,4 +94,12 @@ def test_every_tile_keeps_its_registers_and_its_scalars(lib, kinds, tmp_path):
             walk = code[name][: code[name].rfind("s_barrier")]
             assert "s_barrier" in walk and "execnz" not in walk and "scratch_" not in walk, name
         seen += len(tiles)
-    assert seen == 13 * kinds      # (the list of tiles, a launch of each for every kind of end)
+    assert seen == len(tile_cases.tiles()) * kinds      # (a launch of each for every kind of end)
+
+
+def test_a_size_reaches_every_tile_with_every_number_of_chunks_left():
+    """What the tests on the card run over; a tile that no size reaches has no business in the list."""
+    sizes = {place: tile_cases.size_for(*place) for place in tile_cases.places()}
+    assert all(sizes.values()), [p for p, s in sizes.items() if s is None]
+    assert len(set(sizes.values())) == len(sizes) == sum(d for _, _, d in tile_cases.tiles())
+    assert all(tile_cases.size_for(i, d, (2, 3, 8, 16, 32)) for i, (_, _, d) in enumerate(tile_cases.tiles()))

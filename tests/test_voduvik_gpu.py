@@ -15,7 +15,7 @@ import torch
 import torch.nn.functional as F
 
 from oracle import voduvik as plain
-from tests import voduvik_cases as cases
+from tests import tile_cases, voduvik_cases as cases
 
 pytestmark = pytest.mark.gpu
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -272,8 +272,8 @@ def test_rows_as_they_are_over_whole_chunks(M, slabs, K):
 @pytest.mark.parametrize("groups,K,N,pad", [(2, 64, 32, 0), (3, 128, 512, 64), (16, 192, 96, 8), (5, 512, 128, 16), (4, 96, 64, 0), (2, 320, 4096, 0)])
 @pytest.mark.parametrize("M", [65, 130, 400, 1100])
 def test_groups_of_many_rows(groups, K, N, pad, M):
-    """group_tiles_kernel, linear_kernel beside its line (few columns more or less, K no whole chunks of 64): groups whose columns of x overlap, stored
-    with a bias and gated, into columns of a wider matrix."""
+    """group_tiles_kernel, linear_kernel past its line (K no whole chunks of 64, short K): groups whose columns of x overlap, stored
+    with a bias and gated, into columns of a wider matrix.  (The list of tiles: test_each_tile_by_itself_over_a_group.)"""
     from vllmini_amd import hybrid_ops as ops
 
     g = torch.Generator(device=dev()).manual_seed(M * K + N)
@@ -350,8 +350,8 @@ def _norm_products(M, N, K):
 @pytest.mark.parametrize("M,N,K,split", [(1, 16, 64, 0), (17, 96, 128, 32), (300, 3088, 320, 16), (1063, 5408, 192, 5408 - 32), (770, 5392, 128, 0), (1442, 6160, 128, 4096), (641, 5920, 576, 48),
                                          (323, 5424, 832, 0), (481, 5392, 64, 2048), (130, 5472, 768, 0), (129, 5552, 1984, 64), (2100, 768, 3072, 256)])
 def test_many_rows_in_tiles_with_the_gated_unit_behind(M, N, K, split):
-    """vmi_hy_linear_tiles, all nine tiles: rows and columns left over, one chunk of K, an odd number of them, halves of unequal length; the line between columns as they
-    are and gated ones inside tiles; outputs that are columns of wider tensors, whose others stay as they were."""
+    """vmi_hy_linear_tiles: rows and columns left over, one chunk of K, two, an odd number of them and many; the line between columns as they
+    are and gated ones inside tiles; outputs that are columns of wider tensors, whose others stay as they were.  (The list of tiles: test_each_tile_by_itself.)"""
     from vllmini_amd import hybrid_ops as ops
 
     g = torch.Generator(device=dev()).manual_seed(M + N + K)
@@ -381,7 +381,7 @@ def test_many_rows_in_tiles_with_the_gated_unit_behind(M, N, K, split):
                                    (257, 6560, 1152), (769, 7616, 128), (391, 6560, 1536), (195, 7104, 128), (199, 7008, 256), (130, 6752, 640), (70, 5472, 512),
                                    (66, 5984, 640), (1, 32, 384), (5, 32, 512), (1, 160, 1152), (1, 160, 64)])
 def test_products_of_many_rows_alone(M, N, K):
-    """vmi_hy_product_tiles, each of its tiles: rows, columns and chunks of K left over, rows of a wider tensor; in bfloat16 with a bias in 32 bits (half a unit of the result) and in
+    """vmi_hy_product_tiles: rows, columns and chunks of K left over, rows of a wider tensor; in bfloat16 with a bias in 32 bits (half a unit of the result) and in
     32 bits (K products summed in another order).  Beside the result nothing is written."""
     from vllmini_amd import hybrid_ops as ops
 
@@ -397,6 +397,24 @@ def test_products_of_many_rows_alone(M, N, K):
         want = y if bias is None else y + b.double()
         got = ops.product_tiles(x, t, bias)
         assert got.dtype == torch.bfloat16 and bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + err + 1e-6).all())
+
+
+@pytest.mark.parametrize("kind", ["alone", "gated", "some gated"])
+@pytest.mark.parametrize("tile,left", tile_cases.places())
+def test_each_tile_by_itself(tile, left, kind):
+    """Each tile of the list with each kind of end, so many chunks of K left behind two rounds of its walk or more: the size is looked up, so the tile runs whatever the costs it is picked by."""
+    M, N, K, _ = tile_cases.size_for(tile, left)
+    if kind == "alone":
+        test_products_of_many_rows_alone(M, N, K)
+    else:
+        test_many_rows_in_tiles_with_the_gated_unit_behind(M, N, K, 0 if kind == "gated" else N // 32 * 16)
+
+
+@pytest.mark.parametrize("tile", range(len(tile_cases.tiles())))
+def test_each_tile_by_itself_over_a_group(tile):
+    """The same of group_tiles_kernel."""
+    M, N, K, groups = tile_cases.size_for(tile, tile_cases.tiles()[tile][2], (2, 3, 8, 16, 32))
+    test_groups_of_many_rows(groups, K, N, 8, M)
 
 
 def test_products_of_many_rows_alone_refuse_what_is_not_built():
