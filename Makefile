@@ -43,13 +43,13 @@ all: $(LIB) $(LAYER_LIB) $(HYBRID_LIB) oracle
 
 hybrid: $(HYBRID_LIB)
 
-$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_linear.hpp $(CSRC)/hybrid_softmax.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp include/vmi_hybrid.h
+$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_linear.hpp $(CSRC)/hybrid_softmax.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp $(CSRC)/lane_ops.hpp include/vmi_hybrid.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $(HYBRID_SRCS) -o $@
 
 layer: $(LAYER_LIB)
 
-$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp $(CSRC)/gpt2_rows.hpp $(CSRC)/gpt2_head.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp include/vmi_gpt2_layer.h
+$(LAYER_LIB): $(CSRC)/gpt2_layer.hip $(CSRC)/gpt2_prompt.hpp $(CSRC)/gpt2_rows.hpp $(CSRC)/gpt2_head.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp $(CSRC)/lane_ops.hpp include/vmi_gpt2_layer.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $< -o $@
 

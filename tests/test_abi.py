@@ -554,3 +554,24 @@ def test_c_abi_is_callable_from_several_host_threads():
     for t in ts:
         t.join()
     assert not errors, errors
+
+
+def test_a_header_that_changes_rebuilds_every_library_that_reads_it():
+    """`make` and vllmini_amd.build name every header of csrc/ that a library's units include, directly or through another."""
+    from vllmini_amd import build
+
+    def read_by(name, seen):
+        for h in re.findall(r'#include "(\w+\.(?:hpp|h|inc))"', open(os.path.join(build.CSRC, name)).read()):
+            if h not in seen and os.path.exists(os.path.join(build.CSRC, h)):
+                seen.add(h)
+                read_by(h, seen)
+        return seen
+
+    make = open(os.path.join(build.REPO_ROOT, "Makefile")).read()
+    for target, units, named in (("$(HYBRID_LIB)", build.SRC_HYBRID, build.HDRS_HYBRID), ("$(LAYER_LIB)", [build.SRC_LAYER], build.HDRS_LAYER), (None, build.SOURCES, build._deps("product"))):
+        wanted = set().union(*(read_by(os.path.basename(u), set()) for u in units))
+        assert wanted and wanted <= {os.path.basename(h) for h in named}, (target, wanted)
+        if target:      # (the other libraries' objects depend on every header)
+            rule = next(ln for ln in make.split("\n") if ln.startswith(target + ":"))
+            assert wanted <= set(re.findall(r"\$\(CSRC\)/(\S+)", rule)), (target, wanted)
+    assert "$(wildcard $(CSRC)/*.hpp)" in make
