@@ -481,13 +481,23 @@ int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   }
 }
 
-// Whether rows that have been normed by a launch of their own go to held_rows_kernel: 9 to 64 of them, whose waves' parts of K are whole chunks, K % 1024 == 0 (a condition around a chunk's products
-// costs the ring), up to the 4096 that registers hold.  Below 4096 columns they are normed for it, where norm_rows_kernel does not take them and resident_kernel, whose workgroups would norm all each, is behind or takes no more than 32; at 4096 norm_first
-// norms them anyway, and a workgroup walks a slab of that length alone: with few slabs the waves of plain_rows_kernel (or linear_kernel, with what it stores gated) end sooner.  Both launches, us, weights not in the
-// Infinity Cache, the other kernels / this one: K 2048, N 12288 8 / 12 / 32 / 40 rows 14.9 / 17.8 / 21.6 / 41.8 -> 14.9 / 15.0 / 17.3 / 17.2, N 20480 19.0 / 22.3 / 26.8 / 47.8 -> 19.9 / 19.9 / 22.2 / 23.5, N 50272 39.4 / 42.3 / 50.4 /
-// 95.1 -> 41.3 / 41.6 / 45.7 / 48.8; K 1024, N 50272 40 rows 49.5 -> 22.1; K 3072, 33 / 47 / 64 rows, N 512 26.2 / 27.2 / 31.7 -> 12.6 / 12.6 / 13.7,
-// N 4096 27.9 / 28.8 / 33.4 -> 14.3 / 14.7 / 16.4, N 24576 57.5 / 57.0 / 58.2 -> 35.2 / 37.2 / 39.0 (9 to 32 rows stay with resident_kernel, which is behind too from N 2048 on: N 6144 16 rows 17.7, 14.3 here); K 4096, N 4096 12.3 / 13.9 / 17.9 -> 13.3 / 17.6 / 16.5 (40 rows gated 27.5 -> 16.9), N 6144 17.9 / 21.1 / 27.7 -> 16.2 / 20.2 / 20.0, N 8192 19.0 / 22.5 /
-// 28.7 -> 19.1 / 23.1 / 23.0 (the walk with its conditions; without them K 1024 to 3072 end 3 to 10 per cent sooner), N 12288 26.6 / 30.4 / 32.8 -> 23.7 / 28.4 / 28.8, N 50272 85.3 / 97.0 / 108 -> 85.5 / 83.2 / 87.7; with weights in that cache N 6144 32 rows 15.5 -> 18.5.
+// Whether rows that have been normed by a launch of their own go to held_rows_kernel: 9 to 64 of them, whose waves' parts of K are whole chunks, K % 1024 == 0 (a condition around a
+// chunk's products costs the ring), up to the 4096 that registers hold.
+//
+// Below 4096 columns rows are normed for it, where norm_rows_kernel does not take them and resident_kernel, whose workgroups would norm all each, is behind or takes
+// no more than 32.  At 4096 norm_first norms them anyway, and a workgroup walks a slab of that length alone: with few slabs the waves of plain_rows_kernel (or
+// linear_kernel, with what it stores gated) end sooner.
+//
+// Both launches, us, weights not in the Infinity Cache, the other kernels / this one (the walk before it lost its conditions, without which K 1024 to 3072 end 3 to 10 per cent sooner):
+//   K 1024  N 50272  40 rows 49.5 / 22.1
+//   K 2048  N 12288   8 14.9 / 14.9   12 17.8 / 15.0   32 21.6 / 17.3   40 41.8 / 17.2
+//           N 20480   8 19.0 / 19.9   12 22.3 / 19.9   32 26.8 / 22.2   40 47.8 / 23.5
+//           N 50272   8 39.4 / 41.3   12 42.3 / 41.6   32 50.4 / 45.7   40 95.1 / 48.8
+//   K 3072  N   512  33 26.2 / 12.6   47 27.2 / 12.6   64 31.7 / 13.7       (9 to 32 rows stay with resident_kernel,
+//           N  4096  33 27.9 / 14.3   47 28.8 / 14.7   64 33.4 / 16.4        which is behind too from N 2048 on:
+//           N 24576  33 57.5 / 35.2   47 57.0 / 37.2   64 58.2 / 39.0        N 6144, 16 rows 17.7, 14.3 here)
+//   K 4096  16 / 24 / 32 rows: N 4096 12.3 / 13.3, 13.9 / 17.6, 17.9 / 16.5 (40 rows gated 27.5 / 16.9)     N 6144 17.9 / 16.2, 21.1 / 20.2, 27.7 / 20.0 (32, weights in that cache, 15.5 / 18.5)
+//           N 8192 19.0 / 19.1, 22.5 / 23.1, 28.7 / 23.0     N 12288 26.6 / 23.7, 30.4 / 28.4, 32.8 / 28.8     N 50272 85.3 / 85.5, 97.0 / 83.2, 108 / 87.7
 bool held_rows_pay(int M, int N, int K, bool stored) {
   if (M < 9 || M > 64 || norm_slabs(M, N, K) > 0) return false;
   if (K == 4096) return M <= 16 ? N >= 6144 : M <= 32 ? N >= 12288 : N >= 4096 || !stored;
@@ -525,18 +535,30 @@ int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   }
 }
 
-// linear_kernel / plain_rows_kernel, in a graph of such launches, us: K 1024, N 1024 1 / 16 / 32 / 64 rows 3.7 / 4.0 / 4.1 / 6.4 -> 2.9 / 3.1 / 3.1 / 3.2, K 3072, N 1024 4.8 / 5.4 / 5.5 / 13.0 ->
-// 3.8 / 4.4 / 4.5 / 4.6, K 8192, N 2048 10.7 / 13.3 / 14.2 / 44.5 -> 10.1 / 12.5 / 12.3 / 15.2, K 4096, N 4096 10.1 / 11.3 / 12.4 / 24.6 -> 8.1 / 9.0 / 10.7 / 17.1, K 12288, N 4096 20.8 / 22.5 / 27.9 /
-// 65.2 -> 20.0 / 21.6 / 25.3 / 41.4; 8 groups of K 128, N 512 3.7 / 3.9 / 4.0 / 3.4 -> 2.3 / 2.4 / 2.5 / 2.6, of K 512, N 128 4.0 / 4.5 / 4.5 / 5.1 -> 2.5 / 2.7 / 2.7 / 2.7.  Of more rows there are tiles.
-// (K 8192 and 12288 before whole chunks had a form of their own: below.)  Every workgroup brings the rows again, so past one slab a compute unit (256) it is ahead only while the rows are few or short: K 2048, N 16384 1 / 32 / 64 rows 13.6 / 13.8 / 16.2 -> 12.7 / 16.8 / 30.8,
-// N 50272 42.8 (1) -> 35.0; K 4096, N 8192 8 / 24 / 64 14.2 / 14.0 / 20.7 -> 13.7 / 15.2 / 28.5, N 16384 16 rows 22.9 -> 24.8; K 512, N 16384 32 rows 7.1 -> 6.1, N 8192 64 rows 5.5 -> 6.0; K 128, N 50272 32
-// rows 10.5 -> 7.7; 32 / 64 groups of K 128, N 512 47 rows 4.2 / 5.3 -> 4.1 / 5.9 and, linear_kernel's nine column blocks of a group padded to sixteen, N 576 5.0 / 8.0 -> 4.4 / 6.5; 64 of K 256, N 128 4.5 -> 3.7.  Past 4608 columns
-// chunks follow each other: K 5120, N 6144 1 / 32 / 64 rows 12.6 / 15.1 / 22.0 -> 14.7 / 18.5 / 29.6, N 1024 16 rows 7.1 -> 7.6 (K 6144 7.9 -> 7.8, N 2048 8.5 -> 8.6), N 4096 10.4 -> 9.9; K 12288, N 6144 64 rows 66 -> 57.
-// Whole chunks (a form of its own, see plain_rows_kernel) keep more on their way: linear_kernel / here, K 6144, N 2048 1 / 16 rows 9.9 / 10.9 -> 7.8 / 9.5, N 6144 18.2 / 22.1 -> 16.3 / 20.8, N 8192 1 / 8 /
-// 16 rows 22.2 / 22.5 / 22.8 -> 19.9 / 20.7 / 23.6; K 8192, N 2048 11.0 / 14.0 -> 8.5 / 11.6, N 8192 28.2 / 28.1 -> 26.1 / 28.4; K 12288, N 2048 14.3 / 18.4 -> 11.7 / 16.0, N 6144 32.2 / 38.8 -> 30.4 / 37.3.
-// Every K of whole chunks for eight waves has it; of the others (us, the form that waits for all loads at every chunk, or linear_kernel past its line / here) K 10240, N 2048 1 / 8 / 16 rows
-// 12.5 / 14.0 / 16.1 -> 10.3 / 12.5 / 14.5, N 8192 1 / 8 32.2 / 32.8 -> 30.2 / 31.6; K 14336, N 2048 16.2 / 18.1 / 21.0 -> 13.6 / 16.4 / 18.7; K 16384, N 4096 28.4 / 29.1 / 30.2 -> 25.9 / 26.8 / 28.8,
-// N 7168 44.5 / 45.3 / 46.1 -> 44.0 / 47.0 / 46.0, N 8192 50.4 / 51.0 / 51.5 -> 49.8 / 51.3 / 51.4.  (Longer ones are not measured.)
+// Rows as they are go to plain_rows_kernel where it is ahead of linear_kernel; past 64 rows there are tiles.  In a graph of such launches, us, linear_kernel / here:
+//   K  1024  N 1024   1 row 3.7 / 2.9     16 4.0 / 3.1     32 4.1 / 3.1     64 6.4 / 3.2
+//   K  3072  N 1024   1  4.8 / 3.8     16 5.4 / 4.4     32 5.5 / 4.5     64 13.0 / 4.6
+//   K  4096  N 4096   1 10.1 / 8.1     16 11.3 / 9.0    32 12.4 / 10.7   64 24.6 / 17.1
+//   8 groups of K 128, N 512  1 3.7 / 2.3   16 3.9 / 2.4   32 4.0 / 2.5   64 3.4 / 2.6      of K 512, N 128  1 4.0 / 2.5   16 4.5 / 2.7   32 4.5 / 2.7   64 5.1 / 2.7
+//
+// Every workgroup brings the rows again, so past one slab a compute unit (256) it is ahead only while the rows are few or short:
+//   K  2048  N 16384  1 13.6 / 12.7    32 13.8 / 16.8   64 16.2 / 30.8      N 50272 1 42.8 / 35.0
+//   K  4096  N  8192  8 14.2 / 13.7    24 14.0 / 15.2   64 20.7 / 28.5      N 16384 16 22.9 / 24.8
+//   K   512  N 16384 32  7.1 / 6.1     N 8192 64 5.5 / 6.0                  K 128  N 50272 32 10.5 / 7.7
+//   groups of K 128, N 512, 47 rows: 32 of them 4.2 / 4.1, 64 5.3 / 5.9; N 576 (linear_kernel's nine column blocks of a group padded to sixteen) 5.0 / 4.4, 8.0 / 6.5; 64 of K 256, N 128 4.5 / 3.7
+//
+// Past 4608 columns chunks follow each other:
+//   K  5120  N 6144   1 12.6 / 14.7    32 15.1 / 18.5   64 22.0 / 29.6      N 1024 16 7.1 / 7.6   N 4096 16 10.4 / 9.9
+//   K 12288  N 4096   1 20.8 / 20.0    32 27.9 / 25.3   64 65.2 / 41.4      N 6144 64 66 / 57
+//
+// Whole chunks for all eight waves have a form of their own (plain_rows_kernel), which keeps more on its way.  linear_kernel, or the form that waits for all loads at every chunk / here:
+//   K  6144  N 2048   1  9.9 / 7.8     16 10.9 / 9.5       N 6144  1 18.2 / 16.3    16 22.1 / 20.8      N 8192  1 22.2 / 19.9   8 22.5 / 20.7   16 22.8 / 23.6
+//   K  8192  N 2048   1 11.0 / 8.5     16 14.0 / 11.6      N 8192  1 28.2 / 26.1    16 28.1 / 28.4
+//   K 10240  N 2048   1 12.5 / 10.3    16 16.1 / 14.5      N 8192  1 32.2 / 30.2     8 32.8 / 31.6
+//   K 12288  N 2048   1 14.3 / 11.7    16 18.4 / 16.0      N 6144  1 32.2 / 30.4    16 38.8 / 37.3
+//   K 14336  N 2048   1 16.2 / 13.6    16 21.0 / 18.7
+//   K 16384  N 4096   1 28.4 / 25.9    16 30.2 / 28.8      N 7168  1 44.5 / 44.0     8 45.3 / 47.0   16 46.1 / 46.0      N 8192  1 50.4 / 49.8   8 51.0 / 51.3
+// (Longer ones are not measured.)
 static bool whole_chunks(int K) { return K % 2048 == 0 && K >= 6144 && K <= 16384; }
 
 template <class F>

@@ -4,7 +4,7 @@
 // A reduction over 64 lanes is six dependent steps; as shuffles each waits for the LDS unit, and a decode step's kernels, chains of latencies of 3 - 7 us, hold two
 // to four such reductions.  The partners of every step are those of the shuffles (lane ^ 32, 16, 8, 4, 2, 1 in that order), so sums
 // keep every bit: after the step over 8 a row's value repeats every 8 lanes, so a rotation by 4 is the exchange over 4, and so on.
-// All lanes of the wave have to be active.  Shuffles -> here: paged attention of 32 sequences of 1 - 132 tokens, 12 heads of 64 6.37 -> 5.85 us, of one of 70 3.75 -> 3.50
+// The lanes that a value is over have to be active: the row's 16 for LANES = 16, the quad's for sum_quad, the wave's for the others, whose rows and halves change places.  Shuffles -> here: paged attention of 32 sequences of 1 - 132 tokens, 12 heads of 64 6.37 -> 5.85 us, of one of 70 3.75 -> 3.50
 // (an empty launch: 1.7); decode of GPT-2 small, 32 sequences, 1.5 per cent of a step; width 1024 behind norms, 12 rows, 2 per cent.
 #pragma once
 
