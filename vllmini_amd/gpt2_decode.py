@@ -10,7 +10,7 @@ for what the operators are actually batched over:
     bookkeeping (kv_pool.PagedKVPool.decode_step_batch) with a single upload;
   * q/k/v are strided views of the fused c_attn output (row stride 3*hidden), exactly the views
     the reference hands to the ops (gpt2.py:35-41);
-  * around the two ops a decode step runs the block's linear layers on this build's own gfx950 kernels
+  * around the two ops a decode step runs the block's linear layers on gfx950 kernels of their own
     (`native_layers`, vllmini_amd/gpt2_layer.py -> csrc/gpt2_layer.hip): LayerNorm + c_attn, c_proj + residual,
     LayerNorm + c_fc + GELU, mlp.c_proj + residual — four launches per layer where the torch modules take eleven
     (67 -> 23 us per layer at batch 256).  `native_layers=False` is the torch-module chain (F.linear -> hipBLASLt, layer_norm,

@@ -17,7 +17,7 @@ What a decoder asks of a mixer: page_rows() and state_shapes(), the cache tensor
 
 The residual stream is float32 (`Residual`).  Steps of few tokens run on the streaming kernels with everything fused around the
 products (norm in front, gated unit / head gate / residual add behind); from DENSE_MIN_TOKENS tokens on (from DENSE_MIN_TOKENS_LARGE
-for matrices of DENSE_LARGE elements, unless the kernel behind a norm can keep its rows in LDS) the products go to tiles of this build's own, with the gated unit
+for matrices of DENSE_LARGE elements, unless the kernel behind a norm can keep its rows in LDS) the products go to tiles of our own, with the gated unit
 where one stands behind them, or to the vendor library where that is ahead (product, gated_product), with one elementwise kernel between two of them.
 """
 from __future__ import annotations
@@ -51,7 +51,7 @@ def float_product(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def product(x: torch.Tensor, w: MatrixTiles, bias: Optional[torch.Tensor] = None, dense_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x W^T (+ bias: float32 for the tiles, the element type for the vendor's) of many rows: in tiles of this build's own where they are ahead of the vendor's product."""
+    """x W^T (+ bias: float32 for the tiles, the element type for the vendor's) of many rows: in tiles of our own where they are ahead of the vendor's product."""
     if ops.product_tiles_pay(x, w):
         return ops.product_tiles(x, w, bias)
     return F.linear(x, w.dense, dense_bias)

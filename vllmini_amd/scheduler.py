@@ -53,7 +53,7 @@ import torch.nn.functional as F
 def sample_top_k(logits: torch.Tensor, top_k: int = 50, temperature: float = 1.0,
                  generator: Optional[torch.Generator] = None) -> torch.Tensor:
     """Batched form of Scheduler.sample_next_token (scheduler.py:144-153): [B, V] -> [B] int64.  Half logits on a HIP device
-    (what the decoder hands over) are drawn by ONE launch of this build's kernel — the same distribution, the uniform numbers
+    (what the decoder hands over) are drawn by ONE launch of our own kernel — the same distribution, the uniform numbers
     from the same torch generator (vllmini_amd/gpt2_layer.py sample_top_k: 127 / 309 us -> 14 for 1 / 256 rows); anything else
     — and a tree without libvmi_gpt2_layer.so — takes the torch chain the reference spells out.  The two draw from the same
     distribution with DIFFERENT random streams (inverse CDF over torch.rand against torch.multinomial): a seeded run
