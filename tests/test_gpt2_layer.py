@@ -616,7 +616,7 @@ def test_prompt_attention_keeps_values_that_are_not_numbers_from_queries_that_do
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,D,T", [(1, 64, 1200), (3, 64, 1217), (1, 128, 1263), (12, 64, 1249), (12, 64, 2900)])
 def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T):
-    """vmi_gpt2_prompts_f16 from 1200 rows on (tiles_kernel: 64 and 128 columns, rows and chunks left over) against its entries called one by one.
+    """vmi_gpt2_prompts_f16 from 1200 rows on (rows and chunks left over; norms and tiles at width 768, the few-row kernels below) against its entries called one by one.
     Both round in the same five places (normed rows, q / k / v, attention, hidden, stream); a sum in another order may fall on the other side,
     2^-10 of a value each, and the two products behind one another pass that on."""
     from vllmini_amd import gpt2_layer as gl
@@ -661,7 +661,10 @@ def test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,D,T", [(1, 64, 6099), (3, 64, 2035), (1, 128, 3049), (12, 64, 508), (16, 64, 381), (9, 128, 339), (18, 64, 1201)])
 def test_prompts_take_tiles_from_fewer_rows_the_wider_they_are(H, D, T):
-    """As above just past the line between the two, T E = 390 000, at widths from 64 to 1152."""
+    """As above at T E = 390 000 and a little more, at widths from 64 to 1152: tiles past a width of 192 (vmi_gpt2_prompts_in_tiles), the few-row kernels up to there."""
+    from vllmini_amd import gpt2_layer as gl
+
+    assert gl.load().vmi_gpt2_prompts_in_tiles(T, H * D) == (H * D > 192)
     assert 390000 <= T * H * D
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
 
@@ -868,7 +871,10 @@ def test_gelu_of_every_half():
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,D,T", [(12, 64, 391), (14, 64, 179), (18, 64, 139), (6, 128, 400), (8, 64, 587)])
 def test_prompts_take_tiles_from_fewer_rows_still_past_a_width_of_768(H, D, T):
-    """As test_prompts_of_many_rows_..., just past the lines T E = 300 000 up to a width of 768 and 160 000 beyond."""
+    """As test_prompts_of_many_rows_..., at T E = 300 000 up to a width of 768 and 160 000 beyond."""
+    from vllmini_amd import gpt2_layer as gl
+
+    assert gl.load().vmi_gpt2_prompts_in_tiles(T, H * D)
     test_prompts_of_many_rows_take_tiles_and_agree_with_the_entries_one_by_one(H, D, T)
 
 
