@@ -815,6 +815,27 @@ def test_products_of_many_rows_in_tiles(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 272, 320), (300, 3088, 320), (770, 768, 3072), (2100, 768, 768), (2029, 6544, 768)])
+def test_residuals_that_begin_anywhere(M, N, K):
+    """tiles_kernel: residuals aligned to eight bytes, not to sixteen, give what aligned ones do, also where they are added in place of themselves."""
+    from vllmini_amd import gpt2_layer as gl
+
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)      # noqa: E731
+    x, w, b, flat = rnd(M, K).half(), gl.pack_weight((rnd(N, K) / K ** 0.5).half()), rnd(N).half(), rnd(M * N + 8).half()
+    want = gl.linear_tiles(x, w, b, residual=flat[4:-4].clone().view(M, N))
+    assert torch.equal(gl.linear_tiles(x, w, b, residual=flat[4:-4].view(M, N)), want)
+    before = flat.clone()
+    for at in (0, 4):
+        flat.copy_(before)
+        y, res = flat[at: at + M * N].view(M, N), flat[at: at + M * N].clone().view(M, N)
+        gl._check(gl.load().vmi_gpt2_linear_tiles_f16(x.data_ptr(), w.tiles.data_ptr(), b.data_ptr(), y.data_ptr(), y.data_ptr(), M, N, K, gl.EPI_BIAS_RESIDUAL, 0,
+                                                      torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(y, gl.linear_tiles(x, w, b, residual=res)) and torch.equal(flat[:at], before[:at]) and torch.equal(flat[at + M * N:], before[at + M * N:])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(2029, 6544, 768), (2024, 6576, 704), (2507, 7216, 256), (2517, 7216, 192), (1859, 3232, 512), (866, 6624, 832), (963, 5920, 1152),
                                    (1375, 4368, 448), (2026, 4400, 128), (2068, 4368, 64), (321, 7536, 128), (354, 6800, 64), (269, 6544, 512), (263, 6688, 832),
                                    (257, 6544, 1152), (259, 6576, 448), (769, 7600, 128), (778, 7568, 64), (391, 6560, 1536), (386, 6560, 1216), (195, 7088, 128),

@@ -417,6 +417,28 @@ def test_each_tile_by_itself_over_a_group(tile):
     test_groups_of_many_rows(groups, K, N, 8, M)
 
 
+@pytest.mark.parametrize("M,N,K,split", [(66, 96, 192, 0), (300, 3104, 320, 1552), (770, 5408, 128, 0), (1063, 2080, 576, 64), (2100, 1568, 1024, 1024)])
+def test_results_of_tiles_in_rows_that_are_not_whole_pieces(M, N, K, split):
+    """lines_out: rows of outputs that begin anywhere and are no multiple of sixteen bytes long hold, bit for bit, what aligned ones do, and nothing beside them is written."""
+    from vllmini_amd import hybrid_ops as ops
+
+    g = torch.Generator(device=dev()).manual_seed(M + N + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev())      # noqa: E731
+    t, x = ops.MatrixTiles(rnd(N, K) / K ** 0.5, torch.bfloat16), rnd(M, K).to(torch.bfloat16)
+    n = (N - split) // 2
+    whole, wide = torch.empty((M, n), dtype=torch.bfloat16, device=dev()), torch.full((M, n + 10), 7.0, dtype=torch.bfloat16, device=dev())
+    a, b = ops.linear_tiles(x, t, ops.SILU_UNIT, split, whole), ops.linear_tiles(x, t, ops.SILU_UNIT, split, wide[:, 2:-8])
+    assert torch.equal(wide[:, 2:-8], whole) and bool((wide[:, :2] == 7).all()) and bool((wide[:, -8:] == 7).all())
+    assert not split or torch.equal(a, b)
+    groups = ops.MatrixTiles(rnd(3, N, K) / K ** 0.5, torch.bfloat16)
+    for gate in (None, rnd(M, 3).to(torch.bfloat16)):
+        whole, wide = torch.empty((M, 3 * N), dtype=torch.bfloat16, device=dev()), torch.full((M, 3 * (N + 4)), 7.0, dtype=torch.bfloat16, device=dev())
+        ops.linear(x, groups, x_gstride=0, y_gstride=N, out=whole, gate=gate)
+        ops.linear(x, groups, x_gstride=0, y_gstride=N + 4, out=wide, gate=gate)
+        y = wide.view(M, 3, N + 4)
+        assert torch.equal(y[..., :N].reshape(M, 3 * N), whole) and bool((y[..., N:] == 7).all())
+
+
 def test_products_of_many_rows_alone_refuse_what_is_not_built():
     from vllmini_amd import hybrid_ops as ops
 

@@ -157,6 +157,7 @@ __device__ __forceinline__ float group_sum(float v) {
 // behind, the product 32 -> 21 us (17 without GELU).  Of all halves 333 come out closer to the exact value than 0.5 v (1 + erff) does (up to 2.7 units in the last
 // place off below -3, where 1 + erff cancels) and none further; infinities and NaN as there.
 __device__ __forceinline__ float gelu(float v) {
+  asm("" : "+v"(v));   // (a float from here on: a multiply-add that widens its half operand by itself takes no constant, which then is a move each)
   const float t = fabsf(v);
   float p = -2.5964232e-08f;
   for (float c : {7.884347e-07f, -1.0245299e-05f, 7.2435578e-05f, -2.6644077e-04f, -2.6124299e-05f, 6.9771572e-03f, -5.2460529e-02f, -4.5921496e-01f, -1.1511048f, -1.f})

@@ -8,38 +8,66 @@ namespace vmi_hybrid {
 // STORE_GLU: columns below n_split as they are, the others, interleaved (gate, up), through the gated unit: what a product and an elementwise launch behind it (a
 // write and a read of 2 N bytes a row) took, and what they give: gate and up are rounded on their way into the unit, so what a prompt comes to does not hang on
 // whether the tokens that happen to share its step are enough for tiles.  STORE, FLOAT: a product alone, with the bias in 32 bits, in bfloat16 or as it is.
+// A product's results in bfloat16, each word of two or four columns a lane as it is, or of a gated unit
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
 template <int MI, int NI, int D, int EPI>
 __global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args p) {
-  const int kc = (threadIdx.x & 63) >> 4;
   f32x4 bias[NI];
   vmi_tiles::tiles_product<vmi_tiles::Bf16, MI, NI, D>(
       p.x, p.ldx, p.w, p.M, p.N, p.K,
-      [&](int, int s, int SL) {
+      [&](const vmi_tiles::Where& at) {
         if constexpr (EPI == VMI_HY_E_STORE) {
 #pragma unroll
-          for (int n = 0; n < NI; ++n) bias[n] = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + min(s + n, SL - 1) * 16 + 4 * kc) : f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int n = 0; n < NI; ++n)
+            bias[n] = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + min(at.s0 + at.wave * NI + n, at.SL - 1) * 16 + 4 * at.kc) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
       },
-      [&](const f32x4(&acc)[NI][MI], int m, int s, int SL) {
+      [&](const f32x4(&acc)[NI][MI], const vmi_tiles::Where& at) {
+        const int first = at.s0 * 16, wave_s = at.s0 + at.wave * NI, m = at.m0 + at.r16;
+        auto stored = [&](int n, int i) {
+          b16x4 o;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[r] = EPI == VMI_HY_E_STORE ? (b16)(acc[n][i][r] + bias[n][r]) : (b16)acc[n][i][r];
+          return __builtin_bit_cast(u32x2, o);
+        };
+        auto gated = [&](int n, int i) {
+          typename Elem<b16>::v2 o;
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+            o[r] = (b16)glu((float)(b16)acc[n][i][2 * r], (float)(b16)acc[n][i][2 * r + 1], p.scale, p.glu_alpha, p.glu_up);
+          return __builtin_bit_cast(uint32_t, o);
+        };
+        if constexpr (EPI != VMI_HY_E_FLOAT) {
+          if (EPI == VMI_HY_E_STORE || first + 64 * NI <= p.n_split) {   // (scalar)
+            const bool wide = ((p.ldy & 7) | ((uintptr_t)p.y & 15)) == 0;
+            vmi_tiles::lines_out<u32x2, MI, NI, false>(at, stored, [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
+              if (at.m0 + row < p.M && first + 8 * piece < p.N) vmi_tiles::put_piece(static_cast<b16*>(p.y) + (int64_t)(at.m0 + row) * p.ldy + first + 8 * piece, v, wide);
+            });
+            return;
+          }
+          if (first >= p.n_split) {
+            const bool wide = ((p.ldy2 & 7) | ((uintptr_t)p.y2 & 15) | (p.n_split & 15)) == 0;
+            vmi_tiles::lines_out<uint32_t, MI, NI, true>(at, gated, [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
+              if (at.m0 + row < p.M && first + 16 * piece < p.N)
+                vmi_tiles::put_piece(static_cast<b16*>(p.y2) + (int64_t)(at.m0 + row) * p.ldy2 + ((first - p.n_split) >> 1) + 8 * piece, v, wide);
+            });
+            return;
+          }
+        }
 #pragma unroll
         for (int n = 0; n < NI; ++n) {
-          if (s + n >= SL) break;   // (scalar)
-          const int col = (s + n) * 16 + 4 * kc;
+          if (wave_s + n >= at.SL) break;   // (scalar)
+          const int n0 = (wave_s + n) * 16, column = n0 + 4 * at.kc;
 #pragma unroll
           for (int i = 0; i < MI; ++i) {
             if (m + 16 * i >= p.M) continue;
-            if constexpr (EPI == VMI_HY_E_STORE) {
-              b16x4 o;
-#pragma unroll
-              for (int r = 0; r < 4; ++r) o[r] = (b16)(acc[n][i][r] + bias[n][r]);
-              *reinterpret_cast<b16x4*>(static_cast<b16*>(p.y) + (int64_t)(m + 16 * i) * p.ldy + col) = o;
-            } else if constexpr (EPI == VMI_HY_E_FLOAT) {
-              epilogue<b16, VMI_HY_E_FLOAT>(p, acc[n][i], m + 16 * i, col, (s + n) * 16, 0);
+            if constexpr (EPI == VMI_HY_E_FLOAT) {
+              epilogue<b16, VMI_HY_E_FLOAT>(p, acc[n][i], m + 16 * i, column, n0, 0);
+            } else if (n0 < p.n_split) {
+              *reinterpret_cast<u32x2*>(static_cast<b16*>(p.y) + (int64_t)(m + 16 * i) * p.ldy + column) = stored(n, i);
             } else {
-              f32x4 v;
-#pragma unroll
-              for (int r = 0; r < 4; ++r) v[r] = (float)(b16)acc[n][i][r];
-              epilogue<b16, VMI_HY_E_STORE_GLU>(p, v, m + 16 * i, col, (s + n) * 16, 0);
+              *reinterpret_cast<uint32_t*>(static_cast<b16*>(p.y2) + (int64_t)(m + 16 * i) * p.ldy2 + ((column - p.n_split) >> 1)) = gated(n, i);
             }
           }
         }
@@ -49,17 +77,32 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args 
 // Products of a group of matrices, a group a y of the grid, each with its own columns of x and of y (the per-head products of latent attention, of low ranks)
 template <int MI, int NI, int D, int EPI>
 __global__ __launch_bounds__(256, 2) void group_tiles_kernel(const vmi_hy_linear_args p) {
-  const int kc = (threadIdx.x & 63) >> 4, grp = blockIdx.y;
+  const int grp = blockIdx.y;
   vmi_tiles::tiles_product<vmi_tiles::Bf16, MI, NI, D>(
-      static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride, p.ldx, static_cast<const b16*>(p.w) + (int64_t)grp * p.N * p.K, p.M, p.N, p.K, [](int, int, int) {},
-      [&](const f32x4(&acc)[NI][MI], int m, int s, int SL) {
+      static_cast<const b16*>(p.x) + (int64_t)grp * p.x_gstride, p.ldx, static_cast<const b16*>(p.w) + (int64_t)grp * p.N * p.K, p.M, p.N, p.K,
+      [](const vmi_tiles::Where&) {},
+      [&](const f32x4(&acc)[NI][MI], const vmi_tiles::Where& at) {
+        float g[MI];
 #pragma unroll
-        for (int n = 0; n < NI; ++n) {
-          if (s + n >= SL) break;   // (scalar)
+        for (int i = 0; i < MI; ++i)
+          g[i] = EPI == VMI_HY_E_GATED ? sigmoid((float)static_cast<const b16*>(p.gate)[(int64_t)min(at.m0 + at.r16 + 16 * i, p.M - 1) * p.ldg + grp]) : 1.f;
+        f32x4 bias[NI];
 #pragma unroll
-          for (int i = 0; i < MI; ++i)
-            if (m + 16 * i < p.M) epilogue<b16, EPI>(p, acc[n][i], m + 16 * i, (s + n) * 16 + 4 * kc, (s + n) * 16, grp);
-        }
+        for (int n = 0; n < NI; ++n)
+          bias[n] = EPI == VMI_HY_E_STORE && p.bias ? *reinterpret_cast<const f32x4*>(p.bias + min(at.s0 + at.wave * NI + n, at.SL - 1) * 16 + 4 * at.kc) : f32x4{0.f, 0.f, 0.f, 0.f};
+        b16* const y = static_cast<b16*>(p.y) + (int64_t)grp * p.y_gstride + at.s0 * 16;
+        const bool wide = ((p.ldy & 7) | (p.y_gstride & 7) | ((uintptr_t)p.y & 15)) == 0;
+        vmi_tiles::lines_out<u32x2, MI, NI, false>(
+            at,
+            [&](int n, int i) {
+              b16x4 o;
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[r] = EPI == VMI_HY_E_GATED ? (b16)(acc[n][i][r] * g[i]) : (b16)(acc[n][i][r] + bias[n][r]);
+              return __builtin_bit_cast(u32x2, o);
+            },
+            [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
+              if (at.m0 + row < p.M && at.s0 * 16 + 8 * piece < p.N) vmi_tiles::put_piece(y + (int64_t)(at.m0 + row) * p.ldy + 8 * piece, v, wide);
+            });
       });
 }
 

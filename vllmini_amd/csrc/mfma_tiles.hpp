@@ -29,8 +29,86 @@ struct Bf16 {
   static __device__ __forceinline__ f32x4 mma(const v8& a, const v8& b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 
-// The product of this workgroup's tile; early(m, s, SL) asks for what finish will read, behind the first requests of the product; finish(acc, m, s, SL) gets a lane's results, acc[n][i] = columns 16 (s + n) + 4 (lane / 16) .. + 3 of row m + 16 i, and does not look at
-// slabs from SL or rows from M on.  K % 64 == 0, N % 16 == 0, x and ldx 16-byte aligned, a matrix of x below 4 GiB.
+// Where a tile's results are: rows m0 on, slabs of 16 columns s0 on; a lane holds acc[n][i] = columns 16 (s0 + wave NI + n) + 4 kc .. + 3 of row m0 + 16 i + r16.  Slabs from SL and
+// rows from M on are none.  lds: two places of 2 KiB MI, free once every wave is past a barrier.
+struct Where {
+  int m0, s0, SL, wave, kc, r16;
+  unsigned char* lds[2];
+};
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Results of 16 bits on their way out, as whole lines: 32 rows of the tile at a time through LDS.  pack(n, i): what a lane has of slab n, tile i, eight bytes (four columns) or
+// four (two, behind a gated unit), all of it FIRST where that is work (between two barriers there is nothing but LDS then); put(row, piece, v, k): sixteen bytes from 16 piece on
+// of a row of the tile, the k-th of this lane, neighbours of a row in neighbouring lanes: NI pieces of every 32 rows, one of (threadIdx.x + 256 j) / PIECES, % PIECES.
+// What bounds it is L2, which takes as long for 32 bytes of a line as for 64 or 128: as the lanes hold them, a store would leave 32 bytes of each of 16 lines (16 behind a gated unit), and
+// products over a short K spent a third of their time on it.  us before / now: 6400 rows, K 768 in halves N 2304 29.3 / 24.7, N 768 with a residual 17.0 / 13.7, K 3072 37.9 / 32.4; gated, bfloat16
+// 2773 rows, N 12288, K 2048 128 / 116, 4600, 6144, 1024 58 / 51; without any stores 6400 rows, N 2304 take 18.4.
+template <class Word, int MI, int NI, bool FIRST, class Pack, class Put>
+__device__ __forceinline__ void lines_out(const Where& at, Pack&& pack, Put&& put) {
+  constexpr int PIECES = NI * (int)sizeof(Word), BYTES = 16 * PIECES, ALL = 32 * PIECES;
+  // (a row's pieces in another order for each of eight rows, or rows an odd number of pieces apart: lanes of one access meet in no bank)
+  constexpr bool TURN = sizeof(Word) == 8;
+  constexpr int ROW = TURN ? BYTES : BYTES + 16;
+  static_assert(32 * ROW <= MI * 2048 && MI % 2 == 0);
+  auto landed = []() {   // (a fence would wait for the stores as well)
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  Word words[FIRST ? MI : 1][NI];
+  if constexpr (FIRST) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int n = 0; n < NI; ++n) words[i][n] = pack(n, i);
+  }
+  landed();
+#pragma unroll
+  for (int t = 0; t < MI / 2; ++t) {
+    unsigned char* const b = at.lds[t & 1];
+#pragma unroll
+    for (int n = 0; n < NI; ++n)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = 16 * h + at.r16, byte = (at.wave * NI + n) * 4 * (int)sizeof(Word) + at.kc * (int)sizeof(Word), piece = byte >> 4;
+        *reinterpret_cast<Word*>(b + row * ROW + (TURN ? piece ^ (row & 7) : piece) * 16 + (byte & 15)) = FIRST ? words[FIRST ? 2 * t + h : 0][n] : pack(n, 2 * t + h);
+      }
+    landed();
+#pragma unroll
+    for (int j = 0; j < (ALL + 255) / 256; ++j) {
+      const int u = (int)threadIdx.x + 256 * j, row = u / PIECES, piece = u - row * PIECES;
+      if (ALL % 256 == 0 || u < ALL) put(32 * t + row, piece, *reinterpret_cast<const u32x4*>(b + row * ROW + (TURN ? piece ^ (row & 7) : piece) * 16), t * ((ALL + 255) / 256) + j);
+    }
+  }
+}
+// The same without LDS and barriers, in sixteen bytes of half a line: two slabs' neighbouring columns meet in a lane, whose (lane / 16) even ones keep slab n, odd ones n + 1.  NI even.
+template <int MI, int NI, class Pack, class Put>
+__device__ __forceinline__ void pairs_out(const Where& at, Pack&& pack, Put&& put) {
+  static_assert(NI % 2 == 0);
+#pragma unroll
+  for (int n = 0; n < NI; n += 2)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const u32x2 a = pack(n, i), b = pack(n + 1, i);
+      const auto l = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false), h = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+      put(16 * i + at.r16, (at.wave * NI + n + (at.kc & 1)) * 2 + (at.kc >> 1), u32x4{l[0], h[0], l[1], h[1]}, 0);
+    }
+}
+// sixteen bytes of results; wide: rows of y and where they begin are aligned to as many, else to four
+__device__ __forceinline__ void put_piece(void* y, const u32x4& v, bool wide) {
+  if (wide) {   // (scalar)
+    *static_cast<u32x4*>(y) = v;
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) static_cast<uint32_t*>(y)[r] = v[r];
+  }
+}
+
+// The product of this workgroup's tile; early(at) asks for what finish(acc, at) will read, behind the first requests of the product.
+// K % 64 == 0, N % 16 == 0, x and ldx 16-byte aligned, a matrix of x below 4 GiB.
 template <class H, int MI, int NI, int D, class Early, class Finish>
 __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const void* w, int M, int N, int K, Early&& early, Finish&& finish) {
   using V8 = typename H::v8;
@@ -99,15 +177,13 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
       if (i == XU - 1 || i == ASKS - 1) __builtin_amdgcn_sched_barrier(0);
     }
   }
-  early(m0 + r16, s0, SL);
+  const Where at{m0, col * 4 * NI, SL, wave, kc, r16, {xs0, xs1}};
+  early(at);
   x_landed(std::integral_constant<int, D - 2>{});
   // The chunk in place d, and chunk kb on its way into the place of the one before (whose readers have all passed the barrier): steps of one fragment of x, which was asked
   // for AHEAD steps before, against the wave's NI of W, and its share of the requests.  A chunk that is none is zeros, x and W
   auto chunk = [&](auto more, int d, int kb, bool on) {
-    auto fragment = [&](int q) {
-      const V8 v = read(xs[d], q);
-      return on ? v : V8{};
-    };
+    auto fragment = [&](int q) { return read(xs[d], q); };
     if (!on) {   // (scalar)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -124,8 +200,9 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
         for (int i = 0; i < PER; ++i) ask(q * PER + i, (d + D - 1) % D, kb);
       }
       __builtin_amdgcn_sched_barrier(0);
+      const V8 now = on ? f[q % AHEAD] : V8{};   // (here and not where it is read, or every read is waited for at once)
 #pragma unroll
-      for (int n = 0; n < NI; ++n) acc[n][q % MI] = H::mma(wr[d][q / MI][n], f[q % AHEAD], acc[n][q % MI]);
+      for (int n = 0; n < NI; ++n) acc[n][q % MI] = H::mma(wr[d][q / MI][n], now, acc[n][q % MI]);
       if (q + AHEAD < STEPS) f[q % AHEAD] = fragment(q + AHEAD);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -150,7 +227,7 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     }
   };
   rest(std::integral_constant<int, 1>{}), rest(std::integral_constant<int, 2>{}), rest(std::integral_constant<int, 3>{});
-  finish(acc, m0 + r16, s0, SL);
+  finish(acc, at);
 }
 
 // ---- which tile -----------------------------------------------------------------------------------------------------------------
