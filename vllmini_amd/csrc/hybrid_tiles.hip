@@ -141,15 +141,20 @@ int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
 // Whether tiles of our own end sooner than the library's product (hipBLASLt as PyTorch 2.10.0+rocm7.0 loads it: another version may move the line, never the result beyond the
 // order of a sum).  Measured in bfloat16, weights that leave the last cache between two products from K 2048 on and others that stay.
 //
-// Alone, 3260 pairs of 48 to 8192 rows, K 256 to 16 384, N 256 to 16 384: 0.87 where the rule says tiles.  Not where whole tiles of 256 columns fill the chip more than once, from
-// K 2048 on at 5.6 million results (N 2048, K 6144: 2400 rows 74 / 70, 4500 103 / 115; N 4096, K 2048 948 24 / 22, 2400 41 / 46; past K 4096 whatever N is), from K 1024 on at 8
-// million (N 3072, K 1536: 5251 rows 42 / 49; N 2048, K 1024: 7455 32 / 36; N 6400, K 1728: 3985 77 / 106; 21 of 21 pairs, 1.14 in the mean), where few of the smallest tiles
-// walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4), where tiles of 64 x 64 are just more than the chip has compute
-// units for (300 rows, N 4096, K 8192 46 / 56; 600 rows, N 2048, K 6144 34 / 37), and past K 16 383.
+// Alone, 5300 pairs of 48 to 9000 rows, K 256 to 12 288, N 256 to 16 384: ours / library's in the mean, from 5.6 million results on (below, nearly all of the library's time is its call:
+// 19 us of host) and whole tiles of 256 columns: K 1024 to 2047 0.88 (8 of 207 more than 5 per cent behind), to 4095 0.96 (52 of 239), to 6144 1.00 (30 of 104), beyond 1.07; other columns
+// 0.74, 0.85, 0.96 and 0.99.  So not past K 6144 from 5.6 million results on, up to there whole columns only where the tiles' own costs promise 1020 TFLOP/s (N 2048, K 6144: 2773 rows
+// 69 / 60, which one round of tiles holds; 4500 103 / 111), and below K 4096 whole columns up to 9 million (N 4096, K 2048: 2400 41 / 42, level from there on), below 2048 up to 15.
+// Not where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4), where tiles of 64 x 64 are just more than
+// the chip has compute units for (300 rows, N 4096, K 8192 46 / 56; 600 rows, N 2048, K 6144 34 / 37), and past K 16 383.
 static bool product_pays(int M, int N, int K) {
   const bool whole = N % 256 == 0;
   const int64_t results = (int64_t)M * N, least = (int64_t)((M + 31) / 32) * ((N + 63) / 64);
-  if (K >= 1024 && results >= (K >= 2048 ? 5600000 : 8000000) && (whole || K >= 4096)) return false;
+  if (K >= 4096) {
+    if (results >= 5600000 && (K > 6144 || (whole && vmi_tiles::tiles_cost(vmi_tiles::tiles_pick(M, N, K), M, N, K, 1) > 2. / 1.02e9 * (double)results * K))) return false;
+  } else if (whole && K >= 1024 && results >= (K >= 2048 ? 9000000 : 15000000)) {
+    return false;
+  }
   if (K >= 3072 && (least <= 128 || (whole && N >= 2048 && results >= 1050000 && results < 2400000))) return false;
   return K < 16384;
 }

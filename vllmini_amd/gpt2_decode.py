@@ -93,12 +93,12 @@ class GPT2PagedDecoder:
 
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
     # prompts of more tokens in all (times the width's square) issue their launches from here: the native call saves the host 150 us, which is what a call of fewer waits for.
-    # Their products are tiles of our own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond.  12
-    # layers of prompts of 100 tokens, tiles / vendor in us: width 256 8000 tokens 1485 / 2541, 512 1681 / 2570; 768 5000 1764 / 2187, 6000 2147 / 2357, 8000 2623 / 2787; 1024
-    # 4000 2084 / 2164, 5000 2522 / 2352, 7000 4024 / 3140; 1152 4000 2579 / 2691, 7000 3736 / 3791
+    # Their products are tiles of our own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond, where
+    # none was measured.  12 layers of prompts of 200 tokens, tiles / vendor in us: width 512 8000 tokens 1964 / 2334, 12 000 2470 / 2901; 768 5000 1791 / 2136, 12 000 3446 / 3972; 1024 4000
+    # 2038 / 2204, 7000 3344 / 3426, 12 000 4879 / 5331; 1152 4000 2585 / 2833, 7000 3691 / 3889, 12 000 5858 / 6833
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
     NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
-    OWN_PRODUCTS_MAX_WORK = 50 * 10 ** 8
+    OWN_PRODUCTS_MAX_WORK = 160 * 10 ** 8
     INFINITY_CACHE = 248 << 20        # bytes of the last cache in front of the memory, 256 MiB, that a step's activations and logits leave
     SCATTER_IN_C_ATTN_MAX_BATCH = 64  # up to here the cache write rides in the q / k / v projection unless the caller says no
 
