@@ -500,3 +500,32 @@ def test_graph_replay_two_streams_and_two_host_threads():
     assert not errs, errs
     for k in range(2):
         assert_close(outs[k], ref, f"thread {k}")
+
+
+@pytest.mark.parametrize("D,H,hkv,lens,room,form", [
+    (128, 32, 8, [40], 40, "d128_h1_w4_u2_nt0"), (128, 32, 8, [130, 1, 0, 77], 130, "d128_h1_w8_u2_nt0"), (128, 32, 8, [700, 16], 700, "d128_h1_w16_u1_nt0"),
+    (128, 32, 8, [300] * 7 + [17] * 4, 300, "d128_h1_w4_u2_nt0"), (128, 32, 8, [300] * 2 + [33] * 10, 300, "d128_gq2_h1_w8_u2_nt1"), (128, 32, 8, [1099, 600], 1099, "d128_h1_w16_u1_nt0"),
+    (128, 32, 8, [1300] + [i * 9 for i in range(11)], 1300, "d128_gq2_h1_w8_u2_nt1"), (128, 32, 8, [1200] + [i * 7 for i in range(31)], 1200, "d128_gq4_h1_w16_u1_nt1"),
+    (128, 64, 8, [250, 3], 250, "d128_h1_w8_u2_nt0"), (64, 16, 4, [20] * 3, 20, "d64_h1_w4_u2_nt0"), (64, 16, 4, [900, 5, 0], 900, "d64_h1_w16_u2_nt0"),
+    (64, 16, 4, [1699, 64, 65], 1699, "d64_h1_w16_u2_nt0"), (64, 16, 4, [640] + [i * 5 for i in range(47)], 640, "d64_gq4_h1_w8_u2_nt1"),
+    (64, 16, 4, [1000] + [i * 11 for i in range(40)], 1000, "d64_gq4_h1_w16_u2_nt1")])
+def test_grouped_queries_of_few_sequences(D, H, hkv, lens, room, form):
+    """The forms that a launch of few sequences takes over shared key and value heads, on either side of their lines: which one runs, and what it gives against the kernel model, with ALiBi and
+    without; a sequence's row is what it is where all the others are empty."""
+    from vllmini_amd import ops
+
+    rng = np.random.default_rng(D + len(lens) + room)
+    case = make_case(rng, len(lens), H, D, lens, num_kv_heads=hkv, q_row_pad=1, poison_tail=True)
+    names = ops.variant_names()
+    assert names[ops.pick_variant(len(lens), H, D, room, num_kv_heads=hkv, workspace=True) - 1] == form
+    t = _upload(case, _dev())
+    got = _launch(case, dict(t, msl=room)).cpu().numpy()
+    assert ops.last_launch_label() == form
+    assert_close(got, run_model(case), form)
+    slopes = rng.uniform(0.01, 0.3, H).astype(np.float32)
+    out = torch.full((len(lens), H, D), float("nan"), dtype=torch.float16, device=_dev())
+    ops.paged_attention_v1(out, t["q"], t["kc"], t["vc"], hkv, case["scale"], t["tab"], t["lens"], 16, room, torch.from_numpy(slopes).to(_dev()), "auto", 1.0)
+    assert_close(out.cpu().numpy(), run_model(case, slopes), form + ", ALiBi")
+    only = t["lens"].clone()
+    only[1:] = 0
+    assert np.array_equal(_launch(case, dict(t, msl=room, lens=only)).cpu().numpy()[0], got[0])

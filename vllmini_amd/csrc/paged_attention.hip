@@ -470,6 +470,30 @@ static int pick_variant_gqa(int num_seqs, int num_heads, int qpk, int head_size,
   }
   return pick_variant_gqa_of(num_seqs, num_heads, qpk, head_size, block_size, max_seq_len, bf, f8, false);
 }
+// Four query heads of a KV head, fp16 pages, contexts of eight waves: which form of the shared-tile kernels.  items: (sequence, four heads).
+// A workgroup that has a compute unit to itself waits for memory: two groups of pages a wave are all it has in flight, and eight waves of 4 KiB (2 at head size 64) fetch
+// 28 bytes a ns where a compute unit of a full chip gets as many beside others.  So while items fit the compute units sixteen waves from 1000 tokens on, at head size 64 two blocks a
+// group too; and up to half of them two heads an item, each tile read twice, twice the vector pipes.  us over 32 / 8 heads of 128 (16 / 4 of 64), contexts equal and U{1 .. longest}:
+//   sixteen waves  24 x 1500 33.2 / 30.5 -> 31.0 / 28.0; 32 x 3000 65.4 / 54.0 -> 64.3 / 47.1; 24 x 4096 76.8 / 69.8 -> 69.9 / 59.8   (48 x 1500 25.5 / 23.8 -> 20.2 / 18.3; 64 x 4096 60.0 / 55.3 ->
+//   48.7 / 37.5).  700 tokens level (4 per cent behind).  Not for more items than compute units, which would go round twice (48 x 4096 137.6 / 82.7 -> 145.4 / 75.4: what
+//   a ragged batch wins, an equal one loses).   two heads  16 x 300 11.6 / 11.2 -> 9.9 / 9.0; 16 x 700 17.6 / 17.0 -> 16.7 / 13.5; 12 x 1400 18 per cent ahead, 16 x 1400 behind; 24 x 700 18.3 / 17.2 -> 24.1 / 15.8
+//   two blocks, head size 64  48 x 700 14.5 / 13.8 -> 13.0 / 12.4; 32 / 8 heads, 64 x 2000 0.95 of it, 128 x 700 1.14: by items as below
+// More items than twice the compute units, head size 128: four waves (80 x 130 1.43 of it, x 300 1.24, x 700 1.11; level from 1500 on).
+struct GqForm {
+  int heads, waves, blocks;
+};
+static GqForm pick_gq4(long items, int head_size, int max_seq_len) {
+  const long cus = g_cus;
+  const int L = max_seq_len;
+  if (head_size == 128) {
+    if (2 * items <= cus && L >= 190 && L < 1700 && items * L <= 600 * cus) return {2, 8, 2};
+    if (items <= cus && L >= 1000) return {4, 16, 1};
+    return {4, items > 2 * cus && L < 1500 ? 4 : 8, 1};
+  }
+  if (items <= cus && L >= 900) return {4, 16, 2};
+  return {4, 8, (items <= cus && L >= 180) || (items <= 2 * cus && L >= 640) ? 2 : 1};
+}
+
 static int pick_variant_gqa_of(int num_seqs, int num_heads, int qpk, int head_size, int block_size, int max_seq_len,
                                bool bf, int f8, bool fpv) {
   if (qpk < 2 || block_size != 16) return 0;
@@ -492,13 +516,22 @@ static int pick_variant_gqa_of(int num_seqs, int num_heads, int qpk, int head_si
     for (int id = 1; id <= nvariants_v1(); ++id) {
       const Variant& c = variant_v1(id);
       if (!c.GQS || c.XW || c.FPV != fpv || c.BF != bf || c.F8 != f8 || c.D != head_size || c.BS != block_size || c.HPT != g ||
-          !fits(c))
+          !fits(c) || (!f8 && !fpv && c.U > 1))   // (fp16 rows of two blocks a group: pick_gq4's alone)
         continue;
       if (wph == 1 ? (c.WPH == 1 && (num_heads / g) % c.HPW == 0)
                    : (c.HPW == 1 && c.WPH <= wph && c.WPH * 4 >= wph)) {  // at most 4x fewer waves than wanted
         if (!best || (wph == 1 ? c.HPW > variant_v1(best).HPW || (c.HPW == variant_v1(best).HPW && c.U < variant_v1(best).U)
                                : c.WPH > variant_v1(best).WPH))
           best = id;
+      }
+    }
+    if (best && g == 4 && wph == 8 && !bf && !f8 && !fpv) {
+      const GqForm form = pick_gq4(units, head_size, max_seq_len);
+      for (int id = 1; id <= nvariants_v1(); ++id) {
+        const Variant& c = variant_v1(id);
+        if (c.GQS && !c.XW && !c.FPV && !c.BF && !c.F8 && c.D == head_size && c.BS == block_size && c.HPW == 1 && c.HPT == form.heads && c.WPH == form.waves &&
+            c.U == form.blocks && fits(c))
+          return id;
       }
     }
     if (best) return best;
@@ -588,6 +621,10 @@ struct PickRules {
                                      //   192 items lost in every cell, 96 won from 8192 tokens on)
   long split_min_item_bytes_per_unit = 20480;   // ... and an item's pages >= 20 KiB x items (head size 64: max_seq_len >= 80 x
                                      //   items — batch 2 from 2048 tokens, batch 4 from 4096, batch 8 from 8192)
+  int split_gqa_many_min_tokens = 1700;   // ... with more than a quarter of the CUs' items of four heads (32 / 8 heads x 128, ragged: 12 x 1500 as a workgroup each 23.5 against 24.0 us,
+                                     //   x 2000 33 % ahead)
+  int split_gqa_blocks_per_wave = 5, split_gqa_blocks_per_wave_d64 = 7;   // ... and so many blocks a wave do on a loaded chip: 12 x 3000 47.0 -> 37.6 us on sixteen waves an item, 16 x 2000 27 % ahead of eight; a query head an
+                                     //   item, 3 x 1400 / 2000 / 2800 26 / 34 / 38 %
   int split_gqa_min_tokens = 1024;   // grouped-query heads: from 1024 tokens on (r05i_split_gqa_sweep_rocprof.json)
   long split_min_item_bytes = 384 * 1024;   // ... and >= 384 KiB (1536 tokens at head size 64: batch 1 at 1024 tokens is level)
   int gate_max_seqs = 2048;          // the gated double launch behind it (launch_pa_v1): every wave of BOTH kernels reads all the
@@ -871,6 +908,23 @@ static int find_split(int D, int xw, int U, int nt, int f8 = 0, int hpt = 1) {
   }
   return 0;
 }
+// Grouped queries, fp16 pages, few sequences of contexts that one compute unit is done with soon: a workgroup a QUERY head, each reading its KV head's tiles itself (the
+// repeats hit the caches), so that four times the compute units work.  Or 0.  Such a launch takes 5 - 7 us and what its reads take from the caches, heads x tokens; the shared-tile
+// kernel it stands for 7 us and its longest context on one compute unit: the line is where the two meet, fitted to 1350 launches of 20 to 4096 tokens, 1 to 128 sequences, 32 / 8 and
+// 16 / 4 heads (349 inside it: the shared-tile kernels 1.7 times as long in the mean; five sizes up to 10 per cent behind another form of their own).  us, contexts equal: 32 / 8 heads
+// of 128 1 x 40 7.9 -> 3.8, 4 x 300 10.7 -> 5.3, 1 x 700 15.8 -> 7.0, 4 x 700 16.7 -> 10.3, 8 x 300 11.3 -> 8.3, 12 x 300 11.4 / 12.5 (outside); 16 / 4 of 64 4 x 700 13.4 -> 5.7, 16 x 700 13.9 -> 9.1,
+// 8 x 1500 15.0 -> 10.8.  Waves a head: the most that still have blocks and compute units to themselves.
+static int pick_per_head(int num_seqs, int num_heads, int qpk, int head_size, int block_size, int max_seq_len) {
+  if (qpk % 4 != 0 || block_size != 16 || (head_size != 64 && head_size != 128)) return 0;
+  const bool wide = head_size == 128;
+  const long units = (long)num_seqs * num_heads, cus = g_cus;
+  const double chip = cus / 256.0, reads = (wide ? 1.05e-4 : 4.5e-5) / chip * (double)units * max_seq_len, shared = wide ? 7.3 + .0133 * max_seq_len : 6.3 + .0105 * max_seq_len;
+  if (max_seq_len >= (wide ? 1100 : 1700) || units > (wide ? 5 : 8) * cus || reads > shared) return 0;
+  const int nblk = (max_seq_len + 15) / 16;
+  if (2 * units <= cus && nblk >= (wide ? 40 : 56)) return find_variant(head_size, block_size, 1, 16, wide ? 1 : 2, 0);
+  return find_variant(head_size, block_size, 1, nblk >= 5 && units <= (wide ? 1 : 2) * cus ? 8 : 4, 2, 0);
+}
+
 // Which split kernel, if any, serves a launch the plain heuristic gave `plain` to.  0 = keep the plain pick.
 // Measured (profiles/r05_split_kernels.md, rocprofv3, 12 heads x 64, batch 1 ... 16 x 1024 ... 16384 tokens): an item's waves
 // pay two trips through memory (exchange of max / exp-sum: 1.5 us on an idle chip, 2.5 - 2.9 us under load; partial rows and
@@ -912,7 +966,7 @@ static int pick_split(int num_seqs, int num_heads, int head_size, int block_size
     if (qpk % 4 == 0 && f8 != 2 && units * 2 >= (long)g_cus) {   // (fp8 E4M3 pages too: r05q_split_gq4_fp8_rocprof.json)
       hpt = 4;
       few = (units / 4) * 2 <= (long)g_cus;
-      if ((units / 4) * 4 > (long)g_cus) big = max_seq_len >= 2 * R.split_gqa_min_tokens;   // (128 such items at 1024 tokens: 23.9 against 22.9 us)
+      if ((units / 4) * 4 > (long)g_cus) big = max_seq_len >= R.split_gqa_many_min_tokens;   // (128 such items at 1024 tokens: 23.9 against 22.9 us)
     } else {
       few = units * (head_size == 128 ? 2 : 1) <= (long)g_cus;
     }
@@ -929,12 +983,13 @@ static int pick_split(int num_seqs, int num_heads, int head_size, int block_size
   // 4-block waves, 16.3 on 384 of 8-block ones, 19.0 unsplit; batch 2 at 16384 tokens 27.3 us on 768 workgroups, 22.8 on 384)
   const int lpad = (int)lpad32(max_seq_len);
   auto lds_fits = [&](int x) { return (size_t)4 * hpt * ((size_t)split_wtok(lpad, x) * 6 + (size_t)head_size * 4) + 16 <= R.lds_per_cu; };
+  const int loaded = qpk == 1 || f8 ? R.split_min_blocks_per_wave_loaded : head_size == 64 ? R.split_gqa_blocks_per_wave_d64 : R.split_gqa_blocks_per_wave;
   int xw = 0;
   for (int x = hpt > 1 ? 64 : SPLIT_MAX_WAVES; x >= 8; x /= 2) {
     const long wgs = nitems * (x / 4);
     const int bpw = nblk / x;
     if (lds_fits(x) &&
-        ((wgs <= g_cus && bpw >= R.split_min_blocks_per_wave) || (wgs <= cap && bpw >= R.split_min_blocks_per_wave_loaded))) { xw = x; break; }
+        ((wgs <= g_cus && bpw >= R.split_min_blocks_per_wave) || (wgs <= cap && bpw >= loaded))) { xw = x; break; }
   }
   if (starved) {
     // Contexts too long for several waves' logits in one workgroup's LDS: at least the narrowest form of which three workgroups
@@ -1151,7 +1206,9 @@ int launch_pa_v1(void* out, const void* query, const void* key_cache,
                        workspace_bytes >= (int64_t)pa_split_layout(head_size).bytes;
   if (!sparse_v && picked && have_ws && !append && f8 != 2 && !bf) {
     // a caller-owned workspace lets an under-filled launch spread each (sequence, head) over several workgroups
-    if (const int sv = pick_split(num_seqs, num_heads, head_size, block_size, max_seq_len, variant, num_heads / num_kv_heads, f8)) variant = sv;
+    const int qpk = num_heads / num_kv_heads, ph = f8 || g_pv_mfma ? 0 : pick_per_head(num_seqs, num_heads, qpk, head_size, block_size, max_seq_len);
+    if (ph) variant = ph;
+    else if (const int sv = pick_split(num_seqs, num_heads, head_size, block_size, max_seq_len, variant, qpk, f8)) variant = sv;
   }
   if (!sparse_v && (variant < 1 || variant > nvariants_v1()))
     return fail(VMI_E_VARIANT, "paged_attention_v1: unknown variant %d", variant);
@@ -1711,6 +1768,8 @@ int vmi_paged_attention_v1_pick_variant_ws(int32_t num_seqs, int32_t num_heads, 
   if (!vmi::head_size_supported(head_size) || !vmi::block_size_supported(block_size)) return 0;
   if (num_kv_heads <= 0) num_kv_heads = num_heads;
   if (num_heads % num_kv_heads) return 0;
+  if (!vmi::g_pv_mfma)
+    if (const int ph = vmi::pick_per_head(num_seqs, num_heads, num_heads / num_kv_heads, head_size, block_size, max_seq_len)) return ph;
   int plain = vmi::pick_variant_gqa(num_seqs, num_heads, num_heads / num_kv_heads, head_size, block_size, max_seq_len, false, 0);
   if (!plain) plain = vmi::pick_variant(num_seqs, num_heads, head_size, block_size, max_seq_len);
   plain = vmi::fit_lds(plain, head_size, block_size, ((max_seq_len + 31) / 32) * 32, false, 0);
