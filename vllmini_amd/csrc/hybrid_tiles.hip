@@ -143,15 +143,17 @@ int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
 //
 // Alone, 5300 pairs of 48 to 9000 rows, K 256 to 12 288, N 256 to 16 384: ours / library's in the mean, from 5.6 million results on (below, nearly all of the library's time is its call:
 // 19 us of host) and whole tiles of 256 columns: K 1024 to 2047 0.88 (8 of 207 more than 5 per cent behind), to 4095 0.96 (52 of 239), to 6144 1.00 (30 of 104), beyond 1.07; other columns
-// 0.74, 0.85, 0.96 and 0.99.  So not past K 6144 from 5.6 million results on, up to there whole columns only where the tiles' own costs promise 1020 TFLOP/s (N 2048, K 6144: 2773 rows
-// 69 / 60, which one round of tiles holds; 4500 103 / 111), and below K 4096 whole columns up to 9 million (N 4096, K 2048: 2400 41 / 42, level from there on), below 2048 up to 15.
+// 0.74, 0.85, 0.96 and 0.99.  So not past K 6144 from 5.6 million results on, up to there whole columns up to 9 million (N 3072, K 4608, 4100 rows 90 / 109) and only where the tiles' own costs promise 1020
+// TFLOP/s (N 2048, K 6144: 2773 rows 69 / 60, which one round of tiles holds; 3250 73 / 85), and below K 4096 whole columns up to 9 million (N 4096, K 2048: 2400 41 / 42, level from there on), below 2048 up to 15.
 // Not where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4), where tiles of 64 x 64 are just more than
 // the chip has compute units for (300 rows, N 4096, K 8192 46 / 56; 600 rows, N 2048, K 6144 34 / 37), and past K 16 383.
 static bool product_pays(int M, int N, int K) {
   const bool whole = N % 256 == 0;
   const int64_t results = (int64_t)M * N, least = (int64_t)((M + 31) / 32) * ((N + 63) / 64);
   if (K >= 4096) {
-    if (results >= 5600000 && (K > 6144 || (whole && vmi_tiles::tiles_cost(vmi_tiles::tiles_pick(M, N, K), M, N, K, 1) > 2. / 1.02e9 * (double)results * K))) return false;
+    if (results >= 5600000 &&
+        (K > 6144 || (whole && (results >= 9000000 || vmi_tiles::tiles_cost(vmi_tiles::tiles_pick(M, N, K), M, N, K, 1) > 2. / 1.02e9 * (double)results * K))))
+      return false;
   } else if (whole && K >= 1024 && results >= (K >= 2048 ? 9000000 : 15000000)) {
     return false;
   }
