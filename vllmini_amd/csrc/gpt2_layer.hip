@@ -895,7 +895,12 @@ static int launch_prompt(const PromptParams& p, int n_tiles, hipStream_t stream)
       return VMI_LAYER_E_HIP;
     }
   }
-  hipLaunchKernelGGL(fn, dim3(n_tiles, p.heads), dim3(256), lds, stream, p);
+  const int most = (1 << 23) / p.heads;   // (a launch is of fewer than 2^32 work items)
+  for (int t0 = 0; t0 < n_tiles; t0 += most) {
+    PromptParams q = p;
+    q.tiles += (int64_t)4 * t0;
+    hipLaunchKernelGGL(fn, dim3((uint32_t)(p.heads * std::min(most, n_tiles - t0))), dim3(256), lds, stream, q);
+  }
   return VMI_LAYER_OK;
 }
 

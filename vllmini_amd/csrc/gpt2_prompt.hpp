@@ -5,18 +5,20 @@
 // positions of one head and walks the keys up to its last position in tiles of 64, each through LDS once (requested one tile ahead,
 // two buffers, one barrier a tile).  A wave owns 16 * MI queries for all of it:
 //   * scores are formed transposed, S^T = K Q^T (D[row = key 4 kc + r][col = query r16]), so a lane keeps the scores of ONE query: its
-//     statistics need no LDS, its maximum two cross-lane swaps, and its probabilities, as they lie, are the B operand of
+//     statistics need no LDS, its maximum two cross-lane swaps, its sum a product with ones, and its probabilities, as they lie, are the B operand of
 //     O^T = V^T P^T: the sum over keys may take them in any order, so k-index 8 kc + e of a step of 32 stands for key 4 kc + e
 //     (e < 4) and 16 + 4 kc + e - 4, and the V^T operand is read column-wise from LDS in that same order (ds_read_b64_tr_b16);
 //   * the key tiles that lie on the workgroup's own positions are its prompt's pages: they leave from LDS as whole 16-byte pieces of
 //     the cache's layout, K[blk, h, d / 8, off, d % 8] and V[blk, h, d, off] — the bytes that reshape_and_cache would write.
 // Scores, softmax and accumulators are fp32; a probability is rounded once to half and what is summed is what multiplies V.
 //
-// What bounds it: the chain of a tile (LDS, scores, softmax, values: about 1.5 us) times the longest prompt's tiles, and from some
-// thousand workgroups on the vector unit's share of the softmax; the matrix cores are mostly idle, as few of a prompt's products are
-// here.  As a sequence of its own per position, for paged_attention_v1, every position read its keys again, and the cache was written by
-// a launch in front in 2-byte pieces.  24 prompts of up to 512 tokens (6 146 in all), 12 heads of 64, a layer: 205.6 + 30.2 -> 23.4 us; one
-// prompt of 37: 5.1 + 3.2 -> 3.9 us.
+// What bounds it: the vector unit's share of the softmax (a maximum, a multiply-add, an exponential and half a conversion a score; the scale is in the multiply-add, the sums are
+// in the matrix cores, which are mostly idle) and the chain of a tile (LDS, scores, softmax, values: 0.65 us) times the longest prompt's tiles.  So the longest walks begin first,
+// over all heads: as one head behind the other the last head's began when the first ones' were done.  Keys shared out over two or four groups of waves of a workgroup, their sums
+// merged at the end: one of 900 13.3 -> 12.3 us, 6 of 900 17.2 -> 15.5, but 24 of up to 512 17.7 -> 21.5 and up to 200 tokens behind everywhere: not kept.
+// As a sequence of its own per position, for paged_attention_v1, every position read its keys again, and the cache was written by a launch in front in 2-byte pieces.
+// 24 prompts of up to 512 tokens (6 439 in all), 12 heads of 64, a layer: 205.6 + 30.2 -> 23.2 us, with a scaled, rounded and added score and heads outermost -> 17.7; one
+// prompt of 37: 5.1 + 3.2 -> 3.9 us, of 900 16.8 -> 13.3; 16 heads of 128, 4 of 900 34.2 -> 27.1.
 #pragma once
 #include "mfma_tiles.hpp"
 
@@ -101,8 +103,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   h16* lds = reinterpret_cast<h16*>(smem);   // [2 buffers][K, V][64][LD]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int4 tile = *reinterpret_cast<const int4*>(p.tiles + 4 * blockIdx.x);
-  const int h = blockIdx.y, q0 = tile.z, len = tile.w, E = p.heads * D;
+  const int h = blockIdx.x % p.heads;   // (the heads of a tile one behind the other: the longest walks, which the list has first, all begin first)
+  const int4 tile = *reinterpret_cast<const int4*>(p.tiles + 4 * (blockIdx.x / p.heads));
+  const int q0 = tile.z, len = tile.w, E = p.heads * D;
   const h16* row0 = p.qkv + (int64_t)tile.y * p.ld + h * D;
   const int32_t* table = p.table + (int64_t)tile.x * p.table_ld;
   const int end = min(len, q0 + 64 * MI), nkt = (end + PKT - 1) / PKT;
@@ -131,6 +134,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
 #pragma unroll
     for (int k = 0; k < NK; ++k)
       qf[mi][k] = *reinterpret_cast<const h16x8*>(row0 + (int64_t)min(w0 + mi * 16 + r16, len - 1) * p.ld + 32 * k + 8 * kc);
+  h16x8 ones;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ones[e] = (h16)1.f;
   f32x4 o[MI][NT];
   float mrun[MI], lrun[MI];
 #pragma unroll
@@ -195,32 +201,35 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
       }
     }
     const bool whole = key0 + PKT - 1 <= w0;   // every query sees every key
+    if (!whole) {
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (key0 + j * 16 + 4 * kc + r > w0 + mi * 16 + r16) sc[mi][j][r] = -INFINITY;
+    }
     h16x8 pf[MI][2];
 #pragma unroll
     for (int mi = 0; mi < MI; ++mi) {
-      const int q = w0 + mi * 16 + r16;
-      float mx = -INFINITY;
+      float mx = sc[mi][0][0];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          sc[mi][j][r] *= p.scale2;
-          if (!whole && key0 + j * 16 + 4 * kc + r > q) sc[mi][j][r] = -INFINITY;
-          mx = fmaxf(mx, sc[mi][j][r]);
-        }
-      mx = fmaxf(mrun[mi], over_kc(mx, [](float a, float b) { return fmaxf(a, b); }));
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[mi][j][r]);
+      mx = fmaxf(mrun[mi], p.scale2 * over_kc(mx, [](float a, float b) { return fmaxf(a, b); }));
       const float alpha = __builtin_amdgcn_exp2f(mrun[mi] - mx);
       mrun[mi] = mx;
-      float sum = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const h16 pr = (h16)__builtin_amdgcn_exp2f(sc[mi][j][r] - mx);
-          sum += (float)pr;
-          pf[mi][j >> 1][(j & 1) * 4 + r] = pr;
-        }
-      lrun[mi] = lrun[mi] * alpha + sum;
+        for (int r = 0; r < 4; ++r) pf[mi][j >> 1][(j & 1) * 4 + r] = (h16)__builtin_amdgcn_exp2f(__builtin_fmaf(sc[mi][j][r], p.scale2, -mx));
+      // (what is summed is what multiplies V: a product with ones, whose every row is the sums)
+      f32x4 sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pf[mi][k], sum, 0, 0, 0);
+      lrun[mi] = __builtin_fmaf(lrun[mi], alpha, sum[0]);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) o[mi][nt] *= alpha;
     }
@@ -247,7 +256,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attention_kernel(const PromptPa
   }
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi) {
-    const float inv = 1.f / over_kc(lrun[mi], [](float a, float b) { return a + b; });
+    const float inv = 1.f / lrun[mi];
     const int q = w0 + mi * 16 + r16;
     if (q >= len) continue;
     h16* out = p.out + (int64_t)(tile.y + q) * p.ldo + h * D + 4 * kc;
