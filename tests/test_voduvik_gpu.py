@@ -626,6 +626,32 @@ def test_recurrence_over_portions_of_every_size(dtype, width, blocks, taps):
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("width,blocks", [(512, 2), (320, 2), (192, 3), (600, 1)])
+def test_recurrence_over_portions_in_wide_blocks(dtype, width, blocks):
+    """Four taps, rows taken together: blocks of one and two shares of a workgroup's channels (the second not all there), and of several chunks."""
+    test_recurrence_over_portions_of_every_size(dtype, width, blocks, 4)
+
+
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("width,blocks", [(512, 2), (96, 3)])
+def test_portions_that_share_rows_taken_together_with_padding(dtype, width, blocks):
+    """Portions of one to nine tokens, so that the eight (four) rows of a thread hold several starts, and rows behind them that are no token's and hold NaN."""
+    from vllmini_amd import hybrid_ops as ops
+
+    counts = [1, 2, 3, 9, 5, 1, 7, 64, 4, 2]
+    k, T, pad = _Rglru(width, blocks, 4, dtype, slots=len(counts)), sum(counts), 5
+    seqs = [k.inputs(n, 90 + i) for i, n in enumerate(counts)]
+    step = layout(counts, [0] * len(counts), [[0]] * len(counts), 64, pos_slots=False)
+    f = dict(step.fields)
+    f["tok_seq"], f["tok_pos"], f["tok_slot"] = (torch.cat([f[n], i32([v] * pad)]) for n, v in (("tok_seq", -1), ("tok_pos", 0), ("tok_slot", -1)))
+    yx = torch.cat([s[2] for s in seqs] + [torch.full((pad, 2 * k.layer.width), float("nan"), dtype=dtype, device=dev())])
+    got = k.run(yx, ops.StepLayout(f, T + pad, len(counts), 64, False, True, max(counts), max(counts)))
+    assert not got[T:].any()
+    for s, g in zip(seqs, got[:T].split(counts)):
+        close(g, k.plain(*s[:2]), dtype, tol32=3e-5, tol16=1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 def test_recurrence_decodes_like_it_prefills_and_skips_padding_rows(dtype):
     from vllmini_amd import hybrid_ops as ops
 

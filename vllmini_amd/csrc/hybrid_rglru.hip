@@ -2,7 +2,7 @@
 // recurrence -> product with gelu(y).
 //
 // The packed tokens are cut into row tiles of BM consecutive rows, whatever entries they belong to.  A workgroup takes one row
-// tile x up to 64 channels of one gate block: the convolution of the block's channels goes to LDS (element type), both gate
+// tile x up to CT channels of one gate block: the convolution of the block's channels goes to LDS (element type), both gate
 // matrices run on the matrix cores (A = gate rows = channels, B = u rows = tokens, fp32 accumulation), and everything behind the
 // product is fp32: r, i, log a = decay * r, a, b = sqrt(1 - a^2) * i * u.  A token that opens an entry's portion folds the state
 // of its slot in at once (b += a * S, a = 0), so one uniform walk S = a S + b, P = a P over the tile serves any mix of entries:
@@ -17,7 +17,6 @@
 
 namespace vmi_hybrid {
 
-constexpr int CT = 64;      // channels of a workgroup
 constexpr int KCH = 256;    // channels of u in LDS at a time
 constexpr int MAX_TAPS = 16;
 
@@ -25,15 +24,39 @@ struct RowMeta {
   int seq, qs, len, ctx, slot, flip, first, last;
 };
 
-template <typename T, int BM>
+template <typename T, int BM, int CT>
 struct Lds {
   static constexpr int LDU = KCH + 16 / (int)sizeof(T), LDA = CT + 4;
-  T u[BM * LDU];
-  float a[BM * LDA];
-  float b[BM * LDA];
-  float end[2][4][CT];
+  union {   // u until the gates' products are done, then the states
+    T u[BM * LDU];
+    float S[BM * LDA];
+  };
   RowMeta meta[BM];
 };
+
+// Lane 15's value to the 16 lanes of its row.
+__device__ __forceinline__ float lane15(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x15f, 0xf, 0xf, true));
+}
+// Four recurrences S = A S + B over the 16 lanes of a row, in place: the lane D below's pair (0 and unchanged where there is none) in front of a lane's own, D = 1, 2, 4, 8.  As
+// builtins a step was six instructions a value, of them four moves; here it is two, and each is eight behind the one whose result it takes from another lane (two are asked for).
+__device__ __forceinline__ void walk16(f32x4& A, f32x4& B) {
+  float a0 = A[0], a1 = A[1], a2 = A[2], a3 = A[3], b0 = B[0], b1 = B[1], b2 = B[2], b3 = B[3];
+#define VMI_STEP(D)                                                                 \
+  "v_fmac_f32_dpp %4, %4, %0 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:0\n" \
+  "v_fmac_f32_dpp %5, %5, %1 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:0\n" \
+  "v_fmac_f32_dpp %6, %6, %2 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:0\n" \
+  "v_fmac_f32_dpp %7, %7, %3 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:0\n" \
+  "v_mul_f32_dpp %0, %0, %0 row_shr:" #D " row_mask:0xf bank_mask:0xf\n"               \
+  "v_mul_f32_dpp %1, %1, %1 row_shr:" #D " row_mask:0xf bank_mask:0xf\n"               \
+  "v_mul_f32_dpp %2, %2, %2 row_shr:" #D " row_mask:0xf bank_mask:0xf\n"               \
+  "v_mul_f32_dpp %3, %3, %3 row_shr:" #D " row_mask:0xf bank_mask:0xf\n"
+  asm("s_nop 1\n" VMI_STEP(1) VMI_STEP(2) VMI_STEP(4) VMI_STEP(8)
+      "s_nop 1"
+      : "+v"(a0), "+v"(a1), "+v"(a2), "+v"(a3), "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3));
+#undef VMI_STEP
+  A = f32x4{a0, a1, a2, a3}, B = f32x4{b0, b1, b2, b3};
+}
 
 // convolution of 8 channels for the token of row m.  TAPS = 0: any number of taps; else exactly that many, every load issued
 // without a condition around it (taps before the start read a valid row and count zero), so that all of them are in flight
@@ -59,6 +82,7 @@ __device__ __forceinline__ f32x8 conv8(const vmi_hy_rglru_args& p, const RowMeta
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) tap(j);
   } else {
+#pragma unroll 1
     for (int j = 0; j < taps; ++j) tap(j);
   }
   return acc;
@@ -72,12 +96,18 @@ __device__ __forceinline__ void store_out8(const vmi_hy_rglru_args& p, int t, in
   *reinterpret_cast<V8<T>*>(static_cast<T*>(p.out) + (int64_t)t * p.ldo + c) = from_f32<T>(o);
 }
 
-template <typename T, int BM, int TAPS>
-__global__ __launch_bounds__(256, 2) void rglru_tile_kernel(const vmi_hy_rglru_args p, const vmi_hy_step s) {
-  constexpr int MT = BM / 16;
+// CT channels of one gate block to a workgroup, 16 to a wave.  A lane's gate results are four channels of one row of each 16, so the walk over a tile stays in registers: four
+// doubling steps across the 16 lanes of a row group, then group after group through lane 15.
+// Bound by the instructions of a wave, some 2500 of them issued one by one (two waves a SIMD, whose registers no more fit: at 128 they spill), and by five trips to memory in front
+// of them.  So 128 channels (each workgroup of a block convolves all of its channels, 64 do so twice as often), inputs and weights asked for before the tables are there, a portion's
+// first rows from the same registers as its others (they went one by one), and no walk through LDS (16 rows a wave, twice, four barriers).  us, blocks of 256: width 1024, 6 x 20
+// tokens 18.7 -> 14.1, 48 x 80 22.2 -> 15.5, 4 x up to 1000 25.1 -> 24.5; 2048, 4 x up to 1024 43.0 -> 38.5, 40 x 100 39.6 -> 28.9; 4096, 4 x 300 32.1 -> 26.3.
+template <typename T, int BM, int TAPS, int CT>
+__global__ __launch_bounds__(4 * CT, 2) void rglru_tile_kernel(const vmi_hy_rglru_args p, const vmi_hy_step s) {
+  constexpr int MT = BM / 16, TH = 4 * CT;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  auto& L = *reinterpret_cast<Lds<T, BM>*>(smem);
-  constexpr int LDU = Lds<T, BM>::LDU, LDA = Lds<T, BM>::LDA;
+  auto& L = *reinterpret_cast<Lds<T, BM, CT>*>(smem);
+  constexpr int LDU = Lds<T, BM, CT>::LDU, LDA = Lds<T, BM, CT>::LDA;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
   const int bw = p.width / p.blocks, per = (bw + CT - 1) / CT;
   const int blk = blockIdx.x / per, cin = (blockIdx.x % per) * CT;   // gate block, first channel inside it
@@ -109,24 +139,37 @@ __global__ __launch_bounds__(256, 2) void rglru_tile_kernel(const vmi_hy_rglru_a
   const T* wi = wr + p.blocks * gsz;
   // requested now, used behind the products
   const int cl = wave * 16 + 4 * kc;
-  f32x4 br, bi, dec, S0[MT];
+  f32x4 br, bi, dec;
   if (wvalid) {
     br = *reinterpret_cast<const f32x4*>(p.gate_b + c0 + cl);
     bi = *reinterpret_cast<const f32x4*>(p.gate_b + p.width + c0 + cl);
     dec = *reinterpret_cast<const f32x4*>(p.decay + c0 + cl);
   }
-  __syncthreads();   // meta is there
+  // eight channels of this many consecutive rows to a thread: past the taps of their portions' starts they share their inputs, which need no table to be asked for
+  constexpr bool TOGETHER = BM == 64 && TAPS > 0;
+  constexpr int RPT = TOGETHER ? BM * (KCH / 8) / TH : 1;
+  const int kr = (tid % (KCH / 8)) * 8, m0 = tid / (KCH / 8) * RPT;
+  V8<T> v[TOGETHER ? TAPS - 1 + RPT : 1];
+  f32x8 w[TOGETHER ? TAPS : 1], wb;
+  auto ask = [&](int k0) {
+    if constexpr (TOGETHER) {
+      const int c = blk * bw + k0 + min(kr, min(KCH, bw - k0) - 8);
 #pragma unroll
-  for (int mi = 0; mi < MT; ++mi) {
-    const RowMeta& r = L.meta[mi * 16 + r16];
-    S0[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (wvalid && r.seq >= 0 && r.first && r.ctx > 0) S0[mi] = *reinterpret_cast<const f32x4*>(p.state + (int64_t)r.slot * p.width + c0 + cl);
-  }
-  constexpr int YU = (BM * (CT / 8) + 255) / 256;   // this thread's units of the output: y
+      for (int j = 0; j < TAPS; ++j) w[j] = load8(p.conv_w + (int64_t)j * p.width + c);
+      wb = load8(p.conv_b + c);
+      const T* in = static_cast<const T*>(p.yx) + p.width + blk * bw + k0 + min(kr, min(KCH, bw - k0) - 8);
+#pragma unroll
+      for (int j = 0; j < TAPS - 1 + RPT; ++j) v[j] = load8(in + (int64_t)min(max(t0 + m0 - (TAPS - 1) + j, 0), s.T - 1) * p.ldx);
+    }
+  };
+  constexpr bool SOON = sizeof(T) == 2;   // (in 32 bits they spill)
+  if constexpr (SOON) ask(0);
+  __syncthreads();   // meta is there
+  constexpr int YU = (BM * (CT / 8) + TH - 1) / TH;   // this thread's units of the output: y
   V8<T> yv[YU];
 #pragma unroll
   for (int i = 0; i < YU; ++i) {
-    const int m = (tid + i * 256) / (CT / 8), k = ((tid + i * 256) % (CT / 8)) * 8;
+    const int m = (tid + i * TH) / (CT / 8), k = ((tid + i * TH) % (CT / 8)) * 8;
     yv[i] = load8(static_cast<const T*>(p.yx) + (int64_t)(t0 + min(m, rows - 1)) * p.ldx + c0 + min(k, nch - 8));
   }
   for (int k0 = 0; k0 < bw; k0 += KCH) {
@@ -143,42 +186,44 @@ __global__ __launch_bounds__(256, 2) void rglru_tile_kernel(const vmi_hy_rglru_a
 #pragma unroll
       for (int k = 0; k < AHEAD; ++k) load_gates(k, k);
     }
+    if (!SOON || k0 > 0) ask(k0);
     if (k0 > 0) __syncthreads();   // the previous chunk has been read
-    auto conv_row = [&](int m, int k) {
+    auto conv_row = [&](int m, int k) {   // (beside rows that are taken together: the loop over taps, whose registers they need)
       const RowMeta& r = L.meta[m];
-      if (r.seq >= 0 && k < kn) *reinterpret_cast<V8<T>*>(L.u + m * LDU + k) = from_f32<T>(conv8<T, TAPS>(p, r, t0 + m, blk * bw + k0 + k));
+      if (r.seq >= 0 && k < kn) *reinterpret_cast<V8<T>*>(L.u + m * LDU + k) = from_f32<T>(conv8<T, TOGETHER ? 0 : TAPS>(p, r, t0 + m, blk * bw + k0 + k));
       else if (k < kn) *reinterpret_cast<V8<T>*>(L.u + m * LDU + k) = zero8<T>();
     };
-    if constexpr (BM == 64 && TAPS > 0) {
-      // eight channels of eight consecutive rows: inside one portion, past its first taps, the rows share their inputs
-      const int k = (tid % (KCH / 8)) * 8, m0 = (tid / (KCH / 8)) * 8;
-      const RowMeta &ra = L.meta[m0], &rb = L.meta[m0 + 7];
-      if (k < kn && ra.seq >= 0 && ra.seq == rb.seq && t0 + m0 - (TAPS - 1) >= ra.qs) {
-        const int c = blk * bw + k0 + k;
-        const T* in = static_cast<const T*>(p.yx) + (int64_t)(t0 + m0 - (TAPS - 1)) * p.ldx + p.width + c;
-        V8<T> v[TAPS + 7];
-        f32x8 w[TAPS];
+    if constexpr (TOGETHER) {
+      const RowMeta &ra = L.meta[m0], &rb = L.meta[m0 + RPT - 1];
+      const bool inside = ra.seq >= 0 && ra.seq == rb.seq && t0 + m0 - (TAPS - 1) >= ra.qs;
+      bool tails = false;   // whether a row's taps reach into what its sequence had before
+      if (!inside) {
 #pragma unroll
-        for (int j = 0; j < TAPS + 7; ++j) v[j] = load8(in + (int64_t)j * p.ldx);
+        for (int m = 0; m < RPT; ++m) {
+          const RowMeta& r = L.meta[m0 + m];
+          tails |= r.seq >= 0 && r.ctx > 0 && t0 + m0 + m - (TAPS - 1) < r.qs;
+        }
+      }
+      if (k0 + kr < k0 + kn && !tails) {
 #pragma unroll
-        for (int j = 0; j < TAPS; ++j) w[j] = load8(p.conv_w + (int64_t)j * p.width + c);
-        const f32x8 b = load8(p.conv_b + c);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-          f32x8 acc = b;
+        for (int m = 0; m < RPT; ++m) {
+          f32x8 acc = wb;
+          const int back = inside ? TAPS - 1 : L.meta[m0 + m].seq < 0 ? -1 : min(t0 + m0 + m - L.meta[m0 + m].qs, TAPS - 1);   // rows of this portion before this one
 #pragma unroll
           for (int j = 0; j < TAPS; ++j)
+            if (TAPS - 1 - j <= back) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = fmaf(w[j][e], (float)v[m + j][e], acc[e]);
-          *reinterpret_cast<V8<T>*>(L.u + (m0 + m) * LDU + k) = from_f32<T>(acc);
+              for (int e = 0; e < 8; ++e) acc[e] = fmaf(w[j][e], (float)v[m + j][e], acc[e]);
+            }
+          *reinterpret_cast<V8<T>*>(L.u + (m0 + m) * LDU + kr) = back < 0 ? zero8<T>() : from_f32<T>(acc);
         }
-      } else {
+      } else if (kr < kn) {
 #pragma unroll 1
-        for (int m = 0; m < 8; ++m) conv_row(m0 + m, k);
+        for (int m = 0; m < RPT; ++m) conv_row(m0 + m, kr);
       }
     } else {
 #pragma unroll 2
-      for (int u = tid; u < BM * (KCH / 8); u += 256) conv_row(u / (KCH / 8), (u % (KCH / 8)) * 8);
+      for (int u = tid; u < BM * (KCH / 8); u += TH) conv_row(u / (KCH / 8), (u % (KCH / 8)) * 8);
     }
     __syncthreads();
     if (wvalid) {
@@ -197,100 +242,79 @@ __global__ __launch_bounds__(256, 2) void rglru_tile_kernel(const vmi_hy_rglru_a
       }
     }
   }
-  // the workgroup's own channels of u: into b, from LDS or (a block of several chunks) computed again
+  // the workgroup's own channels of u are in LDS, or (a block of several chunks) computed again
   const bool held = bw <= KCH;
-  if (held) __syncthreads();
-  for (int u = tid; u < BM * (CT / 8); u += 256) {
-    const int m = u / (CT / 8), k = (u % (CT / 8)) * 8;
-    const RowMeta& r = L.meta[m];
-    f32x8 v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = 0.f;
-    if (held && k < nch) v = to_f32<T>(load8(L.u + m * LDU + cin + k));
-    else if (r.seq >= 0 && k < nch) v = to_f32<T>(from_f32<T>(conv8<T, TAPS>(p, r, t0 + m, c0 + k)));   // rounded as the gates saw it
-    *reinterpret_cast<f32x8*>(L.b + m * LDA + k) = v;
+  if (!held) {
+    __syncthreads();
+    for (int u = tid; u < BM * (CT / 8); u += TH) {
+      const int m = u / (CT / 8), k = (u % (CT / 8)) * 8;
+      const RowMeta& r = L.meta[m];
+      V8<T> x = zero8<T>();
+      if (r.seq >= 0 && k < nch) x = from_f32<T>(conv8<T, TOGETHER ? 0 : TAPS>(p, r, t0 + m, c0 + k));   // rounded as the gates saw it
+      *reinterpret_cast<V8<T>*>(L.u + m * LDU + k) = x;
+    }
+    __syncthreads();
   }
-  __syncthreads();
+  const bool lead0 = L.meta[0].seq >= 0 && !L.meta[0].first;   // the tile opens inside a portion
+  const int lead_end = lead0 ? min(rows, L.meta[0].qs + L.meta[0].len - t0) : 0;   // rows of the leading segment
+  // a row that is unfinished, or what the next tile's carry starts from: its state and product go to scratch
+  auto kept = [&](int m, const RowMeta& r) { return m < rows && r.seq >= 0 && (m < lead_end || (m == BM - 1 && !r.last)); };
+  f32x4 Sc{0.f, 0.f, 0.f, 0.f}, Pc;
+  Pc[0] = Pc[1] = Pc[2] = Pc[3] = lead0 ? 1.f : 0.f;
   if (wvalid) {
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) {
       const int m = mi * 16 + r16;
       const RowMeta& r = L.meta[m];
-      const f32x4 u = *reinterpret_cast<const f32x4*>(L.b + m * LDA + cl);
-      f32x4 a, b;
+      const T* u = L.u + m * LDU + (held ? cin : 0) + cl;
+      f32x4 &a = ar[mi], &b = ai[mi];
+      const bool first = r.first, goes_on = first && r.ctx > 0;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float la = dec[e] * sigmoid(ar[mi][e] + br[e]);
+      for (int e = 0; e < 4; ++e) {   // (a row that is no token's: u and with it b is 0, and what follows it opens a portion)
+        const float la = dec[e] * sigmoid(a[e] + br[e]);
         a[e] = exp_hw(la);
-        b[e] = __builtin_amdgcn_sqrtf(one_minus_exp(-2.f * la, a[e] * a[e])) * sigmoid(ai[mi][e] + bi[e]) * u[e];
-        if (r.seq < 0) a[e] = 1.f, b[e] = 0.f;
-        if (r.first) {
-          b[e] = fmaf(a[e], S0[mi][e], b[e]);
-          a[e] = 0.f;
+        b[e] = __builtin_amdgcn_sqrtf(one_minus_exp(-2.f * la, a[e] * a[e])) * sigmoid(b[e] + bi[e]) * (float)u[e];
+      }
+      if (goes_on) b += a * *reinterpret_cast<const f32x4*>(p.state + (int64_t)r.slot * p.width + c0 + cl);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] = first ? 0.f : a[e];
+      if (!p.single) {
+        walk16(a, b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          b[e] = fmaf(a[e], Sc[e], b[e]);
+          a[e] *= Pc[e];
+          if (mi + 1 < MT) Sc[e] = lane15(b[e]), Pc[e] = lane15(a[e]);
         }
-      }
-      *reinterpret_cast<f32x4*>(L.a + m * LDA + cl) = a;
-      *reinterpret_cast<f32x4*>(L.b + m * LDA + cl) = b;
-    }
-  }
-  __syncthreads();
-  const bool lead0 = L.meta[0].seq >= 0 && !L.meta[0].first;   // the tile opens inside a portion
-  if (!p.single) {   // the walk, in place (b becomes S, a becomes P): a wave takes a quarter of the rows, a lane a channel
-    constexpr int RW = BM / 4;
-    float* pa = L.a + wave * RW * LDA + lane;
-    float* pb = L.b + wave * RW * LDA + lane;
-    if (lane < nch) {
-      float S = 0.f, P = wave == 0 ? (lead0 ? 1.f : 0.f) : 1.f;
-#pragma unroll 8
-      for (int m = 0; m < RW; ++m) {
-        const float a = pa[m * LDA], b = pb[m * LDA];
-        S = fmaf(a, S, b);
-        P *= a;
-        pb[m * LDA] = S;
-        pa[m * LDA] = P;
-      }
-      L.end[0][wave][lane] = S;
-      L.end[1][wave][lane] = P;
-    }
-    __syncthreads();
-    if (lane < nch && wave > 0) {   // what the quarters before this one hand over
-      float S = L.end[0][0][lane], P = L.end[1][0][lane];
-      for (int w = 1; w < wave; ++w) {
-        S = fmaf(L.end[1][w][lane], S, L.end[0][w][lane]);
-        P *= L.end[1][w][lane];
-      }
-#pragma unroll 8
-      for (int m = 0; m < RW; ++m) {
-        pb[m * LDA] = fmaf(pa[m * LDA], S, pb[m * LDA]);
-        pa[m * LDA] *= P;
+        if (kept(m, r)) *reinterpret_cast<f32x4*>(p.scratch + ((int64_t)s.T + t0 + m) * p.width + c0 + cl) = a;
       }
     }
   }
+  __syncthreads();   // (u has been read)
+  if (wvalid) {
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) *reinterpret_cast<f32x4*>(L.S + (mi * 16 + r16) * LDA + cl) = ai[mi];
+  }
   __syncthreads();
-  const int lead_end = lead0 ? min(rows, L.meta[0].qs + L.meta[0].len - t0) : 0;   // rows of the leading segment
 #pragma unroll
   for (int i = 0; i < YU; ++i) {
-    const int u = tid + i * 256, m = u / (CT / 8), k = (u % (CT / 8)) * 8;
+    const int u = tid + i * TH, m = u / (CT / 8), k = (u % (CT / 8)) * 8;
     if (m >= rows || k >= nch) continue;
     const RowMeta& r = L.meta[m];
-    const f32x8 S = *reinterpret_cast<const f32x8*>(L.b + m * LDA + k);
+    const f32x8 S = *reinterpret_cast<const f32x8*>(L.S + m * LDA + k);
     const int t = t0 + m, c = c0 + k;
     if (r.seq < 0) {
       *reinterpret_cast<V8<T>*>(static_cast<T*>(p.out) + (int64_t)t * p.ldo + c) = zero8<T>();
       continue;
     }
-    const bool lead = m < lead_end;
-    if (lead || (m == BM - 1 && !r.last)) {   // unfinished, or what the next tile's carry starts from
-      *reinterpret_cast<f32x8*>(p.scratch + (int64_t)t * p.width + c) = S;
-      *reinterpret_cast<f32x8*>(p.scratch + ((int64_t)s.T + t) * p.width + c) = *reinterpret_cast<const f32x8*>(L.a + m * LDA + k);
-    }
-    if (lead) continue;
+    if (!p.single && kept(m, r)) *reinterpret_cast<f32x8*>(p.scratch + (int64_t)t * p.width + c) = S;
+    if (m < lead_end) continue;
     store_out8<T>(p, t, c, S, to_f32<T>(yv[i]));
     if (r.last) *reinterpret_cast<f32x8*>(p.state + (int64_t)r.slot * p.width + c) = S;
   }
   // the convolution tail of entries that end in this tile, into its other half
   const int nt = p.taps - 1;
-  for (int u = tid; u < rows * nt * (CT / 8); u += 256) {
+  for (int u = tid; u < rows * nt * (CT / 8); u += TH) {
     const int k = (u % (CT / 8)) * 8, e = u / (CT / 8) % nt, m = u / (CT / 8) / nt, c = c0 + k;
     const RowMeta& r = L.meta[m];
     if (k >= nch || r.seq < 0 || !r.last) continue;
@@ -505,12 +529,12 @@ static int launch_step(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStre
   return launched("vmi_hy_rglru");
 }
 
-template <typename T, int BM, int TAPS>
+template <typename T, int BM, int TAPS, int CT>
 static int launch_tile(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream_t st) {
-  auto* fn = rglru_tile_kernel<T, BM, TAPS>;
-  if (int rc = allow_lds(fn, sizeof(Lds<T, BM>), "vmi_hy_rglru")) return rc;
+  auto* fn = rglru_tile_kernel<T, BM, TAPS, CT>;
+  if (int rc = allow_lds(fn, sizeof(Lds<T, BM, CT>), "vmi_hy_rglru")) return rc;
   const int bw = p.width / p.blocks;
-  hipLaunchKernelGGL(fn, dim3(p.blocks * ((bw + CT - 1) / CT), (s.T + BM - 1) / BM), dim3(256), sizeof(Lds<T, BM>), st, p, s);
+  hipLaunchKernelGGL(fn, dim3(p.blocks * ((bw + CT - 1) / CT), (s.T + BM - 1) / BM), dim3(4 * CT), sizeof(Lds<T, BM, CT>), st, p, s);
   return launched("vmi_hy_rglru");
 }
 
@@ -523,9 +547,13 @@ static int run_rglru(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream
     if (p.single && n <= 1024) return n <= 256 ? launch_step<1>(p, s, st) : n <= 512 ? launch_step<2>(p, s, st) : launch_step<4>(p, s, st);
   }
   if (p.single) {
-    return p.taps == 4 ? launch_tile<T, 16, 4>(p, s, st) : launch_tile<T, 16, 0>(p, s, st);
+    return p.taps == 4 ? launch_tile<T, 16, 4, 64>(p, s, st) : launch_tile<T, 16, 0, 64>(p, s, st);
   }
-  if (int rc = p.taps == 4 ? launch_tile<T, 64, 4>(p, s, st) : launch_tile<T, 64, 0>(p, s, st)) return rc;
+  constexpr int CT = sizeof(T) == 2 ? 128 : 64;   // (in 32 bits twice the channels spill twice the registers)
+  const bool wide = CT > 64 && p.width / p.blocks > 64;
+  if (int rc = p.taps == 4 ? (wide ? launch_tile<T, 64, 4, CT>(p, s, st) : launch_tile<T, 64, 4, 64>(p, s, st))
+                           : (wide ? launch_tile<T, 64, 0, CT>(p, s, st) : launch_tile<T, 64, 0, 64>(p, s, st)))
+    return rc;
   if (!p.spans) return VMI_HY_OK;
   hipLaunchKernelGGL(rglru_carry_kernel, dim3((p.width + 63) / 64, s.B), dim3(64), 0, st, p, s);
   hipLaunchKernelGGL(rglru_finish_kernel<T>, dim3((p.width / 8 + 255) / 256, s.T), dim3(256), 0, st, p, s);
