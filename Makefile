@@ -36,7 +36,7 @@ DEPS   := $(wildcard $(CSRC)/*.hpp) $(wildcard $(CSRC)/*.inc) include/vmi_paged_
 LAYER_LIB := $(OUTDIR)/libvmi_gpt2_layer.so
 
 HYBRID_LIB := $(OUTDIR)/libvmi_hybrid.so
-HYBRID_UNITS := hybrid_linear hybrid_rows hybrid_tiles hybrid_rglru hybrid_latent hybrid_state hybrid_attention
+HYBRID_UNITS := hybrid_linear hybrid_rows hybrid_tiles hybrid_rglru hybrid_latent hybrid_latent_prompt hybrid_state hybrid_attention
 HYBRID_SRCS := $(HYBRID_UNITS:%=$(CSRC)/%.hip)
 
 all: $(LIB) $(LAYER_LIB) $(HYBRID_LIB) oracle

@@ -174,6 +174,9 @@ typedef struct {
   int32_t dtype, device;
 } vmi_hy_latent_prep_args;
 VMI_HY_API int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream);
+/* The same for vmi_hy_latent_prompt: the query parts are rotated where they are, in proj (q is not looked at), and the cache row goes to row t of
+ * rows [T, rank + rot] too.  rot_n a multiple of 16. */
+VMI_HY_API int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream);
 
 /* out [T, heads, rank] = softmax(scale * q . k) . latent over the visible cache rows (causal).  Query rows of an entry are
  * (token, head) pairs, head fastest, cut into tiles of 16 * row_tiles: tiles [n_tiles][2] = (entry, first row), entry -1: none.  splits > 1: the
@@ -190,6 +193,22 @@ typedef struct {
 } vmi_hy_latent_attention_args;
 VMI_HY_API int32_t vmi_hy_latent_row_tiles(int32_t row_dim, int32_t want, int32_t dtype);   /* 1, 2 or 4, at most `want` */
 VMI_HY_API int vmi_hy_latent_attention(const vmi_hy_latent_attention_args* a, const vmi_hy_step* s, void* stream);
+
+/* Latent attention of a step whose entries have no past (every ctx is 0), over the keys and values themselves: kv [T, ldkv] = per head [dim | vdim], the latents' product with the
+ * up-projections; proj and rows as vmi_hy_latent_prompt_prep leaves them; out [T, ldo], heads of vdim, times sigmoid of the head's column of gate. */
+typedef struct {
+  const void* proj;
+  const void* kv;
+  const void* rows;
+  const void* gate;
+  void* out;
+  int64_t ldp, ldkv, ldr, ldg, ldo;
+  int32_t heads, dim, rot, vdim, rank, max_len;   /* max_len: the longest entry's rows */
+  float scale;
+  int32_t dtype, device;
+} vmi_hy_latent_prompt_args;
+VMI_HY_API int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_t rank, int32_t rot_n, int32_t dtype);   /* whether it is built for these */
+VMI_HY_API int vmi_hy_latent_prompt(const vmi_hy_latent_prompt_args* a, const vmi_hy_step* s, void* stream);
 
 /* Linear attention with a matrix state per head, S [dim, vdim] float32 (csrc/hybrid_state.hip).  proj [T, ldp] begins with the
  * columns q [kv_heads dim] | k [kv_heads dim] | v [heads vdim]; head h uses q / k head h / (heads / kv_heads).

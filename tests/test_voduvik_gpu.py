@@ -852,6 +852,73 @@ def test_latent_prep_normalises_rotates_and_writes_the_cache(dtype):
     assert (flat[rest] == 9).all()
 
 
+@pytest.mark.parametrize("dim,rot,rank,rot_n,lens", [(128, 64, 512, 64, [64, 1, 65, 16]), (128, 32, 64, 16, [130, 63]), (64, 64, 128, 32, [15, 200, 17]), (64, 32, 192, 32, [321])])
+def test_latent_prompt_matches_plain_attention_and_leaves_the_caches_rows(dim, rot, rank, rot_n, lens):
+    """A step whose entries have no past: the cache rows, bytes, that latent_prep writes, and plain attention over them in float64.  Rounded to bfloat16 (2^-8 of it at most) are a
+    key, a value, a probability and the result; the scores of keys off by 2^-9 in the mean, of |score| up to about 4, move a probability by 1 per cent."""
+    from vllmini_amd import hybrid_ops as ops
+
+    H, page, T, D, bf = 3, 32, sum(lens), rank + rot, torch.bfloat16
+    g = torch.Generator().manual_seed(T + dim)
+    hd, scale = dim + rot, (dim + rot) ** -0.5
+    proj = torch.randn(T, H * hd + D + 32, generator=g).to(bf).to(dev())
+    up = (torch.randn(H, 2 * dim, rank, generator=g) * rank ** -0.5).to(bf).to(dev())
+    w = (1 + 0.3 * torch.randn(rank, generator=g)).to(dev())
+    freq = (500.0 ** (-2.0 * torch.arange(rot_n // 2, dtype=torch.float64) / rot_n)).to(dev())
+    per = [-(-n // page) for n in lens]
+    tables = np.zeros((len(lens), max(per)), dtype=np.int64)
+    for i, n in enumerate(per):
+        tables[i, :n] = sum(per) - sum(per[:i]) - np.arange(n)
+    step = layout(lens, [0] * len(lens), tables, page)
+    step.fresh = True
+    caches = [torch.full((sum(per) + 1, page, D), 9.0, dtype=bf, device=dev()) for _ in range(2)]
+    q = torch.zeros((T, H * D), dtype=bf, device=dev())
+    names = dict(norm_w=w, freq=freq, heads=H, dim=dim, rot=rot, rank=rank, rot_n=rot_n, rank_n=rank, eps=1e-5)
+    ops.latent_prep(proj, q, caches[0], step, **names)
+    out = ops.latent_prompt(proj.clone(), ops.MatrixTiles(up.reshape(-1, rank), bf), caches[1], step, vdim=dim, scale=scale, gate=proj[:, H * hd + D:], **names)
+    assert torch.equal(caches[0], caches[1])
+    rows = caches[0].view(-1, D).double().cpu()
+    at = 0
+    for i, n in enumerate(lens):
+        c = rows[[int(tables[i, t // page]) * page + t % page for t in range(n)]]
+        hide = torch.full((n, n), float("-inf"), dtype=torch.float64).triu(1)
+        for h in range(H):
+            own = proj[at: at + n, h * hd: h * hd + dim].double().cpu()
+            turned = q[at: at + n].view(n, H, D)[:, h, rank:].double().cpu()
+            kv = c[:, :rank] @ up[h].double().cpu().T
+            p = torch.softmax((own @ kv[:, :dim].T + turned @ c[:, rank:].T) * scale + hide, dim=-1)
+            gate = torch.sigmoid(proj[at: at + n, H * hd + D + h].double().cpu())[:, None]
+            close(out[at: at + n, h * dim: (h + 1) * dim], p @ kv[:, dim:] * gate, bf, tol16=1.2e-2)
+        at += n
+
+
+@pytest.mark.parametrize("lens", [[60], [90, 3, 40, 1]])
+def test_prompts_over_keys_and_over_latents_lead_to_the_same_decoder(lens, monkeypatch):
+    """Heads that latent_prompt is built for: prompts in one step, in one of its own and with the kernel over latents, and the tokens behind them, against the plain model."""
+    from vllmini_amd import hybrid_ops as ops
+    from vllmini_amd.hybrid_decoder import HybridDecoder
+    from vllmini_amd.voduvik import VoduvikConfig, build_model
+
+    c = cases.config([cases.attention(2, 64, 32, 64, 128, 0.1, mlp=cases.dense(64, 1.0)), cases.rglru(64, 1)], width=64)
+    w, took, prompt = cases.tensors(c), [], ops.latent_prompt
+    m = build_model(VoduvikConfig.from_json(c), w, torch.bfloat16, dev())
+    monkeypatch.setattr(ops, "latent_prompt", lambda *a, **k: took.append(1) or prompt(*a, **k))
+    toks = [cases.tokens(c, n + 2, i) for i, n in enumerate(lens)]
+    want = [plain.forward(c, w, t)[0] for t in toks]
+    for keys in (True, False):
+        if not keys:
+            monkeypatch.setattr(ops, "latent_prompt_pays", lambda step: False)
+        took.clear()
+        d = HybridDecoder(m, m.make_pool(640, 4, 16))
+        ids = list(range(len(lens)))
+        got = [d.prefill_batch(ids, [list(t[:n]) for t, n in zip(toks, lens)])]
+        assert bool(took) == keys
+        for k in range(2):
+            got.append(d.decode(ids, torch.tensor([int(t[n + k]) for t, n in zip(toks, lens)])))
+        for i, n in enumerate(lens):
+            logits_close(torch.stack([x[i] for x in got]), want[i][n - 1: n + 2], torch.bfloat16)
+
+
 # ---- the whole decoder -------------------------------------------------------------------------------------------------------------
 _PLAIN = {}
 

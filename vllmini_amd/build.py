@@ -92,7 +92,7 @@ HDRS_LAYER = [os.path.join(CSRC, "gpt2_prompt.hpp"), os.path.join(CSRC, "gpt2_ro
 LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 
 # the layers of decoders that mix recurrences, linear and softmax attention (include/vmi_hybrid.h), loaded by hybrid_ops.py only
-SRC_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hip") for t in ("linear", "rows", "tiles", "rglru", "latent", "state", "attention")]
+SRC_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hip") for t in ("linear", "rows", "tiles", "rglru", "latent", "latent_prompt", "state", "attention")]
 HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "linear", "softmax")] + [os.path.join(CSRC, f"{t}.hpp") for t in ("mfma_tiles", "step_inputs", "lane_ops")]
 HYBRID_LIB_PATH = os.path.join(OUT_DIR, "libvmi_hybrid.so")
 

@@ -240,9 +240,10 @@ __global__ __launch_bounds__(64 * W, EXACT && (RT == 1 || W == 8) ? 2 : 1) void 
   }
 }
 
-// RMS norm of the latent, rotation of the shared key and of the query parts; one workgroup per token
-template <typename T>
-__global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s) {
+// RMS norm of the latent, rotation of the shared key and of the query parts; one workgroup per token.  PROMPT: the query parts in place (a thread's pairs are nobody else's), the
+// cache row to row t of `rows` too
+template <typename T, bool PROMPT>
+__global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, void* const rows) {
   extern __shared__ float cs[];   // [rot_n / 2][2]
   __shared__ float part[4];
   need(p.proj), need(p.q), need(p.cache), need(p.norm_w), need(p.freq), need(p.ldp), need(p.heads), need(p.dim), need(p.rot), need(p.rank), need(p.rot_n), need(p.rank_n),
@@ -272,22 +273,25 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_pr
   __syncthreads();
   const float rms = 1.f / sqrtf((part[0] + part[1] + part[2] + part[3]) / (float)p.rank_n + p.eps);
   T* crow = slot >= 0 ? static_cast<T*>(p.cache) + slot * D : nullptr;
-  if (crow) {
+  T* prow = PROMPT ? static_cast<T*>(rows) + (int64_t)t * D : nullptr;
+  if (crow || PROMPT) {
     for (int k = tid * 8; k < p.rank; k += 2048) {
       f32x8 v = k < 2048 ? v0 : to_f32<T>(load8(lat + k));
       const f32x8 w = k < 2048 ? w0 : load8(p.norm_w + k);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = v[e] * rms * w[e];
-      *reinterpret_cast<V8<T>*>(crow + k) = from_f32<T>(v);
+      if (crow) *reinterpret_cast<V8<T>*>(crow + k) = from_f32<T>(v);
+      if constexpr (PROMPT) *reinterpret_cast<V8<T>*>(prow + k) = from_f32<T>(v);
     }
   }
-  if ((half & 7) == 0) {   // eight pairs at a time
+  if (PROMPT || (half & 7) == 0) {   // eight pairs at a time
     const int per = half >> 3;
     for (int u = tid; u < (p.heads + 1) * per; u += 256) {
       const int h = u / per, i = (u - h * per) * 8;
       const T* src = h < p.heads ? row + h * hd + p.dim : lat + p.rank;
-      T* dst = h < p.heads ? static_cast<T*>(p.q) + ((int64_t)t * p.heads + h) * D + p.rank : (crow ? crow + p.rank : nullptr);
-      if (!dst) continue;
+      T* dst = h < p.heads ? (PROMPT ? const_cast<T*>(src) : static_cast<T*>(p.q) + ((int64_t)t * p.heads + h) * D + p.rank) : (crow ? crow + p.rank : nullptr);
+      T* const second = PROMPT && h == p.heads ? prow + p.rank : nullptr;
+      if (!dst && !second) continue;
       const f32x8 a = to_f32<T>(load8(src + i)), b = to_f32<T>(load8(src + i + half));
       f32x8 x, y;
 #pragma unroll
@@ -296,13 +300,18 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_pr
         x[e] = a[e] * c - b[e] * sn;
         y[e] = b[e] * c + a[e] * sn;
       }
-      *reinterpret_cast<V8<T>*>(dst + i) = from_f32<T>(x);
-      *reinterpret_cast<V8<T>*>(dst + i + half) = from_f32<T>(y);
-      if (i == 0)
-        for (int k = p.rot_n; k < p.rot; k += 8) *reinterpret_cast<V8<T>*>(dst + k) = load8(src + k);   // passes unrotated
+      auto put = [&](T* to) {
+        *reinterpret_cast<V8<T>*>(to + i) = from_f32<T>(x);
+        *reinterpret_cast<V8<T>*>(to + i + half) = from_f32<T>(y);
+        if (i == 0 && to != src)
+          for (int k = p.rot_n; k < p.rot; k += 8) *reinterpret_cast<V8<T>*>(to + k) = load8(src + k);   // passes unrotated
+      };
+      if (dst) put(dst);
+      if (second) put(second);
     }
     return;
   }
+  if constexpr (PROMPT) return;
   // heads 0 .. heads - 1: the query's rotated part; "head" `heads`: the shared key
   T* qrow = static_cast<T*>(p.q) + (int64_t)t * p.heads * D;
   for (int u = tid; u < (p.heads + 1) * p.rot; u += 256) {
@@ -388,9 +397,22 @@ int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, v
   hipStream_t st = static_cast<hipStream_t>(stream);
   const size_t lds = (size_t)a->rot_n * 4;
   if (a->dtype == VMI_HY_BF16)
-    hipLaunchKernelGGL(latent_prep_kernel<b16>, dim3(s->T), dim3(256), lds, st, *a, *s);
+    hipLaunchKernelGGL((latent_prep_kernel<b16, false>), dim3(s->T), dim3(256), lds, st, *a, *s, nullptr);
   else
-    hipLaunchKernelGGL(latent_prep_kernel<float>, dim3(s->T), dim3(256), lds, st, *a, *s);
+    hipLaunchKernelGGL((latent_prep_kernel<float, false>), dim3(s->T), dim3(256), lds, st, *a, *s, nullptr);
+  return launched(who);
+}
+
+int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_latent_prompt_prep";
+  if (!a || !rows || !s || !a->proj || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 ||
+      a->heads <= 0 || a->rank_n <= 0 || a->rank_n > a->rank)
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->dim, a->rank, a->rot_n, a->dtype) || (a->ldp & 7) || (((uintptr_t)a->proj | (uintptr_t)rows | (uintptr_t)a->cache) & 15))
+    return fail(VMI_HY_E_SHAPE, who, "needs sizes that vmi_hy_latent_prompt is built for, rows aligned to 16 bytes");
+  DeviceScope dev(a->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  hipLaunchKernelGGL((latent_prep_kernel<b16, true>), dim3(s->T), dim3(256), (size_t)a->rot_n * 4, static_cast<hipStream_t>(stream), *a, *s, rows);
   return launched(who);
 }
 

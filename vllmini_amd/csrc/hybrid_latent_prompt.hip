@@ -1,0 +1,184 @@
+// Latent attention of whole prompts (include/vmi_hybrid.h: vmi_hy_latent_prompt): where no sequence of a step has a past, its keys and values are the step's own rows, and a head's
+// 128 + 64 columns of key and 128 of value, made for all tokens by one product, are a third of the 576 + 512 that the latent stands for.  csrc/hybrid_latent.hip walks
+// the latents, as it must where they come from pages.
+//
+// A workgroup takes 64 query positions of one head and walks the keys up to its last position in tiles of 64, each through LDS once (requested one tile ahead into registers, two
+// barriers a tile, so that three workgroups fit a compute unit).  A wave owns 16 queries for all of it: scores are formed transposed, S^T = K Q^T, so a lane keeps the scores of ONE
+// query and its probabilities, as they lie, are the B operand of O^T = V^T P^T: the sum over keys may take them in any order, so k-index 8 kc + e of a step of 32 stands for
+// key 4 kc + e (e < 4) and 16 + 4 kc + e - 4, and the V^T operand is read column-wise from LDS in that order.  Sums are a product with ones.  Scores, softmax and accumulators are
+// fp32; a probability is rounded once to the element type and what is summed is what multiplies V.  The longest walks come first, over all heads.
+//
+// Bound by the vector unit's share of the softmax and the chain of a tile (1.4 us).  Attention, us, the latents walked -> here, rank 512: 16 heads, 4 prompts of up to 1024 tokens
+// 117 -> 39, 1 of 500 28 + 12 (its splits added up) -> 16, 16 of up to 200 33 -> 15; 8 heads, 1 of 60 14.6 -> 5.8, 35 of up to 21 14.4 -> 5.7, 1 of 1024 45 + 12 -> 26; and one product of the latents
+// with both up-projections stands for two by heads, of the same work (16 heads, 2773 rows 27 + 19 us).
+#include "hybrid_softmax.hpp"
+
+namespace vmi_hybrid {
+
+constexpr int PQ = 64;   // queries of a workgroup, keys of a tile
+
+// DN + DR columns of a key, the last DR shared by the heads; VD of a value
+template <int DN, int DR, int VD>
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const vmi_hy_latent_prompt_args p, const vmi_hy_step s, const int places) {
+  constexpr int DK = DN + DR, LDK = DK + 8, LDV = VD + 8, NK = DK / 32, NT = VD / 16;
+  constexpr int UN = PQ * DN / 2048, UR = PQ * DR / 2048, UV = PQ * VD / 2048;   // units of eight columns a thread
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  b16* ks = reinterpret_cast<b16*>(smem);   // [64][LDK]
+  b16* vs = ks + PQ * LDK;                  // [64][LDV]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
+  const int H = p.heads, each = H * s.B, at = blockIdx.x / each, rest = blockIdx.x - at * each, e = rest / H, h = rest - e * H;
+  const int qs = s.q_start[e], len = s.q_len[e], q0 = (places - 1 - at) * PQ;
+  if (q0 >= len) return;
+  const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
+  const b16* kv = static_cast<const b16*>(p.kv) + (int64_t)qs * p.ldkv + h * (DN + VD);
+  const b16* shared = static_cast<const b16*>(p.rows) + (int64_t)qs * p.ldr + p.rank;
+  const b16* qrow = static_cast<const b16*>(p.proj) + (int64_t)qs * p.ldp + h * DK;
+
+  b16x8 kn[UN], kr[UR], vr[UV];
+  auto load = [&](int kt) {   // (keys past the end repeat the last one: no lane-wise condition around a load)
+    auto row = [&](int key) { return (int64_t)min(kt * PQ + key, len - 1); };
+#pragma unroll
+    for (int i = 0; i < UN; ++i) {
+      const int u = tid + 256 * i;
+      kn[i] = load8(kv + row(u / (DN / 8)) * p.ldkv + u % (DN / 8) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < UR; ++i) {
+      const int u = tid + 256 * i;
+      kr[i] = load8(shared + row(u / (DR / 8)) * p.ldr + u % (DR / 8) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < UV; ++i) {
+      const int u = tid + 256 * i;
+      vr[i] = load8(kv + row(u / (VD / 8)) * p.ldkv + DN + u % (VD / 8) * 8);
+    }
+  };
+  load(0);
+  const int w0 = q0 + wave * 16;   // this wave's first position
+  b16x8 qf[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) qf[k] = load8(qrow + (int64_t)min(w0 + r16, len - 1) * p.ldp + 32 * k + 8 * kc);
+  b16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (b16)1.f;
+  f32x4 o[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float mrun = -1e30f, lrun = 0.f;
+  const float sc2 = p.scale * 1.4426950408889634f;   // scores in units of log 2
+
+  for (int kt = 0; kt < nkt; ++kt) {
+    const int key0 = kt * PQ;
+    if (kt > 0) __syncthreads();   // the tile before has been read
+#pragma unroll
+    for (int i = 0; i < UN; ++i) {
+      const int u = tid + 256 * i;
+      *reinterpret_cast<b16x8*>(ks + u / (DN / 8) * LDK + u % (DN / 8) * 8) = kn[i];
+    }
+#pragma unroll
+    for (int i = 0; i < UR; ++i) {
+      const int u = tid + 256 * i;
+      *reinterpret_cast<b16x8*>(ks + u / (DR / 8) * LDK + DN + u % (DR / 8) * 8) = kr[i];
+    }
+#pragma unroll
+    for (int i = 0; i < UV; ++i) {
+      const int u = tid + 256 * i;
+      *reinterpret_cast<b16x8*>(vs + u / (VD / 8) * LDV + u % (VD / 8) * 8) = vr[i];
+    }
+    if (kt + 1 < nkt) load(kt + 1);
+    __syncthreads();
+    if (w0 >= len || key0 > w0 + 15) continue;   // (wave-uniform: none of its queries exists, or sees the tile)
+    f32x4 sc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < NK; ++k) mma(sc[j], load8(ks + (j * 16 + r16) * LDK + 32 * k + 8 * kc), qf[k]);
+    }
+    if (key0 + PQ - 1 > w0) {   // some query does not see every key
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (key0 + j * 16 + 4 * kc + r > w0 + r16) sc[j][r] = -INFINITY;
+    }
+    float mx = sc[0][0];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[j][r]);
+    auto more = [](float a, float b) { return fmaxf(a, b); };
+    mx = fmaxf(mrun, sc2 * vmi_lanes::across32(vmi_lanes::across16(mx, more), more));
+    const float alpha = exp2_hw(mrun - mx);
+    mrun = mx;
+    b16x8 pf[2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pf[j >> 1][(j & 1) * 4 + r] = (b16)exp2_hw(fmaf(sc[j][r], sc2, -mx));
+    f32x4 sum{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) mma(sum, ones, pf[k]);
+    lrun = fmaf(lrun, alpha, sum[0]);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) o[nt] *= alpha;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const b16* a = vs + (32 * k + 4 * kc + (r16 >> 2)) * LDV + nt * 16 + 4 * (r16 & 3);
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)a);
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(a + 16 * LDV));
+        mma(o[nt], __builtin_shufflevector(__builtin_bit_cast(b16x4, lo), __builtin_bit_cast(b16x4, hi), 0, 1, 2, 3, 4, 5, 6, 7), pf[k]);
+      }
+  }
+  const int q = w0 + r16;
+  if (q >= len) return;
+  const float inv = sigmoid((float)static_cast<const b16*>(p.gate)[(int64_t)(qs + q) * p.ldg + h]) / lrun;
+  b16* out = static_cast<b16*>(p.out) + (int64_t)(qs + q) * p.ldo + h * VD + 4 * kc;
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    b16x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[r] = (b16)(o[nt][r] * inv);
+    *reinterpret_cast<b16x4*>(out + nt * 16) = y;
+  }
+}
+
+template <int DN, int DR>
+static int launch_prompt(const vmi_hy_latent_prompt_args& p, const vmi_hy_step& s, hipStream_t st) {
+  auto* fn = latent_prompt_kernel<DN, DR, DN>;
+  constexpr size_t lds = (size_t)PQ * (DN + DR + 8 + DN + 8) * 2;
+  if (int rc = allow_lds(fn, lds, "vmi_hy_latent_prompt")) return rc;
+  const int places = (p.max_len + PQ - 1) / PQ;
+  const int64_t groups = (int64_t)places * p.heads * s.B;
+  if (groups >= (1 << 24)) return fail(VMI_HY_E_SHAPE, "vmi_hy_latent_prompt", "too many heads, entries and positions");   // (2^32 work items)
+  hipLaunchKernelGGL(fn, dim3((uint32_t)groups), dim3(256), lds, st, p, s, places);
+  return launched("vmi_hy_latent_prompt");
+}
+
+}  // namespace vmi_hybrid
+
+using namespace vmi_hybrid;
+
+extern "C" {
+
+int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_t rank, int32_t rot_n, int32_t dtype) {
+  return dtype == VMI_HY_BF16 && (dim == 64 || dim == 128) && vdim == dim && (rot == 32 || rot == 64) && rank > 0 && (rank & 63) == 0 && rot_n > 0 && (rot_n & 15) == 0 && rot_n <= rot;
+}
+
+int vmi_hy_latent_prompt(const vmi_hy_latent_prompt_args* a, const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_latent_prompt";
+  if (!a || !s || !a->proj || !a->kv || !a->rows || !a->gate || !a->out || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || a->heads <= 0 || a->max_len <= 0 || !(a->scale > 0.f))
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->vdim, a->rank, 16, a->dtype) || ((a->ldp | a->ldkv | a->ldr) & 7) || (a->ldo & 3) ||
+      (((uintptr_t)a->proj | (uintptr_t)a->kv | (uintptr_t)a->rows) & 15) || ((uintptr_t)a->out & 7))
+    return fail(VMI_HY_E_SHAPE, who, "built for bfloat16 heads of 64 or 128 beside 32 or 64 rotated columns, rows aligned to 16 bytes");
+  DeviceScope dev(a->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a->dim == 128) return a->rot == 64 ? launch_prompt<128, 64>(*a, *s, st) : launch_prompt<128, 32>(*a, *s, st);
+  return a->rot == 64 ? launch_prompt<64, 64>(*a, *s, st) : launch_prompt<64, 32>(*a, *s, st);
+}
+
+}  // extern "C"

@@ -260,7 +260,8 @@ class HybridDecoder:
         if "ids" in v:
             ids = v.pop("ids").view(torch.int64)
         spans = bool((starts // ops.ROW_TILE != (starts + counts - 1) // ops.ROW_TILE).any())
-        layout = ops.StepLayout(v, T, B, self.pool.block_size, bool((counts == 1).all()), spans, int(counts.max()), keys)
+        layout = ops.StepLayout(v, T, B, self.pool.block_size, bool((counts == 1).all()), spans, int(counts.max()), keys,
+                                fresh=not a["ctx"].any())
         return self._forward(ids, layout, plan, v["rows"] if len(rows) else None)
 
     # ---- what the scheduler calls -------------------------------------------------------------------------------------------

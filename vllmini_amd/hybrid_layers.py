@@ -212,6 +212,11 @@ class LatentAttention:
         self.w_in = MatrixTiles(rows, dtype, dense=True)
         self.w_uk = MatrixTiles(uk.view(heads, dim, rank).transpose(1, 2).contiguous(), dtype)     # [rank, dim]: q into the latent space
         self.w_uv = MatrixTiles(uv.view(heads, vdim, rank), dtype)
+        # ... and, for prompts that nothing stands in front of, the latents into every head's keys and values
+        self.w_kv = None
+        if self.scale > 0 and ops.latent_prompt_fits(self.dim, self.rot, self.vdim, self.rank, rot_dims, dtype):
+            kv = torch.cat([spread(uk.view(heads, dim, rank), 1, torch.arange(dim), self.dim), spread(uv.view(heads, vdim, rank), 1, torch.arange(vdim), self.vdim)], dim=1)
+            self.w_kv = MatrixTiles(spread(kv.reshape(-1, rank), 1, torch.arange(rank), self.rank), dtype)
         self.w_o = MatrixTiles(spread(spread(o, 1, strided_index(heads, vdim, self.vdim), heads * self.vdim), 0, torch.arange(width), E),
                                dtype, dense=True)
         self.norm_w = torch.zeros(self.rank, dtype=torch.float32, device=dev)
@@ -232,6 +237,11 @@ class LatentAttention:
     def run(self, res: Residual, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor]) -> None:
         H, D, plan, (cache,) = self.heads, self.row, plans[self.tiling()], held
         proj = res.branch_in(self.norm, self.w_in, step)
+        # (below DENSE_MIN_TOKENS the projections run in the few-row kernels, and there the latents stay: 1 prompt of 60, 8 heads, a whole step's kernels 501 -> 449 us, 6 of up to 20 558 -> 501)
+        if self.w_kv is not None and step.fresh and step.T >= DENSE_MIN_TOKENS and ops.latent_prompt_pays(step):
+            res.branch_out(ops.latent_prompt(proj, self.w_kv, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, vdim=self.vdim, rank=self.rank,
+                                             rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps, scale=self.scale, gate=proj[:, self.gate_at:]), self.w_o, step)
+            return
         q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
         ops.linear(proj, self.w_uk, x_gstride=self.dim + self.rot, y_gstride=D, out=q)
         ops.latent_prep(proj, q, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank,

@@ -55,6 +55,8 @@ RglruArgs = _struct("RglruArgs", [(_vp, "yx out conv_w conv_b gates gate_b decay
                                   (_i32, "width blocks taps single spans dtype device")])
 PrepArgs = _struct("PrepArgs", [(_vp, "proj q cache norm_w freq"), (_i64, "ldp"), (_i32, "heads dim rot rank rot_n rank_n"),
                                 (_f32, "eps"), (_i32, "dtype device")])
+LatentPromptArgs = _struct("LatentPromptArgs", [(_vp, "proj kv rows gate out"), (_i64, "ldp ldkv ldr ldg ldo"), (_i32, "heads dim rot vdim rank max_len"), (_f32, "scale"),
+                                                (_i32, "dtype device")])
 AttentionArgs = _struct("AttentionArgs", [(_vp, "q cache out tiles partial"), (_i32, "heads rank rot n_tiles row_tiles splits"),
                                           (_f32, "scale"), (_i32, "dtype device")])
 StateArgs = _struct("StateArgs", [(_vp, "proj beta z conv_w rate dt_bias decay log2_decay turns state tail o scratch out gate norm_w"),
@@ -97,6 +99,9 @@ SIGNATURES = {
     "vmi_hy_argmax": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_hy_rglru": (ctypes.c_int, [ctypes.POINTER(RglruArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
+    "vmi_hy_latent_prompt": (ctypes.c_int, [ctypes.POINTER(LatentPromptArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_row_tiles": (_i32, [_i32, _i32, _i32]),
     "vmi_hy_latent_attention": (ctypes.c_int, [ctypes.POINTER(AttentionArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hybrid_last_error": (ctypes.c_char_p, []),
@@ -439,9 +444,9 @@ ROW_TILE = 64      # rows of a tile of the recurrence's kernel
 
 class StepLayout:
     """The tokens of a step on the device: `fields` maps the names of vmi_hy_step to int32 tensors; `single`: every portion is one
-    token; `spans`: some portion crosses a row tile."""
+    token; `spans`: some portion crosses a row tile; `fresh`: no entry has a past, and every row is an entry's."""
 
-    def __init__(self, fields: dict, T: int, B: int, page_size: int, single: bool, spans: bool, max_len: int, max_keys: int):
+    def __init__(self, fields: dict, T: int, B: int, page_size: int, single: bool, spans: bool, max_len: int, max_keys: int, fresh: bool = False):
         for name in ("tok_seq", "tok_pos", "tok_slot"):
             _need(fields[name].dtype == torch.int32 and fields[name].numel() >= T and fields[name].is_contiguous(), f"StepLayout: {name}")
         for name in ("q_start", "q_len", "ctx", "state_slot", "flip"):
@@ -454,7 +459,7 @@ class StepLayout:
             _need(fields["chunk_start"].dtype == torch.int32 and fields["chunk_start"].numel() >= B, "StepLayout: chunk_start")
         self.n_chunks = 0 if chunks is None else int(chunks.shape[0])
         self.fields = fields      # (keeps the tensors alive)
-        self.T, self.B, self.single, self.spans = T, B, single, spans
+        self.T, self.B, self.single, self.spans, self.fresh = T, B, single, spans, fresh
         self.max_len, self.max_keys = max_len, max_keys      # longest portion, most keys any token sees
         self.args = StepArgs(**{k: fields[k].data_ptr() for k in ("tok_seq", "tok_pos", "tok_slot", "q_start", "q_len", "ctx",
                                                                   "state_slot", "flip", "table")},
@@ -518,6 +523,38 @@ def latent_prep(proj: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, step: 
                  ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank, rot_n=rot_n, rank_n=rank_n, eps=eps,
                  dtype=DTYPES[proj.dtype], device=device)
     _check(load().vmi_hy_latent_prep(ctypes.byref(a), step.ref, stream))
+
+
+def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int, rot_n: int, dtype: torch.dtype) -> bool:
+    return dtype == torch.bfloat16 and bool(load().vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, rot_n, DTYPES[dtype]))
+
+
+def latent_prompt_pays(step: StepLayout) -> bool:
+    """Whether a launch of as many places as the longest entry has, for every entry, is not mostly empty ones (each some ns; 48 prompts of up to 80 tokens 27.7 us over the latents, 9.5 so)."""
+    return -(-step.max_len // 64) * step.B <= 1024 + step.T
+
+
+def latent_prompt(proj: torch.Tensor, w_kv: MatrixTiles, cache: torch.Tensor, step: StepLayout, *, norm_w: torch.Tensor, freq: torch.Tensor, heads: int, dim: int, rot: int, vdim: int,
+                  rank: int, rot_n: int, rank_n: int, eps: float, scale: float, gate: torch.Tensor) -> torch.Tensor:
+    """Latent attention of a `fresh` step, gates included: proj (whose query parts are rotated in place) -> [T, heads * vdim], the cache's rows written.
+    w_kv: the up-projections, per head [dim | vdim] rows of rank."""
+    device, stream = _on(proj)
+    T, D = step.T, rank + rot
+    _need(step.fresh and proj.shape[0] == T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and cache.dtype == proj.dtype and cache.shape[-1] == D
+          and cache.is_contiguous() and norm_w.numel() == rank and norm_w.dtype == torch.float32 and freq.dtype == torch.float64 and freq.numel() == rot_n // 2
+          and w_kv.groups == 1 and (w_kv.N, w_kv.K) == (heads * (dim + vdim), rank) and gate.dtype == proj.dtype and gate.shape[0] == T and gate.shape[1] >= heads
+          and gate.stride(1) == 1, "hybrid_ops.latent_prompt: operand sizes")
+    rows = torch.empty((T, D), dtype=proj.dtype, device=proj.device)
+    a = PrepArgs(proj=proj.data_ptr(), cache=cache.data_ptr(), norm_w=norm_w.data_ptr(), freq=freq.data_ptr(), ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank,
+                 rot_n=rot_n, rank_n=rank_n, eps=eps, dtype=DTYPES[proj.dtype], device=device)
+    _check(load().vmi_hy_latent_prompt_prep(ctypes.byref(a), rows.data_ptr(), step.ref, stream))
+    kv = product_tiles(rows[:, :rank], w_kv)
+    out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
+    b = LatentPromptArgs(proj=proj.data_ptr(), kv=kv.data_ptr(), rows=rows.data_ptr(), gate=gate.data_ptr(), out=out.data_ptr(), ldp=proj.stride(0), ldkv=kv.stride(0), ldr=D,
+                         ldg=gate.stride(0), ldo=out.stride(0), heads=heads, dim=dim, rot=rot, vdim=vdim, rank=rank, max_len=step.max_len, scale=scale,
+                         dtype=DTYPES[proj.dtype], device=device)
+    _check(load().vmi_hy_latent_prompt(ctypes.byref(b), step.ref, stream))
+    return out
 
 
 def latent_row_tiles(row_dim: int, want: int, dtype: torch.dtype) -> int:
