@@ -7,7 +7,9 @@
 // operand is read column-wise from the same LDS rows.  Scores, softmax and sums are fp32; the sink opens the running maximum and sum.
 //   gqa_kernel       16 rows (steps of few tokens): wave w scores the 16 keys 16 w .., statistics meet in LDS, then wave w adds the
 //                    value columns w, w + 4, ... (tiles of 16)
-//   gqa_rows_kernel  64 rows (portions of prompts, bfloat16): every wave owns 16 of them, so only the key tile is shared
+//   gqa_rows_kernel  64 rows (portions of prompts, bfloat16): every wave owns 16 of them, so only the key tile is shared; scores are formed transposed, S^T = K Q^T, so a lane
+//                    keeps the scores of ONE row, and its probabilities, as they lie, are an operand of O^T = V^T P^T (k-index 8 kc + e of a step of 32 is key
+//                    4 kc + e, e < 4, or 16 + 4 kc + e - 4, and the values are read in that order); sums are a product with ones
 // Tiles too few for the chip have their keys dealt to `splits` workgroups.
 #include "hybrid_softmax.hpp"
 
@@ -259,51 +261,49 @@ __global__ __launch_bounds__(256) void gqa_kernel(const vmi_hy_attention_args p,
 }
 
 inline size_t gqa_rows_lds(int dim, int vdim, int rep, bool bias) {
-  return ((size_t)64 * (dim + vdim + 8) + (size_t)64 * 72) * 2 + (bias ? (size_t)rep * bias_window(64, 64, rep) * 4 : 0);
+  return (size_t)64 * (dim + vdim + 8) * 2 + (bias ? (size_t)rep * bias_window(64, 64, rep) * 4 : 0);
 }
 
 // NK k-steps (of 32) of a query row, NV value tiles (of 16 columns): at most that many, or (EXACT) just that many, so that no condition stands between a read of LDS and the product
 // behind it and they overlap: a branch a product, a bias and a mask each waited for its own read (heads of 128, 8 over 2 of them, 1 x 1500 rows 84 -> 53 us, 6 x up to 1500 91 -> 63;
 // 16 over 4, 32 x up to 200 33 -> 25; 16 over 4, 4 x up to 1000 rows, heads of 32 / 64 / 96 / 192 / 256 57 / 62 / 66 / 166 / 183 -> 32 / 34 / 51 / 92 / 126)
+// Rows against keys, with four rows a lane and the probabilities through LDS -> transposed: 8 over 2 of 128, 1 x 1500 rows 52 -> 44 us, 6 x up to 1500 65 -> 55, 12 x up to 300 17.2 -> 15.4, 1 x 60
+// 8.6 -> 7.4; heads of 32 / 64 / 96 / 192 / 256, 6 x up to 1500 46 / 49 / 57 / 93 / 129 -> 33 / 40 / 50 / 83 / 114.  Bound by the longest walk, 1.3 to 1.8 us a tile of one wave a SIMD; neither shifts
+// for the divisions by a page's size nor a branch around the masks (some 80 of 500 instructions) change that, and three workgroups a compute unit spill (55 -> 70).
 template <int NK, int NV, int U, bool EXACT>
 __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vmi_hy_attention_args p, const vmi_hy_step s) {
-  constexpr int R = 64, KT = 64, LDP = KT + 8;
+  constexpr int R = 64, KT = 64;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
   const int dim = EXACT ? 32 * NK : p.dim, vdim = EXACT ? 16 * NV : p.vdim, LDK = dim + vdim + 8;
   b16* ks = reinterpret_cast<b16*>(smem);          // [64][LDK]
-  b16* ps = ks + (size_t)KT * LDK + wave * 16 * LDP;   // [16][LDP], this wave's
-  float* bl = reinterpret_cast<float*>(ks + (size_t)KT * LDK + 64 * LDP);
+  float* bl = reinterpret_cast<float*>(ks + (size_t)KT * LDK);
   const QueryTile q(p, s, R, KT);
   if (q.nrows <= 0 || q.empty(p, s, tid)) return;
   KeyTile<b16, KT, U> keys;
   keys.open(p, s, q, R);
-  const int m0 = wave * 16;   // (rows past the last one repeat it and are not stored)
+  const int m0 = wave * 16, m = m0 + r16;   // (rows past the last one repeat it and are not stored)
+  const int row = q.r0 + min(m, q.nrows - 1), hh = row % q.rep;
+  const int64_t token = q.tok0 + row / q.rep;
   b16x8 qr[NK];
   {
-    const int row = q.r0 + min(m0 + r16, q.nrows - 1);
-    const b16* src = static_cast<const b16*>(p.q) + ((int64_t)(q.tok0 + row / q.rep) * p.heads + q.h0 + row % q.rep) * dim + 8 * kc;
+    const b16* src = static_cast<const b16*>(p.q) + (token * p.heads + q.h0 + hh) * dim + 8 * kc;
 #pragma unroll
     for (int k = 0; k < NK; ++k) qr[k] = load8(src + min(32 * k, dim - 32));
   }
+  b16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (b16)1.f;
   f32x4 o[NV];
-  float mrun[4], lrun[4];
-  int lim[4], low[4], boff[4];   // last and first key row m sees, its place in the bias window
 #pragma unroll
   for (int nt = 0; nt < NV; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = q.r0 + min(m0 + 4 * kc + r, q.nrows - 1), hh = row % q.rep;
-    mrun[r] = -1e30f;
-    lrun[r] = 0.f;
-    if (p.sink && q.split == 0) {   // counted once: by one lane of the first split
-      mrun[r] = p.sink[q.h0 + hh];
-      lrun[r] = r16 == 0 ? 1.f : 0.f;
-    }
-    lim[r] = q.ctx + row / q.rep;
-    low[r] = p.chunk > 0 ? lim[r] / p.chunk * p.chunk : 0;
-    boff[r] = hh * keys.BW + lim[r] - q.first + KT - 1 - r16;
+  float mrun = -1e30f, lrun = 0.f;
+  if (p.sink && q.split == 0) {   // (counted once: in the first split)
+    mrun = p.sink[q.h0 + hh];
+    lrun = 1.f;
   }
+  const int lim = q.ctx + row / q.rep, low = p.chunk > 0 ? lim / p.chunk * p.chunk : 0;   // last and first key this lane's row sees,
+  const int boff = hh * keys.BW + lim - q.first + KT - 1 - 4 * kc;                        // ... and its place in the bias window
   const float sc2 = p.scale * 1.4426950408889634f;   // scores in units of log 2
   // what the wave's rows see, all of them and any of them: tiles outside need no look at single keys
   const int lim0 = q.ctx + (q.r0 + min(m0, q.nrows - 1)) / q.rep, lim1 = q.ctx + (q.r0 + min(m0 + 15, q.nrows - 1)) / q.rep;
@@ -315,16 +315,16 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
     __syncthreads();
     const int key0 = kt * KT;
     if (key0 <= lim1 && key0 + KT > low0) {
-      float bias[4][4];
+      float bias[4][4];   // of keys 16 j + 4 kc + r
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bias[r][j] = 0.f;
+        for (int r = 0; r < 4; ++r) bias[j][r] = 0.f;
       if (keys.bn) {   // (all of them at once, in front of the products: one condition a tile)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) bias[r][j] = bl[boff[r] - 16 * j];
+          for (int r = 0; r < 4; ++r) bias[j][r] = bl[boff - 16 * j - r];
       }
       f32x4 sc[4];
 #pragma unroll
@@ -333,75 +333,85 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
         const b16* krow = ks + (j * 16 + r16) * LDK + 8 * kc;
 #pragma unroll
         for (int k = 0; k < NK; ++k)
-          if (EXACT || NK <= 4 || k < nk) mma(sc[j], qr[k], EXACT || k < nk ? load8(krow + 32 * k) : zero8<b16>());
+          if (EXACT || k < nk) mma(sc[j], load8(krow + 32 * k), qr[k]);
       }
-      const bool whole = key0 + KT - 1 <= lim0 && key0 >= low1;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j][r] = fmaf(sc[j][r], sc2, bias[r][j]);
-      if (!whole) {
+        for (int r = 0; r < 4; ++r) sc[j][r] = fmaf(sc[j][r], sc2, bias[j][r]);
+      if (!(key0 + KT - 1 <= lim0 && key0 >= low1)) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const int key = key0 + j * 16 + r16;
-            sc[j][r] = key <= lim[r] && key >= low[r] ? sc[j][r] : -INFINITY;
+          for (int r = 0; r < 4; ++r) {
+            const int key = key0 + j * 16 + 4 * kc + r;
+            sc[j][r] = key <= lim && key >= low ? sc[j][r] : -INFINITY;
           }
       }
-      f32x4 mx;
+      float mx = sc[0][0];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) mx[r] = max16(fmaxf(fmaxf(sc[0][r], sc[1][r]), fmaxf(sc[2][r], sc[3][r])));
-      float alpha[4];
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float mn = fmaxf(mrun[r], mx[r]);
-        alpha[r] = exp2_hw(mrun[r] - mn);
-        mrun[r] = mn;
-        lrun[r] *= alpha[r];
+        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[j][r]);
+      auto more = [](float a, float b) { return fmaxf(a, b); };
+      mx = fmaxf(mrun, vmi_lanes::across32(vmi_lanes::across16(mx, more), more));
+      const float alpha = exp2_hw(mrun - mx);
+      mrun = mx;
+      b16x8 pf[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const b16 pr = (b16)exp2_hw(sc[j][r] - mn);
-          lrun[r] += (float)pr;   // (what is summed is what multiplies the values)
-          ps[(4 * kc + r) * LDP + j * 16 + r16] = pr;
-        }
-      }
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pf[j >> 1][(j & 1) * 4 + r] = (b16)exp2_hw(sc[j][r] - mx);
+      f32x4 sum{0.f, 0.f, 0.f, 0.f};   // (what is summed is what multiplies the values)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) mma(sum, ones, pf[k]);
+      lrun = fmaf(lrun, alpha, sum[0]);
+#pragma unroll
+      for (int nt = 0; nt < NV; ++nt) o[nt] *= alpha;
 #pragma unroll
       for (int nt = 0; nt < NV; ++nt)
+        if (EXACT || nt < n16) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[nt][r] *= alpha[r];
-#pragma unroll
-      for (int k = 0; k < KT; k += 32) {
-        const b16x8 pf = load8(ps + r16 * LDP + k + 8 * kc);
-#pragma unroll
-        for (int nt = 0; nt < NV; ++nt)
-          if (EXACT || nt < n16) mma(o[nt], pf, column8(ks, LDK, k + 8 * kc, dim + nt * 16, r16));
-      }
+          for (int k = 0; k < 2; ++k) {
+            const b16* a = ks + (32 * k + 4 * kc + (r16 >> 2)) * LDK + dim + nt * 16 + 4 * (r16 & 3);
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)a);
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(a + 16 * LDK));
+            mma(o[nt], __builtin_shufflevector(__builtin_bit_cast(b16x4, lo), __builtin_bit_cast(b16x4, hi), 0, 1, 2, 3, 4, 5, 6, 7), pf[k]);
+          }
+        }
     }
     __syncthreads();
   }
+  if (m >= q.nrows) return;
+  if (p.splits == 1) {
+    const int h = q.h0 + hh;
+    const float gate = p.gate ? sigmoid((float)static_cast<const b16*>(p.gate)[token * p.ldg + h]) : 1.f, inv = gate / lrun;
+    b16* out = static_cast<b16*>(p.out) + token * p.ldo + (int64_t)h * vdim + 4 * kc;
+    const bool wide = ((p.ldo & 3) | ((uintptr_t)p.out & 7)) == 0;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float l = sum16(lrun[r]);
-    const int m = m0 + 4 * kc + r;
-    if (m >= q.nrows) continue;
-    if (p.splits == 1) {
-      const int64_t t = q.tok0 + (q.r0 + m) / q.rep;
-      const int h = q.h0 + (q.r0 + m) % q.rep;
-      const float gate = p.gate ? sigmoid((float)static_cast<const b16*>(p.gate)[t * p.ldg + h]) : 1.f, inv = gate / l;
-      b16* out = static_cast<b16*>(p.out) + t * p.ldo + (int64_t)h * vdim + r16;
+    for (int nt = 0; nt < NV; ++nt)
+      if (EXACT || nt < n16) {
+        b16x4 y;
 #pragma unroll
-      for (int nt = 0; nt < NV; ++nt)
-        if (EXACT || nt < n16) out[nt * 16] = (b16)(o[nt][r] * inv);
-    } else {
-      float* out = q.part(p, s, m);
+        for (int r = 0; r < 4; ++r) y[r] = (b16)(o[nt][r] * inv);
+        if (wide) {   // (scalar)
+          *reinterpret_cast<b16x4*>(out + nt * 16) = y;
+        } else {
 #pragma unroll
-      for (int nt = 0; nt < NV; ++nt)
-        if (EXACT || nt < n16) out[nt * 16 + r16] = o[nt][r];
-      if (r16 == 0) {
-        out[vdim] = mrun[r];
-        out[vdim + 1] = l;
+          for (int r = 0; r < 4; ++r) out[nt * 16 + r] = y[r];
+        }
       }
+  } else {
+    float* out = q.part(p, s, m);
+#pragma unroll
+    for (int nt = 0; nt < NV; ++nt)
+      if (EXACT || nt < n16) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out[nt * 16 + 4 * kc + r] = o[nt][r];
+      }
+    if (kc == 0) {
+      out[vdim] = mrun;
+      out[vdim + 1] = lrun;
     }
   }
 }
