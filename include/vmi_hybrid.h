@@ -174,6 +174,8 @@ typedef struct {
   int32_t dtype, device;
 } vmi_hy_latent_prep_args;
 VMI_HY_API int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream);
+/* vmi_hy_linear (l: the queries by heads into q) and vmi_hy_latent_prep, neither of which reads what the other writes; few rows in one launch. */
+VMI_HY_API int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream);
 /* The same for vmi_hy_latent_prompt: the query parts are rotated where they are, in proj (q is not looked at), and the cache row goes to row t of
  * rows [T, rank + rot] too.  rot_n a multiple of 16. */
 VMI_HY_API int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream);

@@ -852,6 +852,31 @@ def test_latent_prep_normalises_rotates_and_writes_the_cache(dtype):
     assert (flat[rest] == 9).all()
 
 
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("T", [1, 16, 17, 50, 64, 65])
+@pytest.mark.parametrize("heads,dim,rank", [(3, 32, 64), (16, 128, 512), (2, 160, 96), (1, 512, 32), (2, 544, 32)])
+def test_latent_in_is_the_product_and_the_preparation(dtype, T, heads, dim, rank):
+    """Every bit of the two launches it stands for, a padding row and rows past the last one left alone; sizes on both sides of what goes into one launch."""
+    from vllmini_amd import hybrid_ops as ops
+
+    rot, rot_n, page = 32, 20, 16
+    g = torch.Generator().manual_seed(T + dim)
+    step = layout([1] * T, list(range(5, 5 + T)), np.arange(T * 6).reshape(T, 6), page)
+    f = dict(step.fields)
+    f["tok_seq"] = torch.cat([f["tok_seq"][: T - 1], i32([-1])]) if T > 1 else f["tok_seq"]
+    step = ops.StepLayout(f, T, T, page, True, False, 1, T + 5)
+    proj = torch.randn(T, heads * (dim + rot) + rank + rot + 32, generator=g).to(dtype).to(dev())
+    w = ops.MatrixTiles((torch.randn(heads, rank, dim, generator=g) * dim ** -0.5).to(dev()), dtype)
+    names = dict(norm_w=torch.rand(rank, generator=g).to(dev()), freq=(500.0 ** (-2.0 * torch.arange(rot_n // 2, dtype=torch.float64) / rot_n)).to(dev()), heads=heads, dim=dim, rot=rot,
+                 rank=rank, rot_n=rot_n, rank_n=rank, eps=1e-5)
+    qs = [torch.full((T + 2, heads * (rank + rot)), 3.0, dtype=dtype, device=dev()) for _ in range(2)]
+    caches = [torch.full((T * 6, page, rank + rot), 9.0, dtype=dtype, device=dev()) for _ in range(2)]
+    ops.linear(proj, w, x_gstride=dim + rot, y_gstride=rank + rot, out=qs[0][:T])
+    ops.latent_prep(proj, qs[0][:T], caches[0], step, **names)
+    ops.latent_in(proj, w, qs[1][:T], caches[1], step, **names)
+    assert torch.equal(*qs) and torch.equal(*caches)
+
+
 @pytest.mark.parametrize("dim,rot,rank,rot_n,lens", [(128, 64, 512, 64, [64, 1, 65, 16]), (128, 32, 64, 16, [130, 63]), (64, 64, 128, 32, [15, 200, 17]), (64, 32, 192, 32, [321])])
 def test_latent_prompt_matches_plain_attention_and_leaves_the_caches_rows(dim, rot, rank, rot_n, lens):
     """A step whose entries have no past: the cache rows, bytes, that latent_prep writes, and plain attention over them in float64.  Rounded to bfloat16 (2^-8 of it at most) are a

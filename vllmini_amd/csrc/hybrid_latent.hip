@@ -7,6 +7,7 @@
 // statistics meet in LDS; then wave w adds the value columns w, w + 4, ... (tiles of 16) of all rows, the value operand read
 // column-wise from the same LDS rows (ds_read_b64_tr_b16).  Scores, softmax and accumulators are fp32.  A sequence whose rows do
 // not fill the chip has its keys dealt to `splits` workgroups, whose unnormalised parts a second kernel adds up.
+#include "hybrid_latent_prep.hpp"
 #include "hybrid_softmax.hpp"
 
 namespace vmi_hybrid {
@@ -240,94 +241,10 @@ __global__ __launch_bounds__(64 * W, EXACT && (RT == 1 || W == 8) ? 2 : 1) void 
   }
 }
 
-// RMS norm of the latent, rotation of the shared key and of the query parts; one workgroup per token.  PROMPT: the query parts in place (a thread's pairs are nobody else's), the
-// cache row to row t of `rows` too
 template <typename T, bool PROMPT>
 __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, void* const rows) {
-  extern __shared__ float cs[];   // [rot_n / 2][2]
-  __shared__ float part[4];
-  need(p.proj), need(p.q), need(p.cache), need(p.norm_w), need(p.freq), need(p.ldp), need(p.heads), need(p.dim), need(p.rot), need(p.rank), need(p.rot_n), need(p.rank_n),
-      need(p.eps), need(s.tok_seq), need(s.tok_pos), need(s.tok_slot);
-  const int t = blockIdx.x, tid = threadIdx.x, half = p.rot_n >> 1, hd = p.dim + p.rot, D = p.rank + p.rot;
-  const int seq = s.tok_seq[t];
-  const int64_t slot = s.tok_slot[t];
-  const double pos = (double)s.tok_pos[t];
-  const T* row = static_cast<const T*>(p.proj) + (int64_t)t * p.ldp;
-  const T* lat = row + p.heads * hd;
-  f32x8 v0 = to_f32<T>(load8(lat + min(tid * 8, p.rank - 8))), w0 = load8(p.norm_w + min(tid * 8, p.rank - 8));
-  if (seq < 0) return;
-  for (int i = tid; i < half; i += 256) {   // the angle reduced in fp64: exact to fp32 at any position
-    const double a = pos * p.freq[i];
-    const float r = (float)(a - 6.283185307179586476925 * rint(a * 0.15915494309189533577));
-    cs[2 * i] = cosf(r);
-    cs[2 * i + 1] = sinf(r);
-  }
-  float ss = 0.f;
-  for (int k = tid * 8; k < p.rank; k += 2048) {
-    const f32x8 v = k < 2048 ? v0 : to_f32<T>(load8(lat + k));
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
-  }
-  ss = wave_sum(ss);
-  if ((tid & 63) == 0) part[tid >> 6] = ss;
-  __syncthreads();
-  const float rms = 1.f / sqrtf((part[0] + part[1] + part[2] + part[3]) / (float)p.rank_n + p.eps);
-  T* crow = slot >= 0 ? static_cast<T*>(p.cache) + slot * D : nullptr;
-  T* prow = PROMPT ? static_cast<T*>(rows) + (int64_t)t * D : nullptr;
-  if (crow || PROMPT) {
-    for (int k = tid * 8; k < p.rank; k += 2048) {
-      f32x8 v = k < 2048 ? v0 : to_f32<T>(load8(lat + k));
-      const f32x8 w = k < 2048 ? w0 : load8(p.norm_w + k);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = v[e] * rms * w[e];
-      if (crow) *reinterpret_cast<V8<T>*>(crow + k) = from_f32<T>(v);
-      if constexpr (PROMPT) *reinterpret_cast<V8<T>*>(prow + k) = from_f32<T>(v);
-    }
-  }
-  if (PROMPT || (half & 7) == 0) {   // eight pairs at a time
-    const int per = half >> 3;
-    for (int u = tid; u < (p.heads + 1) * per; u += 256) {
-      const int h = u / per, i = (u - h * per) * 8;
-      const T* src = h < p.heads ? row + h * hd + p.dim : lat + p.rank;
-      T* dst = h < p.heads ? (PROMPT ? const_cast<T*>(src) : static_cast<T*>(p.q) + ((int64_t)t * p.heads + h) * D + p.rank) : (crow ? crow + p.rank : nullptr);
-      T* const second = PROMPT && h == p.heads ? prow + p.rank : nullptr;
-      if (!dst && !second) continue;
-      const f32x8 a = to_f32<T>(load8(src + i)), b = to_f32<T>(load8(src + i + half));
-      f32x8 x, y;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float c = cs[2 * (i + e)], sn = cs[2 * (i + e) + 1];
-        x[e] = a[e] * c - b[e] * sn;
-        y[e] = b[e] * c + a[e] * sn;
-      }
-      auto put = [&](T* to) {
-        *reinterpret_cast<V8<T>*>(to + i) = from_f32<T>(x);
-        *reinterpret_cast<V8<T>*>(to + i + half) = from_f32<T>(y);
-        if (i == 0 && to != src)
-          for (int k = p.rot_n; k < p.rot; k += 8) *reinterpret_cast<V8<T>*>(to + k) = load8(src + k);   // passes unrotated
-      };
-      if (dst) put(dst);
-      if (second) put(second);
-    }
-    return;
-  }
-  if constexpr (PROMPT) return;
-  // heads 0 .. heads - 1: the query's rotated part; "head" `heads`: the shared key
-  T* qrow = static_cast<T*>(p.q) + (int64_t)t * p.heads * D;
-  for (int u = tid; u < (p.heads + 1) * p.rot; u += 256) {
-    const int h = u / p.rot, i = u - h * p.rot;
-    const T* src = h < p.heads ? row + h * hd + p.dim : lat + p.rank;
-    T* dst = h < p.heads ? qrow + (int64_t)h * D + p.rank : (crow ? crow + p.rank : nullptr);
-    if (!dst) continue;
-    if (i >= p.rot_n) {
-      dst[i] = src[i];   // passes unrotated (padding: zeros)
-    } else if (i < half) {
-      dst[i] = (T)((float)src[i] * cs[2 * i] - (float)src[i + half] * cs[2 * i + 1]);
-    } else {
-      const int j = i - half;
-      dst[i] = (T)((float)src[i] * cs[2 * j] + (float)src[j] * cs[2 * j + 1]);
-    }
-  }
+  extern __shared__ float cs[];   // 4, [rot_n / 2][2]
+  latent_prep_token<T, PROMPT>(p, s, rows, blockIdx.x, cs);
 }
 
 template <typename T, int KT, int RT, int NT, int U, bool EXACT = false>
@@ -378,6 +295,16 @@ static int run_attention(const vmi_hy_latent_attention_args& p, const vmi_hy_ste
   return attention_lds<T, 64, 1>(D) <= LDS_PER_CU ? attention_width<T, 64, 1>(p, s, st) : attention_width<T, 32, 1>(p, s, st);
 }
 
+int check_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, const char* who) {
+  if (!a || !s || !a->proj || !a->q || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 ||
+      a->heads <= 0 || a->dim <= 0 || a->rot <= 0 || a->rank <= 0 || a->rot_n <= 0 || a->rot_n > a->rot || (a->rot_n & 1) ||
+      a->rank_n <= 0 || a->rank_n > a->rank)
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if ((a->dim & 31) || (a->rot & 31) || (a->rank & 31) || (a->ldp & 7) || a->rot_n > 8192)
+    return fail(VMI_HY_E_SHAPE, who, "needs sizes that are multiples of 32");
+  return VMI_HY_OK;
+}
+
 }  // namespace vmi_hybrid
 
 using namespace vmi_hybrid;
@@ -386,16 +313,11 @@ extern "C" {
 
 int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_latent_prep";
-  if (!a || !s || !a->proj || !a->q || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 ||
-      a->heads <= 0 || a->dim <= 0 || a->rot <= 0 || a->rank <= 0 || a->rot_n <= 0 || a->rot_n > a->rot || (a->rot_n & 1) ||
-      a->rank_n <= 0 || a->rank_n > a->rank)
-    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
-  if ((a->dim & 31) || (a->rot & 31) || (a->rank & 31) || (a->ldp & 7) || a->rot_n > 8192)
-    return fail(VMI_HY_E_SHAPE, who, "needs sizes that are multiples of 32");
+  if (int rc = check_latent_prep(a, s, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const size_t lds = (size_t)a->rot_n * 4;
+  const size_t lds = latent_prep_lds(a->rot_n);
   if (a->dtype == VMI_HY_BF16)
     hipLaunchKernelGGL((latent_prep_kernel<b16, false>), dim3(s->T), dim3(256), lds, st, *a, *s, nullptr);
   else
@@ -412,7 +334,7 @@ int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, cons
     return fail(VMI_HY_E_SHAPE, who, "needs sizes that vmi_hy_latent_prompt is built for, rows aligned to 16 bytes");
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  hipLaunchKernelGGL((latent_prep_kernel<b16, true>), dim3(s->T), dim3(256), (size_t)a->rot_n * 4, static_cast<hipStream_t>(stream), *a, *s, rows);
+  hipLaunchKernelGGL((latent_prep_kernel<b16, true>), dim3(s->T), dim3(256), latent_prep_lds(a->rot_n), static_cast<hipStream_t>(stream), *a, *s, rows);
   return launched(who);
 }
 

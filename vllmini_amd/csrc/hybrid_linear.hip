@@ -747,6 +747,21 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float* __restrict__ 
   }
 }
 
+int check_linear(const vmi_hy_linear_args* a, const char* who) {
+  if (!a || !a->x || !a->w || !a->y || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->groups <= 0 || a->dtype < 0 || a->dtype > 1 ||
+      (a->x_kind == VMI_HY_X_NORM && (!a->norm_w || a->norm_n <= 0 || a->norm_n > a->K)) || (a->x_kind == VMI_HY_X_CONCAT && !a->x2) ||
+      (a->epilogue == VMI_HY_E_GATED && !a->gate) || (a->epilogue == VMI_HY_E_STORE_GLU && !a->y2))
+    return fail(VMI_HY_E_ARG, who, "null pointer, non-positive size or unknown element type");
+  if ((a->K & 31) || (a->N & 15) || (a->x_kind == VMI_HY_X_CONCAT && (a->K & 63)) || (a->ldx & 7) || (a->x_gstride & 7) ||
+      (a->epilogue != VMI_HY_E_FLOAT && ((a->ldy & 3) || (a->y_gstride & 3))) || ((uintptr_t)a->x & 15) || ((uintptr_t)a->w & 15) ||
+      ((uintptr_t)a->y & 15) || ((uintptr_t)a->normed & 15) ||
+      (a->epilogue == VMI_HY_E_FLOAT && (a->n_out <= 0 || a->n_out > a->N || a->groups != 1)) ||
+      (a->epilogue == VMI_HY_E_STORE_GLU && (a->n_split < 0 || a->n_split > a->N || (a->n_split & 15) || (a->ldy2 & 1) ||
+                                             ((uintptr_t)a->y2 & 7) || a->groups != 1)))
+    return fail(VMI_HY_E_SHAPE, who, "needs K % 32 == 0, N % 16 == 0 and 16-byte aligned rows");
+  return VMI_HY_OK;
+}
+
 }  // namespace vmi_hybrid
 
 using namespace vmi_hybrid;
@@ -779,17 +794,7 @@ int32_t vmi_hy_linear_holds(int32_t M, int32_t N, int32_t K, int32_t stored, int
 
 int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   static const char* who = "vmi_hy_linear";
-  if (!a || !a->x || !a->w || !a->y || a->M <= 0 || a->N <= 0 || a->K <= 0 || a->groups <= 0 || a->dtype < 0 || a->dtype > 1 ||
-      (a->x_kind == VMI_HY_X_NORM && (!a->norm_w || a->norm_n <= 0 || a->norm_n > a->K)) || (a->x_kind == VMI_HY_X_CONCAT && !a->x2) ||
-      (a->epilogue == VMI_HY_E_GATED && !a->gate) || (a->epilogue == VMI_HY_E_STORE_GLU && !a->y2))
-    return fail(VMI_HY_E_ARG, who, "null pointer, non-positive size or unknown element type");
-  if ((a->K & 31) || (a->N & 15) || (a->x_kind == VMI_HY_X_CONCAT && (a->K & 63)) || (a->ldx & 7) || (a->x_gstride & 7) ||
-      (a->epilogue != VMI_HY_E_FLOAT && ((a->ldy & 3) || (a->y_gstride & 3))) || ((uintptr_t)a->x & 15) || ((uintptr_t)a->w & 15) ||
-      ((uintptr_t)a->y & 15) || ((uintptr_t)a->normed & 15) ||
-      (a->epilogue == VMI_HY_E_FLOAT && (a->n_out <= 0 || a->n_out > a->N || a->groups != 1)) ||
-      (a->epilogue == VMI_HY_E_STORE_GLU && (a->n_split < 0 || a->n_split > a->N || (a->n_split & 15) || (a->ldy2 & 1) ||
-                                             ((uintptr_t)a->y2 & 7) || a->groups != 1)))
-    return fail(VMI_HY_E_SHAPE, who, "needs K % 32 == 0, N % 16 == 0 and 16-byte aligned rows");
+  if (int rc = check_linear(a, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);

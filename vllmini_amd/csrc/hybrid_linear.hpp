@@ -59,6 +59,7 @@ int norm_slabs(int M, int N, int K);   // behind a norm, one group: 0 where it i
 int launch_norm_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool held_rows_pay(int M, int N, int K, bool stored);   // of the element type behind a norm of their own, one group; stored: as they are
 int launch_held_rows(const vmi_hy_linear_args& p, hipStream_t st);
+int check_linear(const vmi_hy_linear_args* a, const char* who);   // the code of what does not fit
 bool plain_rows_fit(int M, int N, int K, int groups);   // of the element type
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st);
 bool concat_rows_fit(int M, int N, int K);   // float32 rows side by side, FLOAT, one group

@@ -4,6 +4,7 @@
 // cores' layout (16 rows x 64 bytes) in LDS; all arguments are asked for at once (`need`: left to itself the compiler asks branch by branch, a trip to
 // memory each); what the epilogue adds to is asked for in front of everything.  The waves' partial tiles meet in LDS; one wave a tile adds them in
 // the order of K and stores.
+#include "hybrid_latent_prep.hpp"
 #include "hybrid_linear.hpp"
 
 namespace vmi_hybrid {
@@ -29,7 +30,7 @@ constexpr int plain_stride(int J, int MT) { return MT * 16 * (64 * J + 16); }   
 // N 1024 12.0 / 16.0 -> 11.0 / 14.7, N 4096 21.9 / 23.8 -> 20.3 / 22.6 (101 MB, 5.0 TB/s).
 // XK = VMI_HY_X_CONCAT: rows of x and x2 side by side, float32, rounded on their way into LDS (half of K is whole units, and of whole chunks a wave's part lies in one).
 template <int RW, int J, int MT, int NB, int EPI, int NCH = 0, int XI = J, int XK = VMI_HY_X_ROWS>
-__global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_hy_linear_args p) {
+__device__ __forceinline__ void plain_rows_slab(const vmi_hy_linear_args& p, const int slab, const int m0, const int grp, unsigned char* const smem) {
   constexpr bool CAT = XK == VMI_HY_X_CONCAT;
   using XT = std::conditional_t<CAT, float, b16>;
   auto rounded = [](const V8<XT>& v) {
@@ -37,11 +38,9 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
     else return v;
   };
   constexpr int LDB = 64 * J + 16, STRIDE = plain_stride(J, MT);
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [RW][STRIDE]
   need_args<EPI>(p), need(p.x_gstride), need(p.y_gstride);
   if constexpr (CAT) need(p.x2);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int slab = blockIdx.x, m0 = blockIdx.y * 16 * MT, grp = blockIdx.z;
   if (slab * 16 >= p.N) return;
   const int nks = p.K >> 5, per = (nks + RW - 1) / RW, k0 = wave * per, nk = min(per, nks - k0);   // (nk <= 0: no part of K is left for it)
   const int nch = (per + J - 1) / J, rows = p.M - m0;
@@ -153,6 +152,26 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
     *reinterpret_cast<f32x4*>(static_cast<float*>(p.y) + (int64_t)m * p.ldy + (int64_t)grp * p.y_gstride + n) = before + sum;
   else
     epilogue<b16, EPI>(p, sum, m, n, slab * 16, grp);
+}
+template <int RW, int J, int MT, int NB, int EPI, int NCH = 0, int XI = J, int XK = VMI_HY_X_ROWS>
+__global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_hy_linear_args p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // [RW][plain_stride]
+  plain_rows_slab<RW, J, MT, NB, EPI, NCH, XI, XK>(p, blockIdx.x, blockIdx.y * 16 * MT, blockIdx.z, smem);
+}
+
+// The queries' way into the latent space, by heads, and what a token's latent attention needs besides: two launches of a chain that do not read each other's results, in one.  The
+// first T workgroups take a token each, the others a slab of 16 columns of 16 MT rows of a head.  8 heads of 128 into 512, 12 rows, us: 4.2 + 4.9 -> 4.8 (each little more than its launch);
+// width 1024, 12 sequences, 24 tokens 7311 -> 7203, width 4096, one, 16 tokens 14 019 -> 13 919.
+template <int J, int MT>
+__global__ __launch_bounds__(256, 1) void latent_in_kernel(const vmi_hy_linear_args p, const vmi_hy_latent_prep_args a, const vmi_hy_step s, const int slabs, const int blocks) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int at = (int)blockIdx.x - s.T;
+  if (at < 0) {
+    latent_prep_token<b16, false>(a, s, nullptr, blockIdx.x, reinterpret_cast<float*>(smem));
+  } else {
+    const int rest = at / slabs, grp = rest / blocks;
+    plain_rows_slab<4, J, MT, 1, VMI_HY_E_STORE>(p, at - rest * slabs, (rest - grp * blocks) * 16 * MT, grp, smem);
+  }
 }
 
 // Rows of the element type over many columns, 16 MT of them: eight waves hold an eighth of K of all rows each, in registers and in the matrix cores' layout,
@@ -645,6 +664,24 @@ int launch_concat_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   return with_chunks(p.K, whole);
 }
 
+// Whether the product of vmi_hy_latent_in is one of plain_rows_kernel's with four waves: of up to 64 rows, K up to 512, as plain_rows_epi has them
+static bool latent_in_fits(const vmi_hy_linear_args& p, const vmi_hy_latent_prep_args& a, const vmi_hy_step& s) {
+  return p.dtype == VMI_HY_BF16 && a.dtype == VMI_HY_BF16 && p.x_kind == VMI_HY_X_ROWS && p.epilogue == VMI_HY_E_STORE && (p.K >> 5) <= 16 && !group_tiles_fit(p) &&
+         plain_rows_fit(p.M, p.N, p.K, p.groups) && a.device == p.device && s.T <= 4096 && latent_prep_lds(a.rot_n) <= 48 * 1024;
+}
+static int launch_latent_in(const vmi_hy_linear_args& p, const vmi_hy_latent_prep_args& a, const vmi_hy_step& s, hipStream_t st) {
+  const int nks = p.K >> 5, slabs = blocks8(p.N >> 4), mt = (int64_t)(p.N >> 4) * p.groups * ((p.M + 15) >> 4) <= 256 || p.M <= 16 ? 1 : 2, blocks = (p.M + 16 * mt - 1) / (16 * mt);
+  auto go = [&](auto* fn, int j) {
+    const size_t lds = std::max((size_t)4 * plain_stride(j, mt), latent_prep_lds(a.rot_n));
+    if (int rc = allow_lds(fn, lds, "vmi_hy_latent_in")) return rc;
+    hipLaunchKernelGGL(fn, dim3(s.T + slabs * blocks * p.groups), dim3(256), lds, st, p, a, s, slabs, blocks);
+    return launched("vmi_hy_latent_in");
+  };
+  if (nks <= 4) return mt == 1 ? go(latent_in_kernel<1, 1>, 1) : go(latent_in_kernel<1, 2>, 1);
+  if (nks <= 8) return mt == 1 ? go(latent_in_kernel<2, 1>, 2) : go(latent_in_kernel<2, 2>, 2);
+  return mt == 1 ? go(latent_in_kernel<4, 1>, 4) : go(latent_in_kernel<4, 2>, 4);
+}
+
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   switch (p.epilogue) {
     case VMI_HY_E_STORE: return plain_rows_epi<VMI_HY_E_STORE>(p, st);
@@ -654,3 +691,17 @@ int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 }
 
 }  // namespace vmi_hybrid
+
+extern "C" int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream) {
+  using namespace vmi_hybrid;
+  static const char* who = "vmi_hy_latent_in";
+  if (int rc = check_linear(l, who)) return rc;
+  if (int rc = check_latent_prep(a, s, who)) return rc;
+  if (!latent_in_fits(*l, *a, *s)) {
+    if (int rc = vmi_hy_linear(l, stream)) return rc;
+    return vmi_hy_latent_prep(a, s, stream);
+  }
+  DeviceScope dev(l->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  return launch_latent_in(*l, *a, *s, static_cast<hipStream_t>(stream));
+}

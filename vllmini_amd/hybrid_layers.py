@@ -243,9 +243,8 @@ class LatentAttention:
                                              rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps, scale=self.scale, gate=proj[:, self.gate_at:]), self.w_o, step)
             return
         q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
-        ops.linear(proj, self.w_uk, x_gstride=self.dim + self.rot, y_gstride=D, out=q)
-        ops.latent_prep(proj, q, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank,
-                        rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps)
+        ops.latent_in(proj, self.w_uk, q, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank,
+                      rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps)
         lat = ops.latent_attention(q, cache, step, plan.tiles, heads=H, rank=self.rank, rot=self.rot, scale=self.scale,
                                    row_tiles=plan.row_tiles, splits=plan.splits)
         o = ops.linear(lat, self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=proj[:, self.gate_at:])

@@ -99,6 +99,7 @@ SIGNATURES = {
     "vmi_hy_argmax": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_hy_rglru": (ctypes.c_int, [ctypes.POINTER(RglruArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_latent_prompt": (ctypes.c_int, [ctypes.POINTER(LatentPromptArgs), ctypes.POINTER(StepArgs), _vp]),
@@ -523,6 +524,23 @@ def latent_prep(proj: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, step: 
                  ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank, rot_n=rot_n, rank_n=rank_n, eps=eps,
                  dtype=DTYPES[proj.dtype], device=device)
     _check(load().vmi_hy_latent_prep(ctypes.byref(a), step.ref, stream))
+
+
+def latent_in(proj: torch.Tensor, w_uk: MatrixTiles, q: torch.Tensor, cache: torch.Tensor, step: StepLayout, *, norm_w: torch.Tensor, freq: torch.Tensor, heads: int, dim: int,
+              rot: int, rank: int, rot_n: int, rank_n: int, eps: float) -> None:
+    """linear(proj, w_uk, out=q), by heads, and latent_prep(); few rows in one launch."""
+    device, stream = _on(proj)
+    D = rank + rot
+    _need(proj.shape[0] == step.T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and q.dtype == proj.dtype == w_uk.tiles.dtype
+          and q.shape == (step.T, heads * D) and q.is_contiguous() and cache.dtype == proj.dtype and cache.shape[-1] == D
+          and cache.is_contiguous() and norm_w.numel() == rank and norm_w.dtype == torch.float32 and freq.dtype == torch.float64
+          and freq.numel() == rot_n // 2 and (w_uk.groups, w_uk.N, w_uk.K) == (heads, rank, dim), "hybrid_ops.latent_in: operand sizes")
+    b = LinearArgs(x=proj.data_ptr(), w=w_uk.tiles.data_ptr(), y=q.data_ptr(), ldx=proj.stride(0), ldy=q.stride(0), x_gstride=dim + rot, y_gstride=D, M=step.T, N=rank, K=dim,
+                   groups=heads, scale=1.0, x_kind=X_ROWS, epilogue=E_STORE, dtype=DTYPES[proj.dtype], device=device)
+    a = PrepArgs(proj=proj.data_ptr(), q=q.data_ptr(), cache=cache.data_ptr(), norm_w=norm_w.data_ptr(), freq=freq.data_ptr(),
+                 ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank, rot_n=rot_n, rank_n=rank_n, eps=eps,
+                 dtype=DTYPES[proj.dtype], device=device)
+    _check(load().vmi_hy_latent_in(ctypes.byref(b), ctypes.byref(a), step.ref, stream))
 
 
 def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int, rot_n: int, dtype: torch.dtype) -> bool:
