@@ -197,20 +197,12 @@ VMI_HY_API int32_t vmi_hy_latent_row_tiles(int32_t row_dim, int32_t want, int32_
 VMI_HY_API int vmi_hy_latent_attention(const vmi_hy_latent_attention_args* a, const vmi_hy_step* s, void* stream);
 
 /* Latent attention of a step whose entries have no past (every ctx is 0), over the keys and values themselves: kv [T, ldkv] = per head [dim | vdim], the latents' product with the
- * up-projections; proj and rows as vmi_hy_latent_prompt_prep leaves them; out [T, ldo], heads of vdim, times sigmoid of the head's column of gate. */
-typedef struct {
-  const void* proj;
-  const void* kv;
-  const void* rows;
-  const void* gate;
-  void* out;
-  int64_t ldp, ldkv, ldr, ldg, ldo;
-  int32_t heads, dim, rot, vdim, rank, max_len;   /* max_len: the longest entry's rows */
-  float scale;
-  int32_t dtype, device;
-} vmi_hy_latent_prompt_args;
+ * up-projections; proj and rows [T, rank + rot] as vmi_hy_latent_prompt_prep leaves them; out [T, ldo], heads of vdim, times sigmoid of the head's column of gate; max_len: the
+ * longest entry's rows. */
 VMI_HY_API int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_t rank, int32_t rot_n, int32_t dtype);   /* whether it is built for these */
-VMI_HY_API int vmi_hy_latent_prompt(const vmi_hy_latent_prompt_args* a, const vmi_hy_step* s, void* stream);
+VMI_HY_API int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads,
+                                    int32_t dim, int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s,
+                                    void* stream);
 
 /* Linear attention with a matrix state per head, S [dim, vdim] float32 (csrc/hybrid_state.hip).  proj [T, ldp] begins with the
  * columns q [kv_heads dim] | k [kv_heads dim] | v [heads vdim]; head h uses q / k head h / (heads / kv_heads).

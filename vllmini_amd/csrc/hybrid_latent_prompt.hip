@@ -17,9 +17,17 @@ namespace vmi_hybrid {
 
 constexpr int PQ = 64;   // queries of a workgroup, keys of a tile
 
+struct LatentPrompt {
+  const b16 *proj, *kv, *rows, *gate;
+  b16* out;
+  int64_t ldp, ldkv, ldr, ldg, ldo;
+  int heads, rank, max_len;
+  float scale;
+};
+
 // DN + DR columns of a key, the last DR shared by the heads; VD of a value
 template <int DN, int DR, int VD>
-__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const vmi_hy_latent_prompt_args p, const vmi_hy_step s, const int places) {
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPrompt p, const vmi_hy_step s, const int places) {
   constexpr int DK = DN + DR, LDK = DK + 8, LDV = VD + 8, NK = DK / 32, NT = VD / 16;
   constexpr int UN = PQ * DN / 2048, UR = PQ * DR / 2048, UV = PQ * VD / 2048;   // units of eight columns a thread
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -30,9 +38,9 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const vmi_hy_late
   const int qs = s.q_start[e], len = s.q_len[e], q0 = (places - 1 - at) * PQ;
   if (q0 >= len) return;
   const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
-  const b16* kv = static_cast<const b16*>(p.kv) + (int64_t)qs * p.ldkv + h * (DN + VD);
-  const b16* shared = static_cast<const b16*>(p.rows) + (int64_t)qs * p.ldr + p.rank;
-  const b16* qrow = static_cast<const b16*>(p.proj) + (int64_t)qs * p.ldp + h * DK;
+  const b16* kv = p.kv + (int64_t)qs * p.ldkv + h * (DN + VD);
+  const b16* shared = p.rows + (int64_t)qs * p.ldr + p.rank;
+  const b16* qrow = p.proj + (int64_t)qs * p.ldp + h * DK;
 
   b16x8 kn[UN], kr[UR], vr[UV];
   auto load = [&](int kt) {   // (keys past the end repeat the last one: no lane-wise condition around a load)
@@ -134,8 +142,8 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const vmi_hy_late
   }
   const int q = w0 + r16;
   if (q >= len) return;
-  const float inv = sigmoid((float)static_cast<const b16*>(p.gate)[(int64_t)(qs + q) * p.ldg + h]) / lrun;
-  b16* out = static_cast<b16*>(p.out) + (int64_t)(qs + q) * p.ldo + h * VD + 4 * kc;
+  const float inv = sigmoid((float)p.gate[(int64_t)(qs + q) * p.ldg + h]) / lrun;
+  b16* out = p.out + (int64_t)(qs + q) * p.ldo + h * VD + 4 * kc;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     b16x4 y;
@@ -146,7 +154,7 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const vmi_hy_late
 }
 
 template <int DN, int DR>
-static int launch_prompt(const vmi_hy_latent_prompt_args& p, const vmi_hy_step& s, hipStream_t st) {
+static int launch_prompt(const LatentPrompt& p, const vmi_hy_step& s, hipStream_t st) {
   auto* fn = latent_prompt_kernel<DN, DR, DN>;
   constexpr size_t lds = (size_t)PQ * (DN + DR + 8 + DN + 8) * 2;
   if (int rc = allow_lds(fn, lds, "vmi_hy_latent_prompt")) return rc;
@@ -167,18 +175,20 @@ int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_
   return dtype == VMI_HY_BF16 && (dim == 64 || dim == 128) && vdim == dim && (rot == 32 || rot == 64) && rank > 0 && (rank & 63) == 0 && rot_n > 0 && (rot_n & 15) == 0 && rot_n <= rot;
 }
 
-int vmi_hy_latent_prompt(const vmi_hy_latent_prompt_args* a, const vmi_hy_step* s, void* stream) {
+int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads, int32_t dim,
+                         int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_latent_prompt";
-  if (!a || !s || !a->proj || !a->kv || !a->rows || !a->gate || !a->out || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || a->heads <= 0 || a->max_len <= 0 || !(a->scale > 0.f))
+  if (!proj || !kv || !rows || !gate || !out || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || heads <= 0 || max_len <= 0 || !(scale > 0.f))
     return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
-  if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->vdim, a->rank, 16, a->dtype) || ((a->ldp | a->ldkv | a->ldr) & 7) || (a->ldo & 3) ||
-      (((uintptr_t)a->proj | (uintptr_t)a->kv | (uintptr_t)a->rows) & 15) || ((uintptr_t)a->out & 7))
+  if (!vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, 16, dtype) || ((ldp | ldkv) & 7) || (ldo & 3) || (((uintptr_t)proj | (uintptr_t)kv | (uintptr_t)rows) & 15) || ((uintptr_t)out & 7))
     return fail(VMI_HY_E_SHAPE, who, "built for bfloat16 heads of 64 or 128 beside 32 or 64 rotated columns, rows aligned to 16 bytes");
-  DeviceScope dev(a->device);
+  DeviceScope dev(device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (a->dim == 128) return a->rot == 64 ? launch_prompt<128, 64>(*a, *s, st) : launch_prompt<128, 32>(*a, *s, st);
-  return a->rot == 64 ? launch_prompt<64, 64>(*a, *s, st) : launch_prompt<64, 32>(*a, *s, st);
+  auto rows_of = [](const void* p) { return static_cast<const b16*>(p); };
+  const LatentPrompt p{rows_of(proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), ldp, ldkv, rank + rot, ldg, ldo, heads, rank, max_len, scale};
+  if (dim == 128) return rot == 64 ? launch_prompt<128, 64>(p, *s, st) : launch_prompt<128, 32>(p, *s, st);
+  return rot == 64 ? launch_prompt<64, 64>(p, *s, st) : launch_prompt<64, 32>(p, *s, st);
 }
 
 }  // extern "C"

@@ -55,8 +55,6 @@ RglruArgs = _struct("RglruArgs", [(_vp, "yx out conv_w conv_b gates gate_b decay
                                   (_i32, "width blocks taps single spans dtype device")])
 PrepArgs = _struct("PrepArgs", [(_vp, "proj q cache norm_w freq"), (_i64, "ldp"), (_i32, "heads dim rot rank rot_n rank_n"),
                                 (_f32, "eps"), (_i32, "dtype device")])
-LatentPromptArgs = _struct("LatentPromptArgs", [(_vp, "proj kv rows gate out"), (_i64, "ldp ldkv ldr ldg ldo"), (_i32, "heads dim rot vdim rank max_len"), (_f32, "scale"),
-                                                (_i32, "dtype device")])
 AttentionArgs = _struct("AttentionArgs", [(_vp, "q cache out tiles partial"), (_i32, "heads rank rot n_tiles row_tiles splits"),
                                           (_f32, "scale"), (_i32, "dtype device")])
 StateArgs = _struct("StateArgs", [(_vp, "proj beta z conv_w rate dt_bias decay log2_decay turns state tail o scratch out gate norm_w"),
@@ -102,7 +100,7 @@ SIGNATURES = {
     "vmi_hy_latent_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
-    "vmi_hy_latent_prompt": (ctypes.c_int, [ctypes.POINTER(LatentPromptArgs), ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_row_tiles": (_i32, [_i32, _i32, _i32]),
     "vmi_hy_latent_attention": (ctypes.c_int, [ctypes.POINTER(AttentionArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hybrid_last_error": (ctypes.c_char_p, []),
@@ -568,10 +566,8 @@ def latent_prompt(proj: torch.Tensor, w_kv: MatrixTiles, cache: torch.Tensor, st
     _check(load().vmi_hy_latent_prompt_prep(ctypes.byref(a), rows.data_ptr(), step.ref, stream))
     kv = product_tiles(rows[:, :rank], w_kv)
     out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
-    b = LatentPromptArgs(proj=proj.data_ptr(), kv=kv.data_ptr(), rows=rows.data_ptr(), gate=gate.data_ptr(), out=out.data_ptr(), ldp=proj.stride(0), ldkv=kv.stride(0), ldr=D,
-                         ldg=gate.stride(0), ldo=out.stride(0), heads=heads, dim=dim, rot=rot, vdim=vdim, rank=rank, max_len=step.max_len, scale=scale,
-                         dtype=DTYPES[proj.dtype], device=device)
-    _check(load().vmi_hy_latent_prompt(ctypes.byref(b), step.ref, stream))
+    _check(load().vmi_hy_latent_prompt(proj.data_ptr(), proj.stride(0), kv.data_ptr(), kv.stride(0), rows.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0), heads,
+                                       dim, rot, vdim, rank, step.max_len, scale, DTYPES[proj.dtype], device, step.ref, stream))
     return out
 
 
