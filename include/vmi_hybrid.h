@@ -257,6 +257,8 @@ typedef struct {
   int32_t dtype, device;
 } vmi_hy_kv_prep_args;
 VMI_HY_API int vmi_hy_kv_prep(const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream);
+/* It and vmi_hy_linear, neither of which reads what the other writes; few rows in one launch. */
+VMI_HY_API int vmi_hy_kv_prep_in(const vmi_hy_linear_args* l, const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream);
 
 /* score = scale q . k + bias[h][min(i - j, bias_n - 1)]; token i sees the j <= i of its own chunk of `chunk` tokens (0: all);
  * sink[h] adds exp(sink) to the denominator; out = softmax . v * sigmoid(gate[t, h]).  bias, sink and gate may be NULL; bias and

@@ -463,6 +463,29 @@ def test_kv_prep_normalises_and_writes_the_cache(dtype):
     assert (flat[rest] == 9).all()
 
 
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("T", [1, 16, 17, 50, 64, 65])
+@pytest.mark.parametrize("N,K", [(64, 32), (1024, 128), (96, 160), (32, 512), (32, 544)])
+def test_a_product_beside_kv_prep_is_the_product_and_kv_prep(dtype, T, N, K):
+    """Every bit of the two launches it stands for, rows past the last one left alone; sizes on both sides of what goes into one launch."""
+    from vllmini_amd import hybrid_ops as ops
+
+    H, G, dim, vdim, page = 4, 2, 64, 32, 16
+    g = torch.Generator().manual_seed(T + K)
+    step = layout([1] * T, list(range(5, 5 + T)), np.arange(T * 6).reshape(T, 6), page)
+    proj = torch.randn(T, (H + G) * dim + G * vdim + 32, generator=g).to(dtype).to(dev())
+    x = torch.randn(T, 3 * K, generator=g).to(dtype).to(dev())
+    w = ops.MatrixTiles((torch.randn(2, N, K, generator=g) * K ** -0.5).to(dev()), dtype)
+    qs = [torch.full((T + 2, H * dim), 3.0, dtype=dtype, device=dev()) for _ in range(2)]
+    caches = [torch.full((T * 6, page, G * (dim + vdim)), 9.0, dtype=dtype, device=dev()) for _ in range(2)]
+    names = dict(heads=H, kv_heads=G, dim=dim, vdim=vdim, dim_n=dim, eps=1e-5)
+    want = ops.linear(x[:, K:], w, x_gstride=K, y_gstride=N)
+    ops.kv_prep(proj, qs[0][:T], caches[0], step, **names)
+    got, beside = ops.linear_beside(x[:, K:], w, K, N)
+    ops.kv_prep(proj, qs[1][:T], caches[1], step, beside=beside, **names)
+    assert torch.equal(got, want) and torch.equal(*qs) and torch.equal(*caches)
+
+
 # ---- the whole decoder -------------------------------------------------------------------------------------------------------------
 _PLAIN = {}
 N = 90

@@ -93,7 +93,7 @@ LAYER_LIB_PATH = os.path.join(OUT_DIR, "libvmi_gpt2_layer.so")
 
 # the layers of decoders that mix recurrences, linear and softmax attention (include/vmi_hybrid.h), loaded by hybrid_ops.py only
 SRC_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hip") for t in ("linear", "rows", "tiles", "rglru", "latent", "latent_prompt", "state", "attention")]
-HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "linear", "latent_prep", "softmax")] + [os.path.join(CSRC, f"{t}.hpp") for t in ("mfma_tiles", "step_inputs", "lane_ops")]
+HDRS_HYBRID = [os.path.join(CSRC, f"hybrid_{t}.hpp") for t in ("common", "kv_prep", "linear", "latent_prep", "softmax")] + [os.path.join(CSRC, f"{t}.hpp") for t in ("mfma_tiles", "step_inputs", "lane_ops")]
 HYBRID_LIB_PATH = os.path.join(OUT_DIR, "libvmi_hybrid.so")
 
 # the operators' checks and calls in native code: an extension module over torch's C++ interface, loaded by _lib.py (no device code)

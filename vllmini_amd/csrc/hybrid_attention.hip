@@ -11,6 +11,7 @@
 //                    keeps the scores of ONE row, and its probabilities, as they lie, are an operand of O^T = V^T P^T (k-index 8 kc + e of a step of 32 is key
 //                    4 kc + e, e < 4, or 16 + 4 kc + e - 4, and the values are read in that order); sums are a product with ones
 // Tiles too few for the chip have their keys dealt to `splits` workgroups.
+#include "hybrid_kv_prep.hpp"
 #include "hybrid_softmax.hpp"
 
 namespace vmi_hybrid {
@@ -416,39 +417,9 @@ __global__ __launch_bounds__(256, NV <= 8 ? 2 : 1) void gqa_rows_kernel(const vm
   }
 }
 
-// q and k over their root mean square, k and v into the cache; one workgroup per token, 16 lanes per head
 template <typename T>
 __global__ __launch_bounds__(256) void kv_prep_kernel(const vmi_hy_kv_prep_args p, const vmi_hy_step s) {
-  const int t = blockIdx.x, tid = threadIdx.x, l = tid & 15, D = p.dim + p.vdim;
-  if (s.tok_seq[t] < 0) return;
-  const int64_t slot = s.tok_slot[t];
-  const T* row = static_cast<const T*>(p.proj) + (int64_t)t * p.ldp;
-  T* crow = slot >= 0 ? static_cast<T*>(p.cache) + slot * p.kv_heads * D : nullptr;
-  for (int u = tid >> 4; u < p.heads + p.kv_heads; u += 16) {
-    const T* src = row + (int64_t)u * p.dim;
-    float ss = 0.f;
-    for (int k = l * 8; k < p.dim; k += 128) {
-      const f32x8 v = to_f32<T>(load8(src + k));
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss = fmaf(v[e], v[e], ss);
-    }
-    ss = sum16(ss);
-    const float r = 1.f / sqrtf(ss / (float)p.dim_n + p.eps);
-    T* dst = u < p.heads ? static_cast<T*>(p.q) + ((int64_t)t * p.heads + u) * p.dim : crow ? crow + (int64_t)(u - p.heads) * D : nullptr;
-    if (!dst) continue;
-    for (int k = l * 8; k < p.dim; k += 128) {
-      f32x8 v = to_f32<T>(load8(src + k));
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= r;
-      *reinterpret_cast<V8<T>*>(dst + k) = from_f32<T>(v);
-    }
-  }
-  if (!crow) return;
-  const T* v = row + (int64_t)(p.heads + p.kv_heads) * p.dim;
-  for (int u = tid * 8; u < p.kv_heads * p.vdim; u += 2048) {
-    const int g = u / p.vdim, k = u - g * p.vdim;
-    *reinterpret_cast<V8<T>*>(crow + (int64_t)g * D + p.dim + k) = load8(v + u);
-  }
+  kv_prep_token<T>(p, s, blockIdx.x);
 }
 
 template <typename T>
@@ -520,6 +491,15 @@ static int run_gqa(const vmi_hy_attention_args& p, const vmi_hy_step& s, hipStre
   return wide ? gqa_width<T, 64>(p, s, st) : gqa_width<T, 32>(p, s, st);
 }
 
+int check_kv_prep(const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, const char* who) {
+  if (!a || !s || !a->proj || !a->q || !a->cache || !s->tok_seq || !s->tok_slot || s->T <= 0 || a->heads <= 0 || a->kv_heads <= 0 ||
+      a->heads % a->kv_heads || a->dim <= 0 || a->vdim <= 0 || a->dim_n <= 0 || a->dim_n > a->dim)
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if ((a->dim & 31) || (a->vdim & 31) || (a->ldp & 7) || ((uintptr_t)a->proj & 15))
+    return fail(VMI_HY_E_SHAPE, who, "needs sizes that are multiples of 32 and aligned rows");
+  return VMI_HY_OK;
+}
+
 }  // namespace vmi_hybrid
 
 using namespace vmi_hybrid;
@@ -528,11 +508,7 @@ extern "C" {
 
 int vmi_hy_kv_prep(const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_kv_prep";
-  if (!a || !s || !a->proj || !a->q || !a->cache || !s->tok_seq || !s->tok_slot || s->T <= 0 || a->heads <= 0 || a->kv_heads <= 0 ||
-      a->heads % a->kv_heads || a->dim <= 0 || a->vdim <= 0 || a->dim_n <= 0 || a->dim_n > a->dim)
-    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
-  if ((a->dim & 31) || (a->vdim & 31) || (a->ldp & 7) || ((uintptr_t)a->proj & 15))
-    return fail(VMI_HY_E_SHAPE, who, "needs sizes that are multiples of 32 and aligned rows");
+  if (int rc = check_kv_prep(a, s, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);

@@ -4,6 +4,7 @@
 // cores' layout (16 rows x 64 bytes) in LDS; all arguments are asked for at once (`need`: left to itself the compiler asks branch by branch, a trip to
 // memory each); what the epilogue adds to is asked for in front of everything.  The waves' partial tiles meet in LDS; one wave a tile adds them in
 // the order of K and stores.
+#include "hybrid_kv_prep.hpp"
 #include "hybrid_latent_prep.hpp"
 #include "hybrid_linear.hpp"
 
@@ -159,15 +160,24 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
   plain_rows_slab<RW, J, MT, NB, EPI, NCH, XI, XK>(p, blockIdx.x, blockIdx.y * 16 * MT, blockIdx.z, smem);
 }
 
-// The queries' way into the latent space, by heads, and what a token's latent attention needs besides: two launches of a chain that do not read each other's results, in one.  The
-// first T workgroups take a token each, the others a slab of 16 columns of 16 MT rows of a head.  8 heads of 128 into 512, 12 rows, us: 4.2 + 4.9 -> 4.8 (each little more than its launch);
-// width 1024, 12 sequences, 24 tokens 7311 -> 7203, width 4096, one, 16 tokens 14 019 -> 13 919.
-template <int J, int MT>
-__global__ __launch_bounds__(256, 1) void latent_in_kernel(const vmi_hy_linear_args p, const vmi_hy_latent_prep_args a, const vmi_hy_step s, const int slabs, const int blocks) {
+// A product by heads and what a token's attention needs besides: two launches of a chain that do not read each other's results, in one.  The
+// first T workgroups take a token each, the others a slab of 16 columns of 16 MT rows of a head.  Few rows, each is little more than its launch: queries into the latent space beside
+// latent_prep, 8 heads of 128 into 512, 12 rows, us: 4.2 + 4.9 -> 4.8; width 1024, 12 sequences, 24 tokens 7311 -> 7203, width 4096, one, 16 tokens 14 019 -> 13 919.
+// The gates' products (2 of 2048 x 128, 32 rows) beside kv_prep 4.5 + 5.1 -> 5.0.
+struct LatentPrep {
+  vmi_hy_latent_prep_args a;
+  __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char* smem) const { latent_prep_token<b16, false>(a, s, nullptr, t, reinterpret_cast<float*>(smem)); }
+};
+struct KvPrep {
+  vmi_hy_kv_prep_args a;
+  __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char*) const { kv_prep_token<b16>(a, s, t); }
+};
+template <int J, int MT, class Prep>
+__global__ __launch_bounds__(256, 1) void rows_beside_kernel(const vmi_hy_linear_args p, const Prep prep, const vmi_hy_step s, const int slabs, const int blocks) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int at = (int)blockIdx.x - s.T;
   if (at < 0) {
-    latent_prep_token<b16, false>(a, s, nullptr, blockIdx.x, reinterpret_cast<float*>(smem));
+    prep.token(s, blockIdx.x, smem);
   } else {
     const int rest = at / slabs, grp = rest / blocks;
     plain_rows_slab<4, J, MT, 1, VMI_HY_E_STORE>(p, at - rest * slabs, (rest - grp * blocks) * 16 * MT, grp, smem);
@@ -664,22 +674,23 @@ int launch_concat_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   return with_chunks(p.K, whole);
 }
 
-// Whether the product of vmi_hy_latent_in is one of plain_rows_kernel's with four waves: of up to 64 rows, K up to 512, as plain_rows_epi has them
-static bool latent_in_fits(const vmi_hy_linear_args& p, const vmi_hy_latent_prep_args& a, const vmi_hy_step& s) {
-  return p.dtype == VMI_HY_BF16 && a.dtype == VMI_HY_BF16 && p.x_kind == VMI_HY_X_ROWS && p.epilogue == VMI_HY_E_STORE && (p.K >> 5) <= 16 && !group_tiles_fit(p) &&
-         plain_rows_fit(p.M, p.N, p.K, p.groups) && a.device == p.device && s.T <= 4096 && latent_prep_lds(a.rot_n) <= 48 * 1024;
+// Whether a product is one of plain_rows_kernel's with four waves: of up to 64 rows, K up to 512, as plain_rows_epi has them
+static bool beside_fits(const vmi_hy_linear_args& p, const vmi_hy_step& s) {
+  return p.dtype == VMI_HY_BF16 && p.x_kind == VMI_HY_X_ROWS && p.epilogue == VMI_HY_E_STORE && (p.K >> 5) <= 16 && !group_tiles_fit(p) && plain_rows_fit(p.M, p.N, p.K, p.groups) &&
+         s.T <= 4096;
 }
-static int launch_latent_in(const vmi_hy_linear_args& p, const vmi_hy_latent_prep_args& a, const vmi_hy_step& s, hipStream_t st) {
+template <class Prep>
+static int launch_beside(const vmi_hy_linear_args& p, const Prep& prep, const vmi_hy_step& s, size_t prep_lds, const char* who, hipStream_t st) {
   const int nks = p.K >> 5, slabs = blocks8(p.N >> 4), mt = (int64_t)(p.N >> 4) * p.groups * ((p.M + 15) >> 4) <= 256 || p.M <= 16 ? 1 : 2, blocks = (p.M + 16 * mt - 1) / (16 * mt);
   auto go = [&](auto* fn, int j) {
-    const size_t lds = std::max((size_t)4 * plain_stride(j, mt), latent_prep_lds(a.rot_n));
-    if (int rc = allow_lds(fn, lds, "vmi_hy_latent_in")) return rc;
-    hipLaunchKernelGGL(fn, dim3(s.T + slabs * blocks * p.groups), dim3(256), lds, st, p, a, s, slabs, blocks);
-    return launched("vmi_hy_latent_in");
+    const size_t lds = std::max((size_t)4 * plain_stride(j, mt), prep_lds);
+    if (int rc = allow_lds(fn, lds, who)) return rc;
+    hipLaunchKernelGGL(fn, dim3(s.T + slabs * blocks * p.groups), dim3(256), lds, st, p, prep, s, slabs, blocks);
+    return launched(who);
   };
-  if (nks <= 4) return mt == 1 ? go(latent_in_kernel<1, 1>, 1) : go(latent_in_kernel<1, 2>, 1);
-  if (nks <= 8) return mt == 1 ? go(latent_in_kernel<2, 1>, 2) : go(latent_in_kernel<2, 2>, 2);
-  return mt == 1 ? go(latent_in_kernel<4, 1>, 4) : go(latent_in_kernel<4, 2>, 4);
+  if (nks <= 4) return mt == 1 ? go(rows_beside_kernel<1, 1, Prep>, 1) : go(rows_beside_kernel<1, 2, Prep>, 1);
+  if (nks <= 8) return mt == 1 ? go(rows_beside_kernel<2, 1, Prep>, 2) : go(rows_beside_kernel<2, 2, Prep>, 2);
+  return mt == 1 ? go(rows_beside_kernel<4, 1, Prep>, 4) : go(rows_beside_kernel<4, 2, Prep>, 4);
 }
 
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
@@ -692,16 +703,34 @@ int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
 
 }  // namespace vmi_hybrid
 
-extern "C" int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream) {
-  using namespace vmi_hybrid;
+using namespace vmi_hybrid;
+
+extern "C" {
+
+int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_latent_in";
   if (int rc = check_linear(l, who)) return rc;
   if (int rc = check_latent_prep(a, s, who)) return rc;
-  if (!latent_in_fits(*l, *a, *s)) {
+  if (a->dtype != l->dtype || a->device != l->device || !beside_fits(*l, *s)) {
     if (int rc = vmi_hy_linear(l, stream)) return rc;
     return vmi_hy_latent_prep(a, s, stream);
   }
   DeviceScope dev(l->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  return launch_latent_in(*l, *a, *s, static_cast<hipStream_t>(stream));
+  return launch_beside(*l, LatentPrep{*a}, *s, latent_prep_lds(a->rot_n), who, static_cast<hipStream_t>(stream));
 }
+
+int vmi_hy_kv_prep_in(const vmi_hy_linear_args* l, const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_kv_prep_in";
+  if (int rc = check_linear(l, who)) return rc;
+  if (int rc = check_kv_prep(a, s, who)) return rc;
+  if (a->dtype != l->dtype || a->device != l->device || !beside_fits(*l, *s)) {
+    if (int rc = vmi_hy_linear(l, stream)) return rc;
+    return vmi_hy_kv_prep(a, s, stream);
+  }
+  DeviceScope dev(l->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  return launch_beside(*l, KvPrep{*a}, *s, 0, who, static_cast<hipStream_t>(stream));
+}
+
+}  // extern "C"

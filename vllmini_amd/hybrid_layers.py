@@ -215,8 +215,9 @@ class LatentAttention:
         # ... and, for prompts that nothing stands in front of, the latents into every head's keys and values
         self.w_kv = None
         if self.scale > 0 and ops.latent_prompt_fits(self.dim, self.rot, self.vdim, self.rank, rot_dims, dtype):
-            kv = torch.cat([spread(uk.view(heads, dim, rank), 1, torch.arange(dim), self.dim), spread(uv.view(heads, vdim, rank), 1, torch.arange(vdim), self.vdim)], dim=1)
-            self.w_kv = MatrixTiles(spread(kv.reshape(-1, rank), 1, torch.arange(rank), self.rank), dtype)
+            kv = uk.new_zeros((heads, self.dim + self.vdim, self.rank), dtype=dtype)
+            kv[:, :dim, :rank], kv[:, self.dim:self.dim + vdim, :rank] = uk.view(heads, dim, rank), uv.view(heads, vdim, rank)
+            self.w_kv = MatrixTiles(kv.view(-1, self.rank), dtype)
         self.w_o = MatrixTiles(spread(spread(o, 1, strided_index(heads, vdim, self.vdim), heads * self.vdim), 0, torch.arange(width), E),
                                dtype, dense=True)
         self.norm_w = torch.zeros(self.rank, dtype=torch.float32, device=dev)
@@ -432,9 +433,14 @@ class GatedDelta:
         z = self.sizes
         return [((z["heads"], z["dim"], z["vdim"]), torch.float32), ((2, self.taps - 1, self.channels), self.dtype)]
 
-    def run(self, proj: torch.Tensor, out: torch.Tensor, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor]) -> None:
+    def beside(self, proj: torch.Tensor) -> Tuple[torch.Tensor, ops.LinearArgs]:
+        """What needs nothing but the projections, still to be launched: run()'s `low`, and the launch."""
+        return ops.linear_beside(proj[:, self.low_at:], self.w_low, self.rank, self.low_n)
+
+    def run(self, proj: torch.Tensor, out: torch.Tensor, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor], low: Optional[torch.Tensor] = None) -> None:
         z, n = self.sizes, self.low_n
-        low = ops.linear(proj[:, self.low_at:], self.w_low, x_gstride=self.rank, y_gstride=n)
+        if low is None:
+            low = ops.linear(proj[:, self.low_at:], self.w_low, x_gstride=self.rank, y_gstride=n)
         ops.linear_state(proj, step, kind=ops.DELTA, state=held[0], tail=held[1], beta=proj[:, self.channels:self.channels + z["heads"]],
                          z=low[:, :z["heads"] * z["dim"]], gate=low[:, n:n + z["heads"] * z["vdim"]], act="sigmoid", norm_w=self.norm_w,
                          conv_w=self.conv_w, rate=self.rate, dt_bias=self.dt_bias, out=out, **z)
@@ -487,10 +493,10 @@ class GroupedAttention:
         z = self.sizes
         return QueryTiling("grouped", z["heads"] // z["kv_heads"], z["kv_heads"], z["vdim"], self.chunk, (z["dim"], z["vdim"]))
 
-    def run(self, proj: torch.Tensor, out: torch.Tensor, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor]) -> None:
+    def run(self, proj: torch.Tensor, out: torch.Tensor, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor], beside: Optional[ops.LinearArgs] = None) -> None:
         z, plan = self.sizes, plans[self.tiling()]
         q = torch.empty((step.T, z["heads"] * z["dim"]), dtype=proj.dtype, device=proj.device)
-        ops.kv_prep(proj, q, held[0], step, dim_n=self.dim_n, eps=self.eps, **z)
+        ops.kv_prep(proj, q, held[0], step, dim_n=self.dim_n, eps=self.eps, beside=beside, **z)
         ops.attention(q, held[0], step, plan.tiles, scale=self.scale, row_tiles=plan.row_tiles, splits=plan.splits, out=out,
                       chunk=self.chunk, bias=self.bias, sink=self.sink, gate=proj[:, self.gate_at:self.gate_at + z["heads"]], **z)
 
@@ -523,9 +529,13 @@ class TwoArms:
     def run(self, proj: torch.Tensor, out: torch.Tensor, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor]) -> None:
         pages = len(self.page_rows())
         pg, st, at, col = list(held[:pages]), list(held[pages:]), 0, 0
-        for a, (rows, cols) in zip(self.arms, self.spans):
+        extra = [{}, {}]
+        if isinstance(self.arms[0], GroupedAttention) and isinstance(self.arms[1], GatedDelta):   # (few rows: the second arm's first launch inside the first one's)
+            low, launch = self.arms[1].beside(proj[:, self.spans[0][0]:])
+            extra = [{"beside": launch}, {"low": low}]
+        for a, (rows, cols), more in zip(self.arms, self.spans, extra):
             n, m = len(a.page_rows()), len(a.state_shapes())
-            a.run(proj[:, at:], out[:, col:col + cols], step, plans, pg[:n] + st[:m])
+            a.run(proj[:, at:], out[:, col:col + cols], step, plans, pg[:n] + st[:m], **more)
             pg, st, at, col = pg[n:], st[m:], at + rows, col + cols
 
     def merge(self, res: Residual, branches: Sequence[torch.Tensor], add: Optional[torch.Tensor]) -> None:
@@ -547,6 +557,9 @@ class ParallelBlock:
         self.w_in = MatrixTiles(rows, dtype, dense=True) if gate is None else gated_matrix(torch.cat([rows, interleaved(gate, up, E)]), dtype, self.n_in)
         groups = [[*outs, *tail]] if len(outs) == 1 else [[w] for w in (*outs, *tail)]
         self.w_out = [MatrixTiles(torch.cat(g, dim=1), dtype, dense=True) for g in groups]
+        self.w_pair = None      # both branches' matrices as groups of one product, where they are alike
+        if len(outs) == 2 and outs[0].shape == outs[1].shape:
+            self.w_pair = MatrixTiles.joined(self.w_out[:2])
         del mixer.in_weight, mixer.outs      # (they live on in the tiles)
 
     def page_rows(self) -> List[int]:
@@ -571,11 +584,17 @@ class ParallelBlock:
         if len(self.w_out) == 1:
             res.branch_out(rows, self.w_out[0], step)
             return
-        at, branches = 0, []
-        for w in self.w_out[:2]:
-            o = rows[:, at:at + w.K]
-            branches.append(product(o, w) if dense(T, w) else ops.linear(o, w))
-            at += w.K
+        branches: List[torch.Tensor] = []
+        if self.w_pair is not None and not dense(T, self.w_out[0]) and ops.linear_plain(T, self.w_pair):
+            K, N = self.w_pair.K, self.w_pair.N
+            both = ops.linear(rows, self.w_pair, x_gstride=K, y_gstride=N)
+            branches = [both[:, :N], both[:, N:]]
+        else:
+            at = 0
+            for w in self.w_out[:2]:
+                o = rows[:, at:at + w.K]
+                branches.append(product(o, w) if dense(T, w) else ops.linear(o, w))
+                at += w.K
         add = None
         if self.ff:
             if dense(T, self.w_out[2]):

@@ -22,7 +22,7 @@ import ctypes
 import functools
 import os
 import threading
-from typing import NamedTuple, Optional, Tuple
+from typing import NamedTuple, Optional, Sequence, Tuple
 
 import torch
 
@@ -97,6 +97,7 @@ SIGNATURES = {
     "vmi_hy_argmax": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp]),
     "vmi_hy_rglru": (ctypes.c_int, [ctypes.POINTER(RglruArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_kv_prep_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(KvPrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
@@ -205,6 +206,16 @@ class MatrixTiles:
         p[:, :N, :K] = w.to(dtype)
         self.tiles = p.view(G, self.N // 16, 16, self.K // 32, 4, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
         self.dense = p[0].contiguous() if dense and G == 1 else None
+
+    @classmethod
+    def joined(cls, parts: "Sequence[MatrixTiles]") -> "MatrixTiles":
+        """Matrices of one size as the groups of one product; their tiles become parts of its."""
+        both = cls.__new__(cls)
+        both.groups, both.N, both.K, both.dense = len(parts), parts[0].N, parts[0].K, None
+        both.tiles = torch.cat([w.tiles for w in parts])
+        for g, w in enumerate(parts):
+            w.tiles = both.tiles[g:g + 1]
+        return both
 
 
 def linear(x: torch.Tensor, w: MatrixTiles, *, norm: Optional[NormArgs] = None, x2: Optional[torch.Tensor] = None,
@@ -332,6 +343,16 @@ def _normed_first(M: int, N: int, K: int, groups: int, dtype: torch.dtype) -> bo
 def linear_normed_first(M: int, w: MatrixTiles) -> bool:
     """Whether linear(x, w, norm=...) of M rows norms them by a launch of their own."""
     return _normed_first(M, w.N, w.K, w.groups, w.tiles.dtype)
+
+
+def linear_plain(M: int, w: MatrixTiles) -> bool:
+    """Whether linear(x, w) of M rows as they are runs in the kernel for few of them."""
+    return _plain(M, w.N, w.K, w.groups, w.tiles.dtype)
+
+
+@functools.lru_cache(maxsize=4096)
+def _plain(M: int, N: int, K: int, groups: int, dtype: torch.dtype) -> bool:
+    return bool(load().vmi_hy_linear_plain(M, N, K, groups, DTYPES[dtype]))
 
 
 def linear_resident(M: int, w: MatrixTiles) -> bool:
@@ -524,6 +545,14 @@ def latent_prep(proj: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, step: 
     _check(load().vmi_hy_latent_prep(ctypes.byref(a), step.ref, stream))
 
 
+def _by_groups(x: torch.Tensor, w: MatrixTiles, y: torch.Tensor, x_gstride: int, y_gstride: int, device: int) -> LinearArgs:
+    """The arguments of linear(x, w, out=y), rows as they are and columns stored."""
+    _need(x.dim() == 2 and x.stride(1) == 1 and x.dtype == y.dtype == w.tiles.dtype and x.shape[1] >= (w.groups - 1) * x_gstride + w.K and y.shape[0] == x.shape[0]
+          and y.shape[1] >= (w.groups - 1) * y_gstride + w.N and y.stride(1) == 1 and x.device == y.device == w.tiles.device, "hybrid_ops: operands of a product by groups")
+    return LinearArgs(x=x.data_ptr(), w=w.tiles.data_ptr(), y=y.data_ptr(), ldx=x.stride(0), ldy=y.stride(0), x_gstride=x_gstride, y_gstride=y_gstride, M=x.shape[0], N=w.N, K=w.K,
+                      groups=w.groups, scale=1.0, x_kind=X_ROWS, epilogue=E_STORE, dtype=DTYPES[x.dtype], device=device)
+
+
 def latent_in(proj: torch.Tensor, w_uk: MatrixTiles, q: torch.Tensor, cache: torch.Tensor, step: StepLayout, *, norm_w: torch.Tensor, freq: torch.Tensor, heads: int, dim: int,
               rot: int, rank: int, rot_n: int, rank_n: int, eps: float) -> None:
     """linear(proj, w_uk, out=q), by heads, and latent_prep(); few rows in one launch."""
@@ -533,8 +562,7 @@ def latent_in(proj: torch.Tensor, w_uk: MatrixTiles, q: torch.Tensor, cache: tor
           and q.shape == (step.T, heads * D) and q.is_contiguous() and cache.dtype == proj.dtype and cache.shape[-1] == D
           and cache.is_contiguous() and norm_w.numel() == rank and norm_w.dtype == torch.float32 and freq.dtype == torch.float64
           and freq.numel() == rot_n // 2 and (w_uk.groups, w_uk.N, w_uk.K) == (heads, rank, dim), "hybrid_ops.latent_in: operand sizes")
-    b = LinearArgs(x=proj.data_ptr(), w=w_uk.tiles.data_ptr(), y=q.data_ptr(), ldx=proj.stride(0), ldy=q.stride(0), x_gstride=dim + rot, y_gstride=D, M=step.T, N=rank, K=dim,
-                   groups=heads, scale=1.0, x_kind=X_ROWS, epilogue=E_STORE, dtype=DTYPES[proj.dtype], device=device)
+    b = _by_groups(proj, w_uk, q, dim + rot, D, device)
     a = PrepArgs(proj=proj.data_ptr(), q=q.data_ptr(), cache=cache.data_ptr(), norm_w=norm_w.data_ptr(), freq=freq.data_ptr(),
                  ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank, rot_n=rot_n, rank_n=rank_n, eps=eps,
                  dtype=DTYPES[proj.dtype], device=device)
@@ -643,16 +671,26 @@ def linear_state(proj: torch.Tensor, step: StepLayout, *, kind: int, heads: int,
     _check(lib.vmi_hy_state(ctypes.byref(a), step.ref, stream))
 
 
+def linear_beside(x: torch.Tensor, w: MatrixTiles, x_gstride: int, y_gstride: int) -> Tuple[torch.Tensor, LinearArgs]:
+    """linear(x, w) by groups, still to be launched (kv_prep's `beside`): where its result will be, and what names it."""
+    device, _ = _on(x)
+    y = torch.empty((x.shape[0], (w.groups - 1) * y_gstride + w.N), dtype=x.dtype, device=x.device)
+    return y, _by_groups(x, w, y, x_gstride, y_gstride, device)
+
+
 def kv_prep(proj: torch.Tensor, q: torch.Tensor, cache: torch.Tensor, step: StepLayout, *, heads: int, kv_heads: int, dim: int, vdim: int,
-            dim_n: int, eps: float) -> None:
-    """proj [T, q | k | v ...]: q and k over their root mean square, q to q, k and v to the cache."""
+            dim_n: int, eps: float, beside: Optional[LinearArgs] = None) -> None:
+    """proj [T, q | k | v ...]: q and k over their root mean square, q to q, k and v to the cache; and a product that reads none of it."""
     device, stream = _on(proj)
     _need(proj.shape[0] == step.T and proj.shape[1] >= (heads + kv_heads) * dim + kv_heads * vdim and proj.stride(1) == 1
           and q.shape == (step.T, heads * dim) and q.is_contiguous() and q.dtype == proj.dtype and cache.dtype == proj.dtype
           and cache.shape[-1] == kv_heads * (dim + vdim) and cache.is_contiguous(), "hybrid_ops.kv_prep: operand sizes")
     a = KvPrepArgs(proj=proj.data_ptr(), q=q.data_ptr(), cache=cache.data_ptr(), ldp=proj.stride(0), heads=heads, kv_heads=kv_heads,
                    dim=dim, vdim=vdim, dim_n=dim_n, eps=eps, dtype=DTYPES[proj.dtype], device=device)
-    _check(load().vmi_hy_kv_prep(ctypes.byref(a), step.ref, stream))
+    if beside is not None:
+        _check(load().vmi_hy_kv_prep_in(ctypes.byref(beside), ctypes.byref(a), step.ref, stream))
+    else:
+        _check(load().vmi_hy_kv_prep(ctypes.byref(a), step.ref, stream))
 
 
 def attention_row_tiles(dim: int, vdim: int, want: int, dtype: torch.dtype) -> int:
