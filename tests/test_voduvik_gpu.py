@@ -633,6 +633,20 @@ def test_recurrence_over_portions_in_wide_blocks(dtype, width, blocks):
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("lens", [[64 * 9 + 1], [30, 64 * 63 + 34], [30, 64 * 63 + 35]])
+def test_recurrence_over_long_portions(dtype, lens):
+    """Carries over more tiles than a request holds, one that ends with its tile, and one tile more than run in one launch; a second portion takes the state up."""
+    k = _Rglru(64, 2, 4, dtype, slots=2)
+    seqs = [k.inputs(n + 3, 40 + i) for i, n in enumerate(lens)]
+    got = []
+    for at, counts in ((0, lens), (1, [3] * len(lens))):
+        step = layout(counts, [0] * len(lens) if at == 0 else lens, [[0]] * len(lens), 64, flips=[at] * len(lens), pos_slots=False)
+        got.append(k.run(torch.cat([s[2][:n] if at == 0 else s[2][n:] for s, n in zip(seqs, lens)]), step).split(counts))
+    for i, s in enumerate(seqs):
+        close(torch.cat([got[0][i], got[1][i]]), k.plain(*s[:2]), dtype, tol32=3e-5, tol16=1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 @pytest.mark.parametrize("width,blocks", [(512, 2), (96, 3)])
 def test_portions_that_share_rows_taken_together_with_padding(dtype, width, blocks):
     """Portions of one to nine tokens, so that the eight (four) rows of a thread hold several starts, and rows behind them that are no token's and hold NaN."""

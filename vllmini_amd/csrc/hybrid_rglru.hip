@@ -376,6 +376,49 @@ __global__ __launch_bounds__(256) void rglru_finish_kernel(const vmi_hy_rglru_ar
   store_out8<T>(p, t, c, o, to_f32<T>(load8(static_cast<const T*>(p.yx) + (int64_t)t * p.ldx + c)));
 }
 
+// Both in one: a workgroup takes a row tile's leading segment and 256 channels, and runs the carry up to it itself.  Each tile so reads the ends of all tiles of its entry in front of
+// it, which is less than a launch of its own takes up to MOST_TILES of them; beyond, that grows with their square.  rglru_carry_kernel + rglru_finish_kernel / here, us: width 2048, 1 x
+// 130 rows 4.2 + 4.2 / 7.6, 4 x up to 1024 5.8 + 11.4 / 15.1, 40 x 100 4.3 + 6.5 / 10.0, 1 x 4096 15.2 + 16.5 / 25.3, x 8192 28.8 + 31.2 / 67.2; 1024, 1 x 4096 25.0 / 19.9, x 8192 43.5 / 37.8.
+constexpr int MOST_TILES = 64;
+template <typename T>
+__global__ __launch_bounds__(256) void rglru_lead_kernel(const vmi_hy_rglru_args p, const vmi_hy_step s) {
+  constexpr int BM = 64, U = 8;
+  const int c = (blockIdx.x * 32 + threadIdx.x % 32) * 8, tile = blockIdx.y, t0 = tile * BM;
+  const int q = s.tok_seq[t0];
+  if (c >= p.width || q < 0) return;
+  const int qs = s.q_start[q], qe = qs + s.q_len[q];
+  if (qs >= t0) return;
+  const float* S = p.scratch + c;
+  const float* P = p.scratch + (int64_t)s.T * p.width + c;
+  auto end_of = [&](int k) { return (int64_t)(k * BM + BM - 1) * p.width; };
+  f32x8 carry = load8(S + end_of(qs / BM));
+  for (int k = qs / BM + 1; k < tile; k += U) {
+    f32x8 sv[U], pv[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {   // (past the last one: that one again)
+      sv[i] = load8(S + end_of(min(k + i, tile - 1)));
+      pv[i] = load8(P + end_of(min(k + i, tile - 1)));
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (k + i < tile) {   // (scalar)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) carry[e] = fmaf(pv[i][e], carry[e], sv[i][e]);
+      }
+  }
+  const int end = min(t0 + BM, qe);
+#pragma unroll 4
+  for (int t = t0 + threadIdx.x / 32; t < end; t += 8) {
+    const f32x8 a = load8(S + (int64_t)t * p.width), b = load8(P + (int64_t)t * p.width);
+    const V8<T> y = load8(static_cast<const T*>(p.yx) + (int64_t)t * p.ldx + c);
+    f32x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = fmaf(b[e], carry[e], a[e]);
+    store_out8<T>(p, t, c, o, to_f32<T>(y));
+    if (t == qe - 1) *reinterpret_cast<f32x8*>(p.state + (int64_t)s.state_slot[q] * p.width + c) = o;
+  }
+}
+
 // A step of single tokens, bfloat16.  A workgroup takes 16 tokens x NO tiles of 16 channels of one gate block; its eight waves share the block's channels, the k of
 // the gate products: a lane convolves eight channels of one token, which is the products' operand as it stands, so nothing goes through LDS but the partial products
 // and the workgroup's own channels.  Tokens are their entries, so what the tables say of a token is asked for at once.  Bound by three trips through memory
@@ -555,6 +598,10 @@ static int run_rglru(const vmi_hy_rglru_args& p, const vmi_hy_step& s, hipStream
                            : (wide ? launch_tile<T, 64, 0, CT>(p, s, st) : launch_tile<T, 64, 0, 64>(p, s, st)))
     return rc;
   if (!p.spans) return VMI_HY_OK;
+  if (const int tiles = (s.T + 63) / 64; tiles <= MOST_TILES) {
+    hipLaunchKernelGGL(rglru_lead_kernel<T>, dim3((p.width / 8 + 31) / 32, tiles), dim3(256), 0, st, p, s);
+    return launched("vmi_hy_rglru");
+  }
   hipLaunchKernelGGL(rglru_carry_kernel, dim3((p.width + 63) / 64, s.B), dim3(64), 0, st, p, s);
   hipLaunchKernelGGL(rglru_finish_kernel<T>, dim3((p.width / 8 + 255) / 256, s.T), dim3(256), 0, st, p, s);
   return launched("vmi_hy_rglru");
