@@ -11,6 +11,7 @@
 // Bound by the vector unit's share of the softmax and the chain of a tile (1.4 us).  Attention, us, the latents walked -> here, rank 512: 16 heads, 4 prompts of up to 1024 tokens
 // 117 -> 39, 1 of 500 28 + 12 (its splits added up) -> 16, 16 of up to 200 33 -> 15; 8 heads, 1 of 60 14.6 -> 5.8, 35 of up to 21 14.4 -> 5.7, 1 of 1024 45 + 12 -> 26; and one product of the latents
 // with both up-projections stands for two by heads, of the same work (16 heads, 2773 rows 27 + 19 us).
+// Off 64 bits by as much, latents / here, eight draws each: 8 heads, 60 rows 0.00346 / 0.00350, 300 + 200 + 100 0.00355 / 0.00357, 600 0.00364 / 0.00363; 16 heads, 1024 0.00362 / 0.00360.
 #include "hybrid_softmax.hpp"
 
 namespace vmi_hybrid {

@@ -145,7 +145,9 @@ int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
 // 19 us of host) and whole tiles of 256 columns: K 1024 to 2047 0.88 (8 of 207 more than 5 per cent behind), to 4095 0.96 (52 of 239), to 6144 1.00 (30 of 104), beyond 1.07; other columns
 // 0.74, 0.85, 0.96 and 0.99.  So not past K 6144 from 5.6 million results on, up to there whole columns up to 9 million (N 3072, K 4608, 4100 rows 90 / 109) and only where the tiles' own costs promise 1020
 // TFLOP/s (N 2048, K 6144: 2773 rows 69 / 60, which one round of tiles holds; 3250 73 / 85), and below K 4096 whole columns up to 9 million (N 4096, K 2048: 2400 41 / 42, level from there on), below 2048 up to 15.
-// Not where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4), where tiles of 64 x 64 are just more than
+// Not where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4): measured again over 380 pairs of up to 128
+// such tiles, now that results leave as lines, ours / library's in the mean K 3072 0.93, 3584 and 4096 up to N 2048 0.96 (N 3072 1.17 and 1.02), 4608 and 5120 0.99 and 1.00 (1.11), 6144 1.15, 8192
+// 1.31; and a call of the library's is 12 us more of host, which is what a short prompt waits for (62 rows, N 1024, K 3072 10.4 / 8.6 us, host 20 / 8).  Nor where tiles of 64 x 64 are just more than
 // the chip has compute units for (300 rows, N 4096, K 8192 46 / 56; 600 rows, N 2048, K 6144 34 / 37), and past K 16 383.
 static bool product_pays(int M, int N, int K) {
   const bool whole = N % 256 == 0;
@@ -157,7 +159,8 @@ static bool product_pays(int M, int N, int K) {
   } else if (whole && K >= 1024 && results >= (K >= 2048 ? 9000000 : 15000000)) {
     return false;
   }
-  if (K >= 3072 && (least <= 128 || (whole && N >= 2048 && results >= 1050000 && results < 2400000))) return false;
+  const bool shared = K > 4096 || (K > 3072 && N > 2048);   // (up to 4096 and 2048 nothing is to be had from sharing K out)
+  if (K >= 3072 && ((shared && least <= 128) || (whole && N >= 2048 && results >= 1050000 && results < 2400000))) return false;
   return K < 16384;
 }
 
