@@ -553,6 +553,34 @@ def test_elementwise_ends(dtype, n):
 
 
 # ---- the recurrent block ---------------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("ld", [32, 1024, 1056, 2080, 4096, 4128, 8192, 8224])
+def test_rows_of_every_width_added_normed_and_merged(dtype, ld):
+    """What a workgroup keeps of a row by its length, and what is read again behind it; columns that are not normed hold numbers for the sum alone."""
+    from vllmini_amd import hybrid_ops as ops
+
+    n, T = ld - 8, 3
+    g = torch.Generator().manual_seed(ld)
+    x, a, b, c = (torch.randn(T, ld, generator=g).to(dev()) for _ in range(4))
+    a, b, c = (t.to(dtype) for t in (a, b, c))
+    w, u = ((1 + 0.3 * torch.randn(ld, generator=g)).to(dev()) for _ in range(2))
+    w[n:] = u[n:] = 0
+    for rms in (False, True):
+        y = x.clone()
+        h = ops.add_norm(y, a, (w, n, 1e-5, rms), dtype)
+        want = x.double() + a.double()
+        close(y, want, torch.float32, tol32=1e-6)
+        d = want[:, :n] - (0 if rms else want[:, :n].mean(-1, keepdim=True))
+        close(h[:, :n], d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-5) * w[:n].double(), dtype, tol16=6e-3)
+        assert not h[:, n:].any()
+    a[:, n:] = b[:, n:] = 0
+    for add in (None, c):
+        y = x.clone()
+        ops.merge(y, a, w, b, u, add, n=n, eps=1e-5, scale=0.5)
+        unit = [t.double() / torch.sqrt((t.double() ** 2).sum(-1, keepdim=True) / n + 1e-5) * v.double() for t, v in ((a, w), (b, u))]
+        close(y, x.double() + 0.5 * (unit[0] + unit[1]) + (0 if add is None else c.double()), torch.float32, tol32=2e-6)
+
+
 def _rglru_weights(width, blocks, taps, seed):
     c = cases.config([cases.rglru(width, blocks, taps)], width=width)
     return cases.tensors(c, seed)

@@ -588,37 +588,52 @@ __global__ __launch_bounds__(256) void embed_kernel(const int64_t* __restrict__ 
   }
 }
 
-// one workgroup per row of x, or of its rows[t]; a row of up to 8192 columns stays in registers between the three passes
-template <typename T>
+// One workgroup per row of x, or of its rows[t]; NV times 1024 columns of it stay in registers between the three passes (what a row has beyond them, with NV = 8, is read again).
+// All of that, the addend and the norm's weight are asked for at once: with a load, an add and a store to the row a step, each step waited for the one before, and the weight came a
+// trip to memory behind the statistics.  us, with an addend, so / here: 60 rows of 1024 / 2048 / 4096 3.9 / 4.0 / 4.7 -> 3.4 / 3.4 / 3.9, 2773 9.8 / 14.0 / 23.6 -> 7.0 / 11.8 / 21.7 (4.4 TB/s).
+template <typename T, int NV>
 __global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, const int* rows, const T* add, int64_t ld_add,
                                                        const float* norm_w, T* out, int n, int ld, float eps, int rms) {
   __shared__ float part[2][4];
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   float* row = x + (rows ? rows[t] : t) * ldx;
-  constexpr int MAXV = 8;
-  f32x4 v[MAXV];
+  f32x4 v[NV], w[NV];
+  V4<T> d[NV];
   float s = 0.f;
-  auto fetch = [&](int k) {
-    f32x4 a = *reinterpret_cast<const f32x4*>(row + k);
-    if (add) {
-      const V4<T> d = *reinterpret_cast<const V4<T>*>(add + (int64_t)t * ld_add + k);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) a[e] += (float)d[e];
-      *reinterpret_cast<f32x4*>(row + k) = a;
-    }
-    return a;
-  };
   auto sum = [&](const f32x4& a, int k) {   // (of the n columns that are normed: what lies behind them may be anything)
     s += (k < n ? a[0] : 0.f) + (k + 1 < n ? a[1] : 0.f) + (k + 2 < n ? a[2] : 0.f) + (k + 3 < n ? a[3] : 0.f);
   };
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
+  for (int i = 0; i < NV; ++i) {   // (past the row: its last columns again)
+    const int k = min((tid + i * 256) * 4, ld - 4);
+    v[i] = *reinterpret_cast<const f32x4*>(row + k);
+    if (add) d[i] = *reinterpret_cast<const V4<T>*>(add + (int64_t)t * ld_add + k);
+    if (out) w[i] = *reinterpret_cast<const f32x4*>(norm_w + k);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
     const int k = (tid + i * 256) * 4;
-    v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (k < ld) v[i] = fetch(k);
+    if (add) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] += (float)d[i][e];
+      if (k < ld) *reinterpret_cast<f32x4*>(row + k) = v[i];
+    }
     sum(v[i], k);
   }
-  for (int k = (tid + MAXV * 256) * 4; k < ld; k += 1024) sum(fetch(k), k);
+  auto rest = [&](auto step) {
+    if constexpr (NV == 8)
+      for (int k = (tid + NV * 256) * 4; k < ld; k += 1024) step(k);
+  };
+  rest([&](int k) {
+    f32x4 a = *reinterpret_cast<const f32x4*>(row + k);
+    if (add) {
+      const V4<T> more = *reinterpret_cast<const V4<T>*>(add + (int64_t)t * ld_add + k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] += (float)more[e];
+      *reinterpret_cast<f32x4*>(row + k) = a;
+    }
+    sum(a, k);
+  });
   if (!out) return;
   float mean = 0.f;
   if (!rms) {
@@ -631,34 +646,39 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* x, int64_t ldx, co
   auto dev2 = [&](const f32x4& a, int k) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float d = k + e < n ? a[e] - mean : 0.f;
-      q = fmaf(d, d, q);
+      const float c = k + e < n ? a[e] - mean : 0.f;
+      q = fmaf(c, c, q);
     }
   };
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) dev2(v[i], (tid + i * 256) * 4);
-  for (int k = (tid + MAXV * 256) * 4; k < ld; k += 1024) dev2(*reinterpret_cast<const f32x4*>(row + k), k);
+  for (int i = 0; i < NV; ++i) dev2(v[i], (tid + i * 256) * 4);
+  rest([&](int k) { dev2(*reinterpret_cast<const f32x4*>(row + k), k); });
   q = wave_sum(q);
   if (lane == 0) part[1][wave] = q;
   __syncthreads();
   const float rstd = 1.f / sqrtf((part[1][0] + part[1][1] + part[1][2] + part[1][3]) / (float)n + eps);
-  auto put = [&](const f32x4& a, int k) {
-    const f32x4 w = *reinterpret_cast<const f32x4*>(norm_w + k);
+  auto put = [&](const f32x4& a, const f32x4& g, int k) {
     V4<T> o;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (T)((a[e] - mean) * rstd * w[e]);
+    for (int e = 0; e < 4; ++e) o[e] = (T)((a[e] - mean) * rstd * g[e]);
     *reinterpret_cast<V4<T>*>(out + (int64_t)t * ld + k) = o;
   };
 #pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
+  for (int i = 0; i < NV; ++i) {
     const int k = (tid + i * 256) * 4;
-    if (k < ld) put(v[i], k);
+    if (k < ld) put(v[i], w[i], k);
   }
-  for (int k = (tid + MAXV * 256) * 4; k < ld; k += 1024) put(*reinterpret_cast<const f32x4*>(row + k), k);
+  rest([&](int k) { put(*reinterpret_cast<const f32x4*>(row + k), *reinterpret_cast<const f32x4*>(norm_w + k), k); });
 }
 
-// x += scale (rms norm of a + rms norm of b) + add; one workgroup per row
 template <typename T>
+static void launch_add_norm(int M, hipStream_t st, float* x, int64_t ldx, const int* rows, const T* add, int64_t ld_add, const float* norm_w, T* out, int n, int ld, float eps, int rms) {
+  auto* fn = ld <= 1024 ? add_norm_kernel<T, 1> : ld <= 2048 ? add_norm_kernel<T, 2> : ld <= 4096 ? add_norm_kernel<T, 4> : add_norm_kernel<T, 8>;
+  hipLaunchKernelGGL(fn, dim3(M), dim3(256), 0, st, x, ldx, rows, add, ld_add, norm_w, out, n, ld, eps, rms);
+}
+
+// x += scale (rms norm of a + rms norm of b) + add; one workgroup per row.  NV times 1024 columns are asked for at once, all that is read of them; NV = 0: any number, read as they come
+template <typename T, int NV>
 __global__ __launch_bounds__(256) void merge_kernel(float* x, const T* a, int64_t ld_a, const T* b, int64_t ld_b, const T* add,
                                                     int64_t ld_add, const float* wa, const float* wb, int n, int ld, float eps,
                                                     float scale) {
@@ -666,13 +686,43 @@ __global__ __launch_bounds__(256) void merge_kernel(float* x, const T* a, int64_
   const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   a += (int64_t)t * ld_a;
   b += (int64_t)t * ld_b;
+  float* row = x + (int64_t)t * ld;
   float sa = 0.f, sb = 0.f;
-  for (int k = tid * 4; k < ld; k += 1024) {   // (padding columns are zeros)
-    const V4<T> va = *reinterpret_cast<const V4<T>*>(a + k), vb = *reinterpret_cast<const V4<T>*>(b + k);
+  struct Four {
+    V4<T> a, b, d;
+    f32x4 x, wa, wb;
+  };
+  auto squares = [&](const Four& u) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      sa = fmaf((float)va[e], (float)va[e], sa);
-      sb = fmaf((float)vb[e], (float)vb[e], sb);
+      sa = fmaf((float)u.a[e], (float)u.a[e], sa);
+      sb = fmaf((float)u.b[e], (float)u.b[e], sb);
+    }
+  };
+  auto branches = [&](Four& u, int k) {
+    u.a = *reinterpret_cast<const V4<T>*>(a + k);
+    u.b = *reinterpret_cast<const V4<T>*>(b + k);
+  };
+  auto others = [&](Four& u, int k) {
+    u.wa = *reinterpret_cast<const f32x4*>(wa + k);
+    u.wb = *reinterpret_cast<const f32x4*>(wb + k);
+    u.x = *reinterpret_cast<const f32x4*>(row + k);
+    if (add) u.d = *reinterpret_cast<const V4<T>*>(add + (int64_t)t * ld_add + k);
+  };
+  [[maybe_unused]] Four held[NV ? NV : 1];
+  if constexpr (NV > 0) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) branches(held[i], min((tid + 256 * i) * 4, ld - 4));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) others(held[i], min((tid + 256 * i) * 4, ld - 4));
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if ((tid + 256 * i) * 4 < ld) squares(held[i]);   // (padding columns are zeros)
+  } else {
+    for (int k = tid * 4; k < ld; k += 1024) {
+      Four u;
+      branches(u, k);
+      squares(u);
     }
   }
   sa = wave_sum(sa);
@@ -681,19 +731,25 @@ __global__ __launch_bounds__(256) void merge_kernel(float* x, const T* a, int64_
   __syncthreads();
   const float ra = scale / sqrtf((part[0][0] + part[0][1] + part[0][2] + part[0][3]) / (float)n + eps);
   const float rb = scale / sqrtf((part[1][0] + part[1][1] + part[1][2] + part[1][3]) / (float)n + eps);
-  float* row = x + (int64_t)t * ld;
-  for (int k = tid * 4; k < ld; k += 1024) {
-    const V4<T> va = *reinterpret_cast<const V4<T>*>(a + k), vb = *reinterpret_cast<const V4<T>*>(b + k);
-    const f32x4 w0 = *reinterpret_cast<const f32x4*>(wa + k), w1 = *reinterpret_cast<const f32x4*>(wb + k);
-    f32x4 v = *reinterpret_cast<const f32x4*>(row + k);
+  auto put = [&](Four& u, int k) {
     if (add) {
-      const V4<T> d = *reinterpret_cast<const V4<T>*>(add + (int64_t)t * ld_add + k);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += (float)d[e];
+      for (int e = 0; e < 4; ++e) u.x[e] += (float)u.d[e];
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += (float)va[e] * ra * w0[e] + (float)vb[e] * rb * w1[e];
-    *reinterpret_cast<f32x4*>(row + k) = v;
+    for (int e = 0; e < 4; ++e) u.x[e] += (float)u.a[e] * ra * u.wa[e] + (float)u.b[e] * rb * u.wb[e];
+    *reinterpret_cast<f32x4*>(row + k) = u.x;
+  };
+  if constexpr (NV > 0) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if ((tid + 256 * i) * 4 < ld) put(held[i], (tid + 256 * i) * 4);
+  } else {
+    for (int k = tid * 4; k < ld; k += 1024) {
+      Four u;
+      branches(u, k), others(u, k);
+      put(u, k);
+    }
   }
 }
 
@@ -800,8 +856,7 @@ int vmi_hy_linear(const vmi_hy_linear_args* a, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (a->x_kind == VMI_HY_X_NORM && a->normed && a->dtype == VMI_HY_BF16 && a->epilogue != VMI_HY_E_RESIDUAL && a->epilogue != VMI_HY_E_GATED) {
     if (launch_norm_few(*a, st) != VMI_HY_OK)
-      hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(a->M), dim3(256), 0, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr,
-                       (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
+      launch_add_norm<b16>(a->M, st, const_cast<float*>(static_cast<const float*>(a->x)), a->ldx, a->rows, nullptr, (int64_t)0, a->norm_w, static_cast<b16*>(a->normed), a->norm_n, a->K, a->eps, a->rms);
     vmi_hy_linear_args rows = *a;
     rows.x = a->normed, rows.ldx = a->K, rows.x_gstride = 0, rows.rows = nullptr, rows.x_kind = VMI_HY_X_ROWS;   // (all groups read the same rows)
     return linear_normed(rows, st);
@@ -838,10 +893,10 @@ int vmi_hy_add_norm(float* x, const void* add, int64_t ld_add, const float* norm
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == VMI_HY_BF16)
-    hipLaunchKernelGGL(add_norm_kernel<b16>, dim3(T), dim3(256), 0, st, x, (int64_t)ld, nullptr, static_cast<const b16*>(add), ld_add, norm_w,
+    launch_add_norm<b16>(T, st, x, (int64_t)ld, nullptr, static_cast<const b16*>(add), ld_add, norm_w,
                        static_cast<b16*>(out), n, ld, eps, rms);
   else
-    hipLaunchKernelGGL(add_norm_kernel<float>, dim3(T), dim3(256), 0, st, x, (int64_t)ld, nullptr, static_cast<const float*>(add), ld_add, norm_w,
+    launch_add_norm<float>(T, st, x, (int64_t)ld, nullptr, static_cast<const float*>(add), ld_add, norm_w,
                        static_cast<float*>(out), n, ld, eps, rms);
   return launched(who);
 }
@@ -872,12 +927,13 @@ int vmi_hy_merge(float* x, const void* a, int64_t ld_a, const void* b, int64_t l
   DeviceScope dev(device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == VMI_HY_BF16)
-    hipLaunchKernelGGL(merge_kernel<b16>, dim3(T), dim3(256), 0, st, x, static_cast<const b16*>(a), ld_a, static_cast<const b16*>(b), ld_b,
-                       static_cast<const b16*>(add), ld_add, wa, wb, n, ld, eps, scale);
-  else
-    hipLaunchKernelGGL(merge_kernel<float>, dim3(T), dim3(256), 0, st, x, static_cast<const float*>(a), ld_a, static_cast<const float*>(b),
-                       ld_b, static_cast<const float*>(add), ld_add, wa, wb, n, ld, eps, scale);
+  auto go = [&](auto kind) {
+    using T_ = decltype(kind);
+    auto* fn = ld <= 1024 ? merge_kernel<T_, 1> : ld <= 2048 ? merge_kernel<T_, 2> : ld <= 4096 ? merge_kernel<T_, 4> : merge_kernel<T_, 0>;
+    hipLaunchKernelGGL(fn, dim3(T), dim3(256), 0, st, x, static_cast<const T_*>(a), ld_a, static_cast<const T_*>(b), ld_b, static_cast<const T_*>(add), ld_add, wa, wb, n, ld, eps, scale);
+  };
+  if (dtype == VMI_HY_BF16) go(b16{});
+  else go(float{});
   return launched(who);
 }
 
