@@ -43,7 +43,7 @@ all: $(LIB) $(LAYER_LIB) $(HYBRID_LIB) oracle
 
 hybrid: $(HYBRID_LIB)
 
-$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_linear.hpp $(CSRC)/hybrid_softmax.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp $(CSRC)/lane_ops.hpp include/vmi_hybrid.h
+$(HYBRID_LIB): $(HYBRID_SRCS) $(CSRC)/hybrid_common.hpp $(CSRC)/hybrid_kv_prep.hpp $(CSRC)/hybrid_latent_prep.hpp $(CSRC)/hybrid_linear.hpp $(CSRC)/hybrid_softmax.hpp $(CSRC)/mfma_tiles.hpp $(CSRC)/step_inputs.hpp $(CSRC)/lane_ops.hpp include/vmi_hybrid.h
 	mkdir -p $(OUTDIR)
 	$(HIPCC) $(filter-out -ffp-contract=off,$(FLAGS)) -shared $(HYBRID_SRCS) -o $@
 
