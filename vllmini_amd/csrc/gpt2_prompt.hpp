@@ -335,7 +335,8 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
   constexpr int PIECES = 8 * NI, MINE = MI / 2 * NI;   // sixteen bytes of results: of a row, and those of a lane
   h16x4 bias[NI];
   h16x8 res[ADD ? MINE : 1];
-  const bool wide = ((p.ldy & 7) | ((uintptr_t)p.y & 15)) == 0, wide_res = ((p.ldr & 7) | ((uintptr_t)p.res & 15)) == 0;
+  typedef h16x8 Eight __attribute__((aligned(8)));   // (rows of four are all that is asked of a residual: one request all the same)
+  const bool wide = ((p.ldy & 7) | ((uintptr_t)p.y & 15)) == 0;
   auto ask_bias = [&](const vmi_tiles::Where& at) {
 #pragma unroll
     for (int n = 0; n < NI; ++n) bias[n] = Tail::load_bias(p, min(at.s0 + at.wave * NI + n, at.SL - 1) * 16 + 4 * at.kc);
@@ -345,12 +346,7 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
     for (int k = 0; k < MINE; ++k) {
       const int u = (int)threadIdx.x + 256 * (k % NI), row = u / PIECES, piece = u - row * PIECES;
       const h16* from = p.res + (int64_t)min(at.m0 + 32 * (k / NI) + row, p.M - 1) * p.ldr + min(at.s0 * 16 + 8 * piece, p.N - 8);
-      if (wide_res) {   // (scalar)
-        res[k] = *reinterpret_cast<const h16x8*>(from);
-      } else {
-        const h16x4 l = *reinterpret_cast<const h16x4*>(from), h = *reinterpret_cast<const h16x4*>(from + 4);
-        res[k] = __builtin_shufflevector(l, h, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
+      res[k] = *reinterpret_cast<const Eight*>(from);
     }
   };
   vmi_tiles::tiles_product<vmi_tiles::Half, MI, NI, D>(
@@ -380,7 +376,7 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const LinearParams p) {
             for (int e = 0; e < 8; ++e) o[e] = (h16)((float)res[k][e] + (float)a[e]);
             v = __builtin_bit_cast(vmi_tiles::u32x4, o);
           }
-          if (m < p.M && n < p.N) vmi_tiles::put_piece(p.y + (int64_t)m * p.ldy + n, v, wide);
+          vmi_tiles::put_piece(m < p.M && n < p.N, p.y + (int64_t)m * p.ldy + n, v, wide);
         };
         // (GELU takes the vector pipes as long as the product takes the matrix cores, so its waves go on one by one: 2000 rows, N 3072, K 768 15.6 us, by lines 15.9; 6400 40.6 / 44)
         if constexpr (EPI == VMI_LAYER_EPI_BIAS_GELU && NI % 2 == 0) vmi_tiles::pairs_out<MI, NI>(at, pack, put);

@@ -42,15 +42,14 @@ __global__ __launch_bounds__(256, 2) void tiles_kernel(const vmi_hy_linear_args 
           if (EPI == VMI_HY_E_STORE || first + 64 * NI <= p.n_split) {   // (scalar)
             const bool wide = ((p.ldy & 7) | ((uintptr_t)p.y & 15)) == 0;
             vmi_tiles::lines_out<u32x2, MI, NI, false>(at, stored, [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
-              if (at.m0 + row < p.M && first + 8 * piece < p.N) vmi_tiles::put_piece(static_cast<b16*>(p.y) + (int64_t)(at.m0 + row) * p.ldy + first + 8 * piece, v, wide);
+              vmi_tiles::put_piece(at.m0 + row < p.M && first + 8 * piece < p.N, static_cast<b16*>(p.y) + (int64_t)(at.m0 + row) * p.ldy + first + 8 * piece, v, wide);
             });
             return;
           }
           if (first >= p.n_split) {
             const bool wide = ((p.ldy2 & 7) | ((uintptr_t)p.y2 & 15) | (p.n_split & 15)) == 0;
             vmi_tiles::lines_out<uint32_t, MI, NI, true>(at, gated, [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
-              if (at.m0 + row < p.M && first + 16 * piece < p.N)
-                vmi_tiles::put_piece(static_cast<b16*>(p.y2) + (int64_t)(at.m0 + row) * p.ldy2 + ((first - p.n_split) >> 1) + 8 * piece, v, wide);
+              vmi_tiles::put_piece(at.m0 + row < p.M && first + 16 * piece < p.N, static_cast<b16*>(p.y2) + (int64_t)(at.m0 + row) * p.ldy2 + ((first - p.n_split) >> 1) + 8 * piece, v, wide);
             });
             return;
           }
@@ -101,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void group_tiles_kernel(const vmi_hy_linear
               return __builtin_bit_cast(u32x2, o);
             },
             [&](int row, int piece, const vmi_tiles::u32x4& v, int) {
-              if (at.m0 + row < p.M && at.s0 * 16 + 8 * piece < p.N) vmi_tiles::put_piece(y + (int64_t)(at.m0 + row) * p.ldy + 8 * piece, v, wide);
+              vmi_tiles::put_piece(at.m0 + row < p.M && at.s0 * 16 + 8 * piece < p.N, y + (int64_t)(at.m0 + row) * p.ldy + 8 * piece, v, wide);
             });
       });
 }

@@ -97,13 +97,15 @@ __device__ __forceinline__ void pairs_out(const Where& at, Pack&& pack, Put&& pu
       put(16 * i + at.r16, (at.wave * NI + n + (at.kc & 1)) * 2 + (at.kc >> 1), u32x4{l[0], h[0], l[1], h[1]}, 0);
     }
 }
-// sixteen bytes of results; wide: rows of y and where they begin are aligned to as many, else to four
-__device__ __forceinline__ void put_piece(void* y, const u32x4& v, bool wide) {
+// sixteen bytes of results, where this lane's are any; wide: rows of y and where they begin are aligned to as many, else to four (the scalar condition outside: inside the other one it is a branch more)
+__device__ __forceinline__ void put_piece(bool on, void* y, const u32x4& v, bool wide) {
   if (wide) {   // (scalar)
-    *static_cast<u32x4*>(y) = v;
+    if (on) *static_cast<u32x4*>(y) = v;
   } else {
+    if (on) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) static_cast<uint32_t*>(y)[r] = v[r];
+      for (int r = 0; r < 4; ++r) static_cast<uint32_t*>(y)[r] = v[r];
+    }
   }
 }
 
@@ -178,7 +180,8 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     }
   }
   const Where at{m0, col * 4 * NI, SL, wave, kc, r16, {xs0, xs1}};
-  early(at);
+  if constexpr (std::is_invocable_v<Early&, const Where&>) early(at);
+  else early(m0 + r16, s0, SL);   // (this lane's first row, this wave's first slab)
   x_landed(std::integral_constant<int, D - 2>{});
   // The chunk in place d, and chunk kb on its way into the place of the one before (whose readers have all passed the barrier): steps of one fragment of x, which was asked
   // for AHEAD steps before, against the wave's NI of W, and its share of the requests.  A chunk that is none is zeros, x and W
@@ -227,7 +230,8 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     }
   };
   rest(std::integral_constant<int, 1>{}), rest(std::integral_constant<int, 2>{}), rest(std::integral_constant<int, 3>{});
-  finish(acc, at);
+  if constexpr (std::is_invocable_v<Finish&, decltype((acc)), const Where&>) finish(acc, at);
+  else finish(acc, m0 + r16, s0, SL);
 }
 
 // ---- which tile -----------------------------------------------------------------------------------------------------------------
