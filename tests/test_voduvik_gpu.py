@@ -986,6 +986,24 @@ def test_prompts_over_keys_and_over_latents_lead_to_the_same_decoder(lens, monke
             logits_close(torch.stack([x[i] for x in got]), want[i][n - 1: n + 2], torch.bfloat16)
 
 
+def test_prompts_of_more_places_than_a_launch_has_workgroups():
+    """Entries of one token each under a longest one of 65 535: places, entries and heads come to more than 2^24, and a token alone attends to its own value."""
+    from vllmini_amd import hybrid_ops as ops
+
+    H, dim, rot, rank, T, bf = 3, 64, 32, 64, 5500, torch.bfloat16
+    g = torch.Generator(device=dev()).manual_seed(1)
+    proj = torch.randn(T, H * (dim + rot) + rank + rot + 32, generator=g, device=dev()).to(bf)
+    up = (torch.randn(H, 2 * dim, rank, generator=g, device=dev()) * rank ** -0.5).to(bf)
+    step = layout([1] * T, [0] * T, np.arange(T)[:, None], 1)
+    step.fresh, step.max_len = True, 65535
+    assert H * T * -(-step.max_len // 64) >= 1 << 24
+    cache, gate = torch.zeros((T, 1, rank + rot), dtype=bf, device=dev()), proj[:, H * (dim + rot) + rank + rot:]
+    out = ops.latent_prompt(proj.clone(), ops.MatrixTiles(up.reshape(-1, rank), bf), cache, step, vdim=dim, scale=0.1, gate=gate, norm_w=torch.ones(rank, device=dev()),
+                            freq=torch.ones(rot // 2, dtype=torch.float64, device=dev()), heads=H, dim=dim, rot=rot, rank=rank, rot_n=rot, rank_n=rank, eps=1e-5)
+    value = cache[:, 0, :rank].float() @ up[:, dim:].reshape(-1, rank).float().T
+    close(out, value.view(T, H, dim).mul(torch.sigmoid(gate[:, :H].float())[:, :, None]).reshape(T, -1), bf, tol16=8e-3)      # (two roundings to bfloat16)
+
+
 # ---- the whole decoder -------------------------------------------------------------------------------------------------------------
 _PLAIN = {}
 

@@ -28,14 +28,14 @@ struct LatentPrompt {
 
 // DN + DR columns of a key, the last DR shared by the heads; VD of a value
 template <int DN, int DR, int VD>
-__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPrompt p, const vmi_hy_step s, const int places) {
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPrompt p, const vmi_hy_step s, const int places, const int first) {
   constexpr int DK = DN + DR, LDK = DK + 8, LDV = VD + 8, NK = DK / 32, NT = VD / 16;
   constexpr int UN = PQ * DN / 2048, UR = PQ * DR / 2048, UV = PQ * VD / 2048;   // units of eight columns a thread
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   b16* ks = reinterpret_cast<b16*>(smem);   // [64][LDK]
   b16* vs = ks + PQ * LDK;                  // [64][LDV]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int H = p.heads, each = H * s.B, at = blockIdx.x / each, rest = blockIdx.x - at * each, e = rest / H, h = rest - e * H;
+  const int H = p.heads, tile = first + (int)blockIdx.x / H, h = (int)blockIdx.x % H, at = tile / s.B, e = tile - at * s.B;
   const int qs = s.q_start[e], len = s.q_len[e], q0 = (places - 1 - at) * PQ;
   if (q0 >= len) return;
   const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
@@ -160,10 +160,14 @@ static int launch_prompt(const LatentPrompt& p, const vmi_hy_step& s, hipStream_
   constexpr size_t lds = (size_t)PQ * (DN + DR + 8 + DN + 8) * 2;
   if (int rc = allow_lds(fn, lds, "vmi_hy_latent_prompt")) return rc;
   const int places = (p.max_len + PQ - 1) / PQ;
-  const int64_t groups = (int64_t)places * p.heads * s.B;
-  if (groups >= (1 << 24)) return fail(VMI_HY_E_SHAPE, "vmi_hy_latent_prompt", "too many heads, entries and positions");   // (2^32 work items)
-  hipLaunchKernelGGL(fn, dim3((uint32_t)groups), dim3(256), lds, st, p, s, places);
-  return launched("vmi_hy_latent_prompt");
+  const int64_t tiles = (int64_t)places * s.B;
+  if (tiles > INT32_MAX || p.heads > 65535) return fail(VMI_HY_E_SHAPE, "vmi_hy_latent_prompt", "too many heads, or entries and positions");
+  const int n = (int)tiles, most = ((1 << 24) - 1) / p.heads;   // (a launch is of fewer than 2^32 work items)
+  for (int first = 0; first < n; first += std::min(most, n - first)) {
+    hipLaunchKernelGGL(fn, dim3((uint32_t)(p.heads * std::min(most, n - first))), dim3(256), lds, st, p, s, places, first);
+    if (int rc = launched("vmi_hy_latent_prompt")) return rc;
+  }
+  return VMI_HY_OK;
 }
 
 }  // namespace vmi_hybrid
