@@ -986,6 +986,55 @@ def test_prompts_over_keys_and_over_latents_lead_to_the_same_decoder(lens, monke
             logits_close(torch.stack([x[i] for x in got]), want[i][n - 1: n + 2], torch.bfloat16)
 
 
+@pytest.mark.parametrize("dim,rot,rank", [(128, 64, 512), (64, 32, 64)])
+@pytest.mark.parametrize("counts,ctx", [([70], [0]), ([1, 70, 1], [40, 0, 3]), ([130, 5, 2, 1], [0, 17, 0, 0]), ([64, 1, 65], [0, 0, 0]), ([1] * 60 + [3], [7] * 60 + [0]),
+                                        ([1, 9, 1, 1], [90, 0, 4, 64])])
+def test_a_prompt_comes_to_the_same_whatever_shares_its_step(dim, rot, rank, counts, ctx):
+    """The layer over a step of prompts and other portions against the same entries in two steps, the prompts' and the others': every bit of the results and of the cache."""
+    from vllmini_amd import hybrid_layers as layers, hybrid_ops as ops
+    from vllmini_amd.hybrid_decoder import HybridDecoder
+
+    H, page, bf = 3, 32, torch.bfloat16
+    g, D, hd, B = torch.Generator().manual_seed(dim + len(counts)), rank + rot, dim + rot, len(counts)
+    w = lambda *s: torch.randn(s, generator=g).mul(s[-1] ** -0.5).to(bf).to(dev())      # noqa: E731
+    layer = layers.LatentAttention(width=32, heads=H, dim=dim, rot=rot, vdim=dim, rank=rank, scale=hd ** -0.5, rot_base=500.0, rot_dims=rot, norm=layers.Norm(torch.ones(32, device=dev()), 32, 1e-5),
+                                   q=w(H * hd, 32), dkv=w(D, 32), dkv_norm=torch.ones(rank, device=dev()), uk=w(H * dim, rank), uv=w(H * dim, rank), g=w(H, 32), o=w(32, H * dim), dtype=bf)
+    counts, ctx = np.asarray(counts), np.asarray(ctx)
+    T, at = int(counts.sum()), np.cumsum(counts) - counts
+    proj = torch.randn(T, layer.w_in.N, generator=g).to(bf).to(dev())
+    per = -(-(ctx + counts) // page)
+    tables = np.zeros((B, per.max()), dtype=np.int64)
+    for b in range(B):
+        tables[b, :per[b]] = per[:b].sum() + np.arange(per[b])
+    pages = torch.randn(int(per.sum()), page, D, generator=g).to(bf).to(dev())
+    d = object.__new__(HybridDecoder)
+    d.model, d._kinds = type("Model", (), {"dtype": bf}), [layer.tiling()]
+
+    def run(own, splits=None):
+        """(the rows of the entries `own`, the cache) of a step of these entries alone."""
+        n, c = counts[own], ctx[own]
+        tok = np.concatenate([np.arange(at[b], at[b] + counts[b]) for b in own])
+        a = {"entry": np.repeat(np.arange(len(own)), n), "pos": tok, "slots": [tok], "ctx": c, "state_slot": n * 0, "parity": n * 0, "tables": tables[own][None]}
+        sec, _, _, plans = d._layout(a, n, np.arange(1), len(tok), len(own), tables.shape[1], int((c + n).max()))
+        rt, sp, nt, spans = plans[0]
+        plan = layers.AttentionPlan(i32(sec["tiles0"]).view(nt, 2), rt, splits or sp, None if spans is None else ops.PromptTiles(i32(sec["prompts0"]).view(-1, 2), *spans))
+        cache, rows, step = pages.clone(), [], layout(n, c, tables[own], page)
+        res = type("Residual", (), {"branch_in": lambda self, *a: proj[torch.as_tensor(tok, device=dev())].clone(), "branch_out": lambda self, o, *a: rows.append(o)})()
+        layer.run(res, step, {layer.tiling(): plan}, [cache])
+        return rows[0], cache, plan
+
+    prompts, others = np.flatnonzero((ctx == 0) & (counts > 1)), np.flatnonzero((ctx > 0) | (counts == 1))
+    got, cache, plan = run(np.arange(B))
+    assert plan.prompts is not None and sorted(set(plan.prompts.tiles[:, 0].tolist())) == prompts.tolist()
+    for own in (prompts, others):
+        if len(own):
+            want, alone, part = run(own, plan.splits if own is others else None)
+            assert (part.prompts is not None) == (own is prompts) and (own is prompts or part.row_tiles == plan.row_tiles)
+            for b, rows in zip(own, want.split(counts[own].tolist())):
+                assert torch.equal(got[at[b]: at[b] + counts[b]], rows), b
+                assert torch.equal(cache[tables[b, :per[b]]], alone[tables[b, :per[b]]])
+
+
 def test_prompts_of_more_places_than_a_launch_has_workgroups():
     """Entries of one token each under a longest one of 65 535: places, entries and heads come to more than 2^24, and a token alone attends to its own value."""
     from vllmini_amd import hybrid_ops as ops

@@ -241,10 +241,15 @@ __global__ __launch_bounds__(64 * W, EXACT && (RT == 1 || W == 8) ? 2 : 1) void 
   }
 }
 
-template <typename T, bool PROMPT>
-__global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, void* const rows) {
+template <typename T>
+__global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s) {
   extern __shared__ float cs[];   // 4, [rot_n / 2][2]
-  latent_prep_token<T, PROMPT>(p, s, rows, blockIdx.x, cs);
+  latent_prep_token<T, false>(p, s, nullptr, blockIdx.x, cs);
+}
+
+__global__ __launch_bounds__(256) void latent_prompt_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, b16* const rows, const int row0, const int min_len) {
+  extern __shared__ float cs[];
+  latent_prompt_prep_token(p, s, rows, row0, min_len, blockIdx.x, cs);
 }
 
 template <typename T, int KT, int RT, int NT, int U, bool EXACT = false>
@@ -305,6 +310,15 @@ int check_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, co
   return VMI_HY_OK;
 }
 
+int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, int min_len, const vmi_hy_step* s, const char* who) {
+  if (!a || !rows || !s || !a->proj || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 || a->heads <= 0 || a->rank_n <= 0 ||
+      a->rank_n > a->rank || row0 < 0 || row0 >= s->T || min_len < 0 || (min_len > 0 && (!a->q || !s->ctx || !s->q_len)))
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->dim, a->rank, a->rot_n, a->dtype) || (a->ldp & 7) || (((uintptr_t)a->proj | (uintptr_t)rows | (uintptr_t)a->cache) & 15))
+    return fail(VMI_HY_E_SHAPE, who, "needs sizes that vmi_hy_latent_prompt is built for, rows aligned to 16 bytes");
+  return VMI_HY_OK;
+}
+
 }  // namespace vmi_hybrid
 
 using namespace vmi_hybrid;
@@ -319,23 +333,26 @@ int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, v
   hipStream_t st = static_cast<hipStream_t>(stream);
   const size_t lds = latent_prep_lds(a->rot_n);
   if (a->dtype == VMI_HY_BF16)
-    hipLaunchKernelGGL((latent_prep_kernel<b16, false>), dim3(s->T), dim3(256), lds, st, *a, *s, nullptr);
+    hipLaunchKernelGGL(latent_prep_kernel<b16>, dim3(s->T), dim3(256), lds, st, *a, *s);
   else
-    hipLaunchKernelGGL((latent_prep_kernel<float, false>), dim3(s->T), dim3(256), lds, st, *a, *s, nullptr);
+    hipLaunchKernelGGL(latent_prep_kernel<float>, dim3(s->T), dim3(256), lds, st, *a, *s);
+  return launched(who);
+}
+
+static int prompt_prep(const char* who, const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
+  if (int rc = check_latent_prompt_prep(a, rows, row0, min_len, s, who)) return rc;
+  DeviceScope dev(a->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  hipLaunchKernelGGL(latent_prompt_prep_kernel, dim3(s->T), dim3(256), latent_prep_lds(a->rot_n), static_cast<hipStream_t>(stream), *a, *s, static_cast<b16*>(rows), row0, min_len);
   return launched(who);
 }
 
 int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream) {
-  static const char* who = "vmi_hy_latent_prompt_prep";
-  if (!a || !rows || !s || !a->proj || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 ||
-      a->heads <= 0 || a->rank_n <= 0 || a->rank_n > a->rank)
-    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
-  if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->dim, a->rank, a->rot_n, a->dtype) || (a->ldp & 7) || (((uintptr_t)a->proj | (uintptr_t)rows | (uintptr_t)a->cache) & 15))
-    return fail(VMI_HY_E_SHAPE, who, "needs sizes that vmi_hy_latent_prompt is built for, rows aligned to 16 bytes");
-  DeviceScope dev(a->device);
-  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  hipLaunchKernelGGL((latent_prep_kernel<b16, true>), dim3(s->T), dim3(256), latent_prep_lds(a->rot_n), static_cast<hipStream_t>(stream), *a, *s, rows);
-  return launched(who);
+  return prompt_prep("vmi_hy_latent_prompt_prep", a, rows, 0, 0, s, stream);
+}
+
+int vmi_hy_latent_prompt_tiles_prep(const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
+  return prompt_prep("vmi_hy_latent_prompt_tiles_prep", a, rows, row0, min_len, s, stream);
 }
 
 int32_t vmi_hy_latent_row_tiles(int32_t row_dim, int32_t want, int32_t dtype) { return row_tiles_for(row_dim, want, dtype); }

@@ -1,5 +1,5 @@
-// What a token's latent attention needs between its projections and its queries (include/vmi_hybrid.h: vmi_hy_latent_prep), for the kernel of that name and for the one that has
-// the product beside it (vmi_hy_latent_in).
+// What a token's latent attention needs between its projections and its queries (include/vmi_hybrid.h: vmi_hy_latent_prep), for the kernels of prompts and of that name and for the
+// one that has a product beside it (vmi_hy_latent_in).
 #pragma once
 #include "hybrid_common.hpp"
 
@@ -97,5 +97,16 @@ __device__ __forceinline__ void latent_prep_token(const vmi_hy_latent_prep_args&
     }
   }
 }
+
+// Entries without a past of min_len tokens on (0: every entry) for latent_prompt_kernel, `rows` beginning at token row0, the others as they are without it
+__device__ __forceinline__ void latent_prompt_prep_token(const vmi_hy_latent_prep_args& p, const vmi_hy_step& s, b16* const rows, const int row0, const int min_len, const int t,
+                                                         float* const lds) {
+  const int e = s.tok_seq[t];
+  if (e < 0) return;
+  if (min_len == 0 || (s.ctx[e] == 0 && s.q_len[e] >= min_len)) latent_prep_token<b16, true>(p, s, rows - (int64_t)row0 * (p.rank + p.rot), t, lds);   // (workgroup-uniform)
+  else latent_prep_token<b16, false>(p, s, nullptr, t, lds);
+}
+
+int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, int min_len, const vmi_hy_step* s, const char* who);
 
 }  // namespace vmi_hybrid

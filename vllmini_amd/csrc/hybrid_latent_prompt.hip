@@ -1,5 +1,5 @@
-// Latent attention of whole prompts (include/vmi_hybrid.h: vmi_hy_latent_prompt): where no sequence of a step has a past, its keys and values are the step's own rows, and a head's
-// 128 + 64 columns of key and 128 of value, made for all tokens by one product, are a third of the 576 + 512 that the latent stands for.  csrc/hybrid_latent.hip walks
+// Latent attention of whole prompts (include/vmi_hybrid.h: vmi_hy_latent_prompt): where an entry has no past, its keys and values are the step's own rows, and a head's
+// 128 + 64 columns of key and 128 of value, made for all its tokens by one product, are a third of the 576 + 512 that the latent stands for.  csrc/hybrid_latent.hip walks
 // the latents, as it must where they come from pages.
 //
 // A workgroup takes 64 query positions of one head and walks the keys up to its last position in tiles of 64, each through LDS once (requested one tile ahead into registers, two
@@ -11,6 +11,10 @@
 // Bound by the vector unit's share of the softmax and the chain of a tile (1.4 us).  Attention, us, the latents walked -> here, rank 512: 16 heads, 4 prompts of up to 1024 tokens
 // 117 -> 39, 1 of 500 28 + 12 (its splits added up) -> 16, 16 of up to 200 33 -> 15; 8 heads, 1 of 60 14.6 -> 5.8, 35 of up to 21 14.4 -> 5.7, 1 of 1024 45 + 12 -> 26; and one product of the latents
 // with both up-projections stands for two by heads, of the same work (16 heads, 2773 rows 27 + 19 us).
+// All kernels of a layer between its norms, latents / here, us, prompts only; 16 heads, dim + rot, rank, 1 x 60, 1 x 200, 16 x up to 200, 4 x up to 1024, 1 x 1024: 128 + 64, 512 52 / 44, 70 / 54, 124 / 92, 243 / 137, 153 / 90;
+// 128 + 64, 64 46 / 43, 58 / 50, 94 / 88, 164 / 126, 110 / 87; 128 + 32, 64 45 / 42, 58 / 50, 93 / 86, 160 / 120, 106 / 86; 64 + 64, 64 44 / 39, 55 / 44, 86 / 76, 153 / 105, 105 / 75; 64 + 32, 64 44 / 39, 55 / 42, 84 / 72, 145 / 95,
+// 103 / 70; so also where a latent row is no longer than a head's columns, as each of 16 ranks and heads measured is, and from prompts of two tokens on: rank 512, 1 x 2 35.2 / 33.7, 1 x 8 42 / 35, 1 x 24 45 / 36, 6 x up to 20 64 / 53.
+// Beside entries with a past, which keep the latents and their launches: 64 of those behind 1000 tokens and 1 x 100 111 / 101; 12 behind 300 and 1 x 8, 48, 100, 500 51 / 57, 64 / 68, 72 / 76, 111 / 110.
 // Off 64 bits by as much, latents / here, eight draws each: 8 heads, 60 rows 0.00346 / 0.00350, 300 + 200 + 100 0.00355 / 0.00357, 600 0.00364 / 0.00363; 16 heads, 1024 0.00362 / 0.00360.
 #include "hybrid_softmax.hpp"
 
@@ -21,26 +25,28 @@ constexpr int PQ = 64;   // queries of a workgroup, keys of a tile
 struct LatentPrompt {
   const b16 *proj, *kv, *rows, *gate;
   b16* out;
+  const int* tiles;   // [..][2]: entry, first position; NULL: every entry's places, the last of `places` first
   int64_t ldp, ldkv, ldr, ldg, ldo;
-  int heads, rank, max_len;
+  int heads, rank, row0, places, tile0;   // kv and rows begin at token row0, a launch at tile tile0
   float scale;
 };
 
 // DN + DR columns of a key, the last DR shared by the heads; VD of a value
 template <int DN, int DR, int VD>
-__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPrompt p, const vmi_hy_step s, const int places, const int first) {
+__global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPrompt p, const vmi_hy_step s) {
   constexpr int DK = DN + DR, LDK = DK + 8, LDV = VD + 8, NK = DK / 32, NT = VD / 16;
   constexpr int UN = PQ * DN / 2048, UR = PQ * DR / 2048, UV = PQ * VD / 2048;   // units of eight columns a thread
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   b16* ks = reinterpret_cast<b16*>(smem);   // [64][LDK]
   b16* vs = ks + PQ * LDK;                  // [64][LDV]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int H = p.heads, tile = first + (int)blockIdx.x / H, h = (int)blockIdx.x % H, at = tile / s.B, e = tile - at * s.B;
-  const int qs = s.q_start[e], len = s.q_len[e], q0 = (places - 1 - at) * PQ;
+  const int group = blockIdx.x / p.heads, h = blockIdx.x - group * p.heads, tile = p.tile0 + group, place = tile / s.B;
+  const int e = p.tiles ? p.tiles[2 * tile] : tile - place * s.B, q0 = p.tiles ? p.tiles[2 * tile + 1] : (p.places - 1 - place) * PQ;
+  const int qs = s.q_start[e], len = s.q_len[e];
   if (q0 >= len) return;
   const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
-  const b16* kv = p.kv + (int64_t)qs * p.ldkv + h * (DN + VD);
-  const b16* shared = p.rows + (int64_t)qs * p.ldr + p.rank;
+  const b16* kv = p.kv + (int64_t)(qs - p.row0) * p.ldkv + h * (DN + VD);
+  const b16* shared = p.rows + (int64_t)(qs - p.row0) * p.ldr + p.rank;
   const b16* qrow = p.proj + (int64_t)qs * p.ldp + h * DK;
 
   b16x8 kn[UN], kr[UR], vr[UV];
@@ -155,16 +161,13 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPromp
 }
 
 template <int DN, int DR>
-static int launch_prompt(const LatentPrompt& p, const vmi_hy_step& s, hipStream_t st) {
+static int launch_prompt(LatentPrompt p, int n_tiles, const vmi_hy_step& s, hipStream_t st) {
   auto* fn = latent_prompt_kernel<DN, DR, DN>;
   constexpr size_t lds = (size_t)PQ * (DN + DR + 8 + DN + 8) * 2;
   if (int rc = allow_lds(fn, lds, "vmi_hy_latent_prompt")) return rc;
-  const int places = (p.max_len + PQ - 1) / PQ;
-  const int64_t tiles = (int64_t)places * s.B;
-  if (tiles > INT32_MAX || p.heads > 65535) return fail(VMI_HY_E_SHAPE, "vmi_hy_latent_prompt", "too many heads, or entries and positions");
-  const int n = (int)tiles, most = ((1 << 24) - 1) / p.heads;   // (a launch is of fewer than 2^32 work items)
-  for (int first = 0; first < n; first += std::min(most, n - first)) {
-    hipLaunchKernelGGL(fn, dim3((uint32_t)(p.heads * std::min(most, n - first))), dim3(256), lds, st, p, s, places, first);
+  const int most = ((1 << 24) - 1) / p.heads;   // (a launch is of fewer than 2^32 work items)
+  for (p.tile0 = 0; p.tile0 < n_tiles; p.tile0 += std::min(most, n_tiles - p.tile0)) {
+    hipLaunchKernelGGL(fn, dim3((uint32_t)(p.heads * std::min(most, n_tiles - p.tile0))), dim3(256), lds, st, p, s);
     if (int rc = launched("vmi_hy_latent_prompt")) return rc;
   }
   return VMI_HY_OK;
@@ -180,10 +183,11 @@ int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_
   return dtype == VMI_HY_BF16 && (dim == 64 || dim == 128) && vdim == dim && (rot == 32 || rot == 64) && rank > 0 && (rank & 63) == 0 && rot_n > 0 && (rot_n & 15) == 0 && rot_n <= rot;
 }
 
-int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads, int32_t dim,
-                         int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s, void* stream) {
-  static const char* who = "vmi_hy_latent_prompt";
-  if (!proj || !kv || !rows || !gate || !out || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || heads <= 0 || max_len <= 0 || !(scale > 0.f))
+static int run_prompt(const char* who, const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, int32_t row0, const void* gate, int64_t ldg, void* out, int64_t ldo,
+                      const int32_t* tiles, int64_t n_tiles, int32_t places, int32_t heads, int32_t dim, int32_t rot, int32_t vdim, int32_t rank, float scale, int32_t dtype, int32_t device,
+                      const vmi_hy_step* s, void* stream) {
+  if (!proj || !kv || !rows || !gate || !out || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || row0 < 0 || row0 >= s->T || n_tiles <= 0 || n_tiles > INT32_MAX ||
+      heads <= 0 || heads > 65535 || !(scale > 0.f))
     return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
   if (!vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, 16, dtype) || ((ldp | ldkv) & 7) || (ldo & 3) || (((uintptr_t)proj | (uintptr_t)kv | (uintptr_t)rows) & 15) || ((uintptr_t)out & 7))
     return fail(VMI_HY_E_SHAPE, who, "built for bfloat16 heads of 64 or 128 beside 32 or 64 rotated columns, rows aligned to 16 bytes");
@@ -191,9 +195,24 @@ int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t 
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto rows_of = [](const void* p) { return static_cast<const b16*>(p); };
-  const LatentPrompt p{rows_of(proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), ldp, ldkv, rank + rot, ldg, ldo, heads, rank, max_len, scale};
-  if (dim == 128) return rot == 64 ? launch_prompt<128, 64>(p, *s, st) : launch_prompt<128, 32>(p, *s, st);
-  return rot == 64 ? launch_prompt<64, 64>(p, *s, st) : launch_prompt<64, 32>(p, *s, st);
+  const LatentPrompt p{rows_of(proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), tiles, ldp, ldkv, rank + rot, ldg, ldo, heads, rank, row0, places, 0, scale};
+  const int n = (int)n_tiles;
+  if (dim == 128) return rot == 64 ? launch_prompt<128, 64>(p, n, *s, st) : launch_prompt<128, 32>(p, n, *s, st);
+  return rot == 64 ? launch_prompt<64, 64>(p, n, *s, st) : launch_prompt<64, 32>(p, n, *s, st);
+}
+
+int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads, int32_t dim,
+                         int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s, void* stream) {
+  const int32_t places = max_len <= 0 ? 0 : (max_len - 1) / PQ + 1;
+  return run_prompt("vmi_hy_latent_prompt", proj, ldp, kv, ldkv, rows, 0, gate, ldg, out, ldo, nullptr, s ? (int64_t)places * s->B : 0, places, heads, dim, rot, vdim, rank, scale, dtype,
+                    device, s, stream);
+}
+
+int vmi_hy_latent_prompt_tiles(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, int32_t row0, const void* gate, int64_t ldg, void* out, int64_t ldo,
+                               const int32_t* tiles, int32_t n_tiles, int32_t heads, int32_t dim, int32_t rot, int32_t vdim, int32_t rank, float scale, int32_t dtype, int32_t device,
+                               const vmi_hy_step* s, void* stream) {
+  return run_prompt("vmi_hy_latent_prompt_tiles", proj, ldp, kv, ldkv, rows, row0, gate, ldg, out, ldo, tiles, tiles ? n_tiles : 0, 0, heads, dim, rot, vdim, rank, scale, dtype, device, s,
+                    stream);
 }
 
 }  // extern "C"

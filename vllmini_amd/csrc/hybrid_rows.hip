@@ -168,6 +168,14 @@ struct LatentPrep {
   vmi_hy_latent_prep_args a;
   __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char* smem) const { latent_prep_token<b16, false>(a, s, nullptr, t, reinterpret_cast<float*>(smem)); }
 };
+struct LatentPromptPrep {
+  vmi_hy_latent_prep_args a;
+  b16* rows;
+  int row0, min_len;
+  __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char* smem) const {
+    latent_prompt_prep_token(a, s, rows, row0, min_len, t, reinterpret_cast<float*>(smem));
+  }
+};
 struct KvPrep {
   vmi_hy_kv_prep_args a;
   __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char*) const { kv_prep_token<b16>(a, s, t); }
@@ -718,6 +726,19 @@ int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args*
   DeviceScope dev(l->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   return launch_beside(*l, LatentPrep{*a}, *s, latent_prep_lds(a->rot_n), who, static_cast<hipStream_t>(stream));
+}
+
+int vmi_hy_latent_prompt_tiles_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_latent_prompt_tiles_in";
+  if (int rc = check_linear(l, who)) return rc;
+  if (int rc = check_latent_prompt_prep(a, rows, row0, min_len, s, who)) return rc;
+  if (a->device != l->device || !beside_fits(*l, *s)) {
+    if (int rc = vmi_hy_linear(l, stream)) return rc;
+    return vmi_hy_latent_prompt_tiles_prep(a, rows, row0, min_len, s, stream);
+  }
+  DeviceScope dev(l->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  return launch_beside(*l, LatentPromptPrep{*a, static_cast<b16*>(rows), row0, min_len}, *s, latent_prep_lds(a->rot_n), who, static_cast<hipStream_t>(stream));
 }
 
 int vmi_hy_kv_prep_in(const vmi_hy_linear_args* l, const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream) {

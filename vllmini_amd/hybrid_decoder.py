@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import dataclasses
 import itertools
-from typing import Dict, List, Optional, Sequence, Union
+from typing import Dict, List, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
@@ -120,20 +120,26 @@ class HybridDecoder:
         put("rows", max(len(rows), 1), rows, 0)
         plans = []
         for kind in self._kinds:
-            rep, longest = kind.rep, int(counts.max())
-            rt = 1 if longest == 1 and kind.one_row_tile(B, max_keys) else kind.row_tiles(longest, self.model.dtype)
-            per = -(-(counts * rep) // (16 * rt))
+            mine, prompts = counts, None      # (the portions of this kind's own tiles, and what of the step is not among them)
+            if kind.prompts and (counts > 1).any():
+                pays = ops.latent_prompt_pays(np.stack([a["ctx"], counts], axis=1))
+                if np.any(pays):
+                    mine, prompts = np.where(pays, 0, counts), self._prompts(sec, f"prompts{len(plans)}", pays, counts, starts)
+            rep, longest, keys = kind.rep, max(int(mine.max()), 1), max_keys if prompts is None else int(((a["ctx"] + mine) * (mine > 0)).max())
+            entries = B if prompts is None else int((mine > 0).sum())
+            rt = 1 if longest == 1 and kind.one_row_tile(entries, keys) else kind.row_tiles(longest, self.model.dtype)
+            per = -(-(mine * rep) // (16 * rt))
             ent = np.repeat(np.arange(b), per)
             first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * 16 * rt
             if b > 1 or len(first) > 1:       # longest first: the tail of the launch is short tiles
-                keys = a["ctx"][ent] + (first + 16 * rt - 1) // rep
-                order = np.argsort(-(keys % kind.chunk if kind.chunk else keys), kind="stable")
+                seen = a["ctx"][ent] + (first + 16 * rt - 1) // rep
+                order = np.argsort(-(seen % kind.chunk if kind.chunk else seen), kind="stable")
                 ent, first = ent[order], first[order]
             nt = len(ent) + (B - b) * (-(-rep // (16 * rt)))
             t = np.full((nt, 2), -1, dtype=np.int32)
             t[: len(ent), 0], t[: len(ent), 1] = ent, first
             sec[f"tiles{len(plans)}"] = t.reshape(-1)
-            plans.append((rt, self._split_of(nt, rt, kind, max_keys, T), nt))
+            plans.append((rt, self._split_of(nt, rt, kind, keys, T), nt, prompts))
         if (counts > 1).any():                # runs of rows for the linear-attention layers
             per = -(-counts // ops.CHUNK_ROWS)
             at = np.cumsum(per) - per
@@ -145,6 +151,18 @@ class HybridDecoder:
             offs[name] = (total, len(v))
             total += (len(v) + 3) // 4 * 4
         return sec, offs, total, plans
+
+    @staticmethod
+    def _prompts(sec: Dict[str, np.ndarray], name: str, pays: np.ndarray, counts: np.ndarray, starts: np.ndarray) -> Tuple[int, int, int, int]:
+        """The tiles of the portions that go through ops.latent_prompt, the longest walks first, and the tokens between which they and the others lie."""
+        own = np.flatnonzero(pays)
+        per = -(-counts[own] // ops.PROMPT_TILE)
+        first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * ops.PROMPT_TILE
+        order = np.argsort(-first, kind="stable")
+        sec[name] = np.stack([np.repeat(own, per)[order], first[order]], axis=1).astype(np.int32).reshape(-1)
+        rest = np.flatnonzero(~pays & (counts > 0))
+        return (*(int(x) for x in (starts[own[0]], starts[own[-1]] + counts[own[-1]])),
+                *((int(starts[rest[0]]), int(starts[rest[-1]] + counts[rest[-1]])) if len(rest) else (0, 0)))
 
     def _staged(self, sec, offs, total: int) -> PinnedBuffer:
         """The sections in pinned memory (a ring of four buffers)."""
@@ -175,7 +193,8 @@ class HybridDecoder:
         v["table"] = v["table"].view(B, table_ld)
         if "chunks" in v:
             v["chunks"] = v["chunks"].view(-1, 2)
-        plan = {kind: AttentionPlan(v[f"tiles{i}"].view(nt, 2), rt, sp) for i, (kind, (rt, sp, nt)) in enumerate(zip(self._kinds, plans))}
+        plan = {kind: AttentionPlan(v[f"tiles{i}"].view(nt, 2), rt, sp, None if at is None else ops.PromptTiles(v[f"prompts{i}"].view(-1, 2), *at))
+                for i, (kind, (rt, sp, nt, at)) in enumerate(zip(self._kinds, plans))}
         return v, plan
 
     # ---- the forward pass --------------------------------------------------------------------------------------------------
@@ -260,8 +279,7 @@ class HybridDecoder:
         if "ids" in v:
             ids = v.pop("ids").view(torch.int64)
         spans = bool((starts // ops.ROW_TILE != (starts + counts - 1) // ops.ROW_TILE).any())
-        layout = ops.StepLayout(v, T, B, self.pool.block_size, bool((counts == 1).all()), spans, int(counts.max()), keys,
-                                fresh=not a["ctx"].any())
+        layout = ops.StepLayout(v, T, B, self.pool.block_size, bool((counts == 1).all()), spans, int(counts.max()), keys)
         return self._forward(ids, layout, plan, v["rows"] if len(rows) else None)
 
     # ---- what the scheduler calls -------------------------------------------------------------------------------------------

@@ -23,7 +23,7 @@ where one stands behind them, or to the vendor library where that is ahead (prod
 from __future__ import annotations
 
 import math
-from typing import Dict, List, NamedTuple, Optional, Sequence, Tuple
+from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -80,6 +80,7 @@ class QueryTiling(NamedTuple):
     width: int
     chunk: int = 0
     sizes: Tuple[int, ...] = ()
+    prompts: bool = False      # portions that ops.latent_prompt_pays names go through ops.latent_prompt
 
     def row_tiles(self, longest: int, dtype: torch.dtype) -> int:
         """Of 16 rows each, a workgroup's: as many as an entry's `longest` portion fills."""
@@ -105,6 +106,7 @@ class AttentionPlan(NamedTuple):
     tiles: torch.Tensor
     row_tiles: int
     splits: int
+    prompts: Optional[ops.PromptTiles] = None      # entries that are not among `tiles`
 
 
 Plans = Dict[QueryTiling, AttentionPlan]
@@ -233,22 +235,30 @@ class LatentAttention:
         return []
 
     def tiling(self) -> Optional[QueryTiling]:
-        return QueryTiling("latent", self.heads, 1, self.row, sizes=(self.row,))
+        return QueryTiling("latent", self.heads, 1, self.row, sizes=(self.row,), prompts=self.w_kv is not None)
 
     def run(self, res: Residual, step: StepLayout, plans: Plans, held: Sequence[torch.Tensor]) -> None:
         H, D, plan, (cache,) = self.heads, self.row, plans[self.tiling()], held
         proj = res.branch_in(self.norm, self.w_in, step)
-        # (below DENSE_MIN_TOKENS the projections run in the few-row kernels, and there the latents stay: 1 prompt of 60, 8 heads, a whole step's kernels 501 -> 449 us, 6 of up to 20 558 -> 501)
-        if self.w_kv is not None and step.fresh and step.T >= DENSE_MIN_TOKENS and ops.latent_prompt_pays(step):
-            res.branch_out(ops.latent_prompt(proj, self.w_kv, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, vdim=self.vdim, rank=self.rank,
-                                             rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps, scale=self.scale, gate=proj[:, self.gate_at:]), self.w_o, step)
-            return
-        q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
-        ops.latent_in(proj, self.w_uk, q, cache, step, norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank,
-                      rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps)
-        lat = ops.latent_attention(q, cache, step, plan.tiles, heads=H, rank=self.rank, rot=self.rot, scale=self.scale,
-                                   row_tiles=plan.row_tiles, splits=plan.splits)
-        o = ops.linear(lat, self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=proj[:, self.gate_at:])
+        sizes = dict(norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank, rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps)
+        gate = proj[:, self.gate_at:]
+
+        def attention(q: torch.Tensor) -> torch.Tensor:
+            return ops.latent_attention(q, cache, step, plan.tiles, heads=H, rank=self.rank, rot=self.rot, scale=self.scale, row_tiles=plan.row_tiles, splits=plan.splits)
+
+        def past(out: torch.Tensor, latent_in: Callable[[slice, MatrixTiles, torch.Tensor], None]) -> None:
+            """The entries that have one, beside prompts (whose rows among them hold nothing: every product is by rows)."""
+            at = slice(plan.prompts.past_first, plan.prompts.past_last)
+            q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
+            latent_in(at, self.w_uk, q)
+            ops.linear(attention(q)[at], self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=gate[at], out=out[at])
+
+        if plan.prompts is not None:
+            o = ops.latent_prompt(proj, self.w_kv, cache, step, vdim=self.vdim, scale=self.scale, gate=gate, prompts=plan.prompts, others=past if plan.prompts.past_last else None, **sizes)
+        else:
+            q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
+            ops.latent_in(proj, self.w_uk, q, cache, step, **sizes)
+            o = ops.linear(attention(q), self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=gate)
         res.branch_out(o, self.w_o, step)
 
 

@@ -22,8 +22,9 @@ import ctypes
 import functools
 import os
 import threading
-from typing import NamedTuple, Optional, Sequence, Tuple
+from typing import Callable, NamedTuple, Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from . import build as _build
@@ -100,8 +101,11 @@ SIGNATURES = {
     "vmi_hy_kv_prep_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(KvPrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt_tiles_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_latent_prompt": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt_tiles_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), _vp, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompt_tiles": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _vp, _i64, _vp, _i64, _vp, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_row_tiles": (_i32, [_i32, _i32, _i32]),
     "vmi_hy_latent_attention": (ctypes.c_int, [ctypes.POINTER(AttentionArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hybrid_last_error": (ctypes.c_char_p, []),
@@ -464,7 +468,7 @@ ROW_TILE = 64      # rows of a tile of the recurrence's kernel
 
 class StepLayout:
     """The tokens of a step on the device: `fields` maps the names of vmi_hy_step to int32 tensors; `single`: every portion is one
-    token; `spans`: some portion crosses a row tile; `fresh`: no entry has a past, and every row is an entry's."""
+    token; `spans`: some portion crosses a row tile; `fresh`: no entry has a past, and every row is an entry's (which latent_prompt without a list of tiles asks for)."""
 
     def __init__(self, fields: dict, T: int, B: int, page_size: int, single: bool, spans: bool, max_len: int, max_keys: int, fresh: bool = False):
         for name in ("tok_seq", "tok_pos", "tok_slot"):
@@ -573,29 +577,64 @@ def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int, rot_n: int, dty
     return dtype == torch.bfloat16 and bool(load().vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, rot_n, DTYPES[dtype]))
 
 
-def latent_prompt_pays(step: StepLayout) -> bool:
-    """Whether a launch of as many places as the longest entry has, for every entry, is not mostly empty ones (each some ns; 48 prompts of up to 80 tokens 27.7 us over the latents, 9.5 so)."""
-    return -(-step.max_len // 64) * step.B <= 1024 + step.T
+PROMPT_TILE, PROMPT_MIN_TOKENS = 64, 2      # positions of a tile of latent_prompt's kernel; the shortest portion that goes there
+
+
+def latent_prompt_pays(portions: np.ndarray) -> np.ndarray:
+    """Which of a step's portions, (ctx, tokens) each, go through latent_prompt: by the portion alone, whatever shares its step, so that a prompt's keys and values are rounded at the same
+    places beside others as by itself (vmi_hy_latent_prompt_tiles_in has the same rule).  Ahead of the latents from two tokens on (csrc/hybrid_latent_prompt.hip); one is a decoding step's."""
+    return (portions[:, 0] == 0) & (portions[:, 1] >= PROMPT_MIN_TOKENS)
+
+
+class PromptTiles(NamedTuple):
+    """The entries of a step that go through latent_prompt: their tiles of positions (int32 [n, 2]: entry, first position), and the tokens, from .. to, that all of them lie among, and
+    all of the others (to = 0: there are no others)."""
+    tiles: torch.Tensor
+    first: int
+    last: int
+    past_first: int = 0
+    past_last: int = 0
 
 
 def latent_prompt(proj: torch.Tensor, w_kv: MatrixTiles, cache: torch.Tensor, step: StepLayout, *, norm_w: torch.Tensor, freq: torch.Tensor, heads: int, dim: int, rot: int, vdim: int,
-                  rank: int, rot_n: int, rank_n: int, eps: float, scale: float, gate: torch.Tensor) -> torch.Tensor:
-    """Latent attention of a `fresh` step, gates included: proj (whose query parts are rotated in place) -> [T, heads * vdim], the cache's rows written.
-    w_kv: the up-projections, per head [dim | vdim] rows of rank."""
+                  rank: int, rot_n: int, rank_n: int, eps: float, scale: float, gate: torch.Tensor, prompts: Optional[PromptTiles] = None,
+                  others: Optional[Callable[[torch.Tensor, Callable[[slice, MatrixTiles, torch.Tensor], None]], None]] = None) -> torch.Tensor:
+    """Latent attention of entries without a past over their keys and values, gates included: proj (whose query parts are rotated in place) -> [T, heads * vdim], the cache's rows of
+    all entries written.  w_kv: the up-projections, per head [dim | vdim] rows of rank.  prompts: which entries (None: all of them, a `fresh` step); others(out, latent_in):
+    what the rest takes, beginning with latent_in(tokens, w_uk, q), its result into its rows of out (and whatever it likes into the prompts')."""
     device, stream = _on(proj)
     T, D = step.T, rank + rot
-    _need(step.fresh and proj.shape[0] == T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and cache.dtype == proj.dtype and cache.shape[-1] == D
+    _need((step.fresh or prompts is not None) and proj.shape[0] == T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and cache.dtype == proj.dtype and cache.shape[-1] == D
           and cache.is_contiguous() and norm_w.numel() == rank and norm_w.dtype == torch.float32 and freq.dtype == torch.float64 and freq.numel() == rot_n // 2
           and w_kv.groups == 1 and (w_kv.N, w_kv.K) == (heads * (dim + vdim), rank) and gate.dtype == proj.dtype and gate.shape[0] == T and gate.shape[1] >= heads
           and gate.stride(1) == 1, "hybrid_ops.latent_prompt: operand sizes")
-    rows = torch.empty((T, D), dtype=proj.dtype, device=proj.device)
+    tiles, first, last, mixed = None, 0, T, False
+    if prompts is not None:
+        tiles, first, last, mixed = prompts.tiles, prompts.first, prompts.last, prompts.past_last > 0
+        _need(tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.dim() == 2 and tiles.shape[1] == 2 and 0 <= first < last <= T, "hybrid_ops.latent_prompt: prompts")
+    _need(mixed == (others is not None), "hybrid_ops.latent_prompt: entries beside the prompts, and what they take")
+    rows = torch.empty((last - first, D), dtype=proj.dtype, device=proj.device)
+    out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
     a = PrepArgs(proj=proj.data_ptr(), cache=cache.data_ptr(), norm_w=norm_w.data_ptr(), freq=freq.data_ptr(), ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank,
                  rot_n=rot_n, rank_n=rank_n, eps=eps, dtype=DTYPES[proj.dtype], device=device)
-    _check(load().vmi_hy_latent_prompt_prep(ctypes.byref(a), rows.data_ptr(), step.ref, stream))
+
+    if others is None:
+        _check(load().vmi_hy_latent_prompt_tiles_prep(ctypes.byref(a), rows.data_ptr(), first, 0, step.ref, stream))
+    else:
+        def latent_in(at: slice, w_uk: MatrixTiles, q: torch.Tensor) -> None:
+            _need(q.shape == (T, heads * D) and q.is_contiguous() and q.dtype == proj.dtype and (w_uk.groups, w_uk.N, w_uk.K) == (heads, rank, dim), "hybrid_ops.latent_prompt: q")
+            a.q = q.data_ptr()      # (which entries, latent_prompt_pays has for the host)
+            b = _by_groups(proj[at], w_uk, q[at], dim + rot, D, device)
+            _check(load().vmi_hy_latent_prompt_tiles_in(ctypes.byref(b), ctypes.byref(a), rows.data_ptr(), first, PROMPT_MIN_TOKENS, step.ref, stream))
+
+        others(out, latent_in)
     kv = product_tiles(rows[:, :rank], w_kv)
-    out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
-    _check(load().vmi_hy_latent_prompt(proj.data_ptr(), proj.stride(0), kv.data_ptr(), kv.stride(0), rows.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0), heads,
-                                       dim, rot, vdim, rank, step.max_len, scale, DTYPES[proj.dtype], device, step.ref, stream))
+    at = (proj.data_ptr(), proj.stride(0), kv.data_ptr(), kv.stride(0), rows.data_ptr())
+    to, sizes = (gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0)), (heads, dim, rot, vdim, rank)
+    if tiles is None:
+        _check(load().vmi_hy_latent_prompt(*at, *to, *sizes, step.max_len, scale, DTYPES[proj.dtype], device, step.ref, stream))
+    else:
+        _check(load().vmi_hy_latent_prompt_tiles(*at, first, *to, tiles.data_ptr(), tiles.shape[0], *sizes, scale, DTYPES[proj.dtype], device, step.ref, stream))
     return out
 
 
