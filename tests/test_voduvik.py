@@ -360,6 +360,17 @@ def test_products_alone_go_to_tiles_but_where_the_library_is_ahead():
         assert pay(M, N, K), (M, N, K)
 
 
+def test_whole_columns_over_a_long_k_go_to_tiles_by_what_is_left_of_the_librarys_turns():
+    """Both sides as measured, 2 % and more apart: how full the library's tiles and ours leave the chip, not how many results there are."""
+    from vllmini_amd import hybrid_ops as h
+
+    pay = lambda M, N, K: h.load().vmi_hy_product_tiles_pay(M, N, K, K, h.DTYPES[torch.bfloat16])      # noqa: E731
+    for M, N, K in ((3417, 2048, 3584), (1751, 5120, 3584), (2604, 3072, 4096), (3906, 2048, 4608), (3662, 2048, 5120), (3173, 2048, 6144), (3568, 2048, 6144), (3906, 2048, 6144), (1464, 5120, 6144), (1057, 6144, 5120)):
+        assert not pay(M, N, K), (M, N, K)
+    for M, N, K in ((2744, 2048, 3584), (1953, 3072, 4096), (2744, 2048, 5120), (4379, 2048, 4608), (1660, 5120, 4608), (1829, 3072, 5120), (914, 6144, 5120), (2744, 2048, 6144), (4379, 2048, 6144), (3125, 2560, 3072)):
+        assert pay(M, N, K), (M, N, K)
+
+
 def test_groups_go_to_tiles_but_where_all_run_at_once_over_a_short_k():
     """The rule against both sides as measured."""
     from vllmini_amd import hybrid_ops as h

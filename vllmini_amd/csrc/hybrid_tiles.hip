@@ -141,22 +141,26 @@ int launch_group_tiles(const vmi_hy_linear_args& p, hipStream_t st) {
 // order of a sum).  Measured in bfloat16, weights that leave the last cache between two products from K 2048 on and others that stay.
 //
 // Alone, 5300 pairs of 48 to 9000 rows, K 256 to 12 288, N 256 to 16 384: ours / library's in the mean, from 5.6 million results on (below, nearly all of the library's time is its call:
-// 19 us of host) and whole tiles of 256 columns: K 1024 to 2047 0.88 (8 of 207 more than 5 per cent behind), to 4095 0.96 (52 of 239), to 6144 1.00 (30 of 104), beyond 1.07; other columns
-// 0.74, 0.85, 0.96 and 0.99.  So not past K 6144 from 5.6 million results on, up to there whole columns up to 9 million (N 3072, K 4608, 4100 rows 90 / 109) and only where the tiles' own costs promise 1020
-// TFLOP/s (N 2048, K 6144: 2773 rows 69 / 60, which one round of tiles holds; 3250 73 / 85), and below K 4096 whole columns up to 9 million (N 4096, K 2048: 2400 41 / 42, level from there on), below 2048 up to 15.
-// Not where few of the smallest tiles walk a long K each, which the library shares out (64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4): measured again over 380 pairs of up to 128
-// such tiles, now that results leave as lines, ours / library's in the mean K 3072 0.93, 3584 and 4096 up to N 2048 0.96 (N 3072 1.17 and 1.02), 4608 and 5120 0.99 and 1.00 (1.11), 6144 1.15, 8192
+// 19 us of host) and whole tiles of 256 columns: K 1024 to 2047 0.88 (8 of 207 more than 5 per cent behind), beyond 6144 1.07; other columns 0.74, 0.85 to K 4095, 0.96 to 6144 and 0.99 beyond.
+// So not past K 6144 from 5.6 million results on, and whole columns up to 9 million, below K 2048 up to 15.  Whole columns between 5.6 and 9 million, K 2048 to 6144, 648 pairs by a grid and 596 by chance, ours / library's:
+//   K up to 3072     always: 0.95 (20 of 376 more than 5 per cent behind, 1.17 at most, at sizes among others that are as far ahead)
+//   beyond           0.99 (178 of 868, 1.23); so where the library's tiles, 256 x 128 as its times have them, leave a quarter of the compute units' turns empty, and the tiles' own costs promise 950 TFLOP/s (past K 4096
+//                    1000), which is 0.92 (4 of 266, 1.10) and leaves 1.02 to the library.  N 2048, K 5120 2744 rows 0.85, 2929 0.92, 3173 to 3906 0.99 to 1.05, 4150 0.94, 4379 0.90; N 6144, K 5120 914 0.84, 1057 1.08, 1383 0.88.
+// Not where few of the smallest tiles walk a long K each, which the library shares out (us, from here on the library's / ours: 64 rows, N 2048, K 6144 14.0 / 16.1; 140 24.4 / 22.4): measured again over 380 pairs of up to 128
+// such tiles, now that results leave as lines, ours over the library's in the mean K 3072 0.93, 3584 and 4096 up to N 2048 0.96 (N 3072 1.17 and 1.02), 4608 and 5120 0.99 and 1.00 (1.11), 6144 1.15, 8192
 // 1.31; and a call of the library's is 12 us more of host, which is what a short prompt waits for (62 rows, N 1024, K 3072 10.4 / 8.6 us, host 20 / 8).  Nor where tiles of 64 x 64 are just more than
 // the chip has compute units for (300 rows, N 4096, K 8192 46 / 56; 600 rows, N 2048, K 6144 34 / 37), and past K 16 383.
 static bool product_pays(int M, int N, int K) {
   const bool whole = N % 256 == 0;
   const int64_t results = (int64_t)M * N, least = (int64_t)((M + 31) / 32) * ((N + 63) / 64);
-  if (K >= 4096) {
-    if (results >= 5600000 &&
-        (K > 6144 || (whole && (results >= 9000000 || vmi_tiles::tiles_cost(vmi_tiles::tiles_pick(M, N, K), M, N, K, 1) > 2. / 1.02e9 * (double)results * K))))
+  if (results >= 5600000 && K > 6144) return false;
+  if (whole && K >= 1024 && results >= (K >= 2048 ? 9000000 : 15000000)) return false;
+  if (whole && results >= 5600000 && K > 3072) {
+    auto turns = [&](int m, int n) { return ((int64_t)((M + m - 1) / m) * ((N + n - 1) / n) + 255) / 256; };   // of 256 compute units
+    const int64_t least_turns = std::min(turns(256, 128), turns(128, 256));
+    if (4 * results >= 3 * least_turns * 256 * 32768 ||
+        2. * (double)results * K < (K <= 4096 ? .95e9 : 1e9) * vmi_tiles::tiles_cost(vmi_tiles::tiles_pick(M, N, K), M, N, K, 1))
       return false;
-  } else if (whole && K >= 1024 && results >= (K >= 2048 ? 9000000 : 15000000)) {
-    return false;
   }
   const bool shared = K > 4096 || (K > 3072 && N > 2048);   // (up to 4096 and 2048 nothing is to be had from sharing K out)
   if (K >= 3072 && ((shared && least <= 128) || (whole && N >= 2048 && results >= 1050000 && results < 2400000))) return false;
