@@ -508,7 +508,12 @@ def test_graph_replay_two_streams_and_two_host_threads():
     (128, 32, 8, [1300] + [i * 9 for i in range(11)], 1300, "d128_gq2_h1_w8_u2_nt1"), (128, 32, 8, [1200] + [i * 7 for i in range(31)], 1200, "d128_gq4_h1_w16_u1_nt1"),
     (128, 64, 8, [250, 3], 250, "d128_h1_w8_u2_nt0"), (64, 16, 4, [20] * 3, 20, "d64_h1_w4_u2_nt0"), (64, 16, 4, [900, 5, 0], 900, "d64_h1_w16_u2_nt0"),
     (64, 16, 4, [1699, 64, 65], 1699, "d64_h1_w16_u2_nt0"), (64, 16, 4, [640] + [i * 5 for i in range(47)], 640, "d64_gq4_h1_w8_u2_nt1"),
-    (64, 16, 4, [1000] + [i * 11 for i in range(40)], 1000, "d64_gq4_h1_w16_u2_nt1")])
+    (64, 16, 4, [1000] + [i * 11 for i in range(40)], 1000, "d64_gq4_h1_w16_u2_nt1"),
+    # two heads an item, as many as the line lets; one more; and more tokens
+    (128, 32, 8, [720] + [17] * 15, 720, "d128_gq2_h1_w8_u2_nt1"), (128, 32, 8, [900] + [i * 13 for i in range(15)], 900, "d128_gq4_h1_w8_u1_nt1"),
+    (128, 32, 8, [1100] + [i * 13 for i in range(15)], 1100, "d128_gq4_h1_w16_u1_nt1"),
+    # 8, 16 and 32 queries a KV head
+    (128, 16, 2, [130, 70], 130, "d128_h1_w8_u2_nt0"), (64, 64, 4, [300, 1], 300, "d64_h1_w8_u2_nt0"), (128, 32, 1, [700, 0, 33], 700, "d128_h1_w16_u1_nt0"), (64, 64, 2, [40] * 3, 40, "d64_h1_w4_u2_nt0")])
 def test_grouped_queries_of_few_sequences(D, H, hkv, lens, room, form):
     """The forms that a launch of few sequences takes over shared key and value heads, on either side of their lines: which one runs, and what it gives against the kernel model, with ALiBi and
     without; a sequence's row is what it is where all the others are empty."""

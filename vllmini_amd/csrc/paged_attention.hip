@@ -476,7 +476,8 @@ static int pick_variant_gqa(int num_seqs, int num_heads, int qpk, int head_size,
 // group too; and up to half of them two heads an item, each tile read twice, twice the vector pipes.  us over 32 / 8 heads of 128 (16 / 4 of 64), contexts equal and U{1 .. longest}:
 //   sixteen waves  24 x 1500 33.2 / 30.5 -> 31.0 / 28.0; 32 x 3000 65.4 / 54.0 -> 64.3 / 47.1; 24 x 4096 76.8 / 69.8 -> 69.9 / 59.8   (48 x 1500 25.5 / 23.8 -> 20.2 / 18.3; 64 x 4096 60.0 / 55.3 ->
 //   48.7 / 37.5).  700 tokens level (4 per cent behind).  Not for more items than compute units, which would go round twice (48 x 4096 137.6 / 82.7 -> 145.4 / 75.4: what
-//   a ragged batch wins, an equal one loses).   two heads  16 x 300 11.6 / 11.2 -> 9.9 / 9.0; 16 x 700 17.6 / 17.0 -> 16.7 / 13.5; 12 x 1400 18 per cent ahead, 16 x 1400 behind; 24 x 700 18.3 / 17.2 -> 24.1 / 15.8
+//   a ragged batch wins, an equal one loses).   two heads, for as many items squared times tokens as both kinds of batch are in the mean ahead, pages from memory: of the better form of four heads 64 x 700 / 1200 / 1600 items
+//   0.87 / 0.93 / 0.92 and 0.83 / 0.88 / 0.86, 96 x 700 / 1200 / 1400 0.94 / 1.02 / 1.10 and 0.86 / 0.92 / 0.96, 128 x 500 / 700 / 900 / 1200 0.99 / 1.05 / 1.15 / 1.18 and 0.86 / 0.90 / 0.96 / 0.96; 24 x 700 18.3 / 17.2 -> 24.1 / 15.8
 //   two blocks, head size 64  48 x 700 14.5 / 13.8 -> 13.0 / 12.4; 32 / 8 heads, 64 x 2000 0.95 of it, 128 x 700 1.14: by items as below
 // More items than twice the compute units, head size 128: four waves (80 x 130 1.43 of it, x 300 1.24, x 700 1.11; level from 1500 on).
 struct GqForm {
@@ -486,7 +487,7 @@ static GqForm pick_gq4(long items, int head_size, int max_seq_len) {
   const long cus = g_cus;
   const int L = max_seq_len;
   if (head_size == 128) {
-    if (2 * items <= cus && L >= 190 && L < 1700 && items * L <= 600 * cus) return {2, 8, 2};
+    if (2 * items <= cus && L >= 190 && L < 1700 && items * items * L <= 186 * cus * cus) return {2, 8, 2};
     if (items <= cus && L >= 1000) return {4, 16, 1};
     return {4, items > 2 * cus && L < 1500 ? 4 : 8, 1};
   }
@@ -911,9 +912,11 @@ static int find_split(int D, int xw, int U, int nt, int f8 = 0, int hpt = 1) {
 // Grouped queries, fp16 pages, few sequences of contexts that one compute unit is done with soon: a workgroup a QUERY head, each reading its KV head's tiles itself (the
 // repeats hit the caches), so that four times the compute units work.  Or 0.  Such a launch takes 5 - 7 us and what its reads take from the caches, heads x tokens; the shared-tile
 // kernel it stands for 7 us and its longest context on one compute unit: the line is where the two meet, fitted to 1350 launches of 20 to 4096 tokens, 1 to 128 sequences, 32 / 8 and
-// 16 / 4 heads (349 inside it: the shared-tile kernels 1.7 times as long in the mean; five sizes up to 10 per cent behind another form of their own).  us, contexts equal: 32 / 8 heads
+// 16 / 4 heads (349 inside it: the shared-tile kernels 1.7 times as long in the mean; again 386, pages in the caches and from memory, 8 / 2 to 64 / 16 heads: 0.58 and 0.62 of the time, seven
+// more than 5 per cent behind, 1.11 at most).  us, contexts equal: 32 / 8 heads
 // of 128 1 x 40 7.9 -> 3.8, 4 x 300 10.7 -> 5.3, 1 x 700 15.8 -> 7.0, 4 x 700 16.7 -> 10.3, 8 x 300 11.3 -> 8.3, 12 x 300 11.4 / 12.5 (outside); 16 / 4 of 64 4 x 700 13.4 -> 5.7, 16 x 700 13.9 -> 9.1,
-// 8 x 1500 15.0 -> 10.8.  Waves a head: the most that still have blocks and compute units to themselves.
+// 8 x 1500 15.0 -> 10.8.  More queries a KV head read its tiles as often from the same caches, and what they leave is slower: over 798 launches of 16 / 2 to 64 / 8, 24 / 2 and 96 / 8, 16 / 1 to
+// 128 / 8, and 32 / 1 and 64 / 2 heads 0.42, 0.57, 0.38 and 0.38 of the time, 1.08 at most (64 / 8 of 128, 1 x 300 20.9 -> 5.4, x 700 34.0 -> 8.5; 32 / 1 4 x 700 35.3 -> 7.8).  Waves a head: the most that still have blocks and compute units to themselves.
 static int pick_per_head(int num_seqs, int num_heads, int qpk, int head_size, int block_size, int max_seq_len) {
   if (qpk % 4 != 0 || block_size != 16 || (head_size != 64 && head_size != 128)) return 0;
   const bool wide = head_size == 128;
