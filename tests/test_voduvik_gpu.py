@@ -694,6 +694,32 @@ def test_portions_that_share_rows_taken_together_with_padding(dtype, width, bloc
 
 
 @pytest.mark.parametrize("dtype", BOTH)
+@pytest.mark.parametrize("width,blocks,taps", [(512, 2, 4), (96, 3, 4), (66, 11, 3)])
+@pytest.mark.parametrize("bad,value", [(0, float("nan")), (1, float("inf")), (3, float("nan")), (3, float("-inf")), (4, None)])
+def test_portions_that_are_no_numbers_leave_the_others_alone(dtype, width, blocks, taps, bad, value):
+    """A NaN or an infinity in one portion's inputs, or (None) in the state it takes up, in front of others in its row tile and across the tile's end: every bit of the others' results, states
+    and tails is as it is without."""
+    counts, ctx = [5, 40, 3, 100, 9, 20], [0, 7, 0, 0, 7, 0]
+    k = _Rglru(width, blocks, taps, dtype, slots=len(counts))
+    g = torch.Generator().manual_seed(width)
+    state, tail = (torch.randn(t.shape, generator=g).to(t.dtype).to(dev()) for t in (k.state, k.tail))
+    yx, at = torch.cat([k.inputs(n, 60 + i)[2] for i, n in enumerate(counts)]), sum(counts[:bad])
+    rest = torch.tensor([i for i in range(len(counts)) if i != bad], device=dev())
+    got = []
+    for poison in (False, True):
+        k.state.copy_(state), k.tail.copy_(tail)
+        rows = yx.clone()
+        if poison and value is None:
+            k.state[bad] = float("nan")
+        elif poison:
+            rows[at + counts[bad] // 3, k.layer.width:] = value
+        out = k.run(rows, layout(counts, ctx, [[0]] * len(counts), 64, pos_slots=False))
+        got.append((torch.cat([o for i, o in enumerate(out.split(counts)) if i != bad]), k.state[rest].clone(), k.tail[rest].clone()))
+        assert poison == (not bool(torch.isfinite(out[at: at + counts[bad]].float()).all()))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and bool(torch.isfinite(got[1][0].float()).all())
+
+
+@pytest.mark.parametrize("dtype", BOTH)
 def test_recurrence_decodes_like_it_prefills_and_skips_padding_rows(dtype):
     from vllmini_amd import hybrid_ops as ops
 

@@ -58,6 +58,20 @@ __device__ __forceinline__ void walk16(f32x4& A, f32x4& B) {
   A = f32x4{a0, a1, a2, a3}, B = f32x4{b0, b1, b2, b3};
 }
 
+// The same where a value is no finite number: a zero of A stops what is in front of it, whatever that is.  first: whether a lane's row opens a portion (A is 0 there); afterwards, whether one of its
+// lanes up to this one does.  Slower by an instruction or three a value, for the rare wave whose portions would else meet.
+template <int D>
+__device__ __forceinline__ void step16(f32x4& A, f32x4& B, int& first) {
+  auto below = [](float old, float v) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, old), __builtin_bit_cast(int, v), 0x110 + D, 0xf, 0xf, false)); };
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float a = below(1.f, A[e]), b = below(0.f, B[e]);
+    B[e] = first ? B[e] : fmaf(A[e], b, B[e]);
+    A[e] = first ? A[e] : A[e] * a;
+  }
+  first |= __builtin_amdgcn_update_dpp(0, first, 0x110 + D, 0xf, 0xf, false);
+}
+
 // convolution of 8 channels for the token of row m.  TAPS = 0: any number of taps; else exactly that many, every load issued
 // without a condition around it (taps before the start read a valid row and count zero), so that all of them are in flight
 template <typename T, int TAPS>
@@ -279,12 +293,28 @@ __global__ __launch_bounds__(4 * CT, 2) void rglru_tile_kernel(const vmi_hy_rglr
 #pragma unroll
       for (int e = 0; e < 4; ++e) a[e] = first ? 0.f : a[e];
       if (!p.single) {
-        walk16(a, b);
+        float odd = 0.f;   // (0, or no number where one of these is none or infinite)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          b[e] = fmaf(a[e], Sc[e], b[e]);
-          a[e] *= Pc[e];
-          if (mi + 1 < MT) Sc[e] = lane15(b[e]), Pc[e] = lane15(a[e]);
+        for (int e = 0; e < 4; ++e) odd = fmaf(b[e], 0.f, fmaf(Sc[e], 0.f, odd));
+        if (__builtin_amdgcn_ballot_w64(odd != odd) == 0) {   // (scalar)
+          walk16(a, b);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            b[e] = fmaf(a[e], Sc[e], b[e]);
+            a[e] *= Pc[e];
+          }
+        } else {
+          int opened = first;
+          step16<1>(a, b, opened), step16<2>(a, b, opened), step16<4>(a, b, opened), step16<8>(a, b, opened);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            b[e] = opened ? b[e] : fmaf(a[e], Sc[e], b[e]);
+            a[e] = opened ? 0.f : a[e] * Pc[e];
+          }
+        }
+        if (mi + 1 < MT) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) Sc[e] = lane15(b[e]), Pc[e] = lane15(a[e]);
         }
         if (kept(m, r)) *reinterpret_cast<f32x4*>(p.scratch + ((int64_t)s.T + t0 + m) * p.width + c0 + cl) = a;
       }
