@@ -44,6 +44,9 @@ CONFIGS = {
                              width=50, vocab=64),
     "large_heads": config([parallel(attention(8, 1, 130, 150, 0.12, 50, 49), delta(2, 1, 140, 150, 5), dense(40)),
                            retention(2, 150, 160, 100, (0.9, 0.98))], width=72, vocab=77),
+    # arms whose outputs are equally long, padded: one product of two groups behind them, with a feed-forward beside it and without
+    "alike": config([parallel(attention(4, 2, 24, 32, 0.35, 37, 50), delta(4, 2, 20, 24, 3), dense(40)),
+                     parallel(attention(2, 1, 40, 40, 0.3, 16, 30), delta(4, 4, 16, 20, 4))], width=80, vocab=101),
 }
 RANKS, BUCKETS = (5, 40), {13: 6, 37: 12, 32: 16, 16: 9, 50: 20}      # of the low-rank gates; of the bias by chunk
 

@@ -575,6 +575,34 @@ def test_portions_single_tokens_and_neighbours_do_not_change_the_logits(name, dt
     assert len(d.pool.free_blocks) == 14 and d.pool.free_state_slots == 3
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 47])
+def test_the_output_products_of_arms_that_are_alike_are_the_groups_of_one(T, monkeypatch):
+    """Every bit of the two products, which the matrices still give by themselves; and it is the joined one that a layer of few rows runs, both halves to the arm they belong to."""
+    from vllmini_amd import hybrid_layers, hybrid_ops as ops
+
+    d, g, linear, joined = decoder("alike", torch.bfloat16), torch.Generator().manual_seed(T), ops.linear, []
+    c = cases.CONFIGS["alike"]
+    w = cases.tensors(c)
+    for i, run in enumerate(d.model.runs):
+        m = run.mixer
+        K, N = m.w_pair.K, m.w_pair.N
+        assert m.w_pair.groups == 2 and ops.linear_plain(T, m.w_pair) and [p.K for p in m.w_out[:2]] == [K, K]
+        rows = torch.randn(T, 2 * K + m.ff, generator=g).to(torch.bfloat16).to(dev())
+        both = linear(rows, m.w_pair, x_gstride=K, y_gstride=N)
+        for k, (p, arm, vdim) in enumerate(zip(m.w_out[:2], ("left", "right"), (c["layers"][i]["mixer"][a]["vdim"] for a in ("left", "right")))):
+            x = rows[:, k * K: (k + 1) * K]
+            assert torch.equal(both[:, k * N: (k + 1) * N], linear(x, p)) and torch.equal(linear(x, p), linear(x, ops.MatrixTiles(p.dense, torch.bfloat16)))
+            o = hybrid_layers.padded_heads(w[f"l{i}.mix.{arm}.o"].to(dev()), K // hybrid_layers.pad32(vdim), hybrid_layers.pad32(vdim), 1)
+            close(both[:, k * N: k * N + c["width"]], x.double() @ o.double().T, torch.bfloat16, tol16=6e-3)      # (rounded once to bfloat16)
+    monkeypatch.setattr(ops, "linear", lambda x, m, **k: joined.append(m) or linear(x, m, **k))
+    toks = cases.tokens(c, 90, 1)
+    d.pool.open(0)
+    got = d.step([0], [toks[:T]], [list(range(T))])
+    assert [sum(m is r.mixer.w_pair for m in joined) for r in d.model.runs] == [1, 1]
+    assert not any(m is p for m in joined for r in d.model.runs for p in r.mixer.w_out[:2])
+    logits_close(got, expected("alike", toks)[0][:T], torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", BOTH)
 def test_long_decoding_from_one_token(dtype):
     name, n = "mixed", 200
@@ -587,7 +615,7 @@ def test_long_decoding_from_one_token(dtype):
 
 
 @pytest.mark.parametrize("vendor", [False, True], ids=["streaming", "vendor"])
-@pytest.mark.parametrize("name", ["mixed", "large_heads"])
+@pytest.mark.parametrize("name", ["mixed", "large_heads", "alike"])
 def test_graph_replay_equals_eager_steps(name, vendor, monkeypatch):
     """Both ways a layer's products may run, captured; eager steps run between the replays, and positions move on in both."""
     from vllmini_amd import hybrid_layers
