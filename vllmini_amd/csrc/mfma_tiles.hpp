@@ -180,8 +180,7 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     }
   }
   const Where at{m0, col * 4 * NI, SL, wave, kc, r16, {xs0, xs1}};
-  if constexpr (std::is_invocable_v<Early&, const Where&>) early(at);
-  else early(m0 + r16, s0, SL);   // (this lane's first row, this wave's first slab)
+  early(at);
   x_landed(std::integral_constant<int, D - 2>{});
   // The chunk in place d, and chunk kb on its way into the place of the one before (whose readers have all passed the barrier): steps of one fragment of x, which was asked
   // for AHEAD steps before, against the wave's NI of W, and its share of the requests.  A chunk that is none is zeros, x and W
@@ -230,8 +229,7 @@ __device__ __forceinline__ void tiles_product(const void* x, int64_t ldx, const 
     }
   };
   rest(std::integral_constant<int, 1>{}), rest(std::integral_constant<int, 2>{}), rest(std::integral_constant<int, 3>{});
-  if constexpr (std::is_invocable_v<Finish&, decltype((acc)), const Where&>) finish(acc, at);
-  else finish(acc, m0 + r16, s0, SL);
+  finish(acc, at);
 }
 
 // ---- which tile -----------------------------------------------------------------------------------------------------------------
