@@ -449,23 +449,27 @@ def test_single_tokens_take_a_row_tile_each_while_they_or_their_keys_are_few(hea
 
 
 def test_portions_over_keys_and_values_by_the_portion_alone():
-    """Which portions of a step go through latent_prompt, their tiles and the tokens they lie among; the others keep the latents, and decode steps have none."""
+    """Which portions of a step go through latent_prompt, between which tokens and entries they and the others lie, and their tiles where others stand among them and the places are many;
+    the others keep the latents, and decode steps have none."""
     from vllmini_amd.hybrid_decoder import HybridDecoder
     from vllmini_amd.hybrid_layers import QueryTiling
 
     d = object.__new__(HybridDecoder)
     d.model = SimpleNamespace(dtype=torch.bfloat16)
     d._kinds = [QueryTiling("latent", 16, 1, 576, sizes=(576,)), QueryTiling("latent", 16, 1, 576, sizes=(576,), prompts=True)]
-    for ctx, counts, tiles, places, own in (
-            ([9, 0, 30, 0, 0], [1, 130, 70, 1, 64], [(1, 128), (1, 64), (1, 0), (4, 0)], (1, 266, 0, 202), {0, 2, 3}), ([0, 0], [2, 65], [(1, 64), (0, 0), (1, 0)], (0, 67, 0, 0), set()),
-            ([5, 8], [1, 1], None, None, {0, 1}), ([0, 0], [1, 1], None, None, {0, 1}), ([64, 0], [64, 300], [(1, 256), (1, 192), (1, 128), (1, 64), (1, 0)], (64, 364, 0, 64), {0})):
+    many = [1] * 100 + [2] * 60 + [1200]
+    for ctx, counts, tiles, span, own in (
+            ([9, 0, 30, 0, 0], [1, 130, 70, 1, 64], None, (1, 266, 0, 202, 1, 5), {0, 2, 3}), ([0, 0], [2, 65], None, (0, 67, 0, 0, 0, 2), set()),
+            ([5, 8], [1, 1], None, None, {0, 1}), ([0, 0], [1, 1], None, None, {0, 1}), ([64, 0], [64, 300], None, (64, 364, 0, 64, 1, 2), {0}),
+            ([3] * 100 + [0] * 61, many, None, (100, 1420, 0, 100, 100, 161), set(range(100))),
+            ([0] + [3] * 99 + [0] * 61, [2] + many[1:], [(160, 64 * i) for i in range(18, 0, -1)] + [(i, 0) for i in (0, *range(100, 161))], (0, 1421, 2, 101, 0, 161), set(range(1, 100)))):
         ctx, counts = np.asarray(ctx), np.asarray(counts)
         n, T = len(counts), int(counts.sum())
         a = {"entry": np.repeat(np.arange(n), counts), "pos": np.zeros(T), "slots": [np.zeros(T)], "ctx": ctx, "state_slot": counts * 0, "parity": counts * 0, "tables": np.zeros((1, n, 1), dtype=np.int32)}
         sec, _, _, plans = d._layout(a, counts, np.arange(n), T, n, 1, int((ctx + counts).max()))
-        assert plans[0][3] is None and set(sec["tiles0"][::2]) == set(range(n)) and "prompts0" not in sec
-        assert plans[1][3] == places and set(sec["tiles1"][::2]) == own
-        assert ("prompts1" in sec) == (tiles is not None) and (tiles is None or list(map(tuple, sec["prompts1"].reshape(-1, 2).tolist())) == tiles)
+        assert plans[0][3] is None and set(sec["tiles0"][::2]) == set(range(n))
+        assert plans[1][3] == span and set(sec["tiles1"][::2]) == own
+        assert ("prompts" in sec) == (tiles is not None) and (tiles is None or list(map(tuple, sec["prompts"].reshape(-1, 2).tolist())) == tiles)
 
 
 def test_products_behind_a_norm_of_few_rows_and_columns_share_one_kernel_whatever_their_width():

@@ -1036,14 +1036,16 @@ def test_a_prompt_comes_to_the_same_whatever_shares_its_step(dim, rot, rank, cou
     d = object.__new__(HybridDecoder)
     d.model, d._kinds = type("Model", (), {"dtype": bf}), [layer.tiling()]
 
-    def run(own, splits=None):
-        """(the rows of the entries `own`, the cache) of a step of these entries alone."""
+    def run(own, splits=None, listed=False):
+        """(the rows of the entries `own`, the cache) of a step of these entries alone; listed: with the prompts' tiles as a list."""
         n, c = counts[own], ctx[own]
         tok = np.concatenate([np.arange(at[b], at[b] + counts[b]) for b in own])
         a = {"entry": np.repeat(np.arange(len(own)), n), "pos": tok, "slots": [tok], "ctx": c, "state_slot": n * 0, "parity": n * 0, "tables": tables[own][None]}
         sec, _, _, plans = d._layout(a, n, np.arange(1), len(tok), len(own), tables.shape[1], int((c + n).max()))
         rt, sp, nt, spans = plans[0]
-        plan = layers.AttentionPlan(i32(sec["tiles0"]).view(nt, 2), rt, splits or sp, None if spans is None else ops.PromptTiles(i32(sec["prompts0"]).view(-1, 2), *spans))
+        assert "prompts" not in sec
+        tiles = i32([(e, m) for e in np.flatnonzero((c == 0) & (n > 1)) for m in range(0, n[e] + 64, 64)]).view(-1, 2) if listed else None      # (one more than there are, each)
+        plan = layers.AttentionPlan(i32(sec["tiles0"]).view(nt, 2), rt, splits or sp, None if spans is None else ops.PromptTiles(tiles, *spans))
         cache, rows, step = pages.clone(), [], layout(n, c, tables[own], page)
         res = type("Residual", (), {"branch_in": lambda self, *a: proj[torch.as_tensor(tok, device=dev())].clone(), "branch_out": lambda self, o, *a: rows.append(o)})()
         layer.run(res, step, {layer.tiling(): plan}, [cache])
@@ -1051,7 +1053,9 @@ def test_a_prompt_comes_to_the_same_whatever_shares_its_step(dim, rot, rank, cou
 
     prompts, others = np.flatnonzero((ctx == 0) & (counts > 1)), np.flatnonzero((ctx > 0) | (counts == 1))
     got, cache, plan = run(np.arange(B))
-    assert plan.prompts is not None and sorted(set(plan.prompts.tiles[:, 0].tolist())) == prompts.tolist()
+    assert plan.prompts is not None
+    again, pages_again, _ = run(np.arange(B), listed=True)
+    assert torch.equal(got, again) and torch.equal(cache, pages_again)
     for own in (prompts, others):
         if len(own):
             want, alone, part = run(own, plan.splits if own is others else None)
@@ -1059,6 +1063,32 @@ def test_a_prompt_comes_to_the_same_whatever_shares_its_step(dim, rot, rank, cou
             for b, rows in zip(own, want.split(counts[own].tolist())):
                 assert torch.equal(got[at[b]: at[b] + counts[b]], rows), b
                 assert torch.equal(cache[tables[b, :per[b]]], alone[tables[b, :per[b]]])
+
+
+def test_the_parts_of_latent_prompts_by_themselves():
+    """The C entries for a step without a past, preparation and attention with a product between them, against the one call that has all three: every bit."""
+    import ctypes
+
+    from vllmini_amd import hybrid_ops as ops
+
+    H, dim, rot, rank, lens, page, bf = 2, 128, 32, 128, [70, 1, 130], 16, torch.bfloat16
+    g, T, D = torch.Generator(device=dev()).manual_seed(5), sum(lens), rank + rot
+    proj = torch.randn(T, H * (dim + rot) + D + 32, generator=g, device=dev()).to(bf)
+    w = ops.MatrixTiles(torch.randn(H * 2 * dim, rank, generator=g, device=dev()) * rank ** -0.5, bf)
+    step = layout(lens, [0] * 3, np.arange(3 * 9).reshape(3, 9), page)
+    step.fresh = True
+    names = dict(norm_w=torch.ones(rank, device=dev()), freq=torch.rand(rot // 2, generator=g, dtype=torch.float64, device=dev()), heads=H, dim=dim, rot=rot, rank=rank, rot_n=rot, rank_n=rank, eps=1e-5)
+    gate, caches = proj[:, H * (dim + rot) + D:], [torch.zeros((27, page, D), dtype=bf, device=dev()) for _ in range(2)]
+    want = ops.latent_prompt(proj.clone(), w, caches[0], step, vdim=dim, scale=0.1, gate=gate, **names)
+    own, rows, got, lib = proj.clone(), torch.empty((T, D), dtype=bf, device=dev()), torch.zeros_like(want), ops.load()
+    stream = torch.cuda.current_stream().cuda_stream
+    a = ops.PrepArgs(proj=own.data_ptr(), cache=caches[1].data_ptr(), norm_w=names["norm_w"].data_ptr(), freq=names["freq"].data_ptr(), ldp=own.stride(0), heads=H, dim=dim, rot=rot, rank=rank,
+                     rot_n=rot, rank_n=rank, eps=1e-5, dtype=ops.DTYPES[bf], device=0)
+    assert lib.vmi_hy_latent_prompt_prep(ctypes.byref(a), rows.data_ptr(), step.ref, stream) == 0
+    kv = ops.product_tiles(rows[:, :rank], w)
+    assert lib.vmi_hy_latent_prompt(own.data_ptr(), own.stride(0), kv.data_ptr(), kv.stride(0), rows.data_ptr(), gate.data_ptr(), gate.stride(0), got.data_ptr(), got.stride(0), H, dim, rot, dim,
+                                    rank, max(lens), 0.1, ops.DTYPES[bf], 0, step.ref, stream) == 0
+    assert torch.equal(got, want) and torch.equal(*caches)
 
 
 def test_prompts_of_more_places_than_a_launch_has_workgroups():

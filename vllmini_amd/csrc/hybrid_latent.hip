@@ -319,6 +319,11 @@ int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows,
   return VMI_HY_OK;
 }
 
+int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who) {
+  hipLaunchKernelGGL(latent_prompt_prep_kernel, dim3(s.T), dim3(256), latent_prep_lds(a.rot_n), st, a, s, static_cast<b16*>(rows), row0, min_len);
+  return launched(who);
+}
+
 }  // namespace vmi_hybrid
 
 using namespace vmi_hybrid;
@@ -339,20 +344,12 @@ int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, v
   return launched(who);
 }
 
-static int prompt_prep(const char* who, const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
-  if (int rc = check_latent_prompt_prep(a, rows, row0, min_len, s, who)) return rc;
+int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_latent_prompt_prep";
+  if (int rc = check_latent_prompt_prep(a, rows, 0, 0, s, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  hipLaunchKernelGGL(latent_prompt_prep_kernel, dim3(s->T), dim3(256), latent_prep_lds(a->rot_n), static_cast<hipStream_t>(stream), *a, *s, static_cast<b16*>(rows), row0, min_len);
-  return launched(who);
-}
-
-int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream) {
-  return prompt_prep("vmi_hy_latent_prompt_prep", a, rows, 0, 0, s, stream);
-}
-
-int vmi_hy_latent_prompt_tiles_prep(const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
-  return prompt_prep("vmi_hy_latent_prompt_tiles_prep", a, rows, row0, min_len, s, stream);
+  return launch_latent_prompt_prep(*a, rows, 0, 0, *s, static_cast<hipStream_t>(stream), who);
 }
 
 int32_t vmi_hy_latent_row_tiles(int32_t row_dim, int32_t want, int32_t dtype) { return row_tiles_for(row_dim, want, dtype); }

@@ -108,5 +108,8 @@ __device__ __forceinline__ void latent_prompt_prep_token(const vmi_hy_latent_pre
 }
 
 int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, int min_len, const vmi_hy_step* s, const char* who);
+int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who);
+// ... and l, the other entries' queries by heads into a's q, which does not read what that writes nor writes what it reads: few rows in one launch
+int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who);
 
 }  // namespace vmi_hybrid

@@ -16,6 +16,8 @@
 // 103 / 70; so also where a latent row is no longer than a head's columns, as each of 16 ranks and heads measured is, and from prompts of two tokens on: rank 512, 1 x 2 35.2 / 33.7, 1 x 8 42 / 35, 1 x 24 45 / 36, 6 x up to 20 64 / 53.
 // Beside entries with a past, which keep the latents and their launches: 64 of those behind 1000 tokens and 1 x 100 111 / 101; 12 behind 300 and 1 x 8, 48, 100, 500 51 / 57, 64 / 68, 72 / 76, 111 / 110.
 // Off 64 bits by as much, latents / here, eight draws each: 8 heads, 60 rows 0.00346 / 0.00350, 300 + 200 + 100 0.00355 / 0.00357, 600 0.00364 / 0.00363; 16 heads, 1024 0.00362 / 0.00360.
+#include "hybrid_latent_prep.hpp"
+#include "hybrid_linear.hpp"
 #include "hybrid_softmax.hpp"
 
 namespace vmi_hybrid {
@@ -25,9 +27,10 @@ constexpr int PQ = 64;   // queries of a workgroup, keys of a tile
 struct LatentPrompt {
   const b16 *proj, *kv, *rows, *gate;
   b16* out;
-  const int* tiles;   // [..][2]: entry, first position; NULL: every entry's places, the last of `places` first
+  const int* tiles;   // [..][2]: entry, first position; NULL: the places of `entries` entries from entry0 on, the last of `places` first
   int64_t ldp, ldkv, ldr, ldg, ldo;
-  int heads, rank, row0, places, tile0;   // kv and rows begin at token row0, a launch at tile tile0
+  int heads, rank, row0, tile0;   // kv and rows begin at token row0, a launch at tile tile0
+  int places, entry0, entries, min_len;   // min_len: 0, or the shortest entry without a past that is meant
   float scale;
 };
 
@@ -40,9 +43,10 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPromp
   b16* ks = reinterpret_cast<b16*>(smem);   // [64][LDK]
   b16* vs = ks + PQ * LDK;                  // [64][LDV]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kc = lane >> 4, r16 = lane & 15;
-  const int group = blockIdx.x / p.heads, h = blockIdx.x - group * p.heads, tile = p.tile0 + group, place = tile / s.B;
-  const int e = p.tiles ? p.tiles[2 * tile] : tile - place * s.B, q0 = p.tiles ? p.tiles[2 * tile + 1] : (p.places - 1 - place) * PQ;
+  const int group = blockIdx.x / p.heads, h = blockIdx.x - group * p.heads, tile = p.tile0 + group, place = tile / p.entries;
+  const int e = p.tiles ? p.tiles[2 * tile] : p.entry0 + tile - place * p.entries, q0 = p.tiles ? p.tiles[2 * tile + 1] : (p.places - 1 - place) * PQ;
   const int qs = s.q_start[e], len = s.q_len[e];
+  if (p.min_len && (s.ctx[e] != 0 || len < p.min_len)) return;
   if (q0 >= len) return;
   const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
   const b16* kv = p.kv + (int64_t)(qs - p.row0) * p.ldkv + h * (DN + VD);
@@ -183,36 +187,66 @@ int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t vdim, int32_
   return dtype == VMI_HY_BF16 && (dim == 64 || dim == 128) && vdim == dim && (rot == 32 || rot == 64) && rank > 0 && (rank & 63) == 0 && rot_n > 0 && (rot_n & 15) == 0 && rot_n <= rot;
 }
 
-static int run_prompt(const char* who, const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, int32_t row0, const void* gate, int64_t ldg, void* out, int64_t ldo,
-                      const int32_t* tiles, int64_t n_tiles, int32_t places, int32_t heads, int32_t dim, int32_t rot, int32_t vdim, int32_t rank, float scale, int32_t dtype, int32_t device,
-                      const vmi_hy_step* s, void* stream) {
-  if (!proj || !kv || !rows || !gate || !out || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || row0 < 0 || row0 >= s->T || n_tiles <= 0 || n_tiles > INT32_MAX ||
-      heads <= 0 || heads > 65535 || !(scale > 0.f))
-    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
-  if (!vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, 16, dtype) || ((ldp | ldkv) & 7) || (ldo & 3) || (((uintptr_t)proj | (uintptr_t)kv | (uintptr_t)rows) & 15) || ((uintptr_t)out & 7))
-    return fail(VMI_HY_E_SHAPE, who, "built for bfloat16 heads of 64 or 128 beside 32 or 64 rotated columns, rows aligned to 16 bytes");
-  DeviceScope dev(device);
-  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  auto rows_of = [](const void* p) { return static_cast<const b16*>(p); };
-  const LatentPrompt p{rows_of(proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), tiles, ldp, ldkv, rank + rot, ldg, ldo, heads, rank, row0, places, 0, scale};
-  const int n = (int)n_tiles;
-  if (dim == 128) return rot == 64 ? launch_prompt<128, 64>(p, n, *s, st) : launch_prompt<128, 32>(p, n, *s, st);
-  return rot == 64 ? launch_prompt<64, 64>(p, n, *s, st) : launch_prompt<64, 32>(p, n, *s, st);
+static int run_prompt(const LatentPrompt& p, int dim, int rot, int64_t tiles, const vmi_hy_step& s, hipStream_t st, const char* who) {
+  if (tiles <= 0 || tiles > INT32_MAX || p.heads <= 0 || p.heads > 65535 || !(p.scale > 0.f)) return fail(VMI_HY_E_ARG, who, "a size out of range");
+  if (((p.ldp | p.ldkv) & 7) || (p.ldo & 3) || (((uintptr_t)p.proj | (uintptr_t)p.kv | (uintptr_t)p.rows) & 15) || ((uintptr_t)p.out & 7))
+    return fail(VMI_HY_E_SHAPE, who, "needs rows aligned to 16 bytes");
+  const int n = (int)tiles;
+  if (dim == 128) return rot == 64 ? launch_prompt<128, 64>(p, n, s, st) : launch_prompt<128, 32>(p, n, s, st);
+  return rot == 64 ? launch_prompt<64, 64>(p, n, s, st) : launch_prompt<64, 32>(p, n, s, st);
 }
+static const b16* rows_of(const void* p) { return static_cast<const b16*>(p); }
 
 int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads, int32_t dim,
                          int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s, void* stream) {
-  const int32_t places = max_len <= 0 ? 0 : (max_len - 1) / PQ + 1;
-  return run_prompt("vmi_hy_latent_prompt", proj, ldp, kv, ldkv, rows, 0, gate, ldg, out, ldo, nullptr, s ? (int64_t)places * s->B : 0, places, heads, dim, rot, vdim, rank, scale, dtype,
-                    device, s, stream);
+  static const char* who = "vmi_hy_latent_prompt";
+  if (!proj || !kv || !rows || !gate || !out || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || max_len <= 0) return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  if (!vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, 16, dtype)) return fail(VMI_HY_E_SHAPE, who, "built for bfloat16 heads of 64 or 128 beside 32 or 64 rotated columns");
+  DeviceScope dev(device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  const int places = (max_len - 1) / PQ + 1;
+  const LatentPrompt p{rows_of(proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), nullptr, ldp, ldkv, rank + rot, ldg, ldo, heads, rank, 0, 0, places, 0, s->B, 0, scale};
+  return run_prompt(p, dim, rot, (int64_t)places * s->B, *s, static_cast<hipStream_t>(stream), who);
 }
 
-int vmi_hy_latent_prompt_tiles(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, int32_t row0, const void* gate, int64_t ldg, void* out, int64_t ldo,
-                               const int32_t* tiles, int32_t n_tiles, int32_t heads, int32_t dim, int32_t rot, int32_t vdim, int32_t rank, float scale, int32_t dtype, int32_t device,
-                               const vmi_hy_step* s, void* stream) {
-  return run_prompt("vmi_hy_latent_prompt_tiles", proj, ldp, kv, ldkv, rows, row0, gate, ldg, out, ldo, tiles, tiles ? n_tiles : 0, 0, heads, dim, rot, vdim, rank, scale, dtype, device, s,
-                    stream);
+int vmi_hy_latent_prompts(const vmi_hy_latent_prep_args* a, const vmi_hy_latent_attention_args* past, const void* w_uk, const void* w_uv, const void* w_kv, const void* gate, int64_t ldg,
+                          void* out, int64_t ldo, void* rows, void* kv, const int32_t* tiles, int32_t n_tiles, int32_t max_len, const int32_t span[6], int32_t min_len, float scale,
+                          const vmi_hy_step* s, void* stream) {
+  static const char* who = "vmi_hy_latent_prompts";
+  if (!a || !w_kv || !gate || !out || !kv || !span || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || span[0] < 0 || span[1] <= span[0] || span[1] > s->T ||
+      (tiles ? n_tiles <= 0 : (max_len <= 0 || span[4] < 0 || span[5] <= span[4] || span[5] > s->B)) || (span[3] == 0) != (min_len == 0))
+    return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
+  const int first = span[0], n = span[1] - first, at = span[2], others = span[3] == 0 ? 0 : span[3] - at, heads = a->heads, dim = a->dim, rank = a->rank, row = rank + a->rot;
+  if (others < 0 || at < 0 || span[3] > s->T || (others && (!past || !w_uk || !w_uv || !a->q || past->q != a->q || !past->out || past->heads != heads || past->rank != rank ||
+                                                            past->rot != a->rot || past->dtype != a->dtype || past->device != a->device)))
+    return fail(VMI_HY_E_ARG, who, "what the entries beside the prompts take does not fit");
+  if (int rc = check_latent_prompt_prep(a, rows, first, min_len, s, who)) return rc;
+  DeviceScope dev(a->device);
+  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t ldkv = (int64_t)heads * 2 * dim;
+  vmi_hy_linear_args l{};
+  l.groups = heads, l.scale = 1.f, l.x_kind = VMI_HY_X_ROWS, l.epilogue = VMI_HY_E_STORE, l.dtype = a->dtype, l.device = a->device;
+  if (others) {   // (their rows among the prompts' hold nothing, and give nothing: products are by rows)
+    vmi_hy_linear_args uk = l, uv = l;
+    uk.x = rows_of(a->proj) + at * a->ldp, uk.w = w_uk, uk.y = static_cast<b16*>(a->q) + (int64_t)at * heads * row, uk.ldx = a->ldp, uk.ldy = (int64_t)heads * row;
+    uk.x_gstride = dim + a->rot, uk.y_gstride = row, uk.M = others, uk.N = rank, uk.K = dim;
+    uv.x = static_cast<b16*>(past->out) + (int64_t)at * heads * rank, uv.w = w_uv, uv.y = static_cast<b16*>(out) + at * ldo, uv.ldx = (int64_t)heads * rank, uv.ldy = ldo;
+    uv.x_gstride = rank, uv.y_gstride = dim, uv.M = others, uv.N = dim, uv.K = rank, uv.epilogue = VMI_HY_E_GATED, uv.gate = rows_of(gate) + at * ldg, uv.ldg = ldg;
+    if (int rc = check_linear(&uk, who)) return rc;
+    if (int rc = check_linear(&uv, who)) return rc;
+    if (int rc = launch_latent_prompt_in(uk, *a, rows, first, min_len, *s, st, who)) return rc;
+    if (int rc = vmi_hy_latent_attention(past, s, st)) return rc;
+    if (int rc = vmi_hy_linear(&uv, st)) return rc;
+  } else if (int rc = launch_latent_prompt_prep(*a, rows, first, min_len, *s, st, who)) {
+    return rc;
+  }
+  l.x = rows, l.w = w_kv, l.y = kv, l.ldx = row, l.ldy = ldkv, l.M = n, l.N = (int)ldkv, l.K = rank, l.groups = 1;
+  if (int rc = vmi_hy_product_tiles(&l, st)) return rc;
+  const int places = tiles ? 0 : (max_len - 1) / PQ + 1, entries = tiles ? 1 : span[5] - span[4];
+  const LatentPrompt p{rows_of(a->proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), tiles, a->ldp, ldkv, row, ldg, ldo, heads, rank, first, 0,
+                       places, span[4], entries, tiles ? 0 : min_len, scale};
+  return run_prompt(p, dim, a->rot, tiles ? n_tiles : (int64_t)places * entries, *s, st, who);
 }
 
 }  // extern "C"

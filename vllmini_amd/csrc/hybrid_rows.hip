@@ -162,7 +162,7 @@ __global__ __launch_bounds__(64 * RW, RW / 4) void plain_rows_kernel(const vmi_h
 
 // A product by heads and what a token's attention needs besides: two launches of a chain that do not read each other's results, in one.  The
 // first T workgroups take a token each, the others a slab of 16 columns of 16 MT rows of a head.  Few rows, each is little more than its launch: queries into the latent space beside
-// latent_prep, 8 heads of 128 into 512, 12 rows, us: 4.2 + 4.9 -> 4.8; width 1024, 12 sequences, 24 tokens 7311 -> 7203, width 4096, one, 16 tokens 14 019 -> 13 919.
+// latent_prep, 8 heads of 128 into 512, 12 rows, us: 4.2 + 4.9 -> 4.8; width 1024, 12 sequences, 24 tokens 7311 -> 7203 (of one sequence, width 4096, less than two runs of it differ by).
 // The gates' products (2 of 2048 x 128, 32 rows) beside kv_prep 4.5 + 5.1 -> 5.0.
 struct LatentPrep {
   vmi_hy_latent_prep_args a;
@@ -701,6 +701,12 @@ static int launch_beside(const vmi_hy_linear_args& p, const Prep& prep, const vm
   return mt == 1 ? go(rows_beside_kernel<4, 1, Prep>, 4) : go(rows_beside_kernel<4, 2, Prep>, 4);
 }
 
+int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who) {
+  if (beside_fits(l, s)) return launch_beside(l, LatentPromptPrep{a, static_cast<b16*>(rows), row0, min_len}, s, latent_prep_lds(a.rot_n), who, st);
+  if (int rc = vmi_hy_linear(&l, st)) return rc;
+  return launch_latent_prompt_prep(a, rows, row0, min_len, s, st, who);
+}
+
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {
   switch (p.epilogue) {
     case VMI_HY_E_STORE: return plain_rows_epi<VMI_HY_E_STORE>(p, st);
@@ -726,19 +732,6 @@ int vmi_hy_latent_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args*
   DeviceScope dev(l->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   return launch_beside(*l, LatentPrep{*a}, *s, latent_prep_lds(a->rot_n), who, static_cast<hipStream_t>(stream));
-}
-
-int vmi_hy_latent_prompt_tiles_in(const vmi_hy_linear_args* l, const vmi_hy_latent_prep_args* a, void* rows, int32_t row0, int32_t min_len, const vmi_hy_step* s, void* stream) {
-  static const char* who = "vmi_hy_latent_prompt_tiles_in";
-  if (int rc = check_linear(l, who)) return rc;
-  if (int rc = check_latent_prompt_prep(a, rows, row0, min_len, s, who)) return rc;
-  if (a->device != l->device || !beside_fits(*l, *s)) {
-    if (int rc = vmi_hy_linear(l, stream)) return rc;
-    return vmi_hy_latent_prompt_tiles_prep(a, rows, row0, min_len, s, stream);
-  }
-  DeviceScope dev(l->device);
-  if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  return launch_beside(*l, LatentPromptPrep{*a, static_cast<b16*>(rows), row0, min_len}, *s, latent_prep_lds(a->rot_n), who, static_cast<hipStream_t>(stream));
 }
 
 int vmi_hy_kv_prep_in(const vmi_hy_linear_args* l, const vmi_hy_kv_prep_args* a, const vmi_hy_step* s, void* stream) {

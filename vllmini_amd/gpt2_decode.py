@@ -94,8 +94,9 @@ class GPT2PagedDecoder:
     NATIVE_LAYERS_MAX_BATCH = 512    # larger steps run the block's linear layers as torch modules (real GEMMs by then)
     # prompts of more tokens in all (times the width's square) issue their launches from here: the native call saves the host 150 us, which is what a call of fewer waits for.
     # Their products are tiles of our own up to OWN_PRODUCTS_MAX_WORK, biases and residual adds in the same launch, and the vendor's but for c_fc with its GELU beyond, where
-    # none was measured.  12 layers of prompts of 200 tokens, tiles / vendor in us: width 512 8000 tokens 1964 / 2334, 12 000 2470 / 2901; 768 5000 1791 / 2136, 12 000 3446 / 3972; 1024 4000
-    # 2038 / 2204, 7000 3344 / 3426, 12 000 4879 / 5331; 1152 4000 2585 / 2833, 7000 3691 / 3889, 12 000 5858 / 6833
+    # none was measured.  12 layers of prompts of 200 tokens, tiles / vendor in us: width 256 8000 tokens 1965 / 2353, 60 000 8950 / 9331; 512 8000 2227 / 2489, 27 000 5946 / 6584, 60 000 13 381 / 14 200;
+    # 768 5000 1791 / 2136, 12 000 4065 / 4665, 20 000 6517 / 6617, 27 000 8804 / 9561; 1024 4000 2253 / 2457, 12 000 5666 / 6080, 16 000 7200 / 7176; 1152 4000 2814 / 3061, 8000 4640 / 5177, 12 000
+    # 6591 / 7484
     NATIVE_PROMPT_MAX_WORK = 28 * 10 ** 8
     NATIVE_PROMPT_MAX_TOKENS = 8192      # (no more of them measured; an instance has its width's)
     OWN_PRODUCTS_MAX_WORK = 160 * 10 ** 8

@@ -119,15 +119,20 @@ class HybridDecoder:
         sec["table"] = tab.reshape(-1)
         put("rows", max(len(rows), 1), rows, 0)
         plans = []
+        several, prompts = bool((counts > 1).any()), None
+        if several and any(kind.prompts for kind in self._kinds):
+            pays = ops.latent_prompt_pays((a["ctx"], counts))
+            prompts = self._prompts(sec, pays, counts, starts) if np.any(pays) else None
         for kind in self._kinds:
-            mine, prompts = counts, None      # (the portions of this kind's own tiles, and what of the step is not among them)
-            if kind.prompts and (counts > 1).any():
-                pays = ops.latent_prompt_pays(np.stack([a["ctx"], counts], axis=1))
-                if np.any(pays):
-                    mine, prompts = np.where(pays, 0, counts), self._prompts(sec, f"prompts{len(plans)}", pays, counts, starts)
-            rep, longest, keys = kind.rep, max(int(mine.max()), 1), max_keys if prompts is None else int(((a["ctx"] + mine) * (mine > 0)).max())
-            entries = B if prompts is None else int((mine > 0).sum())
-            rt = 1 if longest == 1 and kind.one_row_tile(entries, keys) else kind.row_tiles(longest, self.model.dtype)
+            mine, keys, entries, own = counts, max_keys, B, prompts if kind.prompts else None      # (the portions of this kind's own tiles)
+            if own is not None:
+                if own[3] == 0:               # (there are none)
+                    sec[f"tiles{len(plans)}"] = np.empty(0, dtype=np.int32)
+                    plans.append((1, 1, 0, own))
+                    continue
+                mine, keys, entries = np.where(pays, 0, counts), int(np.where(pays, 0, a["ctx"] + counts).max()), b - int(np.count_nonzero(pays))
+            rep, most = kind.rep, max(int(mine.max()), 1)
+            rt = 1 if most == 1 and kind.one_row_tile(entries, keys) else kind.row_tiles(most, self.model.dtype)
             per = -(-(mine * rep) // (16 * rt))
             ent = np.repeat(np.arange(b), per)
             first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * 16 * rt
@@ -139,8 +144,8 @@ class HybridDecoder:
             t = np.full((nt, 2), -1, dtype=np.int32)
             t[: len(ent), 0], t[: len(ent), 1] = ent, first
             sec[f"tiles{len(plans)}"] = t.reshape(-1)
-            plans.append((rt, self._split_of(nt, rt, kind, keys, T), nt, prompts))
-        if (counts > 1).any():                # runs of rows for the linear-attention layers
+            plans.append((rt, self._split_of(nt, rt, kind, keys, T), nt, own))
+        if several:                           # runs of rows for the linear-attention layers
             per = -(-counts // ops.CHUNK_ROWS)
             at = np.cumsum(per) - per
             put("chunk_start", B, at, 0)
@@ -153,16 +158,19 @@ class HybridDecoder:
         return sec, offs, total, plans
 
     @staticmethod
-    def _prompts(sec: Dict[str, np.ndarray], name: str, pays: np.ndarray, counts: np.ndarray, starts: np.ndarray) -> Tuple[int, int, int, int]:
-        """The tiles of the portions that go through ops.latent_prompt, the longest walks first, and the tokens between which they and the others lie."""
-        own = np.flatnonzero(pays)
-        per = -(-counts[own] // ops.PROMPT_TILE)
-        first = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * ops.PROMPT_TILE
-        order = np.argsort(-first, kind="stable")
-        sec[name] = np.stack([np.repeat(own, per)[order], first[order]], axis=1).astype(np.int32).reshape(-1)
-        rest = np.flatnonzero(~pays & (counts > 0))
-        return (*(int(x) for x in (starts[own[0]], starts[own[-1]] + counts[own[-1]])),
-                *((int(starts[rest[0]]), int(starts[rest[-1]] + counts[rest[-1]])) if len(rest) else (0, 0)))
+    def _prompts(sec: Dict[str, np.ndarray], pays: np.ndarray, counts: np.ndarray, starts: np.ndarray) -> Tuple[int, ...]:
+        """The tokens between which the portions that go through ops.latent_prompt lie, those between which the others do, and the former's entries (as ops.PromptTiles has them); and, where
+        others stand among them or the longest is one of few, so that a launch over all their places would be mostly empty ones (each some ns), a list of their tiles, longest walks first."""
+        b = len(pays)
+        e0, e1, r0, r1 = int(np.argmax(pays)), b - int(np.argmax(pays[::-1])), int(np.argmin(pays)), b - int(np.argmin(pays[::-1]))
+        first, last, others = int(starts[e0]), int(starts[e1 - 1] + counts[e1 - 1]), not pays[r0]
+        if -(-int(counts.max()) // ops.PROMPT_TILE) * (e1 - e0) > 1024 + last - first:
+            own = np.flatnonzero(pays)
+            per = -(-counts[own] // ops.PROMPT_TILE)
+            at = (np.arange(int(per.sum())) - np.repeat(np.cumsum(per) - per, per)) * ops.PROMPT_TILE
+            order = np.argsort(-at, kind="stable")
+            sec["prompts"] = np.stack([np.repeat(own, per)[order], at[order]], axis=1).astype(np.int32).reshape(-1)
+        return (first, last, *((int(starts[r0]), int(starts[r1 - 1] + counts[r1 - 1])) if others else (0, 0)), e0, e1)
 
     def _staged(self, sec, offs, total: int) -> PinnedBuffer:
         """The sections in pinned memory (a ring of four buffers)."""
@@ -193,7 +201,8 @@ class HybridDecoder:
         v["table"] = v["table"].view(B, table_ld)
         if "chunks" in v:
             v["chunks"] = v["chunks"].view(-1, 2)
-        plan = {kind: AttentionPlan(v[f"tiles{i}"].view(nt, 2), rt, sp, None if at is None else ops.PromptTiles(v[f"prompts{i}"].view(-1, 2), *at))
+        listed = v["prompts"].view(-1, 2) if "prompts" in v else None
+        plan = {kind: AttentionPlan(v[f"tiles{i}"].view(nt, 2), rt, sp, None if at is None else ops.PromptTiles(listed, *at))
                 for i, (kind, (rt, sp, nt, at)) in enumerate(zip(self._kinds, plans))}
         return v, plan
 

@@ -23,7 +23,7 @@ where one stands behind them, or to the vendor library where that is ahead (prod
 from __future__ import annotations
 
 import math
-from typing import Callable, Dict, List, NamedTuple, Optional, Sequence, Tuple
+from typing import Dict, List, NamedTuple, Optional, Sequence, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -242,23 +242,14 @@ class LatentAttention:
         proj = res.branch_in(self.norm, self.w_in, step)
         sizes = dict(norm_w=self.norm_w, freq=self.freq, heads=H, dim=self.dim, rot=self.rot, rank=self.rank, rot_n=self.rot_n, rank_n=self.rank_n, eps=self.eps)
         gate = proj[:, self.gate_at:]
-
-        def attention(q: torch.Tensor) -> torch.Tensor:
-            return ops.latent_attention(q, cache, step, plan.tiles, heads=H, rank=self.rank, rot=self.rot, scale=self.scale, row_tiles=plan.row_tiles, splits=plan.splits)
-
-        def past(out: torch.Tensor, latent_in: Callable[[slice, MatrixTiles, torch.Tensor], None]) -> None:
-            """The entries that have one, beside prompts (whose rows among them hold nothing: every product is by rows)."""
-            at = slice(plan.prompts.past_first, plan.prompts.past_last)
-            q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
-            latent_in(at, self.w_uk, q)
-            ops.linear(attention(q)[at], self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=gate[at], out=out[at])
-
         if plan.prompts is not None:
-            o = ops.latent_prompt(proj, self.w_kv, cache, step, vdim=self.vdim, scale=self.scale, gate=gate, prompts=plan.prompts, others=past if plan.prompts.past_last else None, **sizes)
+            o = ops.latent_prompt(proj, self.w_kv, cache, step, vdim=self.vdim, scale=self.scale, gate=gate, prompts=plan.prompts,
+                                  past=ops.PastTiles(self.w_uk, self.w_uv, plan.tiles, plan.row_tiles, plan.splits) if plan.prompts.past_last else None, **sizes)
         else:
             q = torch.empty((step.T, H * D), dtype=proj.dtype, device=proj.device)
             ops.latent_in(proj, self.w_uk, q, cache, step, **sizes)
-            o = ops.linear(attention(q), self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=gate)
+            lat = ops.latent_attention(q, cache, step, plan.tiles, heads=H, rank=self.rank, rot=self.rot, scale=self.scale, row_tiles=plan.row_tiles, splits=plan.splits)
+            o = ops.linear(lat, self.w_uv, x_gstride=self.rank, y_gstride=self.vdim, gate=gate)
         res.branch_out(o, self.w_o, step)
 
 

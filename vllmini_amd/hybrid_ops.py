@@ -22,7 +22,7 @@ import ctypes
 import functools
 import os
 import threading
-from typing import Callable, NamedTuple, Optional, Sequence, Tuple
+from typing import NamedTuple, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -101,11 +101,10 @@ SIGNATURES = {
     "vmi_hy_kv_prep_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(KvPrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
-    "vmi_hy_latent_prompt_tiles_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_latent_prompt": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
-    "vmi_hy_latent_prompt_tiles_in": (ctypes.c_int, [ctypes.POINTER(LinearArgs), ctypes.POINTER(PrepArgs), _vp, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
-    "vmi_hy_latent_prompt_tiles": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _i32, _vp, _i64, _vp, _i64, _vp, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
+    "vmi_hy_latent_prompts": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(AttentionArgs), *[_vp] * 4, _i64, _vp, _i64, *[_vp] * 3, _i32, _i32, ctypes.POINTER(_i32 * 6), _i32, _f32,
+                                             ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_row_tiles": (_i32, [_i32, _i32, _i32]),
     "vmi_hy_latent_attention": (ctypes.c_int, [ctypes.POINTER(AttentionArgs), ctypes.POINTER(StepArgs), _vp]),
     "vmi_hybrid_last_error": (ctypes.c_char_p, []),
@@ -580,61 +579,70 @@ def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int, rot_n: int, dty
 PROMPT_TILE, PROMPT_MIN_TOKENS = 64, 2      # positions of a tile of latent_prompt's kernel; the shortest portion that goes there
 
 
-def latent_prompt_pays(portions: np.ndarray) -> np.ndarray:
-    """Which of a step's portions, (ctx, tokens) each, go through latent_prompt: by the portion alone, whatever shares its step, so that a prompt's keys and values are rounded at the same
-    places beside others as by itself (vmi_hy_latent_prompt_tiles_in has the same rule).  Ahead of the latents from two tokens on (csrc/hybrid_latent_prompt.hip); one is a decoding step's."""
-    return (portions[:, 0] == 0) & (portions[:, 1] >= PROMPT_MIN_TOKENS)
+def latent_prompt_pays(portions: Tuple[np.ndarray, np.ndarray]) -> np.ndarray:
+    """Which of a step's portions (their contexts, their tokens) go through latent_prompt: by the portion alone, whatever shares its step, so that a prompt's keys and values are rounded at the
+    same places beside others as by itself (vmi_hy_latent_prompts has the same rule).  Ahead of the latents from two tokens on (csrc/hybrid_latent_prompt.hip); one is a decoding
+    step's."""
+    ctx, tokens = portions
+    return (ctx == 0) & (tokens >= PROMPT_MIN_TOKENS)
 
 
 class PromptTiles(NamedTuple):
-    """The entries of a step that go through latent_prompt: their tiles of positions (int32 [n, 2]: entry, first position), and the tokens, from .. to, that all of them lie among, and
-    all of the others (to = 0: there are no others)."""
-    tiles: torch.Tensor
+    """The entries of a step that go through latent_prompt: their tiles of positions (int32 [n, 2]: entry, first position; None: the places of all between two entries), the tokens,
+    from .. to, that all of them lie among, and all of the others (to = 0: there are no others), and the entries that they lie among."""
+    tiles: Optional[torch.Tensor]
     first: int
     last: int
-    past_first: int = 0
-    past_last: int = 0
+    past_first: int
+    past_last: int
+    entry_first: int
+    entry_last: int
+
+
+class PastTiles(NamedTuple):
+    """What the entries of a step that do not go through latent_prompt take beside it: the up-projections by heads, and their latent_attention's arguments."""
+    w_uk: MatrixTiles
+    w_uv: MatrixTiles
+    tiles: torch.Tensor
+    row_tiles: int
+    splits: int
 
 
 def latent_prompt(proj: torch.Tensor, w_kv: MatrixTiles, cache: torch.Tensor, step: StepLayout, *, norm_w: torch.Tensor, freq: torch.Tensor, heads: int, dim: int, rot: int, vdim: int,
-                  rank: int, rot_n: int, rank_n: int, eps: float, scale: float, gate: torch.Tensor, prompts: Optional[PromptTiles] = None,
-                  others: Optional[Callable[[torch.Tensor, Callable[[slice, MatrixTiles, torch.Tensor], None]], None]] = None) -> torch.Tensor:
+                  rank: int, rot_n: int, rank_n: int, eps: float, scale: float, gate: torch.Tensor, prompts: Optional[PromptTiles] = None, past: Optional[PastTiles] = None) -> torch.Tensor:
     """Latent attention of entries without a past over their keys and values, gates included: proj (whose query parts are rotated in place) -> [T, heads * vdim], the cache's rows of
-    all entries written.  w_kv: the up-projections, per head [dim | vdim] rows of rank.  prompts: which entries (None: all of them, a `fresh` step); others(out, latent_in):
-    what the rest takes, beginning with latent_in(tokens, w_uk, q), its result into its rows of out (and whatever it likes into the prompts')."""
+    all entries written.  w_kv: the up-projections, per head [dim | vdim] rows of rank.  prompts: which entries (None: all of them, a `fresh` step); past: what the others, which go over the
+    latents as by latent_in(), latent_attention() and linear(), take for it.  All launches from one native call: each of them from here is as many microseconds of host as a short
+    prompt's kernel takes."""
     device, stream = _on(proj)
-    T, D = step.T, rank + rot
-    _need((step.fresh or prompts is not None) and proj.shape[0] == T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and cache.dtype == proj.dtype and cache.shape[-1] == D
+    T, D, dt, dev = step.T, rank + rot, proj.dtype, proj.device
+    _need((step.fresh or prompts is not None) and proj.shape[0] == T and proj.shape[1] >= heads * (dim + rot) + D and proj.stride(1) == 1 and cache.dtype == dt and cache.shape[-1] == D
           and cache.is_contiguous() and norm_w.numel() == rank and norm_w.dtype == torch.float32 and freq.dtype == torch.float64 and freq.numel() == rot_n // 2
-          and w_kv.groups == 1 and (w_kv.N, w_kv.K) == (heads * (dim + vdim), rank) and gate.dtype == proj.dtype and gate.shape[0] == T and gate.shape[1] >= heads
-          and gate.stride(1) == 1, "hybrid_ops.latent_prompt: operand sizes")
-    tiles, first, last, mixed = None, 0, T, False
-    if prompts is not None:
-        tiles, first, last, mixed = prompts.tiles, prompts.first, prompts.last, prompts.past_last > 0
-        _need(tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.dim() == 2 and tiles.shape[1] == 2 and 0 <= first < last <= T, "hybrid_ops.latent_prompt: prompts")
-    _need(mixed == (others is not None), "hybrid_ops.latent_prompt: entries beside the prompts, and what they take")
-    rows = torch.empty((last - first, D), dtype=proj.dtype, device=proj.device)
-    out = torch.empty((T, heads * vdim), dtype=proj.dtype, device=proj.device)
+          and w_kv.groups == 1 and (w_kv.N, w_kv.K) == (heads * (dim + vdim), rank) and w_kv.tiles.dtype == dt and gate.dtype == dt and gate.shape[0] == T and gate.shape[1] >= heads
+          and gate.stride(1) == 1 and vdim == dim, "hybrid_ops.latent_prompt: operand sizes")
+    tiles, *span = prompts if prompts is not None else (None, 0, T, 0, 0, 0, step.B)
+    first, last, at, to = span[:4]
+    mixed = to > 0
+    _need(0 <= first < last <= T and (tiles is None or (tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.dim() == 2 and tiles.shape[1] == 2)), "hybrid_ops.latent_prompt: prompts")
+    rows, kv = torch.empty((last - first, D), dtype=dt, device=dev), torch.empty((last - first, w_kv.N), dtype=dt, device=dev)
+    out = torch.empty((T, heads * vdim), dtype=dt, device=dev)
     a = PrepArgs(proj=proj.data_ptr(), cache=cache.data_ptr(), norm_w=norm_w.data_ptr(), freq=freq.data_ptr(), ldp=proj.stride(0), heads=heads, dim=dim, rot=rot, rank=rank,
-                 rot_n=rot_n, rank_n=rank_n, eps=eps, dtype=DTYPES[proj.dtype], device=device)
-
-    if others is None:
-        _check(load().vmi_hy_latent_prompt_tiles_prep(ctypes.byref(a), rows.data_ptr(), first, 0, step.ref, stream))
-    else:
-        def latent_in(at: slice, w_uk: MatrixTiles, q: torch.Tensor) -> None:
-            _need(q.shape == (T, heads * D) and q.is_contiguous() and q.dtype == proj.dtype and (w_uk.groups, w_uk.N, w_uk.K) == (heads, rank, dim), "hybrid_ops.latent_prompt: q")
-            a.q = q.data_ptr()      # (which entries, latent_prompt_pays has for the host)
-            b = _by_groups(proj[at], w_uk, q[at], dim + rot, D, device)
-            _check(load().vmi_hy_latent_prompt_tiles_in(ctypes.byref(b), ctypes.byref(a), rows.data_ptr(), first, PROMPT_MIN_TOKENS, step.ref, stream))
-
-        others(out, latent_in)
-    kv = product_tiles(rows[:, :rank], w_kv)
-    at = (proj.data_ptr(), proj.stride(0), kv.data_ptr(), kv.stride(0), rows.data_ptr())
-    to, sizes = (gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0)), (heads, dim, rot, vdim, rank)
-    if tiles is None:
-        _check(load().vmi_hy_latent_prompt(*at, *to, *sizes, step.max_len, scale, DTYPES[proj.dtype], device, step.ref, stream))
-    else:
-        _check(load().vmi_hy_latent_prompt_tiles(*at, first, *to, tiles.data_ptr(), tiles.shape[0], *sizes, scale, DTYPES[proj.dtype], device, step.ref, stream))
+                 rot_n=rot_n, rank_n=rank_n, eps=eps, dtype=DTYPES[dt], device=device)
+    b = w_uk = w_uv = None
+    _need(mixed == (past is not None), "hybrid_ops.latent_prompt: entries beside the prompts, and what they take")
+    if past is not None:
+        w_uk, w_uv = past.w_uk.tiles, past.w_uv.tiles
+        _need((past.w_uk.groups, past.w_uk.N, past.w_uk.K) == (heads, rank, dim) and (past.w_uv.groups, past.w_uv.N, past.w_uv.K) == (heads, vdim, rank) and w_uk.dtype == w_uv.dtype == dt
+              and cache.dim() == 3 and cache.shape[1] == step.args.page_size and past.tiles.dtype == torch.int32 and past.tiles.dim() == 2 and past.tiles.shape[1] == 2
+              and past.tiles.is_contiguous() and 0 <= at < to <= T, "hybrid_ops.latent_prompt: what the entries beside the prompts take")
+        q, latents = torch.empty((T, heads * D), dtype=dt, device=dev), torch.empty((T, heads * rank), dtype=dt, device=dev)
+        partial = torch.empty((past.splits, T * heads, rank + 2), dtype=torch.float32, device=dev) if past.splits > 1 else None
+        a.q = q.data_ptr()
+        b = ctypes.byref(AttentionArgs(q=a.q, cache=a.cache, out=latents.data_ptr(), tiles=past.tiles.data_ptr(), partial=_ptr(partial), heads=heads, rank=rank, rot=rot,
+                                       n_tiles=past.tiles.shape[0], row_tiles=past.row_tiles, splits=past.splits, scale=scale, dtype=a.dtype, device=device))
+    _check(load().vmi_hy_latent_prompts(ctypes.byref(a), b, _ptr(w_uk), _ptr(w_uv), w_kv.tiles.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0), rows.data_ptr(),
+                                        kv.data_ptr(), _ptr(tiles), 0 if tiles is None else tiles.shape[0], step.max_len, ctypes.byref((_i32 * 6)(*span)),
+                                        PROMPT_MIN_TOKENS if mixed else 0, scale, step.ref, stream))      # (which entries, latent_prompt_pays has for the host)
     return out
 
 
