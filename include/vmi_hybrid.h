@@ -203,14 +203,15 @@ VMI_HY_API int32_t vmi_hy_latent_prompt_fits(int32_t dim, int32_t rot, int32_t v
 VMI_HY_API int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t ldkv, const void* rows, const void* gate, int64_t ldg, void* out, int64_t ldo, int32_t heads,
                                     int32_t dim, int32_t rot, int32_t vdim, int32_t rank, int32_t max_len, float scale, int32_t dtype, int32_t device, const vmi_hy_step* s,
                                     void* stream);
-/* The whole of latent attention, up-projections included, of a step whose entries without a past and with min_len tokens or more go over their keys and values (min_len 0: every entry) and whose
- * others over the latents, in one call: a as vmi_hy_latent_prep takes it, dim columns of value a head; matrices in the layout of vmi_hy_linear, w_kv [heads][dim | dim][rank], w_uk and w_uv
- * groups of heads; out and gate as above.  tiles [n_tiles][2]: entry and first position, one for every 64 positions of every entry of the former kind, in any order (a position past
- * the entry's last: none); NULL: of entries span[4] .. span[5] - 1, of max_len tokens at most.  span (host memory): from which token to which the former lie, and the others (to = 0:
- * there are none, then past, w_uk, w_uv and a's q may be NULL).  rows [span[1] - span[0]][rank + rot] and kv [..][heads][dim | dim]: scratch.  past: the others' attention, its tiles theirs alone, q a's, out scratch. */
+/* The whole of latent attention, up-projections included, of a step whose entries without a past (ctx is 0) go over their keys and values and whose others over the latents, in one
+ * call: a as vmi_hy_latent_prep takes it, dim columns of value a head; matrices in the layout of vmi_hy_linear, w_kv [heads][dim | dim][rank], w_uk and w_uv groups of heads; out and gate
+ * as above.  tiles [n_tiles][2]: entry and first position, one for every 64 positions of every entry without a past, in any order (a position past the entry's last: none); NULL: all of
+ * those among entries span[4] .. span[5] - 1, of max_len tokens at most.  span (host memory): from which token to which they lie, and the others (to = 0: there are none, then past,
+ * w_uk, w_uv and a's q may be NULL).  rows [span[1] - span[0]][rank + rot] and kv [..][heads][dim | dim]: scratch.  past: the others' attention, its tiles theirs alone, q a's, out
+ * scratch. */
 VMI_HY_API int vmi_hy_latent_prompts(const vmi_hy_latent_prep_args* a, const vmi_hy_latent_attention_args* past, const void* w_uk, const void* w_uv, const void* w_kv, const void* gate,
                                      int64_t ldg, void* out, int64_t ldo, void* rows, void* kv, const int32_t* tiles, int32_t n_tiles, int32_t max_len, const int32_t span[6],
-                                     int32_t min_len, float scale, const vmi_hy_step* s, void* stream);
+                                     float scale, const vmi_hy_step* s, void* stream);
 
 /* Linear attention with a matrix state per head, S [dim, vdim] float32 (csrc/hybrid_state.hip).  proj [T, ldp] begins with the
  * columns q [kv_heads dim] | k [kv_heads dim] | v [heads vdim]; head h uses q / k head h / (heads / kv_heads).

@@ -450,7 +450,7 @@ def test_single_tokens_take_a_row_tile_each_while_they_or_their_keys_are_few(hea
 
 def test_portions_over_keys_and_values_by_the_portion_alone():
     """Which portions of a step go through latent_prompt, between which tokens and entries they and the others lie, and their tiles where others stand among them and the places are many;
-    the others keep the latents, and decode steps have none."""
+    the others keep the latents, and captured steps have none."""
     from vllmini_amd.hybrid_decoder import HybridDecoder
     from vllmini_amd.hybrid_layers import QueryTiling
 
@@ -459,8 +459,8 @@ def test_portions_over_keys_and_values_by_the_portion_alone():
     d._kinds = [QueryTiling("latent", 16, 1, 576, sizes=(576,)), QueryTiling("latent", 16, 1, 576, sizes=(576,), prompts=True)]
     many = [1] * 100 + [2] * 60 + [1200]
     for ctx, counts, tiles, span, own in (
-            ([9, 0, 30, 0, 0], [1, 130, 70, 1, 64], None, (1, 266, 0, 202, 1, 5), {0, 2, 3}), ([0, 0], [2, 65], None, (0, 67, 0, 0, 0, 2), set()),
-            ([5, 8], [1, 1], None, None, {0, 1}), ([0, 0], [1, 1], None, None, {0, 1}), ([64, 0], [64, 300], None, (64, 364, 0, 64, 1, 2), {0}),
+            ([9, 0, 30, 0, 0], [1, 130, 70, 1, 64], None, (1, 266, 0, 201, 1, 5), {0, 2}), ([0, 0], [2, 65], None, (0, 67, 0, 0, 0, 2), set()),
+            ([5, 8], [1, 1], None, None, {0, 1}), ([5, 0], [1, 1], None, (1, 2, 0, 1, 1, 2), {0}), ([64, 0], [64, 300], None, (64, 364, 0, 64, 1, 2), {0}),
             ([3] * 100 + [0] * 61, many, None, (100, 1420, 0, 100, 100, 161), set(range(100))),
             ([0] + [3] * 99 + [0] * 61, [2] + many[1:], [(160, 64 * i) for i in range(18, 0, -1)] + [(i, 0) for i in (0, *range(100, 161))], (0, 1421, 2, 101, 0, 161), set(range(1, 100)))):
         ctx, counts = np.asarray(ctx), np.asarray(counts)
@@ -469,6 +469,7 @@ def test_portions_over_keys_and_values_by_the_portion_alone():
         sec, _, _, plans = d._layout(a, counts, np.arange(n), T, n, 1, int((ctx + counts).max()))
         assert plans[0][3] is None and set(sec["tiles0"][::2]) == set(range(n))
         assert plans[1][3] == span and set(sec["tiles1"][::2]) == own
+        assert d._layout(a, counts, np.arange(n), T, n, 1, int((ctx + counts).max()), captured=True)[3][1][3] is None
         assert ("prompts" in sec) == (tiles is not None) and (tiles is None or list(map(tuple, sec["prompts"].reshape(-1, 2).tolist())) == tiles)
 
 

@@ -1044,14 +1044,14 @@ def test_a_prompt_comes_to_the_same_whatever_shares_its_step(dim, rot, rank, cou
         sec, _, _, plans = d._layout(a, n, np.arange(1), len(tok), len(own), tables.shape[1], int((c + n).max()))
         rt, sp, nt, spans = plans[0]
         assert "prompts" not in sec
-        tiles = i32([(e, m) for e in np.flatnonzero((c == 0) & (n > 1)) for m in range(0, n[e] + 64, 64)]).view(-1, 2) if listed else None      # (one more than there are, each)
+        tiles = i32([(e, m) for e in np.flatnonzero(c == 0) for m in range(0, n[e] + 64, 64)]).view(-1, 2) if listed else None      # (one more than there are, each)
         plan = layers.AttentionPlan(i32(sec["tiles0"]).view(nt, 2), rt, splits or sp, None if spans is None else ops.PromptTiles(tiles, *spans))
         cache, rows, step = pages.clone(), [], layout(n, c, tables[own], page)
         res = type("Residual", (), {"branch_in": lambda self, *a: proj[torch.as_tensor(tok, device=dev())].clone(), "branch_out": lambda self, o, *a: rows.append(o)})()
         layer.run(res, step, {layer.tiling(): plan}, [cache])
         return rows[0], cache, plan
 
-    prompts, others = np.flatnonzero((ctx == 0) & (counts > 1)), np.flatnonzero((ctx > 0) | (counts == 1))
+    prompts, others = np.flatnonzero(ctx == 0), np.flatnonzero(ctx > 0)
     got, cache, plan = run(np.arange(B))
     assert plan.prompts is not None
     again, pages_again, _ = run(np.arange(B), listed=True)

@@ -247,9 +247,9 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const vmi_hy_latent_pr
   latent_prep_token<T, false>(p, s, nullptr, blockIdx.x, cs);
 }
 
-__global__ __launch_bounds__(256) void latent_prompt_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, b16* const rows, const int row0, const int min_len) {
+__global__ __launch_bounds__(256) void latent_prompt_prep_kernel(const vmi_hy_latent_prep_args p, const vmi_hy_step s, b16* const rows, const int row0, const bool mixed) {
   extern __shared__ float cs[];
-  latent_prompt_prep_token(p, s, rows, row0, min_len, blockIdx.x, cs);
+  latent_prompt_prep_token(p, s, rows, row0, mixed, blockIdx.x, cs);
 }
 
 template <typename T, int KT, int RT, int NT, int U, bool EXACT = false>
@@ -310,17 +310,17 @@ int check_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, co
   return VMI_HY_OK;
 }
 
-int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, int min_len, const vmi_hy_step* s, const char* who) {
+int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, bool mixed, const vmi_hy_step* s, const char* who) {
   if (!a || !rows || !s || !a->proj || !a->cache || !a->norm_w || !a->freq || !s->tok_seq || !s->tok_pos || !s->tok_slot || s->T <= 0 || a->heads <= 0 || a->rank_n <= 0 ||
-      a->rank_n > a->rank || row0 < 0 || row0 >= s->T || min_len < 0 || (min_len > 0 && (!a->q || !s->ctx || !s->q_len)))
+      a->rank_n > a->rank || row0 < 0 || row0 >= s->T || (mixed && (!a->q || !s->ctx)))
     return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
   if (!vmi_hy_latent_prompt_fits(a->dim, a->rot, a->dim, a->rank, a->rot_n, a->dtype) || (a->ldp & 7) || (((uintptr_t)a->proj | (uintptr_t)rows | (uintptr_t)a->cache) & 15))
     return fail(VMI_HY_E_SHAPE, who, "needs sizes that vmi_hy_latent_prompt is built for, rows aligned to 16 bytes");
   return VMI_HY_OK;
 }
 
-int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who) {
-  hipLaunchKernelGGL(latent_prompt_prep_kernel, dim3(s.T), dim3(256), latent_prep_lds(a.rot_n), st, a, s, static_cast<b16*>(rows), row0, min_len);
+int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, bool mixed, const vmi_hy_step& s, hipStream_t st, const char* who) {
+  hipLaunchKernelGGL(latent_prompt_prep_kernel, dim3(s.T), dim3(256), latent_prep_lds(a.rot_n), st, a, s, static_cast<b16*>(rows), row0, mixed);
   return launched(who);
 }
 
@@ -346,10 +346,10 @@ int vmi_hy_latent_prep(const vmi_hy_latent_prep_args* a, const vmi_hy_step* s, v
 
 int vmi_hy_latent_prompt_prep(const vmi_hy_latent_prep_args* a, void* rows, const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_latent_prompt_prep";
-  if (int rc = check_latent_prompt_prep(a, rows, 0, 0, s, who)) return rc;
+  if (int rc = check_latent_prompt_prep(a, rows, 0, false, s, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
-  return launch_latent_prompt_prep(*a, rows, 0, 0, *s, static_cast<hipStream_t>(stream), who);
+  return launch_latent_prompt_prep(*a, rows, 0, false, *s, static_cast<hipStream_t>(stream), who);
 }
 
 int32_t vmi_hy_latent_row_tiles(int32_t row_dim, int32_t want, int32_t dtype) { return row_tiles_for(row_dim, want, dtype); }

@@ -98,18 +98,18 @@ __device__ __forceinline__ void latent_prep_token(const vmi_hy_latent_prep_args&
   }
 }
 
-// Entries without a past of min_len tokens on (0: every entry) for latent_prompt_kernel, `rows` beginning at token row0, the others as they are without it
-__device__ __forceinline__ void latent_prompt_prep_token(const vmi_hy_latent_prep_args& p, const vmi_hy_step& s, b16* const rows, const int row0, const int min_len, const int t,
+// Entries for latent_prompt_kernel, `rows` beginning at token row0: all, or, mixed, those without a past, and the others as they are without it
+__device__ __forceinline__ void latent_prompt_prep_token(const vmi_hy_latent_prep_args& p, const vmi_hy_step& s, b16* const rows, const int row0, const bool mixed, const int t,
                                                          float* const lds) {
   const int e = s.tok_seq[t];
   if (e < 0) return;
-  if (min_len == 0 || (s.ctx[e] == 0 && s.q_len[e] >= min_len)) latent_prep_token<b16, true>(p, s, rows - (int64_t)row0 * (p.rank + p.rot), t, lds);   // (workgroup-uniform)
+  if (!mixed || s.ctx[e] == 0) latent_prep_token<b16, true>(p, s, rows - (int64_t)row0 * (p.rank + p.rot), t, lds);   // (workgroup-uniform)
   else latent_prep_token<b16, false>(p, s, nullptr, t, lds);
 }
 
-int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, int min_len, const vmi_hy_step* s, const char* who);
-int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who);
+int check_latent_prompt_prep(const vmi_hy_latent_prep_args* a, const void* rows, int row0, bool mixed, const vmi_hy_step* s, const char* who);
+int launch_latent_prompt_prep(const vmi_hy_latent_prep_args& a, void* rows, int row0, bool mixed, const vmi_hy_step& s, hipStream_t st, const char* who);
 // ... and l, the other entries' queries by heads into a's q, which does not read what that writes nor writes what it reads: few rows in one launch
-int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who);
+int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, bool mixed, const vmi_hy_step& s, hipStream_t st, const char* who);
 
 }  // namespace vmi_hybrid

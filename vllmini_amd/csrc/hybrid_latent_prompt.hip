@@ -13,7 +13,7 @@
 // with both up-projections stands for two by heads, of the same work (16 heads, 2773 rows 27 + 19 us).
 // All kernels of a layer between its norms, latents / here, us, prompts only; 16 heads, dim + rot, rank, 1 x 60, 1 x 200, 16 x up to 200, 4 x up to 1024, 1 x 1024: 128 + 64, 512 52 / 44, 70 / 54, 124 / 92, 243 / 137, 153 / 90;
 // 128 + 64, 64 46 / 43, 58 / 50, 94 / 88, 164 / 126, 110 / 87; 128 + 32, 64 45 / 42, 58 / 50, 93 / 86, 160 / 120, 106 / 86; 64 + 64, 64 44 / 39, 55 / 44, 86 / 76, 153 / 105, 105 / 75; 64 + 32, 64 44 / 39, 55 / 42, 84 / 72, 145 / 95,
-// 103 / 70; so also where a latent row is no longer than a head's columns, as each of 16 ranks and heads measured is, and from prompts of two tokens on: rank 512, 1 x 2 35.2 / 33.7, 1 x 8 42 / 35, 1 x 24 45 / 36, 6 x up to 20 64 / 53.
+// 103 / 70; so also where a latent row is no longer than a head's columns, as each of 16 ranks and heads measured is, and for prompts of any length: rank 512, 1 x 2 35.2 / 33.7, 1 x 8 42 / 35, 1 x 24 45 / 36, 6 x up to 20 64 / 53.
 // Beside entries with a past, which keep the latents and their launches: 64 of those behind 1000 tokens and 1 x 100 111 / 101; 12 behind 300 and 1 x 8, 48, 100, 500 51 / 57, 64 / 68, 72 / 76, 111 / 110.
 // Off 64 bits by as much, latents / here, eight draws each: 8 heads, 60 rows 0.00346 / 0.00350, 300 + 200 + 100 0.00355 / 0.00357, 600 0.00364 / 0.00363; 16 heads, 1024 0.00362 / 0.00360.
 #include "hybrid_latent_prep.hpp"
@@ -30,7 +30,7 @@ struct LatentPrompt {
   const int* tiles;   // [..][2]: entry, first position; NULL: the places of `entries` entries from entry0 on, the last of `places` first
   int64_t ldp, ldkv, ldr, ldg, ldo;
   int heads, rank, row0, tile0;   // kv and rows begin at token row0, a launch at tile tile0
-  int places, entry0, entries, min_len;   // min_len: 0, or the shortest entry without a past that is meant
+  int places, entry0, entries, mixed;   // mixed: some of them have a past, and are others'
   float scale;
 };
 
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(256, 2) void latent_prompt_kernel(const LatentPromp
   const int group = blockIdx.x / p.heads, h = blockIdx.x - group * p.heads, tile = p.tile0 + group, place = tile / p.entries;
   const int e = p.tiles ? p.tiles[2 * tile] : p.entry0 + tile - place * p.entries, q0 = p.tiles ? p.tiles[2 * tile + 1] : (p.places - 1 - place) * PQ;
   const int qs = s.q_start[e], len = s.q_len[e];
-  if (p.min_len && (s.ctx[e] != 0 || len < p.min_len)) return;
+  if (p.mixed && s.ctx[e] != 0) return;
   if (q0 >= len) return;
   const int nkt = (min(len, q0 + PQ) + PQ - 1) / PQ;
   const b16* kv = p.kv + (int64_t)(qs - p.row0) * p.ldkv + h * (DN + VD);
@@ -210,17 +210,17 @@ int vmi_hy_latent_prompt(const void* proj, int64_t ldp, const void* kv, int64_t 
 }
 
 int vmi_hy_latent_prompts(const vmi_hy_latent_prep_args* a, const vmi_hy_latent_attention_args* past, const void* w_uk, const void* w_uv, const void* w_kv, const void* gate, int64_t ldg,
-                          void* out, int64_t ldo, void* rows, void* kv, const int32_t* tiles, int32_t n_tiles, int32_t max_len, const int32_t span[6], int32_t min_len, float scale,
+                          void* out, int64_t ldo, void* rows, void* kv, const int32_t* tiles, int32_t n_tiles, int32_t max_len, const int32_t span[6], float scale,
                           const vmi_hy_step* s, void* stream) {
   static const char* who = "vmi_hy_latent_prompts";
   if (!a || !w_kv || !gate || !out || !kv || !span || !s || !s->q_start || !s->q_len || s->T <= 0 || s->B <= 0 || span[0] < 0 || span[1] <= span[0] || span[1] > s->T ||
-      (tiles ? n_tiles <= 0 : (max_len <= 0 || span[4] < 0 || span[5] <= span[4] || span[5] > s->B)) || (span[3] == 0) != (min_len == 0))
+      (tiles ? n_tiles <= 0 : (max_len <= 0 || span[4] < 0 || span[5] <= span[4] || span[5] > s->B)) || span[3] < 0 || (span[3] > 0 && !s->ctx))
     return fail(VMI_HY_E_ARG, who, "null pointer or a size out of range");
   const int first = span[0], n = span[1] - first, at = span[2], others = span[3] == 0 ? 0 : span[3] - at, heads = a->heads, dim = a->dim, rank = a->rank, row = rank + a->rot;
   if (others < 0 || at < 0 || span[3] > s->T || (others && (!past || !w_uk || !w_uv || !a->q || past->q != a->q || !past->out || past->heads != heads || past->rank != rank ||
                                                             past->rot != a->rot || past->dtype != a->dtype || past->device != a->device)))
     return fail(VMI_HY_E_ARG, who, "what the entries beside the prompts take does not fit");
-  if (int rc = check_latent_prompt_prep(a, rows, first, min_len, s, who)) return rc;
+  if (int rc = check_latent_prompt_prep(a, rows, first, others > 0, s, who)) return rc;
   DeviceScope dev(a->device);
   if (!dev.ok) return fail(VMI_HY_E_HIP, who, "hipSetDevice failed");
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -235,17 +235,17 @@ int vmi_hy_latent_prompts(const vmi_hy_latent_prep_args* a, const vmi_hy_latent_
     uv.x_gstride = rank, uv.y_gstride = dim, uv.M = others, uv.N = dim, uv.K = rank, uv.epilogue = VMI_HY_E_GATED, uv.gate = rows_of(gate) + at * ldg, uv.ldg = ldg;
     if (int rc = check_linear(&uk, who)) return rc;
     if (int rc = check_linear(&uv, who)) return rc;
-    if (int rc = launch_latent_prompt_in(uk, *a, rows, first, min_len, *s, st, who)) return rc;
+    if (int rc = launch_latent_prompt_in(uk, *a, rows, first, others > 0, *s, st, who)) return rc;
     if (int rc = vmi_hy_latent_attention(past, s, st)) return rc;
     if (int rc = vmi_hy_linear(&uv, st)) return rc;
-  } else if (int rc = launch_latent_prompt_prep(*a, rows, first, min_len, *s, st, who)) {
+  } else if (int rc = launch_latent_prompt_prep(*a, rows, first, others > 0, *s, st, who)) {
     return rc;
   }
   l.x = rows, l.w = w_kv, l.y = kv, l.ldx = row, l.ldy = ldkv, l.M = n, l.N = (int)ldkv, l.K = rank, l.groups = 1;
   if (int rc = vmi_hy_product_tiles(&l, st)) return rc;
   const int places = tiles ? 0 : (max_len - 1) / PQ + 1, entries = tiles ? 1 : span[5] - span[4];
   const LatentPrompt p{rows_of(a->proj), rows_of(kv), rows_of(rows), rows_of(gate), static_cast<b16*>(out), tiles, a->ldp, ldkv, row, ldg, ldo, heads, rank, first, 0,
-                       places, span[4], entries, tiles ? 0 : min_len, scale};
+                       places, span[4], entries, !tiles && others, scale};
   return run_prompt(p, dim, a->rot, tiles ? n_tiles : (int64_t)places * entries, *s, st, who);
 }
 

@@ -171,9 +171,10 @@ struct LatentPrep {
 struct LatentPromptPrep {
   vmi_hy_latent_prep_args a;
   b16* rows;
-  int row0, min_len;
+  int row0;
+  bool mixed;
   __device__ __forceinline__ void token(const vmi_hy_step& s, int t, unsigned char* smem) const {
-    latent_prompt_prep_token(a, s, rows, row0, min_len, t, reinterpret_cast<float*>(smem));
+    latent_prompt_prep_token(a, s, rows, row0, mixed, t, reinterpret_cast<float*>(smem));
   }
 };
 struct KvPrep {
@@ -701,10 +702,10 @@ static int launch_beside(const vmi_hy_linear_args& p, const Prep& prep, const vm
   return mt == 1 ? go(rows_beside_kernel<4, 1, Prep>, 4) : go(rows_beside_kernel<4, 2, Prep>, 4);
 }
 
-int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, int min_len, const vmi_hy_step& s, hipStream_t st, const char* who) {
-  if (beside_fits(l, s)) return launch_beside(l, LatentPromptPrep{a, static_cast<b16*>(rows), row0, min_len}, s, latent_prep_lds(a.rot_n), who, st);
+int launch_latent_prompt_in(const vmi_hy_linear_args& l, const vmi_hy_latent_prep_args& a, void* rows, int row0, bool mixed, const vmi_hy_step& s, hipStream_t st, const char* who) {
+  if (beside_fits(l, s)) return launch_beside(l, LatentPromptPrep{a, static_cast<b16*>(rows), row0, mixed}, s, latent_prep_lds(a.rot_n), who, st);
   if (int rc = vmi_hy_linear(&l, st)) return rc;
-  return launch_latent_prompt_prep(a, rows, row0, min_len, s, st, who);
+  return launch_latent_prompt_prep(a, rows, row0, mixed, s, st, who);
 }
 
 int launch_plain_rows(const vmi_hy_linear_args& p, hipStream_t st) {

@@ -94,8 +94,8 @@ class HybridDecoder:
             n *= 2
         return n
 
-    def _layout(self, a: dict, counts: np.ndarray, rows: np.ndarray, T: int, B: int, table_ld: int, max_keys: int):
-        """One int32 buffer with everything a step's kernels read, as named sections; T / B may exceed what is there (padding)."""
+    def _layout(self, a: dict, counts: np.ndarray, rows: np.ndarray, T: int, B: int, table_ld: int, max_keys: int, captured: bool = False):
+        """One int32 buffer with everything a step's kernels read, as named sections; T / B may exceed what is there (padding).  captured: the launches stand already, for any contexts."""
         n, b = int(counts.sum()), len(counts)
         starts = np.cumsum(counts) - counts
         sec: Dict[str, np.ndarray] = {}
@@ -119,9 +119,9 @@ class HybridDecoder:
         sec["table"] = tab.reshape(-1)
         put("rows", max(len(rows), 1), rows, 0)
         plans = []
-        several, prompts = bool((counts > 1).any()), None
-        if several and any(kind.prompts for kind in self._kinds):
-            pays = ops.latent_prompt_pays((a["ctx"], counts))
+        prompts = None
+        if not captured and not a["ctx"].all() and any(kind.prompts for kind in self._kinds):
+            pays = ops.latent_prompt_pays(a["ctx"])
             prompts = self._prompts(sec, pays, counts, starts) if np.any(pays) else None
         for kind in self._kinds:
             mine, keys, entries, own = counts, max_keys, B, prompts if kind.prompts else None      # (the portions of this kind's own tiles)
@@ -145,7 +145,7 @@ class HybridDecoder:
             t[: len(ent), 0], t[: len(ent), 1] = ent, first
             sec[f"tiles{len(plans)}"] = t.reshape(-1)
             plans.append((rt, self._split_of(nt, rt, kind, keys, T), nt, own))
-        if several:                           # runs of rows for the linear-attention layers
+        if (counts > 1).any():                # runs of rows for the linear-attention layers
             per = -(-counts // ops.CHUNK_ROWS)
             at = np.cumsum(per) - per
             put("chunk_start", B, at, 0)
@@ -348,7 +348,7 @@ class HybridDecoder:
         bucket = 2 * self.KEY_TILE
         while bucket < keys:
             bucket *= 2
-        sec, offs, total, plans = self._layout(a, counts, np.arange(Bp), Bp, Bp, MB, bucket)
+        sec, offs, total, plans = self._layout(a, counts, np.arange(Bp), Bp, Bp, MB, bucket, captured=True)
         key = (Bp, tuple(plans))
         hit = self._sets.get(key)
         if hit is None:

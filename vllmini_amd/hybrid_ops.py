@@ -103,7 +103,7 @@ SIGNATURES = {
     "vmi_hy_latent_prompt_prep": (ctypes.c_int, [ctypes.POINTER(PrepArgs), _vp, ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_prompt_fits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "vmi_hy_latent_prompt": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, *[_i32] * 6, _f32, _i32, _i32, ctypes.POINTER(StepArgs), _vp]),
-    "vmi_hy_latent_prompts": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(AttentionArgs), *[_vp] * 4, _i64, _vp, _i64, *[_vp] * 3, _i32, _i32, ctypes.POINTER(_i32 * 6), _i32, _f32,
+    "vmi_hy_latent_prompts": (ctypes.c_int, [ctypes.POINTER(PrepArgs), ctypes.POINTER(AttentionArgs), *[_vp] * 4, _i64, _vp, _i64, *[_vp] * 3, _i32, _i32, ctypes.POINTER(_i32 * 6), _f32,
                                              ctypes.POINTER(StepArgs), _vp]),
     "vmi_hy_latent_row_tiles": (_i32, [_i32, _i32, _i32]),
     "vmi_hy_latent_attention": (ctypes.c_int, [ctypes.POINTER(AttentionArgs), ctypes.POINTER(StepArgs), _vp]),
@@ -576,15 +576,13 @@ def latent_prompt_fits(dim: int, rot: int, vdim: int, rank: int, rot_n: int, dty
     return dtype == torch.bfloat16 and bool(load().vmi_hy_latent_prompt_fits(dim, rot, vdim, rank, rot_n, DTYPES[dtype]))
 
 
-PROMPT_TILE, PROMPT_MIN_TOKENS = 64, 2      # positions of a tile of latent_prompt's kernel; the shortest portion that goes there
+PROMPT_TILE = 64      # positions of a tile of latent_prompt's kernel
 
 
-def latent_prompt_pays(portions: Tuple[np.ndarray, np.ndarray]) -> np.ndarray:
-    """Which of a step's portions (their contexts, their tokens) go through latent_prompt: by the portion alone, whatever shares its step, so that a prompt's keys and values are rounded at the
-    same places beside others as by itself (vmi_hy_latent_prompts has the same rule).  Ahead of the latents from two tokens on (csrc/hybrid_latent_prompt.hip); one is a decoding
-    step's."""
-    ctx, tokens = portions
-    return (ctx == 0) & (tokens >= PROMPT_MIN_TOKENS)
+def latent_prompt_pays(ctx: np.ndarray) -> np.ndarray:
+    """Which of a step's portions, behind `ctx` tokens each, go through latent_prompt: those without a past, whatever shares their step, so that a prompt's keys and values are rounded at the
+    same places beside others as by itself (vmi_hy_latent_prompts has the same rule); ahead of the latents, or level, from one token on (csrc/hybrid_latent_prompt.hip)."""
+    return ctx == 0
 
 
 class PromptTiles(NamedTuple):
@@ -642,7 +640,7 @@ def latent_prompt(proj: torch.Tensor, w_kv: MatrixTiles, cache: torch.Tensor, st
                                        n_tiles=past.tiles.shape[0], row_tiles=past.row_tiles, splits=past.splits, scale=scale, dtype=a.dtype, device=device))
     _check(load().vmi_hy_latent_prompts(ctypes.byref(a), b, _ptr(w_uk), _ptr(w_uv), w_kv.tiles.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(), out.stride(0), rows.data_ptr(),
                                         kv.data_ptr(), _ptr(tiles), 0 if tiles is None else tiles.shape[0], step.max_len, ctypes.byref((_i32 * 6)(*span)),
-                                        PROMPT_MIN_TOKENS if mixed else 0, scale, step.ref, stream))      # (which entries, latent_prompt_pays has for the host)
+                                        scale, step.ref, stream))
     return out
 
 
